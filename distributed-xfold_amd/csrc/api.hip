@@ -85,7 +85,7 @@ const char* af3_error_string(int code) {
 // ------------------------------------------------------ triangle multiplication
 // The N x N x N contraction of the triangle multiplication: the 256x256-tile
 // kernel once a token count fills at least part of a second 128-row tile,
-// the general 128x128-tile GEMM below that.
+// the general GEMM below that.
 static int contraction(const GemmArgs& g, hipStream_t s) {
   if (g.M > 128 && contract_supported(g)) return launch_contract(g, s);
   return launch_gemm_nt(g, s);

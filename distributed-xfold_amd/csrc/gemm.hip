@@ -1,15 +1,37 @@
 // Batched "NT" GEMM on bf16 MFMA:  C[b][m][n] = epi( sum_k A[b][m][k] * B[b][n][k] )
 //
 // Both operands are k-contiguous, which is the natural fragment order of
-// v_mfma_f32_32x32x16_bf16, so a 16-byte load feeds one fragment.  The
-// workgroup tile is 128x128 with a 64-deep k slab, double-buffered in LDS and
-// prefetched through registers; four waves each own a 64x64 quadrant (2x2 MFMA
-// tiles, 64 fp32 accumulators).
+// v_mfma_f32_32x32x16_bf16, so a 16-byte read feeds one fragment.  This file
+// carries the dense projections outside the 128-channel pair path (single /
+// diffusion / atom attention and transitions) and the triangle contraction of
+// small token counts; large products whose epilogue the 256x256-tile kernel
+// (contract.hip) knows are handed to it by launch_gemm_nt.
 //
-// This kernel carries the dense projections outside the 128-channel pair path
-// (single / diffusion / atom attention and transitions) and the triangle
-// contraction of small token counts; large products whose epilogue the
-// 256x256-tile kernel (contract.hip) knows are handed to it by launch_gemm_nt.
+// Most of these products are short: 64 to 4000 rows, K = 128 ... 1536, 0.1 to
+// 10 GFLOP, so that what they cost is not matrix time but the number of CUs
+// that have a tile and the length of one workgroup's chain (first miss, K loop,
+// hand-over, store).  Hence:
+//   * the tile shrinks with the product (128x128 down to 32x32) until about every
+//     CU has one, and where that is not enough the waves of a workgroup share the K
+//     range of one tile instead of its area (WK groups; their fp32 partial tiles
+//     are added in LDS): K = 1536 is then a chain of three slabs, not of 24;
+//   * slabs are 64 deep, so a slab row is one whole 128-byte cache line.  From L2 a CU takes
+//     in 115 bytes/ns that way; in 64-byte row pieces it is 62 (measured, LDS-direct loads);
+//   * slabs go from global memory straight into LDS, all of a workgroup's first ones
+//     before anything is waited for.  A group of one wave (ALONE) shares its slabs with
+//     nobody: its K loop has no barrier, only waits for its own loads;
+//   * the accumulators hold C^T tiles (weight fragments as the MFMA's A operand): a
+//     lane owns one row and four consecutive columns per register quad, so a partial
+//     tile goes to LDS in 16-byte stores.
+//
+// The order in which K is summed depends on N and K alone, never on M (gemm_k_groups): a
+// sample gives the same bits alone and in a batch, whatever tile either takes.  Where K is
+// summed in four groups, (p0 + p1) + (p2 + p3), a tile whose waves do not share the K range
+// keeps the groups apart in its accumulators.
+//
+// Measured against the register-staged 128x128-tile kernel this replaces: 64x384x384
+// 3.5 us (was 8.9), 64x384x1536 5.2 (19.6), 500x768x768 5.3 (14.3), 500x3072x768 10.9 (16.2), 1920x3072x768
+// 17.4 (22.6), 3840x768x768 12.8 (15.3), 768x73728x384 to fp32 112 (125), 12000x256x128 6.4 (11.3).
 #include <type_traits>
 
 #include "common.h"
@@ -17,22 +39,47 @@
 
 namespace {
 
-constexpr int BM = 128, BN = 128, BK = 64;
-constexpr int LDT = BK + 8;  // padded LDS row (bf16 elements): 144 B keeps 16-B reads conflict-free
+constexpr int KS = 64;        // slab depth
+constexpr int ROWB = KS * 2;  // bytes of a slab row in LDS (unpadded, 16-byte chunks permuted)
 
-constexpr int LDC_S = BN + 4;  // fp32 staging row stride of the C tile
+// 64 lanes x 16 bytes from global (uniform base + per-lane byte offset) to the ith KB of LDS behind the
+// wave-uniform address lds.  Inline assembly, because the compiler's own form makes later LDS reads wait for every
+// such load in flight; here a buffer is read only behind an explicit wait.
+__device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint32_t lds, int i) {
+  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base), "n"(i * 1024)
+               : "m0", "scc", "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads_but() {
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 
-// K_TAIL: K is not a multiple of the slab depth, so chunks past K have to be zeroed on their way to LDS.
-template <bool OUT_F32, bool K_TAIL>
-__global__ __launch_bounds__(256, 2) void gemm_nt_kernel(GemmArgs g) {
-  // A/B slabs, double buffered; after the k loop the same memory stages the C tile
-  __shared__ __attribute__((aligned(16))) bf16_t smem[2 * (BM + BN) * LDT];
-  static_assert(BM * LDC_S * 4 <= 2 * (BM + BN) * LDT * 2, "C staging must fit");
-  constexpr int STAGE = (BM + BN) * LDT;  // buffer `buf`: A slab at smem + buf * STAGE, B slab BM rows later
-  float* sC = reinterpret_cast<float*>(smem);
+// A workgroup of WM x WN x WK waves computes BM = 32 MT WM rows x BN = 32 NT WN columns; ST slab buffers per group.
+// KIND: the epilogue.  VEC: all of its loads and stores are 16-byte ones (without: element by element, for odd column
+// counts and unaligned operands).  GROUPS: K is summed in four groups.  WPS: waves per SIMD the tile's LDS leaves room for; the
+// registers have to as well (a wave more or less per SIMD is up to a factor of two in the short products).
+enum { KIND_COLUMNS = 0, KIND_GATE_RES = 1, KIND_SWIGLU = 2 };
+template <int MT, int NT, int WM, int WN, int WK, int ST, int WPS, bool GROUPS, int KIND, bool VEC, bool OUT_F32>
+__global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArgs g) {
+  constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN, NTHR = 64 * WM * WN * WK, GW = WM * WN;
+  constexpr int SLAB = (BM + BN) * ROWB;     // A rows first, then B rows
+  constexpr int NLOAD = (BM + BN) / 8 / GW;  // 1 KB loads per wave and slab
+  constexpr int LA = BM / 8 / GW;            // of which A
+  static_assert(WK == 1 || WK == 2 || WK == 4, "");
+  static_assert((BM / 8) % GW == 0 && (BN / 8) % GW == 0, "loads of a slab are dealt evenly");
+  constexpr bool ALONE = GW == 1;
+  constexpr int FLY = ALONE ? ST : ST - 1;   // slabs requested ahead
+  static_assert(FLY >= 1 && FLY <= 2 && FLY * NLOAD < 64, "");
+  constexpr int LDS_C = BN + 4;              // row stride (fp32) of a partial tile
+  constexpr int BYTES = WK * ST * SLAB > WK * BM * LDS_C * 4 ? WK * ST * SLAB : WK * BM * LDS_C * 4;
+  __shared__ __attribute__((aligned(1024))) char smem[BYTES];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hh = lane >> 5, l31 = lane & 31;
+  const int grp = wave / GW, gw = wave % GW;
+  const int wm = (gw / WN) * 32 * MT, wn = (gw % WN) * 32 * NT;
 
   // XCD-aware mapping: workgroup ids are dealt round-robin to the 8 XCDs, so
   // id -> (xcd, slot) -> logical id makes each XCD walk a contiguous range of
@@ -42,243 +89,245 @@ __global__ __launch_bounds__(256, 2) void gemm_nt_kernel(GemmArgs g) {
   const int total = tiles_m * tiles_n * g.batch;
   const int per_xcd = (total + 7) / 8;
   const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (logical >= total) return;
-  const int tm = logical % tiles_m, tn = (logical / tiles_m) % tiles_n;
-  const int bz = logical / (tiles_m * tiles_n);
-  const int m0 = tm * BM, n0 = tn * BN;
+  if ((int)(blockIdx.x >> 3) >= per_xcd || logical >= total) return;
+  const int m0 = __builtin_amdgcn_readfirstlane(logical % tiles_m) * BM;
+  const int n0 = __builtin_amdgcn_readfirstlane((logical / tiles_m) % tiles_n) * BN;
+  const int bz = __builtin_amdgcn_readfirstlane(logical / (tiles_m * tiles_n));
 
-  const bf16_t* A = g.A + (int64_t)bz * g.sA;
-  const bf16_t* B = g.B + (int64_t)bz * g.sB;
+  // the tile's first rows: what a lane adds to these fits 32 bits whatever the operands' size
+  const char* A = reinterpret_cast<const char*>(g.A + (int64_t)bz * g.sA + (int64_t)m0 * g.lda);
+  const char* B = reinterpret_cast<const char*>(g.B + (int64_t)bz * g.sB + (int64_t)n0 * g.ldb);
 
-  // each thread moves 4 16-byte chunks of A and 4 of B per k slab.  Two register
-  // sets: a slab is requested two iterations before it goes to LDS.  The small
-  // products this kernel is mostly used for (a few hundred rows, K = 384 ...
-  // 1536) run on fewer workgroups than there are CUs, so each workgroup is one
-  // chain of K / 64 memory round trips and nothing else covers their latency.
-  const int ld_row = tid >> 3, ld_kc = (tid & 7) * 8;  // + 32 rows per step
-  u32x4 ra[2][4], rb[2][4];
-  const bf16_t* pa[4];
-  const bf16_t* pb[4];
+  // Load i of a wave covers eight rows of A (i < LA) or B, one 128-byte row per 8 lanes.  Chunk c of row r lives at
+  // position c ^ ((r >> 1) & 7) of the row (a load cannot pad rows): 16 consecutive rows' reads of one chunk then
+  // cover all 64 banks.  Rows past the end repeat the last one; what they produce is not stored.
+  const int lr = lane >> 3;
+  auto row_of = [&](int i) { return i < LA ? 8 * (LA * gw + i) + lr : 8 * ((NLOAD - LA) * gw + i - LA) + lr; };
+  auto chunk_of = [&](int i) { return (lane & 7) ^ ((row_of(i) >> 1) & 7); };
+  uint32_t off[NLOAD];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = ld_row + 32 * i;
-    pa[i] = A + (int64_t)min(m0 + row, g.M - 1) * g.lda + ld_kc;
-    pb[i] = B + (int64_t)min(n0 + row, g.N - 1) * g.ldb + ld_kc;
-  }
-  // unconditional loads (a chunk past K re-reads the row's first one) whose
-  // values are zeroed on their way to LDS
-  bool k_ok[2] = {true, true};
-  auto gload = [&](int set, int k0) {
-    k_ok[set] = k0 + ld_kc < g.K;
-    const int kk = k_ok[set] ? k0 : -ld_kc;
+  for (int i = 0; i < NLOAD; ++i)
+    off[i] = i < LA ? ((uint32_t)min(row_of(i), g.M - 1 - m0) * (uint32_t)g.lda + chunk_of(i) * 8) * 2u
+                    : ((uint32_t)min(row_of(i), g.N - 1 - n0) * (uint32_t)g.ldb + chunk_of(i) * 8) * 2u;
+  const int ns = (g.K + KS - 1) / KS;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)smem;
+  const int s0 = grp * ns / WK, cnt = (grp + 1) * ns / WK - s0;
+  constexpr int NG = GROUPS ? 4 / WK : 1;  // groups of the K sum that this wave goes through
+  const uint32_t mine = (uint32_t)(grp * (ST * SLAB));  // this group's buffers in smem
+  auto issue = [&](int s, uint32_t dst) {
+    const uint32_t da = __builtin_amdgcn_readfirstlane(lds0 + dst + LA * gw * 1024);
+    const uint32_t db = __builtin_amdgcn_readfirstlane(lds0 + dst + BM * ROWB + (NLOAD - LA) * gw * 1024);
+    const uint32_t k0 = (uint32_t)(s0 + s) * KS;
+    const bool tail = k0 + KS > (uint32_t)g.K;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      ra[set][i] = *reinterpret_cast<const u32x4*>(pa[i] + kk);
-      rb[set][i] = *reinterpret_cast<const u32x4*>(pb[i] + kk);
-    }
-  };
-  auto sstore = [&](int set, int buf) {
-    const u32x4 z = {0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = ld_row + 32 * i;
-      *reinterpret_cast<u32x4*>(smem + buf * STAGE + row * LDT + ld_kc) = !K_TAIL || k_ok[set] ? ra[set][i] : z;
-      *reinterpret_cast<u32x4*>(smem + buf * STAGE + (BM + row) * LDT + ld_kc) = !K_TAIL || k_ok[set] ? rb[set][i] : z;
+    for (int i = 0; i < NLOAD; ++i) {
+      uint32_t kb = k0 * 2u;
+      // a chunk past K is fetched from its place in the row's first slab (K >= 64) or from the row's start, and
+      // zeroed in LDS before the slab is used
+      if (tail && k0 + chunk_of(i) * 8 >= (uint32_t)g.K) kb = g.K >= KS ? 0u : 0u - (uint32_t)chunk_of(i) * 16u;
+      if (i < LA) load_to_lds(A, off[i] + kb, da, i);
+      else load_to_lds(B, off[i] + kb, db, i - LA);
     }
   };
 
-  f32x16 acc[2][2];
+  // ------------------------------------------------------------- epilogue operands
+  // After the K loop a thread finishes chunks of 8 consecutive columns.  Gate and residual of PRE chunks are
+  // requested at a time, ahead of the stores (which may alias the residual, so no load moves above one); where a
+  // thread has no more chunks than that, ahead of the K loop.
+  constexpr int CPR = BN / 8;                        // chunks per row
+  constexpr int NCH = (BM * CPR + NTHR - 1) / NTHR;  // chunks per thread
+  constexpr int PRE = NCH < 2 ? NCH : 2;
+  constexpr bool EARLY = NCH == 1;
+  struct Pre { float gate[8]; u32x4 r0, r1; };
+  Pre pre[PRE];
+  auto fetch = [&](int k, Pre& p) {
+    const int idx = tid + k * NTHR, m = min(m0 + idx / CPR, g.M - 1), n = n0 + (idx % CPR) * 8;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int e = 0; e < 8; ++e) p.gate[e] = 1.f;
+    p.r0 = p.r1 = u32x4{0, 0, 0, 0};
+    if ((BM * CPR < NTHR && idx >= BM * CPR) || n >= g.N) return;
+    const int64_t roff = (int64_t)bz * g.sRes + (int64_t)m * g.ld_res + n;
+    const float* gp = g.gate && !g.gate_per_row ? g.gate + (int64_t)(m % g.gate_rows) * g.ld_gate + n : nullptr;
+    if (g.gate && g.gate_per_row) {
+      const float f = g.gate[m % g.gate_rows];
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  const int nk = (g.K + BK - 1) / BK;
-  gload(0, 0);
-  gload(1, BK);  // past K when nk == 1: a clamped re-read, never stored
-  sstore(0, 0);
-  lds_barrier();
-
-  // slab kt is in LDS buffer kt & 1, slab kt + 1 in register set (kt + 1) & 1,
-  // and set kt & 1 (just stored) takes slab kt + 2
-  auto stage = [&](int kt, auto par_c) {
-    constexpr int par = decltype(par_c)::value;
-    // Requested on every iteration, also past the last slab (a clamped
-    // re-read that is never stored): a load under a condition leaves the
-    // compiler unable to count the loads in flight, and it then waits for all
-    // of them, the slab just requested included, before the LDS stores below.
-    gload(par, (kt + 2) * BK);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      bf16x8 fa[2], fb[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) fa[i] = lds_frag(smem + par * STAGE, LDT, wm + 32 * i, ks * 16, lane);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) fb[j] = lds_frag(smem + par * STAGE + BM * LDT, LDT, wn + 32 * j, ks * 16, lane);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = mfma32(fa[i], fb[j], acc[i][j]);
+      for (int e = 0; e < 8; ++e) p.gate[e] = f;
     }
-    // The next slab (requested one stage ago) goes into the other LDS buffer, which nobody reads during
-    // this stage, while the matrix unit works: its eight stores are dealt out between the MFMAs of the
-    // second half, behind the fragment reads (issued four ahead of the MFMAs that use them).  Unconditional,
-    // so that it stays in one basic block with them: after the last slab it stores a clamped re-read that
-    // nobody uses (the C tile is staged over it only after the barrier below).
-    sstore(par ^ 1, par ^ 1);
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    lds_barrier();
-  };
-  for (int kt = 0; kt < nk; kt += 2) {
-    stage(kt, std::integral_constant<int, 0>{});
-    if (kt + 1 < nk) stage(kt + 1, std::integral_constant<int, 1>{});
-  }
-
-  // ------------------------------------------------------------- epilogue
-  // accumulators (lane = column, registers = rows) -> fp32 tile in LDS, then
-  // each thread finishes 8 consecutive columns of a row with 16/32-byte stores
-  const int cc = (tid & 15) * 8, r0 = tid >> 4;
-  // Gate and residual of the thread's eight output chunks are requested here,
-  // all at once and ahead of the staging: asked for one chunk at a time between
-  // the stores (which may alias the residual, so the compiler keeps the order)
-  // they would be eight memory round trips in a row at the end of a workgroup
-  // that, in the small products, has nothing else to hide them behind.
-  const bool gr_ahead = g.epi == EPI_GATE_RES && g.vec_ok && n0 + cc + 8 <= g.N && !g.res_f32 &&
-                        (!g.gate || g.gate_per_row || g.gate_vec_ok) && (!g.res_bf16 || g.res_vec_ok);
-  f32x4 gate_lo[8], gate_hi[8];
-  u32x4 res_pk[8];
-  float gate_row[8];
-  if (gr_ahead) {
-#pragma unroll
-    for (int it = 0; it < 8; ++it) {
-      const int m = min(m0 + it * 16 + r0, g.M - 1), n = n0 + cc;
-      gate_row[it] = 1.f;
-      gate_lo[it] = gate_hi[it] = f32x4{1.f, 1.f, 1.f, 1.f};
-      res_pk[it] = u32x4{0, 0, 0, 0};
-      if (g.gate && g.gate_per_row) gate_row[it] = g.gate[m % g.gate_rows];
-      else if (g.gate) {
-        const float* gp = g.gate + (int64_t)(m % g.gate_rows) * g.ld_gate + n;
-        gate_lo[it] = *reinterpret_cast<const f32x4*>(gp);
-        gate_hi[it] = *reinterpret_cast<const f32x4*>(gp + 4);
+    if constexpr (VEC) {
+      if (gp) Elem<float>::load8(gp, p.gate);
+      if (g.res_f32) {
+        p.r0 = *reinterpret_cast<const u32x4*>(g.res_f32 + roff);
+        p.r1 = *reinterpret_cast<const u32x4*>(g.res_f32 + roff + 4);
+      } else if (g.res_bf16) {
+        p.r0 = *reinterpret_cast<const u32x4*>(g.res_bf16 + roff);
       }
-      if (g.res_bf16)
-        res_pk[it] = *reinterpret_cast<const u32x4*>(g.res_bf16 + (int64_t)bz * g.sRes + (int64_t)m * g.ld_res + n);
+    } else {
+      for (int e = 0; e < min(8, g.N - n); ++e) {
+        if (gp) p.gate[e] = gp[e];
+        if (g.res_f32) (e < 4 ? p.r0 : p.r1)[e & 3] = __float_as_uint(g.res_f32[roff + e]);
+        else if (g.res_bf16) p.r0[e >> 1] |= (uint32_t)g.res_bf16[roff + e] << (16 * (e & 1));
+      }
+    }
+  };
+
+  f32x16 acc[MT][NT], sum0[MT][NT], sum1[MT][NT];
+  auto each = [&](auto f) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) f(acc[i][j], sum0[i][j], sum1[i][j]);
+  };
+  const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  each([&](f32x16& a, f32x16& s, f32x16& t) { a = s = t = zero; });
+
+  uint32_t fo[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) fo[ks] = (uint32_t)(l31 * ROWB + (((2 * ks + hh) ^ ((l31 >> 1) & 7)) << 4));
+
+#pragma unroll
+  for (int p = 0; p < FLY; ++p)
+    if (p < cnt) issue(p, mine + p * SLAB);
+  if constexpr (KIND == KIND_GATE_RES && EARLY) fetch(0, pre[0]);
+
+  // One barrier per slab where waves share it (all groups take part in all of them): behind it the slab has
+  // landed for every wave of the group and the buffer of the slab before is free.
+  int cur = 0, i = 0;
+#pragma unroll 1
+  for (int gq = 0; gq < NG; ++gq) {
+    // (the last group of waves has the most slabs; the others join it at its barriers)
+    const int end = gq < NG - 1 ? (NG * grp + gq + 1) * ns / (NG * WK) - s0 : ALONE ? cnt : (ns + WK - 1) / WK;
+#pragma unroll 1
+    for (; i < end; ++i) {
+      const int rem = cnt - 1 - i;  // slabs of this wave still to come
+      if (FLY >= 2 && rem >= 1) wait_loads_but<(FLY >= 2 ? NLOAD : 0)>();
+      else wait_loads_but<0>();
+      const uint32_t bo = mine + cur * SLAB;
+      char* b = smem + bo;
+      const int k0 = (s0 + i) * KS;
+      if (!ALONE) lds_barrier();
+      if (i < cnt && k0 + KS > g.K) {
+        const u32x4 z = {0, 0, 0, 0};
+        for (int row = lane + 64 * gw; row < BM + BN; row += 64 * GW)
+          for (int c = (g.K - k0) >> 3; c < 8; ++c) *reinterpret_cast<u32x4*>(b + row * ROWB + ((c ^ ((row >> 1) & 7)) << 4)) = z;
+      }
+      if (!ALONE && ns * KS > g.K && i == (ns + WK - 1) / WK - 1) lds_barrier();
+      if (!ALONE && i + FLY < cnt) issue(i + FLY, mine + (cur == 0 ? ST - 1 : cur - 1) * SLAB);
+      if (ALONE || i < cnt) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+          bf16x8 fa[MT], fb[NT];
+#pragma unroll
+          for (int t = 0; t < MT; ++t) fa[t] = as_frag(*reinterpret_cast<const u32x4*>(b + (wm + t * 32) * ROWB + fo[ks]));
+#pragma unroll
+          for (int t = 0; t < NT; ++t) fb[t] = as_frag(*reinterpret_cast<const u32x4*>(b + (BM + wn + t * 32) * ROWB + fo[ks]));
+#pragma unroll
+          for (int x = 0; x < MT; ++x)
+#pragma unroll
+            for (int y = 0; y < NT; ++y) acc[x][y] = mfma32(fb[y], fa[x], acc[x][y]);
+        }
+      }
+      if (ALONE && i + ST < cnt) {  // the wave's fragment reads of the buffer must be done before it is refilled
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        issue(i + ST, bo);
+      }
+      cur = cur + 1 == ST ? 0 : cur + 1;
+    }
+    if (NG > 1 && gq < NG - 1) {
+      if (NG == 4 && gq == 1) each([&](f32x16& a, f32x16& s, f32x16& t) { t = s + a; a = zero; });
+      else each([&](f32x16& a, f32x16& s, f32x16&) { s = a; a = zero; });
     }
   }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        sC[(wm + 32 * i + acc_row(r, lane)) * LDC_S + wn + 32 * j + (lane & 31)] = acc[i][j][r];
-  lds_barrier();
+  if constexpr (NG == 4) each([](f32x16& a, f32x16& s, f32x16& t) { a = t + (s + a); });
+  if constexpr (NG == 2) each([](f32x16& a, f32x16& s, f32x16&) { a = s + a; });
 
-  if (g.epi == EPI_SWIGLU) {
-    // weight rows are packed in blocks of 64: 32 "a" rows then the 32 matching
-    // "b" rows; output has N/2 columns.  Threads with cc < 64 produce 8 outputs each.
-    if (cc >= 64) return;
-    const int blk = cc >> 5, off = cc & 31;         // which 64-column block, offset inside its a half
-    const int oc = n0 / 2 + cc;                     // first output column
-    if (n0 + blk * 64 >= g.N) return;               // N % 64 == 0
-    bf16_t* C = reinterpret_cast<bf16_t*>(g.C) + (int64_t)bz * g.sC;
+  if constexpr (KIND == KIND_GATE_RES && !EARLY)
 #pragma unroll
-    for (int it = 0; it < 8; ++it) {
-      const int row = it * 16 + r0, m = m0 + row;
-      if (m >= g.M) continue;
-      const float* sa = sC + row * LDC_S + blk * 64 + off;
-      float o[8];
+    for (int k = 0; k < PRE; ++k) fetch(k, pre[k]);
+  // partial tiles -> LDS, over the slab buffers: every wave must have finished its slabs
+  float* sC = reinterpret_cast<float*>(smem);
+  lds_barrier();
 #pragma unroll
-      for (int e = 0; e < 8; ++e) { const float a = sa[e], b = sa[32 + e]; o[e] = a * sigmoidf_(a) * b; }
-      bf16_t* dst = C + (int64_t)m * g.ldc + oc;
-      if (g.vec_ok) *reinterpret_cast<u32x4*>(dst) = pack8(o);
-      else
+  for (int x = 0; x < MT; ++x)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) dst[e] = f2bf(o[e]);
+    for (int y = 0; y < NT; ++y)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 v = {acc[x][y][4 * q], acc[x][y][4 * q + 1], acc[x][y][4 * q + 2], acc[x][y][4 * q + 3]};
+        *reinterpret_cast<f32x4*>(sC + (grp * BM + wm + 32 * x + l31) * LDS_C + wn + 32 * y + 8 * q + 4 * hh) = v;
+      }
+  lds_barrier();
+  auto gather8 = [&](int row, int c, float* v) {
+    auto part = [&](int w, int at) { return *reinterpret_cast<const f32x4*>(sC + (w * BM + row) * LDS_C + at); };
+    f32x4 lo = part(0, c), hi = part(0, c + 4);
+    if constexpr (WK >= 2) { lo += part(1, c); hi += part(1, c + 4); }
+    if constexpr (WK == 4) { lo += part(2, c) + part(3, c); hi += part(2, c + 4) + part(3, c + 4); }
+    v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+  };
+  using OutT = std::conditional_t<OUT_F32, float, bf16_t>;
+  OutT* C = reinterpret_cast<OutT*>(g.C);
+  auto put = [&](int64_t o, const float* v, int nv) {
+    if constexpr (VEC) Elem<OutT>::store8(C + o, v);
+    else
+      for (int e = 0; e < nv; ++e) Elem<OutT>::store(C + o + e, v[e]);
+  };
+
+  if constexpr (KIND == KIND_SWIGLU) {
+    static_assert(KIND != KIND_SWIGLU || BN >= 64, "");
+    // weight rows are packed in blocks of 64: 32 "a" rows then the 32 matching "b" rows; N / 2 output columns
+    constexpr int OPR = BN >= 64 ? BN / 16 : 1;  // chunks of 8 output columns per row
+#pragma unroll
+    for (int k = 0; k < (BM * OPR + NTHR - 1) / NTHR; ++k) {
+      const int idx = tid + k * NTHR;
+      const int row = idx / OPR, oc = (idx % OPR) * 8, m = m0 + row;
+      if (idx >= BM * OPR || m >= g.M || n0 + 2 * oc >= g.N) continue;
+      const int c = (oc >> 5) * 64 + (oc & 31);
+      float a[8], b[8], o[8];
+      gather8(row, c, a);
+      gather8(row, BN >= 64 ? c + 32 : c, b);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = a[e] * sigmoidf_(a[e]) * b[e];
+      put((int64_t)bz * g.sC + (int64_t)m * g.ldc + n0 / 2 + oc, o, 8);
     }
     return;
   }
-
-  const int n = n0 + cc;
-  if (n >= g.N) return;
-  const int nv = min(8, g.N - n);  // valid columns of this chunk
-  float bias[8];
-  int op = SEG_PLAIN;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) bias[e] = 0.f;
-  if (g.epi == EPI_SEGMENTED) {
-    op = (g.seg_ops >> (4 * (n / g.seg_len))) & 15;  // seg_len % 8 == 0: a chunk never straddles segments
-    if (gemm_col_uses_bias(g, n))
+  for (int k = 0; k < NCH; ++k) {
+    if (KIND == KIND_GATE_RES && k > 0 && k % PRE == 0)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) if (e < nv) bias[e] = g.bias[n + e];
-  } else if (g.bias) {
+      for (int j = 0; j < PRE; ++j) fetch(k + j, pre[j]);
+    const int idx = tid + k * NTHR;
+    const int row = idx / CPR, c = (idx % CPR) * 8;
+    const int m = m0 + row, n = n0 + c;
+    if (idx >= BM * CPR || m >= g.M || n >= g.N) continue;
+    const int nv = min(8, g.N - n);  // valid columns of this chunk
+    const Pre& p = pre[k % PRE];
+    float v[8], bias[8];
+    gather8(row, c, v);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) if (e < nv) bias[e] = g.bias[n + e];
-  }
-#pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int row = it * 16 + r0, m = m0 + row;
-    if (m >= g.M) continue;
-    float v[8];
-    const f32x4 lo = *reinterpret_cast<const f32x4*>(sC + row * LDC_S + cc);
-    const f32x4 hi = *reinterpret_cast<const f32x4*>(sC + row * LDC_S + cc + 4);
-    v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
-    const bool full = g.vec_ok && nv == 8;
-    if (g.epi == EPI_SEGMENTED) {
+    for (int e = 0; e < 8; ++e) bias[e] = 0.f;
+    if (gemm_col_uses_bias(g, n))  // seg_len % 8 == 0: a chunk never straddles segments
+    {
+      if constexpr (VEC) Elem<float>::load8(g.bias + n, bias);
+      else
+        for (int e = 0; e < nv; ++e) bias[e] = g.bias[n + e];
+    }
+    if (KIND == KIND_COLUMNS && g.epi == EPI_SEGMENTED) {
+      const int op = (g.seg_ops >> (4 * (n / g.seg_len))) & 15;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         if (op == SEG_BIAS_SCALE) v[e] = (v[e] + bias[e]) * g.alpha;
         else if (op == SEG_SIGMOID) v[e] = sigmoidf_(v[e]);
       }
-    } else if (gr_ahead) {
-      const f32x4 gl = gate_lo[it], gh = gate_hi[it];
-      const float gt[8] = {gl.x * gate_row[it], gl.y * gate_row[it], gl.z * gate_row[it], gl.w * gate_row[it],
-                           gh.x * gate_row[it], gh.y * gate_row[it], gh.z * gate_row[it], gh.w * gate_row[it]};
+    } else if (KIND == KIND_GATE_RES) {
       float rs[8];
-      unpack8(res_pk[it], rs);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = (v[e] + bias[e]) * gt[e] + rs[e];
-    } else if (g.epi == EPI_GATE_RES) {
-      const int64_t roff = (int64_t)bz * g.sRes + (int64_t)m * g.ld_res + n;
-      float gt[8], rs[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) { gt[e] = 1.f; rs[e] = 0.f; }
-      if (g.gate && g.gate_per_row) {
-        const float f = g.gate[m % g.gate_rows];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) gt[e] = f;
-      } else if (g.gate) {
-        const float* gp = g.gate + (int64_t)(m % g.gate_rows) * g.ld_gate + n;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) if (e < nv) gt[e] = gp[e];
-      }
       if (g.res_f32) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) if (e < nv) rs[e] = g.res_f32[roff + e];
-      } else if (g.res_bf16) {
-        if (full && g.res_vec_ok) unpack8(*reinterpret_cast<const u32x4*>(g.res_bf16 + roff), rs);
-        else
-#pragma unroll
-          for (int e = 0; e < 8; ++e) if (e < nv) rs[e] = bf2f(g.res_bf16[roff + e]);
+        for (int e = 0; e < 8; ++e) rs[e] = __uint_as_float(e < 4 ? p.r0[e & 3] : p.r1[e & 3]);
+      } else {
+        unpack8(p.r0, rs);
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = (v[e] + bias[e]) * gt[e] + rs[e];
+      for (int e = 0; e < 8; ++e) v[e] = (v[e] + bias[e]) * p.gate[e] + rs[e];
     } else {  // EPI_PLAIN
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -286,36 +335,43 @@ __global__ __launch_bounds__(256, 2) void gemm_nt_kernel(GemmArgs g) {
         if (g.act_sigmoid) v[e] = sigmoidf_(v[e]);
       }
     }
-    const int64_t off = g.regroup32
-                            ? ((((int64_t)(m >> 5) * (g.N >> 5) + (n >> 5)) * 32 + (m & 31)) * 32 + (n & 31))
-                            : (int64_t)bz * g.sC + (int64_t)m * g.ldc + n;
-    if (OUT_F32) {
-      float* dst = reinterpret_cast<float*>(g.C) + off;
-      if (full) {
-        *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-        *reinterpret_cast<f32x4*>(dst + 4) = f32x4{v[4], v[5], v[6], v[7]};
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) if (e < nv) dst[e] = v[e];
-      }
-    } else {
-      bf16_t* dst = reinterpret_cast<bf16_t*>(g.C) + off;
-      if (full) *reinterpret_cast<u32x4*>(dst) = pack8(v);
-      else
-#pragma unroll
-        for (int e = 0; e < 8; ++e) if (e < nv) dst[e] = f2bf(v[e]);
-    }
+    put(g.regroup32 ? ((((int64_t)(m >> 5) * (g.N >> 5) + (n >> 5)) * 32 + (m & 31)) * 32 + (n & 31))
+                    : (int64_t)bz * g.sC + (int64_t)m * g.ldc + n, v, nv);
   }
+}
+
+template <int MT, int NT, int WM, int WN, int WK, int ST, int WPS, bool GROUPS, bool VEC = true>
+int launch_tile(const GemmArgs& g, hipStream_t stream) {
+  constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN;
+  const int64_t total = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN) * g.batch;
+  const int64_t blocks = (total + 7) / 8 * 8;
+  if (blocks > 0x3fffffff) return AF3_ERR_BAD_ARG;
+  const dim3 grid((unsigned)blocks), block(64 * WM * WN * WK);
+#define LAUNCH(KIND, OUT_F32) hipLaunchKernelGGL((gemm_nt_kernel<MT, NT, WM, WN, WK, ST, WPS, GROUPS, KIND, VEC, OUT_F32>), grid, block, 0, stream, g)
+  if (g.epi == EPI_SWIGLU) {
+    if constexpr (BN >= 64) LAUNCH(KIND_SWIGLU, false);
+    else return AF3_ERR_BAD_ARG;
+  } else if (g.epi == EPI_GATE_RES) {
+    if (g.out_f32) LAUNCH(KIND_GATE_RES, true);
+    else LAUNCH(KIND_GATE_RES, false);
+  } else {
+    if (g.out_f32) LAUNCH(KIND_COLUMNS, true);
+    else LAUNCH(KIND_COLUMNS, false);
+  }
+#undef LAUNCH
+  return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
 
 }  // namespace
 
-// Products of at least 120 tiles of 256x256 go to the large-tile kernel where
-// one of its epilogues fits: from there on the 128x128 tiles no longer fit
-// the chip in one round (two workgroups per CU) and the large tile, with
-// half the fragment reads per MFMA, is 1.3 to 1.45 times faster;
-// below, the two kernels are within a few percent of each other and the
-// small tile wins where it fills more CUs.
+// How K is summed: in four groups where a short product is likely to have its K range split between waves (the
+// K loop is five slabs or longer and the columns alone do not make enough tiles), in one go otherwise.  N = 2048
+// on: the wide projections of the diffusion transformer, which large batches hand to the 256x256 tile.
+static int gemm_k_groups(const GemmArgs& g) { return g.K > 256 && g.N < 2048 ? 4 : 1; }
+
+// Products of at least 120 tiles of 256x256 go to the large-tile kernel where one of its epilogues fits: a
+// 128x128 tile of the kernel above needs twice the fragment reads per MFMA and is bound by them from there on
+// (3840x3072x768: 34 us against 25; 1920x3072x768, 96 such tiles: 17 against 23 the other way).
 int gemm_big_tile_choice(const GemmArgs& g) {
   constexpr int64_t BIG_TILE_MIN_TILES = 120;
   const int64_t tiles = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256) * g.batch;
@@ -331,6 +387,8 @@ int launch_gemm_nt(const GemmArgs& g_in, hipStream_t stream) {
   }
   if ((g.K & 7) || (g.lda & 7) || (g.ldb & 7) || (g.sA & 7) || (g.sB & 7)) return AF3_ERR_BAD_ARG;
   if (((uintptr_t)g.A & 15) || ((uintptr_t)g.B & 15)) return AF3_ERR_BAD_ARG;
+  if (g.K > g.lda || g.K > g.ldb) return AF3_ERR_BAD_ARG;
+  if (g.lda >= (1ll << 23) || g.ldb >= (1ll << 23)) return AF3_ERR_BAD_ARG;  // 32-bit byte offsets inside a tile
   if (g.epi == EPI_SWIGLU && ((g.N & 63) || g.out_f32)) return AF3_ERR_BAD_ARG;
   if (g.epi == EPI_SEGMENTED && (g.seg_len <= 0 || (g.seg_len & 7))) return AF3_ERR_BAD_ARG;
   if (g.gate && g.gate_rows <= 0) return AF3_ERR_BAD_ARG;
@@ -340,19 +398,33 @@ int launch_gemm_nt(const GemmArgs& g_in, hipStream_t stream) {
     if (first < 0 || last > g.bias_len) return AF3_ERR_BAD_ARG;
   }
   if (g.regroup32 && (g.epi != EPI_PLAIN || g.batch != 1 || (g.M & 31) || (g.N & 31))) return AF3_ERR_BAD_ARG;
-  // 16/32-byte stores need aligned rows; otherwise the epilogue stores element-wise
+  // 16-byte stores and loads need aligned rows and whole chunks of 8 columns (a plain bf16 result may have the rest
+  // of its last chunk in row padding, which nobody reads)
   const int esz = g.out_f32 ? 4 : 2;
-  g.vec_ok = ((uintptr_t)g.C % 16 == 0) && ((g.ldc * esz) % 16 == 0) && ((g.sC * esz) % 16 == 0);
-  g.gate_vec_ok = g.gate && !g.gate_per_row && ((uintptr_t)g.gate % 16 == 0) && (g.ld_gate % 4 == 0);
-  g.res_vec_ok = g.res_bf16 && ((uintptr_t)g.res_bf16 % 16 == 0) && (g.ld_res % 8 == 0) && (g.sRes % 8 == 0);
-  const int64_t total = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN) * g.batch;
-  const int64_t blocks = (total + 7) / 8 * 8;
-  if (blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
-  dim3 grid((unsigned)blocks);
-  const bool k_tail = (g.K % BK) != 0;
-  if (g.out_f32 && k_tail) hipLaunchKernelGGL((gemm_nt_kernel<true, true>), grid, dim3(256), 0, stream, g);
-  else if (g.out_f32) hipLaunchKernelGGL((gemm_nt_kernel<true, false>), grid, dim3(256), 0, stream, g);
-  else if (k_tail) hipLaunchKernelGGL((gemm_nt_kernel<false, true>), grid, dim3(256), 0, stream, g);
-  else hipLaunchKernelGGL((gemm_nt_kernel<false, false>), grid, dim3(256), 0, stream, g);
-  return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+  auto al = [](const void* p, int64_t bytes0, int64_t bytes1) { return !p || ((uintptr_t)p % 16 == 0 && bytes0 % 16 == 0 && bytes1 % 16 == 0); };
+  const bool whole = (g.N & 7) == 0;
+  const bool padded = g.epi == EPI_PLAIN && !g.bias && !g.out_f32 && g.ldc >= ((g.N + 7) & ~7);
+  const bool vec = (whole || padded) && al(g.C, g.ldc * esz, g.sC * esz) && al(g.bias, 0, 0) &&
+                   (g.gate_per_row || al(g.gate, g.ld_gate * 4, 0)) && al(g.res_f32, g.ld_res * 4, g.sRes * 4) &&
+                   al(g.res_bf16, g.ld_res * 2, g.sRes * 2);
+
+  // The tile, by the number T of 64x64 tiles (256 CUs; measured over M = 64 ... 92160, N = 128 ... 73728,
+  // K = 64 ... 1536):
+  //   T <= 128  32x32 tiles, K split four ways: the 64x64 tiles would leave half of the CUs without one
+  //   T <= 384  64x64 with K split two ways (eight waves per tile)
+  //   T <= 1000 64x64, two to three workgroups per CU
+  //   T <= 2600 64x128, else 128x128: bytes per FLOP count once every CU has several tiles (and never wider than N)
+  // (a split tile only where K is summed in groups; SwiGLU pairs 32-column blocks, so its tiles are 64 columns or more)
+  const bool groups = gemm_k_groups(g) == 4;
+  const int64_t T = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch;
+  if (!vec) return groups ? launch_tile<1, 1, 2, 2, 1, 2, 4, true, false>(g, stream) : launch_tile<1, 1, 2, 2, 1, 2, 4, false, false>(g, stream);
+  if (groups) {
+    if (T <= 128 && g.epi != EPI_SWIGLU) return launch_tile<1, 1, 1, 1, 4, 2, 2, true>(g, stream);
+    if (T <= 384) return launch_tile<1, 1, 2, 2, 2, 2, 4, true>(g, stream);
+    if (T <= 1000 || g.N <= 64) return launch_tile<1, 1, 2, 2, 1, 2, 4, true>(g, stream);
+    return launch_tile<1, 2, 2, 2, 1, 2, 3, true>(g, stream);
+  }
+  if (T <= 1000 || g.N <= 64) return launch_tile<1, 1, 2, 2, 1, 2, 4, false>(g, stream);
+  if (T <= 2600 || g.N <= 128) return launch_tile<1, 2, 2, 2, 1, 2, 3, false>(g, stream);
+  return launch_tile<2, 2, 2, 2, 1, 2, 2, false>(g, stream);
 }

@@ -27,7 +27,6 @@ struct GemmArgs {
   const float* res_f32 = nullptr;   // GATE_RES: residual added last (either dtype)
   const bf16_t* res_bf16 = nullptr;
   int64_t ld_res = 0, sRes = 0;
-  int vec_ok = 0, res_vec_ok = 0, gate_vec_ok = 0;  // set by launch_gemm_nt: rows aligned for 16-byte stores / loads
   // regroup32 (PLAIN, batch 1, M and N multiples of 32): element (m, n) is stored
   // at [(m / 32, n / 32)][(m % 32, n % 32)], i.e. C is [(M/32)(N/32)][1024]:
   // the outer products of 32-channel rows, one contiguous 1024-vector per pair.
@@ -60,7 +59,7 @@ int launch_contract(const GemmArgs& g, hipStream_t stream);
 // kernel instance that can take `g`, or -1
 int big_tile_mode(const GemmArgs& g);
 int launch_big_tile(const GemmArgs& g, int mode, hipStream_t stream);
-// the large-tile instance launch_gemm_nt hands `g` to, or -1: the 128x128-tile kernel
+// the large-tile instance launch_gemm_nt hands `g` to, or -1: the kernel of gemm.hip
 int gemm_big_tile_choice(const GemmArgs& g);
 
 // ---------------------------------------------------------------- rowops.hip

@@ -484,7 +484,7 @@ int af3_pair_cond_init_forward(const void* pair, int pair_dtype, float in_scale,
 
 /* ---------------------------------------------------------------------------
  * Diagnostic, no counterpart in the reference.  The dense kernels fetch a
- * column bias in groups (eight entries on the 128x128 tile, four per lane on the
+ * column bias in groups (eight entries on the smaller tiles, four per lane on the
  * 256x256 tile, the last group pulled back to end at column n), and a segmented
  * epilogue (the q-k-v-gate projection of the attentions: segments of seg_len
  * columns, op of segment s in bits [4s, 4s+4) of seg_ops, 1 = biased and

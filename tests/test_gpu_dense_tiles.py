@@ -1,0 +1,74 @@
+"""GPU parity of the dense products below the 256x256-tile sizes, one case at the edges of every tile the launcher
+chooses from (32x32 with the K range split by four, 64x64 split by two and not, 64x128, 128x128, the element-wise form): first and last rows
+and columns alone in a tile, K shorter than a slab, K with a partial last slab, column counts that force element-wise
+stores; and the order of summation, which must not depend on the number of rows."""
+
+import pytest
+import torch
+
+from oracle import af3_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    (1, 8, 264), (33, 40, 312), (64, 384, 384), (97, 72, 1032), (161, 384, 1536),    # 32x32, K split by four
+    (387, 1536, 384), (1921, 768, 776), (130, 1984, 264),                             # 64x64, by two
+    (1, 8, 8), (12001, 136, 128), (3841, 768, 768), (129, 3072, 384), (70001, 64, 264),   # 64x64
+    (31, 3, 64), (97, 65, 200), (500, 765, 392),                                      # 64x64, element by element
+    (1921, 3080, 136), (8001, 384, 1032), (70, 70000, 72), (180001, 128, 40),         # 64x128
+    (20001, 1032, 104),                      # 128x128 (odd columns keep it off the large tile)
+]
+
+
+def ulp_ok(name, got, want, atol=2e-4):
+    got, want = got.double().cpu(), want.double().cpu()
+    bad = (got - want).abs() > 1.01 * 2.0 ** -8 * want.abs() + atol
+    assert not bad.any(), f"{name}: {int(bad.sum())} elements beyond one bf16 ulp"
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_epilogues(gpu_pkg, m, n, k):
+    print(f"dense tiles m={m} n={n} k={k}", flush=True)
+    ops, L = gpu_pkg.ops, gpu_pkg.lib
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, w, b = rnd(m, k).bfloat16(), (rnd(n, k) * 0.1).bfloat16(), rnd(n)
+    y = x.float() @ w.float().t()
+    ulp_ok("fp32, bias, scale", ops.linear(x, w, bias=b, alpha=0.5, out_dtype=torch.float32), (y + b) * 0.5)
+    ulp_ok("sigmoid", ops.linear(x, w, bias=b, sigmoid=True), torch.sigmoid(y + b))
+    gate = torch.rand(1 if m % 7 else 7, n, generator=g, device="cuda")
+    rows = gate.repeat(m // gate.shape[0], 1)
+    for dt in (torch.bfloat16, torch.float32):
+        res = rnd(m, n).to(dt)
+        want = y * rows + res.float()
+        out = ops.linear(x, w, out_dtype=dt, mode=L.LINEAR_GATE_RES, gate=gate, residual=res, out=res)
+        assert out is res
+        ulp_ok(f"gate, residual in place {dt}", out, want)
+    if n % 64 == 0:
+        h = ops.linear(x, w, mode=L.LINEAR_SWIGLU)
+        a, c = y.view(m, n // 64, 2, 32).unbind(2)
+        ulp_ok("swiglu", h, (torch.nn.functional.silu(a) * c).reshape(m, n // 2))
+    if m % 32 == 0 and n % 32 == 0:
+        r = ops.linear(x, w, mode=L.LINEAR_REGROUP32)
+        ulp_ok("regrouped", r, y.view(m // 32, 32, n // 32, 32).transpose(1, 2).reshape(-1, 1024))
+
+
+@pytest.mark.parametrize("batch,m,n,k", [(128, 64, 64, 64), (128, 61, 61, 64), (3, 130, 24, 72), (8, 100, 300, 104)])
+def test_batched_product(gpu_pkg, batch, m, n, k):
+    print(f"dense tiles batch={batch} m={m} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(m)
+    a, b = (O.round_bf16(torch.randn(batch, s, k, generator=g)) for s in (m, n))
+    got = gpu_pkg.ops.batched_nt_product(a.cuda().bfloat16(), b.cuda().bfloat16())
+    ulp_ok("batched", got, torch.stack([p.double() @ q.double().t() for p, q in zip(a, b)]))
+
+
+@pytest.mark.parametrize("n,k", [(768, 768), (384, 1536), (128, 128), (3072, 768)])
+def test_rows_do_not_change_with_the_batch(gpu_pkg, n, k):
+    """Every tile sums K in the same order, so the first rows of a product are the same bits however many follow."""
+    print(f"dense tiles: batch invariance n={n} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(9000, k, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(n, k, generator=g, device="cuda") * 0.1).bfloat16()
+    want = gpu_pkg.ops.linear(x, w, mode=gpu_pkg.lib.LINEAR_GATE_RES)
+    for m in (1, 100, 500, 1900, 3840):
+        assert torch.equal(gpu_pkg.ops.linear(x[:m], w, mode=gpu_pkg.lib.LINEAR_GATE_RES), want[:m]), m
