@@ -14,6 +14,18 @@ LINEAR_PLAIN, LINEAR_SWIGLU, LINEAR_GATE_RES, LINEAR_REGROUP32, LINEAR_ROWGATE_R
 
 _vp, _i, _i64, _sz, _f = C.c_void_p, C.c_int, C.c_int64, C.c_size_t, C.c_float
 
+
+class PairformerBlockStruct(C.Structure):
+    """af3_pairformer_block."""
+    _fields_ = (
+        [(k, _vp * 2) for k in ("tm_ln_in_w", "tm_ln_in_b", "tm_ln_c_w", "tm_ln_c_b", "tm_w_proj_gate", "tm_w_out",
+                                "tm_w_gating", "ta_ln_w", "ta_ln_b", "ta_w_bias", "ta_w_qkvg", "ta_w_out")]
+        + [(k, _vp) for k in ("pt_ln_w", "pt_ln_b", "pt_w1", "pt_w2", "sl_ln_w", "sl_ln_b", "sl_w", "sa_ln_w", "sa_ln_b",
+                              "sa_w_qkvg", "sa_q_b", "sa_w_out", "st_ln_w", "st_ln_b", "st_w1", "st_w2")]
+        + [(k, C.c_int32) for k in ("valid_channels", "num_head_pair", "pair_hidden", "with_single", "num_head",
+                                    "c_single", "single_hidden")])
+
+
 # name -> (restype, argtypes); must list every symbol include/af3_hip.h declares
 SIGNATURES = {
     "af3_abi_version": (_i, []),
@@ -59,6 +71,10 @@ SIGNATURES = {
                                         _i64, _i64, _i64, _vp]),
     "af3_atom_pair_logits_forward": (_i, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _i, _vp]),
     "af3_pair_cond_init_forward": (_i, [_vp, _i, _f, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
+    "af3_pairformer_stack_workspace_bytes": (_sz, [_i64, _i]),
+    "af3_pairformer_single_workspace_bytes": (_sz, [_i64, _i, _i]),
+    "af3_pairformer_stack_forward": (
+        _i, [_vp, _i, _vp, _i, _vp, _vp, _vp, _i, _vp, _i64, _vp, _vp, _sz, _vp, _sz, _vp, _vp, _i]),
     "af3_linear_bias_span": (_i, [_i64, _i, _i, _i, _i, _vp, _vp]),
     "af3_grid_attention_core_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "af3_check_gemm_f32": (

@@ -8,6 +8,7 @@ import torch
 import torch.nn as nn
 
 from .. import check, ops
+from .. import lib as L
 from .attention import GridSelfAttention
 from .base import HipModule, bf16, drop_mesh, f32, in_check_mode, pad_channels, pad_rows
 from .diffusion_transformer import SelfAttention
@@ -33,6 +34,7 @@ class PairformerBlock(HipModule):
         n_heads, c_pair, c_single, c_hidden_mul, n_heads_pair, num_intermediate_factor, with_single = vals[:7]
         self.n_heads, self.c_pair, self.c_single = n_heads, c_pair, c_single
         self.with_single, self.num_intermediate_factor = with_single, num_intermediate_factor
+        self._native = None
         self.triangle_multiplication_outgoing = TriangleMultiplication(c_pair=c_pair, _outgoing=True)
         self.triangle_multiplication_incoming = TriangleMultiplication(c_pair=c_pair, _outgoing=False)
         self.pair_attention1 = GridSelfAttention(c_pair=c_pair, num_head=n_heads_pair, transpose=False)
@@ -51,6 +53,51 @@ class PairformerBlock(HipModule):
         return dict(ln_w=f32(self.single_pair_logits_norm.weight), ln_b=f32(self.single_pair_logits_norm.bias),
                     w_logits=pad_rows(bf16(self.single_pair_logits_projection.weight), 32))
 
+    @property
+    def one_call(self) -> bool:
+        """Whether the whole block runs as one call of the library (`native`): the fused pair operators, and a
+        single track wide enough for the unfused transition."""
+        return ((self.pair_attention1.fused or (self.pair_attention1.padded and not self.with_single))
+                and (not self.with_single or self.c_single > 128))
+
+    def native(self) -> "L.PairformerBlockStruct":
+        """The packed weights of the block's modules as the library's structure; made again when any of them has
+        been packed again."""
+        tm = (self.triangle_multiplication_outgoing, self.triangle_multiplication_incoming)
+        ta = (self.pair_attention1, self.pair_attention2)
+        mods = (self, *tm, *ta, self.pair_transition)
+        if self.with_single:
+            sa, st = self.single_attention_, self.single_transition
+            mods += (sa, sa.adaptive_layernorm, sa.adaptive_zero_init, st)
+        packs = [m.packed() for m in mods]
+        if self._native is not None and all(a is b for a, b in zip(self._native[1], packs)):
+            return self._native[0]
+        by = dict(zip(mods, packs))
+        s = L.PairformerBlockStruct()
+        for d in (0, 1):
+            p, q = by[tm[d]], by[ta[d]]
+            for name, t in (("tm_ln_in_w", p["ln_in_w"]), ("tm_ln_in_b", p["ln_in_b"]), ("tm_ln_c_w", p["ln_c_w"]),
+                            ("tm_ln_c_b", p["ln_c_b"]), ("tm_w_proj_gate", p["w_proj_gate"]), ("tm_w_out", p["w_out"]),
+                            ("tm_w_gating", p["w_gl"]), ("ta_ln_w", q["ln_w"]), ("ta_ln_b", q["ln_b"]),
+                            ("ta_w_bias", q["w_bias"]), ("ta_w_qkvg", q["w_qkvg"]), ("ta_w_out", q["w_out"])):
+                getattr(s, name)[d] = t.data_ptr()
+        p = by[self.pair_transition]
+        s.pt_ln_w, s.pt_ln_b, s.pt_w1, s.pt_w2 = (p[k].data_ptr() for k in ("ln_w", "ln_b", "w1", "w2"))
+        s.valid_channels, s.num_head_pair, s.pair_hidden = self.c_pair, ta[0].num_head, p["w2"].shape[1]
+        s.with_single = int(self.with_single)
+        if self.with_single:
+            p = by[self]
+            s.sl_ln_w, s.sl_ln_b, s.sl_w = (p[k].data_ptr() for k in ("ln_w", "ln_b", "w_logits"))
+            p = by[sa.adaptive_layernorm]
+            s.sa_ln_w, s.sa_ln_b = p["ln_w"].data_ptr(), p["ln_b"].data_ptr()
+            s.sa_w_qkvg, s.sa_q_b = by[sa]["w_qkvg"].data_ptr(), by[sa]["q_b"].data_ptr()
+            s.sa_w_out = by[sa.adaptive_zero_init]["w"].data_ptr()
+            p = by[st]
+            s.st_ln_w, s.st_ln_b, s.st_w1, s.st_w2 = (p[k].data_ptr() for k in ("ln_w", "ln_b", "w1", "w2"))
+            s.num_head, s.c_single, s.single_hidden = self.n_heads, self.c_single, p["w2"].shape[1]
+        self._native = (s, packs)
+        return s
+
     def forward(self, pair: torch.Tensor, pair_mask: torch.Tensor, single: Optional[torch.Tensor] = None,
                 seq_mask: Optional[torch.Tensor] = None, head: int = 0,
                 single_stream: Optional["torch.cuda.Stream"] = None):
@@ -65,16 +112,19 @@ class PairformerBlock(HipModule):
             return check.pairformer_block(self, pair, pair_mask, single, seq_mask)
         if not pair.is_contiguous():
             raise ValueError("pair must be contiguous (it is updated in place)")
-        if self.c_pair < 128 and not self.with_single and self.pair_attention1.padded:
-            # the 64-channel block of the template embedding (nn/d_template.py:198-201): the five operators run
-            # on the 128-channel kernels over one zero-padded copy of the tensor, which stays padded in between
-            x = pad_channels(pair)
-            self.triangle_multiplication_outgoing.run_padded(x, pair_mask, residual=True)
-            self.triangle_multiplication_incoming.run_padded(x, pair_mask, residual=True)
-            self.pair_attention1.run_padded(x, pair_mask, residual=True)
-            self.pair_attention2.run_padded(x, pair_mask, residual=True)
-            self.pair_transition.run_padded(x, residual=True)
-            pair.copy_(x[..., :self.c_pair])
+        if self.with_single and not single.is_contiguous():
+            raise ValueError("single must be contiguous (it is updated in place)")
+        if self.one_call and self.with_single:
+            ops.pairformer_stack([self.native()], pair, pair_mask, single, seq_mask, single_stream=single_stream,
+                                 join=single_stream is None)
+            return pair, single
+        if self.one_call:
+            # (fewer than 128 channels, the template embedding of nn/d_template.py:198-201: the five operators run on
+            # the 128-channel kernels over one zero-padded copy of the tensor, which stays padded in between)
+            x = pad_channels(pair) if self.c_pair < 128 else pair
+            ops.pairformer_stack([self.native()], x, pair_mask, None, None)
+            if x is not pair:
+                pair.copy_(x[..., :self.c_pair])
             return pair
         self.triangle_multiplication_outgoing.run(pair, pair_mask, residual=True)
         self.triangle_multiplication_incoming.run(pair, pair_mask, residual=True)
@@ -83,8 +133,6 @@ class PairformerBlock(HipModule):
         self.pair_transition.run(pair, residual=True)
         if not self.with_single:
             return pair
-        if not single.is_contiguous():
-            raise ValueError("single must be contiguous (it is updated in place)")
         p = self.packed()
         # the only reader of `pair` on the single path: it stays on the caller's stream, in front of
         # whatever updates `pair` next
@@ -124,8 +172,15 @@ def pairformer_loop(blocks, pair, pair_mask, single, seq_mask, overlap_single: b
         for blk in blocks:
             pair, single = blk(pair, pair_mask, single, seq_mask)
         return pair, single
-    main = torch.cuda.current_stream(pair.device)
     side = _side_stream(pair.device)
+    blocks = list(blocks)
+    if blocks and all(type(b) is PairformerBlock and b.one_call and b.with_single and b.n_heads == blocks[0].n_heads
+                      and b.c_single == blocks[0].c_single for b in blocks):
+        if not (pair.is_contiguous() and single.is_contiguous()):
+            raise ValueError("pair and single must be contiguous (they are updated in place)")
+        ops.pairformer_stack([b.native() for b in blocks], pair, pair_mask, single, seq_mask, single_stream=side)
+        return pair, single
+    main = torch.cuda.current_stream(pair.device)
     side.wait_stream(main)          # whatever produced `single` and `seq_mask`
     for blk in blocks:
         pair, single = blk(pair, pair_mask, single, seq_mask, single_stream=side)

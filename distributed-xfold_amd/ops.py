@@ -10,6 +10,7 @@ non-zero return code into a RuntimeError.  No arithmetic happens here.
 
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
@@ -19,10 +20,14 @@ from . import lib as _L
 _workspaces: dict = {}
 
 
-def _ws(nbytes: int, device) -> torch.Tensor:
+def _ws(nbytes: int, device, stream=None) -> torch.Tensor:
     """Scratch buffer per device and stream, grown on demand and reused between
     calls (calls on one stream are ordered, so reuse is safe; calls on different
-    streams may run at the same time and get different buffers)."""
+    streams may run at the same time and get different buffers).  `stream`: a
+    torch stream other than the current one that the scratch is used on."""
+    if stream is not None:
+        with torch.cuda.stream(stream):
+            return _ws(nbytes, device)
     key = (device.type, device.index, torch.cuda.current_stream(device).cuda_stream)
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
@@ -191,6 +196,40 @@ def transition128(act, layernorm_weight, layernorm_bias, w1_packed, w2, residual
                                     _stream(act.device))
     _L.check(rc, "af3_transition_forward")
     return out
+
+
+def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incoming=None, single_stream=None, join=True):
+    """A run of Pairformer blocks in one call (af3_pairformer_stack_forward), pair [N, N, 128] and single [N, c]
+    updated in place.  `blocks`: af3_pairformer_block structures (nn.PairformerBlock.native()); `single_stream`: a
+    torch stream for the single updates, see the entry point."""
+    lib = _L.load()
+    _gpu(pair, "pair")
+    if pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair.shape[2] != 128:
+        raise ValueError(f"pair: expected [N, N, 128], got {tuple(pair.shape)}")
+    n, dev = pair.shape[0], pair.device
+    io = _dt(pair)
+    maskf = _mask_f32(pair_mask, (n, n), "mask")
+    mask_in = _mask_f32(pair_mask_incoming, (n, n), "mask")
+    ws = _ws(lib.af3_pairformer_stack_workspace_bytes(n, blocks[0].num_head_pair), dev)
+    seqf = logits = sws = None
+    single_dt = 0
+    if blocks[0].with_single:
+        b = blocks[0]
+        _gpu(single, "single", shape=(n, b.c_single))
+        single_dt = _dt(single)
+        seqf = _mask_f32(seq_mask, (n,), "key_mask")
+        logits = torch.empty((min(len(blocks), 2), b.num_head, n, n), dtype=torch.float32, device=dev)
+        sws = _ws(lib.af3_pairformer_single_workspace_bytes(n, b.c_single, b.single_hidden), dev, single_stream)
+        if single_stream is not None and not join:
+            for t in (logits, seqf):
+                if t is not None:
+                    t.record_stream(single_stream)
+    ptrs = (ctypes.c_void_p * len(blocks))(*[ctypes.addressof(b) for b in blocks])
+    rc = lib.af3_pairformer_stack_forward(
+        ptrs, len(blocks), _p(pair), io, _p(maskf), _p(mask_in), _p(single) if logits is not None else None,
+        single_dt, _p(seqf), n, _p(logits), _p(ws), ws.numel(), _p(sws), 0 if sws is None else sws.numel(), _stream(dev),
+        None if single_stream is None else single_stream.cuda_stream, int(bool(join)))
+    _L.check(rc, "af3_pairformer_stack_forward")
 
 
 def batch_diffusion_self_attention(q_data, key_mask, nonbatched_bias, w_qkvg, query_b, num_head,

@@ -483,6 +483,59 @@ int af3_pair_cond_init_forward(const void* pair, int pair_dtype, float in_scale,
                                af3_stream_t stream);
 
 /* ---------------------------------------------------------------------------
+ * A run of Pairformer blocks (nn/d_pairformer.py:99-171, the loop of
+ * d_alphafold3.py:242-244) as ONE call: every launch of every block is enqueued
+ * from here.  A block is some twenty launches of a few microseconds each on short
+ * sequences; a caller that makes them one by one from an interpreter is what
+ * sets the pace there.
+ *
+ * af3_pairformer_block: the packed weights of one block, each array in the layout
+ * of the entry point named beside it.
+ * pair [n,n,128] (zero-padded when valid_channels < 128) and single [n,c_single]
+ * are updated in place.  pair_mask [n,n] or NULL; pair_mask_incoming, when not
+ * NULL, replaces it for the incoming triangle multiplication (the Evoformer block
+ * transposes it, nn/d_pairformer.py:217); seq_mask [n] or NULL.
+ * with_single = 0 in a block leaves `single` alone.
+ * single_stream: NULL, or a second stream on which the updates of `single` run
+ * beside the pair operators of the next block (they meet only in the pair
+ * logits).  The call makes single_stream wait for what `stream` holds on entry,
+ * and with join != 0 makes `stream` wait for single_stream at the end; with
+ * join = 0 the caller does that before anything else touches `single` or the
+ * scratch.  logits: 2 * num_head * n * n floats (one block: half of it), used on
+ * both streams; single_workspace is used on single_stream only.
+ */
+typedef struct af3_pairformer_block {
+  /* af3_triangle_multiplication_forward: [0] outgoing, [1] incoming */
+  const float *tm_ln_in_w[2], *tm_ln_in_b[2], *tm_ln_c_w[2], *tm_ln_c_b[2];
+  const uint16_t *tm_w_proj_gate[2], *tm_w_out[2], *tm_w_gating[2];
+  /* af3_grid_self_attn_forward: [0] starting node, [1] ending node */
+  const float *ta_ln_w[2], *ta_ln_b[2];
+  const uint16_t *ta_w_bias[2], *ta_w_qkvg[2], *ta_w_out[2];
+  /* af3_transition_forward */
+  const float *pt_ln_w, *pt_ln_b;
+  const uint16_t *pt_w1, *pt_w2;
+  /* single track: af3_pair_logits_forward; LayerNorm, af3_batch_diffusion_self_attention_forward, output
+   * projection; LayerNorm, SwiGLU and second layer as af3_linear_forward takes them */
+  const float *sl_ln_w, *sl_ln_b;
+  const uint16_t* sl_w;
+  const float *sa_ln_w, *sa_ln_b;
+  const uint16_t* sa_w_qkvg;
+  const float* sa_q_b;
+  const uint16_t* sa_w_out;
+  const float *st_ln_w, *st_ln_b;
+  const uint16_t *st_w1, *st_w2;
+  int32_t valid_channels, num_head_pair, pair_hidden; /* pair_hidden: hidden units of the pair transition */
+  int32_t with_single, num_head, c_single, single_hidden;
+} af3_pairformer_block;
+size_t af3_pairformer_stack_workspace_bytes(int64_t n_token, int num_head_pair);
+size_t af3_pairformer_single_workspace_bytes(int64_t n_token, int c_single, int single_hidden);
+int af3_pairformer_stack_forward(
+    const af3_pairformer_block* const* blocks, int num_blocks, void* pair, int pair_dtype,
+    const float* pair_mask, const float* pair_mask_incoming, void* single, int single_dtype, const float* seq_mask,
+    int64_t n_token, float* logits, void* workspace, size_t workspace_bytes,
+    void* single_workspace, size_t single_workspace_bytes, af3_stream_t stream, af3_stream_t single_stream, int join);
+
+/* ---------------------------------------------------------------------------
  * Diagnostic, no counterpart in the reference.  The dense kernels fetch a
  * column bias in groups (eight entries on the smaller tiles, four per lane on the
  * 256x256 tile, the last group pulled back to end at column n), and a segmented
