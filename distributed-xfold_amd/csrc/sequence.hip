@@ -130,4 +130,89 @@ int af3_pairformer_stack_forward(
   return rc;
 }
 
+size_t af3_diffusion_transformer_workspace_bytes(int64_t batch, int64_t seq, int channels, int hidden) {
+  if (batch <= 0 || seq <= 0 || channels <= 0 || hidden <= 0) return 0;
+  const size_t rows = (size_t)batch * seq;
+  return align_up(rows * channels * 2) + align_up(rows * (channels > hidden ? channels : hidden) * 2) +
+         align_up(af3_batch_diffusion_self_attention_workspace_bytes(batch, seq, channels));
+}
+
+int af3_diffusion_transformer_forward(
+    const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t batch, int64_t seq, int channels,
+    int hidden, int num_head, const float* key_mask, const float* const* pair_logits, int bias_quad_major,
+    const float* scale_shift, const float* gate, int64_t cond_rows, void* workspace, size_t workspace_bytes,
+    af3_stream_t stream) {
+  if (!blocks || num_blocks <= 0 || !act || !pair_logits || !scale_shift || !gate || cond_rows <= 0 || batch <= 0 || seq <= 0 ||
+      channels <= 0 || hidden <= 0)
+    return AF3_ERR_BAD_ARG;
+  const int c = channels;
+  const int64_t rows = batch * seq, ld_ss = (int64_t)2 * num_blocks * 2 * c, ld_g = (int64_t)2 * num_blocks * c;
+  Carver w(workspace, workspace_bytes);
+  uint16_t* x = static_cast<uint16_t*>(w.take((size_t)rows * c * 2));
+  uint16_t* y = static_cast<uint16_t*>(w.take((size_t)rows * (c > hidden ? c : hidden) * 2));
+  const size_t ab = af3_batch_diffusion_self_attention_workspace_bytes(batch, seq, c);
+  void* aw = w.take(ab);
+  if (!w.ok) return AF3_ERR_WORKSPACE;
+  for (int i = 0; i < num_blocks; ++i) {
+    const af3_diffusion_block& b = blocks[i];
+    const float *ss = scale_shift + (int64_t)2 * i * 2 * c, *g = gate + (int64_t)2 * i * c;
+    STEP(af3_layer_norm_forward(act, act_dtype, x, rows, c, nullptr, nullptr, ss, ss + c, cond_rows, ld_ss, stream));
+    STEP(af3_batch_diffusion_self_attention_forward(x, key_mask, 1, pair_logits[i], bias_quad_major, b.w_q, b.q_b, num_head, y,
+                                                    AF3_BF16, batch, seq, c, aw, ab, stream));
+    STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, cond_rows, ld_g, act,
+                            act_dtype, stream));
+    STEP(af3_layer_norm_forward(act, act_dtype, x, rows, c, nullptr, nullptr, ss + 2 * c, ss + 3 * c, cond_rows, ld_ss, stream));
+    STEP(af3_linear_forward(x, b.w_tr1, nullptr, y, AF3_BF16, rows, 2 * hidden, c, AF3_LINEAR_SWIGLU, 1.f, 0, nullptr, 0, 0, nullptr, 0,
+                            stream));
+    STEP(af3_linear_forward(y, b.w_tr2, nullptr, act, act_dtype, rows, c, hidden, AF3_LINEAR_GATE_RES, 1.f, 0, g + c, cond_rows, ld_g,
+                            act, act_dtype, stream));
+  }
+  return AF3_OK;
+}
+
+size_t af3_atom_transformer_workspace_bytes(int64_t samples, int64_t subsets, int64_t queries, int channels, int hidden) {
+  if (samples <= 0 || subsets <= 0 || queries <= 0 || channels <= 0 || hidden <= 0) return 0;
+  const size_t rows = (size_t)samples * subsets * queries;
+  return 2 * align_up(rows * channels * 2) + align_up(rows * (channels > hidden ? channels : hidden) * 2) +
+         align_up(af3_gathered_cross_attention_workspace_bytes(samples * subsets, queries, samples, subsets * queries, channels));
+}
+
+int af3_atom_transformer_forward(
+    const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t samples, int64_t subsets,
+    int64_t queries, int64_t keys, int channels, int hidden, int num_head, const int32_t* key_rows, const float* mask_q,
+    const float* mask_k, const float* pair_logits, const float* scale_shift_q, const float* scale_shift_k, const float* gate,
+    void* workspace, size_t workspace_bytes, af3_stream_t stream) {
+  if (!blocks || num_blocks <= 0 || !act || !key_rows || !scale_shift_q || !scale_shift_k || !gate || samples <= 0 ||
+      subsets <= 0 || queries <= 0 || keys <= 0 || channels <= 0 || hidden <= 0 || num_head <= 0)
+    return AF3_ERR_BAD_ARG;
+  const int c = channels;
+  const int64_t atoms = subsets * queries, rows = samples * atoms;
+  const int64_t ld_q = (int64_t)2 * num_blocks * 2 * c, ld_k = (int64_t)num_blocks * 2 * c;
+  Carver w(workspace, workspace_bytes);
+  uint16_t* xq = static_cast<uint16_t*>(w.take((size_t)rows * c * 2));
+  uint16_t* xk = static_cast<uint16_t*>(w.take((size_t)rows * c * 2));
+  uint16_t* y = static_cast<uint16_t*>(w.take((size_t)rows * (c > hidden ? c : hidden) * 2));
+  const size_t ab = af3_gathered_cross_attention_workspace_bytes(samples * subsets, queries, samples, atoms, c);
+  void* aw = w.take(ab);
+  if (!w.ok) return AF3_ERR_WORKSPACE;
+  for (int i = 0; i < num_blocks; ++i) {
+    const af3_diffusion_block& b = blocks[i];
+    const float *ss = scale_shift_q + (int64_t)2 * i * 2 * c, *sk = scale_shift_k + (int64_t)i * 2 * c;
+    const float* g = gate + (int64_t)2 * i * atoms * c;
+    const float* pl = pair_logits ? pair_logits + (int64_t)i * subsets * num_head * queries * keys : nullptr;
+    STEP(af3_layer_norm_forward(act, act_dtype, xq, rows, c, nullptr, nullptr, ss, ss + c, atoms, ld_q, stream));
+    STEP(af3_layer_norm_forward(act, act_dtype, xk, rows, c, nullptr, nullptr, sk, sk + c, atoms, ld_k, stream));
+    STEP(af3_gathered_cross_attention_forward(xq, xk, key_rows, pl, mask_q, mask_k, subsets, b.w_q, b.w_kv, b.q_b, num_head, y,
+                                              AF3_BF16, samples * subsets, queries, keys, samples, atoms, c, aw, ab, stream));
+    STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, atoms, 0, act, act_dtype,
+                            stream));
+    STEP(af3_layer_norm_forward(act, act_dtype, xq, rows, c, nullptr, nullptr, ss + 2 * c, ss + 3 * c, atoms, ld_q, stream));
+    STEP(af3_linear_forward(xq, b.w_tr1, nullptr, y, AF3_BF16, rows, 2 * hidden, c, AF3_LINEAR_SWIGLU, 1.f, 0, nullptr, 0, 0, nullptr,
+                            0, stream));
+    STEP(af3_linear_forward(y, b.w_tr2, nullptr, act, act_dtype, rows, c, hidden, AF3_LINEAR_GATE_RES, 1.f, 0, g + atoms * c, atoms, 0,
+                            act, act_dtype, stream));
+  }
+  return AF3_OK;
+}
+
 }  // extern "C"

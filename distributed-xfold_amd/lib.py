@@ -26,6 +26,11 @@ class PairformerBlockStruct(C.Structure):
                                     "c_single", "single_hidden")])
 
 
+class DiffusionBlockStruct(C.Structure):
+    """af3_diffusion_block."""
+    _fields_ = [(k, _vp) for k in ("w_q", "w_kv", "q_b", "w_out", "w_tr1", "w_tr2")]
+
+
 # name -> (restype, argtypes); must list every symbol include/af3_hip.h declares
 SIGNATURES = {
     "af3_abi_version": (_i, []),
@@ -75,6 +80,12 @@ SIGNATURES = {
     "af3_pairformer_single_workspace_bytes": (_sz, [_i64, _i, _i]),
     "af3_pairformer_stack_forward": (
         _i, [_vp, _i, _vp, _i, _vp, _vp, _vp, _i, _vp, _i64, _vp, _vp, _sz, _vp, _sz, _vp, _vp, _i]),
+    "af3_diffusion_transformer_workspace_bytes": (_sz, [_i64, _i64, _i, _i]),
+    "af3_diffusion_transformer_forward": (
+        _i, [_vp, _i, _vp, _i, _i64, _i64, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _i64, _vp, _sz, _vp]),
+    "af3_atom_transformer_workspace_bytes": (_sz, [_i64, _i64, _i64, _i, _i]),
+    "af3_atom_transformer_forward": (
+        _i, [_vp, _i, _vp, _i, _i64, _i64, _i64, _i64, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "af3_linear_bias_span": (_i, [_i64, _i, _i, _i, _i, _vp, _vp]),
     "af3_grid_attention_core_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "af3_check_gemm_f32": (

@@ -15,6 +15,28 @@ from .. import ops
 from .base import HipModule, bf16, drop_mesh, f32, in_check_mode, pack_swiglu, pad_rows
 
 
+class BlockTable:
+    """The packed weights of a transformer's blocks as the array of structures the library takes; made again when
+    any of the modules has been packed again."""
+
+    def __init__(self):
+        self.packs, self.array = None, None
+
+    def get(self, blocks):
+        """`blocks`: (attention, transition) modules."""
+        mods = [m for att, tr in blocks for m in (att, att.adaptive_zero_init, tr, tr.adaptive_zero_init)]
+        packs = [m.packed() for m in mods]
+        if self.packs is None or not all(a is b for a, b in zip(self.packs, packs)):
+            self.packs, self.array = packs, (L.DiffusionBlockStruct * len(blocks))()
+            for i, s in enumerate(self.array):
+                att, att_out, tr, tr_out = packs[4 * i:4 * i + 4]
+                s.w_q = (att["w_qkvg"] if "w_qkvg" in att else att["w_qg"]).data_ptr()
+                s.w_kv = att["w_kv"].data_ptr() if "w_kv" in att else None
+                s.q_b, s.w_out = att["q_b"].data_ptr(), att_out["w"].data_ptr()
+                s.w_tr1, s.w_tr2 = tr["w1"].data_ptr(), tr_out["w"].data_ptr()
+        return self.array
+
+
 class AdaptiveLayerNorm(HipModule):
     """nn/d_diffusion_transformer.py:37-74.  Output is bf16 (it always feeds a
     projection)."""
@@ -210,6 +232,7 @@ class DiffusionTransformer(HipModule):
         self.transition_block = nn.ModuleList(
             [DiffusionTransition(c_x=c_act, c_single_cond=c_single_cond, use_single_cond=True)
              for _ in range(num_blocks)])
+        self._table = BlockTable()
 
     def _pack(self):
         # Every block conditions on the same single_cond, so the 4 conditioning
@@ -262,27 +285,25 @@ class DiffusionTransformer(HipModule):
         p = self.packed()
         if not act.is_contiguous():
             raise ValueError("act must be contiguous (it is updated in place)")
-        n_out = self.super_block_size * self.num_head
         c, n_mod = self.c_act, 2 * self.num_blocks
         sc = single_cond.contiguous()
         rows = sc.numel() // sc.shape[-1]
         ss_all = ops.linear(ops.layer_norm(sc), p["w_ss"], bias=p["b_ss"], out_dtype=torch.float32)
-        ss_all = ss_all.view(rows, n_mod, 2 * c)                       # column slices, read in place
         gate_all = ops.linear(sc.to(torch.bfloat16), p["w_gate"], bias=p["b_gate"], out_dtype=torch.float32,
                               sigmoid=True)
-        gate_all = gate_all.view(rows, n_mod, c).permute(1, 0, 2)      # [module][row][c]: column slices, read in place
-        for sb in range(self.num_super_blocks):
-            if pair_logits is not None:
-                logits = pair_logits[sb]
-            else:
-                logits = ops.pair_logits(pair_cond.contiguous(), p["ln_w"], None, p["w_logits"][sb], n_out)
-                logits = logits.view(self.super_block_size, self.num_head, *logits.shape[1:])  # (b h) n s -> b h n s
-            for j in range(self.super_block_size):
-                i = sb * self.super_block_size + j
-                self.self_attention[i].run(act, mask, logits[j], single_cond, residual=True,
-                                           cond=(ss_all[:, 2 * i], gate_all[2 * i]))
-                self.transition_block[i].run(act, single_cond, residual=True,
-                                             cond=(ss_all[:, 2 * i + 1], gate_all[2 * i + 1]))
+        if pair_logits is None:    # read once: in the order the projection writes them
+            pair_logits = [ops.pair_logits(pair_cond.contiguous(), p["ln_w"], None, w, self.super_block_size * self.num_head)
+                           .view(self.super_block_size, self.num_head, *pair_cond.shape[:2]) for w in p["w_logits"]]
+        ss_all, gate_all = ss_all.view(rows, n_mod, 2 * c), gate_all.view(rows, n_mod, c)
+        run = self.num_super_blocks * self.super_block_size      # blocks beyond the last whole super-block never run
+        if run == 0:
+            return act
+        if run < self.num_blocks:
+            ss_all, gate_all = ss_all[:, :2 * run].contiguous(), gate_all[:, :2 * run].contiguous()
+        ops.diffusion_transformer(
+            self._table.get(list(zip(self.self_attention, self.transition_block))[:run]), act if act.dim() == 3 else act[None],
+            mask, [logits[j] for logits in pair_logits for j in range(self.super_block_size)], ss_all, gate_all,
+            self.num_head, self.transition_block[0].num_intermediate_factor * c)
         return act
 
 
@@ -337,27 +358,6 @@ class CrossAttention(HipModule):
         return self.adaptive_zero_init.run(avg, single_cond_q, x_q.dtype, residual=x_q if residual else None,
                                            gate=gate)
 
-    def run_gathered(self, x_q, key_rows, mask_q, mask_k, pair_logits, single_cond_q, cond):
-        """`run(..., residual=True)` for keys that are query atoms: key k of
-        subset s is atom key_rows[s, k] of the flattened (subset, query) axis of
-        x_q (negative: a masked slot, whose gathered activation and conditioning
-        are zero, hence K = V = 0).  The keys' adaptive LayerNorm and K / V
-        projection then run once per atom, not once per (subset, key), and no
-        key tensor is gathered: cond = (scale_shift_q, scale_shift_k of the
-        ATOMS [S * Q, 2c], gate)."""
-        p = self.packed()
-        n_sub, n_q, c = x_q.shape[-3:]
-        ss_q, ss_k_atoms, gate = cond
-        xq = self.q_adaptive_layernorm(x_q, single_cond_q, scale_shift=ss_q)
-        xk = self.k_adaptive_layernorm(x_q, single_cond_q, scale_shift=ss_k_atoms)
-        pl = None
-        if pair_logits is not None:
-            pl = pair_logits.reshape(-1, self.num_head, n_q, key_rows.shape[-1]).to(torch.float32).contiguous()
-        avg = ops.gathered_cross_attention(
-            xq.reshape(-1, n_q, c), xk.reshape(-1, n_sub * n_q, c), key_rows, pl, mask_q.reshape(-1, n_q),
-            mask_k.reshape(-1, key_rows.shape[-1]), p["w_qg"], p["w_kv"], p["q_b"], self.num_head)
-        return self.adaptive_zero_init.run(avg.reshape(x_q.shape), single_cond_q, x_q.dtype, residual=x_q, gate=gate)
-
     def forward(self, x_q, x_k, mask_q, mask_k, pair_logits=None, single_cond_q=None, single_cond_k=None):
         """x_q [(B,) S, Q, c], x_k [(B,) S, K, c], masks [(1,) S, Q] / [(1,) S, K],
         pair_logits [(1,) S, H, Q, K], conditioning [(1,) S, Q|K, c]."""
@@ -391,6 +391,7 @@ class DiffusionCrossAttTransformer(HipModule):
         self.transition_block = nn.ModuleList(
             [DiffusionTransition(c_x=c_query, c_single_cond=c_single_cond, use_single_cond=True)
              for _ in range(num_blocks)])
+        self._table = BlockTable()
 
     def _pack(self):
         # The conditioning inputs are the same for every block: all adaptive
@@ -444,8 +445,9 @@ class DiffusionCrossAttTransformer(HipModule):
         `keys_are_query_atoms`: the `queries_to_keys` gather, given by a caller
         whose keys_single_cond IS that gather of queries_single_cond (the atom
         cross-attention encoder and decoder build it so,
-        nn/d_atom_cross_attention.py:205-209).  The key side is then computed per
-        atom (see CrossAttention.run_gathered) instead of per (subset, key)."""
+        nn/d_atom_cross_attention.py:205-209).  The key side (adaptive
+        LayerNorm, K / V projection) is then computed per atom instead of per
+        (subset, key), and no key tensor is gathered."""
         p = self.packed()
         key_rows = None
         if keys_are_query_atoms is not None:
@@ -487,16 +489,16 @@ class DiffusionCrossAttTransformer(HipModule):
         if cond is None:
             cond = self.conditioning(queries_single_cond, keys_single_cond, pair_cond)
         logits, ss_q, ss_k, gate, key_rows = cond
+        if key_rows is not None:
+            return ops.atom_transformer(
+                self._table.get(list(zip(self.cross_attention, self.transition_block))), queries_act, key_rows, queries_mask,
+                keys_mask, logits, ss_q, ss_k, gate, self.num_head,
+                self.transition_block[0].num_intermediate_factor * self.c_query)
         for blk in range(self.num_blocks):
-            if key_rows is not None:
-                self.cross_attention[blk].run_gathered(queries_act, key_rows, queries_mask, keys_mask, logits[blk],
-                                                       queries_single_cond,
-                                                       cond=(ss_q[:, 2 * blk], ss_k[:, blk], gate[2 * blk]))
-            else:
-                keys_act = self._gather(queries_to_keys, queries_act)
-                self.cross_attention[blk].run(queries_act, keys_act, queries_mask, keys_mask, logits[blk],
-                                              queries_single_cond, keys_single_cond, residual=True,
-                                              cond=(ss_q[:, 2 * blk], ss_k[:, blk], gate[2 * blk]))
+            keys_act = self._gather(queries_to_keys, queries_act)
+            self.cross_attention[blk].run(queries_act, keys_act, queries_mask, keys_mask, logits[blk],
+                                          queries_single_cond, keys_single_cond, residual=True,
+                                          cond=(ss_q[:, 2 * blk], ss_k[:, blk], gate[2 * blk]))
             self.transition_block[blk].run(queries_act, queries_single_cond, residual=True,
                                            cond=(ss_q[:, 2 * blk + 1], gate[2 * blk + 1]))
         return queries_act

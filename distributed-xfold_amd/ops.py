@@ -232,6 +232,61 @@ def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incomi
     _L.check(rc, "af3_pairformer_stack_forward")
 
 
+def diffusion_transformer(blocks, act, mask, pair_logits, scale_shift, gate, num_head, hidden):
+    """The blocks of the diffusion transformer in one call (af3_diffusion_transformer_forward), act [B, S, C] updated
+    in place.  `blocks`: an array of lib.DiffusionBlockStruct; pair_logits: one fp32 tensor per block, [H, S, S] or
+    [H, S/4, S, 4]; scale_shift [cond_rows, 2 blocks, 2 C] and gate [cond_rows, 2 blocks, C] fp32."""
+    lib = _L.load()
+    _gpu(act, "act")
+    b, s, c = act.shape
+    nb = len(blocks)
+    quad = int(pair_logits[0].dim() == 4)
+    shape = (num_head, s // 4, s, 4) if quad else (num_head, s, s)
+    for t in pair_logits:
+        _gpu(t, "pair_logits", torch.float32, shape)
+    rows = scale_shift.shape[0]
+    _gpu(scale_shift, "scale_shift", torch.float32, (rows, 2 * nb, 2 * c))
+    _gpu(gate, "gate", torch.float32, (rows, 2 * nb, c))
+    if (b * s) % rows or len(pair_logits) != nb:
+        raise ValueError("rows must be a multiple of the conditioning rows, with one pair-logit tensor per block")
+    km = _mask_f32(mask, (s,), "key_mask")
+    ws = _ws(lib.af3_diffusion_transformer_workspace_bytes(b, s, c, hidden), act.device)
+    ptrs = (ctypes.c_void_p * nb)(*[t.data_ptr() for t in pair_logits])
+    rc = lib.af3_diffusion_transformer_forward(
+        blocks, nb, _p(act), _dt(act), b, s, c, hidden, num_head, _p(km), ptrs, quad, _p(scale_shift), _p(gate), rows,
+        _p(ws), ws.numel(), _stream(act.device))
+    _L.check(rc, "af3_diffusion_transformer_forward")
+    return act
+
+
+def atom_transformer(blocks, act, key_rows, mask_q, mask_k, pair_logits, scale_shift_q, scale_shift_k, gate, num_head,
+                     hidden):
+    """The blocks of the windowed atom transformer in one call (af3_atom_transformer_forward), act
+    [(B,) S, Q, C] updated in place.  key_rows [S, K] int32; pair_logits [blocks, S, H, Q, K]; scale_shift_q
+    [S Q, 2 blocks, 2 C], scale_shift_k [S Q, blocks, 2 C], gate [2 blocks, S Q, C] fp32."""
+    lib = _L.load()
+    _gpu(act, "act")
+    s, q, c = act.shape[-3:]
+    b = act.numel() // (s * q * c)
+    nb, k = len(blocks), key_rows.shape[-1]
+    _gpu(key_rows, "key_rows", torch.int32, (s, k))
+    if getattr(key_rows, "_af3_checked_rows", None) != s * q:
+        if int(key_rows.max()) >= s * q:
+            raise ValueError("key_rows: row index beyond the atoms")
+        key_rows._af3_checked_rows = s * q
+    _gpu(pair_logits, "pair_logits", torch.float32, (nb, s, num_head, q, k))
+    _gpu(scale_shift_q, "scale_shift_q", torch.float32, (s * q, 2 * nb, 2 * c))
+    _gpu(scale_shift_k, "scale_shift_k", torch.float32, (s * q, nb, 2 * c))
+    _gpu(gate, "gate", torch.float32, (2 * nb, s * q, c))
+    mq, mk = _mask_f32(mask_q.reshape(s, q), (s, q), "mask_q"), _mask_f32(mask_k.reshape(s, k), (s, k), "mask_k")
+    ws = _ws(lib.af3_atom_transformer_workspace_bytes(b, s, q, c, hidden), act.device)
+    rc = lib.af3_atom_transformer_forward(
+        blocks, nb, _p(act), _dt(act), b, s, q, k, c, hidden, num_head, _p(key_rows), _p(mq), _p(mk), _p(pair_logits),
+        _p(scale_shift_q), _p(scale_shift_k), _p(gate), _p(ws), ws.numel(), _stream(act.device))
+    _L.check(rc, "af3_atom_transformer_forward")
+    return act
+
+
 def batch_diffusion_self_attention(q_data, key_mask, nonbatched_bias, w_qkvg, query_b, num_head,
                                    out_dtype=torch.bfloat16, out=None, static_scratch=False):
     """batch_diffusion_self_attention_forward (csrc/Alpha_Attention.cpp:72-92).

@@ -536,6 +536,45 @@ int af3_pairformer_stack_forward(
     void* single_workspace, size_t single_workspace_bytes, af3_stream_t stream, af3_stream_t single_stream, int join);
 
 /* ---------------------------------------------------------------------------
+ * The blocks of the diffusion transformer (nn/d_diffusion_transformer.py:267-310)
+ * and of the windowed atom transformer (:466-543) as one call each, act updated in
+ * place.  The conditioning enters as the caller has projected it for all blocks at
+ * once (module 2 i: attention of block i, module 2 i + 1: its transition):
+ *   scale_shift [cond_rows][2 num_blocks][2 c] fp32 (adaptive LayerNorm scale | shift)
+ *   gate        [cond_rows][2 num_blocks][c]   fp32 (AdaLN-Zero gates, sigmoid taken)
+ * shared by the samples of the batch (rows modulo cond_rows).
+ *
+ * af3_diffusion_transformer_forward: act [batch,seq,c] in act_dtype, key_mask [seq]
+ *   or NULL, pair_logits: num_blocks HOST pointers to device planes [num_head,seq,seq]
+ *   fp32, or [num_head,seq/4,seq,4] with bias_quad_major.
+ * af3_atom_transformer_forward: act [samples,subsets,queries,c]; key k of subset s is
+ *   atom key_rows[s,k] of the sample's subsets * queries (negative: empty slot, K = V
+ *   = 0), see af3_gathered_cross_attention_forward; scale_shift_k [subsets * queries]
+ *   [num_blocks][2 c] per atom, pair_logits [num_blocks,subsets,num_head,queries,keys],
+ *   gate here [2 num_blocks][subsets * queries][c].
+ */
+typedef struct af3_diffusion_block {
+  const uint16_t* w_q;  /* diffusion: [4 c][c] q, k, v, gate;  atom: [2 c][c] q, gate */
+  const uint16_t* w_kv; /* atom: [2 c][c] k, v;  diffusion: NULL */
+  const float* q_b;     /* [c] */
+  const uint16_t* w_out; /* [c][c] */
+  const uint16_t* w_tr1; /* [2 hidden][c], packed for AF3_LINEAR_SWIGLU */
+  const uint16_t* w_tr2; /* [c][hidden] */
+} af3_diffusion_block;
+size_t af3_diffusion_transformer_workspace_bytes(int64_t batch, int64_t seq, int channels, int hidden);
+int af3_diffusion_transformer_forward(
+    const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t batch, int64_t seq, int channels,
+    int hidden, int num_head, const float* key_mask, const float* const* pair_logits, int bias_quad_major,
+    const float* scale_shift, const float* gate, int64_t cond_rows,
+    void* workspace, size_t workspace_bytes, af3_stream_t stream);
+size_t af3_atom_transformer_workspace_bytes(int64_t samples, int64_t subsets, int64_t queries, int channels, int hidden);
+int af3_atom_transformer_forward(
+    const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t samples, int64_t subsets,
+    int64_t queries, int64_t keys, int channels, int hidden, int num_head, const int32_t* key_rows, const float* mask_q,
+    const float* mask_k, const float* pair_logits, const float* scale_shift_q, const float* scale_shift_k,
+    const float* gate, void* workspace, size_t workspace_bytes, af3_stream_t stream);
+
+/* ---------------------------------------------------------------------------
  * Diagnostic, no counterpart in the reference.  The dense kernels fetch a
  * column bias in groups (eight entries on the smaller tiles, four per lane on the
  * 256x256 tile, the last group pulled back to end at column n), and a segmented
