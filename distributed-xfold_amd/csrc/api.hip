@@ -327,9 +327,10 @@ static int self_attention_args_ok(
 static int self_attention_run(
     const uint16_t* q_data, const float* key_mask, int64_t mask_batches, const float* nonbatched_bias,
     int bias_quad_major, const uint16_t* w_qkvg, const float* query_b, int num_head,
-    void* out, int out_dtype, int64_t batch, int64_t seq, int channels, bf16_t* qkvg, hipStream_t s) {
+    void* out, int out_dtype, int64_t batch, int64_t seq, int channels, bf16_t* qkvg, int split_k, hipStream_t s) {
   const int d = channels / num_head;
   GemmArgs g;
+  g.split_k = split_k;
   g.A = q_data; g.B = w_qkvg; g.C = qkvg;
   g.M = (int)(batch * seq); g.N = 4 * channels; g.K = channels;
   g.lda = channels; g.ldb = channels; g.ldc = 4 * channels;
@@ -357,14 +358,8 @@ int af3_batch_diffusion_self_attention_forward(
     int bias_quad_major, const uint16_t* w_qkvg, const float* query_b, int num_head,
     void* out, int out_dtype, int64_t batch, int64_t seq, int channels,
     void* workspace, size_t workspace_bytes, af3_stream_t stream) {
-  int rc = self_attention_args_ok(q_data, key_mask, mask_batches, bias_quad_major, w_qkvg, out, out_dtype, num_head,
-                                  batch, seq, channels);
-  if (rc) return rc;
-  Carver ws(workspace, workspace_bytes);
-  bf16_t* qkvg = ws.take<bf16_t>((size_t)batch * seq * 4 * channels);
-  if (!ws.ok) return AF3_ERR_WORKSPACE;
-  return self_attention_run(q_data, key_mask, mask_batches, nonbatched_bias, bias_quad_major, w_qkvg, query_b,
-                            num_head, out, out_dtype, batch, seq, channels, qkvg, static_cast<hipStream_t>(stream));
+  return run_self_attention(q_data, key_mask, mask_batches, nonbatched_bias, bias_quad_major, w_qkvg, query_b, num_head, out,
+                            out_dtype, batch, seq, channels, workspace, workspace_bytes, 0, static_cast<hipStream_t>(stream));
 }
 
 int af3_batch_diffusion_self_attention_forward_static(
@@ -381,7 +376,7 @@ int af3_batch_diffusion_self_attention_forward_static(
   // The q/k/v/gate product writes every element of [batch * seq][4 * channels] before the attention kernel reads
   // any of them, so nothing left in the array by an earlier (possibly larger) call is ever read: no clearing.
   return self_attention_run(q_data, key_mask, mask_batches, nonbatched_bias, bias_quad_major, w_qkvg, query_b,
-                            num_head, out, out_dtype, batch, seq, channels, qkvg, static_cast<hipStream_t>(stream));
+                            num_head, out, out_dtype, batch, seq, channels, qkvg, 0, static_cast<hipStream_t>(stream));
 }
 
 // ---------------------------------------------------- masked row softmax, narrow fp32 layers
@@ -627,36 +622,8 @@ int af3_linear_forward(
     const uint16_t* x, const uint16_t* w, const float* bias, void* y, int y_dtype,
     int64_t m, int n, int k, int mode, float alpha, int sigmoid,
     const float* gate, int64_t gate_rows, int64_t gate_ld, const void* residual, int res_dtype, af3_stream_t stream) {
-  if (!x || !w || !y || bad_dtype(y_dtype) || m <= 0 || m > 0x7fffffff || n <= 0 || k <= 0) return AF3_ERR_BAD_ARG;
-  if (gate_ld != 0 && gate_ld < n) return AF3_ERR_BAD_ARG;
-  if (mode != AF3_LINEAR_PLAIN && mode != AF3_LINEAR_SWIGLU && mode != AF3_LINEAR_GATE_RES &&
-      mode != AF3_LINEAR_REGROUP32 && mode != AF3_LINEAR_ROWGATE_RES)
-    return AF3_ERR_BAD_ARG;
-  if (residual && bad_dtype(res_dtype)) return AF3_ERR_BAD_ARG;
-  GemmArgs g;
-  if (mode == AF3_LINEAR_REGROUP32) {
-    if ((m & 31) || (n & 31) || gate || residual) return AF3_ERR_BAD_ARG;
-    g.regroup32 = 1;
-    mode = AF3_LINEAR_PLAIN;
-  }
-  if (mode == AF3_LINEAR_ROWGATE_RES) {
-    if (!gate || gate_rows <= 0) return AF3_ERR_BAD_ARG;
-    g.gate_per_row = 1;
-    mode = AF3_LINEAR_GATE_RES;
-  }
-  g.A = x; g.B = w; g.C = y;
-  g.M = (int)m; g.N = n; g.K = k;
-  g.lda = k; g.ldb = k;
-  g.ldc = mode == AF3_LINEAR_SWIGLU ? n / 2 : n;
-  g.out_f32 = y_dtype == AF3_F32;
-  g.epi = mode; g.alpha = alpha; g.bias = bias; g.bias_len = n; g.act_sigmoid = sigmoid;
-  g.gate = gate; g.gate_rows = (int)gate_rows; g.ld_gate = gate_ld ? gate_ld : n;
-  if (residual) {
-    if (res_dtype == AF3_F32) g.res_f32 = static_cast<const float*>(residual);
-    else g.res_bf16 = static_cast<const bf16_t*>(residual);
-    g.ld_res = n;
-  }
-  return launch_gemm_nt(g, static_cast<hipStream_t>(stream));
+  return run_linear(x, w, bias, y, y_dtype, m, n, k, mode, alpha, sigmoid, gate, gate_rows, gate_ld, residual, res_dtype, 0,
+                    static_cast<hipStream_t>(stream));
 }
 
 // ----------------------------------------------------------------- diagnostics
@@ -744,3 +711,53 @@ int af3_check_attention_f32(
 }
 
 }  // extern "C"
+
+int run_self_attention(const bf16_t* q_data, const float* key_mask, int64_t mask_batches, const float* nonbatched_bias,
+                       int bias_quad_major, const bf16_t* w_qkvg, const float* query_b, int num_head, void* out, int out_dtype,
+                       int64_t batch, int64_t seq, int channels, void* workspace, size_t workspace_bytes, int split_k,
+                       hipStream_t stream) {
+  int rc = self_attention_args_ok(q_data, key_mask, mask_batches, bias_quad_major, w_qkvg, out, out_dtype, num_head,
+                                  batch, seq, channels);
+  if (rc) return rc;
+  Carver ws(workspace, workspace_bytes);
+  bf16_t* qkvg = ws.take<bf16_t>((size_t)batch * seq * 4 * channels);
+  if (!ws.ok) return AF3_ERR_WORKSPACE;
+  return self_attention_run(q_data, key_mask, mask_batches, nonbatched_bias, bias_quad_major, w_qkvg, query_b, num_head, out,
+                            out_dtype, batch, seq, channels, qkvg, split_k, stream);
+}
+
+int run_linear(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int y_dtype, int64_t m, int n, int k, int mode,
+               float alpha, int sigmoid, const float* gate, int64_t gate_rows, int64_t gate_ld, const void* residual,
+               int res_dtype, int split_k, hipStream_t stream) {
+  if (!x || !w || !y || bad_dtype(y_dtype) || m <= 0 || m > 0x7fffffff || n <= 0 || k <= 0) return AF3_ERR_BAD_ARG;
+  if (gate_ld != 0 && gate_ld < n) return AF3_ERR_BAD_ARG;
+  if (mode != AF3_LINEAR_PLAIN && mode != AF3_LINEAR_SWIGLU && mode != AF3_LINEAR_GATE_RES &&
+      mode != AF3_LINEAR_REGROUP32 && mode != AF3_LINEAR_ROWGATE_RES)
+    return AF3_ERR_BAD_ARG;
+  if (residual && bad_dtype(res_dtype)) return AF3_ERR_BAD_ARG;
+  GemmArgs g;
+  g.split_k = split_k;
+  if (mode == AF3_LINEAR_REGROUP32) {
+    if ((m & 31) || (n & 31) || gate || residual) return AF3_ERR_BAD_ARG;
+    g.regroup32 = 1;
+    mode = AF3_LINEAR_PLAIN;
+  }
+  if (mode == AF3_LINEAR_ROWGATE_RES) {
+    if (!gate || gate_rows <= 0) return AF3_ERR_BAD_ARG;
+    g.gate_per_row = 1;
+    mode = AF3_LINEAR_GATE_RES;
+  }
+  g.A = x; g.B = w; g.C = y;
+  g.M = (int)m; g.N = n; g.K = k;
+  g.lda = k; g.ldb = k;
+  g.ldc = mode == AF3_LINEAR_SWIGLU ? n / 2 : n;
+  g.out_f32 = y_dtype == AF3_F32;
+  g.epi = mode; g.alpha = alpha; g.bias = bias; g.bias_len = n; g.act_sigmoid = sigmoid;
+  g.gate = gate; g.gate_rows = (int)gate_rows; g.ld_gate = gate_ld ? gate_ld : n;
+  if (residual) {
+    if (res_dtype == AF3_F32) g.res_f32 = static_cast<const float*>(residual);
+    else g.res_bf16 = static_cast<const bf16_t*>(residual);
+    g.ld_res = n;
+  }
+  return launch_gemm_nt(g, stream);
+}

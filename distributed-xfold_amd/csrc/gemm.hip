@@ -11,10 +11,10 @@
 // 10 GFLOP, so that what they cost is not matrix time but the number of CUs
 // that have a tile and the length of one workgroup's chain (first miss, K loop,
 // hand-over, store).  Hence:
-//   * the tile shrinks with the product (128x128 down to 32x32) until about every
-//     CU has one, and where that is not enough the waves of a workgroup share the K
-//     range of one tile instead of its area (WK groups; their fp32 partial tiles
-//     are added in LDS): K = 1536 is then a chain of three slabs, not of 24;
+//   * the tile shrinks with the product (128x128 down to 32x32) until about every CU has one, and
+//     where that is not enough and the caller does not mind the order of summation (GemmArgs::split_k)
+//     the waves of a workgroup share the K range of one tile instead of its area (WK groups; their fp32
+//     partial tiles are added in LDS): K = 1536 is then a chain of three slabs, not of 24;
 //   * slabs are 64 deep, so a slab row is one whole 128-byte cache line.  From L2 a CU takes
 //     in 115 bytes/ns that way; in 64-byte row pieces it is 62 (measured, LDS-direct loads);
 //   * slabs go from global memory straight into LDS, all of a workgroup's first ones
@@ -24,14 +24,13 @@
 //     lane owns one row and four consecutive columns per register quad, so a partial
 //     tile goes to LDS in 16-byte stores.
 //
-// The order in which K is summed depends on N and K alone, never on M (gemm_k_groups): a
-// sample gives the same bits alone and in a batch, whatever tile either takes.  Where K is
-// summed in four groups, (p0 + p1) + (p2 + p3), a tile whose waves do not share the K range
-// keeps the groups apart in its accumulators.
+// Without split_k every tile sums K in the same order, one 16-deep MFMA step after the other
+// from k = 0, as the 256x256 tile does: a row gives the same bits alone and in a batch, whatever
+// tile it lands in.
 //
-// Measured against the register-staged 128x128-tile kernel this replaces: 64x384x384
-// 3.5 us (was 8.9), 64x384x1536 5.2 (19.6), 500x768x768 5.3 (14.3), 500x3072x768 10.9 (16.2), 1920x3072x768
-// 17.4 (22.6), 3840x768x768 12.8 (15.3), 768x73728x384 to fp32 112 (125), 12000x256x128 6.4 (11.3).
+// Measured against the register-staged 128x128-tile kernel this replaces (weights not in L2): 500x768x768 5.6 us
+// (was 14.3), 500x768x1536 7.5 (21.4), 500x3072x768 8.7 (16.2), 1920x3072x768 16.7 (22.6), 3840x768x768 13.8 (15.3),
+// 768x73728x384 to fp32 112 (125), 12000x256x128 6.4 (11.3); with split_k 64x384x384 3.4 (8.9), 64x384x1536 4.9 (19.6).
 #include <type_traits>
 
 #include "common.h"
@@ -41,13 +40,23 @@ namespace {
 
 constexpr int KS = 64;        // slab depth
 constexpr int ROWB = KS * 2;  // bytes of a slab row in LDS (unpadded, 16-byte chunks permuted)
+constexpr uint32_t BUFFER_END = 0x7fffffffu;  // size of a buffer descriptor that covers every offset of a tile
 
-// 64 lanes x 16 bytes from global (uniform base + per-lane byte offset) to the ith KB of LDS behind the
-// wave-uniform address lds.  Inline assembly, because the compiler's own form makes later LDS reads wait for every
-// such load in flight; here a buffer is read only behind an explicit wait.
-__device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint32_t lds, int i) {
-  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base), "n"(i * 1024)
+// 64 lanes x 16 bytes from a range-checked buffer (descriptor, wave-uniform byte offset, per-lane byte offset) to
+// the ith KB of LDS behind the wave-uniform address lds.  An offset past the descriptor's size writes zeros and fetches
+// nothing, but the load counts like any other: the waits of a loop can be constants, and K needs no tail.  Inline assembly, because the
+// compiler's own form makes later LDS reads wait for every such load in flight; here a buffer is read only behind
+// an explicit wait.
+__device__ __forceinline__ void load_to_lds(const u32x4 rsrc, uint32_t soff, uint32_t off, uint32_t lds, int i) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(off), "s"(rsrc),
+               "s"(soff), "n"(i * 1024)
                : "m0", "scc", "memory");
+}
+// raw buffer descriptor of a uniform pointer (word 3: untyped 32-bit data)
+__device__ __forceinline__ u32x4 buffer_of(const void* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return u32x4{lo, hi & 0xffffu, BUFFER_END, 0x00020000u};
 }
 template <int N>
 __device__ __forceinline__ void wait_loads_but() {
@@ -56,21 +65,20 @@ __device__ __forceinline__ void wait_loads_but() {
 }
 
 // A workgroup of WM x WN x WK waves computes BM = 32 MT WM rows x BN = 32 NT WN columns; ST slab buffers per group.
-// KIND: the epilogue.  VEC: all of its loads and stores are 16-byte ones (without: element by element, for odd column
-// counts and unaligned operands).  GROUPS: K is summed in four groups.  WPS: waves per SIMD the tile's LDS leaves room for; the
+// CLEAN: K is a multiple of the slab depth.  KIND: the epilogue.  VEC: all of its loads and stores are 16-byte ones (without: element by element, for odd column
+// counts and unaligned operands).  WPS: waves per SIMD the tile's LDS leaves room for; the
 // registers have to as well (a wave more or less per SIMD is up to a factor of two in the short products).
 enum { KIND_COLUMNS = 0, KIND_GATE_RES = 1, KIND_SWIGLU = 2 };
-template <int MT, int NT, int WM, int WN, int WK, int ST, int WPS, bool GROUPS, int KIND, bool VEC, bool OUT_F32>
+template <int MT, int NT, int WM, int WN, int WK, int ST, int WPS, bool CLEAN, int KIND, bool VEC, bool OUT_F32>
 __global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArgs g) {
   constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN, NTHR = 64 * WM * WN * WK, GW = WM * WN;
   constexpr int SLAB = (BM + BN) * ROWB;     // A rows first, then B rows
   constexpr int NLOAD = (BM + BN) / 8 / GW;  // 1 KB loads per wave and slab
   constexpr int LA = BM / 8 / GW;            // of which A
-  static_assert(WK == 1 || WK == 2 || WK == 4, "");
+  static_assert(WK == 1 || WK == 2 || WK == 4 || WK == 8, "");
   static_assert((BM / 8) % GW == 0 && (BN / 8) % GW == 0, "loads of a slab are dealt evenly");
   constexpr bool ALONE = GW == 1;
-  constexpr int FLY = ALONE ? ST : ST - 1;   // slabs requested ahead
-  static_assert(FLY >= 1 && FLY <= 2 && FLY * NLOAD < 64, "");
+  static_assert(ST >= 2 && (ST - 1) * NLOAD < 64, "vmcnt has six bits");
   constexpr int LDS_C = BN + 4;              // row stride (fp32) of a partial tile
   constexpr int BYTES = WK * ST * SLAB > WK * BM * LDS_C * 4 ? WK * ST * SLAB : WK * BM * LDS_C * 4;
   __shared__ __attribute__((aligned(1024))) char smem[BYTES];
@@ -95,8 +103,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArg
   const int bz = __builtin_amdgcn_readfirstlane(logical / (tiles_m * tiles_n));
 
   // the tile's first rows: what a lane adds to these fits 32 bits whatever the operands' size
-  const char* A = reinterpret_cast<const char*>(g.A + (int64_t)bz * g.sA + (int64_t)m0 * g.lda);
-  const char* B = reinterpret_cast<const char*>(g.B + (int64_t)bz * g.sB + (int64_t)n0 * g.ldb);
+  const u32x4 A = buffer_of(g.A + (int64_t)bz * g.sA + (int64_t)m0 * g.lda);
+  const u32x4 B = buffer_of(g.B + (int64_t)bz * g.sB + (int64_t)n0 * g.ldb);
 
   // Load i of a wave covers eight rows of A (i < LA) or B, one 128-byte row per 8 lanes.  Chunk c of row r lives at
   // position c ^ ((r >> 1) & 7) of the row (a load cannot pad rows): 16 consecutive rows' reads of one chunk then
@@ -112,21 +120,19 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArg
   const int ns = (g.K + KS - 1) / KS;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)smem;
   const int s0 = grp * ns / WK, cnt = (grp + 1) * ns / WK - s0;
-  constexpr int NG = GROUPS ? 4 / WK : 1;  // groups of the K sum that this wave goes through
   const uint32_t mine = (uint32_t)(grp * (ST * SLAB));  // this group's buffers in smem
-  auto issue = [&](int s, uint32_t dst) {
+  auto issue = [&](int s, uint32_t dst) {  // slab s of this wave's share; past its end: zeros
     const uint32_t da = __builtin_amdgcn_readfirstlane(lds0 + dst + LA * gw * 1024);
     const uint32_t db = __builtin_amdgcn_readfirstlane(lds0 + dst + BM * ROWB + (NLOAD - LA) * gw * 1024);
-    const uint32_t k0 = (uint32_t)(s0 + s) * KS;
-    const bool tail = k0 + KS > (uint32_t)g.K;
+    const int k0 = (s0 + s) * KS;
+    const uint32_t kb = __builtin_amdgcn_readfirstlane((uint32_t)k0 * 2u);
+    u32x4 ra = A, rb = B;
+    ra.z = rb.z = __builtin_amdgcn_readfirstlane(s < cnt ? BUFFER_END : 0u);
 #pragma unroll
     for (int i = 0; i < NLOAD; ++i) {
-      uint32_t kb = k0 * 2u;
-      // a chunk past K is fetched from its place in the row's first slab (K >= 64) or from the row's start, and
-      // zeroed in LDS before the slab is used
-      if (tail && k0 + chunk_of(i) * 8 >= (uint32_t)g.K) kb = g.K >= KS ? 0u : 0u - (uint32_t)chunk_of(i) * 16u;
-      if (i < LA) load_to_lds(A, off[i] + kb, da, i);
-      else load_to_lds(B, off[i] + kb, db, i - LA);
+      const uint32_t o = CLEAN || k0 + chunk_of(i) * 8 < g.K ? off[i] : 0x80000000u;
+      if (i < LA) load_to_lds(ra, kb, o, da, i);
+      else load_to_lds(rb, kb, o, db, i - LA);
     }
   };
 
@@ -170,80 +176,78 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArg
     }
   };
 
-  f32x16 acc[MT][NT], sum0[MT][NT], sum1[MT][NT];
-  auto each = [&](auto f) {
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) f(acc[i][j], sum0[i][j], sum1[i][j]);
-  };
+  f32x16 acc[MT][NT];
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  each([&](f32x16& a, f32x16& s, f32x16& t) { a = s = t = zero; });
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = zero;
 
   uint32_t fo[4];
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) fo[ks] = (uint32_t)(l31 * ROWB + (((2 * ks + hh) ^ ((l31 >> 1) & 7)) << 4));
 
 #pragma unroll
-  for (int p = 0; p < FLY; ++p)
-    if (p < cnt) issue(p, mine + p * SLAB);
+  for (int p = 0; p < ST; ++p) issue(p, mine + p * SLAB);
   if constexpr (KIND == KIND_GATE_RES && EARLY) fetch(0, pre[0]);
 
-  // One barrier per slab where waves share it (all groups take part in all of them): behind it the slab has
-  // landed for every wave of the group and the buffer of the slab before is free.
-  int cur = 0, i = 0;
-#pragma unroll 1
-  for (int gq = 0; gq < NG; ++gq) {
-    // (the last group of waves has the most slabs; the others join it at its barriers)
-    const int end = gq < NG - 1 ? (NG * grp + gq + 1) * ns / (NG * WK) - s0 : ALONE ? cnt : (ns + WK - 1) / WK;
-#pragma unroll 1
-    for (; i < end; ++i) {
-      const int rem = cnt - 1 - i;  // slabs of this wave still to come
-      if (FLY >= 2 && rem >= 1) wait_loads_but<(FLY >= 2 ? NLOAD : 0)>();
-      else wait_loads_but<0>();
-      const uint32_t bo = mine + cur * SLAB;
-      char* b = smem + bo;
-      const int k0 = (s0 + i) * KS;
-      if (!ALONE) lds_barrier();
-      if (i < cnt && k0 + KS > g.K) {
-        const u32x4 z = {0, 0, 0, 0};
-        for (int row = lane + 64 * gw; row < BM + BN; row += 64 * GW)
-          for (int c = (g.K - k0) >> 3; c < 8; ++c) *reinterpret_cast<u32x4*>(b + row * ROWB + ((c ^ ((row >> 1) & 7)) << 4)) = z;
-      }
-      if (!ALONE && ns * KS > g.K && i == (ns + WK - 1) / WK - 1) lds_barrier();
-      if (!ALONE && i + FLY < cnt) issue(i + FLY, mine + (cur == 0 ? ST - 1 : cur - 1) * SLAB);
-      if (ALONE || i < cnt) {
+  struct Frags { bf16x8 a[4][MT], b[4][NT]; };
+  auto read_frags = [&](Frags& f, uint32_t bo) {
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          bf16x8 fa[MT], fb[NT];
+    for (int ks = 0; ks < 4; ++ks) {
 #pragma unroll
-          for (int t = 0; t < MT; ++t) fa[t] = as_frag(*reinterpret_cast<const u32x4*>(b + (wm + t * 32) * ROWB + fo[ks]));
+      for (int t = 0; t < MT; ++t) f.a[ks][t] = as_frag(*reinterpret_cast<const u32x4*>(smem + bo + (wm + t * 32) * ROWB + fo[ks]));
 #pragma unroll
-          for (int t = 0; t < NT; ++t) fb[t] = as_frag(*reinterpret_cast<const u32x4*>(b + (BM + wn + t * 32) * ROWB + fo[ks]));
-#pragma unroll
-          for (int x = 0; x < MT; ++x)
-#pragma unroll
-            for (int y = 0; y < NT; ++y) acc[x][y] = mfma32(fb[y], fa[x], acc[x][y]);
-        }
-      }
-      if (ALONE && i + ST < cnt) {  // the wave's fragment reads of the buffer must be done before it is refilled
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        issue(i + ST, bo);
-      }
-      cur = cur + 1 == ST ? 0 : cur + 1;
+      for (int t = 0; t < NT; ++t) f.b[ks][t] = as_frag(*reinterpret_cast<const u32x4*>(smem + bo + (BM + wn + t * 32) * ROWB + fo[ks]));
     }
-    if (NG > 1 && gq < NG - 1) {
-      if (NG == 4 && gq == 1) each([&](f32x16& a, f32x16& s, f32x16& t) { t = s + a; a = zero; });
-      else each([&](f32x16& a, f32x16& s, f32x16&) { s = a; a = zero; });
-    }
+  };
+  auto products = [&](const Frags& f) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int x = 0; x < MT; ++x)
+#pragma unroll
+        for (int y = 0; y < NT; ++y) acc[x][y] = mfma32(f.b[ks][y], f.a[ks][x], acc[x][y]);
+  };
+  // the waves that share slabs meet; a lone wave waits for its own LDS reads
+  auto meet = [&]() {
+    if constexpr (ALONE) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    else lds_barrier();
+  };
+  // Step i: slab i + 1 has landed (for every wave that shares it), slab i's fragments are in registers, so its buffer
+  // takes slab i + ST; the fragments of slab i + 1 are read while the products of slab i run.  A 32x32 accumulator is
+  // one chain of dependent MFMAs, and nothing else should lengthen it.  (Groups of waves with a slab less than the
+  // next take part in all steps: their last slab is zeros.)
+  const int trips = (ns + WK - 1) / WK;
+  Frags f0, f1;
+  uint32_t cur = 0;  // byte offset of slab i's buffer
+  auto step = [&](int i, const Frags& now, Frags& then) {
+    const uint32_t nxt = cur + SLAB == ST * SLAB ? 0 : cur + SLAB;
+    // (towards the end nothing younger than slab i + 1 may be in flight any more)
+    if (ST > 2 && i + ST - 1 < trips) wait_loads_but<(ST - 2) * NLOAD>();
+    else wait_loads_but<0>();
+    meet();
+    if (i + ST < trips) issue(i + ST, mine + cur);
+    read_frags(then, mine + nxt);
+    products(now);
+    cur = nxt;
+  };
+  wait_loads_but<(ST - 1) * NLOAD>();
+  meet();
+  read_frags(f0, mine);
+  int i = 0;
+  for (; i + 1 < trips; i += 2) {
+    step(i, f0, f1);
+    step(i + 1, f1, f0);
   }
-  if constexpr (NG == 4) each([](f32x16& a, f32x16& s, f32x16& t) { a = t + (s + a); });
-  if constexpr (NG == 2) each([](f32x16& a, f32x16& s, f32x16&) { a = s + a; });
+  if (i < trips) products(f0);
 
   if constexpr (KIND == KIND_GATE_RES && !EARLY)
 #pragma unroll
     for (int k = 0; k < PRE; ++k) fetch(k, pre[k]);
-  // partial tiles -> LDS, over the slab buffers: every wave must have finished its slabs
+  // partial tiles -> LDS, over the slab buffers: every wave must have finished its slabs (and the loads past their
+  // end must have written their zeros)
+  wait_loads_but<0>();
   float* sC = reinterpret_cast<float*>(smem);
   lds_barrier();
 #pragma unroll
@@ -260,7 +264,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArg
     auto part = [&](int w, int at) { return *reinterpret_cast<const f32x4*>(sC + (w * BM + row) * LDS_C + at); };
     f32x4 lo = part(0, c), hi = part(0, c + 4);
     if constexpr (WK >= 2) { lo += part(1, c); hi += part(1, c + 4); }
-    if constexpr (WK == 4) { lo += part(2, c) + part(3, c); hi += part(2, c + 4) + part(3, c + 4); }
+    if constexpr (WK >= 4) { lo += part(2, c) + part(3, c); hi += part(2, c + 4) + part(3, c + 4); }
+    if constexpr (WK == 8) {
+      lo += (part(4, c) + part(5, c)) + (part(6, c) + part(7, c));
+      hi += (part(4, c + 4) + part(5, c + 4)) + (part(6, c + 4) + part(7, c + 4));
+    }
     v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
   };
   using OutT = std::conditional_t<OUT_F32, float, bf16_t>;
@@ -340,14 +348,14 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArg
   }
 }
 
-template <int MT, int NT, int WM, int WN, int WK, int ST, int WPS, bool GROUPS, bool VEC = true>
+template <int MT, int NT, int WM, int WN, int WK, int ST, int WPS, bool CLEAN = true, bool VEC = true>
 int launch_tile(const GemmArgs& g, hipStream_t stream) {
   constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN;
   const int64_t total = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN) * g.batch;
   const int64_t blocks = (total + 7) / 8 * 8;
   if (blocks > 0x3fffffff) return AF3_ERR_BAD_ARG;
   const dim3 grid((unsigned)blocks), block(64 * WM * WN * WK);
-#define LAUNCH(KIND, OUT_F32) hipLaunchKernelGGL((gemm_nt_kernel<MT, NT, WM, WN, WK, ST, WPS, GROUPS, KIND, VEC, OUT_F32>), grid, block, 0, stream, g)
+#define LAUNCH(KIND, OUT_F32) hipLaunchKernelGGL((gemm_nt_kernel<MT, NT, WM, WN, WK, ST, WPS, CLEAN, KIND, VEC, OUT_F32>), grid, block, 0, stream, g)
   if (g.epi == EPI_SWIGLU) {
     if constexpr (BN >= 64) LAUNCH(KIND_SWIGLU, false);
     else return AF3_ERR_BAD_ARG;
@@ -363,11 +371,6 @@ int launch_tile(const GemmArgs& g, hipStream_t stream) {
 }
 
 }  // namespace
-
-// How K is summed: in four groups where a short product is likely to have its K range split between waves (the
-// K loop is five slabs or longer and the columns alone do not make enough tiles), in one go otherwise.  N = 2048
-// on: the wide projections of the diffusion transformer, which large batches hand to the 256x256 tile.
-static int gemm_k_groups(const GemmArgs& g) { return g.K > 256 && g.N < 2048 ? 4 : 1; }
 
 // Products of at least 120 tiles of 256x256 go to the large-tile kernel where one of its epilogues fits: a
 // 128x128 tile of the kernel above needs twice the fragment reads per MFMA and is bound by them from there on
@@ -388,7 +391,7 @@ int launch_gemm_nt(const GemmArgs& g_in, hipStream_t stream) {
   if ((g.K & 7) || (g.lda & 7) || (g.ldb & 7) || (g.sA & 7) || (g.sB & 7)) return AF3_ERR_BAD_ARG;
   if (((uintptr_t)g.A & 15) || ((uintptr_t)g.B & 15)) return AF3_ERR_BAD_ARG;
   if (g.K > g.lda || g.K > g.ldb) return AF3_ERR_BAD_ARG;
-  if (g.lda >= (1ll << 23) || g.ldb >= (1ll << 23)) return AF3_ERR_BAD_ARG;  // 32-bit byte offsets inside a tile
+  if (g.lda >= (1ll << 22) || g.ldb >= (1ll << 22)) return AF3_ERR_BAD_ARG;  // 31-bit byte offsets inside a tile
   if (g.epi == EPI_SWIGLU && ((g.N & 63) || g.out_f32)) return AF3_ERR_BAD_ARG;
   if (g.epi == EPI_SEGMENTED && (g.seg_len <= 0 || (g.seg_len & 7))) return AF3_ERR_BAD_ARG;
   if (g.gate && g.gate_rows <= 0) return AF3_ERR_BAD_ARG;
@@ -409,22 +412,24 @@ int launch_gemm_nt(const GemmArgs& g_in, hipStream_t stream) {
                    al(g.res_bf16, g.ld_res * 2, g.sRes * 2);
 
   // The tile, by the number T of 64x64 tiles (256 CUs; measured over M = 64 ... 92160, N = 128 ... 73728,
-  // K = 64 ... 1536):
-  //   T <= 128  32x32 tiles, K split four ways: the 64x64 tiles would leave half of the CUs without one
-  //   T <= 384  64x64 with K split two ways (eight waves per tile)
-  //   T <= 1000 64x64, two to three workgroups per CU
-  //   T <= 2600 64x128, else 128x128: bytes per FLOP count once every CU has several tiles (and never wider than N)
-  // (a split tile only where K is summed in groups; SwiGLU pairs 32-column blocks, so its tiles are 64 columns or more)
-  const bool groups = gemm_k_groups(g) == 4;
+  // K = 64 ... 1536; SwiGLU pairs 32-column blocks, so its tiles are 64 columns or more):
+  //   T <= 128   32x32, the 64x64 tiles would leave half of the CUs without one; with split_k the K range goes to four
+  //              waves, or eight where it is long
+  //   T <= 384   with split_k: 64x64, K split two ways (eight waves per tile); long ones are faster unsplit
+  //   T <= 1000  64x64, with as many slab buffers as leave room for the workgroups a CU gets: four, three or two
+  //   T <= 2600  64x128, else 128x128: bytes per FLOP count once every CU has several tiles (and never wider than N)
   const int64_t T = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch;
-  if (!vec) return groups ? launch_tile<1, 1, 2, 2, 1, 2, 4, true, false>(g, stream) : launch_tile<1, 1, 2, 2, 1, 2, 4, false, false>(g, stream);
-  if (groups) {
-    if (T <= 128 && g.epi != EPI_SWIGLU) return launch_tile<1, 1, 1, 1, 4, 2, 2, true>(g, stream);
-    if (T <= 384) return launch_tile<1, 1, 2, 2, 2, 2, 4, true>(g, stream);
-    if (T <= 1000 || g.N <= 64) return launch_tile<1, 1, 2, 2, 1, 2, 4, true>(g, stream);
-    return launch_tile<1, 2, 2, 2, 1, 2, 3, true>(g, stream);
+  const bool wide = g.epi == EPI_SWIGLU;
+  if (!vec) return launch_tile<1, 1, 2, 2, 1, 2, 4, false, false>(g, stream);
+  if (g.K % KS) return launch_tile<1, 1, 2, 2, 1, 2, 4, false>(g, stream);
+  if (g.split_k && g.K > 256) {
+    if (T <= 128 && !wide) return g.K >= 1024 ? launch_tile<1, 1, 1, 1, 8, 2, 2>(g, stream) : launch_tile<1, 1, 1, 1, 4, 2, 2>(g, stream);
+    if (T <= 384 && g.K < 1024) return launch_tile<1, 1, 2, 2, 2, 2, 4>(g, stream);
   }
-  if (T <= 1000 || g.N <= 64) return launch_tile<1, 1, 2, 2, 1, 2, 4, false>(g, stream);
-  if (T <= 2600 || g.N <= 128) return launch_tile<1, 2, 2, 2, 1, 2, 3, false>(g, stream);
-  return launch_tile<2, 2, 2, 2, 1, 2, 2, false>(g, stream);
+  if (T <= 128 && !wide) return launch_tile<1, 1, 1, 1, 1, 4, 1>(g, stream);
+  if (T <= 256) return launch_tile<1, 1, 2, 2, 1, 4, 2>(g, stream);
+  if (T <= 640) return launch_tile<1, 1, 2, 2, 1, 3, 3>(g, stream);
+  if (T <= 1000 || g.N <= 64) return launch_tile<1, 1, 2, 2, 1, 2, 4>(g, stream);
+  if (T <= 2600 || g.N <= 128) return launch_tile<1, 2, 2, 2, 1, 2, 3>(g, stream);
+  return launch_tile<2, 2, 2, 2, 1, 2, 2>(g, stream);
 }

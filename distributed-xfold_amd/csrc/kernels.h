@@ -31,8 +31,18 @@ struct GemmArgs {
   // at [(m / 32, n / 32)][(m % 32, n % 32)], i.e. C is [(M/32)(N/32)][1024]:
   // the outer products of 32-channel rows, one contiguous 1024-vector per pair.
   int regroup32 = 0;
+  int split_k = 0;  // the K range may be summed in parts by several waves (another order of summation)
 };
 int launch_gemm_nt(const GemmArgs& g, hipStream_t stream);
+// af3_linear_forward and af3_batch_diffusion_self_attention_forward (api.hip) for callers inside the library that do
+// not mind the order in which the products sum K (GemmArgs::split_k)
+int run_linear(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int y_dtype, int64_t m, int n, int k, int mode,
+               float alpha, int sigmoid, const float* gate, int64_t gate_rows, int64_t gate_ld, const void* residual,
+               int res_dtype, int split_k, hipStream_t stream);
+int run_self_attention(const bf16_t* q_data, const float* key_mask, int64_t mask_batches, const float* nonbatched_bias,
+                       int bias_quad_major, const bf16_t* w_qkvg, const float* query_b, int num_head, void* out, int out_dtype,
+                       int64_t batch, int64_t seq, int channels, void* workspace, size_t workspace_bytes, int split_k,
+                       hipStream_t stream);
 // Which bias entries a launch reads.  Column c takes bias[c] when the epilogue is not segmented, or
 // when c lies in a segment whose op is SEG_BIAS_SCALE; the kernels read whole groups of entries
 // (gemm_nt_kernel up to 8 from a multiple of 8, the large tile 4 from a multiple of 4, the last

@@ -64,13 +64,18 @@ int single_update(const af3_pairformer_block& b, void* single, int dt, const flo
   const size_t ab = af3_batch_diffusion_self_attention_workspace_bytes(1, n, c);
   void* aw = w.take(ab);
   if (!w.ok) return AF3_ERR_WORKSPACE;
+  hipStream_t st = static_cast<hipStream_t>(s);
+  // The products here are a few hundred rows: their K range may be split between waves (nothing compares one
+  // sequence's bits with a batch's).
+  auto product = [&](const uint16_t* in, const uint16_t* wt, void* out, int out_dt, int n_out, int k, int mode, const void* res) {
+    return run_linear(in, wt, nullptr, out, out_dt, n, n_out, k, mode, 1.f, 0, nullptr, 0, 0, res, dt, 1, st);
+  };
   STEP(af3_layer_norm_forward(single, dt, x, n, c, b.sa_ln_w, b.sa_ln_b, nullptr, nullptr, 0, 0, s));
-  STEP(af3_batch_diffusion_self_attention_forward(x, mask, 1, logits, 0, b.sa_w_qkvg, b.sa_q_b, b.num_head, y, AF3_BF16, 1, n,
-                                                  c, aw, ab, s));
-  STEP(af3_linear_forward(y, b.sa_w_out, nullptr, single, dt, n, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, nullptr, 0, 0, single, dt, s));
+  STEP(run_self_attention(x, mask, 1, logits, 0, b.sa_w_qkvg, b.sa_q_b, b.num_head, y, AF3_BF16, 1, n, c, aw, ab, 1, st));
+  STEP(product(y, b.sa_w_out, single, dt, c, c, AF3_LINEAR_GATE_RES, single));
   STEP(af3_layer_norm_forward(single, dt, x, n, c, b.st_ln_w, b.st_ln_b, nullptr, nullptr, 0, 0, s));
-  STEP(af3_linear_forward(x, b.st_w1, nullptr, y, AF3_BF16, n, 2 * h, c, AF3_LINEAR_SWIGLU, 1.f, 0, nullptr, 0, 0, nullptr, 0, s));
-  return af3_linear_forward(y, b.st_w2, nullptr, single, dt, n, c, h, AF3_LINEAR_GATE_RES, 1.f, 0, nullptr, 0, 0, single, dt, s);
+  STEP(product(x, b.st_w1, y, AF3_BF16, 2 * h, c, AF3_LINEAR_SWIGLU, nullptr));
+  return product(y, b.st_w2, single, dt, c, h, AF3_LINEAR_GATE_RES, single);
 }
 
 }  // namespace

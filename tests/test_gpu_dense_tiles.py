@@ -1,7 +1,7 @@
 """GPU parity of the dense products below the 256x256-tile sizes, one case at the edges of every tile the launcher
-chooses from (32x32 with the K range split by four, 64x64 split by two and not, 64x128, 128x128, the element-wise form): first and last rows
-and columns alone in a tile, K shorter than a slab, K with a partial last slab, column counts that force element-wise
-stores; and the order of summation, which must not depend on the number of rows."""
+chooses from (32x32, 64x64, 64x128, 128x128, the element-wise form): first and last rows and columns alone in a tile,
+K shorter than a slab, K with a partial last slab, column counts that force element-wise stores; the order of
+summation, which must not depend on the number of rows; and the K split of the Pairformer's single track."""
 
 import pytest
 import torch
@@ -11,12 +11,13 @@ from oracle import af3_oracle as O
 pytestmark = pytest.mark.gpu
 
 SHAPES = [
-    (1, 8, 264), (33, 40, 312), (64, 384, 384), (97, 72, 1032), (161, 384, 1536),    # 32x32, K split by four
-    (387, 1536, 384), (1921, 768, 776), (130, 1984, 264),                             # 64x64, by two
-    (1, 8, 8), (12001, 136, 128), (3841, 768, 768), (129, 3072, 384), (70001, 64, 264),   # 64x64
+    (1, 8, 8), (33, 40, 320), (64, 384, 384), (97, 72, 1536), (500, 768, 128),        # 32x32
+    (387, 1536, 384), (65, 8200, 64), (12001, 64, 64), (1921, 768, 768),              # 64x64, four and three buffers
+    (3841, 768, 768), (129, 12352, 384), (70001, 64, 320),                            # 64x64, two buffers
+    (12001, 136, 120), (129, 3072, 392), (97, 72, 1032),                              # 64x64, K with a partial last slab
     (31, 3, 64), (97, 65, 200), (500, 765, 392),                                      # 64x64, element by element
-    (1921, 3080, 136), (8001, 384, 1032), (70, 70000, 72), (180001, 128, 40),         # 64x128
-    (20001, 1032, 104),                      # 128x128 (odd columns keep it off the large tile)
+    (1921, 3080, 128), (8001, 384, 1024), (70, 70016, 64), (180001, 128, 64),         # 64x128
+    (20001, 1032, 128),                      # 128x128 (odd columns keep it off the large tile)
 ]
 
 
@@ -72,3 +73,29 @@ def test_rows_do_not_change_with_the_batch(gpu_pkg, n, k):
     want = gpu_pkg.ops.linear(x, w, mode=gpu_pkg.lib.LINEAR_GATE_RES)
     for m in (1, 100, 500, 1900, 3840):
         assert torch.equal(gpu_pkg.ops.linear(x[:m], w, mode=gpu_pkg.lib.LINEAR_GATE_RES), want[:m]), m
+
+
+@pytest.mark.parametrize("n,c", [(1, 384), (33, 384), (130, 384), (700, 384), (1000, 256)])
+def test_single_track_products(gpu_pkg, n, c):
+    """The single track of a Pairformer block, whose products may split K between waves (by four, eight and two),
+    against the same modules run one by one, whose products do not."""
+    print(f"dense tiles: single track n={n} c={c}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n + c)
+    with torch.device("cuda"):
+        blk = gpu_pkg.nn.PairformerBlock(c_single=c, n_heads=c // 32)
+    with torch.no_grad():
+        for p in blk.parameters():
+            p.normal_(0.0, 0.05, generator=g)
+    blk.invalidate()
+    pair = torch.randn(n, n, 128, generator=g, device="cuda").bfloat16()
+    single = torch.randn(n, c, generator=g, device="cuda")
+    mask = torch.ones(n, device="cuda")
+    ones = torch.ones(n, n, device="cuda")
+    out_pair, got = blk(pair.clone(), ones, single.clone(), mask)
+    p = blk.packed()
+    logits = gpu_pkg.ops.pair_logits(out_pair, p["ln_w"], p["ln_b"], p["w_logits"], blk.n_heads)
+    want = single.clone()
+    blk.single_attention_.run(want, mask, logits, None, residual=True)
+    blk.single_transition.run(want, residual=True)
+    upd, ref = got - single, want - single
+    assert float((upd - ref).norm() / ref.norm()) < 3e-3
