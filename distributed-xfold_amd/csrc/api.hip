@@ -93,7 +93,7 @@ static int contraction(const GemmArgs& g, hipStream_t s) {
 
 size_t af3_triangle_multiplication_workspace_bytes(int64_t n) {
   if (n <= 0) return 0;
-  return 3 * align_up((size_t)C_PAIR * n * pad8(n) * sizeof(bf16_t), 256);
+  return 3 * align_up((size_t)C_PAIR * tri_plane(n) * sizeof(bf16_t), 256);
 }
 
 static int triangle_multiplication_impl(
@@ -107,11 +107,11 @@ static int triangle_multiplication_impl(
   if (valid_channels < 8 || valid_channels > C_PAIR) return AF3_ERR_BAD_ARG;
   if (bad_dtype(io_dtype) || n <= 0 || n > 8192 || (equation_flag != 0 && equation_flag != 1)) return AF3_ERR_BAD_ARG;
   if (misaligned(act) || misaligned(out) || misaligned(mask)) return AF3_ERR_BAD_ARG;
-  const int64_t np = pad8(n);
+  const int64_t np = pad8(n), plane = tri_plane(n);
   Carver ws(workspace, workspace_bytes);
-  bf16_t* a_buf = ws.take<bf16_t>((size_t)C_PAIR * n * np);
-  bf16_t* b_buf = ws.take<bf16_t>((size_t)C_PAIR * n * np);
-  bf16_t* t_buf = ws.take<bf16_t>((size_t)C_PAIR * n * np);
+  bf16_t* a_buf = ws.take<bf16_t>((size_t)C_PAIR * plane);
+  bf16_t* b_buf = ws.take<bf16_t>((size_t)C_PAIR * plane);
+  bf16_t* t_buf = ws.take<bf16_t>((size_t)C_PAIR * plane);
   if (!ws.ok) return AF3_ERR_WORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
 
@@ -123,7 +123,7 @@ static int triangle_multiplication_impl(
   a.outgoing = equation_flag == 0; a.residual = residual != 0;
   a.ln_in_w = ln_in_w; a.ln_in_b = ln_in_b; a.ln_c_w = ln_c_w; a.ln_c_b = ln_c_b;
   a.w_pg = w_proj_gate; a.w_gl = w_gl; a.w_out = w_out;
-  a.a_buf = a_buf; a.b_buf = b_buf; a.t_buf = t_buf;
+  a.a_buf = a_buf; a.b_buf = b_buf; a.t_buf = t_buf; a.plane = plane;
   int rc = launch_trimul_prologue(a, s);
   if (rc) return rc;
 
@@ -136,7 +136,7 @@ static int triangle_multiplication_impl(
   // (the hidden layer has as many channels as the pair tensor: the padded ones are zero and are left out)
   g.M = g.N = (int)n; g.K = (int)np; g.batch = valid_channels;
   g.lda = g.ldb = g.ldc = np;
-  g.sA = g.sB = g.sC = n * np;
+  g.sA = g.sB = g.sC = plane;
   rc = contraction(g, s);
   if (rc) return rc;
   return launch_trimul_epilogue(a, s);

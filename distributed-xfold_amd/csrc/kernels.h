@@ -145,9 +145,12 @@ struct TriMulArgs {
   const bf16_t* w_pg = nullptr;   // [4][128][128]: per chunk 64 projection rows + 64 gate rows
   const bf16_t* w_gl = nullptr;   // [128][128] gating_linear
   const bf16_t* w_out = nullptr;  // [128][128] output_projection
-  bf16_t *a_buf = nullptr, *b_buf = nullptr;  // [128][N][Np] channel-major operands
-  const bf16_t* t_buf = nullptr;              // [128][N][Np] contraction result
+  // channel-major planes [N][Np], `plane` elements apart (tri_plane: whole tiles of 128 positions)
+  bf16_t *a_buf = nullptr, *b_buf = nullptr;  // 128 planes each: operands
+  const bf16_t* t_buf = nullptr;              // 128 planes: contraction result
+  int64_t plane = 0;
 };
+inline int64_t tri_plane(int64_t n) { return (n * ((n + 7) / 8 * 8) + 127) / 128 * 128; }
 int launch_trimul_prologue(const TriMulArgs& a, hipStream_t s);
 int launch_trimul_epilogue(const TriMulArgs& a, hipStream_t s);
 

@@ -1,8 +1,8 @@
 // Row-tile kernels of the 128-channel pair path.
 //
 // Every kernel here walks the [N, N, 128] pair tensor in tiles of 128
-// consecutive positions along one axis (a row segment, or a column segment for
-// the transposed operators), keeps the tile's LayerNorm-ed activations in LDS /
+// consecutive positions along one axis (rows, or columns for the transposed
+// operators, laid end to end), keeps the tile's LayerNorm-ed activations in LDS /
 // registers as bf16 MFMA fragments and multiplies them with 128x128 weight
 // chunks streamed through LDS.  They are HBM-bound (one read of the pair tensor,
 // one write of each product) except the SwiGLU transition, which is MFMA-bound.
@@ -30,7 +30,7 @@ namespace {
 // ============================================================================
 // triangle multiplication, prologue
 // ============================================================================
-template <typename TIO>
+template <typename TIO, bool CROSS>
 __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
   // 34.8 KB + 17.4 KB + 0.5 KB of LDS and at most 168 registers: three workgroups per CU.
   //
@@ -50,7 +50,11 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // outgoing: tiles run along k for fixed i (a[c][i][k]); incoming: along k for
   // fixed j, i.e. a column segment of the pair tensor (a'[c][j][k] = a[k][j][c]).
-  const Tile t = make_tile(a.N, !a.outgoing);
+  // (flat over rows of Np positions: a 16-byte piece of a channel's plane is position l0 + 8 pc of it, whatever the row;
+  // the planes have room for the last tile's positions past the end)
+  const auto t = make_tile<CROSS>(a.N, a.Np, !a.outgoing);
+  // a thread's 16-byte pieces, from the first of 16 channels' planes on (one 32-bit offset: at most 2^31)
+  const uint32_t lane_out = ((uint32_t)(tid >> 4) * (uint32_t)a.plane + (tid & 15) * 8) * 2u;
   const TIO* x = reinterpret_cast<const TIO*>(a.pair);
 
   // Weight chunks in memory: [P(64 ch) | G(64 ch)] for a ch 0-63, a ch 64-127, b ch 0-63, b ch 64-127.
@@ -78,9 +82,8 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
     // whatever the activations are.  Write the zeros and skip the rest.
     const u32x4 z = {0, 0, 0, 0};
     for (int idx = tid; idx < 2 * C * 16; idx += 256) {
-      const int op = idx >> 11, ch = (idx >> 4) & (C - 1), r = t.r0 + (idx & 15) * 8;
-      if (r < a.Np)
-        *reinterpret_cast<u32x4*>((op ? a.b_buf : a.a_buf) + ((int64_t)ch * a.N + t.o) * a.Np + r) = z;
+      const int op = idx >> 11, ch = (idx >> 4) & (C - 1);
+      *reinterpret_cast<u32x4*>((op ? a.b_buf : a.a_buf) + ch * a.plane + t.l0 + (idx & 15) * 8) = z;
     }
     return;
   }
@@ -157,13 +160,10 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
         }
         if (S >= 2) {
           constexpr int SO = S >= 2 ? S - 2 : 0;
-          bf16_t* dst = (SO < 4 ? a.a_buf : a.b_buf) + ((int64_t)(((SO >> 1) & 1) * 64 + (SO & 1) * 32) * a.N + t.o) * a.Np;
+          bf16_t* dst = (SO < 4 ? a.a_buf : a.b_buf) + (((SO >> 1) & 1) * 64 + (SO & 1) * 32) * a.plane + t.l0;
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const int idx = tid + 256 * i, c2 = idx >> 4, pc = idx & 15;
-            const int r = t.r0 + pc * 8;
-            if (r < a.Np) *reinterpret_cast<u32x4*>(dst + (int64_t)c2 * a.N * a.Np + r) = outv[i];
-          }
+          for (int i = 0; i < 2; ++i)
+            *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(dst + 16 * i * a.plane) + lane_out) = outv[i];
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -181,22 +181,18 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
   step(std::integral_constant<int, 8>{}, accA, accB);  // gating of step 7, results of step 6
   {
     // results of step 7
-    bf16_t* dst = a.b_buf + ((int64_t)(64 + 32) * a.N + t.o) * a.Np;
+    bf16_t* dst = a.b_buf + (64 + 32) * a.plane + t.l0;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int idx = tid + 256 * i, c2 = idx >> 4, pc = idx & 15;
-      const int r = t.r0 + pc * 8;
-      if (r < a.Np)
-        *reinterpret_cast<u32x4*>(dst + (int64_t)c2 * a.N * a.Np + r) =
-            *reinterpret_cast<const u32x4*>(sS1 + c2 * LDX + pc * 8);
-    }
+    for (int i = 0; i < 2; ++i)
+      *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(dst + 16 * i * a.plane) + lane_out) =
+          *reinterpret_cast<const u32x4*>(sS1 + (16 * i + (tid >> 4)) * LDX + (tid & 15) * 8);
   }
 }
 
 // ============================================================================
 // triangle multiplication, epilogue
 // ============================================================================
-template <typename TIO>
+template <typename TIO, bool CROSS>
 __global__ __launch_bounds__(256, 2) void trimul_epilogue_kernel(TriMulArgs a) {
   __shared__ __attribute__((aligned(16))) bf16_t smem[2 * TM * LDX];
   bf16_t* sX = smem;
@@ -205,22 +201,21 @@ __global__ __launch_bounds__(256, 2) void trimul_epilogue_kernel(TriMulArgs a) {
   static_assert(TM * LDS_F * 4 <= 2 * TM * LDX * 2, "staging tile must fit");
   __shared__ __attribute__((aligned(16))) float sP[2 * C];  // center LayerNorm weight | bias
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const Tile t = make_tile(a.N, false);
+  const auto t = make_tile<CROSS>(a.N, a.Np, false);
   const TIO* x = reinterpret_cast<const TIO*>(a.pair);
 
   // everything this tile needs from memory is requested up front
   WChunkRegs wr;
   wr.load(a.w_gl, tid);
-  u32x4 rt[8];  // contraction result t[c][i][j0 + 8 pc ..], c = 16 it + tid / 16
+  u32x4 rt[8];  // contraction result, positions l0 + 8 pc .. of channel c = 16 it + tid / 16
   const int pc = tid & 15, crow = tid >> 4;
-  // (a chunk that starts past the row's end re-reads the tile's first one; its pixels are zeroed later)
-  const int j_chunk = t.r0 + pc * 8 < a.Np ? t.r0 + pc * 8 : t.r0;
+  // (positions past the last row hold whatever the workspace held; their pixels are zeroed later)
 #pragma unroll
   for (int it = 0; it < 8; ++it) {
     // (channels past the valid ones were not contracted: their rows hold whatever the workspace held;
     // the load goes to a valid channel's row instead and is replaced by zeros below)
     const int c = it * 16 + crow;
-    rt[it] = *reinterpret_cast<const u32x4*>(a.t_buf + ((int64_t)(c < a.valid_c ? c : 0) * a.N + t.o) * a.Np + j_chunk);
+    rt[it] = *reinterpret_cast<const u32x4*>(a.t_buf + (c < a.valid_c ? c : 0) * a.plane + t.l0 + pc * 8);
   }
 
   // 1. output gate from the LayerNorm-ed input: sigmoid(LN(x) Wgl^T), T form, kept in registers
@@ -307,13 +302,13 @@ __global__ __launch_bounds__(256, 2) void trimul_epilogue_kernel(TriMulArgs a) {
 // ============================================================================
 // triangle attention: projections
 // ============================================================================
-template <typename TIO>
+template <typename TIO, bool CROSS>
 __global__ __launch_bounds__(256, 2) void attn_proj_kernel(AttnProjArgs a) {
   __shared__ __attribute__((aligned(16))) bf16_t sX[TM * LDX];
   __shared__ __attribute__((aligned(16))) bf16_t sW[TM * LDX];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // (b, s) = (o, r): for the transposed operator a tile is a column segment
-  const Tile t = make_tile(a.N, a.transpose != 0);
+  const auto t = make_tile<CROSS>(a.N, a.N, a.transpose != 0);
   const TIO* x = reinterpret_cast<const TIO*>(a.pair);
   load_ln_tile<TIO>(x, t, a.ln_w, a.ln_b, sX, tid, a.skip_ln != 0, a.lw.inv_c, a.lw.pad);
   lds_barrier();
@@ -345,7 +340,7 @@ __global__ __launch_bounds__(256, 2) void attn_proj_kernel(AttnProjArgs a) {
     for (int it = 0; it < 8; ++it) {
       const int p = it * 16 + prow;
       if (t.valid(p))
-        *reinterpret_cast<u32x4*>(a.out_main + ((int64_t)t.o * a.N + t.r0 + p) * a.ld_main + chunk * C + ck * 8) =
+        *reinterpret_cast<u32x4*>(a.out_main + (int64_t)(t.l0 + p) * a.ld_main + chunk * C + ck * 8) =
             *reinterpret_cast<const u32x4*>(sW + p * LDX + ck * 8);
     }
     lds_barrier();
@@ -387,14 +382,14 @@ __global__ __launch_bounds__(256, 2) void attn_proj_kernel(AttnProjArgs a) {
 // holds channel swap23(rho): bits 2 and 3 exchanged) a lane-half's registers 8 a .. 8 a + 7 of tile nt are
 // the eight consecutive channels 32 nt + 16 a + 8 hh .. of its pixel: exactly the B fragment of k-step
 // 2 nt + a of the output projection, so gate and attention output meet register by register.
-template <typename TIO>
+template <typename TIO, bool CROSS>
 __global__ __launch_bounds__(256, 2) void attn_out_kernel(AttnOutArgs a) {
   __shared__ __attribute__((aligned(16))) bf16_t smem[2 * TM * LDX];
   bf16_t* sX = smem;
   bf16_t* sW = smem + TM * LDX;
   float* sS = reinterpret_cast<float*>(smem);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const Tile t = make_tile(a.N, a.transpose != 0);  // where the result lands in the pair tensor
+  const auto t = make_tile<CROSS>(a.N, a.N, a.transpose != 0);  // where the result lands in the pair tensor
   // Loads are unconditional (rows past the end re-read a valid one and are zeroed / skipped later).
   // The attention output is requested once the gate's MFMAs are issued (its 32 registers would not
   // fit beside them), and the pair rows are read a second time, out of the cache, for the residual:
@@ -416,7 +411,7 @@ __global__ __launch_bounds__(256, 2) void attn_out_kernel(AttnOutArgs a) {
 #pragma unroll
   for (int it = 0; it < 8; ++it) {
     const int p = it * 16 + prow;
-    og[it] = *reinterpret_cast<const u32x4*>(a.og + ((int64_t)t.o * a.N + t.r0 + (t.valid(p) ? p : 0)) * a.ld_og + ck * 8);
+    og[it] = *reinterpret_cast<const u32x4*>(a.og + (int64_t)(t.l0 + (t.valid(p) ? p : 0)) * a.ld_og + ck * 8);
   }
   wr.load<false>(a.w_out, tid);
 #pragma unroll
@@ -501,7 +496,7 @@ __global__ __launch_bounds__(256, 2) void transition_kernel(TransitionArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 31, hh = lane >> 5;
-  const Tile t = make_tile(a.N, false);
+  const auto t = make_tile_1d(a.N);
   const TIO* x = reinterpret_cast<const TIO*>(a.x);
   const int n_slabs = a.hidden / 32;
 
@@ -664,12 +659,12 @@ __global__ __launch_bounds__(256, 2) void pair_cond_init_kernel(PairCondInitArgs
   float* sS = reinterpret_cast<float*>(smem);
   __shared__ float sRstd[TM], sMeanRstd[TM];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const Tile t = make_tile(a.N, false);
+  const auto t = make_tile_in_row(a.N);
   const TIO* x = reinterpret_cast<const TIO*>(a.pair);
   using E = Elem<TIO>;
   constexpr int NB = E::kBatch;
   const int chunk = tid & 15, prow = tid >> 4;
-  const int i = t.o;
+  const int i = t.o0;
   const int ent_i = a.entity_id[i];
   const float inv_c = 1.f / (float)(C + a.n_rel);
 
@@ -753,31 +748,38 @@ __global__ __launch_bounds__(256, 2) void pair_cond_init_kernel(PairCondInitArgs
 }
 
 template <typename K, typename A>
-int launch_tiles(K kern, const A& a, int64_t n_outer, int N, hipStream_t stream) {
-  const int64_t tiles = n_outer * ((N + TM - 1) / TM);
+int launch_tiles(K kern, const A& a, int64_t positions, hipStream_t stream) {
+  const int64_t tiles = (positions + TM - 1) / TM;
   if (tiles <= 0 || tiles > 0x7fffffff) return AF3_ERR_BAD_ARG;
   hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(256), 0, stream, a);
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
+
+// the instance of a tile kernel for the residual stream's type and for tiles that cross rows or do not
+#define LAUNCH_TILES(KERN, CROSS, POSITIONS)                                                                      \
+  do {                                                                                                            \
+    const int64_t n_ = (POSITIONS);                                                                               \
+    if (CROSS)                                                                                                    \
+      return a.io_f32 ? launch_tiles(KERN<float, true>, a, n_, s) : launch_tiles(KERN<bf16_t, true>, a, n_, s);   \
+    return a.io_f32 ? launch_tiles(KERN<float, false>, a, n_, s) : launch_tiles(KERN<bf16_t, false>, a, n_, s);   \
+  } while (0)
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
 
 int launch_trimul_prologue(const TriMulArgs& a, hipStream_t s) {
-  if (a.N <= 0 || a.Np < a.N || (a.Np & 7) || !a.pair || !a.a_buf || !a.b_buf || !a.w_pg) return AF3_ERR_BAD_ARG;
+  if (a.N <= 0 || a.Np < a.N || (a.Np & 7) || a.plane < tri_plane(a.N) || !a.pair || !a.a_buf || !a.b_buf || !a.w_pg) return AF3_ERR_BAD_ARG;
   if (!aligned16(a.pair) || !aligned16(a.a_buf) || !aligned16(a.b_buf) || !aligned16(a.w_pg)) return AF3_ERR_BAD_ARG;
-  return a.io_f32 ? launch_tiles(trimul_prologue_kernel<float>, a, a.N, a.N, s)
-                  : launch_tiles(trimul_prologue_kernel<bf16_t>, a, a.N, a.N, s);
+  LAUNCH_TILES(trimul_prologue_kernel, tile_crosses(a.Np), (int64_t)a.N * a.Np);
 }
 int launch_trimul_epilogue(const TriMulArgs& a, hipStream_t s) {
-  if (a.N <= 0 || a.Np < a.N || (a.Np & 7) || !a.pair || !a.t_buf || !a.out || !a.w_gl || !a.w_out ||
+  if (a.N <= 0 || a.Np < a.N || (a.Np & 7) || a.plane < tri_plane(a.N) || !a.pair || !a.t_buf || !a.out || !a.w_gl || !a.w_out ||
       !a.ln_c_w || !a.ln_c_b)
     return AF3_ERR_BAD_ARG;
   if (!aligned16(a.pair) || !aligned16(a.t_buf) || !aligned16(a.out) || !aligned16(a.w_gl) || !aligned16(a.w_out))
     return AF3_ERR_BAD_ARG;
-  return a.io_f32 ? launch_tiles(trimul_epilogue_kernel<float>, a, a.N, a.N, s)
-                  : launch_tiles(trimul_epilogue_kernel<bf16_t>, a, a.N, a.N, s);
+  LAUNCH_TILES(trimul_epilogue_kernel, tile_crosses(a.Np), (int64_t)a.N * a.Np);
 }
 int launch_attn_proj(const AttnProjArgs& a, hipStream_t s) {
   if (a.N <= 0 || !a.pair || a.n_chunks < 0 || a.n_chunks > 4 || a.n_bias < 0) return AF3_ERR_BAD_ARG;
@@ -785,16 +787,14 @@ int launch_attn_proj(const AttnProjArgs& a, hipStream_t s) {
   if (a.n_bias > 0 && (!a.w_bias || (!a.out_bias && !a.out_bias_bf16))) return AF3_ERR_BAD_ARG;
   if (a.out_bias_bf16 && a.ld_bias < a.N) return AF3_ERR_BAD_ARG;
   if (!aligned16(a.pair) || !aligned16(a.w_main) || !aligned16(a.out_main) || !aligned16(a.w_bias)) return AF3_ERR_BAD_ARG;
-  return a.io_f32 ? launch_tiles(attn_proj_kernel<float>, a, a.N, a.N, s)
-                  : launch_tiles(attn_proj_kernel<bf16_t>, a, a.N, a.N, s);
+  LAUNCH_TILES(attn_proj_kernel, tile_crosses(a.N), (int64_t)a.N * a.N);
 }
 int launch_attn_out(const AttnOutArgs& a, hipStream_t s) {
   if (a.N <= 0 || !a.og || !a.w_out || !a.w_gate || !a.out || (a.ld_og & 7) || !a.pair) return AF3_ERR_BAD_ARG;
   if ((a.ln_w == nullptr) != (a.ln_b == nullptr) || (a.skip_ln == 0) != (a.ln_w != nullptr)) return AF3_ERR_BAD_ARG;
   if (!aligned16(a.og) || !aligned16(a.w_out) || !aligned16(a.w_gate) || !aligned16(a.out) || !aligned16(a.pair))
     return AF3_ERR_BAD_ARG;
-  return a.io_f32 ? launch_tiles(attn_out_kernel<float>, a, a.N, a.N, s)
-                  : launch_tiles(attn_out_kernel<bf16_t>, a, a.N, a.N, s);
+  LAUNCH_TILES(attn_out_kernel, tile_crosses(a.N), (int64_t)a.N * a.N);
 }
 int launch_pair_cond_init(const PairCondInitArgs& a, hipStream_t s) {
   if (a.N <= 0 || !a.pair || !a.out || !a.w_pair || !a.ln_w || !a.g_hot || !a.g_sum || !a.asym_id || !a.residue_index ||
@@ -804,13 +804,13 @@ int launch_pair_cond_init(const PairCondInitArgs& a, hipStream_t s) {
   if (!aligned16(a.pair) || !aligned16(a.out) || !aligned16(a.w_pair) || !aligned16(a.g_hot) || !aligned16(a.g_sum) ||
       !aligned16(a.ln_w))
     return AF3_ERR_BAD_ARG;
-  return a.io_f32 ? launch_tiles(pair_cond_init_kernel<float>, a, a.N, a.N, s)
-                  : launch_tiles(pair_cond_init_kernel<bf16_t>, a, a.N, a.N, s);
+  return a.io_f32 ? launch_tiles(pair_cond_init_kernel<float>, a, (int64_t)a.N * ((a.N + TM - 1) / TM) * TM, s)
+                  : launch_tiles(pair_cond_init_kernel<bf16_t>, a, (int64_t)a.N * ((a.N + TM - 1) / TM) * TM, s);
 }
 int launch_transition(const TransitionArgs& a, hipStream_t s) {
   // x is [rows][128]; handled as `rows` positions in one long row
   if (a.N <= 0 || !a.x || !a.out || !a.w1 || !a.w2 || a.hidden <= 0 || (a.hidden & 63)) return AF3_ERR_BAD_ARG;
   if (!aligned16(a.x) || !aligned16(a.out) || !aligned16(a.w1) || !aligned16(a.w2)) return AF3_ERR_BAD_ARG;
-  return a.io_f32 ? launch_tiles(transition_kernel<float>, a, 1, a.N, s)
-                  : launch_tiles(transition_kernel<bf16_t>, a, 1, a.N, s);
+  return a.io_f32 ? launch_tiles(transition_kernel<float>, a, a.N, s)
+                  : launch_tiles(transition_kernel<bf16_t>, a, a.N, s);
 }

@@ -12,26 +12,86 @@ constexpr int TM = 128;   // positions per tile
 constexpr int LDX = 136;  // LDS row stride (bf16) for [row][128] tiles: 272 B
 constexpr int LDS_F = 132;  // LDS row stride (fp32) for staged output tiles
 
-struct Tile {
-  int o, r0, N;
-  int64_t so, sr;  // pixel index = o * so + r * sr
-  __device__ __forceinline__ int64_t pix(int p) const { return (int64_t)o * so + (int64_t)(r0 + p) * sr; }
-  __device__ __forceinline__ bool valid(int p) const { return r0 + p < N; }
+// A tile is TM consecutive positions of the operator's frame laid out flat, rows o of W positions each: W = N, or N
+// rounded up to what the kernel's channel-major planes are padded to (positions N .. W - 1 of a row are padding).
+// A tile runs on from one row into the next, so that a row length that is no multiple of TM costs no partly filled
+// tile per row (at 387 tokens a quarter, at 160 three eighths of the positions computed).  Position (o, r) is pixel
+// o * so + r * sr of the pair tensor.
+// CROSS: false where W is a multiple of TM (or there is one row): the row is the workgroup's, and the indexing costs
+// nothing.
+template <bool CROSS>
+struct TileT {
+  int l0;          // flat index of the first position
+  int o0, r0;      // its row and place in the row
+  int N, W;
+  uint32_t magic;  // CROSS: ceil(2^32 / W); v / W = umulhi(v, magic) for v < W + TM, as W (W + TM) < 2^32
+  int64_t so, sr;
+  __device__ __forceinline__ void at(int p, int* o, int* r) const {
+    *o = o0;
+    *r = r0 + p;
+    if constexpr (CROSS) {
+      const int q = (int)__umulhi((uint32_t)*r, magic);
+      *o += q;
+      *r -= q * W;
+    }
+  }
+  __device__ __forceinline__ bool valid(int p) const {
+    int o, r;
+    at(p, &o, &r);
+    return r < N && (!CROSS || o < N);
+  }
+  // pixel of position p; of one that is not valid, that of some valid position
+  __device__ __forceinline__ int64_t pix(int p) const {
+    int o, r;
+    at(p, &o, &r);
+    if constexpr (CROSS) return r < N && o < N ? (uint32_t)o * (uint32_t)so + (uint32_t)r * (uint32_t)sr : 0u;
+    return (int64_t)o * so + (int64_t)(r < N ? r : r0) * sr;
+  }
+  // every position is valid (uniform over the workgroup; rows that are crossed are left to the per-position test)
+  __device__ __forceinline__ bool full() const { return r0 + TM <= N; }
 };
 
 // `reverse`: walk the tiles from the last to the first.  A kernel that reads
 // what the previous kernel has just written (and whose output the next kernel
 // starts reading from the other end) finds the most recently written part
 // still in the last-level cache when it starts there.
-__device__ __forceinline__ Tile make_tile(int N, bool column_mode, bool reverse = false) {
-  const int tiles_r = (N + TM - 1) / TM;
-  Tile t;
-  t.N = N;
+template <bool CROSS>
+__device__ __forceinline__ TileT<CROSS> make_tile(int N, int W, bool column_mode, bool reverse = false) {
+  TileT<CROSS> t;
   const unsigned bid = reverse ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
-  t.o = bid / tiles_r;
-  t.r0 = (bid % tiles_r) * TM;
+  t.N = N;
+  t.W = W;
+  // (the divisions go through the vector unit; say again that the results are uniform)
+  const uint32_t o0 = __builtin_amdgcn_readfirstlane(bid * TM / (uint32_t)W);
+  t.l0 = (int)(bid * TM);
+  t.o0 = (int)o0;
+  t.r0 = t.l0 - (int)o0 * W;
+  t.magic = W == 1 ? 1u : __builtin_amdgcn_readfirstlane(0xffffffffu / (uint32_t)W) + 1u;  // (W = 1: one pixel, position 0)
   t.so = column_mode ? 1 : N;
   t.sr = column_mode ? N : 1;
+  return t;
+}
+inline bool tile_crosses(int64_t W) { return W % TM != 0; }
+// One row of n positions (any count).
+__device__ __forceinline__ TileT<false> make_tile_1d(int n) {
+  TileT<false> t;
+  t.N = t.W = n;
+  t.l0 = t.r0 = (int)blockIdx.x * TM;
+  t.o0 = 0;
+  t.so = 0;
+  t.sr = 1;
+  return t;
+}
+// A piece of one row: tiles do not cross rows (the kernel takes per-row values from o0).
+__device__ __forceinline__ TileT<false> make_tile_in_row(int N) {
+  const int tiles_r = (N + TM - 1) / TM;
+  TileT<false> t;
+  t.N = t.W = N;
+  t.o0 = blockIdx.x / tiles_r;
+  t.r0 = (blockIdx.x % tiles_r) * TM;
+  t.l0 = t.o0 * N + t.r0;
+  t.so = N;
+  t.sr = 1;
   return t;
 }
 
@@ -99,10 +159,10 @@ __device__ __forceinline__ u32x4 ln_pixel8(const typename Elem<TIO>::Raw& raw, c
 // Thread (prow = tid / 16, chunk = tid % 16) handles channels 8*chunk..+7 of
 // pixels prow, prow + 16, ...; 16 lanes cooperate on one pixel's statistics.
 // Out-of-range pixels become zero rows.  The loads of a batch of pixels are
-// unconditional (an out-of-range pixel re-reads the tile's first one) and all
+// unconditional (an out-of-range position re-reads some valid pixel) and all
 // issued before any value is converted: a load under a lane mask, or one whose
 // value is touched at once, costs a full memory round trip per pixel.
-template <typename TIO>
+template <typename TIO, typename Tile>
 __device__ __forceinline__ void load_ln_tile(const TIO* x, const Tile& t, const float* lnw,
                                              const float* lnb, bf16_t* sX, int tid, bool skip_ln = false,
                                              float inv_c = 1.f / C, float pad = 0.f) {
@@ -112,14 +172,14 @@ __device__ __forceinline__ void load_ln_tile(const TIO* x, const Tile& t, const 
   float w[8], b[8];
   load_param8(lnw ? lnw + chunk * 8 : nullptr, 1.f, w);
   load_param8(lnb ? lnb + chunk * 8 : nullptr, 0.f, b);
-  const bool full = t.r0 + TM <= t.N;  // every pixel of the tile is in range (uniform over the workgroup)
+  const bool full = t.full();
 #pragma unroll
   for (int base = 0; base < 8; base += NB) {
     typename E::Raw raw[NB];
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       const int p = (base + i) * 16 + prow;
-      raw[i] = E::load_raw(x + t.pix(t.valid(p) ? p : 0) * C + chunk * 8);
+      raw[i] = E::load_raw(x + t.pix(p) * C + chunk * 8);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
@@ -232,7 +292,7 @@ __device__ __forceinline__ void stage_t_bf16(const f32x16* acc, bf16_t* sS, int 
 // The residual rows of a batch of pixels are loaded (unconditionally, from a
 // clamped pixel) before the batch's first store: out may alias res, so the
 // compiler cannot move a load above a store on its own.
-template <typename TIO>
+template <typename TIO, typename Tile>
 __device__ __forceinline__ void store_tile_f32(const float* sS, const Tile& t, TIO* out, const TIO* res, int tid) {
   using E = Elem<TIO>;
   constexpr int NB = E::kBatch;
@@ -244,7 +304,7 @@ __device__ __forceinline__ void store_tile_f32(const float* sS, const Tile& t, T
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
         const int p = (base + i) * 16 + prow;
-        raw[i] = E::load_raw(res + t.pix(t.valid(p) ? p : 0) * C + chunk * 8);
+        raw[i] = E::load_raw(res + t.pix(p) * C + chunk * 8);
       }
     }
 #pragma unroll

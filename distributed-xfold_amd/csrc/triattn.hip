@@ -18,18 +18,19 @@ constexpr int H = 4, D = 32;
 // projections: LN -> q (scaled), k (position-major) and v (channel-major),
 // + pair-bias heads
 // ============================================================================
-template <typename TIO>
+template <typename TIO, bool CROSS>
 __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a) {
   // 34.8 KB + 17.4 KB of LDS and at most 168 registers: three workgroups per CU.  The kernel is a chain of
   // short dependent phases (load, LayerNorm, MFMA, stage, store), so what it needs is company.
   __shared__ __attribute__((aligned(16))) bf16_t sX[TM * LDX];  // LN tile, then staging
   __shared__ __attribute__((aligned(16))) bf16_t sW[64 * LDX];  // 64 weight rows at a time
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // (b, s) = (o, r): for the transposed operator a tile is a column segment
+  // (b, s) = (o, r), flat over rows of ldn positions (the row length of V transposed, a multiple of 16: a tile starts on
+  // a group of 16 keys); for the transposed operator the rows are columns of the pair tensor.
   // last tile first: the pair tensor was written front to back by the operator
   // before this one, and the attention core that follows starts with row 0,
   // which is then the freshest part of q / k / v (measured: 1.4 % of the block)
-  const Tile t = make_tile(a.N, a.transpose != 0, true);
+  const auto t = make_tile<CROSS>(a.N, (int)a.ldn, a.transpose != 0, true);
   const TIO* x = reinterpret_cast<const TIO*>(a.pair);
   // Step s = 2 * chunk + half: weight rows 64 half .. + 63 of chunk s / 2 (chunks q, k, v of w_qkvg),
   // four 16-byte pieces per thread; the 32 (padded) pair-bias rows ride in the same registers.
@@ -64,7 +65,6 @@ __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a)
   load_x_frags(sX, wave, lane, xf);
   lds_barrier();  // sX is free from here on: it becomes the staging tile
 
-  const int64_t bh0 = (int64_t)t.o * H;  // (b * H + h) for h = 0
   // v takes the channel-major route.  The step index is a compile-time constant of the body: with a
   // run-time index the compiler evaluates the sigmoid for every chunk and selects.
   auto do_step = [&](auto step_c) {
@@ -123,9 +123,10 @@ __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a)
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int idx = tid + 256 * i, ch = idx >> 4, pc = idx & 15;
-          const int r = t.r0 + pc * 8;
-          if (r < a.ldn)
-            *reinterpret_cast<u32x4*>(a.vt + (bh0 * D + ch) * a.ldn + r) =
+          int o, r;
+          t.at(pc * 8, &o, &r);
+          if (o < a.N)
+            *reinterpret_cast<u32x4*>(a.vt + ((int64_t)o * H * D + ch) * a.ldn + r) =
                 *reinterpret_cast<const u32x4*>(sX + ch * LDX + pc * 8);
         }
       } else {
@@ -135,8 +136,10 @@ __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a)
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
           const int p = it * 16 + prow;
-          if (t.valid(p))
-            *reinterpret_cast<u32x4*>(plane + ((bh0 + h) * a.N + t.r0 + p) * D + part * 8) =
+          int o, r;
+          t.at(p, &o, &r);
+          if (r < a.N && o < a.N)
+            *reinterpret_cast<u32x4*>(plane + (((int64_t)o * H + h) * a.N + r) * D + part * 8) =
                 *reinterpret_cast<const u32x4*>(sX + p * LDX + ck * 8);
         }
       }
@@ -157,23 +160,18 @@ __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a)
     mfma_chunk<true, 1>(xf, sW, lane, acc);
     if ((lane >> 5) == 0) {  // heads 0..3 are accumulator rows 0..3: registers 0..3 of the low half
       const int p = wave * 32 + lane;
-      const int r = t.r0 + p;
-      const int kpad = (int)tri_bias_ktiles(a.N) * 64;  // keys N..kpad-1 are padding: zero bias
-      if (!a.transpose) {
-        // q = o, k = r
-        if (r < kpad) {
+      int o, r;
+      t.at(p, &o, &r);
+      if (r < a.N && o < a.N) {
+        const int q = a.transpose ? r : o, k = a.transpose ? o : r;
 #pragma unroll
-          for (int h = 0; h < H; ++h)
-            a.bias[tri_bias_offset(a.N, h, t.o, r)] = f2h_sat(t.valid(p) ? acc[0][h] * a.bias_scale : 0.f);
-        }
-      } else if (t.valid(p)) {
-        // q = r, k = o
+        for (int h = 0; h < H; ++h) a.bias[tri_bias_offset(a.N, h, q, k)] = f2h_sat(acc[0][h] * a.bias_scale);
+        // keys N .. of the last key tile are padding and read as zero bias: the tile's real keys share them out
+        const int k_last = (a.N - 1) & ~63, real = a.N - k_last;
+        if (k >= k_last)
+          for (int kp = a.N + k - k_last; kp < k_last + 64; kp += real)
 #pragma unroll
-        for (int h = 0; h < H; ++h) {
-          a.bias[tri_bias_offset(a.N, h, r, t.o)] = f2h_sat(acc[0][h] * a.bias_scale);
-          if (t.o == a.N - 1)
-            for (int k = a.N; k < kpad; ++k) a.bias[tri_bias_offset(a.N, h, r, k)] = 0;
-        }
+            for (int h = 0; h < H; ++h) a.bias[tri_bias_offset(a.N, h, q, kp)] = 0;
       }
     }
   }
@@ -190,9 +188,13 @@ int launch_triattn_proj(const TriAttnProjArgs& a, hipStream_t stream) {
   if (!al16(a.pair) || !al16(a.w_qkvg) || !al16(a.w_bias) || !al16(a.q) || !al16(a.k) || !al16(a.vt) ||
       !al16(a.bias))
     return AF3_ERR_BAD_ARG;
-  const int64_t tiles = (int64_t)a.N * ((a.N + TM - 1) / TM);
+  const int64_t tiles = ((int64_t)a.N * a.ldn + TM - 1) / TM;
   if (tiles > 0x7fffffff) return AF3_ERR_BAD_ARG;
-  if (a.io_f32) hipLaunchKernelGGL(triattn_proj_kernel<float>, dim3((unsigned)tiles), dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL(triattn_proj_kernel<bf16_t>, dim3((unsigned)tiles), dim3(256), 0, stream, a);
+  const dim3 grid((unsigned)tiles), block(256);
+  const bool cross = tile_crosses(a.ldn);
+  if (a.io_f32 && cross) hipLaunchKernelGGL((triattn_proj_kernel<float, true>), grid, block, 0, stream, a);
+  else if (a.io_f32) hipLaunchKernelGGL((triattn_proj_kernel<float, false>), grid, block, 0, stream, a);
+  else if (cross) hipLaunchKernelGGL((triattn_proj_kernel<bf16_t, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((triattn_proj_kernel<bf16_t, false>), grid, block, 0, stream, a);
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
