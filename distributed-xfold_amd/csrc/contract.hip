@@ -11,20 +11,18 @@
 // 512-entry register file of a lone wave per SIMD), half a 16-byte fragment
 // read per MFMA and 128 FLOPs per byte fetched from L2.
 //
-// What paces the kernel is the CU's vector memory path: every 64-byte row piece of a slab
-// is a miss in the CU's L1 and a round trip to L2 (about 450 cycles on average with a
-// quarter of them going on to memory), the L1 holds a limited number of them in flight, and
-// a wave that issues a load into a full queue stalls with its MFMAs behind it.  A lone wave
-// per SIMD has nobody to cover for it.  So:
-//   * slabs (32 k deep) go from global memory straight into LDS
-//     (global_load_lds_dwordx4: no staging registers, no LDS stores in the
-//     instruction stream);
-//   * the loads are spread evenly, one per four MFMAs per wave, which keeps the
-//     memory path evenly busy instead of saturated in bursts;
-//   * four LDS buffers: a load is issued two to three slabs (2000-3000 cycles)
-//     before anybody waits for it, about the latency of a miss that goes to HBM;
-//   * the one barrier per slab sits between its two k-steps, after the wave has
-//     read all its fragments of the slab: the MFMAs of the second k-step cover
+// What paces the kernel is the CU's vector memory path: it takes in about one cache line every two
+// cycles, whole or in part, and a wave that issues a load into a full queue stalls with its MFMAs behind it.
+// A lone wave per SIMD has nobody to cover for it.  So:
+//   * slabs are 64 k deep, a slab row is one whole 128-byte line: 115 bytes/ns into a CU where 64-byte
+//     pieces bring 62 (32-deep slabs, in four buffers).  Two buffers of 64 KB are what LDS holds;
+//   * slabs go from global memory straight into LDS (buffer_load_dwordx4 .. lds: no staging
+//     registers, no LDS stores in the instruction stream), range-checked, so that a ragged K end
+//     arrives as zeros and needs no other code;
+//   * the loads are dealt between the fragment reads of two of a slab's four k-steps, which keeps
+//     the memory path evenly busy instead of saturated in bursts;
+//   * the one barrier per slab sits in front of its last k-step, after the wave has
+//     read all its fragments of the slab: the MFMAs of that k-step cover
 //     the barrier and the first fragment reads of the next slab, and the
 //     buffer is free for refill the moment the barrier is passed;
 //   * the workgroups are persistent, one per CU, and the slab pipeline never drains: the
@@ -33,11 +31,16 @@
 //     not wait for its stores, so a tile's first slab is in LDS when the previous tile's
 //     last store has been issued.
 // A load puts lane l's 16 bytes at LDS base + 16 l, so rows cannot be padded;
-// instead the four 16-byte chunks of a 64-byte row are permuted, chunk c of row
-// r living at position c ^ ((r >> 2) & 3), which makes the fragment reads (32
+// instead the eight 16-byte chunks of a row are permuted, chunk c of row
+// r living at position c ^ ((r >> 1) & 7), which makes the fragment reads (32
 // rows x one chunk per half-wave) conflict-free over the 64 banks.  The
 // permutation is applied on the global side, where a lane is free to fetch
 // any chunk.
+//
+// 32-deep -> 64-deep slabs, us: contraction of 128 channels at N = 187 9.9 -> 8.9, 300 25.4 -> 22.0, 387 40.3 -> 35.5,
+// 500 46.2 -> 44.0, 1536 881 -> 860; 4096 x 24576 x 1024 regrouped 224 -> 206; 3840 x 3072 x 768 with column epilogue
+// 29.1 -> 26.0, with SwiGLU 23.6 -> 20.2; 8192^3 852 -> 805 (1366 TFLOP/s).  At N = 768 (140 both) memory decides: 450 MB
+// pass in and out.  In large products the matrix cores are busy 77 % of the time and power sets the clock (1.66 GHz).
 //
 // The accumulators hold T^T tiles (B fragments as the MFMA's A operand), so a
 // lane owns one output row i and four consecutive columns j per register quad:
@@ -45,6 +48,7 @@
 // through LDS and writes 128-byte row segments.
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "kernels.h"
@@ -53,22 +57,41 @@ namespace {
 
 // The block is 64 IT x 256: IT = 4 MFMA tiles per wave along i (256 x 256), or IT = 3 (192 x 256) where
 // that saves enough rounds of workgroups (N = 384: tiles of 256 would be half empty).
-constexpr int CN = 256, CK = 32;
-constexpr int ROWB = CK * 2;            // bytes of a slab row in LDS (unpadded)
-constexpr int SLAB = (256 + CN) * ROWB;  // 32 KB at IT = 4: A rows first, then B rows
+constexpr int CN = 256, CK = 64;
+constexpr int ROWB = CK * 2;            // bytes of a slab row in LDS (unpadded): one cache line
+constexpr uint32_t SLAB = (256 + CN) * ROWB;  // 64 KB at IT = 4: A rows first, then B rows
 constexpr int LDE = 64 + 8;             // LDS row stride of a wave's output staging area (bf16)
 constexpr int EPI_BYTES = 32 * LDE * 2;  // 32 rows x 64 columns per wave at a time
 constexpr int RSRC_RAW = 0x00020000;     // last word of a raw (unstructured, range-checked) buffer descriptor
 
-// 64 lanes x 16 bytes from global (uniform base + per-lane byte offset) to
-// 1 KB of LDS starting at the wave-uniform address dst.  Issued as inline assembly on purpose:
+// 64 lanes x 16 bytes from a range-checked buffer (descriptor, wave-uniform byte offset, per-lane byte offset) to
+// the KB of LDS at the wave-uniform address lds + BYTES.  An offset past the descriptor's size writes zeros.  Issued
+// as inline assembly on purpose:
 // the compiler keeps a scoreboard of the loads into LDS that it can see and, where paths with
 // different waits meet, makes a later fragment read wait for ALL of them (vmcnt(0)), the ones
 // issued a moment ago for slabs far ahead included.  Here every buffer is read only after an
 // explicit wait and barrier that follow the load's issue.
-__device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, const char* dst) {
-  const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)dst;
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "m0");
+template <int BYTES>
+__device__ __forceinline__ void load_to_lds(const u32x4 rsrc, uint32_t soff, uint32_t off, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(off), "s"(rsrc),
+               "s"(soff), "n"(BYTES)
+               : "m0", "scc");
+}
+__device__ __forceinline__ u32x4 buffer_of(const void* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return u32x4{lo, hi & 0xffffu, 0x7fffffffu, RSRC_RAW};
+}
+
+template <int N>
+using I = std::integral_constant<int, N>;
+// f(I<0>{}), .., f(I<N - 1>{})
+template <int N, typename F>
+__device__ __forceinline__ void each(F&& f) {
+  if constexpr (N > 0) {
+    each<N - 1>(f);
+    f(I<N - 1>{});
+  }
 }
 
 // a pointer the compiler cannot prove wave-uniform, moved to scalar registers
@@ -107,17 +130,16 @@ template <int MODE, int IT = 4>
 __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
   constexpr int CM = 64 * IT, WM = 32 * IT;  // block and wave extent along i
   constexpr int SLAB_A = CM * ROWB;
-  constexpr int NLOAD = IT + 4;              // loads per wave and slab
+  constexpr int LA = 2 * IT, NLOAD = LA + 8;  // loads per wave and slab, of which A
   constexpr int NSTORE = (MODE == BIG_SWIGLU ? 4 : 8) * IT;  // stores per wave and full tile
-  static_assert(2 * NLOAD + IT + NSTORE < 64, "vmcnt has six bits");
-  // four slab buffers and the waves' output staging areas
-  __shared__ __attribute__((aligned(1024))) char sb0[SLAB];
-  __shared__ __attribute__((aligned(1024))) char sb1[SLAB];
-  __shared__ __attribute__((aligned(1024))) char sb2[SLAB];
-  __shared__ __attribute__((aligned(1024))) char sb3[SLAB];
+  // A slab's loads go out in two halves, the first into a buffer the moment it is free, the second over the next
+  // k-step: they have two to three and a half k-steps (1000 to 1800 cycles) to land.
+  constexpr int EARLY = NLOAD / 2;
+  static_assert(NLOAD < 64 && NSTORE < 64, "vmcnt has six bits");
+  // two slab buffers and the waves' output staging areas
+  __shared__ __attribute__((aligned(1024))) char smem[2 * SLAB];
   __shared__ __attribute__((aligned(16))) char sOut[4 * EPI_BYTES];
   __shared__ __attribute__((aligned(16))) float sColBias[MODE == BIG_COLUMN_OPS ? 4 * 128 : 4];  // a wave's 128 bias values
-  auto buf = [&](int i) -> char* { return (i & 3) == 0 ? sb0 : (i & 3) == 1 ? sb1 : (i & 3) == 2 ? sb2 : sb3; };
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -155,92 +177,95 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
     t.bz = __builtin_amdgcn_readfirstlane(t.bz);
     return true;
   };
-  int slot = blockIdx.x >> 3;
-  Tile cur_t, next_t;
+  int slot = blockIdx.x >> 3, load_slot = slot;
+  Tile cur_t, load_t;
   if (!tile_at(slot, cur_t)) return;
+  load_t = cur_t;
 
-  // Per slab a wave issues IT loads for A and four for B: load i covers rows
-  // 16 IT wave + 16 i .. + 16 of A, 64 wave + 16 i .. + 16 of B (one 64-byte row per 4 lanes).  The lane at position
-  // pc of row r fetches chunk pc ^ ((r >> 2) & 3) = pc ^ (lane >> 4).  Rows past
-  // the end repeat the last one (what they produce lands in output rows that
+  // Per slab a wave issues LA loads for A and eight for B: load i covers rows 16 IT wave + 8 i .. + 8 of A, 64 wave +
+  // 8 i .. + 8 of B (one 128-byte row per 8 lanes).  The lane at position pc of row r fetches chunk pc ^ ((r >> 1) & 7).
+  // Rows past the end repeat the last one (what they produce lands in output rows that
   // are never stored or in columns N..ldc-1 of T, which no consumer reads); a
-  // chunk past K is fetched from the row's first slab instead and zeroed in
-  // LDS before the slab is used.
-  const int ld_r = lane >> 2;
-  const int ld_c = (lane & 3) ^ (lane >> 4);
-  const char* A;
-  const char* B;
-  uint32_t offa[4], offb[4];
-  auto point_a = [&](const Tile& t) {
-    A = reinterpret_cast<const char*>(g.A + (int64_t)t.bz * g.sA);
+  // chunk past K gets an offset past the buffer's end and arrives as zeros.
+  const int ld_r = lane >> 3;
+  const int ld_c[2] = {(lane & 7) ^ (lane >> 4), (lane & 7) ^ (4 + (lane >> 4))};  // even and odd i
+  u32x4 A, B;
+  uint32_t offa[LA], offb[8];
+  auto point = [&](const Tile& t) {
+    A = buffer_of(g.A + (int64_t)t.bz * g.sA);
+    B = buffer_of(g.B + (int64_t)t.bz * g.sB);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      offa[i] = ((uint32_t)min(t.m0 + 16 * IT * wave + 16 * i + ld_r, g.M - 1) * (uint32_t)g.lda + ld_c * 8) * 2u;
-  };
-  auto point_b = [&](const Tile& t) {
-    B = reinterpret_cast<const char*>(g.B + (int64_t)t.bz * g.sB);
+    for (int i = 0; i < LA; ++i)
+      offa[i] = ((uint32_t)min(t.m0 + 16 * IT * wave + 8 * i + ld_r, g.M - 1) * (uint32_t)g.lda + ld_c[i & 1] * 8) * 2u;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      offb[i] = ((uint32_t)min(t.n0 + 64 * wave + 16 * i + ld_r, g.N - 1) * (uint32_t)g.ldb + ld_c * 8) * 2u;
+    for (int i = 0; i < 8; ++i)
+      offb[i] = ((uint32_t)min(t.n0 + 64 * wave + 8 * i + ld_r, g.N - 1) * (uint32_t)g.ldb + ld_c[i & 1] * 8) * 2u;
   };
-  point_a(cur_t);
-  point_b(cur_t);
-  // Load i of half a slab: `first` = the wave's loads of A, else its four of B, of slab kt of the
-  // tile that A / B point at.
-  auto slab_load_one = [&](char* dst, int kt, bool first, int i) {
-    const int k0 = kt * CK;
-    const uint32_t kb = k0 + ld_c * 8 < g.K ? (uint32_t)k0 * 2u : 0u;
-    if (first) load_to_lds(A, offa[i] + kb, dst + (16 * IT * wave + 16 * i) * ROWB);
-    else load_to_lds(B, offb[i] + kb, dst + SLAB_A + (64 * wave + 16 * i) * ROWB);
+  const int nk = (g.K + CK - 1) / CK;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)smem;
+  // The slab being loaded: slab load_k of load_t, to the buffer at load_a (its A part, this wave's share) / load_b.
+  // It runs on across tiles: behind a tile's last slab come the workgroup's next tile's (behind the last tile's,
+  // its own first ones again, unused), so a tile's first slabs arrive while the previous tile finishes and is stored.
+  int load_k = 0;
+  uint32_t load_a = __builtin_amdgcn_readfirstlane(lds0 + 16 * IT * wave * ROWB);
+  uint32_t load_b = __builtin_amdgcn_readfirstlane(lds0 + SLAB_A + 64 * wave * ROWB);
+  uint32_t kb = 0;
+  bool in_k[2];
+  auto begin_slab = [&]() {
+    kb = __builtin_amdgcn_readfirstlane((uint32_t)load_k * (CK * 2));
+    in_k[0] = load_k * CK + ld_c[0] * 8 < g.K;
+    in_k[1] = load_k * CK + ld_c[1] * 8 < g.K;
   };
-  auto slab_load = [&](char* dst, int kt, bool first) {
-#pragma unroll
-    for (int i = 0; i < (first ? IT : 4); ++i) slab_load_one(dst, kt, first, i);
-  };
-  // Chunks at or past K of slab kt (the last slab, and the all-zero slabs that
-  // pad the slab count to a multiple of four): thread t clears them in row t
-  // of A and row t of B.  Every wave's loads of the slab must have landed.
-  auto slab_clear_tail = [&](char* b, int kt) {
-    const int valid = max(0, min(4, (g.K - kt * CK) >> 3));
-    const u32x4 z = {0, 0, 0, 0};
-    const int swz = (tid >> 2) & 3;
-    for (int c = valid; c < 4; ++c) {
-      if (tid < CM) *reinterpret_cast<u32x4*>(b + tid * ROWB + ((c ^ swz) << 4)) = z;
-      *reinterpret_cast<u32x4*>(b + SLAB_A + tid * ROWB + ((c ^ swz) << 4)) = z;
+  auto next_slab = [&]() {
+    load_a ^= SLAB;
+    load_b ^= SLAB;
+    if (++load_k == nk) {
+      load_k = 0;
+      load_slot += slot_step;
+      if (!tile_at(load_slot, load_t)) load_t = cur_t;
+      point(load_t);
     }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    begin_slab();
+  };
+  auto load = [&](auto i_c) {
+    constexpr int i = decltype(i_c)::value;
+    if constexpr (i < LA) load_to_lds<i * 8 * ROWB>(A, kb, in_k[i & 1] ? offa[i] : 0x80000000u, load_a);
+    else load_to_lds<(i - LA) * 8 * ROWB>(B, kb, in_k[(i - LA) & 1] ? offb[i - LA] : 0x80000000u, load_b);
+  };
+  auto loads = [&](auto from_c, auto to_c) {  // loads from .. to - 1 of the slab
+    constexpr int from = decltype(from_c)::value;
+    each<decltype(to_c)::value - from>([&](auto i_c) { load(I<from + decltype(i_c)::value>{}); });
   };
 
   // Fragment (row R = base + 32 t + l31, k-step ks, half hh) is chunk 2 ks + hh
-  // of row R, at position (2 ks + hh) ^ ((R >> 2) & 3); the bases are multiples
+  // of row R, at position (2 ks + hh) ^ ((R >> 1) & 7); the bases are multiples
   // of 32, so the permutation depends on l31 only.
-  uint32_t fo[2];
+  uint32_t fra[4], frb[4];
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) fo[ks] = (uint32_t)(l31 * ROWB + (((2 * ks + hh) ^ ((l31 >> 2) & 3)) << 4));
-  const uint32_t a_base = (uint32_t)(wm * ROWB), b_base = (uint32_t)(SLAB_A + wn * ROWB);
+  for (int ks = 0; ks < 4; ++ks) {
+    const uint32_t fo = (uint32_t)(l31 * ROWB + (((2 * ks + hh) ^ ((l31 >> 1) & 7)) << 4));
+    fra[ks] = wm * ROWB + fo;
+    frb[ks] = SLAB_A + wn * ROWB + fo;
+  }
 
   // acc[jt][it] = (T^T) tile: rows j = wn + 32 jt + .., columns i = wm + 32 it + ..
   f32x16 acc[4][IT];
 
-  bf16x8 fa[2][IT], fb[2][4];  // set 0: first k-step of a slab, set 1: second
-  auto frag = [&](int set, const char* b, int ks, int j) {
-    if (j < IT) fa[set][j] = as_frag(*reinterpret_cast<const u32x4*>(b + a_base + j * (32 * ROWB) + fo[ks]));
-    else fb[set][j - IT] = as_frag(*reinterpret_cast<const u32x4*>(b + b_base + (j - IT) * (32 * ROWB) + fo[ks]));
+  bf16x8 fa[2][IT], fb[2][4];
+  auto frag = [&](int set, int ks, int j) {
+    if (j < IT) fa[set][j] = as_frag(*reinterpret_cast<const u32x4*>(smem + fra[ks] + j * (32 * ROWB)));
+    else fb[set][j - IT] = as_frag(*reinterpret_cast<const u32x4*>(smem + frb[ks] + (j - IT) * (32 * ROWB)));
   };
-  auto frags = [&](int set, const char* b, int ks) {
-#pragma unroll
-    for (int j = 0; j < IT + 4; ++j) frag(set, b, ks, j);
-  };
-  // The IT + 4 fragment reads of a k-step with half a slab's loads dealt evenly between them, in
+  // The IT + 4 fragment reads of a k-step with loads FROM .. TO - 1 dealt evenly between them, in
   // this order in the source: the loads are opaque to the scheduler, which keeps memory
   // operations on their side of one, so this is what spreads the loads over the k-step.
-  auto frags_and_loads = [&](int set, const char* b, int ks, char* dst, int kt, bool first) {
-    const int nl = first ? IT : 4;
-#pragma unroll
-    for (int j = 0; j < IT + 4; ++j) {
-      frag(set, b, ks, j);
-      if (((j + 1) * nl) / (IT + 4) > (j * nl) / (IT + 4)) slab_load_one(dst, kt, first, (j * nl) / (IT + 4));
-    }
+  auto frags_and_loads = [&](int set, int ks, auto from_c, auto to_c) {
+    constexpr int from = decltype(from_c)::value, n = decltype(to_c)::value - from, J = IT + 4;
+    each<J>([&](auto j_c) {
+      constexpr int j = decltype(j_c)::value;
+      frag(set, ks, j);
+      loads(I<from + j * n / J>{}, I<from + (j + 1) * n / J>{});
+    });
   };
   // `fresh`: the first k-step of a tile starts its accumulators from the constant zero
   auto mfmas = [&](int set, auto fresh_c) {
@@ -260,58 +285,49 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
       __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
 
-  const int nk = (g.K + CK - 1) / CK;
-  const int nk4 = (nk + 3) & ~3;  // stages come in fours (the buffers are addressed statically)
-  // Loads in flight, oldest first, whenever a wave reaches the barrier of
-  // slab kt: [slab kt + 1] [slab kt + 2] [slab kt + 3]; the barrier needs the
-  // first group, so two slabs' worth may stay outstanding.
-  slab_load(sb0, 0, true);
-  slab_load(sb0, 0, false);
-  slab_load(sb1, 1, true);
-  slab_load(sb1, 1, false);
-  slab_load(sb2, 2, true);
-  slab_load(sb2, 2, false);
-  slab_load(sb3, 3, true);
-  wait_loads_but<2 * NLOAD + IT>();  // everything but slab 0
+  point(cur_t);
+  begin_slab();
+  loads(I<0>{}, I<NLOAD>{});
+  next_slab();
+  loads(I<0>{}, I<NLOAD>{});
+  wait_loads_but<NLOAD>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  if (CK > g.K) slab_clear_tail(sb0, 0);
-  frags(0, sb0, 0);
+#pragma unroll
+  for (int j = 0; j < IT + 4; ++j) frag(0, 0, j);
 
-  // The slab pipeline runs on across tiles: slabs nk4, nk4 + 1, .. of a tile are slabs 0, 1, ..
-  // of the workgroup's next one (A and B are pointed at it just before the first such load), so
-  // a tile's first slabs arrive while the previous tile finishes and is stored.  `last`: the
-  // tile's last four stages.  `stores_between`: the wave has issued NSTORE stores since the loads
-  // of the slab this stage waits for (vector memory operations retire in order and share the
-  // counter), so that many more may be outstanding.
-  auto stage = [&](int kt, auto b_c, auto fresh_c, bool last, bool stores_between) {
-    constexpr int b = decltype(b_c)::value;  // kt & 3
-    char* cur = buf(b);
-    char* nxt = buf(b + 1);
-    // first k-step (fragments already in set 0); meanwhile the second k-step's
-    // fragments and the B half of slab kt + 3
-    if (b == 1 && last) point_b(next_t);
-    frags_and_loads(1, cur, 1, buf(b + 3), kt + 3 >= nk4 ? kt + 3 - nk4 : kt + 3, false);
+  // One slab, its first fragments already in set 0.  FRESH: a tile's first (all of the next slab's loads are under way,
+  // and the previous tile's NSTORE stores, if any, behind them).
+  const I<0> none{};
+  auto stage = [&](auto fresh_c, bool stores_behind) {
+    constexpr bool fresh = decltype(fresh_c)::value;
+    frags_and_loads(1, 1, I<fresh ? NLOAD : EARLY>{}, I<NLOAD>{});
     mfmas(0, fresh_c);
     interleave();
-    __builtin_amdgcn_sched_barrier(0);
-    // This wave has read all it needs of slab kt; its share of slab kt + 1 has
-    // landed once at most two slabs' worth of younger loads are outstanding.  Past the barrier
-    // that holds for every wave: slab kt + 1 is complete, buffer b is free.
-    if (stores_between) wait_loads_but<2 * NLOAD + NSTORE>();
-    else wait_loads_but<2 * NLOAD>();  // two slabs' worth
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (kt + 1 < nk4 ? (kt + 2) * CK > g.K : CK > g.K) slab_clear_tail(nxt, kt + 1 < nk4 ? kt + 1 : 0);
-    // second k-step; meanwhile the next slab's first fragments and the A half
-    // of slab kt + 4 into the buffer just freed
-    if (b == 0 && last) point_a(next_t);
-    frags_and_loads(0, nxt, 0, cur, kt + 4 >= nk4 ? kt + 4 - nk4 : kt + 4, true);
+    frags_and_loads(0, 2, none, none);
     mfmas(1, std::false_type{});
     interleave();
-    __builtin_amdgcn_sched_barrier(0);
+    frags_and_loads(1, 3, none, none);
+    mfmas(0, std::false_type{});
+    interleave();
+    // This wave has read all it needs of the slab, and its share of the next one has landed.  Past the barrier
+    // that holds for every wave: the next slab is complete, this one's buffer is free.
+    if (fresh && stores_behind) wait_loads_but<NSTORE>();
+    else wait_loads_but<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      fra[ks] ^= SLAB;
+      frb[ks] ^= SLAB;
+    }
+    next_slab();
+    frags_and_loads(0, 0, I<0>{}, I<EARLY>{});
+    mfmas(1, std::false_type{});
+    interleave();
   };
 
   // Epilogue of one tile, per wave and without a barrier: the wave stages 32 rows i x 64 columns j
@@ -434,28 +450,14 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
 
   bool stored = false;  // a tile's epilogue (NSTORE stores per wave, whatever the bounds) lies behind
   while (true) {
-    const bool has_next = tile_at(slot + slot_step, next_t);
-    if (!has_next) next_t = cur_t;  // the loads past the tile's end then re-read its first slabs, unused
-    // the tile's first four stages apart: its very first k-step starts the accumulators from the
-    // constant zero (no 256 moves to clear them), and a branch on "first" inside the loop would
-    // have the accumulators meet at its join
-    stage(0, std::integral_constant<int, 0>{}, std::true_type{}, nk4 == 4, stored);
-    stage(1, std::integral_constant<int, 1>{}, std::false_type{}, nk4 == 4, stored);
-    stage(2, std::integral_constant<int, 2>{}, std::false_type{}, nk4 == 4, false);
-    stage(3, std::integral_constant<int, 3>{}, std::false_type{}, nk4 == 4, false);
-    for (int kt = 4; kt < nk4; kt += 4) {
-      const bool last = kt + 4 == nk4;
-      stage(kt, std::integral_constant<int, 0>{}, std::false_type{}, last, false);
-      stage(kt + 1, std::integral_constant<int, 1>{}, std::false_type{}, last, false);
-      stage(kt + 2, std::integral_constant<int, 2>{}, std::false_type{}, last, false);
-      stage(kt + 3, std::integral_constant<int, 3>{}, std::false_type{}, last, false);
-    }
+    stage(std::true_type{}, stored);
+    for (int kt = 1; kt < nk; ++kt) stage(std::false_type{}, false);
+    loads(I<EARLY>{}, I<NLOAD>{});
     store_tile(cur_t);
     __builtin_amdgcn_sched_barrier(0);
-    if (!has_next) break;
-    stored = true;
-    cur_t = next_t;
     slot += slot_step;
+    if (!tile_at(slot, cur_t)) break;
+    stored = true;
   }
   wait_loads_but<0>();  // nothing may be in flight into LDS when the workgroup ends
 }

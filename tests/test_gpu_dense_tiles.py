@@ -1,5 +1,5 @@
 """GPU parity of the dense products below the 256x256-tile sizes, one case at the edges of every tile the launcher
-chooses from (32x32, 64x64, 64x128, 128x128, the element-wise form): first and last rows and columns alone in a tile,
+chooses from (32x32, 64x64, 64x128, 128x128, the element-wise form), and of the large tile: first and last rows and columns alone in a tile,
 K shorter than a slab, K with a partial last slab, column counts that force element-wise stores; the order of
 summation, which must not depend on the number of rows; and the K split of the Pairformer's single track."""
 
@@ -17,6 +17,7 @@ SHAPES = [
     (12001, 136, 120), (129, 3072, 392), (97, 72, 1032),                              # 64x64, K with a partial last slab
     (31, 3, 64), (97, 65, 200), (500, 765, 392),                                      # 64x64, element by element
     (1921, 3080, 128), (8001, 384, 1024), (70, 70016, 64), (180001, 128, 64),         # 64x128
+    (8000, 1024, 104), (7777, 2112, 40), (30720, 256, 192),                           # 256x256: K in one, two, three slabs
     (20001, 1032, 128),                      # 128x128 (odd columns keep it off the large tile)
 ]
 
