@@ -124,7 +124,10 @@ __device__ __forceinline__ void wait_loads_but() {
 //         seg_len columns, and optionally the 32x32-regrouped output order.
 // MODE 2: SwiGLU, weight rows packed in blocks of 64 (32 "a" rows, then the 32
 //         matching "b" rows): output column 32 p + x = silu(a) * b of block p.
-enum { BIG_PLAIN = 0, BIG_COLUMN_OPS = 1, BIG_SWIGLU = 2 };
+// MODE 3: outer-product mean. Rows and columns are (token, 32 channels); the tile, 8 x 8 token pairs' outer
+//         products, never leaves the workgroup: it goes to LDS in bf16, [pair][1024], and is multiplied there with
+//         the output weights [128][1024] (outer_tile).
+enum { BIG_PLAIN = 0, BIG_COLUMN_OPS = 1, BIG_SWIGLU = 2, BIG_OUTER_MEAN = 3 };
 
 template <int MODE, int IT = 4>
 __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
@@ -138,10 +141,11 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
   static_assert(NLOAD < 64 && NSTORE < 64, "vmcnt has six bits");
   // two slab buffers and the waves' output staging areas
   __shared__ __attribute__((aligned(1024))) char smem[2 * SLAB];
-  __shared__ __attribute__((aligned(16))) char sOut[4 * EPI_BYTES];
-  __shared__ __attribute__((aligned(16))) float sColBias[MODE == BIG_COLUMN_OPS ? 4 * 128 : 4];  // a wave's 128 bias values
+  __shared__ __attribute__((aligned(16))) char sOut[MODE == BIG_OUTER_MEAN ? 16 : 4 * EPI_BYTES];
+  __shared__ __attribute__((aligned(16))) float sColBias[MODE == BIG_COLUMN_OPS ? 4 * 128 : MODE == BIG_OUTER_MEAN ? 128 : 4];  // (a wave's) 128 bias values
 
   const int tid = threadIdx.x, lane = tid & 63;
+  if (MODE == BIG_OUTER_MEAN && tid < 128) sColBias[tid] = g.bias[tid];  // (read behind many barriers)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hh = lane >> 5, l31 = lane & 31;
   const int wm = (wave >> 1) * WM, wn = (wave & 1) * 128;
@@ -161,7 +165,20 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
   // resident while the XCD streams through its half of B once.
   const bool rect = g.batch == 1 && (tiles_m & 3) == 0 && (tiles_n & 1) == 0;
   struct Tile { int m0, n0, bz; };
-  auto tile_at = [&](int slot, Tile& t) -> bool {
+  auto tile_at = [&](int& slot, Tile& t) -> bool {
+    if constexpr (MODE == BIG_OUTER_MEAN) {
+      // Both operands are much larger than an L2: an XCD's 32 CUs take 4 x 8 tiles at a time, 12 panels for 32 tiles.
+      const int gm = (tiles_m + 3) / 4, groups = gm * ((tiles_n + 7) / 8);
+      for (;; slot += slot_step) {
+        const int group = (slot >> 5) * 8 + xcd;
+        if (group >= groups) return false;
+        const int tm = group % gm * 4 + (slot & 3), tn = group / gm * 8 + (slot >> 2 & 7);
+        t.m0 = __builtin_amdgcn_readfirstlane(tm * CM);
+        t.n0 = __builtin_amdgcn_readfirstlane(tn * CN);
+        t.bz = 0;
+        if (tm < tiles_m && tn < tiles_n) return true;
+      }
+    }
     const int logical = xcd * per_xcd + slot;
     if (slot >= per_xcd || logical >= total) return false;
     int tm = logical % tiles_m, tn = (logical / tiles_m) % tiles_n;
@@ -192,6 +209,17 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
   u32x4 A, B;
   uint32_t offa[LA], offb[8];
   auto point = [&](const Tile& t) {
+    if constexpr (MODE == BIG_OUTER_MEAN) {  // operands of any size: offsets from the tile's first rows
+      A = buffer_of(g.A + t.m0 * g.lda);
+      B = buffer_of(g.B + t.n0 * g.ldb);
+#pragma unroll
+      for (int i = 0; i < LA; ++i)
+        offa[i] = ((uint32_t)min(16 * IT * wave + 8 * i + ld_r, g.M - 1 - t.m0) * (uint32_t)g.lda + ld_c[i & 1] * 8) * 2u;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        offb[i] = ((uint32_t)min(64 * wave + 8 * i + ld_r, g.N - 1 - t.n0) * (uint32_t)g.ldb + ld_c[i & 1] * 8) * 2u;
+      return;
+    }
     A = buffer_of(g.A + (int64_t)t.bz * g.sA);
     B = buffer_of(g.B + (int64_t)t.bz * g.sB);
 #pragma unroll
@@ -219,7 +247,7 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
   auto next_slab = [&]() {
     load_a ^= SLAB;
     load_b ^= SLAB;
-    if (++load_k == nk) {
+    if (++load_k == nk && MODE != BIG_OUTER_MEAN) {  // (there the loads past the end are zeros without a fetch)
       load_k = 0;
       load_slot += slot_step;
       if (!tile_at(load_slot, load_t)) load_t = cur_t;
@@ -288,16 +316,23 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  point(cur_t);
-  begin_slab();
-  loads(I<0>{}, I<NLOAD>{});
-  next_slab();
-  loads(I<0>{}, I<NLOAD>{});
-  wait_loads_but<NLOAD>();
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
+  auto issue_first = [&]() {  // the first two slabs of cur_t
+    point(cur_t);
+    load_k = 0;
+    begin_slab();
+    loads(I<0>{}, I<NLOAD>{});
+    next_slab();
+    loads(I<0>{}, I<NLOAD>{});
+  };
+  auto await_first = [&]() {  // its first slab has landed, the first fragments are read
+    wait_loads_but<NLOAD>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 #pragma unroll
-  for (int j = 0; j < IT + 4; ++j) frag(0, 0, j);
+    for (int j = 0; j < IT + 4; ++j) frag(0, 0, j);
+  };
+  issue_first();
+  await_first();
 
   // One slab, its first fragments already in set 0.  FRESH: a tile's first (all of the next slab's loads are under way,
   // and the previous tile's NSTORE stores, if any, behind them).
@@ -448,16 +483,148 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
     }
   };
 
+  // Outer-product mean of the tile's 8 x 8 token pairs (b, d): pair = (res ? pair : 0) + (W vec(outer) + bias) * gate.
+  // The outer products go to the slab buffers (which hold nothing by now) as 64 rows of 1024 bf16, chunk c of row r at
+  // position c ^ (c >> 4 & 3) ^ (r & 15): both the 8-byte writes and the fragment reads spread over the banks.  Wave w
+  // takes outputs 32 w .. 32 w + 31 of all pairs; its share of the weights, packed in the order of its loads, comes
+  // from L2, 64 KB per tile (W's rows in the order swap23: eight consecutive outputs per lane).
+  // 768 tokens, 1024 MSA rows: 1080 us, of which a tile's K loop is two thirds.  As two products with the outer products
+  // in memory between them (six times 205 + 66 us) the same bits took 1630; 187 tokens, 301 rows 47 (75), 160 tokens,
+  // 128 rows 25 (55).
+  f32x16 outer[2];    // 32 outputs x 32 pairs each
+  float outer_gate[2];
+  u32x4 outer_res[2][2][2];
+  auto outer_pixel = [&](const Tile& t, int p, bool* ok) {
+    const int n = g.N >> 5, b = (t.m0 >> 5) + 4 * p + (l31 >> 3), d = (t.n0 >> 5) + (l31 & 7);
+    *ok = b < n && d < n;
+    return (int64_t)min(b, n - 1) * n + min(d, n - 1);
+  };
+  auto outer_tile = [&](const Tile& t) {
+    constexpr int KSTEPS = 64, RW = 8, RX = 6;  // fragments under way: weights from L2, outer products from LDS
+    const bf16_t* wp = uniform_ptr(g.w2 + wave * KSTEPS * 512) + lane * 8;
+    u32x4 wf[RW], xf[RX][2];
+    auto load_w = [&](int ks) {
+      if (ks < KSTEPS) wf[ks % RW] = *reinterpret_cast<const u32x4*>(wp + ks * 512);
+    };
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) load_w(ks);
+    // (a lane number that the compiler cannot know to be the same for every tile: it would keep the 128 addresses below
+    // in registers for the kernel's lifetime)
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int hh = ln >> 5, l31 = ln & 31;
+    const uint32_t st = (uint32_t)((8 * (wm >> 5) + (wn >> 5)) * 2048 + 8 * hh);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t chunk = (uint32_t)(4 * l31 + (q ^ (l31 >> 2 & 3))) ^ (uint32_t)(wn >> 5);
+#pragma unroll
+      for (int it = 0; it < IT; ++it)
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) {
+          u32x2 v;
+          v.x = pack2bf(acc_read(acc[jt][it][4 * q]), acc_read(acc[jt][it][4 * q + 1]));
+          v.y = pack2bf(acc_read(acc[jt][it][4 * q + 2]), acc_read(acc[jt][it][4 * q + 3]));
+          *reinterpret_cast<u32x2*>(smem + st + ((chunk ^ (8 * (it & 1) + jt)) << 4) + (8 * it + jt) * 2048) = v;
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const uint32_t rd = (uint32_t)(l31 * 2048 + ((hh ^ (l31 & 15)) << 4));
+    auto read_x = [&](int ks) {
+      if (ks < KSTEPS) {
+        const uint32_t at = rd ^ (uint32_t)((2 * ks ^ (ks >> 3 & 3)) << 4);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) xf[ks % RX][p] = *reinterpret_cast<const u32x4*>(smem + at + p * 65536);
+      }
+    };
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) outer[p][r] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < RX - 1; ++ks) read_x(ks);
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      if (ks == 0) {
+#pragma unroll
+        for (int i = 4; i < RW - 1; ++i) load_w(i);
+      }
+      if (ks == KSTEPS / 2) {  // what the results are joined with
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          bool ok;
+          const int64_t pix = outer_pixel(t, p, &ok);
+          outer_gate[p] = g.gate[pix];
+#pragma unroll
+          for (int s = 0; s < 2; ++s) {
+            const int64_t o = pix * 128 + 32 * wave + 16 * s + 8 * hh;
+            outer_res[p][s][0] = outer_res[p][s][1] = u32x4{0, 0, 0, 0};
+            if (g.res_f32) {
+              outer_res[p][s][0] = *reinterpret_cast<const u32x4*>(g.res_f32 + o);
+              outer_res[p][s][1] = *reinterpret_cast<const u32x4*>(g.res_f32 + o + 4);
+            }
+            if (g.res_bf16) outer_res[p][s][0] = *reinterpret_cast<const u32x4*>(g.res_bf16 + o);
+          }
+        }
+      }
+      load_w(ks + RW - 1);
+      read_x(ks + RX - 1);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) outer[p] = mfma32(as_frag(wf[ks % RW]), as_frag(xf[ks % RX][p]), outer[p]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto outer_store = [&](const Tile& t) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      bool ok;
+      const int64_t pix = outer_pixel(t, p, &ok);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int64_t o = 32 * wave + 16 * s + 8 * hh;
+        float v[8], bias[8], res[8];
+        Elem<float>::load8(sColBias + o, bias);
+        if (g.res_f32)
+          for (int e = 0; e < 8; ++e) res[e] = __uint_as_float(outer_res[p][s][e >> 2][e & 3]);
+        else unpack8(outer_res[p][s][0], res);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (outer[p][8 * s + e] + bias[e]) * outer_gate[p] + res[e];
+        if (!ok) continue;
+        if (g.out_f32) Elem<float>::store8(reinterpret_cast<float*>(g.C) + pix * 128 + o, v);
+        else Elem<bf16_t>::store8(reinterpret_cast<bf16_t*>(g.C) + pix * 128 + o, v);
+      }
+    }
+  };
+
   bool stored = false;  // a tile's epilogue (NSTORE stores per wave, whatever the bounds) lies behind
   while (true) {
     stage(std::true_type{}, stored);
     for (int kt = 1; kt < nk; ++kt) stage(std::false_type{}, false);
-    loads(I<EARLY>{}, I<NLOAD>{});
-    store_tile(cur_t);
-    __builtin_amdgcn_sched_barrier(0);
-    slot += slot_step;
-    if (!tile_at(slot, cur_t)) break;
-    stored = true;
+    if constexpr (MODE == BIG_OUTER_MEAN) {
+      wait_loads_but<0>();
+      __builtin_amdgcn_s_barrier();  // every wave has read its last fragments, and no load into the buffers is under way
+      asm volatile("" ::: "memory");
+      outer_tile(cur_t);
+      // every wave has read its outer products: the next tile's slabs may come, while this one's results go
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      const Tile done = cur_t;
+      slot += slot_step;
+      const bool more = tile_at(slot, cur_t);
+      if (more) {
+        load_a ^= SLAB;  // back to the buffer that the fragments are read from next
+        load_b ^= SLAB;
+        issue_first();
+      }
+      outer_store(done);
+      if (!more) break;
+      await_first();
+    } else {
+      loads(I<EARLY>{}, I<NLOAD>{});
+      store_tile(cur_t);
+      __builtin_amdgcn_sched_barrier(0);
+      slot += slot_step;
+      if (!tile_at(slot, cur_t)) break;
+      stored = true;
+    }
   }
   wait_loads_but<0>();  // nothing may be in flight into LDS when the workgroup ends
 }
@@ -521,6 +688,20 @@ void gemm_bias_span(const GemmArgs& g, bool big, int64_t* first, int64_t* last) 
   *last = hi;
 }
 
+// the device's CUs, at least 8
+static int cu_count() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev_id = 0;
+    hipDeviceProp_t prop;
+    cus = hipGetDevice(&dev_id) == hipSuccess && hipGetDeviceProperties(&prop, dev_id) == hipSuccess &&
+                  prop.multiProcessorCount > 0
+              ? std::max(prop.multiProcessorCount, 8)
+              : 256;
+  }
+  return cus;
+}
+
 int launch_big_tile(const GemmArgs& g, int mode, hipStream_t stream) {
   if (!g.A || !g.B || !g.C) return AF3_ERR_BAD_ARG;
   if (mode != big_tile_mode(g) && !(mode == BIG_PLAIN && contract_supported(g))) return AF3_ERR_BAD_ARG;
@@ -538,15 +719,7 @@ int launch_big_tile(const GemmArgs& g, int mode, hipStream_t stream) {
   // block costs 0.83 - 0.86 of a 256 x 256 one, not 0.75 (measured: pipeline fill and the epilogue do not
   // shrink with it), so it is taken for the plain product only when it saves more rounds than that:
   // N = 256 .. 576, not 768 (six rounds against five) or beyond.
-  static int cus = 0;
-  if (cus == 0) {
-    int dev_id = 0;
-    hipDeviceProp_t prop;
-    cus = hipGetDevice(&dev_id) == hipSuccess && hipGetDeviceProperties(&prop, dev_id) == hipSuccess &&
-                  prop.multiProcessorCount > 0
-              ? prop.multiProcessorCount
-              : 256;
-  }
+  const int cus = cu_count();
   const bool flat = ((total3 + cus - 1) / cus) * 7 < ((total4 + cus - 1) / cus) * 8;
   const int64_t total = flat ? total3 : total4;
   if (total > 0x3fffffff) return AF3_ERR_BAD_ARG;
@@ -559,6 +732,22 @@ int launch_big_tile(const GemmArgs& g, int mode, hipStream_t stream) {
   else if (mode == BIG_PLAIN) hipLaunchKernelGGL(contract_kernel<BIG_PLAIN>, grid, block, 0, stream, g);
   else if (mode == BIG_COLUMN_OPS) hipLaunchKernelGGL(contract_kernel<BIG_COLUMN_OPS>, grid, block, 0, stream, g);
   else hipLaunchKernelGGL(contract_kernel<BIG_SWIGLU>, grid, block, 0, stream, g);
+  return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+}
+
+// A = left [(b, c)][lda], B = right [(d, e)][ldb] with c, e < 32 and M = N = 32 n, w2 the packed output weights
+// (outer_mean_weight), bias [128], gate [n][n], C (and residual) [n][n][128].
+int launch_outer_mean(const GemmArgs& g, hipStream_t stream) {
+  if (!g.A || !g.B || !g.C || !g.w2 || !g.bias || !g.gate || g.M <= 0 || g.M != g.N || (g.M & 31) || g.K <= 0 || g.batch != 1)
+    return AF3_ERR_BAD_ARG;
+  if ((g.K & 7) || (g.lda & 7) || (g.ldb & 7) || g.K > g.lda || g.K > g.ldb || g.lda >= (1 << 21) || g.ldb >= (1 << 21))
+    return AF3_ERR_BAD_ARG;
+  if (!al16(g.A) || !al16(g.B) || !al16(g.C) || !al16(g.w2) || !al16(g.bias) || !al16(g.res_f32) || !al16(g.res_bf16))
+    return AF3_ERR_BAD_ARG;
+  const int64_t tiles = (g.M + 255) / 256, slots = ((tiles + 3) / 4 * ((tiles + 7) / 8) + 7) / 8 * 256;
+  if (slots > 0x3fffffff) return AF3_ERR_BAD_ARG;
+  hipLaunchKernelGGL(contract_kernel<BIG_OUTER_MEAN>, dim3((unsigned)std::min<int64_t>(slots, cu_count() / 8 * 8)), dim3(256), 0,
+                     stream, g);
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
 

@@ -31,6 +31,7 @@ struct GemmArgs {
   // at [(m / 32, n / 32)][(m % 32, n % 32)], i.e. C is [(M/32)(N/32)][1024]:
   // the outer products of 32-channel rows, one contiguous 1024-vector per pair.
   int regroup32 = 0;
+  const bf16_t* w2 = nullptr;  // launch_outer_mean only
   int split_k = 0;  // the K range may be summed in parts by several waves (another order of summation)
 };
 int launch_gemm_nt(const GemmArgs& g, hipStream_t stream);
@@ -69,6 +70,7 @@ int launch_contract(const GemmArgs& g, hipStream_t stream);
 // kernel instance that can take `g`, or -1
 int big_tile_mode(const GemmArgs& g);
 int launch_big_tile(const GemmArgs& g, int mode, hipStream_t stream);
+int launch_outer_mean(const GemmArgs& g, hipStream_t stream);
 // the large-tile instance launch_gemm_nt hands `g` to, or -1: the kernel of gemm.hip
 int gemm_big_tile_choice(const GemmArgs& g);
 
@@ -297,6 +299,34 @@ struct TriAttnArgs {
   int64_t ldn = 0;
 };
 int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream);
+
+// ---------------------------------------------------------------------- msa.hip
+struct MsaProjectArgs {
+  const void* msa = nullptr;  // [rows][n][64]
+  int io_f32 = 0, rows = 0, n = 0;
+  const float *ln_w = nullptr, *ln_b = nullptr;
+  const bf16_t* w = nullptr;      // [64][64]
+  const float* mask = nullptr;    // [rows][n]; not for values
+  bf16_t* out[2] = {nullptr, nullptr};
+  int64_t ld = 0;                 // rows (values: n) rounded up to 8
+};
+int launch_msa_project(const MsaProjectArgs& a, bool values, hipStream_t s);
+
+struct MsaUpdateArgs {
+  const void* msa = nullptr;  // [rows][n][64]
+  void* out = nullptr;        // may be msa
+  int io_f32 = 0, rows = 0, n = 0, residual = 0;
+  const bf16_t* avg = nullptr;  // [8][n][rows][8], or null: no attention part
+  const float *att_ln_w = nullptr, *att_ln_b = nullptr;
+  const bf16_t *w_g = nullptr, *w_o = nullptr;  // [64][64]
+  const float *tr_ln_w = nullptr, *tr_ln_b = nullptr;
+  const bf16_t* w1 = nullptr;   // [2 hidden][64], the silu half first, or null: no transition
+  const bf16_t* w2 = nullptr;   // [64][hidden]
+  int hidden = 0;               // a multiple of 32, at most 256
+};
+int launch_msa_update(const MsaUpdateArgs& a, hipStream_t s);
+int launch_msa_coverage(const float* mask, int rows, int n, float eps, float* inv, float* live, hipStream_t s);
+int launch_transpose_f32(const float* in, float* out, int n, hipStream_t s);  // [n][n]
 
 // --------------------------------------------------------------- check_f32.hip
 struct CkGemmArgs {

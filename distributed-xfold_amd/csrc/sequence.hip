@@ -78,9 +78,143 @@ int single_update(const af3_pairformer_block& b, void* single, int dt, const flo
   return product(y, b.st_w2, single, dt, c, h, AF3_LINEAR_GATE_RES, single);
 }
 
+inline int64_t up8(int64_t v) { return (v + 7) / 8 * 8; }
+inline bool msa_size_ok(int64_t rows, int64_t n) { return rows > 0 && n > 0 && n <= 8192 && rows <= (1ll << 30) / n; }
+
+size_t opm_bytes(int64_t rows, int64_t n) {
+  return 2 * align_up((size_t)n * 32 * up8(rows) * 2);
+}
+size_t msa_attention_bytes(int64_t rows, int64_t n) {
+  return align_up((size_t)8 * n * n * 4) + align_up((size_t)8 * n * up8(n) * 2) + align_up((size_t)64 * rows * up8(n) * 2) +
+         align_up((size_t)64 * rows * n * 2);
+}
+size_t msa_mask_bytes(int64_t n) { return align_up((size_t)n * n * 4) + align_up((size_t)n * 4); }
+
+// pair (+)= (outer product W + b) / (eps + coverage)
+int outer_product_mean(const af3_msa_block& b, const void* msa, int msa_dt, const float* msa_mask, const float* inv, void* pair,
+                       int pair_dt, int residual, int64_t rows, int64_t n, Carver w, hipStream_t s) {
+  MsaProjectArgs p;
+  p.msa = msa; p.io_f32 = msa_dt == AF3_F32; p.rows = (int)rows; p.n = (int)n; p.ld = up8(rows);
+  p.ln_w = b.opm_ln_w; p.ln_b = b.opm_ln_b; p.w = b.opm_w_lr; p.mask = msa_mask;
+  for (bf16_t*& o : p.out) o = static_cast<bf16_t*>(w.take((size_t)n * 32 * p.ld * 2));
+  if (!w.ok) return AF3_ERR_WORKSPACE;
+  STEP(launch_msa_project(p, false, s));
+  GemmArgs g;
+  g.A = p.out[0]; g.B = p.out[1]; g.C = pair; g.out_f32 = pair_dt == AF3_F32;
+  g.M = g.N = (int)n * 32; g.K = (int)p.ld; g.lda = g.ldb = p.ld;
+  g.w2 = b.opm_w_out; g.bias = b.opm_b_out; g.gate = inv;
+  if (residual && g.out_f32) g.res_f32 = static_cast<const float*>(pair);
+  else if (residual) g.res_bf16 = static_cast<const bf16_t*>(pair);
+  return launch_outer_mean(g, s);
+}
+
+// The weighted average of the MSA's values, [head][token][row][8]
+int msa_average(const af3_msa_block& b, const void* msa, int msa_dt, const float* live, const float* logits, int64_t rows, int64_t n,
+                Carver& w, const bf16_t** avg_out, hipStream_t s) {
+  MsaProjectArgs p;
+  p.msa = msa; p.io_f32 = msa_dt == AF3_F32; p.rows = (int)rows; p.n = (int)n; p.ld = up8(n);
+  p.ln_w = b.ma_ln_w; p.ln_b = b.ma_ln_b; p.w = b.ma_w_v;
+  bf16_t* weights = static_cast<bf16_t*>(w.take((size_t)8 * n * p.ld * 2));
+  p.out[0] = static_cast<bf16_t*>(w.take((size_t)64 * rows * p.ld * 2));
+  bf16_t* avg = static_cast<bf16_t*>(w.take((size_t)64 * rows * n * 2));
+  if (!w.ok) return AF3_ERR_WORKSPACE;
+  STEP(launch_msa_project(p, true, s));
+  STEP(launch_softmax_rows(logits, live, weights, 8 * n, (int)n, p.ld, s));
+  *avg_out = avg;
+  return af3_batched_nt_product_forward(weights, p.out[0], avg, 8, n, 8 * rows, p.ld, s);
+}
+
+void msa_attention_args(const af3_msa_block& b, const bf16_t* avg, MsaUpdateArgs& u) {
+  u.avg = avg; u.att_ln_w = b.ma_ln_w; u.att_ln_b = b.ma_ln_b; u.w_g = b.ma_w_g; u.w_o = b.ma_w_o;
+}
+void msa_transition_args(const float* ln_w, const float* ln_b, const uint16_t* w1, const uint16_t* w2, int hidden, MsaUpdateArgs& u) {
+  u.tr_ln_w = ln_w; u.tr_ln_b = ln_b; u.w1 = w1; u.w2 = w2; u.hidden = hidden;
+}
+
 }  // namespace
 
 extern "C" {
+
+size_t af3_msa_workspace_bytes(int64_t rows, int64_t n) {
+  if (!msa_size_ok(rows, n)) return 0;
+  const size_t a = opm_bytes(rows, n), b = msa_attention_bytes(rows, n);
+  return msa_mask_bytes(n) + align_up((size_t)n * n * 4) + (a > b ? a : b);
+}
+
+int af3_outer_product_mean_forward(const af3_msa_block* block, const void* msa, int msa_dtype, const float* msa_mask, void* pair,
+                                   int pair_dtype, int residual, int64_t rows, int64_t n, void* workspace,
+                                   size_t workspace_bytes, af3_stream_t stream) {
+  if (!block || !msa || !msa_mask || !pair || !msa_size_ok(rows, n)) return AF3_ERR_BAD_ARG;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  Carver w(workspace, workspace_bytes);
+  float *inv = static_cast<float*>(w.take((size_t)n * n * 4)), *live = static_cast<float*>(w.take((size_t)n * 4));
+  if (!w.ok) return AF3_ERR_WORKSPACE;
+  STEP(launch_msa_coverage(msa_mask, (int)rows, (int)n, block->epsilon, inv, live, s));
+  return outer_product_mean(*block, msa, msa_dtype, msa_mask, inv, pair, pair_dtype, residual, rows, n, w, s);
+}
+
+int af3_msa_attention_forward(const af3_msa_block* block, const void* msa, int msa_dtype, const float* msa_mask, const void* pair,
+                              int pair_dtype, void* out, int residual, int64_t rows, int64_t n, void* workspace,
+                              size_t workspace_bytes, af3_stream_t stream) {
+  if (!block || !msa || !msa_mask || !pair || !out || !msa_size_ok(rows, n)) return AF3_ERR_BAD_ARG;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  Carver w(workspace, workspace_bytes);
+  float *inv = static_cast<float*>(w.take((size_t)n * n * 4)), *live = static_cast<float*>(w.take((size_t)n * 4));
+  float* logits = static_cast<float*>(w.take((size_t)8 * n * n * 4));
+  if (!w.ok) return AF3_ERR_WORKSPACE;
+  STEP(launch_msa_coverage(msa_mask, (int)rows, (int)n, block->epsilon, inv, live, s));
+  STEP(af3_pair_logits_forward(pair, pair_dtype, block->ma_pn_w, block->ma_pn_b, block->ma_w_logits, 8, logits, n, stream));
+  MsaUpdateArgs u;
+  u.msa = msa; u.out = out; u.io_f32 = msa_dtype == AF3_F32; u.rows = (int)rows; u.n = (int)n; u.residual = residual;
+  const bf16_t* avg;
+  STEP(msa_average(*block, msa, msa_dtype, live, logits, rows, n, w, &avg, s));
+  msa_attention_args(*block, avg, u);
+  return launch_msa_update(u, s);
+}
+
+int af3_transition64_forward(const void* x, int io_dtype, const float* ln_w, const float* ln_b, const uint16_t* w1,
+                             const uint16_t* w2, int hidden, void* out, int residual, int64_t rows, af3_stream_t stream) {
+  if (!x || !out || rows <= 0 || rows > (1ll << 30) || (io_dtype != AF3_F32 && io_dtype != AF3_BF16)) return AF3_ERR_BAD_ARG;
+  MsaUpdateArgs u;
+  u.msa = x; u.out = out; u.io_f32 = io_dtype == AF3_F32; u.rows = (int)rows; u.n = 1; u.residual = residual;
+  msa_transition_args(ln_w, ln_b, w1, w2, hidden, u);
+  return launch_msa_update(u, static_cast<hipStream_t>(stream));
+}
+
+int af3_evoformer_stack_forward(const af3_msa_block* const* blocks, int num_blocks, void* msa, int msa_dtype, const float* msa_mask,
+                                void* pair, int pair_dtype, const float* pair_mask, int64_t rows, int64_t n, void* workspace,
+                                size_t workspace_bytes, void* pair_workspace, size_t pair_workspace_bytes, af3_stream_t stream) {
+  if (!blocks || num_blocks <= 0 || !msa || !msa_mask || !pair || !msa_size_ok(rows, n)) return AF3_ERR_BAD_ARG;
+  if ((msa_dtype != AF3_F32 && msa_dtype != AF3_BF16) || (pair_dtype != AF3_F32 && pair_dtype != AF3_BF16)) return AF3_ERR_BAD_ARG;
+  for (int i = 0; i < num_blocks; ++i)
+    if (!blocks[i] || blocks[i]->epsilon != blocks[0]->epsilon) return AF3_ERR_BAD_ARG;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  Carver w(workspace, workspace_bytes);
+  float *inv = static_cast<float*>(w.take((size_t)n * n * 4)), *live = static_cast<float*>(w.take((size_t)n * 4));
+  float* mask_in = static_cast<float*>(w.take((size_t)n * n * 4));
+  if (!w.ok) return AF3_ERR_WORKSPACE;
+  // what depends on the masks alone: once for all blocks
+  STEP(launch_msa_coverage(msa_mask, (int)rows, (int)n, blocks[0]->epsilon, inv, live, s));
+  if (pair_mask) STEP(launch_transpose_f32(pair_mask, mask_in, (int)n, s));
+  for (int i = 0; i < num_blocks; ++i) {
+    const af3_msa_block& b = *blocks[i];
+    STEP(outer_product_mean(b, msa, msa_dtype, msa_mask, inv, pair, pair_dtype, 1, rows, n, w, s));
+    Carver v = w;  // the outer product's operands are done with
+    float* logits = static_cast<float*>(v.take((size_t)8 * n * n * 4));
+    if (!v.ok) return AF3_ERR_WORKSPACE;
+    STEP(af3_pair_logits_forward(pair, pair_dtype, b.ma_pn_w, b.ma_pn_b, b.ma_w_logits, 8, logits, n, stream));
+    MsaUpdateArgs u;
+    u.msa = u.out = msa; u.io_f32 = msa_dtype == AF3_F32; u.rows = (int)rows; u.n = (int)n; u.residual = 1;
+    const bf16_t* avg;
+    STEP(msa_average(b, msa, msa_dtype, live, logits, rows, n, v, &avg, s));
+    msa_attention_args(b, avg, u);
+    msa_transition_args(b.mt_ln_w, b.mt_ln_b, b.mt_w1, b.mt_w2, b.mt_hidden, u);
+    STEP(launch_msa_update(u, s));
+    STEP(pair_operators(b.pair, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace,
+                        pair_workspace_bytes, stream));
+  }
+  return AF3_OK;
+}
 
 size_t af3_pairformer_stack_workspace_bytes(int64_t n, int num_head_pair) {
   const size_t a = af3_triangle_multiplication_workspace_bytes(n), b = af3_grid_self_attn_workspace_bytes(n, num_head_pair);

@@ -26,6 +26,14 @@ class PairformerBlockStruct(C.Structure):
                                     "c_single", "single_hidden")])
 
 
+class MsaBlockStruct(C.Structure):
+    """af3_msa_block."""
+    _fields_ = (
+        [(k, _vp) for k in ("opm_ln_w", "opm_ln_b", "opm_w_lr", "opm_w_out", "opm_b_out", "ma_ln_w", "ma_ln_b", "ma_pn_w",
+                            "ma_pn_b", "ma_w_logits", "ma_w_v", "ma_w_g", "ma_w_o", "mt_ln_w", "mt_ln_b", "mt_w1", "mt_w2")]
+        + [("pair", PairformerBlockStruct), ("mt_hidden", C.c_int32), ("epsilon", C.c_float)])
+
+
 class DiffusionBlockStruct(C.Structure):
     """af3_diffusion_block."""
     _fields_ = [(k, _vp) for k in ("w_q", "w_kv", "q_b", "w_out", "w_tr1", "w_tr2")]
@@ -47,6 +55,12 @@ SIGNATURES = {
     "af3_grid_self_attn_forward_padded": (
         _i, [_vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _i64, _i, _vp, _sz, _vp]),
     "af3_transition_forward_padded": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _i, _i64, _i, _vp]),
+    "af3_msa_workspace_bytes": (_sz, [_i64, _i64]),
+    "af3_outer_product_mean_forward": (_i, [_vp, _vp, _i, _vp, _vp, _i, _i, _i64, _i64, _vp, _sz, _vp]),
+    "af3_msa_attention_forward": (_i, [_vp, _vp, _i, _vp, _vp, _i, _vp, _i, _i64, _i64, _vp, _sz, _vp]),
+    "af3_transition64_forward": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _i, _i64, _vp]),
+    "af3_evoformer_stack_forward": (
+        _i, [_vp, _i, _vp, _i, _vp, _vp, _i, _vp, _i64, _i64, _vp, _sz, _vp, _sz, _vp]),
     "af3_batch_diffusion_self_attention_workspace_bytes": (_sz, [_i64, _i64, _i]),
     "af3_batch_diffusion_self_attention_forward": (
         _i, [_vp, _vp, _i64, _vp, _i, _vp, _vp, _i, _vp, _i, _i64, _i64, _i, _vp, _sz, _vp]),

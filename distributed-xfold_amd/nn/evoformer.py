@@ -5,20 +5,19 @@ keywords, parameter names and `forward` signatures as the reference's
 Distribute* classes; msa and pair are updated in place as the reference's `+=`.
 
 Both MSA operators are products over long axes and run on the bf16 MFMA
-kernels:
+kernels; at the width of the published model (64 channels) a run of blocks is one
+call of the library (`evoformer_loop`).
   * outer-product mean: out[b, d, :] = W^T vec(sum_a L[a, b, :] (x) R[a, d, :]).
-    The sum over the MSA rows is one product [(b, c), a] x [(d, e), a]^T per
-    block of 128 tokens b, whose epilogue stores element ((b, c), (d, e)) at
-    [(b, d)][(c, e)], the layout the second product with W [(c, e), f] reads
-    (a 200 MB bf16 slab at 768 tokens, inside the 256 MB last-level cache); the
-    [N, N, 32, 32] tensor the reference's einsum materialises (1.2 GB) never
-    exists as a whole and nothing is permuted.
+    The sum over the MSA rows is one product [(b, c), a] x [(d, e), a]^T whose
+    tiles, 8 x 8 token pairs' outer products, are multiplied with W where they
+    arise: neither the [N, N, 32, 32] tensor that the reference's einsum
+    materialises (1.2 GB) nor any part of it goes to memory.
   * pair-weighted averaging: per head, softmax(pair logits) [q, k] times the
     head's values of all MSA rows [(row, channel), k]^T.
 Both sum over an index (MSA rows, tokens) that the activations [rows, N, c]
-carry as an outer one, while the dense kernels want it innermost: the operands
-are produced transposed (projection weights as the left operand) or run through
-the bf16 transpose kernel, not through strided copies.
+carry as an outer one, while the dense kernels want it innermost: the
+projections are written transposed.  Other widths go operator by operator
+through the general kernels and torch permutations.
 """
 
 from __future__ import annotations
@@ -30,8 +29,10 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import check, ops
+from .. import lib as L
 from .attention import GridSelfAttention
 from .base import HipModule, bf16, drop_mesh, f32, in_check_mode, pad_rows
+from .pairformer import fill_pair_weights
 from .primitives import Transition
 from .triangle_multiplication import TriangleMultiplication
 
@@ -58,11 +59,24 @@ class OuterProductMean(HipModule):
         self.output_w = nn.Parameter(torch.zeros(num_outer_channel, num_outer_channel, num_output_channel))
         self.output_b = nn.Parameter(torch.zeros(num_output_channel))
 
+    @property
+    def native(self) -> bool:
+        return self.c_msa == 64 and self.num_outer_channel == 32 and self.num_output_channel == 128
+
     def _pack(self):
         co = self.num_outer_channel
-        return dict(ln_w=f32(self.layer_norm_input.weight), ln_b=f32(self.layer_norm_input.bias),
+        d = dict(ln_w=f32(self.layer_norm_input.weight), ln_b=f32(self.layer_norm_input.bias),
                     w_l=bf16(self.left_projection.weight), w_r=bf16(self.right_projection.weight),
                     w_out=bf16(self.output_w.detach().reshape(co * co, -1).t()), b_out=f32(self.output_b))
+        if self.native:
+            d["w_lr"] = torch.cat([d["w_l"], d["w_r"]])
+            rows = [(r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1) for r in range(32)]
+            d["w_packed"] = d["w_out"].view(4, 32, 64, 2, 8)[:, rows].permute(0, 2, 3, 1, 4).contiguous()
+            s = d["block"] = L.MsaBlockStruct()
+            s.epsilon = self.epsilon
+            s.opm_ln_w, s.opm_ln_b, s.opm_w_lr, s.opm_w_out, s.opm_b_out = (
+                d[k].data_ptr() for k in ("ln_w", "ln_b", "w_lr", "w_packed", "b_out"))
+        return d
 
     @torch.no_grad()
     def run(self, msa, mask, residual: Optional[torch.Tensor] = None, block: int = 128):
@@ -70,18 +84,18 @@ class OuterProductMean(HipModule):
         p = self.packed()
         a, n, _ = msa.shape
         co, cf = self.num_outer_channel, self.num_output_channel
+        out = residual if residual is not None else torch.zeros((n, n, cf), dtype=torch.float32, device=msa.device)
+        if self.native:
+            return ops.outer_product_mean(p["block"], msa.contiguous(), mask, out, True)
         m = mask.float()
         x = ops.layer_norm(msa.contiguous(), p["ln_w"], p["ln_b"])
         mb = m[..., None].to(torch.bfloat16)
 
         def projected(w):        # [(token, channel), MSA row]: the summation index innermost
             y = ops.linear(x, w) * mb                                                       # [a, N, co]
-            if a % 8 == 0 and (n * co) % 8 == 0:
-                return ops.transpose2d(y.view(a, n * co))
             return _pad_last(y.permute(1, 2, 0).reshape(n * co, a)).contiguous()
         lt, rt = projected(p["w_l"]), projected(p["w_r"])
         inv_norm = (1.0 / (self.epsilon + m.t() @ m)).contiguous()                         # [b, d]
-        out = residual if residual is not None else torch.zeros((n, n, cf), dtype=torch.float32, device=msa.device)
         for b0 in range(0, n, block):
             b1 = min(n, b0 + block)
             if co == 32:
@@ -120,37 +134,38 @@ class MSAAttention(HipModule):
         self.gating_query = nn.Linear(c_msa, c_msa, bias=False)
         self.output_projection = nn.Linear(c_msa, c_msa, bias=False)
 
+    @property
+    def native(self) -> bool:
+        return self.c_msa == 64 and self.num_head == 8
+
     def _pack(self):
-        return dict(ln_w=f32(self.act_norm.weight), ln_b=f32(self.act_norm.bias),
+        d = dict(ln_w=f32(self.act_norm.weight), ln_b=f32(self.act_norm.bias),
                     pn_w=f32(self.pair_norm.weight), pn_b=f32(self.pair_norm.bias),
                     w_logits=pad_rows(bf16(self.pair_logits.weight), 32), w_v=bf16(self.v_projection.weight),
                     w_g=bf16(self.gating_query.weight), w_o=bf16(self.output_projection.weight))
+        if self.native:
+            s = d["block"] = L.MsaBlockStruct()
+            (s.ma_ln_w, s.ma_ln_b, s.ma_pn_w, s.ma_pn_b, s.ma_w_logits, s.ma_w_v, s.ma_w_g, s.ma_w_o) = (
+                d[k].data_ptr() for k in ("ln_w", "ln_b", "pn_w", "pn_b", "w_logits", "w_v", "w_g", "w_o"))
+            s.epsilon = 1.0
+        return d
 
     @torch.no_grad()
     def run(self, msa, msa_mask, pair, residual: bool):
         p = self.packed()
+        if self.native:
+            return ops.msa_attention(p["block"], msa.contiguous(), msa_mask, pair.contiguous(), residual)
         a, n, c = msa.shape
         h, d = self.num_head, self.value_dim
         x = ops.layer_norm(msa.contiguous(), p["ln_w"], p["ln_b"])
         logits = ops.pair_logits(pair.contiguous(), p["pn_w"], p["pn_b"], p["w_logits"], h)     # [h, q, k] fp32
         # softmax over the keys of logits + 1e9 (key mask - 1), bf16, rows padded to a multiple of 8
         w = ops.masked_softmax_rows(logits, msa_mask.float().max(dim=0).values.contiguous())        # [h, q, k]
-        if n % 8 == 0 and (a * n) % 8 == 0 and c % 8 == 0:
-            # Everything with the tokens innermost: the value and gate projections are taken
-            # transposed (weights as the left operand), [(h, d), (row, k)], which is per head the
-            # k-contiguous right operand of the averaging product; its result [(h, d), (row, q)]
-            # has the same layout, takes the gate there and is transposed once for the output projection.
-            x2 = x.view(a * n, c)
-            v_t = ops.linear(p["w_v"], x2)                                                        # [(h d), (row, k)]
-            gate_t = ops.linear(p["w_g"], x2, sigmoid=True)
-            avg_t = ops.batched_nt_product(v_t.view(h, d * a, n), w)                              # [h, (d, row), q]
-            avg = ops.transpose2d(avg_t.view(c, a * n) * gate_t).view(a, n, c)
-        else:
-            v = ops.linear(x, p["w_v"])                                                           # [a, k, (h d)]
-            gate = ops.linear(x, p["w_g"], sigmoid=True)
-            vt = _pad_last(v.view(a, n, h, d).permute(2, 0, 3, 1).reshape(h, a * d, n)).contiguous()
-            avg = ops.batched_nt_product(w, vt)                                                   # [h, q, (row, d)]
-            avg = avg.view(h, n, a, d).permute(2, 1, 0, 3).reshape(a, n, c) * gate
+        v = ops.linear(x, p["w_v"])                                                               # [a, k, (h d)]
+        gate = ops.linear(x, p["w_g"], sigmoid=True)
+        vt = _pad_last(v.view(a, n, h, d).permute(2, 0, 3, 1).reshape(h, a * d, n)).contiguous()
+        avg = ops.batched_nt_product(w, vt)                                                       # [h, q, (row, d)]
+        avg = avg.view(h, n, a, d).permute(2, 1, 0, 3).reshape(a, n, c) * gate
         if residual:
             return ops.linear(avg, p["w_o"], out_dtype=msa.dtype, mode=ops._L.LINEAR_GATE_RES, residual=msa, out=msa)
         return ops.linear(avg, p["w_o"], out_dtype=msa.dtype)
@@ -179,8 +194,36 @@ class EvoformerBlock(HipModule):
         self.pair_attention2 = GridSelfAttention(c_pair=c_pair, num_head=n_heads_pair, transpose=True)
         self.pair_transition = Transition(c_x=c_pair)
 
+        self._native = None
+
     def _pack(self):
         return {}
+
+    @property
+    def one_call(self) -> bool:
+        """Whether the whole block runs as one call of the library (`native`)."""
+        return (self.outer_product_mean.native and self.msa_attention1.native and self.msa_transition.narrow
+                and self.pair_attention1.fused)
+
+    def native(self) -> "L.MsaBlockStruct":
+        """The packed weights of the block's modules as the library's structure; made again when any of them has been
+        packed again."""
+        tm = (self.triangle_multiplication_outgoing, self.triangle_multiplication_incoming)
+        ta = (self.pair_attention1, self.pair_attention2)
+        mods = (self.outer_product_mean, self.msa_attention1, self.msa_transition, *tm, *ta, self.pair_transition)
+        packs = [m.packed() for m in mods]
+        if self._native is not None and all(a is b for a, b in zip(self._native[1], packs)):
+            return self._native[0]
+        s = L.MsaBlockStruct()
+        for src in (packs[1]["block"], packs[0]["block"]):      # (epsilon is the outer-product mean's)
+            for name, _ in s._fields_:
+                if name != "pair" and getattr(src, name):
+                    setattr(s, name, getattr(src, name))
+        s.mt_ln_w, s.mt_ln_b, s.mt_w1, s.mt_w2 = (packs[2][k].data_ptr() for k in ("ln_w64", "ln_b64", "w1_64", "w2_64"))
+        s.mt_hidden = packs[2]["w2_64"].shape[1]
+        fill_pair_weights(s.pair, tm, ta, self.pair_transition, self.c_pair)
+        self._native = (s, packs)
+        return s
 
     @torch.no_grad()
     def forward(self, msa: torch.Tensor, pair: torch.Tensor, msa_mask: torch.Tensor, pair_mask: torch.Tensor):
@@ -198,6 +241,9 @@ class EvoformerBlock(HipModule):
             return msa, pair
         if not (pair.is_contiguous() and msa.is_contiguous()):
             raise ValueError("msa and pair must be contiguous (they are updated in place)")
+        if self.one_call:
+            ops.evoformer_stack([self.native()], msa, pair, msa_mask, pair_mask)
+            return msa, pair
         self.outer_product_mean.run(msa, msa_mask, residual=pair)
         self.msa_attention1.run(msa, msa_mask, pair, residual=True)
         self.msa_transition.run(msa, residual=True)
@@ -207,6 +253,19 @@ class EvoformerBlock(HipModule):
         self.pair_attention2.run(pair, pair_mask, residual=True)
         self.pair_transition.run(pair, residual=True)
         return msa, pair
+
+
+def evoformer_loop(blocks, msa, pair, msa_mask, pair_mask):
+    """Run Evoformer blocks one after the other (d_alphafold3.py:228-231), in one call where they allow it."""
+    blocks = list(blocks)
+    if (not in_check_mode() and pair.is_cuda and len(blocks) > 1 and msa.is_contiguous() and pair.is_contiguous()
+            and all(type(b) is EvoformerBlock and b.one_call and
+                    b.outer_product_mean.epsilon == blocks[0].outer_product_mean.epsilon for b in blocks)):
+        ops.evoformer_stack([b.native() for b in blocks], msa, pair, msa_mask, pair_mask)
+        return msa, pair
+    for blk in blocks:
+        msa, pair = blk(msa=msa, pair=pair, msa_mask=msa_mask, pair_mask=pair_mask)
+    return msa, pair
 
 
 # ------------------------------------------------------------ fp32 check mode

@@ -16,6 +16,21 @@ from .primitives import Transition
 from .triangle_multiplication import TriangleMultiplication
 
 
+def fill_pair_weights(s, tm, ta, transition, c_pair) -> None:
+    """The pair operators' packed weights into an af3_pairformer_block: triangle multiplications (outgoing, incoming),
+    triangle attentions (starting, ending node), pair transition."""
+    for d in (0, 1):
+        p, q = tm[d].packed(), ta[d].packed()
+        for name, t in (("tm_ln_in_w", p["ln_in_w"]), ("tm_ln_in_b", p["ln_in_b"]), ("tm_ln_c_w", p["ln_c_w"]),
+                        ("tm_ln_c_b", p["ln_c_b"]), ("tm_w_proj_gate", p["w_proj_gate"]), ("tm_w_out", p["w_out"]),
+                        ("tm_w_gating", p["w_gl"]), ("ta_ln_w", q["ln_w"]), ("ta_ln_b", q["ln_b"]),
+                        ("ta_w_bias", q["w_bias"]), ("ta_w_qkvg", q["w_qkvg"]), ("ta_w_out", q["w_out"])):
+            getattr(s, name)[d] = t.data_ptr()
+    p = transition.packed()
+    s.pt_ln_w, s.pt_ln_b, s.pt_w1, s.pt_w2 = (p[k].data_ptr() for k in ("ln_w", "ln_b", "w1", "w2"))
+    s.valid_channels, s.num_head_pair, s.pair_hidden = c_pair, ta[0].num_head, p["w2"].shape[1]
+
+
 class PairformerBlock(HipModule):
     """Same constructor keywords, sub-module names and call signature as the
     reference's DistributePairformerBlock (nn/d_pairformer.py:32-106).
@@ -74,16 +89,7 @@ class PairformerBlock(HipModule):
             return self._native[0]
         by = dict(zip(mods, packs))
         s = L.PairformerBlockStruct()
-        for d in (0, 1):
-            p, q = by[tm[d]], by[ta[d]]
-            for name, t in (("tm_ln_in_w", p["ln_in_w"]), ("tm_ln_in_b", p["ln_in_b"]), ("tm_ln_c_w", p["ln_c_w"]),
-                            ("tm_ln_c_b", p["ln_c_b"]), ("tm_w_proj_gate", p["w_proj_gate"]), ("tm_w_out", p["w_out"]),
-                            ("tm_w_gating", p["w_gl"]), ("ta_ln_w", q["ln_w"]), ("ta_ln_b", q["ln_b"]),
-                            ("ta_w_bias", q["w_bias"]), ("ta_w_qkvg", q["w_qkvg"]), ("ta_w_out", q["w_out"])):
-                getattr(s, name)[d] = t.data_ptr()
-        p = by[self.pair_transition]
-        s.pt_ln_w, s.pt_ln_b, s.pt_w1, s.pt_w2 = (p[k].data_ptr() for k in ("ln_w", "ln_b", "w1", "w2"))
-        s.valid_channels, s.num_head_pair, s.pair_hidden = self.c_pair, ta[0].num_head, p["w2"].shape[1]
+        fill_pair_weights(s, tm, ta, self.pair_transition, self.c_pair)
         s.with_single = int(self.with_single)
         if self.with_single:
             p = by[self]

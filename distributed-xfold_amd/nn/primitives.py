@@ -37,16 +37,26 @@ class Transition(HipModule):
         """Fewer than 128 channels: run on the fused 128-channel kernel with zero-padded operands."""
         return self.c_x < 128
 
+    @property
+    def narrow(self) -> bool:
+        """The MSA's width: a kernel of its own on the rows as they are."""
+        hidden = self.num_intermediate_factor * self.c_x
+        return self.c_x == 64 and hidden % 32 == 0 and hidden <= 256
+
     def _pack(self):
         if self.padded:
             hidden = self.num_intermediate_factor * self.c_x
             hp = (hidden + 63) // 64 * 64            # zero hidden units give silu(0) * 0 = 0
             w1 = self.transition1.weight.detach()
             w1p = torch.cat([pad_to(w1[:hidden], hp, 128), pad_to(w1[hidden:], hp, 128)], dim=0)
-            return dict(ln_w=f32(pad_to(self.input_layer_norm.weight, 128)),
-                        ln_b=f32(pad_to(self.input_layer_norm.bias, 128)),
-                        w1=bf16(pack_swiglu(w1p, 64)).reshape(hp // 64, 128, 128),
-                        w2=bf16(pad_to(self.transition2.weight, 128, hp)))
+            d = dict(ln_w=f32(pad_to(self.input_layer_norm.weight, 128)),
+                     ln_b=f32(pad_to(self.input_layer_norm.bias, 128)),
+                     w1=bf16(pack_swiglu(w1p, 64)).reshape(hp // 64, 128, 128),
+                     w2=bf16(pad_to(self.transition2.weight, 128, hp)))
+            if self.narrow:
+                d.update(ln_w64=f32(self.input_layer_norm.weight), ln_b64=f32(self.input_layer_norm.bias), w1_64=bf16(w1),
+                         w2_64=bf16(self.transition2.weight))
+            return d
         d = dict(ln_w=f32(self.input_layer_norm.weight), ln_b=f32(self.input_layer_norm.bias),
                  w2=bf16(self.transition2.weight))
         if self.c_x == 128:
@@ -63,6 +73,9 @@ class Transition(HipModule):
                                  valid_channels=self.c_x)
 
     def run(self, x, residual: bool):
+        if self.narrow:
+            p = self.packed()
+            return ops.transition64(x, p["ln_w64"], p["ln_b64"], p["w1_64"], p["w2_64"], residual)
         if self.padded:
             res = self.run_padded(pad_channels(x), residual)[..., :self.c_x]
             if residual:

@@ -20,7 +20,7 @@ import torch.nn.functional as F
 from .. import check, ops
 from .base import HipModule, bf16, drop_mesh, f32, in_check_mode
 from .diffusion_head import create_relative_encoding
-from .evoformer import EvoformerBlock
+from .evoformer import EvoformerBlock, evoformer_loop
 from .pairformer import PairformerBlock, pairformer_loop
 
 
@@ -126,8 +126,7 @@ class Evoformer(HipModule):
         msa = self._lin(batch.msa_feat, self.msa_activations, p["w_msa"])
         msa = (msa + self._lin(target_feat, self.extra_msa_target_feat, p["w_tf_msa"])[None]).to(dt).contiguous()
         msa_mask = batch.msa_mask.float().contiguous()
-        for blk in self.msa_stack:
-            msa, pair = blk(msa=msa, pair=pair, msa_mask=msa_mask, pair_mask=pair_mask)
+        msa, pair = evoformer_loop(self.msa_stack, msa, pair, msa_mask, pair_mask)
         single = self._lin(target_feat, self.single_activations, p["w_tf_single"])
         if chk:
             single = single + check._lin(check._ln(prev["single"].float().contiguous(),

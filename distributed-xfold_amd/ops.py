@@ -232,6 +232,74 @@ def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incomi
     _L.check(rc, "af3_pairformer_stack_forward")
 
 
+def _msa_inputs(msa, msa_mask):
+    _gpu(msa, "msa")
+    if msa.dim() != 3 or msa.shape[2] != 64:
+        raise ValueError(f"msa: expected [rows, N, 64], got {tuple(msa.shape)}")
+    return _dt(msa), _mask_f32(msa_mask, tuple(msa.shape[:2]), "msa_mask")
+
+
+def outer_product_mean(block, msa, msa_mask, pair, residual):
+    """af3_outer_product_mean_forward into `pair` [N, N, 128]; `block`: an af3_msa_block structure."""
+    lib = _L.load()
+    dt, maskf = _msa_inputs(msa, msa_mask)
+    rows, n, _ = msa.shape
+    _gpu(pair, "pair", shape=(n, n, 128))
+    ws = _ws(lib.af3_msa_workspace_bytes(rows, n), msa.device)
+    rc = lib.af3_outer_product_mean_forward(ctypes.addressof(block), _p(msa), dt, _p(maskf), _p(pair), _dt(pair),
+                                            int(residual), rows, n, _p(ws), ws.numel(), _stream(msa.device))
+    _L.check(rc, "af3_outer_product_mean_forward")
+    return pair
+
+
+def msa_attention(block, msa, msa_mask, pair, residual):
+    """af3_msa_attention_forward -> `msa` updated in place (residual) or a new tensor."""
+    lib = _L.load()
+    dt, maskf = _msa_inputs(msa, msa_mask)
+    rows, n, _ = msa.shape
+    _gpu(pair, "pair", shape=(n, n, 128))
+    out = msa if residual else torch.empty_like(msa)
+    ws = _ws(lib.af3_msa_workspace_bytes(rows, n), msa.device)
+    rc = lib.af3_msa_attention_forward(ctypes.addressof(block), _p(msa), dt, _p(maskf), _p(pair), _dt(pair), _p(out),
+                                       int(residual), rows, n, _p(ws), ws.numel(), _stream(msa.device))
+    _L.check(rc, "af3_msa_attention_forward")
+    return out
+
+
+def transition64(x, ln_weight, ln_bias, w1, w2, residual):
+    """Transition of 64-channel rows, weights in their natural order -> `x` updated in place or a new tensor."""
+    lib = _L.load()
+    _gpu(x, "x")
+    hidden = w2.shape[1]
+    for nm, t, dt, shape in (("ln_weight", ln_weight, torch.float32, (64,)), ("ln_bias", ln_bias, torch.float32, (64,)),
+                             ("w1", w1, torch.bfloat16, (2 * hidden, 64)), ("w2", w2, torch.bfloat16, (64, hidden))):
+        _gpu(t, nm, dt, shape)
+    if x.shape[-1] != 64:
+        raise ValueError("x: last dimension must be 64")
+    out = x if residual else torch.empty_like(x)
+    rc = lib.af3_transition64_forward(_p(x), _dt(x), _p(ln_weight), _p(ln_bias), _p(w1), _p(w2), hidden, _p(out),
+                                      int(residual), x.numel() // 64, _stream(x.device))
+    _L.check(rc, "af3_transition64_forward")
+    return out
+
+
+def evoformer_stack(blocks, msa, pair, msa_mask, pair_mask):
+    """A run of Evoformer blocks in one call, msa [rows, N, 64] and pair [N, N, 128] updated in place."""
+    lib = _L.load()
+    dt, maskf = _msa_inputs(msa, msa_mask)
+    rows, n, _ = msa.shape
+    _gpu(pair, "pair", shape=(n, n, 128))
+    pmf = _mask_f32(pair_mask, (n, n), "pair_mask")
+    need = lib.af3_msa_workspace_bytes(rows, n)
+    pws = lib.af3_pairformer_stack_workspace_bytes(n, blocks[0].pair.num_head_pair)
+    split = (need + 255) // 256 * 256
+    ws = _ws(split + pws, msa.device)
+    ptrs = (ctypes.c_void_p * len(blocks))(*[ctypes.addressof(b) for b in blocks])
+    rc = lib.af3_evoformer_stack_forward(ptrs, len(blocks), _p(msa), dt, _p(maskf), _p(pair), _dt(pair), _p(pmf), rows, n,
+                                         _p(ws), split, _p(ws) + split, pws, _stream(msa.device))
+    _L.check(rc, "af3_evoformer_stack_forward")
+
+
 def diffusion_transformer(blocks, act, mask, pair_logits, scale_shift, gate, num_head, hidden):
     """The blocks of the diffusion transformer in one call (af3_diffusion_transformer_forward), act [B, S, C] updated
     in place.  `blocks`: an array of lib.DiffusionBlockStruct; pair_logits: one fp32 tensor per block, [H, S, S] or

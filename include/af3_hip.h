@@ -536,6 +536,52 @@ int af3_pairformer_stack_forward(
     void* single_workspace, size_t single_workspace_bytes, af3_stream_t stream, af3_stream_t single_stream, int join);
 
 /* ---------------------------------------------------------------------------
+ * The Evoformer's MSA track on 64 channels (nn/d_primitives.py:42-70,
+ * nn/d_attention.py:113-156, nn/d_pairformer.py:174-252): msa [rows,n,64] and pair
+ * [n,n,128] in their own dtypes, msa_mask [rows,n], pair_mask [n,n] or NULL.
+ *
+ * af3_outer_product_mean_forward: pair = (residual ? pair : 0) + the outer-product mean.
+ * af3_msa_attention_forward: out = (residual ? msa : 0) + the pair-weighted average
+ *   of 8 heads; out may be msa.
+ * af3_transition64_forward: out = (residual ? x : 0) + transition(x) on rows of 64
+ *   channels, hidden <= 256 units (a multiple of 32); out may be x.
+ * af3_evoformer_stack_forward: a run of blocks, msa and pair updated in place; the
+ *   incoming triangle multiplication takes the transposed pair mask (:217), the pair
+ *   operators scratch of af3_pairformer_stack_workspace_bytes.
+ * epsilon is the same in all blocks of a run.
+ */
+typedef struct af3_msa_block {
+  const float *opm_ln_w, *opm_ln_b;
+  const uint16_t* opm_w_lr;  /* [64][64]: left, then right projection */
+  /* output weights W [128][1024] (column 32 c + e of the outer product) in the order of the kernel's loads:
+   * [f / 32][k / 16][(k / 8) % 2][l][k % 8] = W[f][k] where l = f % 32 with its bits 2 and 3 exchanged */
+  const uint16_t* opm_w_out;
+  const float* opm_b_out;
+  const float *ma_ln_w, *ma_ln_b, *ma_pn_w, *ma_pn_b;
+  const uint16_t* ma_w_logits;                /* [32][128], rows 8.. zero */
+  const uint16_t *ma_w_v, *ma_w_g, *ma_w_o;   /* [64][64] */
+  const float *mt_ln_w, *mt_ln_b;
+  const uint16_t *mt_w1, *mt_w2;              /* [2 hidden][64], the silu half first; [64][hidden] */
+  af3_pairformer_block pair;                  /* with_single = 0 */
+  int32_t mt_hidden;
+  float epsilon;
+} af3_msa_block;
+size_t af3_msa_workspace_bytes(int64_t rows, int64_t n_token);
+int af3_outer_product_mean_forward(
+    const af3_msa_block* block, const void* msa, int msa_dtype, const float* msa_mask, void* pair, int pair_dtype,
+    int residual, int64_t rows, int64_t n_token, void* workspace, size_t workspace_bytes, af3_stream_t stream);
+int af3_msa_attention_forward(
+    const af3_msa_block* block, const void* msa, int msa_dtype, const float* msa_mask, const void* pair, int pair_dtype,
+    void* out, int residual, int64_t rows, int64_t n_token, void* workspace, size_t workspace_bytes, af3_stream_t stream);
+int af3_transition64_forward(
+    const void* x, int io_dtype, const float* ln_w, const float* ln_b, const uint16_t* w1, const uint16_t* w2, int hidden,
+    void* out, int residual, int64_t rows, af3_stream_t stream);
+int af3_evoformer_stack_forward(
+    const af3_msa_block* const* blocks, int num_blocks, void* msa, int msa_dtype, const float* msa_mask,
+    void* pair, int pair_dtype, const float* pair_mask, int64_t rows, int64_t n_token, void* workspace,
+    size_t workspace_bytes, void* pair_workspace, size_t pair_workspace_bytes, af3_stream_t stream);
+
+/* ---------------------------------------------------------------------------
  * The blocks of the diffusion transformer (nn/d_diffusion_transformer.py:267-310)
  * and of the windowed atom transformer (:466-543) as one call each, act updated in
  * place.  The conditioning enters as the caller has projected it for all blocks at
