@@ -151,19 +151,12 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
   const int wm = (wave >> 1) * WM, wn = (wave & 1) * 128;
 
   // The workgroups are persistent (one per CU) and walk their tiles in a fixed order.
-  // XCD-aware mapping: workgroup ids are dealt round-robin to the 8 XCDs, so
-  // id -> (xcd, slot) -> logical id makes each XCD walk a contiguous range of
-  // (channel, j-tile, i-tile), i-tile fastest: the tiles that share a channel's
-  // A and B panels run on one XCD at about the same time and find them in its L2.
+  // Workgroup ids are dealt round-robin to the 8 XCDs: id -> (xcd, slot) -> tile (XcdWalk), so that the tiles that
+  // share a panel of A or B run on one XCD at about the same time and find it in its L2.
   const int tiles_m = (g.M + CM - 1) / CM, tiles_n = (g.N + CN - 1) / CN;
   const int total = tiles_m * tiles_n * g.batch;
   const int per_xcd = (total + 7) / 8;
   const int xcd = blockIdx.x & 7, slot_step = gridDim.x >> 3;
-  // One large product: an XCD that walks whole columns of tiles re-reads all of
-  // A for every column, and A (8 MB at 4096 x 1024) does not stay in its 4 MB
-  // L2.  Deal the XCDs a 4 x 2 grid of rectangles instead: a quarter of A stays
-  // resident while the XCD streams through its half of B once.
-  const bool rect = g.batch == 1 && (tiles_m & 3) == 0 && (tiles_n & 1) == 0;
   struct Tile { int m0, n0, bz; };
   auto tile_at = [&](int& slot, Tile& t) -> bool {
     if constexpr (MODE == BIG_OUTER_MEAN) {
@@ -179,14 +172,16 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
         if (tm < tiles_m && tn < tiles_n) return true;
       }
     }
-    const int logical = xcd * per_xcd + slot;
-    if (slot >= per_xcd || logical >= total) return false;
-    int tm = logical % tiles_m, tn = (logical / tiles_m) % tiles_n;
-    t.bz = logical / (tiles_m * tiles_n);
-    if (rect) {
-      const int mq = tiles_m >> 2, nh = tiles_n >> 1;
-      tm = (xcd & 3) * mq + slot % mq;
-      tn = (xcd >> 2) * nh + slot / mq;
+    int tm, tn;
+    t.bz = 0;
+    if (g.xcd_m) {
+      if (!xcd_rect_tile(g.xcd_m, xcd, slot, tiles_m, tiles_n, &tm, &tn)) return false;
+    } else {
+      const int logical = xcd * per_xcd + slot;
+      if (slot >= per_xcd || logical >= total) return false;
+      tm = logical % tiles_m;
+      tn = (logical / tiles_m) % tiles_n;
+      t.bz = logical / (tiles_m * tiles_n);
     }
     // (the divisions above go through the vector unit; say again that the results are uniform)
     t.m0 = __builtin_amdgcn_readfirstlane(tm * CM);
@@ -702,7 +697,8 @@ static int cu_count() {
   return cus;
 }
 
-int launch_big_tile(const GemmArgs& g, int mode, hipStream_t stream) {
+int launch_big_tile(const GemmArgs& g_in, int mode, hipStream_t stream) {
+  GemmArgs g = g_in;
   if (!g.A || !g.B || !g.C) return AF3_ERR_BAD_ARG;
   if (mode != big_tile_mode(g) && !(mode == BIG_PLAIN && contract_supported(g))) return AF3_ERR_BAD_ARG;
   if (mode < BIG_PLAIN || mode > BIG_SWIGLU) return AF3_ERR_BAD_ARG;
@@ -721,10 +717,11 @@ int launch_big_tile(const GemmArgs& g, int mode, hipStream_t stream) {
   // N = 256 .. 576, not 768 (six rounds against five) or beyond.
   const int cus = cu_count();
   const bool flat = ((total3 + cus - 1) / cus) * 7 < ((total4 + cus - 1) / cus) * 8;
-  const int64_t total = flat ? total3 : total4;
-  if (total > 0x3fffffff) return AF3_ERR_BAD_ARG;
+  const XcdWalk walk = xcd_walk((g.M + (flat ? 191 : 255)) / (flat ? 192 : 256), tiles_n, g.batch, flat ? 192 : 256, CN);
+  if (walk.slots * 8 > 0x3fffffff) return AF3_ERR_BAD_ARG;
+  g.xcd_m = walk.rows;
   // persistent workgroups, one per CU (a multiple of 8: ids are dealt round-robin to the 8 XCDs)
-  const int64_t blocks = std::min<int64_t>((total + 7) / 8 * 8, std::max(cus / 8 * 8, 8));
+  const int64_t blocks = std::min<int64_t>(walk.slots * 8, cus / 8 * 8);
   const dim3 grid((unsigned)blocks), block(256);
   if (flat && mode == BIG_PLAIN) hipLaunchKernelGGL((contract_kernel<BIG_PLAIN, 3>), grid, block, 0, stream, g);
   else if (flat && mode == BIG_COLUMN_OPS) hipLaunchKernelGGL((contract_kernel<BIG_COLUMN_OPS, 3>), grid, block, 0, stream, g);

@@ -89,18 +89,20 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArg
   const int grp = wave / GW, gw = wave % GW;
   const int wm = (gw / WN) * 32 * MT, wn = (gw % WN) * 32 * NT;
 
-  // XCD-aware mapping: workgroup ids are dealt round-robin to the 8 XCDs, so
-  // id -> (xcd, slot) -> logical id makes each XCD walk a contiguous range of
-  // (batch, n-tile, m-tile), m-tile fastest: the tiles that share a batch's A
-  // and B panels run on one XCD and find them in its L2.
+  // Workgroup ids are dealt round-robin to the 8 XCDs: id -> (xcd, slot) -> tile (XcdWalk).
   const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
-  const int total = tiles_m * tiles_n * g.batch;
-  const int per_xcd = (total + 7) / 8;
-  const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per_xcd || logical >= total) return;
-  const int m0 = __builtin_amdgcn_readfirstlane(logical % tiles_m) * BM;
-  const int n0 = __builtin_amdgcn_readfirstlane((logical / tiles_m) % tiles_n) * BN;
-  const int bz = __builtin_amdgcn_readfirstlane(logical / (tiles_m * tiles_n));
+  int tm, tn, bz = 0;
+  if (g.xcd_m) {
+    if (!xcd_rect_tile(g.xcd_m, blockIdx.x & 7, blockIdx.x >> 3, tiles_m, tiles_n, &tm, &tn)) return;
+  } else {
+    const int total = tiles_m * tiles_n * g.batch, per_xcd = (total + 7) / 8;
+    const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || logical >= total) return;
+    tm = logical % tiles_m;
+    tn = (logical / tiles_m) % tiles_n;
+    bz = __builtin_amdgcn_readfirstlane(logical / (tiles_m * tiles_n));
+  }
+  const int m0 = __builtin_amdgcn_readfirstlane(tm) * BM, n0 = __builtin_amdgcn_readfirstlane(tn) * BN;
 
   // the tile's first rows: what a lane adds to these fits 32 bits whatever the operands' size
   const u32x4 A = buffer_of(g.A + (int64_t)bz * g.sA + (int64_t)m0 * g.lda);
@@ -349,11 +351,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArg
 }
 
 template <int MT, int NT, int WM, int WN, int WK, int ST, int WPS, bool CLEAN = true, bool VEC = true>
-int launch_tile(const GemmArgs& g, hipStream_t stream) {
+int launch_tile(GemmArgs g, hipStream_t stream) {
   constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN;
-  const int64_t total = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN) * g.batch;
-  const int64_t blocks = (total + 7) / 8 * 8;
+  const XcdWalk walk = xcd_walk((g.M + BM - 1) / BM, (g.N + BN - 1) / BN, g.batch, BM, BN);
+  const int64_t blocks = walk.slots * 8;
   if (blocks > 0x3fffffff) return AF3_ERR_BAD_ARG;
+  g.xcd_m = walk.rows;
   const dim3 grid((unsigned)blocks), block(64 * WM * WN * WK);
 #define LAUNCH(KIND, OUT_F32) hipLaunchKernelGGL((gemm_nt_kernel<MT, NT, WM, WN, WK, ST, WPS, CLEAN, KIND, VEC, OUT_F32>), grid, block, 0, stream, g)
   if (g.epi == EPI_SWIGLU) {
@@ -372,12 +375,31 @@ int launch_tile(const GemmArgs& g, hipStream_t stream) {
 
 }  // namespace
 
+// Wide products whose tiles come out just below a whole number per CU (256 CUs), which is worth more than the tile's
+// bytes per FLOP: one product's tiles all run at once, and a few tiles more than that cost another round.  Eight waves.
+//   128x128, one per CU, four slab buffers   200 < T <= 256 tiles (1250x3072x768 14.5 us, was 16.0; SwiGLU 11.4, 14.3;
+//                                            4200x768x1536 22.6, 26.7); not the short ones with gate and residual
+//   128x192, one per CU                      where that many hold the product (1700x3072x768 17.6, 18.6; SwiGLU 12.8, 15.4;
+//                                            5400x768x1536 25.1, 30.5)
+//   128x128, two per CU                      352 < T <= 512 (2300x3072x768 20.7, 26.4; SwiGLU 16.7, 21.5;
+//                                            9000x768x1536 31.2, 47.0)
+enum { MID_NONE = 0, MID_128_ONE, MID_192, MID_128_TWO };
+static int mid_tile_choice(const GemmArgs& g) {
+  if (g.batch != 1 || (g.K % KS) || g.M <= 128 || g.N <= 128) return MID_NONE;
+  const int64_t rows = (g.M + 127) / 128, t128 = rows * ((g.N + 127) / 128), t192 = rows * ((g.N + 191) / 192);
+  const bool swiglu = g.epi == EPI_SWIGLU, gated = g.epi == EPI_GATE_RES;
+  if (g.K >= 512 && t128 > (swiglu ? 190 : 200) && t128 <= 256 && (!gated || g.K >= 1024)) return MID_128_ONE;
+  if (g.K >= 512 && g.N >= 768 && t128 > 256 && t192 <= 256) return MID_192;
+  return t128 > 352 && t128 <= 512 ? MID_128_TWO : MID_NONE;
+}
+
 // Products of at least 120 tiles of 256x256 go to the large-tile kernel where one of its epilogues fits: a
 // 128x128 tile of the kernel above needs twice the fragment reads per MFMA and is bound by them from there on
-// (3840x3072x768: 34 us against 25; 1920x3072x768, 96 such tiles: 17 against 23 the other way).
+// (3840x3072x768: 34 us against 26).
 int gemm_big_tile_choice(const GemmArgs& g) {
   constexpr int64_t BIG_TILE_MIN_TILES = 120;
   const int64_t tiles = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256) * g.batch;
+  if (mid_tile_choice(g) != MID_NONE) return -1;
   return g.M > 128 && g.N > 128 && tiles >= BIG_TILE_MIN_TILES ? big_tile_mode(g) : -1;
 }
 
@@ -417,6 +439,7 @@ int launch_gemm_nt(const GemmArgs& g_in, hipStream_t stream) {
   //              waves, or eight where it is long
   //   T <= 384   with split_k: 64x64, K split two ways (eight waves per tile); long ones are faster unsplit
   //   T <= 1000  64x64, with as many slab buffers as leave room for the workgroups a CU gets: four, three or two
+  //              (a SwiGLU of more than 352: 128x64, two of whose tiles a CU holds; 500x3072x768 8.5 us, was 9.3)
   //   T <= 2600  64x128, else 128x128: bytes per FLOP count once every CU has several tiles (and never wider than N)
   const int64_t T = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch;
   const bool wide = g.epi == EPI_SWIGLU;
@@ -426,8 +449,14 @@ int launch_gemm_nt(const GemmArgs& g_in, hipStream_t stream) {
     if (T <= 128 && !wide) return g.K >= 1024 ? launch_tile<1, 1, 1, 1, 8, 2, 2>(g, stream) : launch_tile<1, 1, 1, 1, 4, 2, 2>(g, stream);
     if (T <= 384 && g.K < 1024) return launch_tile<1, 1, 2, 2, 2, 2, 4>(g, stream);
   }
+  switch (mid_tile_choice(g)) {
+    case MID_128_ONE: return launch_tile<1, 2, 4, 2, 1, 4, 2>(g, stream);
+    case MID_192: return launch_tile<1, 3, 4, 2, 1, 3, 2>(g, stream);
+    case MID_128_TWO: return launch_tile<1, 2, 4, 2, 1, 2, 4>(g, stream);
+  }
   if (T <= 128 && !wide) return launch_tile<1, 1, 1, 1, 1, 4, 1>(g, stream);
   if (T <= 256) return launch_tile<1, 1, 2, 2, 1, 4, 2>(g, stream);
+  if (T > 352 && T <= 640 && wide) return launch_tile<2, 1, 2, 2, 1, 3, 2>(g, stream);
   if (T <= 640) return launch_tile<1, 1, 2, 2, 1, 3, 3>(g, stream);
   if (T <= 1000 || g.N <= 64) return launch_tile<1, 1, 2, 2, 1, 2, 4>(g, stream);
   if (T <= 2600 || g.N <= 128) return launch_tile<1, 2, 2, 2, 1, 2, 3>(g, stream);

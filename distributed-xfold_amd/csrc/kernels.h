@@ -32,9 +32,47 @@ struct GemmArgs {
   // the outer products of 32-channel rows, one contiguous 1024-vector per pair.
   int regroup32 = 0;
   const bf16_t* w2 = nullptr;  // launch_outer_mean only
+  int xcd_m = 0;               // set by the launchers: XcdWalk::rows
   int split_k = 0;  // the K range may be summed in parts by several waves (another order of summation)
 };
 int launch_gemm_nt(const GemmArgs& g, hipStream_t stream);
+
+// Which tiles of a product run on which XCD.  Each XCD has an L2 of its own, 4 MB, and fetches for itself every row of A
+// and B that its tiles touch.  rows = 0: the XCDs share the tiles (batch, n, m), m fastest, in eight runs: every XCD
+// fetches all of A for an eighth of B, right for few rows and for many small products.  rows = 1, 2, 4 or 8: one
+// product's tiles are dealt as a rows x (8 / rows) grid of rectangles, an XCD fetches 1 / rows of A and rows / 8 of B.
+struct XcdWalk {
+  int rows = 0;
+  int64_t slots = 0;  // tiles of the busiest XCD
+};
+// The walk that fetches least, if that is at least a third less and no XCD gets 4 % more tiles than its share: an uneven
+// deal costs what it saves (1920 x 768 x 1536 in 64 x 64 tiles: 48 tiles against 45, 16.8 us against 15.4).
+// 3840 x 768 x 768 14.3 -> 12.4 us, 3840 x 768 x 1536 24.1 -> 22.0, 3200 x 768 x 1536 22.9 -> 20.5.
+inline XcdWalk xcd_walk(int64_t tiles_m, int64_t tiles_n, int64_t batch, int bm, int bn) {
+  XcdWalk w;
+  w.slots = (tiles_m * tiles_n * batch + 7) / 8;
+  if (batch != 1) return w;
+  int64_t least = (w.slots < tiles_m ? w.slots : tiles_m) * bm + ((w.slots + tiles_m - 1) / tiles_m) * bn;
+  const int64_t limit = least * 2 / 3;
+  for (int rows = 1; rows <= 8; rows *= 2) {
+    const int64_t m = (tiles_m + rows - 1) / rows, n = (tiles_n + 8 / rows - 1) / (8 / rows), fetch = m * bm + n * bn;
+    if (m * n * 25 > w.slots * 26 || fetch > limit || fetch >= least) continue;
+    least = fetch;
+    w.rows = rows;
+  }
+  if (w.rows) w.slots = ((tiles_m + w.rows - 1) / w.rows) * ((tiles_n + 8 / w.rows - 1) / (8 / w.rows));
+  return w;
+}
+// tile number `slot` of an XCD's rectangle; false behind its last
+__device__ __forceinline__ bool xcd_rect_tile(int rows, int xcd, int slot, int tiles_m, int tiles_n, int* tm, int* tn) {
+  const int cols = 8 / rows, i = xcd & (rows - 1), j = xcd / rows;
+  const int m0 = tiles_m * i / rows, mh = tiles_m * (i + 1) / rows - m0;
+  const int n0 = tiles_n * j / cols, nh = tiles_n * (j + 1) / cols - n0;
+  if (slot >= mh * nh) return false;
+  *tm = m0 + slot % mh;
+  *tn = n0 + slot / mh;
+  return true;
+}
 // af3_linear_forward and af3_batch_diffusion_self_attention_forward (api.hip) for callers inside the library that do
 // not mind the order in which the products sum K (GemmArgs::split_k)
 int run_linear(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int y_dtype, int64_t m, int n, int k, int mode,
