@@ -406,7 +406,14 @@ int af3_atom_pair_cond_forward(const float* row, const float* col, const float* 
 int af3_atom_pair_logits_forward(const float* pair_cond, const float* ln_w, const float* w, float* out, int64_t subsets,
                                  int64_t queries, int64_t keys, int num_blocks, int num_head, af3_stream_t stream) {
   if (queries <= 0 || keys <= 0) return AF3_ERR_BAD_ARG;
-  return launch_atom_pair_logits(pair_cond, ln_w, w, out, subsets, queries * keys, num_blocks, num_head,
+  return launch_atom_pair_logits(pair_cond, ln_w, w, out, subsets, queries, keys, num_blocks, num_head, 0,
+                                 static_cast<hipStream_t>(stream));
+}
+
+int af3_atom_pair_logits_quads_forward(const float* pair_cond, const float* ln_w, const float* w, float* out, int64_t subsets,
+                                       int64_t queries, int64_t keys, int num_blocks, int num_head, af3_stream_t stream) {
+  if (queries <= 0 || keys <= 0) return AF3_ERR_BAD_ARG;
+  return launch_atom_pair_logits(pair_cond, ln_w, w, out, subsets, queries, keys, num_blocks, num_head, 1,
                                  static_cast<hipStream_t>(stream));
 }
 
@@ -545,50 +552,9 @@ int af3_gathered_cross_attention_forward(
     const uint16_t* w_qg, const uint16_t* w_kv, const float* query_b, int num_head,
     void* out, int out_dtype, int64_t batch, int64_t sq, int64_t sk, int64_t samples, int64_t n_atoms, int channels,
     void* workspace, size_t workspace_bytes, af3_stream_t stream) {
-  if (!q_data || !atom_data || !key_rows || !w_qg || !w_kv || !out) return AF3_ERR_BAD_ARG;
-  if (bad_dtype(out_dtype) || batch <= 0 || sq <= 0 || sk <= 0 || samples <= 0 || n_atoms <= 0 || channels <= 0 ||
-      (channels & 7) || num_head <= 0 || channels % num_head)
-    return AF3_ERR_BAD_ARG;
-  if ((mask_q == nullptr) != (mask_k == nullptr)) return AF3_ERR_BAD_ARG;
-  if (bias_batches <= 0 || batch != samples * bias_batches) return AF3_ERR_BAD_ARG;
-  if (batch * sq > 0x7fffffff || samples * n_atoms > 0x7fffffff) return AF3_ERR_BAD_ARG;
-  const int d = channels / num_head;
-  if (d != 24 && d != 32 && d != 48) return AF3_ERR_UNSUPPORTED;
-  Carver ws(workspace, workspace_bytes);
-  bf16_t* qg = ws.take<bf16_t>((size_t)batch * sq * 2 * channels);
-  bf16_t* kv = ws.take<bf16_t>((size_t)samples * n_atoms * 2 * channels);
-  if (!ws.ok) return AF3_ERR_WORKSPACE;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-
-  GemmArgs g;
-  g.A = q_data; g.B = w_qg; g.C = qg;
-  g.M = (int)(batch * sq); g.N = 2 * channels; g.K = channels;
-  g.lda = channels; g.ldb = channels; g.ldc = 2 * channels;
-  g.epi = EPI_SEGMENTED; g.seg_len = channels;
-  g.seg_ops = SEG_BIAS_SCALE | (SEG_SIGMOID << 4);
-  g.alpha = 1.0f / sqrtf((float)d);
-  g.bias = query_b; g.bias_len = channels;  // the query segment's columns only
-  int rc = launch_gemm_nt(g, s);
-  if (rc) return rc;
-  GemmArgs g2;
-  g2.A = atom_data; g2.B = w_kv; g2.C = kv;
-  g2.M = (int)(samples * n_atoms); g2.N = 2 * channels; g2.K = channels;
-  g2.lda = channels; g2.ldb = channels; g2.ldc = 2 * channels;
-  rc = launch_gemm_nt(g2, s);
-  if (rc) return rc;
-
-  FlashArgs f;
-  f.q = qg; f.g = qg + channels; f.k = kv; f.v = kv + channels;
-  f.q_ss = f.g_ss = f.k_ss = f.v_ss = 2 * channels;
-  f.q_sb = f.g_sb = sq * 2 * channels;
-  f.k_sb = f.v_sb = n_atoms * 2 * channels;   // one K / V table per sample
-  f.key_rows = key_rows;
-  f.out = out; f.out_f32 = out_dtype == AF3_F32; f.o_ss = channels; f.o_sb = sq * channels;
-  f.B = (int)batch; f.H = num_head; f.Sq = (int)sq; f.Sk = (int)sk; f.d = d;
-  f.bias = pair_logits; f.bias_sb = (int64_t)num_head * sq * sk; f.bias_sh = sq * sk; f.bias_sq = sk;
-  f.qpad = mask_q; f.kpad = mask_k; f.qp_sb = sq; f.kp_sb = sk;
-  f.bias_mod = (int)bias_batches;
-  return launch_flash_attention(f, s);
+  return run_gathered_attention(q_data, atom_data, key_rows, pair_logits, 0, mask_q, mask_k, bias_batches, w_qg, w_kv, query_b,
+                                num_head, out, out_dtype, batch, sq, sk, samples, n_atoms, channels, workspace, workspace_bytes,
+                                static_cast<hipStream_t>(stream));
 }
 
 // ------------------------------------------------------------------ pair logits
@@ -760,4 +726,58 @@ int run_linear(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int
     g.ld_res = n;
   }
   return launch_gemm_nt(g, stream);
+}
+
+int run_gathered_attention(const bf16_t* q_data, const bf16_t* atom_data, const int32_t* key_rows, const float* pair_logits,
+                           int bias_quad_major, const float* mask_q, const float* mask_k, int64_t bias_batches, const bf16_t* w_qg,
+                           const bf16_t* w_kv, const float* query_b, int num_head, void* out, int out_dtype, int64_t batch,
+                           int64_t sq, int64_t sk, int64_t samples, int64_t n_atoms, int channels, void* workspace,
+                           size_t workspace_bytes, hipStream_t stream) {
+  if (!q_data || !atom_data || !key_rows || !w_qg || !w_kv || !out) return AF3_ERR_BAD_ARG;
+  if (bad_dtype(out_dtype) || batch <= 0 || sq <= 0 || sk <= 0 || samples <= 0 || n_atoms <= 0 || channels <= 0 ||
+      (channels & 7) || num_head <= 0 || channels % num_head)
+    return AF3_ERR_BAD_ARG;
+  if ((mask_q == nullptr) != (mask_k == nullptr)) return AF3_ERR_BAD_ARG;
+  if (bias_quad_major && (sk & 3)) return AF3_ERR_BAD_ARG;
+  if (bias_batches <= 0 || batch != samples * bias_batches) return AF3_ERR_BAD_ARG;
+  if (batch * sq > 0x7fffffff || samples * n_atoms > 0x7fffffff) return AF3_ERR_BAD_ARG;
+  const int d = channels / num_head;
+  if (d != 24 && d != 32 && d != 48) return AF3_ERR_UNSUPPORTED;
+  Carver ws(workspace, workspace_bytes);
+  bf16_t* qg = ws.take<bf16_t>((size_t)batch * sq * 2 * channels);
+  bf16_t* kv = ws.take<bf16_t>((size_t)samples * n_atoms * 2 * channels);
+  if (!ws.ok) return AF3_ERR_WORKSPACE;
+  hipStream_t s = stream;
+
+  GemmArgs g;
+  g.A = q_data; g.B = w_qg; g.C = qg;
+  g.M = (int)(batch * sq); g.N = 2 * channels; g.K = channels;
+  g.lda = channels; g.ldb = channels; g.ldc = 2 * channels;
+  g.epi = EPI_SEGMENTED; g.seg_len = channels;
+  g.seg_ops = SEG_BIAS_SCALE | (SEG_SIGMOID << 4);
+  g.alpha = 1.0f / sqrtf((float)d);
+  g.bias = query_b; g.bias_len = channels;  // the query segment's columns only
+  int rc = launch_gemm_nt(g, s);
+  if (rc) return rc;
+  GemmArgs g2;
+  g2.A = atom_data; g2.B = w_kv; g2.C = kv;
+  g2.M = (int)(samples * n_atoms); g2.N = 2 * channels; g2.K = channels;
+  g2.lda = channels; g2.ldb = channels; g2.ldc = 2 * channels;
+  rc = launch_gemm_nt(g2, s);
+  if (rc) return rc;
+
+  FlashArgs f;
+  f.q = qg; f.g = qg + channels; f.k = kv; f.v = kv + channels;
+  f.q_ss = f.g_ss = f.k_ss = f.v_ss = 2 * channels;
+  f.q_sb = f.g_sb = sq * 2 * channels;
+  f.k_sb = f.v_sb = n_atoms * 2 * channels;   // one K / V table per sample
+  f.key_rows = key_rows; f.table_rows = n_atoms;
+  f.out = out; f.out_f32 = out_dtype == AF3_F32; f.o_ss = channels; f.o_sb = sq * channels;
+  f.B = (int)batch; f.H = num_head; f.Sq = (int)sq; f.Sk = (int)sk; f.d = d;
+  f.bias = pair_logits; f.bias_sb = (int64_t)num_head * sq * sk; f.bias_sh = sq * sk;
+  f.bias_sq = bias_quad_major ? 4 : sk;
+  f.bias_squad = bias_quad_major ? 4 * sq : 0;
+  f.qpad = mask_q; f.kpad = mask_k; f.qp_sb = sq; f.kp_sb = sk;
+  f.bias_mod = (int)bias_batches;
+  return launch_flash_attention(f, s);
 }

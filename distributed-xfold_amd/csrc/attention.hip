@@ -451,6 +451,227 @@ void flash_kernel(FlashArgs a) {
     }
 }
 
+// ------------------------------------------------------------------ windows of gathered keys
+// The atom transformers' attention: many short windows (32 queries, up to 128 keys that are looked up in a table of
+// rows), four heads of 32 channels.  There is next to no arithmetic in one (0.5 MFLOP a head); what counts is the CU's
+// vector memory path, which takes a cache line every two cycles or so, whole or in part, and the number of round trips
+// one after the other.  The form above, a wave per window and head, touches every line many times over (a key's row is
+// 64 bytes to a head, the bias of a lane's query 16 bytes to a load) and goes through rows, K and V, LDS twice.  Here a
+// workgroup of four waves takes the four heads of a window: K and V rows of all heads come as runs of 256 bytes straight
+// into LDS (an empty slot or a key past the end: an offset past the buffer's end, which writes zeros), everything else
+// is asked for at the same time, gate and result travel in 16-byte pieces, and the bias, with quads of keys as the outer
+// index (bias_squad), in whole lines.  The samples' windows of one place, which share the bias, follow each other on
+// one XCD.  The arithmetic is that of flash_kernel, in the same order: the same bits.
+// 2880 windows (768 tokens, 5 samples) 46 us (flash_kernel 80), 1440 windows 27 (45), 375 windows 13.5 (17).
+// In LDS chunk c (16 bytes) of a key's row lies at position c ^ (key % 4 * 4 + key / 4 % 4): fragment reads of 32 keys
+// and the transposing reads of 8 keys x 64 bytes both spread over the banks.
+__device__ __forceinline__ u32x4 table_buffer(const void* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return u32x4{lo, hi & 0xffffu, 0x7fffffffu, 0x00020000u};
+}
+// a's upper half of the wave and b's lower half change places
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
+// TILES: tiles of 64 keys in LDS at a time.  With both (66 KB, two workgroups on a CU) a window is the shortest chain;
+// with one after the other a CU takes four windows, which hide each other's waits.
+constexpr int WKEYS = 128;
+template <int TILES>
+__global__ __launch_bounds__(256, TILES == 2 ? 2 : 4) void window_kernel(FlashArgs a) {
+  __shared__ __attribute__((aligned(1024))) bf16_t sK[64 * TILES * 128];
+  __shared__ __attribute__((aligned(1024))) bf16_t sV[64 * TILES * 128];
+  __shared__ __attribute__((aligned(16))) int sCode[WKEYS];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int h = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hh = lane >> 5, j = lane & 31;
+  const int xaddr = half_swap_addr();
+  const int per_xcd = (int)(gridDim.x >> 3), logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (logical >= a.B) return;
+  const int samples = a.B / a.bias_mod;
+  const int bb = logical / samples, sample = logical % samples, b = sample * a.bias_mod + bb;
+  const int qi = min(j, a.Sq - 1);
+  const bool q_ok = j < a.Sq;
+
+  // the wave's share of the key rows, four to a load
+  const int* krows = a.key_rows + (int64_t)bb * a.Sk;
+  auto key_of = [&](int i) { return (i / (4 * TILES)) * (64 * TILES) + 16 * TILES * h + 4 * (i % (4 * TILES)) + (lane >> 4); };
+  int row[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) row[i] = krows[min(key_of(i), a.Sk - 1)];
+  if (tid < WKEYS) {
+    float pad = 1.f;
+    if (a.kpad) pad = a.kpad[(int64_t)bb * a.kp_sb + min(tid, a.Sk - 1)];
+    sCode[tid] = (tid >= a.Sk ? KEY_BEYOND : 0) | (pad == 0.f ? KEY_PAD : 0);
+  }
+  const bool q_is_pad = a.qpad ? (a.qpad[(int64_t)bb * a.qp_sb + qi] == 0.f) : false;
+  bf16x8 qf[2];
+  u32x4 gate[2];
+  const int64_t q_at = (int64_t)qi * a.q_ss + h * 32 + 8 * hh;
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    qf[ks] = as_frag(*reinterpret_cast<const u32x4*>(a.q + (int64_t)b * a.q_sb + q_at + 16 * ks));
+    gate[ks] = u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+    if (a.g) gate[ks] = *reinterpret_cast<const u32x4*>(a.g + (int64_t)b * a.g_sb + (int64_t)qi * a.g_ss + h * 32 + 8 * hh + 16 * ks);
+  }
+  const float* bias_row = a.bias + (int64_t)bb * a.bias_sb + (int64_t)h * a.bias_sh + (int64_t)qi * a.bias_sq;
+  const int64_t quad_step = a.bias_squad ? a.bias_squad : 4;
+  const u32x4 kt = table_buffer(a.k + (int64_t)sample * a.k_sb), vt = table_buffer(a.v + (int64_t)sample * a.v_sb);
+  auto lds_of = [&](const bf16_t* p) {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const bf16_t*)p + h * 16 * TILES * 256);
+  };
+  const uint32_t k_lds = lds_of(sK), v_lds = lds_of(sV);
+  const uint32_t swz = (uint32_t)((j & 3) << 2 | (j >> 2 & 3));
+  const char* kl = reinterpret_cast<const char*>(sK) + j * 256;
+  const int i16 = lane & 15;
+  const uint32_t v_chunk = 4 * h + 2 * (lane >> 4 & 1) + (i16 >> 1 & 1), v_swz = (uint32_t)((i16 >> 2) << 2 | hh);
+  const char* vl = reinterpret_cast<const char*>(sV) + (4 * hh + (i16 >> 2)) * 256 + 8 * (i16 & 1);
+  const uint32_t v_lo = (v_chunk ^ v_swz) << 4, v_hi = ((v_chunk ^ v_swz ^ 2) << 4) + 8 * 256;
+  const bf16x8 onesf = as_frag(u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+  f32x16 o;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) o[r] = 0.f;
+  float m_run = NEG_INF, l_run = 0.f;
+  bool any = false;
+#pragma unroll
+  for (int st = 0; st < 2 / TILES; ++st) {
+    const int first = 64 * TILES * st;
+    if (first >= a.Sk) break;
+    if (st > 0) lds_barrier();  // every wave is through with the previous tile
+    // s[u][4g + e]: the logit of key first + 32u + 8g + 4hh + e, accumulated on the bias
+    f32x16 s[2 * TILES];
+#pragma unroll
+    for (int u = 0; u < 2 * TILES; ++u)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(bias_row + (min(first + 32 * u + 8 * g + 4 * hh, a.Sk - 4) >> 2) * quad_step);
+        s[u][4 * g] = v.x; s[u][4 * g + 1] = v.y; s[u][4 * g + 2] = v.z; s[u][4 * g + 3] = v.w;
+      }
+#pragma unroll
+    for (int i = 0; i < 4 * TILES; ++i) {
+      const int r = row[4 * TILES * st + i];
+      const bool ok = r >= 0 && key_of(4 * TILES * st + i) < a.Sk;
+      const uint32_t chunk = (uint32_t)((lane & 15) ^ ((lane >> 4 & 3) << 2 | (i & 3))) * 16u;
+      const uint32_t ko = ok ? (uint32_t)r * (uint32_t)a.k_ss * 2u + chunk : 0x80000000u;
+      const uint32_t vo = ok ? (uint32_t)r * (uint32_t)a.v_ss * 2u + chunk : 0x80000000u;
+      asm volatile("s_add_u32 m0, %0, %6\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
+                   "s_add_u32 m0, %3, %6\n\ts_nop 0\n\tbuffer_load_dwordx4 %4, %5, 0 offen lds" ::"s"(k_lds), "v"(ko), "s"(kt),
+                   "s"(v_lds), "v"(vo), "s"(vt), "n"(i * 1024)
+                   : "m0", "scc", "memory");
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // key codes (a key of padding, a key past the end): most windows have none
+    if (st == 0) any = __any((sCode[lane] | sCode[64 + lane]) != 0);
+#pragma unroll
+    for (int u = 0; u < 2 * TILES; ++u)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        s[u] = mfma32(as_frag(*reinterpret_cast<const u32x4*>(kl + u * 32 * 256 + (((4 * h + 2 * ks + hh) ^ swz) << 4))), qf[ks], s[u]);
+    if (any) {
+#pragma unroll
+      for (int u = 0; u < 2 * TILES; ++u)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int* cp = &sCode[first + u * 32 + 8 * g + 4 * hh];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float v = s[u][4 * g + e];
+            if (q_is_pad && (cp[e] & KEY_PAD)) v += 1e9f;
+            if (cp[e] & KEY_BEYOND) v = NEG_INF;
+            s[u][4 * g + e] = v;
+          }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {  // tiles of 64 keys, as flash_kernel takes them
+      if (first + 64 * t >= a.Sk) break;
+      float m4[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x16& x = s[2 * t + (i >> 1)];
+        const int r = 8 * (i & 1);
+        m4[i] = fmaxf(fmaxf(fmaxf(x[r], x[r + 1]), fmaxf(x[r + 2], x[r + 3])), fmaxf(fmaxf(x[r + 4], x[r + 5]), fmaxf(x[r + 6], x[r + 7])));
+      }
+      float mx = fmaxf(fmaxf(m4[0], m4[1]), fmaxf(m4[2], m4[3]));
+      mx = fmaxf(mx, half_swap(xaddr, mx));
+      constexpr float BASE_SLACK = 8.f;
+      const float m_new = mx - m_run > BASE_SLACK ? mx : m_run;
+      const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * LOG2E);
+      m_run = m_new;
+      const float m2 = m_new * LOG2E;
+      bf16x8 pf[2][2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          float pv[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * t + u][8 * half + e], LOG2E, -m2));
+          pf[u][half] = as_frag(pack8(pv));
+        }
+      f32x16 lsum;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) lsum[r] = 0.f;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) lsum = mfma32(onesf, pf[u][half], lsum);
+      l_run = l_run * alpha + lsum[0];
+      if (__any(alpha != 1.f)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[r] *= alpha;
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          const char* vp = vl + (64 * t + u * 32 + 16 * half) * 256;
+          const v4s lo = lds_read_tr16(reinterpret_cast<const bf16_t*>(vp + v_lo)), hi = lds_read_tr16(reinterpret_cast<const bf16_t*>(vp + v_hi));
+          o = mfma32(as_frag(__builtin_bit_cast(u32x4, v8s{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w})), pf[u][half], o);
+        }
+    }
+  }
+  // o[4g + e] = out(query j, channel 8g + 4hh + e); gate[ks] holds channels 16 ks + 8 hh .. + 7: exchanging its middle
+  // quads with the other half of the wave makes them quads g = 2 ks and 2 ks + 1, and takes the result the other way
+  const float inv = 1.f / l_run;
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    uint32_t w[4] = {gate[ks].x, gate[ks].y, gate[ks].z, gate[ks].w};
+    swap_halves(w[0], w[2]);
+    swap_halves(w[1], w[3]);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = o[8 * ks + e] * inv;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      v[4 * g] *= bflo(w[2 * g]); v[4 * g + 1] *= bfhi(w[2 * g]); v[4 * g + 2] *= bflo(w[2 * g + 1]); v[4 * g + 3] *= bfhi(w[2 * g + 1]);
+    }
+    const int64_t at = (int64_t)b * a.o_sb + (int64_t)qi * a.o_ss + h * 32 + 16 * ks;
+    if (a.out_f32) {
+      float* out = reinterpret_cast<float*>(a.out) + at + 4 * hh;
+      if (q_ok) {
+        *reinterpret_cast<f32x4*>(out) = f32x4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f32x4*>(out + 8) = f32x4{v[4], v[5], v[6], v[7]};
+      }
+    } else {
+      uint32_t p[4] = {pack2bf(v[0], v[1]), pack2bf(v[2], v[3]), pack2bf(v[4], v[5]), pack2bf(v[6], v[7])};
+      swap_halves(p[0], p[2]);
+      swap_halves(p[1], p[3]);
+      if (q_ok) *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(a.out) + at + 8 * hh) = u32x4{p[0], p[1], p[2], p[3]};
+    }
+  }
+}
+
+// what window_kernel takes: its shapes, a bias in rows of whole quads, tables whose byte offsets fit 31 bits
+bool window_fits(const FlashArgs& a) {
+  return a.key_rows && a.bias && !a.key_mask && a.H == 4 && a.d == 32 && a.Sq <= 32 && a.Sk <= WKEYS && (a.Sk & 3) == 0 &&
+         ((a.bias_sq | a.bias_sb | a.bias_sh | a.bias_squad) & 3) == 0 && ((uintptr_t)a.bias & 15) == 0 && a.k_ss > 0 && a.v_ss > 0 &&
+         a.table_rows > 0 && a.table_rows * (a.k_ss > a.v_ss ? a.k_ss : a.v_ss) < (1ll << 30);
+}
+
 // Queries per workgroup: 128 (four waves share the K / V tiles), or 64 when
 // that would leave the 256 CUs with too few workgroups, or 32 for the short
 // query windows of the atom cross-attention.
@@ -506,6 +727,12 @@ int launch_flash_attention(const FlashArgs& a, hipStream_t stream) {
   if ((a.qpad == nullptr) != (a.kpad == nullptr)) return AF3_ERR_BAD_ARG;
   if (a.bias_mod < 0 || (a.bias_mod > 0 && a.B % a.bias_mod) || (a.key_rows && a.bias_mod <= 0)) return AF3_ERR_BAD_ARG;
   if (a.bias_squad && (a.bias_sq != 4 || (a.bias_squad & 3))) return AF3_ERR_BAD_ARG;
+  if (window_fits(a)) {
+    const dim3 grid((unsigned)((a.B + 7) / 8 * 8)), block(256);
+    if (a.B <= 512) hipLaunchKernelGGL(window_kernel<2>, grid, block, 0, stream, a);  // two on every CU hold them all
+    else hipLaunchKernelGGL(window_kernel<1>, grid, block, 0, stream, a);
+    return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+  }
   if (a.d == 48) return launch_nw<3, 2>(a, stream);
   if (a.d == 16) return launch_nw<1, 1>(a, stream);
   return launch_nw<2, 1>(a, stream);

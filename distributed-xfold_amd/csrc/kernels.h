@@ -82,6 +82,12 @@ int run_self_attention(const bf16_t* q_data, const float* key_mask, int64_t mask
                        int bias_quad_major, const bf16_t* w_qkvg, const float* query_b, int num_head, void* out, int out_dtype,
                        int64_t batch, int64_t seq, int channels, void* workspace, size_t workspace_bytes, int split_k,
                        hipStream_t stream);
+// af3_gathered_cross_attention_forward, with the pair logits in rows or (bias_quad_major) in quads of keys
+int run_gathered_attention(const bf16_t* q_data, const bf16_t* atom_data, const int32_t* key_rows, const float* pair_logits,
+                           int bias_quad_major, const float* mask_q, const float* mask_k, int64_t bias_batches, const bf16_t* w_qg,
+                           const bf16_t* w_kv, const float* query_b, int num_head, void* out, int out_dtype, int64_t batch,
+                           int64_t sq, int64_t sk, int64_t samples, int64_t n_atoms, int channels, void* workspace,
+                           size_t workspace_bytes, hipStream_t stream);
 // Which bias entries a launch reads.  Column c takes bias[c] when the epilogue is not segmented, or
 // when c lies in a segment whose op is SEG_BIAS_SCALE; the kernels read whole groups of entries
 // (gemm_nt_kernel up to 8 from a multiple of 8, the large tile 4 from a multiple of 4, the last
@@ -126,6 +132,11 @@ struct RowNormArgs {
   const float* scale = nullptr;   // [cond_rows][ld_cond] pre-sigmoid, or null
   const float* shift = nullptr;
   int64_t cond_rows = 0, ld_cond = 0;
+  // C <= 128: a second result of the same rows, y2 [rows][ldy] with scale2 / shift2 [cond_rows][ld_cond2]
+  const float *scale2 = nullptr, *shift2 = nullptr;
+  bf16_t* y2 = nullptr;
+  int64_t ld_cond2 = 0;
+  int samples = 1;  // set by launch_row_norm
   int param_vec = 0, cond_vec = 0;  // set by launch_row_norm: arrays aligned for 16-byte loads
 };
 int launch_row_norm(const RowNormArgs& a, hipStream_t stream);
@@ -150,8 +161,8 @@ int launch_softmax_rows(const float* x, const float* mask, bf16_t* y, int64_t ro
 // y[r][:] = (res ? res[r][:] : 0) + W relu?(x[r][:]), fp32, W [n_out][k], n_out 16 or 3, k % 4 == 0, k <= 128
 int launch_narrow_linear_f32(const float* x, const float* w, const float* res, float* y, int64_t rows, int k, int n_out,
                              int relu_in, hipStream_t stream);
-int launch_atom_pair_logits(const float* x, const float* ln_w, const float* w, float* out, int64_t n_groups, int64_t group,
-                            int n_blocks, int n_head, hipStream_t stream);
+int launch_atom_pair_logits(const float* x, const float* ln_w, const float* w, float* out, int64_t n_groups, int64_t queries,
+                            int64_t keys, int n_blocks, int n_head, int quad_major, hipStream_t stream);
 int launch_atom_pair_cond(const float* row, const float* col, const float* tp, const int* tq, const int* tk, int n_tok,
                           const float* q_pos, const float* k_pos, const int* q_uid, const int* k_uid, const float* w_off,
                           const float* w_dist, const float* w_valid, const float* w1, const float* w2, const float* w3,
@@ -281,6 +292,7 @@ struct FlashArgs {
   // of the K / V table of sample b / bias_mod (k_sb / v_sb: table stride); a
   // negative row is a key with zero K and V.  Null: key s is row s of batch b.
   const int* key_rows = nullptr;
+  int64_t table_rows = 0;  // rows of a sample's table: every entry of key_rows is below this
   int n_blocks = 0;  // workgroups that have work (set by the launcher; the grid is rounded up to a multiple of 8)
 };
 int launch_flash_attention(const FlashArgs& a, hipStream_t stream);

@@ -26,39 +26,58 @@ __device__ __forceinline__ void load8f(const float* p, bool vec, float* out) {
   }
 }
 
-// y = LN(x) [* weight] [+ bias], then [sigmoid(scale) * y + shift], 8 channels
-__device__ __forceinline__ void finish8(const RowNormArgs& a, const float* v, float mean, float rstd, int c,
-                                        int64_t crow, float* o) {
+// The parameters that eight channels of a row take: y = LN(x) [* weight] [+ bias], then [sigmoid(scale) * y + shift].
+struct Params8 {
   float w[8], b[8], sc[8], sh[8];
-  if (a.weight) load8f(a.weight + c, a.param_vec, w);
-  if (a.bias) load8f(a.bias + c, a.param_vec, b);
-  if (a.scale) {
-    load8f(a.scale + crow * a.ld_cond + c, a.cond_vec, sc);
-    load8f(a.shift + crow * a.ld_cond + c, a.cond_vec, sh);
+  __device__ __forceinline__ void load(const RowNormArgs& a, int c) {
+    if (a.weight) load8f(a.weight + c, a.param_vec, w);
+    if (a.bias) load8f(a.bias + c, a.param_vec, b);
   }
+  __device__ __forceinline__ void load_cond(const float* scale, const float* shift, int64_t at, int vec) {
+    load8f(scale + at, vec, sc);
+    load8f(shift + at, vec, sh);
+  }
+  __device__ __forceinline__ void finish(const RowNormArgs& a, const float* v, float mean, float rstd, float* o) const {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    float t = (v[e] - mean) * rstd;
-    if (a.weight) t *= w[e];
-    if (a.bias) t += b[e];
-    if (a.scale) t = sigmoidf_(sc[e]) * t + sh[e];
-    o[e] = t;
+    for (int e = 0; e < 8; ++e) {
+      float t = (v[e] - mean) * rstd;
+      if (a.weight) t *= w[e];
+      if (a.bias) t += b[e];
+      if (a.scale) t = sigmoidf_(sc[e]) * t + sh[e];
+      o[e] = t;
+    }
   }
+};
+__device__ __forceinline__ int64_t cond_row(const RowNormArgs& a, int64_t row) {  // (cond_rows and, with them, rows fit 31 bits)
+  return a.cond_rows > 0 ? (int64_t)((uint32_t)row % (uint32_t)a.cond_rows) : 0;
 }
 
-template <typename TIn>
+// A row is a chain of two memory round trips, the activations and (the conditioning of an adaptive norm is as large as
+// the row, twice over in fp32) the parameters, with two reductions between them: with the parameters asked for at the
+// start it is one (500 rows of 768: 4.3 us, was 4.9).  NCH chunks of 512 channels.
+template <typename TIn, int NCH>
 __global__ __launch_bounds__(256) void ln_rows_kernel(RowNormArgs a) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= a.rows) return;
   const TIn* x = reinterpret_cast<const TIn*>(a.x) + row * a.ldx;
-  float v[MAX_CHUNKS][8];
+  const int64_t crow = cond_row(a, row);
+  typename Elem<TIn>::Raw raw[NCH];
+  Params8 p[NCH];
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) raw[i] = Elem<TIn>::load_raw(x + min((i * 64 + lane) * 8, a.C - 8));
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int c = min((i * 64 + lane) * 8, a.C - 8);
+    p[i].load(a, c);
+    if (a.scale) p[i].load_cond(a.scale, a.shift, crow * a.ld_cond + c, a.cond_vec);
+  }
+  float v[NCH][8];
   float s = 0.f;
 #pragma unroll
-  for (int i = 0; i < MAX_CHUNKS; ++i) {
-    const int c = (i * 64 + lane) * 8;
-    if (c < a.C) {
-      Elem<TIn>::load8(x + c, v[i]);
+  for (int i = 0; i < NCH; ++i) {
+    Elem<TIn>::unpack_raw(raw[i], v[i]);
+    if ((i * 64 + lane) * 8 < a.C) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) s += v[i][e];
     }
@@ -66,22 +85,20 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(RowNormArgs a) {
   const float mean = wave_sum(s) / (float)a.C;
   float q = 0.f;
 #pragma unroll
-  for (int i = 0; i < MAX_CHUNKS; ++i) {
-    const int c = (i * 64 + lane) * 8;
-    if (c < a.C) {
+  for (int i = 0; i < NCH; ++i) {
+    if ((i * 64 + lane) * 8 < a.C) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) { const float d = v[i][e] - mean; q += d * d; }
     }
   }
   const float rstd = rsqrtf(wave_sum(q) / (float)a.C + LN_EPS);
-  const int64_t crow = a.cond_rows > 0 ? row % a.cond_rows : 0;
   bf16_t* y = a.y + row * a.ldy;
 #pragma unroll
-  for (int i = 0; i < MAX_CHUNKS; ++i) {
+  for (int i = 0; i < NCH; ++i) {
     const int c = (i * 64 + lane) * 8;
     if (c < a.C) {
       float o[8];
-      finish8(a, v[i], mean, rstd, c, crow, o);
+      p[i].finish(a, v[i], mean, rstd, o);
       *reinterpret_cast<u32x4*>(y + c) = pack8(o);
     }
   }
@@ -90,41 +107,62 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(RowNormArgs a) {
 // Narrow rows (C <= 128, e.g. the 16-channel atom pair conditioning with its
 // millions of rows): G lanes per row, 64 / G rows per wave, so a wave still
 // moves a full kilobyte per instruction instead of one lane group's worth.
+// A second pair of scale and shift (the atoms as keys beside the atoms as queries) shares the row and its statistics.
+// samples > 1: a lane group takes a conditioning row's activation rows of all samples (row, row + cond_rows, ..) one
+// after the other: the conditioning is larger than the activations (fp32 scale and shift against bf16) and is fetched
+// once instead of once per sample.
 template <typename TIn, int G>
 __global__ __launch_bounds__(256) void ln_rows_small_kernel(RowNormArgs a) {
   constexpr int RPW = 64 / G;
   const int lane = threadIdx.x & 63, sub = lane % G;
-  const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + lane / G;
-  const bool ok = row < a.rows && sub * 8 < a.C;
-  const int64_t rr = row < a.rows ? row : a.rows - 1;
+  const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + lane / G;
+  const int64_t end = a.samples > 1 ? a.cond_rows : a.rows;
+  const bool ok = first < end && sub * 8 < a.C;
+  const int64_t at = first < end ? first : end - 1;
   const int c = sub * 8 < a.C ? sub * 8 : 0;
-  float v[8];
-  Elem<TIn>::load8(reinterpret_cast<const TIn*>(a.x) + rr * a.ldx + c, v);
-  float s = 0.f;
+  const int64_t crow = a.samples > 1 ? at : cond_row(a, at);
+  const TIn* x = reinterpret_cast<const TIn*>(a.x) + at * a.ldx + c;
+  typename Elem<TIn>::Raw raw = Elem<TIn>::load_raw(x);
+  Params8 p, p2;
+  p.load(a, c);
+  if (a.scale) p.load_cond(a.scale, a.shift, crow * a.ld_cond + c, a.cond_vec);
+  if (a.scale2) p2.load_cond(a.scale2, a.shift2, crow * a.ld_cond2 + c, a.cond_vec);
+  for (int k = 0; k < a.samples; ++k) {
+    float v[8];
+    Elem<TIn>::unpack_raw(raw, v);
+    const int64_t row = at + k * a.cond_rows;
+    if (k + 1 < a.samples) raw = Elem<TIn>::load_raw(x + (k + 1) * a.cond_rows * a.ldx);
+    float s = 0.f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) { v[e] = ok ? v[e] : 0.f; s += v[e]; }
+    for (int e = 0; e < 8; ++e) { v[e] = ok ? v[e] : 0.f; s += v[e]; }
 #pragma unroll
-  for (int m = 1; m < G; m <<= 1) s += __shfl_xor(s, m);
-  const float mean = s / (float)a.C;
-  float q = 0.f;
+    for (int m = 1; m < G; m <<= 1) s += __shfl_xor(s, m);
+    const float mean = s / (float)a.C;
+    float q = 0.f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) { const float d = ok ? v[e] - mean : 0.f; q += d * d; }
+    for (int e = 0; e < 8; ++e) { const float d = ok ? v[e] - mean : 0.f; q += d * d; }
 #pragma unroll
-  for (int m = 1; m < G; m <<= 1) q += __shfl_xor(q, m);
-  const float rstd = rsqrtf(q / (float)a.C + LN_EPS);
-  if (!ok) return;
-  const int64_t crow = a.cond_rows > 0 ? row % a.cond_rows : 0;
-  float o[8];
-  finish8(a, v, mean, rstd, c, crow, o);
-  *reinterpret_cast<u32x4*>(a.y + row * a.ldy + c) = pack8(o);
+    for (int m = 1; m < G; m <<= 1) q += __shfl_xor(q, m);
+    const float rstd = rsqrtf(q / (float)a.C + LN_EPS);
+    if (!ok) continue;
+    float o[8];
+    p.finish(a, v, mean, rstd, o);
+    *reinterpret_cast<u32x4*>(a.y + row * a.ldy + c) = pack8(o);
+    if (a.scale2) {
+      p2.finish(a, v, mean, rstd, o);
+      *reinterpret_cast<u32x4*>(a.y2 + row * a.ldy + c) = pack8(o);
+    }
+  }
 }
 
 template <typename TIn>
-int launch_small(const RowNormArgs& a, hipStream_t stream) {
+int launch_small(RowNormArgs a, hipStream_t stream) {
   const int chunks = a.C / 8;
   const int g = chunks <= 1 ? 1 : chunks <= 2 ? 2 : chunks <= 4 ? 4 : chunks <= 8 ? 8 : 16;
   const int64_t rows_per_block = 4 * (64 / g);
-  const int64_t blocks = (a.rows + rows_per_block - 1) / rows_per_block;
+  // samples in turn where the conditioning rows alone are eight waves per CU or more (512 blocks)
+  a.samples = a.scale && a.rows % a.cond_rows == 0 && a.cond_rows >= 512 * rows_per_block ? (int)(a.rows / a.cond_rows) : 1;
+  const int64_t blocks = ((a.samples > 1 ? a.cond_rows : a.rows) + rows_per_block - 1) / rows_per_block;
   if (blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
   const dim3 grid((unsigned)blocks), block(256);
   switch (g) {
@@ -137,22 +175,34 @@ int launch_small(const RowNormArgs& a, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
 
+template <typename TIn>
+int launch_wide(const RowNormArgs& a, hipStream_t stream) {
+  const int64_t blocks = (a.rows + 3) / 4;
+  if (blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
+  const dim3 grid((unsigned)blocks), block(256);
+  switch ((a.C + 511) / 512) {
+    case 1: hipLaunchKernelGGL((ln_rows_kernel<TIn, 1>), grid, block, 0, stream, a); break;
+    case 2: hipLaunchKernelGGL((ln_rows_kernel<TIn, 2>), grid, block, 0, stream, a); break;
+    case 3: hipLaunchKernelGGL((ln_rows_kernel<TIn, 3>), grid, block, 0, stream, a); break;
+    default: hipLaunchKernelGGL((ln_rows_kernel<TIn, 4>), grid, block, 0, stream, a); break;
+  }
+  return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+}
+
 }  // namespace
 
 int launch_row_norm(const RowNormArgs& a_in, hipStream_t stream) {
   RowNormArgs a = a_in;
   auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   a.param_vec = al16(a.weight) && al16(a.bias);
-  a.cond_vec = al16(a.scale) && al16(a.shift) && (a.ld_cond & 3) == 0;
+  a.cond_vec = al16(a.scale) && al16(a.shift) && (a.ld_cond & 3) == 0 && al16(a.scale2) && al16(a.shift2) && (a.ld_cond2 & 3) == 0;
   if (a.rows <= 0 || a.C <= 0 || (a.C & 7) || a.C > 64 * 8 * MAX_CHUNKS) return AF3_ERR_BAD_ARG;
   if ((a.ldx & 7) || (a.ldy & 7) || ((uintptr_t)a.x & 15) || ((uintptr_t)a.y & 15)) return AF3_ERR_BAD_ARG;
   if ((a.scale == nullptr) != (a.shift == nullptr)) return AF3_ERR_BAD_ARG;
-  if (a.scale && a.cond_rows <= 0) return AF3_ERR_BAD_ARG;
+  if (a.scale && (a.cond_rows <= 0 || a.rows > 0x7fffffff || a.cond_rows > 0x7fffffff)) return AF3_ERR_BAD_ARG;
+  if (a.scale2 && (!a.scale || !a.shift2 || !a.y2 || a.C > 128 || ((uintptr_t)a.y2 & 15))) return AF3_ERR_BAD_ARG;
   if (a.C <= 128) return a.x_f32 ? launch_small<float>(a, stream) : launch_small<bf16_t>(a, stream);
-  const unsigned blocks = (unsigned)((a.rows + 3) / 4);
-  if (a.x_f32) hipLaunchKernelGGL(ln_rows_kernel<float>, dim3(blocks), dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL(ln_rows_kernel<bf16_t>, dim3(blocks), dim3(256), 0, stream, a);
-  return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+  return a.x_f32 ? launch_wide<float>(a, stream) : launch_wide<bf16_t>(a, stream);
 }
 
 // ------------------------------------------------------------------ transpose
@@ -391,18 +441,24 @@ __global__ __launch_bounds__(256) void narrow_linear_f32_kernel(const float* __r
 // bias) and a 16 -> n_out projection, n_out = blocks x heads, each output written to its own
 // [block][subset][head][query][key] plane: the layout the attention kernel reads its bias in.  Rows are
 // (subset, query, key) in this order, `group` = queries x keys rows per subset.  One thread per row, fp32.
+// quad_queries != 0 (the queries): quads of four keys are the outer index of a plane, [key / 4][query][key % 4].
 // ----------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void atom_pair_logits_kernel(const float* __restrict__ x, const float* __restrict__ ln_w,
                                                                const float* __restrict__ w, float* __restrict__ out,
                                                                int64_t rows, int64_t group, int64_t n_groups, int n_blocks,
-                                                               int n_head) {
+                                                               int n_head, int quad_queries, int keys) {
   __shared__ __attribute__((aligned(16))) float sW[32 * 16];
   const int n_out = n_blocks * n_head;
   // the LayerNorm weight goes into the projection: (xhat * g) . w = xhat . (g * w)
   for (int i = threadIdx.x; i < n_out * 16; i += 256) sW[i] = w[i] * ln_w[i & 15];
   __syncthreads();
-  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (r >= rows) return;
+  const int64_t s = r / group, at = r - s * group;  // place in the subset's plane
+  if (quad_queries) {  // [key / 4][query][key % 4]: the row that belongs there
+    const int cell = (int)at >> 2, quad = cell / quad_queries;
+    r = s * group + (int64_t)(cell - quad * quad_queries) * keys + 4 * quad + ((int)at & 3);
+  }
   float v[16];
 #pragma unroll
   for (int c = 0; c < 16; c += 4) {
@@ -417,7 +473,6 @@ __global__ __launch_bounds__(256) void atom_pair_logits_kernel(const float* __re
 #pragma unroll
   for (int c = 0; c < 16; ++c) { v[c] -= mean; var = fmaf(v[c], v[c], var); }
   const float rstd = rsqrtf(var * (1.f / 16) + LN_EPS);
-  const int64_t s = r / group, qk = r - s * group;
   for (int o = 0; o < n_out; ++o) {
     float acc = 0.f;
 #pragma unroll
@@ -426,7 +481,7 @@ __global__ __launch_bounds__(256) void atom_pair_logits_kernel(const float* __re
       acc = fmaf(v[c], ww.x, fmaf(v[c + 1], ww.y, fmaf(v[c + 2], ww.z, fmaf(v[c + 3], ww.w, acc))));
     }
     const int blk = o / n_head, h = o - blk * n_head;
-    out[(((int64_t)blk * n_groups + s) * n_head + h) * group + qk] = acc * rstd;
+    out[(((int64_t)blk * n_groups + s) * n_head + h) * group + at] = acc * rstd;
   }
 }
 
@@ -612,15 +667,17 @@ int launch_narrow_linear_f32(const float* x, const float* w, const float* res, f
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
 
-int launch_atom_pair_logits(const float* x, const float* ln_w, const float* w, float* out, int64_t n_groups, int64_t group,
-                            int n_blocks, int n_head, hipStream_t stream) {
+int launch_atom_pair_logits(const float* x, const float* ln_w, const float* w, float* out, int64_t n_groups, int64_t queries,
+                            int64_t keys, int n_blocks, int n_head, int quad_major, hipStream_t stream) {
+  const int64_t group = queries * keys;
+  if (quad_major && ((keys & 3) || group > 0x7fffffff)) return AF3_ERR_BAD_ARG;
   if (!x || !ln_w || !w || !out || n_groups <= 0 || group <= 0 || n_blocks <= 0 || n_head <= 0) return AF3_ERR_BAD_ARG;
   if (n_blocks * n_head > 32) return AF3_ERR_UNSUPPORTED;
   if ((uintptr_t)x & 15) return AF3_ERR_BAD_ARG;
   const int64_t rows = n_groups * group, blocks = (rows + 255) / 256;
   if (blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
   hipLaunchKernelGGL(atom_pair_logits_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, ln_w, w, out, rows, group,
-                     n_groups, n_blocks, n_head);
+                     n_groups, n_blocks, n_head, quad_major ? (int)queries : 0, (int)keys);
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
 

@@ -319,7 +319,7 @@ size_t af3_atom_transformer_workspace_bytes(int64_t samples, int64_t subsets, in
 int af3_atom_transformer_forward(
     const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t samples, int64_t subsets,
     int64_t queries, int64_t keys, int channels, int hidden, int num_head, const int32_t* key_rows, const float* mask_q,
-    const float* mask_k, const float* pair_logits, const float* scale_shift_q, const float* scale_shift_k, const float* gate,
+    const float* mask_k, const float* pair_logits, int bias_quad_major, const float* scale_shift_q, const float* scale_shift_k, const float* gate,
     void* workspace, size_t workspace_bytes, af3_stream_t stream) {
   if (!blocks || num_blocks <= 0 || !act || !key_rows || !scale_shift_q || !scale_shift_k || !gate || samples <= 0 ||
       subsets <= 0 || queries <= 0 || keys <= 0 || channels <= 0 || hidden <= 0 || num_head <= 0)
@@ -339,10 +339,19 @@ int af3_atom_transformer_forward(
     const float *ss = scale_shift_q + (int64_t)2 * i * 2 * c, *sk = scale_shift_k + (int64_t)i * 2 * c;
     const float* g = gate + (int64_t)2 * i * atoms * c;
     const float* pl = pair_logits ? pair_logits + (int64_t)i * subsets * num_head * queries * keys : nullptr;
-    STEP(af3_layer_norm_forward(act, act_dtype, xq, rows, c, nullptr, nullptr, ss, ss + c, atoms, ld_q, stream));
-    STEP(af3_layer_norm_forward(act, act_dtype, xk, rows, c, nullptr, nullptr, sk, sk + c, atoms, ld_k, stream));
-    STEP(af3_gathered_cross_attention_forward(xq, xk, key_rows, pl, mask_q, mask_k, subsets, b.w_q, b.w_kv, b.q_b, num_head, y,
-                                              AF3_BF16, samples * subsets, queries, keys, samples, atoms, c, aw, ab, stream));
+    if (c <= 128) {
+      RowNormArgs ln;
+      ln.x = act; ln.x_f32 = act_dtype == AF3_F32; ln.rows = rows; ln.ldx = ln.ldy = ln.C = c;
+      ln.y = xq; ln.scale = ss; ln.shift = ss + c; ln.cond_rows = atoms; ln.ld_cond = ld_q;
+      ln.y2 = xk; ln.scale2 = sk; ln.shift2 = sk + c; ln.ld_cond2 = ld_k;
+      STEP(launch_row_norm(ln, static_cast<hipStream_t>(stream)));
+    } else {
+      STEP(af3_layer_norm_forward(act, act_dtype, xq, rows, c, nullptr, nullptr, ss, ss + c, atoms, ld_q, stream));
+      STEP(af3_layer_norm_forward(act, act_dtype, xk, rows, c, nullptr, nullptr, sk, sk + c, atoms, ld_k, stream));
+    }
+    STEP(run_gathered_attention(xq, xk, key_rows, pl, bias_quad_major, mask_q, mask_k, subsets, b.w_q, b.w_kv, b.q_b, num_head, y,
+                                AF3_BF16, samples * subsets, queries, keys, samples, atoms, c, aw, ab,
+                                static_cast<hipStream_t>(stream)));
     STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, atoms, 0, act, act_dtype,
                             stream));
     STEP(af3_layer_norm_forward(act, act_dtype, xq, rows, c, nullptr, nullptr, ss + 2 * c, ss + 3 * c, atoms, ld_q, stream));

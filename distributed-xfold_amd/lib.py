@@ -89,6 +89,7 @@ SIGNATURES = {
     "af3_atom_pair_cond_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                         _i64, _i64, _i64, _vp]),
     "af3_atom_pair_logits_forward": (_i, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _i, _vp]),
+    "af3_atom_pair_logits_quads_forward": (_i, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _i, _vp]),
     "af3_pair_cond_init_forward": (_i, [_vp, _i, _f, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "af3_pairformer_stack_workspace_bytes": (_sz, [_i64, _i]),
     "af3_pairformer_single_workspace_bytes": (_sz, [_i64, _i, _i]),
@@ -99,7 +100,7 @@ SIGNATURES = {
         _i, [_vp, _i, _vp, _i, _i64, _i64, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _i64, _vp, _sz, _vp]),
     "af3_atom_transformer_workspace_bytes": (_sz, [_i64, _i64, _i64, _i, _i]),
     "af3_atom_transformer_forward": (
-        _i, [_vp, _i, _vp, _i, _i64, _i64, _i64, _i64, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+        _i, [_vp, _i, _vp, _i, _i64, _i64, _i64, _i64, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _sz, _vp]),
     "af3_linear_bias_span": (_i, [_i64, _i, _i, _i, _i, _vp, _vp]),
     "af3_grid_attention_core_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "af3_check_gemm_f32": (

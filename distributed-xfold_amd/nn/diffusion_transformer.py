@@ -461,7 +461,8 @@ class DiffusionCrossAttTransformer(HipModule):
         if pair_cond.dtype == torch.float32 and pair_cond.dim() == 4 and pair_cond.shape[-1] == 16 \
                 and self.num_blocks * self.num_head <= 32:
             # LayerNorm, projection and the split into [block][S][head][Q][K] planes in one fp32 pass
-            logits = ops.atom_pair_logits(pair_cond.contiguous(), p["ln_w"], p["w_f32"], self.num_blocks, self.num_head)
+            logits = ops.atom_pair_logits(pair_cond.contiguous(), p["ln_w"], p["w_f32"], self.num_blocks, self.num_head,
+                                          quad_major=key_rows is not None and pair_cond.shape[2] % 4 == 0)
         else:
             pair_act = ops.layer_norm(pair_cond.contiguous(), p["ln_w"])
             logits = ops.linear(pair_act, p["w"], out_dtype=torch.float32)           # [S, Q, K, (b h)]

@@ -330,7 +330,7 @@ def diffusion_transformer(blocks, act, mask, pair_logits, scale_shift, gate, num
 def atom_transformer(blocks, act, key_rows, mask_q, mask_k, pair_logits, scale_shift_q, scale_shift_k, gate, num_head,
                      hidden):
     """The blocks of the windowed atom transformer in one call (af3_atom_transformer_forward), act
-    [(B,) S, Q, C] updated in place.  key_rows [S, K] int32; pair_logits [blocks, S, H, Q, K]; scale_shift_q
+    [(B,) S, Q, C] updated in place.  key_rows [S, K] int32; pair_logits [blocks, S, H, Q, K] or [blocks, S, H, K / 4, Q, 4]; scale_shift_q
     [S Q, 2 blocks, 2 C], scale_shift_k [S Q, blocks, 2 C], gate [2 blocks, S Q, C] fp32."""
     lib = _L.load()
     _gpu(act, "act")
@@ -342,14 +342,15 @@ def atom_transformer(blocks, act, key_rows, mask_q, mask_k, pair_logits, scale_s
         if int(key_rows.max()) >= s * q:
             raise ValueError("key_rows: row index beyond the atoms")
         key_rows._af3_checked_rows = s * q
-    _gpu(pair_logits, "pair_logits", torch.float32, (nb, s, num_head, q, k))
+    quads = pair_logits.dim() == 6
+    _gpu(pair_logits, "pair_logits", torch.float32, (nb, s, num_head) + ((k // 4, q, 4) if quads else (q, k)))
     _gpu(scale_shift_q, "scale_shift_q", torch.float32, (s * q, 2 * nb, 2 * c))
     _gpu(scale_shift_k, "scale_shift_k", torch.float32, (s * q, nb, 2 * c))
     _gpu(gate, "gate", torch.float32, (2 * nb, s * q, c))
     mq, mk = _mask_f32(mask_q.reshape(s, q), (s, q), "mask_q"), _mask_f32(mask_k.reshape(s, k), (s, k), "mask_k")
     ws = _ws(lib.af3_atom_transformer_workspace_bytes(b, s, q, c, hidden), act.device)
     rc = lib.af3_atom_transformer_forward(
-        blocks, nb, _p(act), _dt(act), b, s, q, k, c, hidden, num_head, _p(key_rows), _p(mq), _p(mk), _p(pair_logits),
+        blocks, nb, _p(act), _dt(act), b, s, q, k, c, hidden, num_head, _p(key_rows), _p(mq), _p(mk), _p(pair_logits), int(quads),
         _p(scale_shift_q), _p(scale_shift_k), _p(gate), _p(ws), ws.numel(), _stream(act.device))
     _L.check(rc, "af3_atom_transformer_forward")
     return act
@@ -687,9 +688,10 @@ def atom_pair_cond(row, col, token_pair, query_token, key_token, query_pos, key_
     return out
 
 
-def atom_pair_logits(pair_cond, ln_w, w, num_blocks: int, num_head: int):
+def atom_pair_logits(pair_cond, ln_w, w, num_blocks: int, num_head: int, quad_major: bool = False):
     """LayerNorm (weight, no bias) and 16 -> blocks x heads projection of the atom pair conditioning, written as
-    the [blocks, S, heads, Q, K] fp32 bias planes of the windowed attention (af3_atom_pair_logits_forward).
+    the [blocks, S, heads, Q, K] fp32 bias planes of the windowed attention (af3_atom_pair_logits_forward), or with
+    `quad_major` (K a multiple of 4) as [blocks, S, heads, K / 4, Q, 4], which atom_transformer reads faster.
     pair_cond [S, Q, K, 16] fp32; ln_w [16] fp32; w [blocks * heads, 16] fp32."""
     lib = _L.load()
     _gpu(pair_cond, "pair_cond", torch.float32)
@@ -698,9 +700,10 @@ def atom_pair_logits(pair_cond, ln_w, w, num_blocks: int, num_head: int):
     s, q, k, _ = pair_cond.shape
     _gpu(ln_w, "ln_w", torch.float32, (16,))
     _gpu(w, "w", torch.float32, (num_blocks * num_head, 16))
-    out = torch.empty((num_blocks, s, num_head, q, k), dtype=torch.float32, device=pair_cond.device)
-    rc = lib.af3_atom_pair_logits_forward(_p(pair_cond), _p(ln_w), _p(w), _p(out), s, q, k, int(num_blocks), int(num_head),
-                                          _stream(pair_cond.device))
+    planes = (k // 4, q, 4) if quad_major else (q, k)
+    out = torch.empty((num_blocks, s, num_head) + planes, dtype=torch.float32, device=pair_cond.device)
+    call = lib.af3_atom_pair_logits_quads_forward if quad_major else lib.af3_atom_pair_logits_forward
+    rc = call(_p(pair_cond), _p(ln_w), _p(w), _p(out), s, q, k, int(num_blocks), int(num_head), _stream(pair_cond.device))
     _L.check(rc, "af3_atom_pair_logits_forward")
     return out
 

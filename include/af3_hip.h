@@ -457,6 +457,10 @@ int af3_atom_pair_cond_forward(const float* row, const float* col, const float* 
  */
 int af3_atom_pair_logits_forward(const float* pair_cond, const float* ln_w, const float* w, float* out, int64_t subsets,
                                  int64_t queries, int64_t keys, int num_blocks, int num_head, af3_stream_t stream);
+/* ... with quads of four keys as the outer index of a plane, [num_blocks,subsets,num_head,keys/4,queries,4] */
+int af3_atom_pair_logits_quads_forward(const float* pair_cond, const float* ln_w, const float* w, float* out,
+                                       int64_t subsets, int64_t queries, int64_t keys, int num_blocks, int num_head,
+                                       af3_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * Pair conditioning of the diffusion head, first layer
@@ -596,8 +600,8 @@ int af3_evoformer_stack_forward(
  * af3_atom_transformer_forward: act [samples,subsets,queries,c]; key k of subset s is
  *   atom key_rows[s,k] of the sample's subsets * queries (negative: empty slot, K = V
  *   = 0), see af3_gathered_cross_attention_forward; scale_shift_k [subsets * queries]
- *   [num_blocks][2 c] per atom, pair_logits [num_blocks,subsets,num_head,queries,keys],
- *   gate here [2 num_blocks][subsets * queries][c].
+ *   [num_blocks][2 c] per atom, pair_logits [num_blocks,subsets,num_head,queries,keys] or,
+ *   with bias_quad_major, [num_blocks,subsets,num_head,keys/4,queries,4], gate here [2 num_blocks][subsets * queries][c].
  */
 typedef struct af3_diffusion_block {
   const uint16_t* w_q;  /* diffusion: [4 c][c] q, k, v, gate;  atom: [2 c][c] q, gate */
@@ -617,7 +621,7 @@ size_t af3_atom_transformer_workspace_bytes(int64_t samples, int64_t subsets, in
 int af3_atom_transformer_forward(
     const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t samples, int64_t subsets,
     int64_t queries, int64_t keys, int channels, int hidden, int num_head, const int32_t* key_rows, const float* mask_q,
-    const float* mask_k, const float* pair_logits, const float* scale_shift_q, const float* scale_shift_k,
+    const float* mask_k, const float* pair_logits, int bias_quad_major, const float* scale_shift_q, const float* scale_shift_k,
     const float* gate, void* workspace, size_t workspace_bytes, af3_stream_t stream);
 
 /* ---------------------------------------------------------------------------
