@@ -36,23 +36,53 @@ struct Position {
   }
 };
 
-// LayerNorm of a position (its two lanes together) -> the four k-step fragments.  sLn: weight [64], bias [64].
+// Sum over a position's eight chunks (a lane's four and those of the other half of the wave), as a tree over the chunks
+// in their order.
+__device__ __forceinline__ float chunk_sum(const float* c, int xaddr) {
+  float t[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) t[ks] = c[ks] + half_swap(xaddr, c[ks]);
+  return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
+// a * b + c, rounded twice: as the row norms of rowops.hip compute weight and bias
+__device__ __forceinline__ float mul_add(float a, float b, float c) {
+#pragma clang fp contract(off)
+  const float t = a * b;
+  return t + c;
+}
+
+// LayerNorm of a position -> the four k-step fragments.  sLn: weight [64], bias [64].  ONE_PASS: sum and sum of squares
+// together, as the pair's tile kernels take a bf16 stream.
+template <bool ONE_PASS>
 __device__ __forceinline__ void layer_norm_frags(const float* v, const float* sLn, int hh, int xaddr, bf16x8* f) {
-  float s = 0.f;
+  float cs[4], cq[4];
 #pragma unroll
-  for (int i = 0; i < 32; ++i) s += v[i];
-  const float mean = (s + half_swap(xaddr, s)) * (1.f / MC);
-  float q = 0.f;
+  for (int ks = 0; ks < 4; ++ks) {
+    cs[ks] = cq[ks] = 0.f;
 #pragma unroll
-  for (int i = 0; i < 32; ++i) { const float d = v[i] - mean; q += d * d; }
-  const float rstd = rsqrtf((q + half_swap(xaddr, q)) * (1.f / MC) + LN_EPS);
+    for (int e = 0; e < 8; ++e) {
+      cs[ks] += v[8 * ks + e];
+      if (ONE_PASS) cq[ks] = fmaf(v[8 * ks + e], v[8 * ks + e], cq[ks]);
+    }
+  }
+  const float mean = chunk_sum(cs, xaddr) * (1.f / MC);
+  if (!ONE_PASS) {
+#pragma unroll
+    for (int i = 0; i < 32; ++i) { const float d = v[i] - mean; cq[i >> 3] += d * d; }
+  }
+  const float q = chunk_sum(cq, xaddr);
+  const float rstd = rsqrtf(ONE_PASS ? fmaxf(fmaf(q, 1.f / MC, -mean * mean), 0.f) + LN_EPS : q * (1.f / MC) + LN_EPS);
+  const float shift = -mean * rstd;
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
     float w[8], b[8], o[8];
     Elem<float>::load8(sLn + 16 * ks + 8 * hh, w);
     Elem<float>::load8(sLn + MC + 16 * ks + 8 * hh, b);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = (v[8 * ks + e] - mean) * rstd * w[e] + b[e];
+    for (int e = 0; e < 8; ++e)
+      o[e] = ONE_PASS ? fmaf(fmaf(v[8 * ks + e], rstd, shift), w[e], b[e])
+                      : mul_add((v[8 * ks + e] - mean) * rstd, w[e], b[e]);
     f[ks] = as_frag(pack8(o));
   }
 }
@@ -114,7 +144,7 @@ __global__ __launch_bounds__(256) void msa_project_kernel(MsaProjectArgs a) {
       float v[32];
       bf16x8 xf[4];
       pos[sub].unpack(v);
-      layer_norm_frags(v, sLn + z, hh, xaddr, xf);
+      layer_norm_frags<false>(v, sLn + z, hh, xaddr, xf);
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         f32x16 acc = zero16();
@@ -213,7 +243,7 @@ __global__ __launch_bounds__(512, 2) void msa_update_kernel(MsaUpdateArgs a) {
     bf16x8 xf[4];
     pos.unpack(v);
     if constexpr (ATT) {
-      layer_norm_frags(v, sLn + z, hh, xaddr, xf);
+      layer_norm_frags<false>(v, sLn + z, hh, xaddr, xf);
       bf16x8 gated[4];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -231,7 +261,7 @@ __global__ __launch_bounds__(512, 2) void msa_update_kernel(MsaUpdateArgs a) {
       add(v, y);
     }
     if constexpr (TRANS) {
-      layer_norm_frags(v, sLn + 2 * MC + z, hh, xaddr, xf);
+      layer_norm_frags<sizeof(TIO) == 2>(v, sLn + 2 * MC + z, hh, xaddr, xf);
       f32x16 y[2] = {zero16(), zero16()};
       f32x16 ga = product64(sW1, 0, xf), gb = product64(sW1, a.hidden, xf);
       for (int h = 0; h < a.hidden; h += 32) {
