@@ -348,7 +348,7 @@ static int self_attention_run(
   f.out = out; f.out_f32 = out_dtype == AF3_F32; f.o_ss = channels; f.o_sb = seq * channels;
   f.B = (int)batch; f.H = num_head; f.Sq = f.Sk = (int)seq; f.d = d;
   f.bias = nonbatched_bias; f.bias_sb = 0; f.bias_sh = seq * seq; f.bias_sq = seq;
-  if (bias_quad_major) { f.bias_sq = 4; f.bias_squad = seq * 4; }
+  if (bias_quad_major) { f.bias_sq = 4; f.bias_squad = seq * 4; f.bias_sh = (seq + 3) / 4 * 4 * seq; }
   f.key_mask = key_mask; f.km_sb = mask_batches == batch && batch > 1 ? seq : 0;
   return launch_flash_attention(f, s);
 }
@@ -358,6 +358,7 @@ int af3_batch_diffusion_self_attention_forward(
     int bias_quad_major, const uint16_t* w_qkvg, const float* query_b, int num_head,
     void* out, int out_dtype, int64_t batch, int64_t seq, int channels,
     void* workspace, size_t workspace_bytes, af3_stream_t stream) {
+  if (bias_quad_major != 0 && (bias_quad_major != 1 || (seq & 3))) return AF3_ERR_BAD_ARG;
   return run_self_attention(q_data, key_mask, mask_batches, nonbatched_bias, bias_quad_major, w_qkvg, query_b, num_head, out,
                             out_dtype, batch, seq, channels, workspace, workspace_bytes, 0, static_cast<hipStream_t>(stream));
 }
@@ -558,16 +559,28 @@ int af3_gathered_cross_attention_forward(
 }
 
 // ------------------------------------------------------------------ pair logits
-int af3_pair_logits_forward(
+static int pair_logits(
     const void* pair, int io_dtype, const float* norm_weight, const float* norm_bias,
-    const uint16_t* w, int n_out, float* out, int64_t n, af3_stream_t stream) {
+    const uint16_t* w, int n_out, float* out, int64_t n, int quads, af3_stream_t stream) {
   if (!pair || !w || !out || !norm_weight) return AF3_ERR_BAD_ARG;
   if (bad_dtype(io_dtype) || n <= 0 || n > 8192 || n_out <= 0) return AF3_ERR_BAD_ARG;
   AttnProjArgs p;
   p.pair = pair; p.io_f32 = io_dtype == AF3_F32; p.N = (int)n;
   p.ln_w = norm_weight; p.ln_b = norm_bias;
-  p.w_bias = w; p.n_bias = n_out; p.out_bias = out;
+  p.w_bias = w; p.n_bias = n_out; p.out_bias = out; p.quads = quads;
   return launch_attn_proj(p, static_cast<hipStream_t>(stream));
+}
+
+int af3_pair_logits_forward(
+    const void* pair, int io_dtype, const float* norm_weight, const float* norm_bias,
+    const uint16_t* w, int n_out, float* out, int64_t n, af3_stream_t stream) {
+  return pair_logits(pair, io_dtype, norm_weight, norm_bias, w, n_out, out, n, 0, stream);
+}
+
+int af3_pair_logits_quads_forward(
+    const void* pair, int io_dtype, const float* norm_weight, const float* norm_bias,
+    const uint16_t* w, int n_out, float* out, int64_t n, af3_stream_t stream) {
+  return pair_logits(pair, io_dtype, norm_weight, norm_bias, w, n_out, out, n, 1, stream);
 }
 
 // ------------------------------------------------------------------- row norm
@@ -682,8 +695,8 @@ int run_self_attention(const bf16_t* q_data, const float* key_mask, int64_t mask
                        int bias_quad_major, const bf16_t* w_qkvg, const float* query_b, int num_head, void* out, int out_dtype,
                        int64_t batch, int64_t seq, int channels, void* workspace, size_t workspace_bytes, int split_k,
                        hipStream_t stream) {
-  int rc = self_attention_args_ok(q_data, key_mask, mask_batches, bias_quad_major, w_qkvg, out, out_dtype, num_head,
-                                  batch, seq, channels);
+  // (inside the library a plane of quads may end in a partly filled one)
+  int rc = self_attention_args_ok(q_data, key_mask, mask_batches, 0, w_qkvg, out, out_dtype, num_head, batch, seq, channels);
   if (rc) return rc;
   Carver ws(workspace, workspace_bytes);
   bf16_t* qkvg = ws.take<bf16_t>((size_t)batch * seq * 4 * channels);

@@ -219,6 +219,7 @@ struct AttnProjArgs {
   const bf16_t* w_bias = nullptr;  // [roundup(n_bias, 32)][128]
   int n_bias = 0;
   float* out_bias = nullptr;       // [n_bias][N][N] fp32, or
+  int quads = 0;                   // out_bias is [n_bias][ceil(N / 4)][N][4], quads of keys outermost
   bf16_t* out_bias_bf16 = nullptr; // [n_bias][N][ld_bias] bf16 (values times bias_scale)
   int64_t ld_bias = 0;
   float bias_scale = 1.f;

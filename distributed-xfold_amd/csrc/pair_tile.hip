@@ -302,19 +302,26 @@ __global__ __launch_bounds__(256, 2) void trimul_epilogue_kernel(TriMulArgs a) {
 // ============================================================================
 // triangle attention: projections
 // ============================================================================
-template <typename TIO, bool CROSS>
+// TILES: those of a pair tile kernel (tiles that cross rows or do not), or TILE_QUADS: 32 queries x 4 keys, for logits
+// with quads of keys outermost, [head][key / 4][query][key % 4] (keys past the end of the last quad: zeros).
+enum { TILE_ROWS = 0, TILE_CROSS = 1, TILE_QUADS = 2 };
+template <typename TIO, int TILES>
 __global__ __launch_bounds__(256, 2) void attn_proj_kernel(AttnProjArgs a) {
   __shared__ __attribute__((aligned(16))) bf16_t sX[TM * LDX];
   __shared__ __attribute__((aligned(16))) bf16_t sW[TM * LDX];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // (b, s) = (o, r): for the transposed operator a tile is a column segment
-  const auto t = make_tile<CROSS>(a.N, a.N, a.transpose != 0);
+  const auto t = [&] {
+    if constexpr (TILES == TILE_QUADS) return make_tile_quads(a.N);
+    else return make_tile<TILES == TILE_CROSS>(a.N, a.N, a.transpose != 0);
+  }();
   const TIO* x = reinterpret_cast<const TIO*>(a.pair);
   load_ln_tile<TIO>(x, t, a.ln_w, a.ln_b, sX, tid, a.skip_ln != 0, a.lw.inv_c, a.lw.pad);
   lds_barrier();
   bf16x8 xf[8];
   load_x_frags(sX, wave, lane, xf);
 
+  if constexpr (TILES != TILE_QUADS) {
   for (int chunk = 0; chunk < a.n_chunks; ++chunk) {
     load_w_rows(a.w_main + (int64_t)chunk * TM * C, sW, TM, tid);
     lds_barrier();
@@ -345,6 +352,7 @@ __global__ __launch_bounds__(256, 2) void attn_proj_kernel(AttnProjArgs a) {
     }
     lds_barrier();
   }
+  }
 
   // pair-bias heads: out_bias[h][q][k] with (q, k) the pixel's own (row, col)
   for (int h0 = 0; h0 < a.n_bias; h0 += 32) {
@@ -353,7 +361,15 @@ __global__ __launch_bounds__(256, 2) void attn_proj_kernel(AttnProjArgs a) {
     f32x16 acc[1];
     mfma_chunk<true, 1>(xf, sW, lane, acc);
     const int p = wave * 32 + (lane & 31);
-    if (t.valid(p)) {
+    if constexpr (TILES == TILE_QUADS) {
+      if (t.query(p) < a.N) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int h = h0 + acc_row(r, lane);
+          if (h < a.n_bias) a.out_bias[((int64_t)h * t.quads + t.quad) * a.N * 4 + t.query(p) * 4 + (p & 3)] = t.valid(p) ? acc[0][r] : 0.f;
+        }
+      }
+    } else if (t.valid(p)) {
       const int64_t pixel = t.pix(p);  // = q * N + k
       const int q = (int)(pixel / a.N), k = (int)(pixel % a.N);
 #pragma unroll
@@ -787,6 +803,11 @@ int launch_attn_proj(const AttnProjArgs& a, hipStream_t s) {
   if (a.n_bias > 0 && (!a.w_bias || (!a.out_bias && !a.out_bias_bf16))) return AF3_ERR_BAD_ARG;
   if (a.out_bias_bf16 && a.ld_bias < a.N) return AF3_ERR_BAD_ARG;
   if (!aligned16(a.pair) || !aligned16(a.w_main) || !aligned16(a.out_main) || !aligned16(a.w_bias)) return AF3_ERR_BAD_ARG;
+  if (a.quads) {
+    if (a.n_chunks > 0 || a.out_bias_bf16 || a.transpose) return AF3_ERR_BAD_ARG;
+    const int64_t n = (int64_t)((a.N + 31) / 32) * ((a.N + 3) / 4) * TM;
+    return a.io_f32 ? launch_tiles(attn_proj_kernel<float, TILE_QUADS>, a, n, s) : launch_tiles(attn_proj_kernel<bf16_t, TILE_QUADS>, a, n, s);
+  }
   LAUNCH_TILES(attn_proj_kernel, tile_crosses(a.N), (int64_t)a.N * a.N);
 }
 int launch_attn_out(const AttnOutArgs& a, hipStream_t s) {

@@ -71,7 +71,7 @@ int single_update(const af3_pairformer_block& b, void* single, int dt, const flo
     return run_linear(in, wt, nullptr, out, out_dt, n, n_out, k, mode, 1.f, 0, nullptr, 0, 0, res, dt, 1, st);
   };
   STEP(af3_layer_norm_forward(single, dt, x, n, c, b.sa_ln_w, b.sa_ln_b, nullptr, nullptr, 0, 0, s));
-  STEP(run_self_attention(x, mask, 1, logits, 0, b.sa_w_qkvg, b.sa_q_b, b.num_head, y, AF3_BF16, 1, n, c, aw, ab, 1, st));
+  STEP(run_self_attention(x, mask, 1, logits, 1, b.sa_w_qkvg, b.sa_q_b, b.num_head, y, AF3_BF16, 1, n, c, aw, ab, 1, st));
   STEP(product(y, b.sa_w_out, single, dt, c, c, AF3_LINEAR_GATE_RES, single));
   STEP(af3_layer_norm_forward(single, dt, x, n, c, b.st_ln_w, b.st_ln_b, nullptr, nullptr, 0, 0, s));
   STEP(product(x, b.st_w1, y, AF3_BF16, 2 * h, c, AF3_LINEAR_SWIGLU, nullptr));
@@ -247,11 +247,11 @@ int af3_pairformer_stack_forward(
     rc = pair_operators(b, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes, stream);
     if (rc != AF3_OK || !b.with_single) continue;
     // the only reader of `pair` on the single path: it stays in front of whatever updates `pair` next
-    float* lg = logits + (size_t)(num_blocks > 1 ? i & 1 : 0) * b.num_head * n * n;
+    float* lg = logits + (size_t)(num_blocks > 1 ? i & 1 : 0) * b.num_head * ((n + 3) / 4 * 4) * n;
     hipEvent_t& done = read_done[i & 1];
     if (done && hipStreamWaitEvent(main_s, done, 0) != hipSuccess) rc = AF3_ERR_LAUNCH;
     if (rc == AF3_OK)
-      rc = af3_pair_logits_forward(pair, pair_dtype, b.sl_ln_w, b.sl_ln_b, b.sl_w, b.num_head, lg, n, stream);
+      rc = af3_pair_logits_quads_forward(pair, pair_dtype, b.sl_ln_w, b.sl_ln_b, b.sl_w, b.num_head, lg, n, stream);
     if (rc == AF3_OK && two) rc = order_streams(main_s, side_s);
     if (rc == AF3_OK)
       rc = single_update(b, single, single_dtype, seq_mask, lg, n, single_workspace, single_workspace_bytes, side_s);

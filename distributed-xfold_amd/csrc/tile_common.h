@@ -95,6 +95,25 @@ __device__ __forceinline__ TileT<false> make_tile_in_row(int N) {
   return t;
 }
 
+// 32 queries x 4 keys of the pair: position p is query q0 + p / 4, key 4 quad + p % 4; a wave's 32 positions are 8 quads.
+struct TileQuads {
+  int N, q0, quad, quads;
+  __device__ __forceinline__ int query(int p) const { return q0 + (p >> 2); }
+  __device__ __forceinline__ bool valid(int p) const { return query(p) < N && 4 * quad + (p & 3) < N; }
+  __device__ __forceinline__ int64_t pix(int p) const {
+    return (int64_t)min(query(p), N - 1) * N + min(4 * quad + (p & 3), N - 1);
+  }
+  __device__ __forceinline__ bool full() const { return q0 + 32 <= N && 4 * quad + 4 <= N; }
+};
+__device__ __forceinline__ TileQuads make_tile_quads(int N) {
+  TileQuads t;
+  t.N = N;
+  t.quads = (N + 3) / 4;
+  t.quad = blockIdx.x % t.quads;
+  t.q0 = blockIdx.x / t.quads * 32;
+  return t;
+}
+
 // Eight consecutive fp32 parameters (LayerNorm weight / bias slice of a thread),
 // or a constant when the pointer is null.
 __device__ __forceinline__ void load_param8(const float* p, float fill, float* out) {

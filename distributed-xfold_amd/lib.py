@@ -80,6 +80,7 @@ SIGNATURES = {
         _i, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i, _vp, _i, _i64, _i64, _i64, _i64, _i64, _i,
              _vp, _sz, _vp]),
     "af3_pair_logits_forward": (_i, [_vp, _i, _vp, _vp, _vp, _i, _vp, _i64, _vp]),
+    "af3_pair_logits_quads_forward": (_i, [_vp, _i, _vp, _vp, _vp, _i, _vp, _i64, _vp]),
     "af3_layer_norm_forward": (_i, [_vp, _i, _vp, _i64, _i, _vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "af3_linear_forward": (
         _i, [_vp, _vp, _vp, _vp, _i, _i64, _i, _i, _i, _f, _i, _vp, _i64, _i64, _vp, _i, _vp]),

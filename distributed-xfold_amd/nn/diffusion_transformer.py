@@ -269,11 +269,8 @@ class DiffusionTransformer(HipModule):
         n_out = self.super_block_size * self.num_head
         out = []
         for sb in range(self.num_super_blocks):
-            logits = ops.pair_logits(pair_cond, p["ln_w"], None, p["w_logits"][sb], n_out)
-            logits = logits.view(self.super_block_size, self.num_head, *logits.shape[1:])     # (b h) n s -> b h n s
-            if logits.shape[-1] % 4 == 0:
-                logits = ops.quad_major_bias(logits)     # computed once, read by every evaluation
-            out.append(logits)
+            logits = ops.pair_logits(pair_cond, p["ln_w"], None, p["w_logits"][sb], n_out, quads=pair_cond.shape[0] % 4 == 0)
+            out.append(logits.view(self.super_block_size, self.num_head, *logits.shape[1:]))     # (b h) .. -> b h ..
         return out
 
     def forward(self, act: torch.Tensor, mask: torch.Tensor, single_cond: torch.Tensor,
@@ -291,9 +288,8 @@ class DiffusionTransformer(HipModule):
         ss_all = ops.linear(ops.layer_norm(sc), p["w_ss"], bias=p["b_ss"], out_dtype=torch.float32)
         gate_all = ops.linear(sc.to(torch.bfloat16), p["w_gate"], bias=p["b_gate"], out_dtype=torch.float32,
                               sigmoid=True)
-        if pair_logits is None:    # read once: in the order the projection writes them
-            pair_logits = [ops.pair_logits(pair_cond.contiguous(), p["ln_w"], None, w, self.super_block_size * self.num_head)
-                           .view(self.super_block_size, self.num_head, *pair_cond.shape[:2]) for w in p["w_logits"]]
+        if pair_logits is None:
+            pair_logits = self.pair_logits(pair_cond)
         ss_all, gate_all = ss_all.view(rows, n_mod, 2 * c), gate_all.view(rows, n_mod, c)
         run = self.num_super_blocks * self.super_block_size      # blocks beyond the last whole super-block never run
         if run == 0:

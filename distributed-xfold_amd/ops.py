@@ -218,7 +218,7 @@ def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incomi
         _gpu(single, "single", shape=(n, b.c_single))
         single_dt = _dt(single)
         seqf = _mask_f32(seq_mask, (n,), "key_mask")
-        logits = torch.empty((min(len(blocks), 2), b.num_head, n, n), dtype=torch.float32, device=dev)
+        logits = torch.empty((min(len(blocks), 2), b.num_head, n, (n + 3) // 4 * 4), dtype=torch.float32, device=dev)
         sws = _ws(lib.af3_pairformer_single_workspace_bytes(n, b.c_single, b.single_hidden), dev, single_stream)
         if single_stream is not None and not join:
             for t in (logits, seqf):
@@ -756,9 +756,9 @@ def batched_nt_product(a, b, out=None):
     return out
 
 
-def pair_logits(pair, norm_weight, norm_bias, w_padded, n_out):
+def pair_logits(pair, norm_weight, norm_bias, w_padded, n_out, quads: bool = False):
     """LayerNorm + projection of the pair tensor to [n_out, N, N] fp32 logits
-    (nn/d_pairformer.py:160-162, nn/d_diffusion_transformer.py:299-305)."""
+    (nn/d_pairformer.py:160-162, nn/d_diffusion_transformer.py:299-305), or with `quads` to [n_out, ceil(N / 4), N, 4]."""
     lib = _L.load()
     _gpu(pair, "pair")
     if pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair.shape[2] != 128:
@@ -770,9 +770,9 @@ def pair_logits(pair, norm_weight, norm_bias, w_padded, n_out):
     _gpu(w_padded, "w_padded", torch.bfloat16)
     if w_padded.dim() != 2 or w_padded.shape[1] != 128 or w_padded.shape[0] % 32 or w_padded.shape[0] < n_out:
         raise ValueError("w_padded: expected [roundup(n_out, 32), 128]")
-    out = torch.empty((n_out, n, n), dtype=torch.float32, device=pair.device)
-    rc = lib.af3_pair_logits_forward(_p(pair), _dt(pair), _p(norm_weight), _p(norm_bias), _p(w_padded),
-                                     int(n_out), _p(out), n, _stream(pair.device))
+    out = torch.empty((n_out, (n + 3) // 4, n, 4) if quads else (n_out, n, n), dtype=torch.float32, device=pair.device)
+    call = lib.af3_pair_logits_quads_forward if quads else lib.af3_pair_logits_forward
+    rc = call(_p(pair), _dt(pair), _p(norm_weight), _p(norm_bias), _p(w_padded), int(n_out), _p(out), n, _stream(pair.device))
     _L.check(rc, "af3_pair_logits_forward")
     return out
 

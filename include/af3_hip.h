@@ -353,6 +353,10 @@ int af3_position_update_forward(const uint16_t* x, const int32_t* rows, const fl
 int af3_pair_logits_forward(
     const void* pair, int io_dtype, const float* norm_weight, const float* norm_bias,
     const uint16_t* w, int n_out, float* out, int64_t n_token, af3_stream_t stream);
+/* ... as [n_out,ceil(n/4),n,4], quads of keys outermost (keys past n: zeros): the order the attention kernels read best */
+int af3_pair_logits_quads_forward(
+    const void* pair, int io_dtype, const float* norm_weight, const float* norm_bias,
+    const uint16_t* w, int n_out, float* out, int64_t n_token, af3_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * Row LayerNorm / adaptive LayerNorm -> bf16.  Replaces fastnn.LayerNorm on
@@ -505,7 +509,7 @@ int af3_pair_cond_init_forward(const void* pair, int pair_dtype, float in_scale,
  * logits).  The call makes single_stream wait for what `stream` holds on entry,
  * and with join != 0 makes `stream` wait for single_stream at the end; with
  * join = 0 the caller does that before anything else touches `single` or the
- * scratch.  logits: 2 * num_head * n * n floats (one block: half of it), used on
+ * scratch.  logits: 2 * num_head * n * roundup(n, 4) floats (one block: half of it), used on
  * both streams; single_workspace is used on single_stream only.
  */
 typedef struct af3_pairformer_block {

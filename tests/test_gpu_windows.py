@@ -55,3 +55,16 @@ def test_adaptive_norm(gpu_pkg, rows, c, dtype):
     n = torch.nn.functional.layer_norm(x.double(), (c,))
     want = torch.sigmoid(ss[:, :c].double()).repeat(3, 1) * n + ss[:, c:].double().repeat(3, 1)
     assert ((y - want).abs() <= 1.01 * 2.0 ** -8 * want.abs() + 1e-4).all()
+
+
+@pytest.mark.parametrize("n,dtype", [(1, torch.float32), (5, torch.bfloat16), (32, torch.float32), (67, torch.bfloat16), (132, torch.float32)])
+def test_pair_logits_of_the_token_attention_in_quads(gpu_pkg, n, dtype):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    pair = torch.randn(n, n, 128, generator=g, device="cuda").to(dtype)
+    w = torch.zeros(64, 128, device="cuda").bfloat16()
+    w[:40] = torch.randn(40, 128, generator=g, device="cuda")
+    ln = torch.rand(128, generator=g, device="cuda")
+    rows = gpu_pkg.ops.pair_logits(pair, ln, None, w, 40)
+    quads = gpu_pkg.ops.pair_logits(pair, ln, None, w, 40, quads=True)
+    want = torch.nn.functional.pad(rows, (0, -n % 4)).view(40, n, -1, 4).transpose(1, 2)
+    assert torch.equal(quads, want)
