@@ -351,6 +351,28 @@ struct TriAttnArgs {
 };
 int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream);
 
+// -------------------------------------------------------------------- embed.hip
+struct PairEmbedArgs {
+  const float* lr = nullptr;    // [n][ld_lr]: left projection, then right
+  int64_t ld_lr = 0;
+  const float* prev = nullptr;  // [n][n][128]
+  const int64_t *asym_id = nullptr, *residue_index = nullptr, *token_index = nullptr, *entity_id = nullptr, *sym_id = nullptr;
+  const float* w_pos = nullptr;    // [139][128]
+  const float* w_bond = nullptr;   // [128]
+  const float* contact = nullptr;  // [n][n]
+  void* out = nullptr;             // [n][n][128]
+  int out_f32 = 0, n = 0;
+};
+int launch_pair_embed(const PairEmbedArgs& a, hipStream_t s);
+int launch_contacts(const int64_t* idx0, const uint8_t* ok0, int n0, const int64_t* idx1, const uint8_t* ok1, int n1, float* contact,
+                    int n, hipStream_t s);
+int launch_add_rows(const float* a, const float* b, int64_t ld_b, int64_t mod, void* out, int out_f32, int64_t rows, int channels,
+                    hipStream_t s);
+int launch_mask_rows(bf16_t* x, const float* mask, int64_t mod, int64_t rows, int channels, hipStream_t s);
+enum { POS_SCALE = 0, POS_BLEND = 1, POS_PLACE = 2, POS_STEP = 3 };
+int launch_positions(int op, const float* x, const float* y, const float* mask, const float* level, const float* other, float f,
+                     float* out, int64_t samples, int64_t atoms, hipStream_t s);
+
 // ---------------------------------------------------------------------- msa.hip
 struct MsaProjectArgs {
   const void* msa = nullptr;  // [rows][n][64]

@@ -363,4 +363,37 @@ int af3_atom_transformer_forward(
   return AF3_OK;
 }
 
+// ------------------------------------------------------------- element-wise passes
+int af3_contact_matrix_forward(const int64_t* idx0, const uint8_t* exists0, int count0, const int64_t* idx1, const uint8_t* exists1,
+                               int count1, float* contact, int64_t n, af3_stream_t stream) {
+  if (n <= 0 || n > 8192) return AF3_ERR_BAD_ARG;
+  return launch_contacts(idx0, exists0, count0, idx1, exists1, count1, contact, (int)n, static_cast<hipStream_t>(stream));
+}
+
+int af3_pair_embed_forward(const float* lr, int64_t ld_lr, const float* prev, const int64_t* asym_id, const int64_t* residue_index,
+                           const int64_t* token_index, const int64_t* entity_id, const int64_t* sym_id, const float* w_pos,
+                           const float* w_bond, const float* contact, void* out, int out_dtype, int64_t n, af3_stream_t stream) {
+  if (n <= 0 || n > 8192 || (out_dtype != AF3_F32 && out_dtype != AF3_BF16)) return AF3_ERR_BAD_ARG;
+  PairEmbedArgs a;
+  a.lr = lr; a.ld_lr = ld_lr; a.prev = prev;
+  a.asym_id = asym_id; a.residue_index = residue_index; a.token_index = token_index; a.entity_id = entity_id; a.sym_id = sym_id;
+  a.w_pos = w_pos; a.w_bond = w_bond; a.contact = contact; a.out = out; a.out_f32 = out_dtype == AF3_F32; a.n = (int)n;
+  return launch_pair_embed(a, static_cast<hipStream_t>(stream));
+}
+
+int af3_add_rows_forward(const float* a, const float* b, int64_t ld_b, int64_t mod, void* out, int out_dtype, int64_t rows,
+                         int channels, af3_stream_t stream) {
+  if (out_dtype != AF3_F32 && out_dtype != AF3_BF16) return AF3_ERR_BAD_ARG;
+  return launch_add_rows(a, b, ld_b, mod, out, out_dtype == AF3_F32, rows, channels, static_cast<hipStream_t>(stream));
+}
+
+int af3_mask_rows_forward(uint16_t* x, const float* mask, int64_t mod, int64_t rows, int channels, af3_stream_t stream) {
+  return launch_mask_rows(x, mask, mod, rows, channels, static_cast<hipStream_t>(stream));
+}
+
+int af3_positions_forward(int op, const float* x, const float* y, const float* mask, const float* level, const float* next,
+                          float factor, float* out, int64_t samples, int64_t atoms, af3_stream_t stream) {
+  return launch_positions(op, x, y, mask, level, next, factor, out, samples, atoms, static_cast<hipStream_t>(stream));
+}
+
 }  // extern "C"

@@ -55,6 +55,12 @@ SIGNATURES = {
     "af3_grid_self_attn_forward_padded": (
         _i, [_vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _i64, _i, _vp, _sz, _vp]),
     "af3_transition_forward_padded": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _i, _i64, _i, _vp]),
+    "af3_contact_matrix_forward": (_i, [_vp, _vp, _i, _vp, _vp, _i, _vp, _i64, _vp]),
+    "af3_pair_embed_forward": (
+        _i, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i64, _vp]),
+    "af3_add_rows_forward": (_i, [_vp, _vp, _i64, _i64, _vp, _i, _i64, _i, _vp]),
+    "af3_mask_rows_forward": (_i, [_vp, _vp, _i64, _i64, _i, _vp]),
+    "af3_positions_forward": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _f, _vp, _i64, _i64, _vp]),
     "af3_msa_workspace_bytes": (_sz, [_i64, _i64]),
     "af3_outer_product_mean_forward": (_i, [_vp, _vp, _i, _vp, _vp, _i, _i, _i64, _i64, _vp, _sz, _vp]),
     "af3_msa_attention_forward": (_i, [_vp, _vp, _i, _vp, _vp, _i, _vp, _i, _i64, _i64, _vp, _sz, _vp]),

@@ -68,6 +68,7 @@ class EncoderConditioning:
     keys_single_cond: torch.Tensor
     pair_cond: torch.Tensor
     transformer_cond: Any
+    atom_count: Optional[torch.Tensor] = None      # [N], atoms per token, at least 1e-10
 
 
 class AtomCrossAttEncoder(HipModule):
@@ -206,7 +207,11 @@ class AtomCrossAttEncoder(HipModule):
         if not in_check_mode():
             tcond = self.atom_transformer_encoder.conditioning(q_cond, k_cond, pair_act,
                                                                keys_are_query_atoms=aca.queries_to_keys)
-        return EncoderConditioning(q_mask, q_cond, k_mask, k_cond, pair_act, tcond)
+        return EncoderConditioning(q_mask, q_cond, k_mask, k_cond, pair_act, tcond, self._atom_count(batch))
+
+    @staticmethod
+    def _atom_count(batch):
+        return torch.clamp(batch.predicted_structure_info.atom_mask.float().sum(-1), min=1e-10)
 
     @torch.no_grad()
     def forward(self, batch, token_atoms_act: Optional[torch.Tensor], trunk_single_cond: Optional[torch.Tensor],
@@ -250,15 +255,17 @@ class AtomCrossAttEncoder(HipModule):
             queries_act=q_act, queries_mask=c.queries_mask, queries_to_keys=aca.queries_to_keys,
             keys_mask=c.keys_mask, queries_single_cond=c.queries_single_cond,
             keys_single_cond=c.keys_single_cond, pair_cond=c.pair_cond, cond=c.transformer_cond)
-        q_act = q_act * qm.to(q_act.dtype)
+        if q_act.dtype == torch.bfloat16:
+            q_act = ops.mask_rows(q_act, c.queries_mask.float().contiguous())
+        else:
+            q_act = q_act * qm.to(q_act.dtype)
         skip = q_act
         if in_check_mode():
             agg = check._lin(q_act.contiguous(), self.project_atom_features_for_aggr)
         else:
             agg = ops.linear(q_act.to(torch.bfloat16).contiguous(), self.packed()["w_aggr"])
-        tm = batch.predicted_structure_info.atom_mask.float()
         # mask_mean over the atoms of a token (:328-331); the gather zeroes the absent atoms
-        count = torch.clamp(tm.sum(-1), min=1e-10)
+        count = c.atom_count if c.atom_count is not None else self._atom_count(batch)
         if in_check_mode():
             tok_atoms = convert(aca.queries_to_token_atoms, agg, (-3, -2))
             tok_act = torch.relu(tok_atoms).float().sum(-2) / count[..., None]
@@ -327,8 +334,6 @@ class AtomCrossAttDecoder(HipModule):
         # conversion to the query layout is the gather of token rows
         ta2q = aca.token_atoms_to_queries
         n_dense = aca.queries_to_token_atoms.gather_idxs.shape[1]
-        qm = enc.queries_mask.to(t.dtype)
-        qm = qm[None, ..., None] if batched else qm[..., None]
         fused = not in_check_mode() and enc.skip_connection.dtype == torch.bfloat16
         if fused:
             # gather, + skip connection and query mask in one pass (the skip connection is zero where the mask is)
@@ -346,6 +351,8 @@ class AtomCrossAttDecoder(HipModule):
         else:
             q_act = convert(GatherInfo(ta2q.gather_idxs // n_dense, ta2q.gather_mask, (t.shape[-2],)), t, (-2,))
             q_act = q_act + enc.skip_connection.to(q_act.dtype)
+            qm = enc.queries_mask.to(t.dtype)
+            qm = qm[None, ..., None] if batched else qm[..., None]
             q_act = (q_act * qm.to(q_act.dtype)).to(enc.skip_connection.dtype).contiguous()
         q_act = self.atom_transformer_decoder(
             queries_act=q_act, queries_mask=enc.queries_mask, queries_to_keys=aca.queries_to_keys,

@@ -244,9 +244,12 @@ class DiffusionHead(HipModule):
         p = self.packed()
         batched = self.use_batch_infer
         positions_noisy = positions_noisy.float()
-        am = batch.predicted_structure_info.atom_mask.float()
-        am = am[None, ..., None] if batched else am[..., None]
-        act = positions_noisy * am / torch.sqrt(noise_level ** 2 + SIGMA_DATA ** 2)
+        if batched and positions_noisy.dim() == 3:
+            positions_noisy = positions_noisy[None]
+        positions_noisy = positions_noisy.contiguous()
+        am = batch.predicted_structure_info.atom_mask.float().contiguous()
+        level = torch.as_tensor(noise_level, dtype=torch.float32, device=positions_noisy.device)
+        act = ops.positions(ops.POS_SCALE, positions_noisy, None, am, level)
         enc = self.atom_cross_att_encoder(batch=batch, token_atoms_act=act, trunk_single_cond=embeddings["single"],
                                           trunk_pair_cond=trunk_pair_cond, conditioning=state.encoder,
                                           act_dtype=act_dtype)
@@ -256,7 +259,7 @@ class DiffusionHead(HipModule):
         else:
             emb = ops.linear(ops.layer_norm(trunk_single_cond.contiguous(), p["emb_ln"]), p["w_emb"],
                              out_dtype=torch.float32)
-        act = (enc.token_act + (emb[None] if batched else emb)).to(act_dtype).contiguous()
+        act = ops.add_rows(enc.token_act.float().contiguous(), emb, act_dtype)
         act = self.transformer(act=act, mask=batch.token_features.mask, single_cond=trunk_single_cond,
                                pair_cond=trunk_pair_cond, pair_logits=state.pair_logits)
         if in_check_mode():
@@ -264,9 +267,7 @@ class DiffusionHead(HipModule):
         else:
             act = ops.layer_norm(act, p["out_ln"])
         upd = self.atom_cross_att_decoder(batch=batch, token_act=act, enc=enc, transformer_cond=state.decoder_cond)
-        skip = SIGMA_DATA ** 2 / (noise_level ** 2 + SIGMA_DATA ** 2)
-        out = noise_level * SIGMA_DATA / torch.sqrt(noise_level ** 2 + SIGMA_DATA ** 2)
-        return (skip * positions_noisy + out * upd) * am
+        return ops.positions(ops.POS_BLEND, positions_noisy, upd.contiguous(), am, level)
 
 
 class DiffusionSampler:
@@ -309,17 +310,21 @@ class DiffusionSampler:
         if positions is None:
             positions = torch.randn((self.num_samples,) + tuple(mask.shape) + (3,), generator=generator, device=dev)
         positions = positions.float() * levels[0]
+        # the mean of random_augmentation divides by a count that no step changes
+        m = mask.to(positions.dtype)[None, ..., None]
+        count = torch.clamp(m.expand_as(positions[..., :1]).sum(dim=(-2, -3), keepdim=True), min=1e-6)
+        mask_f = mask.float().contiguous()
         for i in range(self.diffusion_steps):
             rot = rotations[i] if rotations is not None else random_rotation(generator, dev)
             trans = translations[i] if translations is not None else torch.randn(3, generator=generator, device=dev)
-            positions = random_augmentation(positions, mask[None], rot.float(), trans.float())
-            if noises is not None:
-                noisy = positions + nscale[i] * noises[i]
-            elif self.gaussian_noise:
-                noisy = positions + nscale[i] * torch.randn(positions.shape, generator=generator, device=dev)
-            else:
-                noisy = positions + nscale[i]
+            if noises is not None or self.gaussian_noise:
+                positions = random_augmentation(positions, mask[None], rot.float(), trans.float())
+                noise = noises[i] if noises is not None else torch.randn(positions.shape, generator=generator, device=dev)
+                noisy = positions + nscale[i] * noise
+            else:   # random_augmentation, and the step's scalar of noise added
+                center = (m * positions).sum(dim=(-2, -3), keepdim=True) / count
+                turned = torch.einsum("...i,ij->...j", positions - center, rot.float())
+                noisy = ops.positions(ops.POS_PLACE, turned.contiguous(), trans.float().contiguous(), mask_f, nscale[i])
             denoised = head(noisy, t_hat[i], batch, embeddings, single_cond[i], pair_cond, state=state)
-            grad = (noisy - denoised) / t_hat[i]
-            positions = noisy + self.step_scale * (levels[i + 1] - t_hat[i]) * grad
+            positions = ops.positions(ops.POS_STEP, noisy, denoised, None, t_hat[i], levels[i + 1], self.step_scale)
         return {"atom_positions": positions, "mask": mask}

@@ -58,8 +58,10 @@ class Evoformer(HipModule):
 
     def _pack(self):
         return dict(
-            w_lr=_pad_k(torch.cat([self.left_single.weight, self.right_single.weight], dim=0)),
-            w_tf_msa=_pad_k(self.extra_msa_target_feat.weight), w_tf_single=_pad_k(self.single_activations.weight),
+            # everything that is projected from the target features, in one product: left, right, msa, single
+            w_tf=_pad_k(torch.cat([self.left_single.weight, self.right_single.weight, self.extra_msa_target_feat.weight,
+                                   self.single_activations.weight], dim=0)),
+            w_pos=f32(self.position_activations.weight.t()), w_bond=f32(self.bond_embedding.weight[:, 0]),
             w_msa=_pad_k(self.msa_activations.weight),
             prev_ln_w=f32(self.prev_embedding_layer_norm.weight), prev_ln_b=f32(self.prev_embedding_layer_norm.bias),
             w_prev=bf16(self.prev_embedding.weight),
@@ -96,45 +98,52 @@ class Evoformer(HipModule):
         dt = torch.float32 if chk else self.act_dtype
         mask = batch.token_features.mask.float()
         n = mask.shape[0]
-        if chk:
-            lr = torch.cat([check._lin(target_feat.float().contiguous(), self.left_single),
-                            check._lin(target_feat.float().contiguous(), self.right_single)], dim=-1)
-        else:
-            lr = self._lin(target_feat, None, p["w_lr"])
         cp = self.pair_channel
-        pair = lr[:, None, :cp] + lr[None, :, cp:]
         pair_mask = (mask[:, None] * mask[None, :]).contiguous()
         if chk:
+            left, right = (check._lin(target_feat.float().contiguous(), m) for m in (self.left_single, self.right_single))
+            pair = left[:, None] + right[None, :]
             pair = pair + check._lin(check._ln(prev["pair"].float().contiguous(), self.prev_embedding_layer_norm),
                                      self.prev_embedding)
+            # one-hot relative encoding and the 0/1 contact matrix: look-ups / a scaled weight column
+            rel = create_relative_encoding(batch.token_features, 32, 2)
+            wpos = self.position_activations.weight.float().t()                      # [139, 128]
+            pair = pair + wpos[rel[..., :66].argmax(-1)] + wpos[66 + rel[..., 66:132].argmax(-1)]
+            pair = pair + rel[..., 132:133].float() * wpos[132] + wpos[133 + rel[..., 133:].argmax(-1)]
+            pair = pair + self.contact_matrix(batch, n, pair.device)[:, :, None] * self.bond_embedding.weight.float()[:, 0]
+            pair = pair.to(dt).contiguous()
         else:
-            pair = pair + ops.linear(ops.layer_norm(prev["pair"].contiguous(), p["prev_ln_w"], p["prev_ln_b"]),
-                                     p["w_prev"], out_dtype=torch.float32)
-        # one-hot relative encoding and the 0/1 contact matrix: look-ups / a scaled weight column
-        rel = create_relative_encoding(batch.token_features, 32, 2)
-        wpos = self.position_activations.weight.float().t()                      # [139, 128]
-        off = (0, 66, 132, 133)
-        pair = pair + wpos[off[0] + rel[..., :66].argmax(-1)] + wpos[off[1] + rel[..., 66:132].argmax(-1)]
-        pair = pair + rel[..., 132:133].float() * wpos[132] + wpos[off[3] + rel[..., 133:].argmax(-1)]
-        pair = pair + self.contact_matrix(batch, n, pair.device)[:, :, None] * self.bond_embedding.weight.float()[:, 0]
-        pair = pair.to(dt).contiguous()
+            tf_all = self._lin(target_feat, None, p["w_tf"])                # [N, left | right | msa | single]
+            prev_pair = ops.linear(ops.layer_norm(prev["pair"].contiguous(), p["prev_ln_w"], p["prev_ln_b"]), p["w_prev"],
+                                   out_dtype=torch.float32)
+            tok = batch.token_features
+            ids = tuple(getattr(tok, k).to(torch.int64).contiguous()
+                        for k in ("asym_id", "residue_index", "token_index", "entity_id", "sym_id"))
+            contact = ops.contact_matrix((batch.polymer_ligand_bond_info.tokens_to_polymer_ligand_bonds,
+                                          batch.ligand_ligand_bond_info.tokens_to_ligand_ligand_bonds), n, prev_pair.device)
+            pair = ops.pair_embed(tf_all, prev_pair, ids, p["w_pos"], p["w_bond"], contact, dt)
         if self.template_embedding is not None:
             asym = batch.token_features.asym_id
             pair = pair + self.template_embedding(query_embedding=pair, templates=batch.templates,
                                                   multichain_mask_2d=(asym[:, None] == asym[None, :]).to(pair.dtype),
                                                   padding_mask_2d=pair_mask)
         msa = self._lin(batch.msa_feat, self.msa_activations, p["w_msa"])
-        msa = (msa + self._lin(target_feat, self.extra_msa_target_feat, p["w_tf_msa"])[None]).to(dt).contiguous()
+        cm = self.msa_channel
+        if chk:
+            msa = (msa + self._lin(target_feat, self.extra_msa_target_feat, None)[None]).to(dt).contiguous()
+        else:
+            msa = ops.add_rows(msa, tf_all[:, 2 * cp:2 * cp + cm], dt)
         msa_mask = batch.msa_mask.float().contiguous()
         msa, pair = evoformer_loop(self.msa_stack, msa, pair, msa_mask, pair_mask)
-        single = self._lin(target_feat, self.single_activations, p["w_tf_single"])
         if chk:
+            single = self._lin(target_feat, self.single_activations, None)
             single = single + check._lin(check._ln(prev["single"].float().contiguous(),
                                                    self.prev_single_embedding_layer_norm), self.prev_single_embedding)
+            single = single.to(dt).contiguous()
         else:
-            single = single + ops.linear(ops.layer_norm(prev["single"].contiguous(), p["prevs_ln_w"], p["prevs_ln_b"]),
-                                         p["w_prevs"], out_dtype=torch.float32)
-        single = single.to(dt).contiguous()
+            single = ops.linear(ops.layer_norm(prev["single"].contiguous(), p["prevs_ln_w"], p["prevs_ln_b"]),
+                                p["w_prevs"], out_dtype=torch.float32)
+            single = ops.add_rows(single, tf_all[:, 2 * cp + cm:], dt)
         pair, single = pairformer_loop(self.trunk_pairformer, pair, pair_mask, single, mask)
         return {"single": single, "pair": pair, "target_feat": target_feat}
 

@@ -232,6 +232,91 @@ def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incomi
     _L.check(rc, "af3_pairformer_stack_forward")
 
 
+def contact_matrix(bonds, n, device):
+    """[n, n] fp32: 1 at every bond of two gather infos (gather_idxs [count, 2], gather_mask [count, 2]), [0, 0] excepted."""
+    lib = _L.load()
+    contact = torch.zeros((n, n), dtype=torch.float32, device=device)
+    idx = [b.gather_idxs.to(device=device, dtype=torch.int64).contiguous() for b in bonds]
+    ok = [b.gather_mask.to(device=device, dtype=torch.bool).contiguous() for b in bonds]
+    for i, m in zip(idx, ok):
+        if i.dim() != 2 or i.shape[1] != 2 or m.shape != i.shape:
+            raise ValueError("bonds: expected gather_idxs and gather_mask [count, 2]")
+    rc = lib.af3_contact_matrix_forward(_p(idx[0]), _p(ok[0]), idx[0].shape[0], _p(idx[1]), _p(ok[1]), idx[1].shape[0],
+                                        _p(contact), n, _stream(contact.device))
+    _L.check(rc, "af3_contact_matrix_forward")
+    return contact
+
+
+def pair_embed(lr, prev, token_ids, w_pos, w_bond, contact, out_dtype):
+    """The trunk's pair embedding [n, n, 128] (af3_pair_embed_forward).  lr: fp32 [n, >= 256] with unit column stride;
+    token_ids: asym_id, residue_index, token_index, entity_id, sym_id, int64 [n]."""
+    lib = _L.load()
+    n = lr.shape[0]
+    if not lr.is_cuda or lr.dtype != torch.float32 or lr.dim() != 2 or lr.shape[1] < 256 or lr.stride(1) != 1:
+        raise ValueError("lr: expected an fp32 GPU matrix [n, >= 256] with unit column stride")
+    _gpu(prev, "prev", torch.float32, (n, n, 128))
+    _gpu(contact, "contact", torch.float32, (n, n))
+    _gpu(w_pos, "w_pos", torch.float32, (139, 128))
+    _gpu(w_bond, "w_bond", torch.float32, (128,))
+    for t in token_ids:
+        _gpu(t, "token_ids", torch.int64, (n,))
+    out = torch.empty((n, n, 128), dtype=out_dtype, device=lr.device)
+    rc = lib.af3_pair_embed_forward(_p(lr), lr.stride(0), _p(prev), *[_p(t) for t in token_ids], _p(w_pos), _p(w_bond),
+                                    _p(contact), _p(out), _dt(out), n, _stream(lr.device))
+    _L.check(rc, "af3_pair_embed_forward")
+    return out
+
+
+def add_rows(a, b, out_dtype):
+    """a [.., n, c] + b [n, c] (a column slice of a wider matrix will do), both fp32, rounded to `out_dtype`."""
+    lib = _L.load()
+    _gpu(a, "a", torch.float32)
+    n, c = a.shape[-2:]
+    if not b.is_cuda or b.dtype != torch.float32 or tuple(b.shape) != (n, c) or b.stride(1) != 1:
+        raise ValueError(f"b: expected an fp32 GPU matrix [{n}, {c}] with unit column stride")
+    out = torch.empty(a.shape, dtype=out_dtype, device=a.device)
+    rc = lib.af3_add_rows_forward(_p(a), _p(b), b.stride(0), n, _p(out), _dt(out), a.numel() // c, c, _stream(a.device))
+    _L.check(rc, "af3_add_rows_forward")
+    return out
+
+
+def mask_rows(x, mask):
+    """x [.., r, c] bf16 times mask [r] fp32 in bf16, in place."""
+    lib = _L.load()
+    _gpu(x, "x", torch.bfloat16)
+    c = x.shape[-1]
+    _gpu(mask, "mask", torch.float32)
+    r = mask.numel()
+    if x.numel() % (r * c):
+        raise ValueError("x: rows must be a multiple of the mask's")
+    rc = lib.af3_mask_rows_forward(_p(x), _p(mask), r, x.numel() // c, c, _stream(x.device))
+    _L.check(rc, "af3_mask_rows_forward")
+    return x
+
+
+POS_SCALE, POS_BLEND, POS_PLACE, POS_STEP = range(4)
+
+
+def positions(op, x, y, mask, level, next_level=None, factor=0.0):
+    """The element-wise passes over atom positions [samples, N, A, 3] (af3_positions_forward); mask [N, A], `level` and
+    `next_level` one-element device tensors, all fp32."""
+    lib = _L.load()
+    _gpu(x, "x", torch.float32)
+    for nm, t in (("mask", mask), ("level", level), ("next_level", next_level), ("y", y)):
+        if t is not None:
+            _gpu(t, nm, torch.float32)
+    atoms = x.numel() // 3 if mask is None else mask.numel()
+    if x.shape[-1] != 3 or x.numel() % (3 * atoms):
+        raise ValueError("x: expected [samples, N, A, 3] over a mask [N, A]")
+    if y is not None and y.numel() != (3 if op == POS_PLACE else x.numel()):
+        raise ValueError(f"y: {tuple(y.shape)} does not go with x {tuple(x.shape)}")
+    out = torch.empty_like(x)
+    rc = lib.af3_positions_forward(op, _p(x), _p(y), _p(mask), _p(level), _p(next_level), factor, _p(out),
+                                   x.numel() // (3 * atoms), atoms, _stream(x.device))
+    _L.check(rc, "af3_positions_forward")
+    return out
+
+
 def _msa_inputs(msa, msa_mask):
     _gpu(msa, "msa")
     if msa.dim() != 3 or msa.shape[2] != 64:

@@ -544,6 +544,36 @@ int af3_pairformer_stack_forward(
     void* single_workspace, size_t single_workspace_bytes, af3_stream_t stream, af3_stream_t single_stream, int join);
 
 /* ---------------------------------------------------------------------------
+ * Element-wise passes of the trunk's input embedding (d_alphafold3.py:103-220) and of
+ * the diffusion head (nn/d_diffusion_head.py:171-227), fp32, every operation rounded.
+ *
+ * af3_contact_matrix_forward: contact [n,n] fp32 (zeroed by the caller) = 1 at every
+ *   bond of two lists (idx [count,2] int64, exists [count,2] bytes), [0,0] excepted.
+ * af3_pair_embed_forward: out [n,n,128] = left[i] + right[j] + prev[i,j] + the relative
+ *   encoding's weights + contact[i,j] * w_bond, summed in this order; lr [n][ld_lr] holds
+ *   left in columns 0.., right in columns 128..; w_pos [139][128] one row per one-hot
+ *   channel (residue offset 66, token offset 66, same entity, chain offset 6).
+ * af3_add_rows_forward: out[r] = a[r] + b[r % mod], a [rows,channels], b [mod][ld_b].
+ * af3_mask_rows_forward: x[r] *= mask[r % mod] in bf16, x [rows,channels] in place.
+ * af3_positions_forward on x [samples,atoms,3], mask [atoms]; level, next: device scalars
+ *   op 0: x mask / sqrt(level^2 + 256)
+ *   op 1: (c_skip x + c_out y) mask, the head's blend of input and update at noise `level`
+ *   op 2: (x + y) mask + level, y [3] (a rotated, shifted structure and a scalar of noise)
+ *   op 3: x + factor (next - level) (x - y) / level, a sampling step from noisy x, denoised y
+ */
+int af3_contact_matrix_forward(const int64_t* idx0, const uint8_t* exists0, int count0, const int64_t* idx1,
+                               const uint8_t* exists1, int count1, float* contact, int64_t n_token, af3_stream_t stream);
+int af3_pair_embed_forward(const float* lr, int64_t ld_lr, const float* prev, const int64_t* asym_id,
+                           const int64_t* residue_index, const int64_t* token_index, const int64_t* entity_id,
+                           const int64_t* sym_id, const float* w_pos, const float* w_bond, const float* contact, void* out,
+                           int out_dtype, int64_t n_token, af3_stream_t stream);
+int af3_add_rows_forward(const float* a, const float* b, int64_t ld_b, int64_t mod, void* out, int out_dtype, int64_t rows,
+                         int channels, af3_stream_t stream);
+int af3_mask_rows_forward(uint16_t* x, const float* mask, int64_t mod, int64_t rows, int channels, af3_stream_t stream);
+int af3_positions_forward(int op, const float* x, const float* y, const float* mask, const float* level, const float* next,
+                          float factor, float* out, int64_t samples, int64_t atoms, af3_stream_t stream);
+
+/* ---------------------------------------------------------------------------
  * The Evoformer's MSA track on 64 channels (nn/d_primitives.py:42-70,
  * nn/d_attention.py:113-156, nn/d_pairformer.py:174-252): msa [rows,n,64] and pair
  * [n,n,128] in their own dtypes, msa_mask [rows,n], pair_mask [n,n] or NULL.
