@@ -30,11 +30,13 @@ namespace {
 // ============================================================================
 // triangle multiplication, prologue
 // ============================================================================
-template <typename TIO, bool CROSS>
+// STEPS: all eight steps, or two or four of them, the others being other workgroups' (blockIdx.y): with few tiles the
+// kernel is one tile's chain of steps, and a LayerNorm more for each part is cheaper than the steps it saves.
+template <typename TIO, bool CROSS, int STEPS>
 __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
   // 34.8 KB + 17.4 KB + 0.5 KB of LDS and at most 168 registers: three workgroups per CU.
   //
-  // Eight steps of 64 weight rows (32 projection rows and the 32 matching gate rows) per tile.  A wave
+  // Steps of 64 weight rows (32 projection rows and the 32 matching gate rows) per tile.  A wave
   // runs them as a software pipeline: the 16 MFMAs of step s are issued one by one with, behind each, the
   // gating arithmetic (mask * proj * sigmoid(gate), packing, staging) of one register pair of step s - 1.
   // Inside one wave the matrix unit works while the wave goes on issuing vector instructions; between
@@ -56,12 +58,18 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
   // a thread's 16-byte pieces, from the first of 16 channels' planes on (one 32-bit offset: at most 2^31)
   const uint32_t lane_out = ((uint32_t)(tid >> 4) * (uint32_t)a.plane + (tid & 15) * 8) * 2u;
   const TIO* x = reinterpret_cast<const TIO*>(a.pair);
+  // This workgroup's steps: first, first + 1, ..; with 64 channels or fewer steps 2, 3, 6 and 7 are nobody's (their
+  // planes are not contracted).
+  const bool narrow = STEPS < 8 && a.valid_c <= 64;
+  const int first = (narrow ? 4 : STEPS) * (int)blockIdx.y;
+  auto global_step = [&](int s) { return first + s + (STEPS == 4 && narrow && s >= 2 ? 2 : 0); };
 
   // Weight chunks in memory: [P(64 ch) | G(64 ch)] for a ch 0-63, a ch 64-127, b ch 0-63, b ch 64-127.
   // Step s = 2 * chunk + half takes projection rows 32 half .. +31 and gate rows 64 + 32 half .. +31 of
   // its chunk: 64 rows x 128, four 16-byte pieces per thread.
   u32x4 wr[4];
   auto wload = [&](int s) {
+    s = global_step(s);
     const bf16_t* base = a.w_pg + ((int64_t)(s >> 1) * TM + (s & 1) * 32) * C;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -81,7 +89,7 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
     // Every position of the tile is masked (padding): a' and b' are zero there
     // whatever the activations are.  Write the zeros and skip the rest.
     const u32x4 z = {0, 0, 0, 0};
-    for (int idx = tid; idx < 2 * C * 16; idx += 256) {
+    for (int idx = tid + first * 512; idx < (global_step(STEPS - 1) + 1) * 512; idx += 256) {  // 32 planes a step
       const int op = idx >> 11, ch = (idx >> 4) & (C - 1);
       *reinterpret_cast<u32x4*>((op ? a.b_buf : a.a_buf) + ch * a.plane + t.l0 + (idx & 15) * 8) = z;
     }
@@ -97,7 +105,7 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
   load_x_frags(sX, wave, lane, xf);
   lds_barrier();  // sX is free from here on
   wstore(sW1);    // W_1
-  wload(2);
+  if constexpr (STEPS > 2) wload(2);
 
   f32x16 zero16;
 #pragma unroll
@@ -105,7 +113,11 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
   f32x16 accA[2], accB[2];  // [0] projection, [1] gate; A: even steps, B: odd steps
   const int ch = lane & 31;
 
-  // Step S (0..8): the MFMAs of step S (S < 8) into `cur`, the gating of step S - 1 (S > 0) out of `prev`.
+  auto results = [&](int s) {  // where step s's 32 channels go
+    s = global_step(s);
+    return (s < 4 ? a.a_buf : a.b_buf) + (s & 3) * 32 * a.plane + t.l0;
+  };
+  // Step S (0..STEPS): the MFMAs of step S (S < STEPS) into `cur`, the gating of step S - 1 (S > 0) out of `prev`.
   auto step = [&](auto step_c, f32x16* cur, f32x16* prev) {
     constexpr int S = decltype(step_c)::value;
     const bf16_t* w = (S & 1) ? sW1 : sW0;                    // W_S
@@ -123,7 +135,7 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
     }
     bf16x8 wf[3];  // weight fragments, read two MFMAs ahead
     auto frag = [&](int m) { return lds_frag(w, LDX, (m & 1) * 32, (m >> 1) * 16, lane); };  // MFMA m: k-step m / 2, tile m % 2
-    if (S < 8) {
+    if (S < STEPS) {
       wf[0] = frag(0);
       wf[1] = frag(1);
     }
@@ -133,7 +145,7 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
     for (int m = 0; m < 16; ++m) {
       if (S > 0 && (m & 3) == 0)  // the masks of pixels p0 .. p0 + 3, p0 = wave * 32 + 8 (m >> 2) + 4 hh
         m4 = *reinterpret_cast<const f32x4*>(sMask + wave * 32 + 2 * m + 4 * (lane >> 5));
-      if (S < 8) {
+      if (S < STEPS) {
         if (m + 2 < 16) wf[(m + 2) % 3] = frag(m + 2);
         cur[m & 1] = mfma32(xf[m >> 1], wf[m % 3], m < 2 ? zero16 : cur[m & 1]);
       }
@@ -154,13 +166,12 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
       if (m == 7) {
         // half way: the next weights go to LDS (the buffer of step S + 1 was last read in step S - 1), the
         // ones after them are requested, and step S - 2's results leave
-        if (S >= 1 && S + 1 < 8) {
+        if (S >= 1 && S + 1 < STEPS) {
           wstore((S + 1) & 1 ? sW1 : sW0);
-          if (S + 2 < 8) wload(S + 2);
+          if (S + 2 < STEPS) wload(S + 2);
         }
         if (S >= 2) {
-          constexpr int SO = S >= 2 ? S - 2 : 0;
-          bf16_t* dst = (SO < 4 ? a.a_buf : a.b_buf) + (((SO >> 1) & 1) * 64 + (SO & 1) * 32) * a.plane + t.l0;
+          bf16_t* dst = results(S >= 2 ? S - 2 : 0);
 #pragma unroll
           for (int i = 0; i < 2; ++i)
             *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(dst + 16 * i * a.plane) + lane_out) = outv[i];
@@ -172,16 +183,20 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
   };
   step(std::integral_constant<int, 0>{}, accA, accB);
   step(std::integral_constant<int, 1>{}, accB, accA);
-  step(std::integral_constant<int, 2>{}, accA, accB);
-  step(std::integral_constant<int, 3>{}, accB, accA);
-  step(std::integral_constant<int, 4>{}, accA, accB);
-  step(std::integral_constant<int, 5>{}, accB, accA);
-  step(std::integral_constant<int, 6>{}, accA, accB);
-  step(std::integral_constant<int, 7>{}, accB, accA);
-  step(std::integral_constant<int, 8>{}, accA, accB);  // gating of step 7, results of step 6
+  if constexpr (STEPS > 2) {
+    step(std::integral_constant<int, 2>{}, accA, accB);
+    step(std::integral_constant<int, 3>{}, accB, accA);
+  }
+  if constexpr (STEPS > 4) {
+    step(std::integral_constant<int, 4>{}, accA, accB);
+    step(std::integral_constant<int, 5>{}, accB, accA);
+    step(std::integral_constant<int, 6>{}, accA, accB);
+    step(std::integral_constant<int, 7>{}, accB, accA);
+  }
+  step(std::integral_constant<int, STEPS>{}, accA, accB);  // gating of the last step, results of the one before
   {
-    // results of step 7
-    bf16_t* dst = a.b_buf + (64 + 32) * a.plane + t.l0;
+    // results of the last step
+    bf16_t* dst = results(STEPS - 1);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(dst + 16 * i * a.plane) + lane_out) =
@@ -764,10 +779,10 @@ __global__ __launch_bounds__(256, 2) void pair_cond_init_kernel(PairCondInitArgs
 }
 
 template <typename K, typename A>
-int launch_tiles(K kern, const A& a, int64_t positions, hipStream_t stream) {
+int launch_tiles(K kern, const A& a, int64_t positions, hipStream_t stream, int parts = 1) {
   const int64_t tiles = (positions + TM - 1) / TM;
   if (tiles <= 0 || tiles > 0x7fffffff) return AF3_ERR_BAD_ARG;
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(256), 0, stream, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)tiles, parts), dim3(256), 0, stream, a);
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
 
@@ -780,6 +795,21 @@ int launch_tiles(K kern, const A& a, int64_t positions, hipStream_t stream) {
     return a.io_f32 ? launch_tiles(KERN<float, false>, a, n_, s) : launch_tiles(KERN<bf16_t, false>, a, n_, s);   \
   } while (0)
 
+// A prologue's eight steps are dealt to four or two workgroups while all of them are on the chip at once (three fit a
+// CU: 768): the kernel then takes one workgroup's chain of steps and no second round.  Kernel alone, N = 64, 128: 11.4 ->
+// 6.9 us, 14.9 -> 12.0 us (four); N = 160, 212: 15.3 -> 14.6 us, 17.3 -> 16.2 us (two; four would take 16.3 and 19.8);
+// one past the line, N = 224, two would take 18.8 for 17.5 us.  64 channels have half the steps: N = 64, 128: 11.4 ->
+// 6.5 us, 14.9 -> 8.1 us, and 24 -> 16.4 us at N = 301.
+constexpr int64_t PROLOGUE_QUARTERS = 192, PROLOGUE_HALVES = 384;
+#define LAUNCH_PROLOGUE(STEPS, PARTS)                                                                              \
+  do {                                                                                                             \
+    const bool cross_ = tile_crosses(a.Np);                                                                        \
+    if (a.io_f32 && cross_) return launch_tiles(trimul_prologue_kernel<float, true, STEPS>, a, n, s, PARTS);       \
+    if (a.io_f32) return launch_tiles(trimul_prologue_kernel<float, false, STEPS>, a, n, s, PARTS);                \
+    return cross_ ? launch_tiles(trimul_prologue_kernel<bf16_t, true, STEPS>, a, n, s, PARTS)                      \
+                  : launch_tiles(trimul_prologue_kernel<bf16_t, false, STEPS>, a, n, s, PARTS);                    \
+  } while (0)
+
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
@@ -787,7 +817,13 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 int launch_trimul_prologue(const TriMulArgs& a, hipStream_t s) {
   if (a.N <= 0 || a.Np < a.N || (a.Np & 7) || a.plane < tri_plane(a.N) || !a.pair || !a.a_buf || !a.b_buf || !a.w_pg) return AF3_ERR_BAD_ARG;
   if (!aligned16(a.pair) || !aligned16(a.a_buf) || !aligned16(a.b_buf) || !aligned16(a.w_pg)) return AF3_ERR_BAD_ARG;
-  LAUNCH_TILES(trimul_prologue_kernel, tile_crosses(a.Np), (int64_t)a.N * a.Np);
+  // (the zeros of masked tiles and the sizes of the planes are the same in every split)
+  const int64_t n = (int64_t)a.N * a.Np, tiles = (n + TM - 1) / TM;
+  const bool narrow = a.valid_c <= 64;
+  if (tiles <= PROLOGUE_QUARTERS) LAUNCH_PROLOGUE(2, narrow ? 2 : 4);
+  if (narrow) LAUNCH_PROLOGUE(4, 1);
+  if (tiles <= PROLOGUE_HALVES) LAUNCH_PROLOGUE(4, 2);
+  LAUNCH_PROLOGUE(8, 1);
 }
 int launch_trimul_epilogue(const TriMulArgs& a, hipStream_t s) {
   if (a.N <= 0 || a.Np < a.N || (a.Np & 7) || a.plane < tri_plane(a.N) || !a.pair || !a.t_buf || !a.out || !a.w_gl || !a.w_out ||

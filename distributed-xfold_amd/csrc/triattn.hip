@@ -18,7 +18,8 @@ constexpr int H = 4, D = 32;
 // projections: LN -> q (scaled), k (position-major) and v (channel-major),
 // + pair-bias heads
 // ============================================================================
-template <typename TIO, bool CROSS>
+// SPLIT: a workgroup takes one of q (with the pair bias), k and v (blockIdx.y), where tiles are few.
+template <typename TIO, bool CROSS, bool SPLIT>
 __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a) {
   // 34.8 KB + 17.4 KB of LDS and at most 168 registers: three workgroups per CU.  The kernel is a chain of
   // short dependent phases (load, LayerNorm, MFMA, stage, store), so what it needs is company.
@@ -57,7 +58,9 @@ __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a)
       if (i < n) *reinterpret_cast<u32x4*>(sW + (idx >> 4) * LDX + (idx & 15) * 8) = wr[i];
     }
   };
-  wload(0);
+  const int part = SPLIT ? (int)blockIdx.y : 0;
+  const bool bias = a.n_bias > 0 && part == 0;
+  wload(2 * part);
   load_ln_tile<TIO>(x, t, a.ln_w, a.ln_b, sX, tid, a.skip_ln != 0, a.lw.inv_c, a.lw.pad);
   wstore(4);
   lds_barrier();
@@ -72,8 +75,9 @@ __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a)
     // The next weights are requested BEFORE this chunk's results are stored:
     // vector memory operations retire in order, so a load issued behind the
     // stores would make its consumer wait for the stores' round trip to HBM.
-    if (step < 5) wload(step + 1);
-    else if (a.n_bias > 0) wload_bias();
+    constexpr bool last = SPLIT ? pairt == 1 : step == 5;
+    if (!last) wload(step + 1);
+    else if (bias) wload_bias();
     {
       f32x16 acc[2];
       if (chunk == 2) {
@@ -113,8 +117,8 @@ __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a)
       }
     }
     lds_barrier();  // staging visible; every wave is done with sW
-    if (step < 5) wstore(4);
-    else if (a.n_bias > 0) wstore(2);
+    if (!last) wstore(4);
+    else if (bias) wstore(2);
     if (pairt == 1) {
       // both halves of the chunk are staged: 128 channels per position go out
       if (chunk == 2) {
@@ -146,16 +150,22 @@ __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a)
     }
     lds_barrier();
   };
-  do_step(std::integral_constant<int, 0>{});
-  do_step(std::integral_constant<int, 1>{});
-  do_step(std::integral_constant<int, 2>{});
-  do_step(std::integral_constant<int, 3>{});
-  do_step(std::integral_constant<int, 4>{});
-  do_step(std::integral_constant<int, 5>{});
+  if (!SPLIT || part == 0) {
+    do_step(std::integral_constant<int, 0>{});
+    do_step(std::integral_constant<int, 1>{});
+  }
+  if (!SPLIT || part == 1) {
+    do_step(std::integral_constant<int, 2>{});
+    do_step(std::integral_constant<int, 3>{});
+  }
+  if (!SPLIT || part == 2) {
+    do_step(std::integral_constant<int, 4>{});
+    do_step(std::integral_constant<int, 5>{});
+  }
 
   // pair-bias heads (T form: lane = pixel, rows = heads): bias[h][q][k] with
   // (q, k) the pixel's own (row, col) in the un-transposed pair tensor
-  if (a.n_bias > 0) {
+  if (bias) {
     f32x16 acc[1];
     mfma_chunk<true, 1>(xf, sW, lane, acc);
     if ((lane >> 5) == 0) {  // heads 0..3 are accumulator rows 0..3: registers 0..3 of the low half
@@ -179,6 +189,11 @@ __global__ __launch_bounds__(256, 3) void triattn_proj_kernel(TriAttnProjArgs a)
 
 bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
+// Tiles up to which q, k and v are three workgroups' work: all of them are on the chip at once (three fit a CU), and the
+// kernel takes two steps of a tile and its LayerNorm instead of six.  Kernel alone, N = 64, 128, 176: 10.6 -> 7.6 us,
+// 15.3 -> 13.3 us, 15.9 -> 13.7 us; past the line, N = 212, 17.9 instead of 16.3 us.
+constexpr int64_t SPLIT_TILES = 256;
+
 }  // namespace
 
 int launch_triattn_proj(const TriAttnProjArgs& a, hipStream_t stream) {
@@ -190,11 +205,16 @@ int launch_triattn_proj(const TriAttnProjArgs& a, hipStream_t stream) {
     return AF3_ERR_BAD_ARG;
   const int64_t tiles = ((int64_t)a.N * a.ldn + TM - 1) / TM;
   if (tiles > 0x7fffffff) return AF3_ERR_BAD_ARG;
-  const dim3 grid((unsigned)tiles), block(256);
-  const bool cross = tile_crosses(a.ldn);
-  if (a.io_f32 && cross) hipLaunchKernelGGL((triattn_proj_kernel<float, true>), grid, block, 0, stream, a);
-  else if (a.io_f32) hipLaunchKernelGGL((triattn_proj_kernel<float, false>), grid, block, 0, stream, a);
-  else if (cross) hipLaunchKernelGGL((triattn_proj_kernel<bf16_t, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((triattn_proj_kernel<bf16_t, false>), grid, block, 0, stream, a);
+  const bool cross = tile_crosses(a.ldn), split = tiles <= SPLIT_TILES;
+  const dim3 grid((unsigned)tiles, split ? 3 : 1), block(256);
+  auto launch = [&](auto split_c) {
+    constexpr bool S = decltype(split_c)::value;
+    if (a.io_f32 && cross) hipLaunchKernelGGL((triattn_proj_kernel<float, true, S>), grid, block, 0, stream, a);
+    else if (a.io_f32) hipLaunchKernelGGL((triattn_proj_kernel<float, false, S>), grid, block, 0, stream, a);
+    else if (cross) hipLaunchKernelGGL((triattn_proj_kernel<bf16_t, true, S>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((triattn_proj_kernel<bf16_t, false, S>), grid, block, 0, stream, a);
+  };
+  if (split) launch(std::true_type{});
+  else launch(std::false_type{});
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }

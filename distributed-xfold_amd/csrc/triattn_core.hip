@@ -665,9 +665,10 @@ int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream) {
   if (!al16(a.q) || !al16(a.k) || !al16(a.vt) || !al16(a.og) || !al16(a.bias)) return AF3_ERR_BAD_ARG;
   const int QT = (a.N + QW - 1) / QW;
   const int nkt = (a.N + KT - 1) / KT;
-  // Two rows per wave once that still leaves every CU several workgroups, one row below that
+  // Two rows per wave once that still leaves the CUs one and a half rounds of workgroups (two to a CU): N = 187
+  // 19.5 us (20.3 with one row), 256 25.4 (28.5), 301 48.5 (53.8), 340 56.3 (65.4), but 160 18.6 (18.2); one row below that
   // (and when the per-key mask codes of two rows would not fit the LDS share of a workgroup).
-  int R = (int64_t)((a.N + 1) / 2) * H * QT >= 2048 ? 2 : 1;
+  int R = (int64_t)((a.N + 1) / 2) * H * QT >= 700 ? 2 : 1;
   // static LDS: K / V buffers, small arrays; dynamic: the mask codes.  Two workgroups must fit a
   // CU's 160 KB.
   const size_t stat2 = 8 * TILE_BYTES + 512;
