@@ -73,7 +73,6 @@ class OuterProductMean(HipModule):
             rows = [(r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1) for r in range(32)]
             d["w_packed"] = d["w_out"].view(4, 32, 64, 2, 8)[:, rows].permute(0, 2, 3, 1, 4).contiguous()
             s = d["block"] = L.MsaBlockStruct()
-            s.epsilon = self.epsilon
             s.opm_ln_w, s.opm_ln_b, s.opm_w_lr, s.opm_w_out, s.opm_b_out = (
                 d[k].data_ptr() for k in ("ln_w", "ln_b", "w_lr", "w_packed", "b_out"))
         return d
@@ -86,6 +85,7 @@ class OuterProductMean(HipModule):
         co, cf = self.num_outer_channel, self.num_output_channel
         out = residual if residual is not None else torch.zeros((n, n, cf), dtype=torch.float32, device=msa.device)
         if self.native:
+            p["block"].epsilon = self.epsilon
             return ops.outer_product_mean(p["block"], msa.contiguous(), mask, out, True)
         m = mask.float()
         x = ops.layer_norm(msa.contiguous(), p["ln_w"], p["ln_b"])
@@ -147,7 +147,7 @@ class MSAAttention(HipModule):
             s = d["block"] = L.MsaBlockStruct()
             (s.ma_ln_w, s.ma_ln_b, s.ma_pn_w, s.ma_pn_b, s.ma_w_logits, s.ma_w_v, s.ma_w_g, s.ma_w_o) = (
                 d[k].data_ptr() for k in ("ln_w", "ln_b", "pn_w", "pn_b", "w_logits", "w_v", "w_g", "w_o"))
-            s.epsilon = 1.0
+            s.epsilon = 1.0      # (of a coverage that this operator does not use)
         return d
 
     @torch.no_grad()
@@ -213,12 +213,15 @@ class EvoformerBlock(HipModule):
         mods = (self.outer_product_mean, self.msa_attention1, self.msa_transition, *tm, *ta, self.pair_transition)
         packs = [m.packed() for m in mods]
         if self._native is not None and all(a is b for a, b in zip(self._native[1], packs)):
+            # (an attribute like any other, not a packed weight: as it is at the call)
+            self._native[0].epsilon = self.outer_product_mean.epsilon
             return self._native[0]
         s = L.MsaBlockStruct()
-        for src in (packs[1]["block"], packs[0]["block"]):      # (epsilon is the outer-product mean's)
+        for prefix, src in (("opm_", packs[0]["block"]), ("ma_", packs[1]["block"])):
             for name, _ in s._fields_:
-                if name != "pair" and getattr(src, name):
+                if name.startswith(prefix):
                     setattr(s, name, getattr(src, name))
+        s.epsilon = self.outer_product_mean.epsilon
         s.mt_ln_w, s.mt_ln_b, s.mt_w1, s.mt_w2 = (packs[2][k].data_ptr() for k in ("ln_w64", "ln_b64", "w1_64", "w2_64"))
         s.mt_hidden = packs[2]["w2_64"].shape[1]
         fill_pair_weights(s.pair, tm, ta, self.pair_transition, self.c_pair)
