@@ -234,7 +234,8 @@ class DiffusionHead(HipModule):
                 trunk_single_cond: torch.Tensor, trunk_pair_cond: torch.Tensor,
                 state: Optional[HeadState] = None, act_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
         """:171-227.  positions_noisy [(samples), N, A, 3]; noise_level a scalar
-        tensor; trunk_single_cond [N, 384] (the row of pre_conditioning's result
+        tensor, or one that broadcasts against the positions (a level per sample,
+        [samples, 1, 1, 1]); trunk_single_cond [N, 384] (the row of pre_conditioning's result
         for this noise level), trunk_pair_cond [N, N, 128].  Returns the
         denoised positions, fp32."""
         if state is None:
@@ -249,7 +250,12 @@ class DiffusionHead(HipModule):
         positions_noisy = positions_noisy.contiguous()
         am = batch.predicted_structure_info.atom_mask.float().contiguous()
         level = torch.as_tensor(noise_level, dtype=torch.float32, device=positions_noisy.device)
-        act = ops.positions(ops.POS_SCALE, positions_noisy, None, am, level)
+        one_level = level.numel() == 1
+        if one_level:
+            act = ops.positions(ops.POS_SCALE, positions_noisy, None, am, level)
+        else:       # the kernels read one level for all positions
+            am = am[None, ..., None] if batched else am[..., None]
+            act = positions_noisy * am / torch.sqrt(level ** 2 + SIGMA_DATA ** 2)
         enc = self.atom_cross_att_encoder(batch=batch, token_atoms_act=act, trunk_single_cond=embeddings["single"],
                                           trunk_pair_cond=trunk_pair_cond, conditioning=state.encoder,
                                           act_dtype=act_dtype)
@@ -267,7 +273,10 @@ class DiffusionHead(HipModule):
         else:
             act = ops.layer_norm(act, p["out_ln"])
         upd = self.atom_cross_att_decoder(batch=batch, token_act=act, enc=enc, transformer_cond=state.decoder_cond)
-        return ops.positions(ops.POS_BLEND, positions_noisy, upd.contiguous(), am, level)
+        if one_level:
+            return ops.positions(ops.POS_BLEND, positions_noisy, upd.contiguous(), am, level)
+        var = level ** 2 + SIGMA_DATA ** 2
+        return (SIGMA_DATA ** 2 / var * positions_noisy + level * SIGMA_DATA / torch.sqrt(var) * upd) * am
 
 
 class DiffusionSampler:

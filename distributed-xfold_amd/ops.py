@@ -300,6 +300,9 @@ POS_SCALE, POS_BLEND, POS_PLACE, POS_STEP = range(4)
 def positions(op, x, y, mask, level, next_level=None, factor=0.0):
     """The element-wise passes over atom positions [samples, N, A, 3] (af3_positions_forward); mask [N, A], `level` and
     `next_level` one-element device tensors, all fp32."""
+    for nm, t in (("level", level), ("next_level", next_level)):
+        if t is not None and t.numel() != 1:
+            raise ValueError(f"{nm}: expected one element, got {tuple(t.shape)}")
     lib = _L.load()
     _gpu(x, "x", torch.float32)
     for nm, t in (("mask", mask), ("level", level), ("next_level", next_level), ("y", y)):

@@ -376,3 +376,16 @@ def test_decoder_layout_kernels(gpu_pkg):
     print(f"  position update: max difference {err:.3e} of the largest value", flush=True)
     assert err <= 2e-3        # a bf16 rounding of a normalised value may fall the other way
     assert torch.all(got[:, ~present] == 0)
+
+
+def test_a_noise_level_per_sample(gpu_pkg):
+    """A level of shape [samples, 1, 1, 1] scales each sample with its own: what the same call gives it with that level
+    for all of them."""
+    _, batch, _, emb, pos, head = case(gpu_pkg, 12, 1, seed=77)
+    gb, ge, levels = batch.to(dev()), on_gpu(emb), torch.tensor([30.0, 0.5], device=dev())
+    sc, pc = head.pre_conditioning(gb, ge, levels, True)
+    noisy = pos.to(dev()) * levels[:, None, None, None]
+    got = head(noisy, levels[:, None, None, None], gb, ge, sc[0], pc)
+    for i in range(2):
+        assert torch.equal(got[i], head(noisy, levels[i], gb, ge, sc[0], pc)[i])
+    assert not torch.equal(got[1], head(noisy, levels[0], gb, ge, sc[0], pc)[1])

@@ -18,3 +18,10 @@ def test_outer_product_mean_epsilon_is_the_modules_at_the_call(pkg, monkeypatch)
         blk.outer_product_mean(msa, torch.ones(2, 3))
         blk(msa, pair, torch.ones(2, 3), torch.ones(3, 3))
         assert seen == [pytest.approx(eps)] * 2
+
+
+def test_position_kernels_take_one_level(pkg):
+    x, mask = torch.zeros(2, 3, 4, 3), torch.ones(3, 4)
+    for levels in ((torch.ones(2, 1, 1, 1), None), (torch.ones(()), torch.ones(2))):
+        with pytest.raises(ValueError, match="one element"):
+            pkg.ops.positions(pkg.ops.POS_STEP, x, x, mask, *levels)
