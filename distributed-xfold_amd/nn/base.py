@@ -93,19 +93,32 @@ class HipModule(nn.Module):
     loop (run_inference.py:197-218) binds these modules unchanged.
     """
 
+    _native = None      # the packed weights as the library's structures, where a module makes them
+
     def __init__(self):
         super().__init__()
         self._packed = None
+
+    # What is packed is derived from the parameters and is made again on demand: a copied or stored module is its
+    # parameters (the structures hold device addresses, which would mean nothing elsewhere).
+    def __getstate__(self):
+        state = dict(self.__dict__, _packed=None)
+        state.pop("_native", None)
+        return state
+
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        self._packed = self._native = None
 
     def invalidate(self):
         """Drop the packed weights of this module and of every HIP module below
         it, however deeply nested (blocks usually sit in an nn.ModuleList)."""
         for m in self.modules():
             if isinstance(m, HipModule):
-                m._packed = None
+                m._packed = m._native = None
 
     def _apply(self, fn, *a, **k):  # .to() / .cuda() move parameters: repack afterwards
-        self._packed = None
+        self._packed = self._native = None
         return super()._apply(fn, *a, **k)
 
     def load_state_dict(self, *a, **k):

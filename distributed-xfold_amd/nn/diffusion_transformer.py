@@ -15,26 +15,23 @@ from .. import ops
 from .base import HipModule, bf16, drop_mesh, f32, in_check_mode, pack_swiglu, pad_rows
 
 
-class BlockTable:
-    """The packed weights of a transformer's blocks as the array of structures the library takes; made again when
-    any of the modules has been packed again."""
-
-    def __init__(self):
-        self.packs, self.array = None, None
-
-    def get(self, blocks):
-        """`blocks`: (attention, transition) modules."""
-        mods = [m for att, tr in blocks for m in (att, att.adaptive_zero_init, tr, tr.adaptive_zero_init)]
-        packs = [m.packed() for m in mods]
-        if self.packs is None or not all(a is b for a, b in zip(self.packs, packs)):
-            self.packs, self.array = packs, (L.DiffusionBlockStruct * len(blocks))()
-            for i, s in enumerate(self.array):
-                att, att_out, tr, tr_out = packs[4 * i:4 * i + 4]
-                s.w_q = (att["w_qkvg"] if "w_qkvg" in att else att["w_qg"]).data_ptr()
-                s.w_kv = att["w_kv"].data_ptr() if "w_kv" in att else None
-                s.q_b, s.w_out = att["q_b"].data_ptr(), att_out["w"].data_ptr()
-                s.w_tr1, s.w_tr2 = tr["w1"].data_ptr(), tr_out["w"].data_ptr()
-        return self.array
+def block_table(owner: HipModule, blocks):
+    """The packed weights of a transformer's blocks, (attention, transition) modules, as the array of structures the
+    library takes; kept in `owner` and made again when any of the modules has been packed again."""
+    mods = [m for att, tr in blocks for m in (att, att.adaptive_zero_init, tr, tr.adaptive_zero_init)]
+    packs = [m.packed() for m in mods]
+    held = owner._native
+    if held is not None and len(held[1]) == len(packs) and all(a is b for a, b in zip(held[1], packs)):
+        return held[0]
+    table = (L.DiffusionBlockStruct * len(blocks))()
+    for i, s in enumerate(table):
+        att, att_out, tr, tr_out = packs[4 * i:4 * i + 4]
+        s.w_q = (att["w_qkvg"] if "w_qkvg" in att else att["w_qg"]).data_ptr()
+        s.w_kv = att["w_kv"].data_ptr() if "w_kv" in att else None
+        s.q_b, s.w_out = att["q_b"].data_ptr(), att_out["w"].data_ptr()
+        s.w_tr1, s.w_tr2 = tr["w1"].data_ptr(), tr_out["w"].data_ptr()
+    owner._native = (table, packs)
+    return table
 
 
 class AdaptiveLayerNorm(HipModule):
@@ -232,7 +229,6 @@ class DiffusionTransformer(HipModule):
         self.transition_block = nn.ModuleList(
             [DiffusionTransition(c_x=c_act, c_single_cond=c_single_cond, use_single_cond=True)
              for _ in range(num_blocks)])
-        self._table = BlockTable()
 
     def _pack(self):
         # Every block conditions on the same single_cond, so the 4 conditioning
@@ -297,7 +293,7 @@ class DiffusionTransformer(HipModule):
         if run < self.num_blocks:
             ss_all, gate_all = ss_all[:, :2 * run].contiguous(), gate_all[:, :2 * run].contiguous()
         ops.diffusion_transformer(
-            self._table.get(list(zip(self.self_attention, self.transition_block))[:run]), act if act.dim() == 3 else act[None],
+            block_table(self, list(zip(self.self_attention, self.transition_block))[:run]), act if act.dim() == 3 else act[None],
             mask, [logits[j] for logits in pair_logits for j in range(self.super_block_size)], ss_all, gate_all,
             self.num_head, self.transition_block[0].num_intermediate_factor * c)
         return act
@@ -387,7 +383,6 @@ class DiffusionCrossAttTransformer(HipModule):
         self.transition_block = nn.ModuleList(
             [DiffusionTransition(c_x=c_query, c_single_cond=c_single_cond, use_single_cond=True)
              for _ in range(num_blocks)])
-        self._table = BlockTable()
 
     def _pack(self):
         # The conditioning inputs are the same for every block: all adaptive
@@ -488,7 +483,7 @@ class DiffusionCrossAttTransformer(HipModule):
         logits, ss_q, ss_k, gate, key_rows = cond
         if key_rows is not None:
             return ops.atom_transformer(
-                self._table.get(list(zip(self.cross_attention, self.transition_block))), queries_act, key_rows, queries_mask,
+                block_table(self, list(zip(self.cross_attention, self.transition_block))), queries_act, key_rows, queries_mask,
                 keys_mask, logits, ss_q, ss_k, gate, self.num_head,
                 self.transition_block[0].num_intermediate_factor * self.c_query)
         for blk in range(self.num_blocks):

@@ -194,8 +194,6 @@ class EvoformerBlock(HipModule):
         self.pair_attention2 = GridSelfAttention(c_pair=c_pair, num_head=n_heads_pair, transpose=True)
         self.pair_transition = Transition(c_x=c_pair)
 
-        self._native = None
-
     def _pack(self):
         return {}
 

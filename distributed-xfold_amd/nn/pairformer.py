@@ -49,7 +49,6 @@ class PairformerBlock(HipModule):
         n_heads, c_pair, c_single, c_hidden_mul, n_heads_pair, num_intermediate_factor, with_single = vals[:7]
         self.n_heads, self.c_pair, self.c_single = n_heads, c_pair, c_single
         self.with_single, self.num_intermediate_factor = with_single, num_intermediate_factor
-        self._native = None
         self.triangle_multiplication_outgoing = TriangleMultiplication(c_pair=c_pair, _outgoing=True)
         self.triangle_multiplication_incoming = TriangleMultiplication(c_pair=c_pair, _outgoing=False)
         self.pair_attention1 = GridSelfAttention(c_pair=c_pair, num_head=n_heads_pair, transpose=False)

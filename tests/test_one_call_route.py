@@ -1,6 +1,11 @@
 """Where a run of modules goes to the library as one call: what that call is given, and which modules and arguments it
 must not be made for.  Host side only (the operator layer is replaced by recorders); no GPU."""
 
+import copy
+import gc
+import io
+import weakref
+
 import pytest
 import torch
 
@@ -25,3 +30,51 @@ def test_position_kernels_take_one_level(pkg):
     for levels in ((torch.ones(2, 1, 1, 1), None), (torch.ones(()), torch.ones(2))):
         with pytest.raises(ValueError, match="one element"):
             pkg.ops.positions(pkg.ops.POS_STEP, x, x, mask, *levels)
+
+
+def _small(nn, name):
+    """A small module of each class that keeps the library's structures, and how it is brought to make them."""
+    if name == "PairformerBlock":
+        return nn.PairformerBlock(), lambda m: m.native()
+    if name == "PairformerStack":
+        return nn.PairformerStack(num_blocks=1), lambda m: m.trunk_pairformer[0].native()
+    if name == "EvoformerBlock":
+        return nn.EvoformerBlock(), lambda m: m.native()
+    if name == "DiffusionTransformer":
+        kw = dict(c_act=48, num_head=2, num_blocks=2, super_block_size=1)
+        table = lambda m: nn.diffusion_transformer.block_table(m, list(zip(m.self_attention, m.transition_block)))
+        return nn.DiffusionTransformer(**kw), table
+    table = lambda m: nn.diffusion_transformer.block_table(m, list(zip(m.cross_attention, m.transition_block)))
+    return nn.DiffusionCrossAttTransformer(num_blocks=1), table
+
+
+NATIVE = ["PairformerBlock", "PairformerStack", "EvoformerBlock", "DiffusionTransformer", "DiffusionCrossAttTransformer"]
+
+
+@pytest.mark.parametrize("name", NATIVE)
+def test_packed_modules_can_be_copied_and_stored(pkg, name):
+    mod, make = _small(pkg.nn, name)
+    mod.load_hip_params()
+    make(mod)
+    stored = io.BytesIO()
+    torch.save(mod, stored)
+    stored.seek(0)
+    for other in (copy.deepcopy(mod), torch.load(stored, weights_only=False)):      # (what this test has just written)
+        assert all(torch.equal(a, b) for a, b in zip(mod.parameters(), other.parameters()))
+        own, others = bytes(make(mod)), bytes(make(other))
+        assert own != others          # the copy's structures point at weights of its own
+
+
+@pytest.mark.parametrize("name", NATIVE)
+def test_invalidate_lets_go_of_the_packed_weights(pkg, name):
+    mod, make = _small(pkg.nn, name)
+    held = []
+    make(mod)
+    for m in mod.modules():
+        if isinstance(m, pkg.nn.HipModule) and m._packed:
+            held += [weakref.ref(t) for t in m._packed.values() if isinstance(t, torch.Tensor)]
+    assert held
+    params = {id(p) for p in mod.parameters()}
+    mod.invalidate()
+    gc.collect()
+    assert all(r() is None or id(r()) in params for r in held)
