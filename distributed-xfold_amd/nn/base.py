@@ -82,6 +82,15 @@ def pack_swiglu(w1: torch.Tensor, block: int) -> torch.Tensor:
     return torch.cat([a, b], dim=1).reshape(2 * hidden, -1).contiguous()
 
 
+def as_written(m: nn.Module, cls: type) -> bool:
+    """Whether using `m` does what class `cls` says and nothing else: no subclass, no forward hook (its own or one for
+    all modules), no method replaced on the instance.  A run of modules that goes to the library as one call passes its
+    modules by, so it is made for such modules only."""
+    d, every = m.__dict__, nn.modules.module
+    return (type(m) is cls and not d["_forward_hooks"] and not d["_forward_pre_hooks"] and not every._global_forward_hooks
+            and not every._global_forward_pre_hooks and "forward" not in d and "run" not in d and "packed" not in d)
+
+
 class HipModule(nn.Module):
     """A module whose `forward` runs on the HIP kernels.
 

@@ -12,7 +12,23 @@ import torch.nn as nn
 from .. import check
 from .. import lib as L
 from .. import ops
-from .base import HipModule, bf16, drop_mesh, f32, in_check_mode, pack_swiglu, pad_rows
+from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pack_swiglu, pad_rows
+
+
+def plain_blocks(blocks, norms, attention: type, num_head: int) -> bool:
+    """Whether (attention, transition) modules are what one call of the library does for all of them alike.  `norms`:
+    the attention's conditioned norms, by name."""
+    if not blocks:
+        return False
+    hidden = blocks[0][1].num_intermediate_factor
+    for att, tr in blocks:
+        sub, t = att._modules, tr._modules
+        if not (as_written(att, attention) and att.num_head == num_head
+                and as_written(tr, DiffusionTransition) and tr.num_intermediate_factor == hidden
+                and all(as_written(sub[k], AdaptiveLayerNorm) for k in norms) and as_written(sub["adaptive_zero_init"], AdaLNZero)
+                and as_written(t["adaptive_layernorm"], AdaptiveLayerNorm) and as_written(t["adaptive_zero_init"], AdaLNZero)):
+            return False
+    return True
 
 
 def block_table(owner: HipModule, blocks):
@@ -290,12 +306,18 @@ class DiffusionTransformer(HipModule):
         run = self.num_super_blocks * self.super_block_size      # blocks beyond the last whole super-block never run
         if run == 0:
             return act
-        if run < self.num_blocks:
-            ss_all, gate_all = ss_all[:, :2 * run].contiguous(), gate_all[:, :2 * run].contiguous()
-        ops.diffusion_transformer(
-            block_table(self, list(zip(self.self_attention, self.transition_block))[:run]), act if act.dim() == 3 else act[None],
-            mask, [logits[j] for logits in pair_logits for j in range(self.super_block_size)], ss_all, gate_all,
-            self.num_head, self.transition_block[0].num_intermediate_factor * c)
+        blocks = list(zip(self.self_attention, self.transition_block))[:run]
+        logits = [pair_logits[i // self.super_block_size][i % self.super_block_size] for i in range(run)]
+        if plain_blocks(blocks, ("adaptive_layernorm",), SelfAttention, self.num_head):
+            if run < self.num_blocks:
+                ss_all, gate_all = ss_all[:, :2 * run].contiguous(), gate_all[:, :2 * run].contiguous()
+            ops.diffusion_transformer(block_table(self, blocks), act if act.dim() == 3 else act[None], mask, logits, ss_all,
+                                      gate_all, self.num_head, blocks[0][1].num_intermediate_factor * c)
+            return act
+        gate_all = gate_all.permute(1, 0, 2)                    # [module][row][c]: column slices, read in place
+        for i, (att, tr) in enumerate(blocks):
+            att.run(act, mask, logits[i], single_cond, residual=True, cond=(ss_all[:, 2 * i], gate_all[2 * i]))
+            tr.run(act, single_cond, residual=True, cond=(ss_all[:, 2 * i + 1], gate_all[2 * i + 1]))
         return act
 
 
@@ -349,6 +371,29 @@ class CrossAttention(HipModule):
         avg = avg.reshape(x_q.shape)
         return self.adaptive_zero_init.run(avg, single_cond_q, x_q.dtype, residual=x_q if residual else None,
                                            gate=gate)
+
+    def run_gathered(self, x_q, key_rows, mask_q, mask_k, pair_logits, single_cond_q, cond):
+        """`run(..., residual=True)` for keys that are query atoms: key k of
+        subset s is atom key_rows[s, k] of the flattened (subset, query) axis of
+        x_q (negative: a masked slot, whose gathered activation and conditioning
+        are zero, hence K = V = 0).  The keys' adaptive LayerNorm and K / V
+        projection then run once per atom, not once per (subset, key), and no
+        key tensor is gathered: cond = (scale_shift_q, scale_shift_k of the
+        ATOMS [S * Q, 2c], gate)."""
+        p = self.packed()
+        n_sub, n_q, c = x_q.shape[-3:]
+        ss_q, ss_k_atoms, gate = cond
+        xq = self.q_adaptive_layernorm(x_q, single_cond_q, scale_shift=ss_q)
+        xk = self.k_adaptive_layernorm(x_q, single_cond_q, scale_shift=ss_k_atoms)
+        pl = None
+        if pair_logits is not None:
+            if pair_logits.dim() == 5:                          # [S, H, K / 4, Q, 4]
+                pair_logits = pair_logits.transpose(-3, -2)
+            pl = pair_logits.reshape(-1, self.num_head, n_q, key_rows.shape[-1]).to(torch.float32).contiguous()
+        avg = ops.gathered_cross_attention(
+            xq.reshape(-1, n_q, c), xk.reshape(-1, n_sub * n_q, c), key_rows, pl, mask_q.reshape(-1, n_q),
+            mask_k.reshape(-1, key_rows.shape[-1]), p["w_qg"], p["w_kv"], p["q_b"], self.num_head)
+        return self.adaptive_zero_init.run(avg.reshape(x_q.shape), single_cond_q, x_q.dtype, residual=x_q, gate=gate)
 
     def forward(self, x_q, x_k, mask_q, mask_k, pair_logits=None, single_cond_q=None, single_cond_k=None):
         """x_q [(B,) S, Q, c], x_k [(B,) S, K, c], masks [(1,) S, Q] / [(1,) S, K],
@@ -481,16 +526,18 @@ class DiffusionCrossAttTransformer(HipModule):
         if cond is None:
             cond = self.conditioning(queries_single_cond, keys_single_cond, pair_cond)
         logits, ss_q, ss_k, gate, key_rows = cond
-        if key_rows is not None:
-            return ops.atom_transformer(
-                block_table(self, list(zip(self.cross_attention, self.transition_block))), queries_act, key_rows, queries_mask,
-                keys_mask, logits, ss_q, ss_k, gate, self.num_head,
-                self.transition_block[0].num_intermediate_factor * self.c_query)
-        for blk in range(self.num_blocks):
-            keys_act = self._gather(queries_to_keys, queries_act)
-            self.cross_attention[blk].run(queries_act, keys_act, queries_mask, keys_mask, logits[blk],
-                                          queries_single_cond, keys_single_cond, residual=True,
-                                          cond=(ss_q[:, 2 * blk], ss_k[:, blk], gate[2 * blk]))
-            self.transition_block[blk].run(queries_act, queries_single_cond, residual=True,
-                                           cond=(ss_q[:, 2 * blk + 1], gate[2 * blk + 1]))
+        blocks = list(zip(self.cross_attention, self.transition_block))
+        if key_rows is not None and plain_blocks(blocks, ("q_adaptive_layernorm", "k_adaptive_layernorm"), CrossAttention,
+                                                 self.num_head):
+            return ops.atom_transformer(block_table(self, blocks), queries_act, key_rows, queries_mask, keys_mask, logits, ss_q,
+                                        ss_k, gate, self.num_head, blocks[0][1].num_intermediate_factor * self.c_query)
+        for i, (att, tr) in enumerate(blocks):
+            cond = ss_q[:, 2 * i], ss_k[:, i], gate[2 * i]
+            if key_rows is not None:
+                att.run_gathered(queries_act, key_rows, queries_mask, keys_mask, logits[i], queries_single_cond, cond=cond)
+            else:
+                keys_act = self._gather(queries_to_keys, queries_act)
+                att.run(queries_act, keys_act, queries_mask, keys_mask, logits[i], queries_single_cond, keys_single_cond,
+                        residual=True, cond=cond)
+            tr.run(queries_act, queries_single_cond, residual=True, cond=(ss_q[:, 2 * i + 1], gate[2 * i + 1]))
         return queries_act

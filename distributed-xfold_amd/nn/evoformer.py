@@ -31,8 +31,8 @@ import torch.nn.functional as F
 from .. import check, ops
 from .. import lib as L
 from .attention import GridSelfAttention
-from .base import HipModule, bf16, drop_mesh, f32, in_check_mode, pad_rows
-from .pairformer import fill_pair_weights
+from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pad_rows
+from .pairformer import fill_pair_weights, plain_pair_track
 from .primitives import Transition
 from .triangle_multiplication import TriangleMultiplication
 
@@ -197,18 +197,24 @@ class EvoformerBlock(HipModule):
     def _pack(self):
         return {}
 
+    def _tracks(self):
+        return ((self.outer_product_mean, self.msa_attention1, self.msa_transition),
+                ((self.triangle_multiplication_outgoing, self.triangle_multiplication_incoming),
+                 (self.pair_attention1, self.pair_attention2), self.pair_transition))
+
     @property
     def one_call(self) -> bool:
         """Whether the whole block runs as one call of the library (`native`)."""
-        return (self.outer_product_mean.native and self.msa_attention1.native and self.msa_transition.narrow
-                and self.pair_attention1.fused)
+        (opm, att, transition), pair_track = self._tracks()
+        return (as_written(opm, OuterProductMean) and opm.native and as_written(att, MSAAttention) and att.native
+                and as_written(transition, Transition) and transition.narrow
+                and plain_pair_track(*pair_track, self.c_pair) and self.pair_attention1.fused)
 
     def native(self) -> "L.MsaBlockStruct":
         """The packed weights of the block's modules as the library's structure; made again when any of them has been
         packed again."""
-        tm = (self.triangle_multiplication_outgoing, self.triangle_multiplication_incoming)
-        ta = (self.pair_attention1, self.pair_attention2)
-        mods = (self.outer_product_mean, self.msa_attention1, self.msa_transition, *tm, *ta, self.pair_transition)
+        msa_track, (tm, ta, transition) = self._tracks()
+        mods = (*msa_track, *tm, *ta, transition)
         packs = [m.packed() for m in mods]
         if self._native is not None and all(a is b for a, b in zip(self._native[1], packs)):
             # (an attribute like any other, not a packed weight: as it is at the call)
@@ -222,7 +228,7 @@ class EvoformerBlock(HipModule):
         s.epsilon = self.outer_product_mean.epsilon
         s.mt_ln_w, s.mt_ln_b, s.mt_w1, s.mt_w2 = (packs[2][k].data_ptr() for k in ("ln_w64", "ln_b64", "w1_64", "w2_64"))
         s.mt_hidden = packs[2]["w2_64"].shape[1]
-        fill_pair_weights(s.pair, tm, ta, self.pair_transition, self.c_pair)
+        fill_pair_weights(s.pair, tm, ta, transition, self.c_pair)
         self._native = (s, packs)
         return s
 
@@ -260,7 +266,7 @@ def evoformer_loop(blocks, msa, pair, msa_mask, pair_mask):
     """Run Evoformer blocks one after the other (d_alphafold3.py:228-231), in one call where they allow it."""
     blocks = list(blocks)
     if (not in_check_mode() and pair.is_cuda and len(blocks) > 1 and msa.is_contiguous() and pair.is_contiguous()
-            and all(type(b) is EvoformerBlock and b.one_call and
+            and all(as_written(b, EvoformerBlock) and b.one_call and
                     b.outer_product_mean.epsilon == blocks[0].outer_product_mean.epsilon for b in blocks)):
         ops.evoformer_stack([b.native() for b in blocks], msa, pair, msa_mask, pair_mask)
         return msa, pair

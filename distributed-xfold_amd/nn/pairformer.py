@@ -10,10 +10,20 @@ import torch.nn as nn
 from .. import check, ops
 from .. import lib as L
 from .attention import GridSelfAttention
-from .base import HipModule, bf16, drop_mesh, f32, in_check_mode, pad_channels, pad_rows
-from .diffusion_transformer import SelfAttention
+from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pad_channels, pad_rows
+from .diffusion_transformer import AdaLNZero, AdaptiveLayerNorm, SelfAttention
 from .primitives import Transition
 from .triangle_multiplication import TriangleMultiplication
+
+
+def plain_pair_track(tm, ta, transition, c_pair) -> bool:
+    """Whether the five pair operators are what one call of the library does: the triangle multiplications (outgoing,
+    incoming), the triangle attentions (starting, ending node) and the transition, all on `c_pair` channels."""
+    return (all(as_written(m, TriangleMultiplication) and m.c_pair == c_pair for m in tm)
+            and all(as_written(m, GridSelfAttention) and m.c_pair == c_pair for m in ta)
+            and as_written(transition, Transition) and transition.c_x == c_pair
+            and tm[0]._outgoing and not tm[1]._outgoing and not ta[0].transpose and ta[1].transpose
+            and ta[0].num_head == ta[1].num_head)
 
 
 def fill_pair_weights(s, tm, ta, transition, c_pair) -> None:
@@ -67,19 +77,31 @@ class PairformerBlock(HipModule):
         return dict(ln_w=f32(self.single_pair_logits_norm.weight), ln_b=f32(self.single_pair_logits_norm.bias),
                     w_logits=pad_rows(bf16(self.single_pair_logits_projection.weight), 32))
 
+    def _pair_track(self):
+        return ((self.triangle_multiplication_outgoing, self.triangle_multiplication_incoming),
+                (self.pair_attention1, self.pair_attention2), self.pair_transition)
+
     @property
     def one_call(self) -> bool:
         """Whether the whole block runs as one call of the library (`native`): the fused pair operators, and a
         single track wide enough for the unfused transition."""
-        return ((self.pair_attention1.fused or (self.pair_attention1.padded and not self.with_single))
-                and (not self.with_single or self.c_single > 128))
+        track = self._pair_track()
+        if not plain_pair_track(*track, self.c_pair):
+            return False
+        att = track[1][0]
+        if not self.with_single:
+            return att.fused or att.padded
+        sa, st, c = self.single_attention_, self.single_transition, self.c_single
+        return (att.fused and c > 128 and as_written(sa, SelfAttention) and sa.c_x == c and sa.num_head == self.n_heads
+                and as_written(sa.adaptive_layernorm, AdaptiveLayerNorm) and not sa.adaptive_layernorm.use_single_cond
+                and as_written(sa.adaptive_zero_init, AdaLNZero) and not sa.adaptive_zero_init.use_single_cond
+                and as_written(st, Transition) and st.c_x == c)
 
     def native(self) -> "L.PairformerBlockStruct":
         """The packed weights of the block's modules as the library's structure; made again when any of them has
         been packed again."""
-        tm = (self.triangle_multiplication_outgoing, self.triangle_multiplication_incoming)
-        ta = (self.pair_attention1, self.pair_attention2)
-        mods = (self, *tm, *ta, self.pair_transition)
+        tm, ta, transition = self._pair_track()
+        mods = (self, *tm, *ta, transition)
         if self.with_single:
             sa, st = self.single_attention_, self.single_transition
             mods += (sa, sa.adaptive_layernorm, sa.adaptive_zero_init, st)
@@ -88,7 +110,7 @@ class PairformerBlock(HipModule):
             return self._native[0]
         by = dict(zip(mods, packs))
         s = L.PairformerBlockStruct()
-        fill_pair_weights(s, tm, ta, self.pair_transition, self.c_pair)
+        fill_pair_weights(s, tm, ta, transition, self.c_pair)
         s.with_single = int(self.with_single)
         if self.with_single:
             p = by[self]
@@ -179,7 +201,7 @@ def pairformer_loop(blocks, pair, pair_mask, single, seq_mask, overlap_single: b
         return pair, single
     side = _side_stream(pair.device)
     blocks = list(blocks)
-    if blocks and all(type(b) is PairformerBlock and b.one_call and b.with_single and b.n_heads == blocks[0].n_heads
+    if blocks and all(as_written(b, PairformerBlock) and b.one_call and b.with_single and b.n_heads == blocks[0].n_heads
                       and b.c_single == blocks[0].c_single for b in blocks):
         if not (pair.is_contiguous() and single.is_contiguous()):
             raise ValueError("pair and single must be contiguous (they are updated in place)")

@@ -1,0 +1,105 @@
+"""Runs of modules that go to the library as one call, against the same modules one by one: what a user has put between
+them (forward hooks, a sub-module of another class) has its effect, and the results are the ones of the single call."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def on_gpu(mod, std=0.05):
+    g = torch.Generator().manual_seed(1)
+    for p in mod.parameters():
+        p.data.normal_(0.0, std, generator=g)
+    return mod.to("cuda:0")
+
+
+def counter(mod, seen):
+    return mod.register_forward_hook(lambda m, args, out: seen.append(m))
+
+
+def trunk_inputs(n=37):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    mask = (torch.arange(n, device="cuda") < n - 3).float()
+    return rnd(n, n, 128), (mask[:, None] * mask[None, :]).contiguous(), rnd(n, 384), mask
+
+
+def test_hooks_in_a_pairformer_stack(gpu_pkg):
+    stack = on_gpu(gpu_pkg.nn.PairformerStack(num_blocks=3))
+    pair, pm, single, sm = trunk_inputs()
+    run = lambda: stack(pair.clone(), pm, single.clone(), sm)
+    want, blocks, seen = run(), stack.trunk_pairformer, []
+    for where, count in ((blocks[1], 1), (blocks[2].single_attention_.adaptive_layernorm, 1), (None, 3)):
+        seen.clear()
+        if where is None:
+            every = lambda m, args, out: seen.append(m) if isinstance(m, gpu_pkg.nn.PairformerBlock) else None
+            hook = torch.nn.modules.module.register_module_forward_hook(every)
+        else:
+            hook = counter(where, seen)
+        got = run()
+        hook.remove()
+        assert len(seen) == count
+        # (module by module the single track's products sum in another order: bf16 roundings of an update of order one)
+        assert torch.equal(got[0], want[0]) and float((got[1] - want[1]).norm() / want[1].norm()) < 1e-2
+    assert all(torch.equal(a, b) for a, b in zip(run(), want))
+
+
+def test_a_sub_module_of_another_class(gpu_pkg):
+    class Doubled(gpu_pkg.nn.Transition):
+        def run(self, x, residual):
+            return super().run(super().run(x, residual), residual)
+
+    blk = on_gpu(gpu_pkg.nn.PairformerBlock(with_single=False))
+    pair, pm, _, _ = trunk_inputs()
+    want = blk.pair_transition.run(blk(pair.clone(), pm), True)
+    other = Doubled(c_x=128)
+    other.load_state_dict(blk.pair_transition.state_dict())
+    blk.pair_transition = other.to("cuda:0")
+    assert torch.equal(blk(pair.clone(), pm), want)
+
+
+def test_hooks_in_a_run_of_evoformer_blocks(gpu_pkg):
+    blocks, seen = [on_gpu(gpu_pkg.nn.EvoformerBlock()) for _ in range(2)], []
+    pair, pm, _, sm = trunk_inputs(19)
+    msa = torch.randn(5, 19, 64, generator=torch.Generator(device="cuda").manual_seed(0), device="cuda")
+    run = lambda: gpu_pkg.nn.evoformer.evoformer_loop(blocks, msa.clone(), pair.clone(), sm.expand(5, -1).contiguous(), pm)
+    want = run()
+    hook = counter(blocks[1], seen)
+    got = run()
+    hook.remove()
+    assert len(seen) == 1 and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("n", [24, 21])       # pair logits in quads of keys, and in rows
+def test_hooks_in_a_diffusion_transformer(gpu_pkg, n):
+    mod, seen = on_gpu(gpu_pkg.nn.DiffusionTransformer(num_blocks=4, super_block_size=2)), []
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    act, cond, pair = rnd(2, n, 768).bfloat16(), rnd(n, 384), rnd(n, n, 128)
+    mask = (torch.arange(n, device="cuda") < n - 3).float()
+    run = lambda: mod(act.clone(), mask, cond, pair)
+    want = run()
+    hook = counter(mod.self_attention[1].adaptive_layernorm, seen)
+    got = run()
+    hook.remove()
+    assert len(seen) == 1 and torch.equal(got, want)
+
+
+def test_hooks_in_an_atom_transformer(gpu_pkg):
+    mod, seen = on_gpu(gpu_pkg.nn.DiffusionCrossAttTransformer()), []
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    s, q, k = 3, 32, 128
+    idx = torch.randint(0, s * q, (s, k), generator=g, device="cuda")
+    gather = (idx, torch.rand(s, k, generator=g, device="cuda") > 0.2)
+    act, mq, mk = rnd(2, s, q, 128).bfloat16(), torch.ones(s, q, device="cuda"), gather[1].float()
+    sq = rnd(s, q, 128)
+    sk = sq.view(s * q, 128)[idx] * gather[1][..., None]
+    cond = mod.conditioning(sq, sk, rnd(s, q, k, 16), keys_are_query_atoms=gather)
+    run = lambda: mod(act.clone(), mq, gather, mk, sq, sk, None, cond=cond)
+    want = run()
+    hook = counter(mod.cross_attention[1].k_adaptive_layernorm, seen)
+    got = run()
+    hook.remove()
+    assert len(seen) == 1 and torch.equal(got, want)

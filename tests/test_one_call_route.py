@@ -78,3 +78,48 @@ def test_invalidate_lets_go_of_the_packed_weights(pkg, name):
     mod.invalidate()
     gc.collect()
     assert all(r() is None or id(r()) in params for r in held)
+
+
+def _hooked(m):
+    m.register_forward_hook(lambda *a: None)
+
+
+def _replaced(m):
+    m.run = lambda *a, **k: None
+
+
+def _another_class(m):
+    m.__class__ = type("Derived", (type(m),), {})
+
+
+@pytest.mark.parametrize("change", [_hooked, _replaced, _another_class])
+def test_one_call_is_not_made_past_changed_modules(pkg, change):
+    for cls, names in ((pkg.nn.PairformerBlock, ("pair_attention2", "triangle_multiplication_incoming", "pair_transition",
+                                                 "single_transition", "single_attention_", "single_attention_.adaptive_layernorm")),
+                       (pkg.nn.EvoformerBlock, ("outer_product_mean", "msa_attention1", "msa_transition", "pair_transition"))):
+        assert cls().one_call
+        for name in names:
+            blk = cls()
+            change(blk.get_submodule(name))
+            assert not blk.one_call, name
+    swapped = pkg.nn.PairformerBlock()
+    swapped.pair_attention1.transpose = True
+    assert not swapped.one_call
+
+
+@pytest.mark.parametrize("change", [_hooked, _replaced, _another_class])
+def test_transformers_are_not_run_past_changed_modules(pkg, change):
+    dt = pkg.nn.diffusion_transformer
+
+    def pairs(mod, att):
+        return list(zip(getattr(mod, att), mod.transition_block))
+    for make, att, cls, norms, heads in (
+            (lambda: dt.DiffusionTransformer(c_act=48, num_head=2, num_blocks=2, super_block_size=1), "self_attention",
+             dt.SelfAttention, ("adaptive_layernorm",), 2),
+            (lambda: dt.DiffusionCrossAttTransformer(num_blocks=2), "cross_attention", dt.CrossAttention,
+             ("q_adaptive_layernorm", "k_adaptive_layernorm"), 4)):
+        assert dt.plain_blocks(pairs(make(), att), norms, cls, heads)
+        for name in [f"{att}.1", "transition_block.1", "transition_block.0.adaptive_zero_init"] + [f"{att}.0.{k}" for k in norms]:
+            mod = make()
+            change(mod.get_submodule(name))
+            assert not dt.plain_blocks(pairs(mod, att), norms, cls, heads), name
