@@ -288,7 +288,7 @@ class DiffusionTransformer(HipModule):
     def forward(self, act: torch.Tensor, mask: torch.Tensor, single_cond: torch.Tensor,
                 pair_cond: torch.Tensor, pair_logits=None) -> torch.Tensor:
         """act [B, N, c_act] (updated in place, as the reference's `act +=`),
-        mask [N], single_cond [N, c_single_cond], pair_cond [N, N, c_pair_cond]."""
+        mask [N] or [B, N], single_cond [N, c_single_cond], pair_cond [N, N, c_pair_cond]."""
         if in_check_mode():
             return check.diffusion_transformer(self, act, mask, single_cond, pair_cond)
         p = self.packed()
@@ -308,7 +308,8 @@ class DiffusionTransformer(HipModule):
             return act
         blocks = list(zip(self.self_attention, self.transition_block))[:run]
         logits = [pair_logits[i // self.super_block_size][i % self.super_block_size] for i in range(run)]
-        if plain_blocks(blocks, ("adaptive_layernorm",), SelfAttention, self.num_head):
+        # (the single call knows one key mask for all samples)
+        if plain_blocks(blocks, ("adaptive_layernorm",), SelfAttention, self.num_head) and (mask is None or mask.dim() == 1):
             if run < self.num_blocks:
                 ss_all, gate_all = ss_all[:, :2 * run].contiguous(), gate_all[:, :2 * run].contiguous()
             ops.diffusion_transformer(block_table(self, blocks), act if act.dim() == 3 else act[None], mask, logits, ss_all,

@@ -71,14 +71,18 @@ def test_hooks_in_a_run_of_evoformer_blocks(gpu_pkg):
     assert len(seen) == 1 and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
-@pytest.mark.parametrize("n", [24, 21])       # pair logits in quads of keys, and in rows
-def test_hooks_in_a_diffusion_transformer(gpu_pkg, n):
-    mod, seen = on_gpu(gpu_pkg.nn.DiffusionTransformer(num_blocks=4, super_block_size=2)), []
+def diffusion_case(pkg, n):
+    mod = on_gpu(pkg.nn.DiffusionTransformer(num_blocks=4, super_block_size=2))
     g = torch.Generator(device="cuda").manual_seed(n)
     rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
     act, cond, pair = rnd(2, n, 768).bfloat16(), rnd(n, 384), rnd(n, n, 128)
     mask = (torch.arange(n, device="cuda") < n - 3).float()
-    run = lambda: mod(act.clone(), mask, cond, pair)
+    return mod, mask, lambda mask=mask, **k: mod(act.clone(), mask, cond, pair, **k)
+
+
+@pytest.mark.parametrize("n", [24, 21])       # pair logits in quads of keys, and in rows
+def test_hooks_in_a_diffusion_transformer(gpu_pkg, n):
+    (mod, _, run), seen = diffusion_case(gpu_pkg, n), []
     want = run()
     hook = counter(mod.self_attention[1].adaptive_layernorm, seen)
     got = run()
@@ -103,3 +107,11 @@ def test_hooks_in_an_atom_transformer(gpu_pkg):
     got = run()
     hook.remove()
     assert len(seen) == 1 and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n", [24, 21])
+def test_a_key_mask_per_sample(gpu_pkg, n):
+    _, mask, run = diffusion_case(gpu_pkg, n)
+    other = mask.roll(5)
+    got = run(torch.stack([mask, other]))
+    assert torch.equal(got[0], run()[0]) and torch.equal(got[1], run(other)[1]) and not torch.equal(got[1], run()[1])
