@@ -307,9 +307,11 @@ class DiffusionTransformer(HipModule):
         if run == 0:
             return act
         blocks = list(zip(self.self_attention, self.transition_block))[:run]
-        logits = [pair_logits[i // self.super_block_size][i % self.super_block_size] for i in range(run)]
-        # (the single call knows one key mask for all samples)
-        if plain_blocks(blocks, ("adaptive_layernorm",), SelfAttention, self.num_head) and (mask is None or mask.dim() == 1):
+        logits = [pair_logits[i // self.super_block_size][i % self.super_block_size].to(torch.float32).contiguous()
+                  for i in range(run)]
+        # (the single call knows one key mask for all samples and one order of the logits for all blocks)
+        if (plain_blocks(blocks, ("adaptive_layernorm",), SelfAttention, self.num_head) and (mask is None or mask.dim() == 1)
+                and all(t.shape == logits[0].shape for t in logits)):
             if run < self.num_blocks:
                 ss_all, gate_all = ss_all[:, :2 * run].contiguous(), gate_all[:, :2 * run].contiguous()
             ops.diffusion_transformer(block_table(self, blocks), act if act.dim() == 3 else act[None], mask, logits, ss_all,
@@ -530,8 +532,9 @@ class DiffusionCrossAttTransformer(HipModule):
         blocks = list(zip(self.cross_attention, self.transition_block))
         if key_rows is not None and plain_blocks(blocks, ("q_adaptive_layernorm", "k_adaptive_layernorm"), CrossAttention,
                                                  self.num_head):
-            return ops.atom_transformer(block_table(self, blocks), queries_act, key_rows, queries_mask, keys_mask, logits, ss_q,
-                                        ss_k, gate, self.num_head, blocks[0][1].num_intermediate_factor * self.c_query)
+            return ops.atom_transformer(block_table(self, blocks), queries_act, key_rows, queries_mask, keys_mask,
+                                        logits.to(torch.float32).contiguous(), ss_q, ss_k, gate, self.num_head,
+                                        blocks[0][1].num_intermediate_factor * self.c_query)
         for i, (att, tr) in enumerate(blocks):
             cond = ss_q[:, 2 * i], ss_k[:, i], gate[2 * i]
             if key_rows is not None:

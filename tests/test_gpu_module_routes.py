@@ -115,3 +115,19 @@ def test_a_key_mask_per_sample(gpu_pkg, n):
     other = mask.roll(5)
     got = run(torch.stack([mask, other]))
     assert torch.equal(got[0], run()[0]) and torch.equal(got[1], run(other)[1]) and not torch.equal(got[1], run()[1])
+
+
+@pytest.mark.parametrize("n", [24, 21])
+def test_pair_logits_of_another_type_or_order(gpu_pkg, n):
+    """Logits that a caller has computed and kept: bf16, a strided view, rows for one super-block and quads for the other."""
+    mod, _, run = diffusion_case(gpu_pkg, n)
+    pair = torch.randn(n, n, 128, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda")
+    logits = mod.pair_logits(pair)
+    want = run(pair_logits=logits)
+    strided = [torch.stack([t, -t], dim=-1)[..., 0] for t in logits]
+    assert not strided[0][0].is_contiguous() and torch.equal(run(pair_logits=strided), want)
+    half = [t.bfloat16() for t in logits]
+    assert torch.equal(run(pair_logits=half), run(pair_logits=[t.float() for t in half]))
+    if n % 4 == 0:
+        rows = logits[0].transpose(-3, -2).reshape(*logits[0].shape[:2], n, n)
+        assert torch.equal(run(pair_logits=[rows, logits[1]]), want)
