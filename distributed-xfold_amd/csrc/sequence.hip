@@ -188,6 +188,9 @@ int af3_evoformer_stack_forward(const af3_msa_block* const* blocks, int num_bloc
   if ((msa_dtype != AF3_F32 && msa_dtype != AF3_BF16) || (pair_dtype != AF3_F32 && pair_dtype != AF3_BF16)) return AF3_ERR_BAD_ARG;
   for (int i = 0; i < num_blocks; ++i)
     if (!blocks[i] || blocks[i]->epsilon != blocks[0]->epsilon) return AF3_ERR_BAD_ARG;
+  if (workspace_bytes < af3_msa_workspace_bytes(rows, n)) return AF3_ERR_WORKSPACE;  // (in place: before the first launch)
+  for (int i = 0; i < num_blocks; ++i)
+    if (pair_workspace_bytes < af3_pairformer_stack_workspace_bytes(n, blocks[i]->pair.num_head_pair)) return AF3_ERR_WORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   Carver w(workspace, workspace_bytes);
   float *inv = static_cast<float*>(w.take((size_t)n * n * 4)), *live = static_cast<float*>(w.take((size_t)n * 4));
@@ -233,9 +236,15 @@ int af3_pairformer_stack_forward(
     void* workspace, size_t workspace_bytes, void* single_workspace, size_t single_workspace_bytes, af3_stream_t stream,
     af3_stream_t single_stream, int join) {
   if (!blocks || num_blocks <= 0 || !pair || n <= 0) return AF3_ERR_BAD_ARG;
-  for (int i = 0; i < num_blocks; ++i)
-    if (!blocks[i] || (blocks[i]->with_single && (!single || !logits || blocks[i]->num_head != blocks[0]->num_head)))
-      return AF3_ERR_BAD_ARG;
+  // all of it before the first launch: the blocks work in place
+  for (int i = 0; i < num_blocks; ++i) {
+    if (!blocks[i]) return AF3_ERR_BAD_ARG;
+    const af3_pairformer_block& b = *blocks[i];
+    if (workspace_bytes < af3_pairformer_stack_workspace_bytes(n, b.num_head_pair)) return AF3_ERR_WORKSPACE;
+    if (!b.with_single) continue;
+    if (!single || !logits || b.num_head != blocks[0]->num_head || b.c_single != blocks[0]->c_single) return AF3_ERR_BAD_ARG;
+    if (single_workspace_bytes < af3_pairformer_single_workspace_bytes(n, b.c_single, b.single_hidden)) return AF3_ERR_WORKSPACE;
+  }
   hipStream_t main_s = static_cast<hipStream_t>(stream);
   hipStream_t side_s = single_stream ? static_cast<hipStream_t>(single_stream) : main_s;
   const bool two = side_s != main_s;

@@ -210,7 +210,7 @@ def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incomi
     io = _dt(pair)
     maskf = _mask_f32(pair_mask, (n, n), "mask")
     mask_in = _mask_f32(pair_mask_incoming, (n, n), "mask")
-    ws = _ws(lib.af3_pairformer_stack_workspace_bytes(n, blocks[0].num_head_pair), dev)
+    ws = _ws(max(lib.af3_pairformer_stack_workspace_bytes(n, b.num_head_pair) for b in blocks), dev)
     seqf = logits = sws = None
     single_dt = 0
     if blocks[0].with_single:
@@ -219,7 +219,8 @@ def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incomi
         single_dt = _dt(single)
         seqf = _mask_f32(seq_mask, (n,), "key_mask")
         logits = torch.empty((min(len(blocks), 2), b.num_head, n, (n + 3) // 4 * 4), dtype=torch.float32, device=dev)
-        sws = _ws(lib.af3_pairformer_single_workspace_bytes(n, b.c_single, b.single_hidden), dev, single_stream)
+        sws = _ws(lib.af3_pairformer_single_workspace_bytes(n, b.c_single, max(x.single_hidden for x in blocks)), dev,
+                  single_stream)
         if single_stream is not None and not join:
             for t in (logits, seqf):
                 if t is not None:
@@ -379,7 +380,7 @@ def evoformer_stack(blocks, msa, pair, msa_mask, pair_mask):
     _gpu(pair, "pair", shape=(n, n, 128))
     pmf = _mask_f32(pair_mask, (n, n), "pair_mask")
     need = lib.af3_msa_workspace_bytes(rows, n)
-    pws = lib.af3_pairformer_stack_workspace_bytes(n, blocks[0].pair.num_head_pair)
+    pws = max(lib.af3_pairformer_stack_workspace_bytes(n, b.pair.num_head_pair) for b in blocks)
     split = (need + 255) // 256 * 256
     ws = _ws(split + pws, msa.device)
     ptrs = (ctypes.c_void_p * len(blocks))(*[ctypes.addressof(b) for b in blocks])

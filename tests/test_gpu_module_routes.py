@@ -131,3 +131,16 @@ def test_pair_logits_of_another_type_or_order(gpu_pkg, n):
     if n % 4 == 0:
         rows = logits[0].transpose(-3, -2).reshape(*logits[0].shape[:2], n, n)
         assert torch.equal(run(pair_logits=[rows, logits[1]]), want)
+
+
+def test_a_later_block_with_a_wider_single_transition(gpu_pkg):
+    """The scratch is one for all blocks of a run."""
+    n, blocks = 37, [on_gpu(gpu_pkg.nn.PairformerBlock()) for _ in range(3)]
+    blocks[1].single_transition = on_gpu(gpu_pkg.nn.Transition(c_x=384, num_intermediate_factor=9))
+    pair, pm, single, sm = trunk_inputs(n)
+    one = pair.clone(), single.clone()
+    for blk in blocks:
+        one = blk(one[0], pm, one[1], sm)
+    gpu_pkg.ops.release_workspaces()
+    two = gpu_pkg.nn.pairformer_loop(blocks, pair.clone(), pm, single.clone(), sm)
+    assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])

@@ -2,6 +2,7 @@
 must not be made for.  Host side only (the operator layer is replaced by recorders); no GPU."""
 
 import copy
+import ctypes
 import gc
 import io
 import weakref
@@ -123,3 +124,29 @@ def test_transformers_are_not_run_past_changed_modules(pkg, change):
             mod = make()
             change(mod.get_submodule(name))
             assert not dt.plain_blocks(pairs(mod, att), norms, cls, heads), name
+
+
+def test_scratch_is_checked_for_every_block_before_anything_is_launched(pkg):
+    lib, some = pkg.lib.load(), 1 << 20      # (an address that is not null: nothing is to touch it)
+    n, narrow, wide = 16, pkg.lib.PairformerBlockStruct(), pkg.lib.PairformerBlockStruct()
+    for b, hidden in ((narrow, 1536), (wide, 3456)):
+        b.valid_channels, b.num_head_pair, b.with_single, b.num_head, b.c_single, b.single_hidden = 128, 4, 1, 16, 384, hidden
+    pair_ws = lib.af3_pairformer_stack_workspace_bytes(n, 4)
+    need = lib.af3_pairformer_single_workspace_bytes(n, 384, 1536)
+    assert need < lib.af3_pairformer_single_workspace_bytes(n, 384, 3456)
+
+    def call(blocks, wsb, swsb):
+        ptrs = (ctypes.c_void_p * len(blocks))(*[ctypes.addressof(b) for b in blocks])
+        return lib.af3_pairformer_stack_forward(ptrs, len(blocks), some, 0, None, None, some, 0, None, n, some, some, wsb, some,
+                                                swsb, None, None, 1)
+    assert call([narrow, wide], pair_ws, need) == -2
+    assert call([narrow], pair_ws, need - 1) == -2 and call([narrow], pair_ws - 1, need) == -2
+    wide.c_single = 256
+    assert call([narrow, wide], pair_ws, 1 << 30) == -1
+
+    m = pkg.lib.MsaBlockStruct()
+    m.pair.num_head_pair = 4
+    ptrs = (ctypes.c_void_p * 1)(ctypes.addressof(m))
+    msa_ws = lib.af3_msa_workspace_bytes(8, n)
+    for a, b in ((msa_ws - 1, pair_ws), (msa_ws, pair_ws - 1)):
+        assert lib.af3_evoformer_stack_forward(ptrs, 1, some, 0, some, some, 0, None, 8, n, some, a, some, b, None) == -2
