@@ -42,6 +42,12 @@ def _pad_last(x: torch.Tensor, multiple: int = 8) -> torch.Tensor:
     return x if k % multiple == 0 else F.pad(x, (0, (-k) % multiple))
 
 
+def _takes(msa, mask) -> bool:
+    """Whether the MSA track's own kernels take these: their range of sizes, and one mask value per position (the general
+    kernels also take masks that broadcast)."""
+    return ops.msa_in_range(*msa.shape[:2]) and mask.shape == msa.shape[:2]
+
+
 class OuterProductMean(HipModule):
     """nn/d_primitives.py:42-70."""
 
@@ -84,7 +90,7 @@ class OuterProductMean(HipModule):
         a, n, _ = msa.shape
         co, cf = self.num_outer_channel, self.num_output_channel
         out = residual if residual is not None else torch.zeros((n, n, cf), dtype=torch.float32, device=msa.device)
-        if self.native:
+        if self.native and _takes(msa, mask):
             p["block"].epsilon = self.epsilon
             return ops.outer_product_mean(p["block"], msa.contiguous(), mask, out, True)
         m = mask.float()
@@ -153,9 +159,9 @@ class MSAAttention(HipModule):
     @torch.no_grad()
     def run(self, msa, msa_mask, pair, residual: bool):
         p = self.packed()
-        if self.native:
-            return ops.msa_attention(p["block"], msa.contiguous(), msa_mask, pair.contiguous(), residual)
         a, n, c = msa.shape
+        if self.native and _takes(msa, msa_mask):
+            return ops.msa_attention(p["block"], msa.contiguous(), msa_mask, pair.contiguous(), residual)
         h, d = self.num_head, self.value_dim
         x = ops.layer_norm(msa.contiguous(), p["ln_w"], p["ln_b"])
         logits = ops.pair_logits(pair.contiguous(), p["pn_w"], p["pn_b"], p["w_logits"], h)     # [h, q, k] fp32
@@ -248,7 +254,7 @@ class EvoformerBlock(HipModule):
             return msa, pair
         if not (pair.is_contiguous() and msa.is_contiguous()):
             raise ValueError("msa and pair must be contiguous (they are updated in place)")
-        if self.one_call:
+        if self.one_call and _takes(msa, msa_mask):
             ops.evoformer_stack([self.native()], msa, pair, msa_mask, pair_mask)
             return msa, pair
         self.outer_product_mean.run(msa, msa_mask, residual=pair)
@@ -266,7 +272,7 @@ def evoformer_loop(blocks, msa, pair, msa_mask, pair_mask):
     """Run Evoformer blocks one after the other (d_alphafold3.py:228-231), in one call where they allow it."""
     blocks = list(blocks)
     if (not in_check_mode() and pair.is_cuda and len(blocks) > 1 and msa.is_contiguous() and pair.is_contiguous()
-            and all(as_written(b, EvoformerBlock) and b.one_call and
+            and _takes(msa, msa_mask) and all(as_written(b, EvoformerBlock) and b.one_call and
                     b.outer_product_mean.epsilon == blocks[0].outer_product_mean.epsilon for b in blocks)):
         ops.evoformer_stack([b.native() for b in blocks], msa, pair, msa_mask, pair_mask)
         return msa, pair

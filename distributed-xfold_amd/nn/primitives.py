@@ -73,7 +73,7 @@ class Transition(HipModule):
                                  valid_channels=self.c_x)
 
     def run(self, x, residual: bool):
-        if self.narrow:
+        if self.narrow and x.is_contiguous() and x.numel() <= 64 << 30:      # (the kernel's range)
             p = self.packed()
             return ops.transition64(x, p["ln_w64"], p["ln_b64"], p["w1_64"], p["w2_64"], residual)
         if self.padded:

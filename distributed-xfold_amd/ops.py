@@ -321,6 +321,11 @@ def positions(op, x, y, mask, level, next_level=None, factor=0.0):
     return out
 
 
+def msa_in_range(rows, n) -> bool:
+    """Whether the MSA track's own kernels take `rows` MSA rows of `n` tokens (their indices are 32 bits wide)."""
+    return _L.load().af3_msa_workspace_bytes(rows, n) > 0
+
+
 def _msa_inputs(msa, msa_mask):
     _gpu(msa, "msa")
     if msa.dim() != 3 or msa.shape[2] != 64:

@@ -144,3 +144,12 @@ def test_a_later_block_with_a_wider_single_transition(gpu_pkg):
     gpu_pkg.ops.release_workspaces()
     two = gpu_pkg.nn.pairformer_loop(blocks, pair.clone(), pm, single.clone(), sm)
     assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])
+
+
+def test_an_msa_mask_that_broadcasts(gpu_pkg):
+    """One mask row for all MSA rows: what the attention takes from the mask is its maximum over the rows."""
+    att = on_gpu(gpu_pkg.nn.MSAAttention())
+    pair, _, _, mask = trunk_inputs(19)
+    msa = torch.randn(5, 19, 64, generator=torch.Generator(device="cuda").manual_seed(0), device="cuda")
+    want, got = att(msa, mask.expand(5, -1).contiguous(), pair), att(msa, mask[None], pair)
+    assert float((got - want).norm() / want.norm()) < 1e-2      # (bf16 products and sums in another order)

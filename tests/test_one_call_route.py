@@ -150,3 +150,39 @@ def test_scratch_is_checked_for_every_block_before_anything_is_launched(pkg):
     msa_ws = lib.af3_msa_workspace_bytes(8, n)
     for a, b in ((msa_ws - 1, pair_ws), (msa_ws, pair_ws - 1)):
         assert lib.af3_evoformer_stack_forward(ptrs, 1, some, 0, some, some, 0, None, 8, n, some, a, some, b, None) == -2
+
+
+class _General(Exception):
+    """The general kernels were called."""
+
+
+@pytest.mark.parametrize("rows,n,mask_rows,taken", [(2, 8192, 2, True), (2, 8193, 2, False), ((1 << 24) + 1, 64, (1 << 24) + 1, False),
+                                                    (4, 6, 1, False)])
+def test_msa_sizes_and_masks_beyond_the_msa_kernels_go_to_the_general_ones(pkg, monkeypatch, rows, n, mask_rows, taken):
+    opm, att, blk = pkg.nn.OuterProductMean(), pkg.nn.MSAAttention(), pkg.nn.EvoformerBlock()
+    for m in (opm.packed, att.packed, blk.native):
+        m()
+    zero = torch.zeros(1)                    # (tensors without memory of their own, and nothing that would give them any)
+    msa, pair, mask = zero.expand(rows, n, 64), zero.expand(n, n, 128), zero.expand(mask_rows, n)
+    for name in ("contiguous", "float"):
+        monkeypatch.setattr(torch.Tensor, name, lambda t: t)
+    monkeypatch.setattr(torch.Tensor, "is_contiguous", lambda t: True)
+
+    def general(*a, **k):
+        raise _General
+    monkeypatch.setattr(pkg.ops, "layer_norm", general)
+    for name in ("outer_product_mean", "msa_attention", "evoformer_stack"):
+        monkeypatch.setattr(pkg.ops, name, lambda *a, **k: "own")
+    for call in (lambda: opm.run(msa, mask, residual=pair), lambda: att.run(msa, mask, pair, True),
+                 lambda: blk(msa, pair, mask, zero.expand(n, n))):
+        if taken:
+            call()
+        else:
+            with pytest.raises(_General):
+                call()
+
+
+def test_a_strided_tensor_goes_to_the_padded_transition(pkg, monkeypatch):
+    monkeypatch.setattr(pkg.ops, "transition128", lambda x, *a, **k: x + 1)
+    x = torch.zeros(64, 6).t()
+    assert pkg.nn.Transition(c_x=64).run(x, True) is x and bool((x == 1).all())
