@@ -26,6 +26,12 @@ def plain_pair_track(tm, ta, transition, c_pair) -> bool:
             and ta[0].num_head == ta[1].num_head)
 
 
+def one_sequence(single, seq_mask) -> bool:
+    """Whether the single track is the one sequence that one call of the library knows ([N, c], mask [N]); a batch of
+    them on one pair tensor runs module by module."""
+    return single.dim() == 2 and (seq_mask is None or seq_mask.dim() == 1)
+
+
 def fill_pair_weights(s, tm, ta, transition, c_pair) -> None:
     """The pair operators' packed weights into an af3_pairformer_block: triangle multiplications (outgoing, incoming),
     triangle attentions (starting, ending node), pair transition."""
@@ -128,7 +134,7 @@ class PairformerBlock(HipModule):
     def forward(self, pair: torch.Tensor, pair_mask: torch.Tensor, single: Optional[torch.Tensor] = None,
                 seq_mask: Optional[torch.Tensor] = None, head: int = 0,
                 single_stream: Optional["torch.cuda.Stream"] = None):
-        """pair [N, N, c_pair], pair_mask [N, N], single [N, c_single], seq_mask [N].
+        """pair [N, N, c_pair], pair_mask [N, N], single [(B,) N, c_single], seq_mask [(B,) N].
 
         `single_stream` (not in the reference): run the update of `single` (attention and
         transition, a chain of small kernels that leave most of the GPU idle) on that
@@ -141,11 +147,11 @@ class PairformerBlock(HipModule):
             raise ValueError("pair must be contiguous (it is updated in place)")
         if self.with_single and not single.is_contiguous():
             raise ValueError("single must be contiguous (it is updated in place)")
-        if self.one_call and self.with_single:
+        if self.with_single and one_sequence(single, seq_mask) and self.one_call:
             ops.pairformer_stack([self.native()], pair, pair_mask, single, seq_mask, single_stream=single_stream,
                                  join=single_stream is None)
             return pair, single
-        if self.one_call:
+        if not self.with_single and self.one_call:
             # (fewer than 128 channels, the template embedding of nn/d_template.py:198-201: the five operators run on
             # the 128-channel kernels over one zero-padded copy of the tensor, which stays padded in between)
             x = pad_channels(pair) if self.c_pair < 128 else pair
@@ -201,8 +207,9 @@ def pairformer_loop(blocks, pair, pair_mask, single, seq_mask, overlap_single: b
         return pair, single
     side = _side_stream(pair.device)
     blocks = list(blocks)
-    if blocks and all(as_written(b, PairformerBlock) and b.one_call and b.with_single and b.n_heads == blocks[0].n_heads
-                      and b.c_single == blocks[0].c_single for b in blocks):
+    if blocks and one_sequence(single, seq_mask) and all(
+            as_written(b, PairformerBlock) and b.one_call and b.with_single and b.n_heads == blocks[0].n_heads
+            and b.c_single == blocks[0].c_single for b in blocks):
         if not (pair.is_contiguous() and single.is_contiguous()):
             raise ValueError("pair and single must be contiguous (they are updated in place)")
         ops.pairformer_stack([b.native() for b in blocks], pair, pair_mask, single, seq_mask, single_stream=side)

@@ -153,3 +153,14 @@ def test_an_msa_mask_that_broadcasts(gpu_pkg):
     msa = torch.randn(5, 19, 64, generator=torch.Generator(device="cuda").manual_seed(0), device="cuda")
     want, got = att(msa, mask.expand(5, -1).contiguous(), pair), att(msa, mask[None], pair)
     assert float((got - want).norm() / want.norm()) < 1e-2      # (bf16 products and sums in another order)
+
+
+def test_a_batch_of_single_representations(gpu_pkg):
+    stack = on_gpu(gpu_pkg.nn.PairformerStack(num_blocks=2))
+    pair, pm, single, sm = trunk_inputs()
+    both = torch.stack([single, single.roll(3, 0)])
+    got = stack(pair.clone(), pm, both.clone(), torch.stack([sm, sm]))
+    for i in range(2):
+        want = stack(pair.clone(), pm, both[i].clone(), sm)
+        # (a single sequence's products may sum in another order)
+        assert torch.equal(got[0], want[0]) and float((got[1][i] - want[1]).norm() / want[1].norm()) < 1e-2
