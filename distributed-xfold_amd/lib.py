@@ -17,6 +17,7 @@ _vp, _i, _i64, _sz, _f = C.c_void_p, C.c_int, C.c_int64, C.c_size_t, C.c_float
 
 class PairformerBlockStruct(C.Structure):
     """af3_pairformer_block."""
+    device = None       # where what the fields point at lives (host side only, as in the other structures)
     _fields_ = (
         [(k, _vp * 2) for k in ("tm_ln_in_w", "tm_ln_in_b", "tm_ln_c_w", "tm_ln_c_b", "tm_w_proj_gate", "tm_w_out",
                                 "tm_w_gating", "ta_ln_w", "ta_ln_b", "ta_w_bias", "ta_w_qkvg", "ta_w_out")]
@@ -28,6 +29,7 @@ class PairformerBlockStruct(C.Structure):
 
 class MsaBlockStruct(C.Structure):
     """af3_msa_block."""
+    device = None
     _fields_ = (
         [(k, _vp) for k in ("opm_ln_w", "opm_ln_b", "opm_w_lr", "opm_w_out", "opm_b_out", "ma_ln_w", "ma_ln_b", "ma_pn_w",
                             "ma_pn_b", "ma_w_logits", "ma_w_v", "ma_w_g", "ma_w_o", "mt_ln_w", "mt_ln_b", "mt_w1", "mt_w2")]
@@ -36,6 +38,7 @@ class MsaBlockStruct(C.Structure):
 
 class DiffusionBlockStruct(C.Structure):
     """af3_diffusion_block."""
+    device = None
     _fields_ = [(k, _vp) for k in ("w_q", "w_kv", "q_b", "w_out", "w_tr1", "w_tr2")]
 
 

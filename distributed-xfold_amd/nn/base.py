@@ -82,6 +82,24 @@ def pack_swiglu(w1: torch.Tensor, block: int) -> torch.Tensor:
     return torch.cat([a, b], dim=1).reshape(2 * hidden, -1).contiguous()
 
 
+def point(s, *fields) -> None:
+    """Set address fields of a library structure from packed weights: (field or (field, index), tensor, shape), vectors
+    fp32 and matrices bf16.  The structures carry neither sizes nor types, so what the operator layer checks of every
+    tensor is checked here: type, shape, contiguity and one device for all, which is kept as `s.device` for the operator
+    layer to compare with the activations'."""
+    for name, t, shape in fields:
+        dtype = torch.float32 if len(shape) == 1 else torch.bfloat16
+        if tuple(t.shape) != shape or t.dtype != dtype or not t.is_contiguous():
+            raise ValueError(f"{name}: expected a contiguous {dtype} weight {shape}, got {t.dtype} {tuple(t.shape)}")
+        if s.device not in (None, t.device):
+            raise ValueError(f"{name}: on {t.device}, other weights of the block on {s.device}")
+        s.device = t.device
+        if isinstance(name, tuple):
+            getattr(s, name[0])[name[1]] = t.data_ptr()
+        else:
+            setattr(s, name, t.data_ptr())
+
+
 def as_written(m: nn.Module, cls: type) -> bool:
     """Whether using `m` does what class `cls` says and nothing else: no subclass, no forward hook (its own or one for
     all modules), no method replaced on the instance.  A run of modules that goes to the library as one call passes its

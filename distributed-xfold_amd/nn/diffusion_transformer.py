@@ -12,7 +12,7 @@ import torch.nn as nn
 from .. import check
 from .. import lib as L
 from .. import ops
-from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pack_swiglu, pad_rows
+from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pack_swiglu, pad_rows, point
 
 
 def plain_blocks(blocks, norms, attention: type, num_head: int) -> bool:
@@ -20,32 +20,38 @@ def plain_blocks(blocks, norms, attention: type, num_head: int) -> bool:
     the attention's conditioned norms, by name."""
     if not blocks:
         return False
-    hidden = blocks[0][1].num_intermediate_factor
+    factor = blocks[0][1].num_intermediate_factor
     for att, tr in blocks:
         sub, t = att._modules, tr._modules
         if not (as_written(att, attention) and att.num_head == num_head
-                and as_written(tr, DiffusionTransition) and tr.num_intermediate_factor == hidden
+                and as_written(tr, DiffusionTransition) and tr.num_intermediate_factor == factor
                 and all(as_written(sub[k], AdaptiveLayerNorm) for k in norms) and as_written(sub["adaptive_zero_init"], AdaLNZero)
                 and as_written(t["adaptive_layernorm"], AdaptiveLayerNorm) and as_written(t["adaptive_zero_init"], AdaLNZero)):
             return False
     return True
 
 
-def block_table(owner: HipModule, blocks):
-    """The packed weights of a transformer's blocks, (attention, transition) modules, as the array of structures the
-    library takes; kept in `owner` and made again when any of the modules has been packed again."""
+def block_table(owner: HipModule, blocks, c: int):
+    """The packed weights of a transformer's blocks, (attention, transition) modules on `c` channels, as the array of
+    structures the library takes, with the `device` they live on and their transitions' `hidden` width; kept in `owner`
+    and made again when any of the modules has been packed again."""
     mods = [m for att, tr in blocks for m in (att, att.adaptive_zero_init, tr, tr.adaptive_zero_init)]
     packs = [m.packed() for m in mods]
     held = owner._native
     if held is not None and len(held[1]) == len(packs) and all(a is b for a, b in zip(held[1], packs)):
         return held[0]
     table = (L.DiffusionBlockStruct * len(blocks))()
+    table.device, table.hidden = None, packs[3]["w"].shape[1]
     for i, s in enumerate(table):
         att, att_out, tr, tr_out = packs[4 * i:4 * i + 4]
-        s.w_q = (att["w_qkvg"] if "w_qkvg" in att else att["w_qg"]).data_ptr()
-        s.w_kv = att["w_kv"].data_ptr() if "w_kv" in att else None
-        s.q_b, s.w_out = att["q_b"].data_ptr(), att_out["w"].data_ptr()
-        s.w_tr1, s.w_tr2 = tr["w1"].data_ptr(), tr_out["w"].data_ptr()
+        s.device = table.device
+        if "w_qkvg" in att:
+            point(s, ("w_q", att["w_qkvg"], (4 * c, c)))
+        else:
+            point(s, ("w_q", att["w_qg"], (2 * c, c)), ("w_kv", att["w_kv"], (2 * c, c)))
+        point(s, ("q_b", att["q_b"], (c,)), ("w_out", att_out["w"], (c, c)), ("w_tr1", tr["w1"], (2 * table.hidden, c)),
+              ("w_tr2", tr_out["w"], (c, table.hidden)))
+        table.device = s.device
     owner._native = (table, packs)
     return table
 
@@ -314,8 +320,9 @@ class DiffusionTransformer(HipModule):
                 and all(t.shape == logits[0].shape for t in logits)):
             if run < self.num_blocks:
                 ss_all, gate_all = ss_all[:, :2 * run].contiguous(), gate_all[:, :2 * run].contiguous()
-            ops.diffusion_transformer(block_table(self, blocks), act if act.dim() == 3 else act[None], mask, logits, ss_all,
-                                      gate_all, self.num_head, blocks[0][1].num_intermediate_factor * c)
+            table = block_table(self, blocks, c)
+            ops.diffusion_transformer(table, act if act.dim() == 3 else act[None], mask, logits, ss_all, gate_all, self.num_head,
+                                      table.hidden)
             return act
         gate_all = gate_all.permute(1, 0, 2)                    # [module][row][c]: column slices, read in place
         for i, (att, tr) in enumerate(blocks):
@@ -532,9 +539,9 @@ class DiffusionCrossAttTransformer(HipModule):
         blocks = list(zip(self.cross_attention, self.transition_block))
         if key_rows is not None and plain_blocks(blocks, ("q_adaptive_layernorm", "k_adaptive_layernorm"), CrossAttention,
                                                  self.num_head):
-            return ops.atom_transformer(block_table(self, blocks), queries_act, key_rows, queries_mask, keys_mask,
-                                        logits.to(torch.float32).contiguous(), ss_q, ss_k, gate, self.num_head,
-                                        blocks[0][1].num_intermediate_factor * self.c_query)
+            table = block_table(self, blocks, self.c_query)
+            return ops.atom_transformer(table, queries_act, key_rows, queries_mask, keys_mask,
+                                        logits.to(torch.float32).contiguous(), ss_q, ss_k, gate, self.num_head, table.hidden)
         for i, (att, tr) in enumerate(blocks):
             cond = ss_q[:, 2 * i], ss_k[:, i], gate[2 * i]
             if key_rows is not None:

@@ -31,7 +31,7 @@ import torch.nn.functional as F
 from .. import check, ops
 from .. import lib as L
 from .attention import GridSelfAttention
-from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pad_rows
+from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pad_rows, point
 from .pairformer import fill_pair_weights, plain_pair_track
 from .primitives import Transition
 from .triangle_multiplication import TriangleMultiplication
@@ -79,8 +79,8 @@ class OuterProductMean(HipModule):
             rows = [(r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1) for r in range(32)]
             d["w_packed"] = d["w_out"].view(4, 32, 64, 2, 8)[:, rows].permute(0, 2, 3, 1, 4).contiguous()
             s = d["block"] = L.MsaBlockStruct()
-            s.opm_ln_w, s.opm_ln_b, s.opm_w_lr, s.opm_w_out, s.opm_b_out = (
-                d[k].data_ptr() for k in ("ln_w", "ln_b", "w_lr", "w_packed", "b_out"))
+            point(s, ("opm_ln_w", d["ln_w"], (64,)), ("opm_ln_b", d["ln_b"], (64,)), ("opm_w_lr", d["w_lr"], (64, 64)),
+                  ("opm_w_out", d["w_packed"], (4, 64, 2, 32, 8)), ("opm_b_out", d["b_out"], (128,)))
         return d
 
     @torch.no_grad()
@@ -151,8 +151,9 @@ class MSAAttention(HipModule):
                     w_g=bf16(self.gating_query.weight), w_o=bf16(self.output_projection.weight))
         if self.native:
             s = d["block"] = L.MsaBlockStruct()
-            (s.ma_ln_w, s.ma_ln_b, s.ma_pn_w, s.ma_pn_b, s.ma_w_logits, s.ma_w_v, s.ma_w_g, s.ma_w_o) = (
-                d[k].data_ptr() for k in ("ln_w", "ln_b", "pn_w", "pn_b", "w_logits", "w_v", "w_g", "w_o"))
+            point(s, ("ma_ln_w", d["ln_w"], (64,)), ("ma_ln_b", d["ln_b"], (64,)), ("ma_pn_w", d["pn_w"], (128,)),
+                  ("ma_pn_b", d["pn_b"], (128,)), ("ma_w_logits", d["w_logits"], (32, 128)),
+                  *((f"ma_{k}", d[k], (64, 64)) for k in ("w_v", "w_g", "w_o")))
             s.epsilon = 1.0      # (of a coverage that this operator does not use)
         return d
 
@@ -228,13 +229,21 @@ class EvoformerBlock(HipModule):
             return self._native[0]
         s = L.MsaBlockStruct()
         for prefix, src in (("opm_", packs[0]["block"]), ("ma_", packs[1]["block"])):
+            if s.device not in (None, src.device):
+                raise ValueError(f"weights of the block on {s.device} and on {src.device}")
+            s.device = src.device
             for name, _ in s._fields_:
                 if name.startswith(prefix):
                     setattr(s, name, getattr(src, name))
         s.epsilon = self.outer_product_mean.epsilon
-        s.mt_ln_w, s.mt_ln_b, s.mt_w1, s.mt_w2 = (packs[2][k].data_ptr() for k in ("ln_w64", "ln_b64", "w1_64", "w2_64"))
-        s.mt_hidden = packs[2]["w2_64"].shape[1]
-        fill_pair_weights(s.pair, tm, ta, transition, self.c_pair)
+        t = packs[2]
+        s.mt_hidden = t["w2_64"].shape[1]
+        point(s, ("mt_ln_w", t["ln_w64"], (64,)), ("mt_ln_b", t["ln_b64"], (64,)), ("mt_w1", t["w1_64"], (2 * s.mt_hidden, 64)),
+              ("mt_w2", t["w2_64"], (64, s.mt_hidden)))
+        p = L.PairformerBlockStruct()
+        p.device = s.device
+        fill_pair_weights(p, tm, ta, transition, self.c_pair)
+        s.pair = p
         self._native = (s, packs)
         return s
 

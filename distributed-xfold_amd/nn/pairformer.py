@@ -10,7 +10,7 @@ import torch.nn as nn
 from .. import check, ops
 from .. import lib as L
 from .attention import GridSelfAttention
-from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pad_channels, pad_rows
+from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pad_channels, pad_rows, point
 from .diffusion_transformer import AdaLNZero, AdaptiveLayerNorm, SelfAttention
 from .primitives import Transition
 from .triangle_multiplication import TriangleMultiplication
@@ -35,16 +35,20 @@ def one_sequence(single, seq_mask) -> bool:
 def fill_pair_weights(s, tm, ta, transition, c_pair) -> None:
     """The pair operators' packed weights into an af3_pairformer_block: triangle multiplications (outgoing, incoming),
     triangle attentions (starting, ending node), pair transition."""
+    vec, mat = (128,), (128, 128)
     for d in (0, 1):
         p, q = tm[d].packed(), ta[d].packed()
-        for name, t in (("tm_ln_in_w", p["ln_in_w"]), ("tm_ln_in_b", p["ln_in_b"]), ("tm_ln_c_w", p["ln_c_w"]),
-                        ("tm_ln_c_b", p["ln_c_b"]), ("tm_w_proj_gate", p["w_proj_gate"]), ("tm_w_out", p["w_out"]),
-                        ("tm_w_gating", p["w_gl"]), ("ta_ln_w", q["ln_w"]), ("ta_ln_b", q["ln_b"]),
-                        ("ta_w_bias", q["w_bias"]), ("ta_w_qkvg", q["w_qkvg"]), ("ta_w_out", q["w_out"])):
-            getattr(s, name)[d] = t.data_ptr()
+        point(s, (("tm_ln_in_w", d), p["ln_in_w"], vec), (("tm_ln_in_b", d), p["ln_in_b"], vec),
+              (("tm_ln_c_w", d), p["ln_c_w"], vec), (("tm_ln_c_b", d), p["ln_c_b"], vec),
+              (("tm_w_proj_gate", d), p["w_proj_gate"], (4, 128, 128)), (("tm_w_out", d), p["w_out"], mat),
+              (("tm_w_gating", d), p["w_gl"], mat), (("ta_ln_w", d), q["ln_w"], vec), (("ta_ln_b", d), q["ln_b"], vec),
+              (("ta_w_bias", d), q["w_bias"], (32, 128)), (("ta_w_qkvg", d), q["w_qkvg"], (4, 128, 128)),
+              (("ta_w_out", d), q["w_out"], mat))
     p = transition.packed()
-    s.pt_ln_w, s.pt_ln_b, s.pt_w1, s.pt_w2 = (p[k].data_ptr() for k in ("ln_w", "ln_b", "w1", "w2"))
-    s.valid_channels, s.num_head_pair, s.pair_hidden = c_pair, ta[0].num_head, p["w2"].shape[1]
+    hidden = p["w2"].shape[1]
+    point(s, ("pt_ln_w", p["ln_w"], vec), ("pt_ln_b", p["ln_b"], vec), ("pt_w1", p["w1"], (hidden // 64, 128, 128)),
+          ("pt_w2", p["w2"], (128, hidden)))
+    s.valid_channels, s.num_head_pair, s.pair_hidden = c_pair, ta[0].num_head, hidden
 
 
 class PairformerBlock(HipModule):
@@ -119,15 +123,14 @@ class PairformerBlock(HipModule):
         fill_pair_weights(s, tm, ta, transition, self.c_pair)
         s.with_single = int(self.with_single)
         if self.with_single:
-            p = by[self]
-            s.sl_ln_w, s.sl_ln_b, s.sl_w = (p[k].data_ptr() for k in ("ln_w", "ln_b", "w_logits"))
-            p = by[sa.adaptive_layernorm]
-            s.sa_ln_w, s.sa_ln_b = p["ln_w"].data_ptr(), p["ln_b"].data_ptr()
-            s.sa_w_qkvg, s.sa_q_b = by[sa]["w_qkvg"].data_ptr(), by[sa]["q_b"].data_ptr()
-            s.sa_w_out = by[sa.adaptive_zero_init]["w"].data_ptr()
-            p = by[st]
-            s.st_ln_w, s.st_ln_b, s.st_w1, s.st_w2 = (p[k].data_ptr() for k in ("ln_w", "ln_b", "w1", "w2"))
-            s.num_head, s.c_single, s.single_hidden = self.n_heads, self.c_single, p["w2"].shape[1]
+            c, p, a, o, t = self.c_single, by[self], by[sa], by[sa.adaptive_zero_init], by[st]
+            n, hidden = by[sa.adaptive_layernorm], t["w2"].shape[1]
+            point(s, ("sl_ln_w", p["ln_w"], (128,)), ("sl_ln_b", p["ln_b"], (128,)),
+                  ("sl_w", p["w_logits"], ((self.n_heads + 31) // 32 * 32, 128)),
+                  ("sa_ln_w", n["ln_w"], (c,)), ("sa_ln_b", n["ln_b"], (c,)), ("sa_w_qkvg", a["w_qkvg"], (4 * c, c)),
+                  ("sa_q_b", a["q_b"], (c,)), ("sa_w_out", o["w"], (c, c)), ("st_ln_w", t["ln_w"], (c,)),
+                  ("st_ln_b", t["ln_b"], (c,)), ("st_w1", t["w1"], (2 * hidden, c)), ("st_w2", t["w2"], (c, hidden)))
+            s.num_head, s.c_single, s.single_hidden = self.n_heads, c, hidden
         self._native = (s, packs)
         return s
 

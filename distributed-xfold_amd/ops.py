@@ -62,6 +62,13 @@ def _gpu(t: torch.Tensor, name: str, dtype=None, shape=None) -> torch.Tensor:
     return t
 
 
+def _weights_with(t: torch.Tensor, *blocks):
+    """The structures of packed weights hold addresses: they must be of the activations' device."""
+    for b in blocks:
+        if b.device != t.device:
+            raise ValueError(f"weights: live on {b.device}, the activations on {t.device}")
+
+
 def _p(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
 
@@ -207,6 +214,7 @@ def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incomi
     if pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair.shape[2] != 128:
         raise ValueError(f"pair: expected [N, N, 128], got {tuple(pair.shape)}")
     n, dev = pair.shape[0], pair.device
+    _weights_with(pair, *blocks)
     io = _dt(pair)
     maskf = _mask_f32(pair_mask, (n, n), "mask")
     mask_in = _mask_f32(pair_mask_incoming, (n, n), "mask")
@@ -338,6 +346,7 @@ def outer_product_mean(block, msa, msa_mask, pair, residual):
     lib = _L.load()
     dt, maskf = _msa_inputs(msa, msa_mask)
     rows, n, _ = msa.shape
+    _weights_with(msa, block)
     _gpu(pair, "pair", shape=(n, n, 128))
     ws = _ws(lib.af3_msa_workspace_bytes(rows, n), msa.device)
     rc = lib.af3_outer_product_mean_forward(ctypes.addressof(block), _p(msa), dt, _p(maskf), _p(pair), _dt(pair),
@@ -351,6 +360,7 @@ def msa_attention(block, msa, msa_mask, pair, residual):
     lib = _L.load()
     dt, maskf = _msa_inputs(msa, msa_mask)
     rows, n, _ = msa.shape
+    _weights_with(msa, block)
     _gpu(pair, "pair", shape=(n, n, 128))
     out = msa if residual else torch.empty_like(msa)
     ws = _ws(lib.af3_msa_workspace_bytes(rows, n), msa.device)
@@ -382,6 +392,7 @@ def evoformer_stack(blocks, msa, pair, msa_mask, pair_mask):
     lib = _L.load()
     dt, maskf = _msa_inputs(msa, msa_mask)
     rows, n, _ = msa.shape
+    _weights_with(msa, *blocks)
     _gpu(pair, "pair", shape=(n, n, 128))
     pmf = _mask_f32(pair_mask, (n, n), "pair_mask")
     need = lib.af3_msa_workspace_bytes(rows, n)
@@ -400,6 +411,7 @@ def diffusion_transformer(blocks, act, mask, pair_logits, scale_shift, gate, num
     [H, S/4, S, 4]; scale_shift [cond_rows, 2 blocks, 2 C] and gate [cond_rows, 2 blocks, C] fp32."""
     lib = _L.load()
     _gpu(act, "act")
+    _weights_with(act, blocks)
     b, s, c = act.shape
     nb = len(blocks)
     quad = int(pair_logits[0].dim() == 4)
@@ -428,6 +440,7 @@ def atom_transformer(blocks, act, key_rows, mask_q, mask_k, pair_logits, scale_s
     [S Q, 2 blocks, 2 C], scale_shift_k [S Q, blocks, 2 C], gate [2 blocks, S Q, C] fp32."""
     lib = _L.load()
     _gpu(act, "act")
+    _weights_with(act, blocks)
     s, q, c = act.shape[-3:]
     b = act.numel() // (s * q * c)
     nb, k = len(blocks), key_rows.shape[-1]

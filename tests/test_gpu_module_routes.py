@@ -164,3 +164,17 @@ def test_a_batch_of_single_representations(gpu_pkg):
         want = stack(pair.clone(), pm, both[i].clone(), sm)
         # (a single sequence's products may sum in another order)
         assert torch.equal(got[0], want[0]) and float((got[1][i] - want[1]).norm() / want[1].norm()) < 1e-2
+
+
+def test_modules_left_on_the_cpu_are_refused(gpu_pkg):
+    nn = gpu_pkg.nn
+    pair, pm, single, sm = trunk_inputs(12)
+    msa, act, cond = torch.zeros(3, 12, 64, device="cuda"), torch.zeros(1, 12, 768, device="cuda"), torch.zeros(12, 384, device="cuda")
+    logits = [torch.zeros(1, 16, 3, 12, 4, device="cuda")]
+    for call in (lambda: nn.PairformerBlock()(pair, pm, single, sm), lambda: nn.PairformerStack(num_blocks=2)(pair, pm, single, sm),
+                 lambda: nn.EvoformerBlock()(msa, pair, sm.expand(3, -1).contiguous(), pm),
+                 lambda: nn.OuterProductMean()(msa, sm.expand(3, -1).contiguous()),
+                 lambda: nn.MSAAttention()(msa, sm.expand(3, -1).contiguous(), pair),
+                 lambda: nn.DiffusionTransformer(num_blocks=1, super_block_size=1)(act, sm, cond, pair, pair_logits=logits)):
+        with pytest.raises(ValueError, match="cpu"):
+            call()

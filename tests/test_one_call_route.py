@@ -43,9 +43,9 @@ def _small(nn, name):
         return nn.EvoformerBlock(), lambda m: m.native()
     if name == "DiffusionTransformer":
         kw = dict(c_act=48, num_head=2, num_blocks=2, super_block_size=1)
-        table = lambda m: nn.diffusion_transformer.block_table(m, list(zip(m.self_attention, m.transition_block)))
+        table = lambda m: nn.diffusion_transformer.block_table(m, list(zip(m.self_attention, m.transition_block)), 48)
         return nn.DiffusionTransformer(**kw), table
-    table = lambda m: nn.diffusion_transformer.block_table(m, list(zip(m.cross_attention, m.transition_block)))
+    table = lambda m: nn.diffusion_transformer.block_table(m, list(zip(m.cross_attention, m.transition_block)), 128)
     return nn.DiffusionCrossAttTransformer(num_blocks=1), table
 
 
@@ -186,3 +186,36 @@ def test_a_strided_tensor_goes_to_the_padded_transition(pkg, monkeypatch):
     monkeypatch.setattr(pkg.ops, "transition128", lambda x, *a, **k: x + 1)
     x = torch.zeros(64, 6).t()
     assert pkg.nn.Transition(c_x=64).run(x, True) is x and bool((x == 1).all())
+
+
+@pytest.mark.parametrize("name,layer,widths", [
+    ("PairformerBlock", "pair_transition.transition2", (256, 128)),
+    ("PairformerBlock", "single_attention_.adaptive_zero_init.transition2", (256, 384)),
+    ("PairformerBlock", "pair_attention1.output_projection", (64, 128)),
+    ("EvoformerBlock", "msa_attention1.gating_query", (32, 64)),
+    ("EvoformerBlock", "msa_transition.transition1", (64, 128)),
+    ("DiffusionTransformer", "self_attention.1.adaptive_zero_init.transition2", (24, 48)),
+    ("DiffusionCrossAttTransformer", "transition_block.0.transition1", (128, 256))])
+def test_weights_of_another_shape_are_refused(pkg, name, layer, widths):
+    """The structures carry addresses without sizes: a kernel would read past a smaller weight."""
+    mod, make = _small(pkg.nn, name)
+    parent, _, leaf = layer.rpartition(".")
+    setattr(mod.get_submodule(parent), leaf, torch.nn.Linear(*widths, bias=False))
+    with pytest.raises(ValueError, match="expected a contiguous|of size|invalid for input"):
+        make(mod)
+
+
+def test_weights_on_another_device_are_refused(pkg):
+    """The addresses of weights that are still on the CPU are nothing a kernel may be given."""
+    nn, ops = pkg.nn, pkg.ops
+    for name in NATIVE:
+        mod, make = _small(nn, name)
+        native = make(mod)
+        assert native.device == torch.device("cpu")
+        with pytest.raises(ValueError, match="weights: live on cpu"):
+            ops._weights_with(torch.empty(1, device="meta"), native)
+        ops._weights_with(torch.empty(1), native)
+    blk = nn.EvoformerBlock()
+    blk.pair_transition._packed = {k: v.to("meta") for k, v in blk.pair_transition.packed().items()}
+    with pytest.raises(ValueError, match="other weights of the block on cpu"):
+        blk.native()
