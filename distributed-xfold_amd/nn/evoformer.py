@@ -17,7 +17,10 @@ call of the library (`evoformer_loop`).
 Both sum over an index (MSA rows, tokens) that the activations [rows, N, c]
 carry as an outer one, while the dense kernels want it innermost: the
 projections are written transposed.  Other widths go operator by operator
-through the general kernels and torch permutations.
+through the general kernels; there the operands are produced transposed
+(projection weights as the left operand) or run through the bf16 transpose
+kernel where rows and tokens are multiples of 8, and through strided copies
+elsewhere.
 """
 
 from __future__ import annotations
@@ -99,6 +102,8 @@ class OuterProductMean(HipModule):
 
         def projected(w):        # [(token, channel), MSA row]: the summation index innermost
             y = ops.linear(x, w) * mb                                                       # [a, N, co]
+            if a % 8 == 0 and (n * co) % 8 == 0:
+                return ops.transpose2d(y.view(a, n * co))
             return _pad_last(y.permute(1, 2, 0).reshape(n * co, a)).contiguous()
         lt, rt = projected(p["w_l"]), projected(p["w_r"])
         inv_norm = (1.0 / (self.epsilon + m.t() @ m)).contiguous()                         # [b, d]
@@ -168,11 +173,22 @@ class MSAAttention(HipModule):
         logits = ops.pair_logits(pair.contiguous(), p["pn_w"], p["pn_b"], p["w_logits"], h)     # [h, q, k] fp32
         # softmax over the keys of logits + 1e9 (key mask - 1), bf16, rows padded to a multiple of 8
         w = ops.masked_softmax_rows(logits, msa_mask.float().max(dim=0).values.contiguous())        # [h, q, k]
-        v = ops.linear(x, p["w_v"])                                                               # [a, k, (h d)]
-        gate = ops.linear(x, p["w_g"], sigmoid=True)
-        vt = _pad_last(v.view(a, n, h, d).permute(2, 0, 3, 1).reshape(h, a * d, n)).contiguous()
-        avg = ops.batched_nt_product(w, vt)                                                       # [h, q, (row, d)]
-        avg = avg.view(h, n, a, d).permute(2, 1, 0, 3).reshape(a, n, c) * gate
+        if n % 8 == 0 and c % 8 == 0:
+            # Everything with the tokens innermost: the value and gate projections are taken
+            # transposed (weights as the left operand), [(h, d), (row, k)], which is per head the
+            # k-contiguous right operand of the averaging product; its result [(h, d), (row, q)]
+            # has the same layout, takes the gate there and is transposed once for the output projection.
+            x2 = x.view(a * n, c)
+            v_t = ops.linear(p["w_v"], x2)                                                        # [(h d), (row, k)]
+            gate_t = ops.linear(p["w_g"], x2, sigmoid=True)
+            avg_t = ops.batched_nt_product(v_t.view(h, d * a, n), w)                              # [h, (d, row), q]
+            avg = ops.transpose2d(avg_t.view(c, a * n) * gate_t).view(a, n, c)
+        else:
+            v = ops.linear(x, p["w_v"])                                                           # [a, k, (h d)]
+            gate = ops.linear(x, p["w_g"], sigmoid=True)
+            vt = _pad_last(v.view(a, n, h, d).permute(2, 0, 3, 1).reshape(h, a * d, n)).contiguous()
+            avg = ops.batched_nt_product(w, vt)                                                   # [h, q, (row, d)]
+            avg = avg.view(h, n, a, d).permute(2, 1, 0, 3).reshape(a, n, c) * gate
         if residual:
             return ops.linear(avg, p["w_o"], out_dtype=msa.dtype, mode=ops._L.LINEAR_GATE_RES, residual=msa, out=msa)
         return ops.linear(avg, p["w_o"], out_dtype=msa.dtype)

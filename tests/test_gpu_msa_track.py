@@ -72,3 +72,21 @@ def test_a_run_of_blocks_is_the_blocks_in_turn(gpu_pkg, rows, n, dtype):
         one = blk(*one, mask.to("cuda:0"), pair_mask)
     two = gpu_pkg.nn.evoformer.evoformer_loop(blocks, *two, mask.to("cuda:0"), pair_mask)
     assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])
+
+
+@pytest.mark.parametrize("rows,n", [(16, 24), (12, 24), (16, 21)])       # operands produced transposed; by strided copies
+@pytest.mark.parametrize("c", [32, 128])
+def test_msa_operators_of_other_widths(gpu_pkg, c, rows, n):
+    g = torch.Generator().manual_seed(c + rows + n)
+    rb = lambda *s: O.round_bf16(torch.randn(*s, generator=g))
+    msa, pair, mask = rb(rows, n, c), rb(n, n, 128), (torch.rand(rows, n, generator=g) > 0.2).float()
+    mask[0] = 1
+    for cls, args in (("OuterProductMean", (mask,)), ("MSAAttention", (mask, pair))):
+        mod = getattr(gpu_pkg.nn, cls)(c_msa=c)
+        for p in mod.parameters():
+            p.data = O.round_bf16(torch.randn(p.shape, generator=g) * 0.1 + (1.0 if p.dim() == 1 else 0.0))
+        q = {k: v.double() for k, v in mod.state_dict().items()}
+        ref = M.outer_product_mean if cls == "OuterProductMean" else M.msa_attention
+        want = ref(msa.double(), *(a.double() for a in args), q)
+        assert not mod.native
+        compare(f"{cls} {c} channels {rows} {n}", mod.to("cuda:0")(msa.to("cuda:0"), *(a.to("cuda:0") for a in args)), want)
