@@ -502,7 +502,7 @@ class DiffusionCrossAttTransformer(HipModule):
             if int(idx.min()) < 0 or int(idx.max()) >= n_atoms:
                 raise ValueError("queries_to_keys indexes beyond the query atoms")
             key_rows = torch.where(gmask.bool(), idx, torch.full_like(idx, -1)).to(torch.int32).contiguous()
-            key_rows._af3_checked_rows = n_atoms
+            ops.rows_in_range(key_rows, n_atoms, known=True)
             keys_single_cond = queries_single_cond          # per atom
         if pair_cond.dtype == torch.float32 and pair_cond.dim() == 4 and pair_cond.shape[-1] == 16 \
                 and self.num_blocks * self.num_head <= 32:

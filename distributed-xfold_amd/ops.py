@@ -445,10 +445,7 @@ def atom_transformer(blocks, act, key_rows, mask_q, mask_k, pair_logits, scale_s
     b = act.numel() // (s * q * c)
     nb, k = len(blocks), key_rows.shape[-1]
     _gpu(key_rows, "key_rows", torch.int32, (s, k))
-    if getattr(key_rows, "_af3_checked_rows", None) != s * q:
-        if int(key_rows.max()) >= s * q:
-            raise ValueError("key_rows: row index beyond the atoms")
-        key_rows._af3_checked_rows = s * q
+    rows_in_range(key_rows, s * q, "key_rows")
     quads = pair_logits.dim() == 6
     _gpu(pair_logits, "pair_logits", torch.float32, (nb, s, num_head) + ((k // 4, q, 4) if quads else (q, k)))
     _gpu(scale_shift_q, "scale_shift_q", torch.float32, (s * q, 2 * nb, 2 * c))
@@ -528,10 +525,7 @@ def atom_position_features(positions, rows, weight, cond, out_dtype=torch.bfloat
     _gpu(cond, "cond", torch.float32, (q, c))
     if c % 8:
         raise ValueError("channels must be a multiple of 8")
-    if getattr(rows, "_af3_checked_rows", None) != n_slots:
-        if int(rows.max()) >= n_slots:
-            raise ValueError("rows: slot index beyond positions")
-        rows._af3_checked_rows = n_slots
+    rows_in_range(rows, n_slots)
     out = torch.empty((b, q, c), dtype=out_dtype, device=positions.device)
     rc = lib.af3_atom_position_features_forward(_p(positions), _p(rows), _p(weight), _p(cond), _p(out), _dt(out),
                                                 b, n_slots, q, c, _stream(positions.device))
@@ -539,13 +533,21 @@ def atom_position_features(positions, rows, weight, cond, out_dtype=torch.bfloat
     return out
 
 
+def rows_in_range(rows, n_src, name="rows", known=False):
+    """Index tensors are checked once, at the cost of a device round trip, and marked with what was checked: the bound and
+    the tensor's version, which every write into it changes.  (Inference tensors have no version: theirs is the bound
+    alone.)  `known`: the caller has made the tensor so."""
+    mark = n_src, None if rows.is_inference() else rows._version
+    if getattr(rows, "_af3_checked_rows", None) != mark:
+        if not known and rows.numel() and int(rows.max()) >= n_src:
+            raise ValueError(f"{name}: row index beyond the source's {n_src}")
+        rows._af3_checked_rows = mark
+
+
 def _rows32(rows, n_src, device, name="rows"):
     if rows.dtype != torch.int32 or rows.dim() != 1 or not rows.is_contiguous() or rows.device != device:
         raise ValueError(f"{name}: expected a contiguous int32 vector on the device of the data")
-    if getattr(rows, "_af3_checked_rows", None) != n_src:
-        if int(rows.max()) >= n_src:
-            raise ValueError(f"{name}: row index beyond the source")
-        rows._af3_checked_rows = n_src             # one device round trip per index tensor
+    rows_in_range(rows, n_src, name)
 
 
 def gather_rows_add(src, rows, add):
@@ -600,10 +602,7 @@ def gathered_relu_mean(src, idx, count):
     t, a = idx.shape
     if a > 32 or c % 8:
         raise ValueError("at most 32 slots, channels a multiple of 8")
-    if not getattr(idx, "_af3_checked_rows", None) == n_src:
-        if int(idx.max()) >= n_src:
-            raise ValueError("idx: row index beyond src")
-        idx._af3_checked_rows = n_src          # one device round trip per index tensor
+    rows_in_range(idx, n_src, "idx")
     _gpu(count, "count", torch.float32, (t,))
     out = torch.empty((b, t, c), dtype=torch.float32, device=src.device)
     rc = lib.af3_gathered_relu_mean_forward(_p(src), _p(idx), _p(count), _p(out), b, n_src, t, a, c,
@@ -682,11 +681,7 @@ def gathered_cross_attention(q_data, atom_data, key_rows, pair_logits, mask_q, m
     bb, sk = key_rows.shape
     if b != samples * bb:
         raise ValueError("q_data: batch must be samples * windows")
-    if getattr(key_rows, "_af3_checked_rows", None) != n_atoms:
-        # (one device round trip; the tensor is marked so that it is paid once)
-        if int(key_rows.max()) >= n_atoms:
-            raise ValueError("key_rows: row index beyond atom_data")
-        key_rows._af3_checked_rows = n_atoms
+    rows_in_range(key_rows, n_atoms, "key_rows")
     if pair_logits is not None:
         _gpu(pair_logits, "pair_logits", torch.float32, (bb, num_head, sq, sk))
     mq = mk = None

@@ -219,3 +219,18 @@ def test_weights_on_another_device_are_refused(pkg):
     blk.pair_transition._packed = {k: v.to("meta") for k, v in blk.pair_transition.packed().items()}
     with pytest.raises(ValueError, match="other weights of the block on cpu"):
         blk.native()
+
+
+def test_an_index_tensor_that_was_written_to_is_checked_again(pkg):
+    """The kernels read the rows that an index tensor names; a check of earlier contents is none of the present ones."""
+    rows = torch.tensor([0, 3, -1], dtype=torch.int32)
+    for _ in range(2):
+        pkg.ops.rows_in_range(rows, 4)
+    rows[2] = 4
+    with pytest.raises(ValueError, match="beyond"):
+        pkg.ops.rows_in_range(rows, 4)
+    pkg.ops.rows_in_range(rows, 5)
+    with pytest.raises(ValueError, match="beyond"):
+        pkg.ops.rows_in_range(rows, 4)
+    with torch.inference_mode():
+        pkg.ops.rows_in_range(rows.clone(), 5)
