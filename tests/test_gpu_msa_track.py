@@ -90,3 +90,23 @@ def test_msa_operators_of_other_widths(gpu_pkg, c, rows, n):
         want = ref(msa.double(), *(a.double() for a in args), q)
         assert not mod.native
         compare(f"{cls} {c} channels {rows} {n}", mod.to("cuda:0")(msa.to("cuda:0"), *(a.to("cuda:0") for a in args)), want)
+
+
+@pytest.mark.parametrize("rows,n", [(33, 70), (9, 21)])
+@pytest.mark.parametrize("poison", [float("nan"), float("inf")])
+def test_a_masked_position_that_is_not_finite(gpu_pkg, rows, n, poison):
+    """The mask multiplies, as in the reference: what is not finite stays so under a mask of zero, in the tokens and rows
+    that it is part of (the last MSA row, which the tiles repeat behind the end, among them) and in no other."""
+    p, msa, pair, mask = inputs(rows, n)
+    for at in ((rows - 1, 3), (2, n - 1)):
+        msa[at], mask[at] = poison, 0
+    for name, cls, ref, more in (("outer_product_mean", "OuterProductMean", M.outer_product_mean, ()),
+                                 ("msa_attention1", "MSAAttention", M.msa_attention, (pair,))):
+        mod = getattr(gpu_pkg.nn, cls)()
+        mod.load_state_dict(O._sub(p, name))
+        mod.to("cuda:0")
+        want = ref(msa.double(), mask.double(), *(x.double() for x in more), O._sub(O.cast_params(p, D), name))
+        got = mod(*(x.to("cuda:0") for x in (msa, mask, *more))).cpu()
+        lost = torch.isnan(want)
+        assert torch.equal(torch.isnan(got), lost) and 0 < int(lost.sum()) < lost.numel() // 2
+        compare(f"{cls} {rows} {n} {poison}", got[~lost], want[~lost])

@@ -68,3 +68,20 @@ def test_pair_logits_of_the_token_attention_in_quads(gpu_pkg, n, dtype):
     quads = gpu_pkg.ops.pair_logits(pair, ln, None, w, 40, quads=True)
     want = torch.nn.functional.pad(rows, (0, -n % 4)).view(40, n, -1, 4).transpose(1, 2)
     assert torch.equal(quads, want)
+
+
+@pytest.mark.parametrize("sq,sk,windows", [(32, 128, 3), (7, 60, 5), (9, 60, 600)])
+@pytest.mark.parametrize("poison", [float("nan"), float("inf")])
+def test_an_empty_slot_reads_nothing(gpu_pkg, sq, sk, windows, poison):
+    """Rows of the table that no slot names, row 0 and the last one among them, decide nothing."""
+    g = torch.Generator(device="cuda").manual_seed(sq + sk)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    c, atoms = 128, 50
+    q, table, bias = rnd(2 * windows, sq, c).bfloat16(), rnd(2, atoms, c).bfloat16(), rnd(windows, 4, sq, sk)
+    rows = torch.randint(-8, atoms - 1, (windows, sk), generator=g, device="cuda")
+    rows = torch.where(rows <= 0, torch.full_like(rows, -1), rows).to(torch.int32)
+    w, b = [(rnd(2 * c, c) * 0.1).bfloat16() for _ in range(2)], rnd(c)
+    run = lambda: gpu_pkg.ops.gathered_cross_attention(q, table, rows, bias, None, None, w[0], w[1], b, 4)
+    want = run()
+    table[:, 0] = table[:, -1] = poison
+    assert torch.isfinite(want).all() and torch.equal(run(), want)
