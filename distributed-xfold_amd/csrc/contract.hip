@@ -717,7 +717,7 @@ int launch_big_tile(const GemmArgs& g_in, int mode, hipStream_t stream) {
   // N = 256 .. 576, not 768 (six rounds against five) or beyond.
   const int cus = cu_count();
   const bool flat = ((total3 + cus - 1) / cus) * 7 < ((total4 + cus - 1) / cus) * 8;
-  const XcdWalk walk = xcd_walk((g.M + (flat ? 191 : 255)) / (flat ? 192 : 256), tiles_n, g.batch, flat ? 192 : 256, CN);
+  const XcdWalk walk = xcd_walk((g.M + (flat ? 191 : 255)) / (flat ? 192 : 256), tiles_n, g.batch, flat ? 192 : 256, CN, cus / 8);
   if (walk.slots * 8 > 0x3fffffff) return AF3_ERR_BAD_ARG;
   g.xcd_m = walk.rows;
   // persistent workgroups, one per CU (a multiple of 8: ids are dealt round-robin to the 8 XCDs)

@@ -353,7 +353,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArg
 template <int MT, int NT, int WM, int WN, int WK, int ST, int WPS, bool CLEAN = true, bool VEC = true>
 int launch_tile(GemmArgs g, hipStream_t stream) {
   constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN;
-  const XcdWalk walk = xcd_walk((g.M + BM - 1) / BM, (g.N + BN - 1) / BN, g.batch, BM, BN);
+  constexpr int PER_CU = WPS * 4 / (WM * WN * WK);  // workgroups that a CU holds
+  static_assert(PER_CU >= 1, "WPS is in waves per SIMD");
+  const XcdWalk walk = xcd_walk((g.M + BM - 1) / BM, (g.N + BN - 1) / BN, g.batch, BM, BN, XCD_CUS * PER_CU);
   const int64_t blocks = walk.slots * 8;
   if (blocks > 0x3fffffff) return AF3_ERR_BAD_ARG;
   g.xcd_m = walk.rows;

@@ -45,18 +45,22 @@ struct XcdWalk {
   int rows = 0;
   int64_t slots = 0;  // tiles of the busiest XCD
 };
-// The walk that fetches least, if that is at least a third less and no XCD gets 4 % more tiles than its share: an uneven
-// deal costs what it saves (1920 x 768 x 1536 in 64 x 64 tiles: 48 tiles against 45, 16.8 us against 15.4).
+// The walk that fetches least, if that is at least a third less, no XCD gets 4 % more tiles than its share, and its
+// tiles take no more rounds.  `per_round`: tiles that an XCD's 32 CUs hold at a time.  An uneven deal costs what it
+// saves (1920 x 768 x 1536 in 64 x 64 tiles: 48 tiles against 45, 16.8 us against 15.4), and a whole round where the
+// even deal just fits: 33 tiles against 32 on one XCD (5300 x 768 x 1536 with gate and residual in 128 x 128 tiles 35.9 us,
+// even 23.8; 3900 x 3072 x 768 in 192 x 256 tiles 42.0, even 27.4, with SwiGLU 32.3 and 22.0).
 // 3840 x 768 x 768 14.3 -> 12.4 us, 3840 x 768 x 1536 24.1 -> 22.0, 3200 x 768 x 1536 22.9 -> 20.5.
-inline XcdWalk xcd_walk(int64_t tiles_m, int64_t tiles_n, int64_t batch, int bm, int bn) {
+constexpr int XCD_CUS = 32;
+inline XcdWalk xcd_walk(int64_t tiles_m, int64_t tiles_n, int64_t batch, int bm, int bn, int64_t per_round) {
   XcdWalk w;
   w.slots = (tiles_m * tiles_n * batch + 7) / 8;
   if (batch != 1) return w;
   int64_t least = (w.slots < tiles_m ? w.slots : tiles_m) * bm + ((w.slots + tiles_m - 1) / tiles_m) * bn;
-  const int64_t limit = least * 2 / 3;
+  const int64_t limit = least * 2 / 3, rounds = (w.slots + per_round - 1) / per_round;
   for (int rows = 1; rows <= 8; rows *= 2) {
     const int64_t m = (tiles_m + rows - 1) / rows, n = (tiles_n + 8 / rows - 1) / (8 / rows), fetch = m * bm + n * bn;
-    if (m * n * 25 > w.slots * 26 || fetch > limit || fetch >= least) continue;
+    if (m * n * 25 > w.slots * 26 || (m * n + per_round - 1) / per_round > rounds || fetch > limit || fetch >= least) continue;
     least = fetch;
     w.rows = rows;
   }
