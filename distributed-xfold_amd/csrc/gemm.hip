@@ -379,12 +379,16 @@ int launch_tile(GemmArgs g, hipStream_t stream) {
 
 // Wide products whose tiles come out just below a whole number per CU (256 CUs), which is worth more than the tile's
 // bytes per FLOP: one product's tiles all run at once, and a few tiles more than that cost another round.  Eight waves.
-//   128x128, one per CU, four slab buffers   200 < T <= 256 tiles (1250x3072x768 14.5 us, was 16.0; SwiGLU 11.4, 14.3;
-//                                            4200x768x1536 22.6, 26.7); not the short ones with gate and residual
-//   128x192, one per CU                      where that many hold the product (1700x3072x768 17.6, 18.6; SwiGLU 12.8, 15.4;
-//                                            5400x768x1536 25.1, 30.5)
-//   128x128, two per CU                      352 < T <= 512 (2300x3072x768 20.7, 26.4; SwiGLU 16.7, 21.5;
-//                                            9000x768x1536 31.2, 47.0)
+// T: 128x128 tiles; us, the tile that the rules of launch_gemm_nt give otherwise behind it.
+//   128x128, one per CU, four slab buffers   200 < T <= 256 and K >= 512: 4600x768x768 11.2 (12.8), 1150x3072x768 11.0
+//                                            (12.6), 9000x384x768 11.2 (12.7), 1150x3072x512 9.7 (9.9).  SwiGLU from 190:
+//                                            1000x3072x768 9.6 (9.9), 1060 rows 9.7 (11.6), 1250 rows 10.0 (12.4).  With
+//                                            gate and residual from K = 1024, 4600x768x1024 16.0 (17.6): at K = 768 it is
+//                                            4600 rows 14.3 (15.3), but 4992 rows 15.6 (15.6) and 1280x3072 16.6 (16.0)
+//   128x192, one per CU                      where that many hold the product: 1700x3072x768 17.6 (18.6), SwiGLU 12.5 (14.3),
+//                                            1900 rows 13.0 (15.2); 7000x768x768 14.7 (15.6); 5400x768x1536 25.1 (30.5)
+//   128x128, two per CU                      352 < T <= 512: 2300x3072x768 20.7 (26.4), SwiGLU 15.3 (19.9);
+//                                            9000x768x1536 31.2 (47.0)
 enum { MID_NONE = 0, MID_128_ONE, MID_192, MID_128_TWO };
 static int mid_tile_choice(const GemmArgs& g) {
   if (g.batch != 1 || (g.K % KS) || g.M <= 128 || g.N <= 128) return MID_NONE;
@@ -435,13 +439,18 @@ int launch_gemm_nt(const GemmArgs& g_in, hipStream_t stream) {
                    (g.gate_per_row || al(g.gate, g.ld_gate * 4, 0)) && al(g.res_f32, g.ld_res * 4, g.sRes * 4) &&
                    al(g.res_bf16, g.ld_res * 2, g.sRes * 2);
 
-  // The tile, by the number T of 64x64 tiles (256 CUs; measured over M = 64 ... 92160, N = 128 ... 73728,
-  // K = 64 ... 1536; SwiGLU pairs 32-column blocks, so its tiles are 64 columns or more):
-  //   T <= 128   32x32, the 64x64 tiles would leave half of the CUs without one; with split_k the K range goes to four
-  //              waves, or eight where it is long
+  // The tile, by the number T of 64x64 tiles, on 256 CUs.  The lines up to 512 lie where a CU gets its second and third
+  // tile; each with both sides at the line, us.  (Measured over M = 64 ... 92160, N = 128 ... 73728, K = 64 ... 1536.)
+  //   T <= 128   32x32, the 64x64 tiles would leave half of the CUs without one (500x768x768 6.2, 64x64 6.7); with split_k
+  //              the K range goes to four waves, or eight where it is long.  (SwiGLU pairs 32-column blocks: 64 columns or
+  //              more)
   //   T <= 384   with split_k: 64x64, K split two ways (eight waves per tile); long ones are faster unsplit
-  //   T <= 1000  64x64, with as many slab buffers as leave room for the workgroups a CU gets: four, three or two
-  //              (a SwiGLU of more than 352: 128x64, two of whose tiles a CU holds; 500x3072x768 8.5 us, was 9.3)
+  //   T <= 256   64x64 with four slab buffers, a workgroup to a CU
+  //   T <= 512   64x64 with three, two to a CU: 2555x768x768 gated 9.8, with two buffers 10.2; K = 1536 14.5, 16.1; past
+  //              the line 2811x768x768 11.9, 10.9; K = 1536 18.5, 16.8.  A SwiGLU of K >= 384 whose 128x64 tiles are at
+  //              most one to a CU, but not many fewer: 500x3072x768 7.4, 64x64 7.7; 635 rows 7.5, 8.0; 571x3072x1536 11.1,
+  //              11.8; past the line 699x3072x768 9.5, 9.2 (two buffers), 763x3072x384 7.2, 6.5; K = 128 6400x256 4.0, 4.0
+  //   T <= 1000  64x64 with two, four to a CU
   //   T <= 2600  64x128, else 128x128: bytes per FLOP count once every CU has several tiles (and never wider than N)
   const int64_t T = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch;
   const bool wide = g.epi == EPI_SWIGLU;
@@ -458,8 +467,9 @@ int launch_gemm_nt(const GemmArgs& g_in, hipStream_t stream) {
   }
   if (T <= 128 && !wide) return launch_tile<1, 1, 1, 1, 1, 4, 1>(g, stream);
   if (T <= 256) return launch_tile<1, 1, 2, 2, 1, 4, 2>(g, stream);
-  if (T > 352 && T <= 640 && wide) return launch_tile<2, 1, 2, 2, 1, 3, 2>(g, stream);
-  if (T <= 640) return launch_tile<1, 1, 2, 2, 1, 3, 3>(g, stream);
+  const int64_t T128x64 = (int64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * g.batch;
+  if (wide && T > 352 && T128x64 <= 256 && g.K >= 384) return launch_tile<2, 1, 2, 2, 1, 3, 2>(g, stream);
+  if (T <= 512) return launch_tile<1, 1, 2, 2, 1, 3, 3>(g, stream);
   if (T <= 1000 || g.N <= 64) return launch_tile<1, 1, 2, 2, 1, 2, 4>(g, stream);
   if (T <= 2600 || g.N <= 128) return launch_tile<1, 2, 2, 2, 1, 2, 3>(g, stream);
   return launch_tile<2, 2, 2, 2, 1, 2, 2>(g, stream);

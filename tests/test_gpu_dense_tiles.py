@@ -19,7 +19,8 @@ SHAPES = [
     (1921, 3080, 128), (8001, 384, 1024), (70, 70016, 64), (180001, 128, 64),         # 64x128
     (8000, 1024, 104), (7777, 2112, 40), (30720, 256, 192),                           # 256x256: K in one, two, three slabs
     (1249, 3072, 512), (1985, 3072, 512), (2113, 3072, 64), (8961, 768, 128), (4225, 768, 1024),   # 128x128, 128x192, eight waves
-    (513, 3008, 128),                        # SwiGLU in 128x64
+    (513, 3008, 128), (513, 3008, 384), (571, 3072, 384),     # SwiGLU in 64x64 and 128x64
+    (2753, 768, 384), (2688, 768, 384), (699, 3072, 384),     # 64x64, just past and below two tiles to a CU
     (20001, 1032, 128),                      # 128x128 (odd columns keep it off the large tile)
 ]
 
