@@ -111,7 +111,9 @@ __device__ __forceinline__ float acc_read(float a) {
   return v;
 }
 
-// s_waitcnt with vmcnt = n, lgkmcnt = 0 (expcnt left alone)
+// s_waitcnt vmcnt(N) lgkmcnt(0): all but the N youngest vector memory operations done, and every LDS read: behind a
+// barrier that follows, the buffers that the waves have read are free.  (vmcnt in bits 0-3 and 14-15, expcnt in bits 4-6,
+// all ones for no wait, lgkmcnt in bits 8-11.)
 template <int N>
 __device__ __forceinline__ void wait_loads_but() {
   static_assert(N >= 0 && N < 64, "vmcnt has six bits");
