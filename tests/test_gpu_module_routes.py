@@ -207,3 +207,42 @@ def test_single_attention_over_a_partly_filled_quad(gpu_pkg, n):
     hook.remove()
     # fp32 sums of products in another order, rounded to bf16 once: an ulp here and there
     assert len(seen) == 1 and float((got - want).norm() / want.norm()) < 2.0 ** -9
+
+
+def test_single_calls_under_capture(gpu_pkg):
+    """Each captured once and replayed on new contents, with the program's own work between the replays.  (One eager call
+    first, as for any capture: it packs the weights and grows the scratch.)"""
+    nn = gpu_pkg.nn
+    stack, blocks = on_gpu(nn.PairformerStack(num_blocks=3)), [on_gpu(nn.EvoformerBlock()) for _ in range(2)]
+    pair, pm, single, sm = trunk_inputs()
+    msa, mm = torch.randn(5, 37, 64, generator=torch.Generator(device="cuda").manual_seed(0), device="cuda"), sm.expand(5, -1).contiguous()
+    act, cond = msa.new_empty(2, 37, 768).normal_().bfloat16(), single.clone()
+    transformer = on_gpu(nn.DiffusionTransformer(num_blocks=2, super_block_size=1))
+    logits = transformer.pair_logits(pair)
+
+    def trunk(p, s):
+        return stack(p.clone(), pm, s.clone(), sm)
+
+    def evoformer(p, m):
+        return nn.evoformer.evoformer_loop(blocks, m.clone(), p.clone(), mm, pm)
+
+    def diffusion(a, c):
+        return (transformer(a.clone(), sm, c, pair, pair_logits=logits),)
+
+    for fn, inputs in ((trunk, (pair, single)), (evoformer, (pair, msa)), (diffusion, (act, cond))):
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            fn(*inputs)
+        torch.cuda.current_stream().wait_stream(side)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = fn(*inputs)
+        for i in range(3):
+            for t in inputs:
+                t.mul_(-1.0).add_(0.125 * i)
+            want = fn(*inputs)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(out, want)), (fn.__name__, i)
