@@ -87,26 +87,40 @@ def point(s, *fields) -> None:
     fp32 and matrices bf16.  The structures carry neither sizes nor types, so what the operator layer checks of every
     tensor is checked here: type, shape, contiguity and one device for all, which is kept as `s.device` for the operator
     layer to compare with the activations'."""
+    device = s.device
     for name, t, shape in fields:
-        dtype = torch.float32 if len(shape) == 1 else torch.bfloat16
-        if tuple(t.shape) != shape or t.dtype != dtype or not t.is_contiguous():
-            raise ValueError(f"{name}: expected a contiguous {dtype} weight {shape}, got {t.dtype} {tuple(t.shape)}")
-        if s.device not in (None, t.device):
-            raise ValueError(f"{name}: on {t.device}, other weights of the block on {s.device}")
-        s.device = t.device
-        if isinstance(name, tuple):
+        if t.shape != shape or t.dtype != (torch.float32 if len(shape) == 1 else torch.bfloat16) or not t.is_contiguous():
+            raise ValueError(f"{name}: expected a contiguous {'fp32' if len(shape) == 1 else 'bf16'} weight {shape}, got "
+                             f"{t.dtype} {tuple(t.shape)}")
+        if t.device != device:
+            if device is not None:
+                raise ValueError(f"{name}: on {t.device}, other weights of the block on {device}")
+            s.device = device = t.device
+        if name.__class__ is tuple:
             getattr(s, name[0])[name[1]] = t.data_ptr()
         else:
             setattr(s, name, t.data_ptr())
 
 
-def as_written(m: nn.Module, cls: type) -> bool:
-    """Whether using `m` does what class `cls` says and nothing else: no subclass, no forward hook (its own or one for
-    all modules), no method replaced on the instance.  A run of modules that goes to the library as one call passes its
-    modules by, so it is made for such modules only."""
-    d, every = m.__dict__, nn.modules.module
-    return (type(m) is cls and not d["_forward_hooks"] and not d["_forward_pre_hooks"] and not every._global_forward_hooks
-            and not every._global_forward_pre_hooks and "forward" not in d and "run" not in d and "packed" not in d)
+_EVERY = nn.modules.module
+
+
+def as_written(*modules) -> bool:
+    """Whether using each of (module, class) does what the class says and nothing else: no subclass, no forward hook (its
+    own or one for all modules), no method replaced on the instance.  A run of modules that goes to the library as one
+    call passes its modules by, so it is made for such modules only.  (Asked at every call: 0.2 us a module.)"""
+    if _EVERY._global_forward_hooks or _EVERY._global_forward_pre_hooks:
+        return False
+    for m, cls in modules:
+        d = m.__dict__
+        if (m.__class__ is not cls or d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d or "run" in d
+                or "packed" in d):
+            return False
+    return True
+
+
+def packs_of(mods) -> list:
+    return [m._packed or m.packed() for m in mods]
 
 
 class HipModule(nn.Module):
@@ -155,10 +169,15 @@ class HipModule(nn.Module):
     def _pack(self):
         raise NotImplementedError
 
+    def _structures(self):
+        """The library's structures of a module that has such, made from the packed weights."""
+
     def load_hip_params(self):
-        for m in self.modules():
-            if isinstance(m, HipModule):
-                m._packed = m._pack()
+        mods = [m for m in self.modules() if isinstance(m, HipModule)]
+        for m in mods:
+            m._packed = m._pack()
+        for m in mods:
+            m._structures()
         return self
 
     def packed(self):
@@ -180,9 +199,9 @@ class HipModule(nn.Module):
 def enable_hip(model: nn.Module) -> int:
     """Counterpart of ModelRunner.enable_xsmm (run_inference.py:197-218): packs
     the weights of every HIP module under `model`.  Returns how many were bound."""
-    n = 0
-    for m in model.modules():
-        if isinstance(m, HipModule):
-            m._packed = m._pack()
-            n += 1
-    return n
+    mods = [m for m in model.modules() if isinstance(m, HipModule)]
+    for m in mods:
+        m._packed = m._pack()
+    for m in mods:
+        m._structures()
+    return len(mods)

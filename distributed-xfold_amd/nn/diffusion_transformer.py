@@ -4,6 +4,7 @@ windowed atom cross-attention transformer."""
 
 from __future__ import annotations
 
+import operator
 from typing import Optional
 
 import torch
@@ -12,33 +13,33 @@ import torch.nn as nn
 from .. import check
 from .. import lib as L
 from .. import ops
-from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pack_swiglu, pad_rows, point
+from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pack_swiglu, packs_of, pad_rows, point
 
 
 def plain_blocks(blocks, norms, attention: type, num_head: int) -> bool:
     """Whether (attention, transition) modules are what one call of the library does for all of them alike.  `norms`:
     the attention's conditioned norms, by name."""
-    if not blocks:
-        return False
-    factor = blocks[0][1].num_intermediate_factor
+    used, factor = [], None
     for att, tr in blocks:
-        sub, t = att._modules, tr._modules
-        if not (as_written(att, attention) and att.num_head == num_head
-                and as_written(tr, DiffusionTransition) and tr.num_intermediate_factor == factor
-                and all(as_written(sub[k], AdaptiveLayerNorm) for k in norms) and as_written(sub["adaptive_zero_init"], AdaLNZero)
-                and as_written(t["adaptive_layernorm"], AdaptiveLayerNorm) and as_written(t["adaptive_zero_init"], AdaLNZero)):
+        if att.__class__ is not attention or tr.__class__ is not DiffusionTransition:
             return False
-    return True
+        factor, sub, t = factor or tr.num_intermediate_factor, att._modules, tr._modules
+        if att.num_head != num_head or tr.num_intermediate_factor != factor:
+            return False
+        used += [(att, attention), (sub["adaptive_zero_init"], AdaLNZero), (tr, DiffusionTransition),
+                 (t["adaptive_layernorm"], AdaptiveLayerNorm), (t["adaptive_zero_init"], AdaLNZero)]
+        used += [(sub[k], AdaptiveLayerNorm) for k in norms]
+    return bool(used) and as_written(*used)
 
 
 def block_table(owner: HipModule, blocks, c: int):
     """The packed weights of a transformer's blocks, (attention, transition) modules on `c` channels, as the array of
     structures the library takes, with the `device` they live on and their transitions' `hidden` width; kept in `owner`
     and made again when any of the modules has been packed again."""
-    mods = [m for att, tr in blocks for m in (att, att.adaptive_zero_init, tr, tr.adaptive_zero_init)]
-    packs = [m.packed() for m in mods]
+    packs = packs_of([m for att, tr in blocks
+                      for m in (att, att._modules["adaptive_zero_init"], tr, tr._modules["adaptive_zero_init"])])
     held = owner._native
-    if held is not None and len(held[1]) == len(packs) and all(a is b for a, b in zip(held[1], packs)):
+    if held is not None and len(held[1]) == len(packs) and all(map(operator.is_, held[1], packs)):
         return held[0]
     table = (L.DiffusionBlockStruct * len(blocks))()
     table.device, table.hidden = None, packs[3]["w"].shape[1]
@@ -275,6 +276,18 @@ class DiffusionTransformer(HipModule):
                     w_ss=bf16(torch.cat(w_ss, dim=0)), b_ss=f32(torch.cat(b_ss)),
                     w_gate=bf16(torch.cat(w_gate, dim=0)), b_gate=f32(torch.cat(b_gate)))
 
+    def _blocks(self):
+        run = self.num_super_blocks * self.super_block_size      # blocks beyond the last whole super-block never run
+        return list(zip(self.self_attention, self.transition_block))[:run]
+
+    def _one_call(self, blocks) -> bool:
+        return plain_blocks(blocks, ("adaptive_layernorm",), SelfAttention, self.num_head)
+
+    def _structures(self):
+        blocks = self._blocks()
+        if self._one_call(blocks):
+            block_table(self, blocks, self.c_act)
+
     def pair_logits(self, pair_cond: torch.Tensor):
         """The pair logits of every super-block, [num_super_blocks] x [b, h, N, N]
         (stored as [b, h, N/4, N, 4], the order the attention kernel reads best,
@@ -309,14 +322,14 @@ class DiffusionTransformer(HipModule):
         if pair_logits is None:
             pair_logits = self.pair_logits(pair_cond)
         ss_all, gate_all = ss_all.view(rows, n_mod, 2 * c), gate_all.view(rows, n_mod, c)
-        run = self.num_super_blocks * self.super_block_size      # blocks beyond the last whole super-block never run
+        blocks = self._blocks()
+        run = len(blocks)
         if run == 0:
             return act
-        blocks = list(zip(self.self_attention, self.transition_block))[:run]
         logits = [pair_logits[i // self.super_block_size][i % self.super_block_size].to(torch.float32).contiguous()
                   for i in range(run)]
         # (the single call knows one key mask for all samples and one order of the logits for all blocks)
-        if (plain_blocks(blocks, ("adaptive_layernorm",), SelfAttention, self.num_head) and (mask is None or mask.dim() == 1)
+        if (self._one_call(blocks) and (mask is None or mask.dim() == 1)
                 and all(t.shape == logits[0].shape for t in logits)):
             if run < self.num_blocks:
                 ss_all, gate_all = ss_all[:, :2 * run].contiguous(), gate_all[:, :2 * run].contiguous()
@@ -465,6 +478,14 @@ class DiffusionCrossAttTransformer(HipModule):
                     w_ss_k=bf16(torch.cat(wk, dim=0)), b_ss_k=f32(torch.cat(bk)),
                     w_gate=bf16(torch.cat(wg, dim=0)), b_gate=f32(torch.cat(bg)))
 
+    def _one_call(self, blocks) -> bool:
+        return plain_blocks(blocks, ("q_adaptive_layernorm", "k_adaptive_layernorm"), CrossAttention, self.num_head)
+
+    def _structures(self):
+        blocks = list(zip(self.cross_attention, self.transition_block))
+        if self._one_call(blocks):
+            block_table(self, blocks, self.c_query)
+
     @staticmethod
     def _gather_info(queries_to_keys):
         if hasattr(queries_to_keys, "gather_idxs"):
@@ -537,8 +558,7 @@ class DiffusionCrossAttTransformer(HipModule):
             cond = self.conditioning(queries_single_cond, keys_single_cond, pair_cond)
         logits, ss_q, ss_k, gate, key_rows = cond
         blocks = list(zip(self.cross_attention, self.transition_block))
-        if key_rows is not None and plain_blocks(blocks, ("q_adaptive_layernorm", "k_adaptive_layernorm"), CrossAttention,
-                                                 self.num_head):
+        if key_rows is not None and self._one_call(blocks):
             table = block_table(self, blocks, self.c_query)
             return ops.atom_transformer(table, queries_act, key_rows, queries_mask, keys_mask,
                                         logits.to(torch.float32).contiguous(), ss_q, ss_k, gate, self.num_head, table.hidden)

@@ -25,6 +25,7 @@ elsewhere.
 
 from __future__ import annotations
 
+import operator
 from typing import Optional
 
 import torch
@@ -34,7 +35,7 @@ import torch.nn.functional as F
 from .. import check, ops
 from .. import lib as L
 from .attention import GridSelfAttention
-from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pad_rows, point
+from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, packs_of, pad_rows, point
 from .pairformer import fill_pair_weights, plain_pair_track
 from .primitives import Transition
 from .triangle_multiplication import TriangleMultiplication
@@ -221,25 +222,28 @@ class EvoformerBlock(HipModule):
         return {}
 
     def _tracks(self):
-        return ((self.outer_product_mean, self.msa_attention1, self.msa_transition),
-                ((self.triangle_multiplication_outgoing, self.triangle_multiplication_incoming),
-                 (self.pair_attention1, self.pair_attention2), self.pair_transition))
+        m = self._modules
+        return ((m["outer_product_mean"], m["msa_attention1"], m["msa_transition"]),
+                (m["triangle_multiplication_outgoing"], m["triangle_multiplication_incoming"], m["pair_attention1"],
+                 m["pair_attention2"], m["pair_transition"]))
 
     @property
     def one_call(self) -> bool:
         """Whether the whole block runs as one call of the library (`native`)."""
-        (opm, att, transition), pair_track = self._tracks()
-        return (as_written(opm, OuterProductMean) and opm.native and as_written(att, MSAAttention) and att.native
-                and as_written(transition, Transition) and transition.narrow
-                and plain_pair_track(*pair_track, self.c_pair) and self.pair_attention1.fused)
+        (opm, att, transition), track = self._tracks()
+        return (as_written((opm, OuterProductMean), (att, MSAAttention), (transition, Transition)) and opm.native and att.native
+                and transition.narrow and plain_pair_track(*track, self.c_pair) and track[2].fused)
+
+    def _structures(self):
+        if self.one_call:
+            self.native()
 
     def native(self) -> "L.MsaBlockStruct":
         """The packed weights of the block's modules as the library's structure; made again when any of them has been
         packed again."""
-        msa_track, (tm, ta, transition) = self._tracks()
-        mods = (*msa_track, *tm, *ta, transition)
-        packs = [m.packed() for m in mods]
-        if self._native is not None and all(a is b for a, b in zip(self._native[1], packs)):
+        msa_track, track = self._tracks()
+        packs = packs_of(msa_track + track)
+        if self._native is not None and all(map(operator.is_, self._native[1], packs)):
             # (an attribute like any other, not a packed weight: as it is at the call)
             self._native[0].epsilon = self.outer_product_mean.epsilon
             return self._native[0]
@@ -258,7 +262,7 @@ class EvoformerBlock(HipModule):
               ("mt_w2", t["w2_64"], (64, s.mt_hidden)))
         p = L.PairformerBlockStruct()
         p.device = s.device
-        fill_pair_weights(p, tm, ta, transition, self.c_pair)
+        fill_pair_weights(p, *track, self.c_pair)
         s.pair = p
         self._native = (s, packs)
         return s
@@ -297,7 +301,7 @@ def evoformer_loop(blocks, msa, pair, msa_mask, pair_mask):
     """Run Evoformer blocks one after the other (d_alphafold3.py:228-231), in one call where they allow it."""
     blocks = list(blocks)
     if (not in_check_mode() and pair.is_cuda and len(blocks) > 1 and msa.is_contiguous() and pair.is_contiguous()
-            and _takes(msa, msa_mask) and all(as_written(b, EvoformerBlock) and b.one_call and
+            and _takes(msa, msa_mask) and all(as_written((b, EvoformerBlock)) and b.one_call and
                     b.outer_product_mean.epsilon == blocks[0].outer_product_mean.epsilon for b in blocks)):
         ops.evoformer_stack([b.native() for b in blocks], msa, pair, msa_mask, pair_mask)
         return msa, pair

@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import operator
 from typing import Optional
 
 import torch
@@ -10,20 +11,20 @@ import torch.nn as nn
 from .. import check, ops
 from .. import lib as L
 from .attention import GridSelfAttention
-from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pad_channels, pad_rows, point
+from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, packs_of, pad_channels, pad_rows, point
 from .diffusion_transformer import AdaLNZero, AdaptiveLayerNorm, SelfAttention
 from .primitives import Transition
 from .triangle_multiplication import TriangleMultiplication
 
 
-def plain_pair_track(tm, ta, transition, c_pair) -> bool:
+def plain_pair_track(tm_out, tm_in, ta_start, ta_end, transition, c_pair) -> bool:
     """Whether the five pair operators are what one call of the library does: the triangle multiplications (outgoing,
     incoming), the triangle attentions (starting, ending node) and the transition, all on `c_pair` channels."""
-    return (all(as_written(m, TriangleMultiplication) and m.c_pair == c_pair for m in tm)
-            and all(as_written(m, GridSelfAttention) and m.c_pair == c_pair for m in ta)
-            and as_written(transition, Transition) and transition.c_x == c_pair
-            and tm[0]._outgoing and not tm[1]._outgoing and not ta[0].transpose and ta[1].transpose
-            and ta[0].num_head == ta[1].num_head)
+    return (as_written((tm_out, TriangleMultiplication), (tm_in, TriangleMultiplication), (ta_start, GridSelfAttention),
+                       (ta_end, GridSelfAttention), (transition, Transition))
+            and c_pair == tm_out.c_pair == tm_in.c_pair == ta_start.c_pair == ta_end.c_pair == transition.c_x
+            and tm_out._outgoing and not tm_in._outgoing and not ta_start.transpose and ta_end.transpose
+            and ta_start.num_head == ta_end.num_head)
 
 
 def one_sequence(single, seq_mask) -> bool:
@@ -32,12 +33,11 @@ def one_sequence(single, seq_mask) -> bool:
     return single.dim() == 2 and (seq_mask is None or seq_mask.dim() == 1)
 
 
-def fill_pair_weights(s, tm, ta, transition, c_pair) -> None:
-    """The pair operators' packed weights into an af3_pairformer_block: triangle multiplications (outgoing, incoming),
-    triangle attentions (starting, ending node), pair transition."""
+def fill_pair_weights(s, tm_out, tm_in, ta_start, ta_end, transition, c_pair) -> None:
+    """The pair operators' packed weights into an af3_pairformer_block."""
     vec, mat = (128,), (128, 128)
-    for d in (0, 1):
-        p, q = tm[d].packed(), ta[d].packed()
+    for d, (tm, ta) in enumerate(((tm_out, ta_start), (tm_in, ta_end))):
+        p, q = tm.packed(), ta.packed()
         point(s, (("tm_ln_in_w", d), p["ln_in_w"], vec), (("tm_ln_in_b", d), p["ln_in_b"], vec),
               (("tm_ln_c_w", d), p["ln_c_w"], vec), (("tm_ln_c_b", d), p["ln_c_b"], vec),
               (("tm_w_proj_gate", d), p["w_proj_gate"], (4, 128, 128)), (("tm_w_out", d), p["w_out"], mat),
@@ -48,7 +48,7 @@ def fill_pair_weights(s, tm, ta, transition, c_pair) -> None:
     hidden = p["w2"].shape[1]
     point(s, ("pt_ln_w", p["ln_w"], vec), ("pt_ln_b", p["ln_b"], vec), ("pt_w1", p["w1"], (hidden // 64, 128, 128)),
           ("pt_w2", p["w2"], (128, hidden)))
-    s.valid_channels, s.num_head_pair, s.pair_hidden = c_pair, ta[0].num_head, hidden
+    s.valid_channels, s.num_head_pair, s.pair_hidden = c_pair, ta_start.num_head, hidden
 
 
 class PairformerBlock(HipModule):
@@ -88,8 +88,9 @@ class PairformerBlock(HipModule):
                     w_logits=pad_rows(bf16(self.single_pair_logits_projection.weight), 32))
 
     def _pair_track(self):
-        return ((self.triangle_multiplication_outgoing, self.triangle_multiplication_incoming),
-                (self.pair_attention1, self.pair_attention2), self.pair_transition)
+        m = self._modules
+        return (m["triangle_multiplication_outgoing"], m["triangle_multiplication_incoming"], m["pair_attention1"],
+                m["pair_attention2"], m["pair_transition"])
 
     @property
     def one_call(self) -> bool:
@@ -98,29 +99,35 @@ class PairformerBlock(HipModule):
         track = self._pair_track()
         if not plain_pair_track(*track, self.c_pair):
             return False
-        att = track[1][0]
+        att = track[2]
         if not self.with_single:
             return att.fused or att.padded
-        sa, st, c = self.single_attention_, self.single_transition, self.c_single
-        return (att.fused and c > 128 and as_written(sa, SelfAttention) and sa.c_x == c and sa.num_head == self.n_heads
-                and as_written(sa.adaptive_layernorm, AdaptiveLayerNorm) and not sa.adaptive_layernorm.use_single_cond
-                and as_written(sa.adaptive_zero_init, AdaLNZero) and not sa.adaptive_zero_init.use_single_cond
-                and as_written(st, Transition) and st.c_x == c)
+        sa, st, c = self._modules["single_attention_"], self._modules["single_transition"], self.c_single
+        if sa.__class__ is not SelfAttention:
+            return False
+        norm, out = sa._modules["adaptive_layernorm"], sa._modules["adaptive_zero_init"]
+        return (att.fused and c > 128
+                and as_written((sa, SelfAttention), (norm, AdaptiveLayerNorm), (out, AdaLNZero), (st, Transition))
+                and c == sa.c_x == st.c_x and sa.num_head == self.n_heads and not norm.use_single_cond and not out.use_single_cond)
+
+    def _structures(self):
+        if self.one_call:
+            self.native()
 
     def native(self) -> "L.PairformerBlockStruct":
         """The packed weights of the block's modules as the library's structure; made again when any of them has
         been packed again."""
-        tm, ta, transition = self._pair_track()
-        mods = (self, *tm, *ta, transition)
+        track = self._pair_track()
+        mods = (self, *track)
         if self.with_single:
-            sa, st = self.single_attention_, self.single_transition
-            mods += (sa, sa.adaptive_layernorm, sa.adaptive_zero_init, st)
-        packs = [m.packed() for m in mods]
-        if self._native is not None and all(a is b for a, b in zip(self._native[1], packs)):
+            sa, st = self._modules["single_attention_"], self._modules["single_transition"]
+            mods += (sa, sa._modules["adaptive_layernorm"], sa._modules["adaptive_zero_init"], st)
+        packs = packs_of(mods)
+        if self._native is not None and all(map(operator.is_, self._native[1], packs)):
             return self._native[0]
         by = dict(zip(mods, packs))
         s = L.PairformerBlockStruct()
-        fill_pair_weights(s, tm, ta, transition, self.c_pair)
+        fill_pair_weights(s, *track, self.c_pair)
         s.with_single = int(self.with_single)
         if self.with_single:
             c, p, a, o, t = self.c_single, by[self], by[sa], by[sa.adaptive_zero_init], by[st]
@@ -211,7 +218,7 @@ def pairformer_loop(blocks, pair, pair_mask, single, seq_mask, overlap_single: b
     side = _side_stream(pair.device)
     blocks = list(blocks)
     if blocks and one_sequence(single, seq_mask) and all(
-            as_written(b, PairformerBlock) and b.one_call and b.with_single and b.n_heads == blocks[0].n_heads
+            as_written((b, PairformerBlock)) and b.one_call and b.with_single and b.n_heads == blocks[0].n_heads
             and b.c_single == blocks[0].c_single for b in blocks):
         if not (pair.is_contiguous() and single.is_contiguous()):
             raise ValueError("pair and single must be contiguous (they are updated in place)")

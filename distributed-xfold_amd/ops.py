@@ -218,7 +218,7 @@ def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incomi
     io = _dt(pair)
     maskf = _mask_f32(pair_mask, (n, n), "mask")
     mask_in = _mask_f32(pair_mask_incoming, (n, n), "mask")
-    ws = _ws(max(lib.af3_pairformer_stack_workspace_bytes(n, b.num_head_pair) for b in blocks), dev)
+    ws = _ws(lib.af3_pairformer_stack_workspace_bytes(n, max(b.num_head_pair for b in blocks)), dev)
     seqf = logits = sws = None
     single_dt = 0
     if blocks[0].with_single:
@@ -396,7 +396,7 @@ def evoformer_stack(blocks, msa, pair, msa_mask, pair_mask):
     _gpu(pair, "pair", shape=(n, n, 128))
     pmf = _mask_f32(pair_mask, (n, n), "pair_mask")
     need = lib.af3_msa_workspace_bytes(rows, n)
-    pws = max(lib.af3_pairformer_stack_workspace_bytes(n, b.pair.num_head_pair) for b in blocks)
+    pws = lib.af3_pairformer_stack_workspace_bytes(n, max(b.pair.num_head_pair for b in blocks))
     split = (need + 255) // 256 * 256
     ws = _ws(split + pws, msa.device)
     ptrs = (ctypes.c_void_p * len(blocks))(*[ctypes.addressof(b) for b in blocks])

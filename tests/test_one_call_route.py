@@ -234,3 +234,25 @@ def test_an_index_tensor_that_was_written_to_is_checked_again(pkg):
         pkg.ops.rows_in_range(rows, 4)
     with torch.inference_mode():
         pkg.ops.rows_in_range(rows.clone(), 5)
+
+
+def test_foreign_modules_are_not_taken_for_the_usual_ones(pkg):
+    nn, foreign = pkg.nn, torch.nn.Identity
+    blk = nn.PairformerBlock()
+    for name in ("pair_attention1", "single_attention_", "single_transition", "pair_transition"):
+        other = nn.PairformerBlock()
+        setattr(other, name, foreign())
+        assert blk.one_call and not other.one_call
+    mod = nn.DiffusionTransformer(c_act=48, num_head=2, num_blocks=2, super_block_size=1)
+    assert mod._one_call(mod._blocks())
+    mod.transition_block[1] = foreign()
+    assert not mod._one_call(mod._blocks())
+
+
+@pytest.mark.parametrize("name", NATIVE)
+def test_packing_makes_the_structures_too(pkg, name):
+    mod, make = _small(pkg.nn, name)
+    mod.load_hip_params()
+    holder = mod.trunk_pairformer[0] if name == "PairformerStack" else mod
+    held = holder._native
+    assert held is not None and make(mod) is held[0]
