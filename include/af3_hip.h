@@ -510,7 +510,9 @@ int af3_pair_cond_init_forward(const void* pair, int pair_dtype, float in_scale,
  * and with join != 0 makes `stream` wait for single_stream at the end; with
  * join = 0 the caller does that before anything else touches `single` or the
  * scratch.  logits: 2 * num_head * n * roundup(n, 4) floats (one block: half of it), used on
- * both streams; single_workspace is used on single_stream only.
+ * both streams; single_workspace is used on single_stream only.  Both workspaces are as
+ * large as the block that needs most asks for, which is checked for every block before
+ * the first launch; num_head and c_single are the same in all blocks.
  */
 typedef struct af3_pairformer_block {
   /* af3_triangle_multiplication_forward: [0] outgoing, [1] incoming */
