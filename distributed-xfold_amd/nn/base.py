@@ -173,11 +173,7 @@ class HipModule(nn.Module):
         """The library's structures of a module that has such, made from the packed weights."""
 
     def load_hip_params(self):
-        mods = [m for m in self.modules() if isinstance(m, HipModule)]
-        for m in mods:
-            m._packed = m._pack()
-        for m in mods:
-            m._structures()
+        _pack_all(self)
         return self
 
     def packed(self):
@@ -196,12 +192,19 @@ class HipModule(nn.Module):
         return self.forward(*a, **k)
 
 
-def enable_hip(model: nn.Module) -> int:
-    """Counterpart of ModelRunner.enable_xsmm (run_inference.py:197-218): packs
-    the weights of every HIP module under `model`.  Returns how many were bound."""
+def _pack_all(model: nn.Module) -> int:
     mods = [m for m in model.modules() if isinstance(m, HipModule)]
     for m in mods:
         m._packed = m._pack()
     for m in mods:
-        m._structures()
+        try:
+            m._structures()
+        except ValueError:      # weights that do not go together: an error of the call that needs them, not of packing
+            pass
     return len(mods)
+
+
+def enable_hip(model: nn.Module) -> int:
+    """Counterpart of ModelRunner.enable_xsmm (run_inference.py:197-218): packs
+    the weights of every HIP module under `model`.  Returns how many were bound."""
+    return _pack_all(model)

@@ -82,10 +82,22 @@ class OuterProductMean(HipModule):
             d["w_lr"] = torch.cat([d["w_l"], d["w_r"]])
             rows = [(r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1) for r in range(32)]
             d["w_packed"] = d["w_out"].view(4, 32, 64, 2, 8)[:, rows].permute(0, 2, 3, 1, 4).contiguous()
-            s = d["block"] = L.MsaBlockStruct()
+        return d
+
+    def block(self) -> "L.MsaBlockStruct":
+        """The packed weights as the library's structure, epsilon as it is now (an attribute, not a weight)."""
+        d = self.packed()
+        if self._native is None or self._native[1] is not d:
+            s = L.MsaBlockStruct()
             point(s, ("opm_ln_w", d["ln_w"], (64,)), ("opm_ln_b", d["ln_b"], (64,)), ("opm_w_lr", d["w_lr"], (64, 64)),
                   ("opm_w_out", d["w_packed"], (4, 64, 2, 32, 8)), ("opm_b_out", d["b_out"], (128,)))
-        return d
+            self._native = (s, d)
+        self._native[0].epsilon = self.epsilon
+        return self._native[0]
+
+    def _structures(self):
+        if self.native:
+            self.block()
 
     @torch.no_grad()
     def run(self, msa, mask, residual: Optional[torch.Tensor] = None, block: int = 128):
@@ -95,8 +107,7 @@ class OuterProductMean(HipModule):
         co, cf = self.num_outer_channel, self.num_output_channel
         out = residual if residual is not None else torch.zeros((n, n, cf), dtype=torch.float32, device=msa.device)
         if self.native and _takes(msa, mask):
-            p["block"].epsilon = self.epsilon
-            return ops.outer_product_mean(p["block"], msa.contiguous(), mask, out, True)
+            return ops.outer_product_mean(self.block(), msa.contiguous(), mask, out, True)
         m = mask.float()
         x = ops.layer_norm(msa.contiguous(), p["ln_w"], p["ln_b"])
         mb = m[..., None].to(torch.bfloat16)
@@ -151,24 +162,33 @@ class MSAAttention(HipModule):
         return self.c_msa == 64 and self.num_head == 8
 
     def _pack(self):
-        d = dict(ln_w=f32(self.act_norm.weight), ln_b=f32(self.act_norm.bias),
+        return dict(ln_w=f32(self.act_norm.weight), ln_b=f32(self.act_norm.bias),
                     pn_w=f32(self.pair_norm.weight), pn_b=f32(self.pair_norm.bias),
                     w_logits=pad_rows(bf16(self.pair_logits.weight), 32), w_v=bf16(self.v_projection.weight),
                     w_g=bf16(self.gating_query.weight), w_o=bf16(self.output_projection.weight))
-        if self.native:
-            s = d["block"] = L.MsaBlockStruct()
+
+    def block(self) -> "L.MsaBlockStruct":
+        """The packed weights as the library's structure."""
+        d = self.packed()
+        if self._native is None or self._native[1] is not d:
+            s = L.MsaBlockStruct()
             point(s, ("ma_ln_w", d["ln_w"], (64,)), ("ma_ln_b", d["ln_b"], (64,)), ("ma_pn_w", d["pn_w"], (128,)),
                   ("ma_pn_b", d["pn_b"], (128,)), ("ma_w_logits", d["w_logits"], (32, 128)),
                   *((f"ma_{k}", d[k], (64, 64)) for k in ("w_v", "w_g", "w_o")))
             s.epsilon = 1.0      # (of a coverage that this operator does not use)
-        return d
+            self._native = (s, d)
+        return self._native[0]
+
+    def _structures(self):
+        if self.native:
+            self.block()
 
     @torch.no_grad()
     def run(self, msa, msa_mask, pair, residual: bool):
         p = self.packed()
         a, n, c = msa.shape
         if self.native and _takes(msa, msa_mask):
-            return ops.msa_attention(p["block"], msa.contiguous(), msa_mask, pair.contiguous(), residual)
+            return ops.msa_attention(self.block(), msa.contiguous(), msa_mask, pair.contiguous(), residual)
         h, d = self.num_head, self.value_dim
         x = ops.layer_norm(msa.contiguous(), p["ln_w"], p["ln_b"])
         logits = ops.pair_logits(pair.contiguous(), p["pn_w"], p["pn_b"], p["w_logits"], h)     # [h, q, k] fp32
@@ -248,7 +268,7 @@ class EvoformerBlock(HipModule):
             self._native[0].epsilon = self.outer_product_mean.epsilon
             return self._native[0]
         s = L.MsaBlockStruct()
-        for prefix, src in (("opm_", packs[0]["block"]), ("ma_", packs[1]["block"])):
+        for prefix, src in (("opm_", msa_track[0].block()), ("ma_", msa_track[1].block())):
             if s.device not in (None, src.device):
                 raise ValueError(f"weights of the block on {s.device} and on {src.device}")
             s.device = src.device

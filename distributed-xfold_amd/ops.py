@@ -63,9 +63,10 @@ def _gpu(t: torch.Tensor, name: str, dtype=None, shape=None) -> torch.Tensor:
 
 
 def _weights_with(t: torch.Tensor, *blocks):
-    """The structures of packed weights hold addresses: they must be of the activations' device."""
+    """The structures of packed weights hold addresses: they must be of the activations' device.  (None: a structure that
+    no module has made, whose maker answers for it.)"""
     for b in blocks:
-        if b.device != t.device:
+        if b.device is not None and b.device != t.device:
             raise ValueError(f"weights: live on {b.device}, the activations on {t.device}")
 
 

@@ -64,6 +64,8 @@ def test_packed_modules_can_be_copied_and_stored(pkg, name):
         assert all(torch.equal(a, b) for a, b in zip(mod.parameters(), other.parameters()))
         own, others = bytes(make(mod)), bytes(make(other))
         assert own != others          # the copy's structures point at weights of its own
+    mod.__setstate__(dict(mod.__dict__, _packed={"of": "another version"}))
+    assert mod._packed is None and mod._native is None
 
 
 @pytest.mark.parametrize("name", NATIVE)
@@ -201,7 +203,8 @@ def test_weights_of_another_shape_are_refused(pkg, name, layer, widths):
     mod, make = _small(pkg.nn, name)
     parent, _, leaf = layer.rpartition(".")
     setattr(mod.get_submodule(parent), leaf, torch.nn.Linear(*widths, bias=False))
-    with pytest.raises(ValueError, match="expected a contiguous|of size|invalid for input"):
+    mod.load_hip_params()                    # (packing is no use of the weights)
+    with pytest.raises(ValueError, match="expected a contiguous"):
         make(mod)
 
 
