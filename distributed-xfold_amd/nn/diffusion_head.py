@@ -326,9 +326,11 @@ class DiffusionSampler:
         for i in range(self.diffusion_steps):
             rot = rotations[i] if rotations is not None else random_rotation(generator, dev)
             trans = translations[i] if translations is not None else torch.randn(3, generator=generator, device=dev)
-            if noises is not None or self.gaussian_noise:
+            if noises is not None or self.gaussian_noise or trans.numel() != 3:
                 positions = random_augmentation(positions, mask[None], rot.float(), trans.float())
-                noise = noises[i] if noises is not None else torch.randn(positions.shape, generator=generator, device=dev)
+                noise = 1.0
+                if noises is not None or self.gaussian_noise:
+                    noise = noises[i] if noises is not None else torch.randn(positions.shape, generator=generator, device=dev)
                 noisy = positions + nscale[i] * noise
             else:   # random_augmentation, and the step's scalar of noise added
                 center = (m * positions).sum(dim=(-2, -3), keepdim=True) / count

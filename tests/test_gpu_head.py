@@ -389,3 +389,16 @@ def test_a_noise_level_per_sample(gpu_pkg):
     for i in range(2):
         assert torch.equal(got[i], head(noisy, levels[i], gb, ge, sc[0], pc)[i])
     assert not torch.equal(got[1], head(noisy, levels[0], gb, ge, sc[0], pc)[1])
+
+
+def test_a_translation_per_sample(gpu_pkg):
+    """Translations [steps, samples, 1, 1, 3]: each sample is moved by its own."""
+    g, batch, _, emb, pos, head = case(gpu_pkg, 12, 1, seed=78)
+    gb, ge = batch.to(dev()), on_gpu(emb)
+    trans, rot = torch.randn(2, 2, 1, 1, 3, generator=g).to(dev()), torch.linalg.qr(torch.randn(2, 3, 3, generator=g))[0].to(dev())
+    sampler = gpu_pkg.nn.DiffusionSampler(head, num_samples=2, diffusion_steps=2)
+    run = lambda t: sampler(gb, ge, positions=pos.to(dev()), rotations=rot, translations=t)["atom_positions"]
+    got = run(trans)
+    for i in range(2):
+        compare(f"sample {i}", got[i], run(trans[:, i, 0, 0])[i], 1e-4, 1e-3)
+    assert not torch.allclose(got[0], run(trans[:, 1, 0, 0])[0], rtol=1e-3, atol=1e-3)
