@@ -11,6 +11,8 @@ non-zero return code into a RuntimeError.  No arithmetic happens here.
 from __future__ import annotations
 
 import ctypes
+import functools
+import threading
 from typing import Optional
 
 import torch
@@ -18,12 +20,24 @@ import torch
 from . import lib as _L
 
 _workspaces: dict = {}
+_enqueuing = threading.RLock()
+
+
+def _uses_scratch(op):
+    """One such operator at a time: a stream's scratch is shared by all threads that work on the stream, and the library
+    call, which enqueues several kernels around it, lets other threads run."""
+    @functools.wraps(op)
+    def alone(*args, **kwargs):
+        with _enqueuing:
+            return op(*args, **kwargs)
+    return alone
 
 
 def _ws(nbytes: int, device, stream=None) -> torch.Tensor:
     """Scratch buffer per device and stream, grown on demand and reused between
-    calls (calls on one stream are ordered, so reuse is safe; calls on different
-    streams may run at the same time and get different buffers).  `stream`: a
+    calls (calls on one stream are ordered, one after the other even from several
+    threads, see _uses_scratch, so reuse is safe; calls on different streams may
+    run at the same time and get different buffers).  `stream`: a
     torch stream other than the current one that the scratch is used on."""
     if stream is not None:
         with torch.cuda.stream(stream):
@@ -89,6 +103,7 @@ def _mask_f32(mask: Optional[torch.Tensor], shape, name: str):
 
 
 # --------------------------------------------------------------------------
+@_uses_scratch
 def triangle_multiplication(act, mask, equation_flag, left_norm_input_weight, left_norm_input_bias,
                             w_proj_gate, center_norm_weight, center_norm_bias,
                             w_output_projection, w_gating_linear, residual=False, out=None, valid_channels=128):
@@ -130,6 +145,7 @@ def triangle_multiplication(act, mask, equation_flag, left_norm_input_weight, le
     return out
 
 
+@_uses_scratch
 def grid_self_attn(pair, mask, transpose, act_norm_weight, act_norm_bias, w_pair_bias, nonbatched_bias,
                    w_qkvg, w_output, num_head, residual=False, out=None, valid_channels=128):
     """grid_self_attn_forward (csrc/Alpha_Attention.cpp:50-70) fused with the steps
@@ -206,6 +222,7 @@ def transition128(act, layernorm_weight, layernorm_bias, w1_packed, w2, residual
     return out
 
 
+@_uses_scratch
 def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incoming=None, single_stream=None, join=True):
     """A run of Pairformer blocks in one call (af3_pairformer_stack_forward), pair [N, N, 128] and single [N, c]
     updated in place.  `blocks`: af3_pairformer_block structures (nn.PairformerBlock.native()); `single_stream`: a
@@ -342,6 +359,7 @@ def _msa_inputs(msa, msa_mask):
     return _dt(msa), _mask_f32(msa_mask, tuple(msa.shape[:2]), "msa_mask")
 
 
+@_uses_scratch
 def outer_product_mean(block, msa, msa_mask, pair, residual):
     """af3_outer_product_mean_forward into `pair` [N, N, 128]; `block`: an af3_msa_block structure."""
     lib = _L.load()
@@ -356,6 +374,7 @@ def outer_product_mean(block, msa, msa_mask, pair, residual):
     return pair
 
 
+@_uses_scratch
 def msa_attention(block, msa, msa_mask, pair, residual):
     """af3_msa_attention_forward -> `msa` updated in place (residual) or a new tensor."""
     lib = _L.load()
@@ -388,6 +407,7 @@ def transition64(x, ln_weight, ln_bias, w1, w2, residual):
     return out
 
 
+@_uses_scratch
 def evoformer_stack(blocks, msa, pair, msa_mask, pair_mask):
     """A run of Evoformer blocks in one call, msa [rows, N, 64] and pair [N, N, 128] updated in place."""
     lib = _L.load()
@@ -406,6 +426,7 @@ def evoformer_stack(blocks, msa, pair, msa_mask, pair_mask):
     _L.check(rc, "af3_evoformer_stack_forward")
 
 
+@_uses_scratch
 def diffusion_transformer(blocks, act, mask, pair_logits, scale_shift, gate, num_head, hidden):
     """The blocks of the diffusion transformer in one call (af3_diffusion_transformer_forward), act [B, S, C] updated
     in place.  `blocks`: an array of lib.DiffusionBlockStruct; pair_logits: one fp32 tensor per block, [H, S, S] or
@@ -434,6 +455,7 @@ def diffusion_transformer(blocks, act, mask, pair_logits, scale_shift, gate, num
     return act
 
 
+@_uses_scratch
 def atom_transformer(blocks, act, key_rows, mask_q, mask_k, pair_logits, scale_shift_q, scale_shift_k, gate, num_head,
                      hidden):
     """The blocks of the windowed atom transformer in one call (af3_atom_transformer_forward), act
@@ -461,6 +483,7 @@ def atom_transformer(blocks, act, key_rows, mask_q, mask_k, pair_logits, scale_s
     return act
 
 
+@_uses_scratch
 def batch_diffusion_self_attention(q_data, key_mask, nonbatched_bias, w_qkvg, query_b, num_head,
                                    out_dtype=torch.bfloat16, out=None, static_scratch=False):
     """batch_diffusion_self_attention_forward (csrc/Alpha_Attention.cpp:72-92).
@@ -624,6 +647,7 @@ def quad_major_bias(bias):
     return bias.reshape(lead + (sq, sk // 4, 4)).permute(*range(k), k + 1, k, k + 2).contiguous()
 
 
+@_uses_scratch
 def batch_diffusion_cross_attention(q_data, m_data, pair_logits, mask_q, mask_k, w_qg, w_kv, query_b,
                                     num_head, out_dtype=torch.bfloat16):
     """batch_diffusion_cross_attention_forward (csrc/Alpha_Attention.cpp:127-146).
@@ -664,6 +688,7 @@ def batch_diffusion_cross_attention(q_data, m_data, pair_logits, mask_q, mask_k,
     return out
 
 
+@_uses_scratch
 def gathered_cross_attention(q_data, atom_data, key_rows, pair_logits, mask_q, mask_k, w_qg, w_kv, query_b,
                              num_head, out_dtype=torch.bfloat16):
     """The cross-attention above with the key windows looked up inside the

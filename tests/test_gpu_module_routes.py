@@ -1,6 +1,8 @@
 """Runs of modules that go to the library as one call, against the same modules one by one: what a user has put between
 them (forward hooks, a sub-module of another class) has its effect, and the results are the ones of the single call."""
 
+import threading
+
 import pytest
 import torch
 
@@ -246,3 +248,26 @@ def test_single_calls_under_capture(gpu_pkg):
             graph.replay()
             torch.cuda.synchronize()
             assert all(torch.equal(a, b) for a, b in zip(out, want)), (fn.__name__, i)
+
+
+def test_two_threads_on_one_stream(gpu_pkg):
+    """Their runs of blocks share the stream's scratch: one is enqueued whole, then the other."""
+    stack = on_gpu(gpu_pkg.nn.PairformerStack(num_blocks=3))
+    stack.load_hip_params()
+    cases = [trunk_inputs(n) for n in (37, 50)]
+    run = lambda c: stack(c[0].clone(), c[1], c[2].clone(), c[3])
+    want, got = [run(c) for c in cases], [[], []]
+    start = threading.Barrier(2)
+
+    def work(i):
+        start.wait()
+        for _ in range(20):
+            got[i].append(run(cases[i]))
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert len(got[i]) == 20 and all(torch.equal(a, b) for out in got[i] for a, b in zip(out, want[i]))

@@ -4,7 +4,11 @@ must not be made for.  Host side only (the operator layer is replaced by recorde
 import copy
 import ctypes
 import gc
+import inspect
 import io
+import re
+import threading
+import time
 import weakref
 
 import pytest
@@ -259,3 +263,24 @@ def test_packing_makes_the_structures_too(pkg, name):
     holder = mod.trunk_pairformer[0] if name == "PairformerStack" else mod
     held = holder._native
     assert held is not None and make(mod) is held[0]
+
+
+def test_operators_with_scratch_run_one_at_a_time(pkg):
+    """Two threads on one stream share its scratch."""
+    inside, worst = [], []
+
+    @pkg.ops._uses_scratch
+    def op():
+        inside.append(1)
+        worst.append(len(inside))
+        time.sleep(0.002)
+        inside.pop()
+    threads = [threading.Thread(target=lambda: [op() for _ in range(10)]) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(worst) == 40 and max(worst) == 1
+    source = inspect.getsource(pkg.ops)
+    users = re.findall(r"^(@_uses_scratch\n)?def (\w+)\((?:(?!^def ).)*? = _ws\(", source, flags=re.M | re.S)
+    assert len(users) >= 11 and all(mark for mark, name in users), users
