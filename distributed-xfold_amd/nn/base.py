@@ -83,15 +83,14 @@ def pack_swiglu(w1: torch.Tensor, block: int) -> torch.Tensor:
 
 
 def point(s, *fields) -> None:
-    """Set address fields of a library structure from packed weights: (field or (field, index), tensor, shape), vectors
-    fp32 and matrices bf16.  The structures carry neither sizes nor types, so what the operator layer checks of every
-    tensor is checked here: type, shape, contiguity and one device for all, which is kept as `s.device` for the operator
-    layer to compare with the activations'."""
+    """Set address fields of a library structure from packed weights: (field or (field, index), tensor, shape).  The
+    structures carry no sizes, so what the operator layer checks of every tensor and packing does not settle (it makes
+    contiguous tensors of the types that the library takes) is checked here: the shape, and one device for all, which is
+    kept as `s.device` for the operator layer to compare with the activations'."""
     device = s.device
     for name, t, shape in fields:
-        if t.shape != shape or t.dtype != (torch.float32 if len(shape) == 1 else torch.bfloat16) or not t.is_contiguous():
-            raise ValueError(f"{name}: expected a contiguous {'fp32' if len(shape) == 1 else 'bf16'} weight {shape}, got "
-                             f"{t.dtype} {tuple(t.shape)}")
+        if t.shape != shape:
+            raise ValueError(f"{name}: expected a weight {shape}, got {tuple(t.shape)}")
         if t.device != device:
             if device is not None:
                 raise ValueError(f"{name}: on {t.device}, other weights of the block on {device}")

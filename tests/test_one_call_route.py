@@ -208,8 +208,23 @@ def test_weights_of_another_shape_are_refused(pkg, name, layer, widths):
     parent, _, leaf = layer.rpartition(".")
     setattr(mod.get_submodule(parent), leaf, torch.nn.Linear(*widths, bias=False))
     mod.load_hip_params()                    # (packing is no use of the weights)
-    with pytest.raises(ValueError, match="expected a contiguous"):
+    with pytest.raises(ValueError, match="expected a weight"):
         make(mod)
+
+
+def test_packed_weights_are_contiguous_and_of_the_librarys_types(pkg):
+    """What the structures take for granted of every address."""
+    nn = pkg.nn
+    for mod in (nn.PairformerBlock(), nn.PairformerBlock(c_pair=64, num_intermediate_factor=2, with_single=False),
+                nn.EvoformerBlock(), nn.DiffusionTransformer(c_act=48, num_head=2, num_blocks=1, super_block_size=1),
+                nn.DiffusionCrossAttTransformer(num_blocks=1)):
+        mod.half()                               # (whatever the parameters are)
+        mod.load_hip_params()
+        for m in mod.modules():
+            for k, t in (getattr(m, "_packed", None) or {}).items():
+                for t in t if isinstance(t, list) else [t]:
+                    want = torch.float32 if t.dim() == 1 or k == "w_f32" else torch.bfloat16
+                    assert t.dtype == want and t.is_contiguous(), (type(m).__name__, k, t.dtype)
 
 
 def test_weights_on_another_device_are_refused(pkg):
