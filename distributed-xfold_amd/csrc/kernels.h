@@ -50,7 +50,7 @@ struct XcdWalk {
 // saves (1920 x 768 x 1536 in 64 x 64 tiles: 48 tiles against 45, 16.8 us against 15.4), and a whole round where the
 // even deal just fits: 33 tiles against 32 on one XCD (5300 x 768 x 1536 with gate and residual in 128 x 128 tiles 35.9 us,
 // even 23.8; 3900 x 3072 x 768 in 192 x 256 tiles 42.0, even 27.4, with SwiGLU 32.3 and 22.0).
-// 3840 x 768 x 768 14.3 -> 12.4 us, 3840 x 768 x 1536 24.1 -> 22.0, 3200 x 768 x 1536 22.9 -> 20.5.
+// 3840 x 768 x 768 14.3 -> 12.4 us, 3840 x 768 x 1536 24.1 -> 22.0.
 constexpr int XCD_CUS = 32;
 inline XcdWalk xcd_walk(int64_t tiles_m, int64_t tiles_n, int64_t batch, int bm, int bn, int64_t per_round) {
   XcdWalk w;
