@@ -66,6 +66,28 @@ void* static_scratch_ptr() {
 
 }  // namespace
 
+// The N x N x N contraction of the triangle multiplication: the 256x256-tile
+// kernel once a token count fills at least part of a second 128-row tile,
+// the general GEMM below that.
+static int contraction(const GemmArgs& g, hipStream_t s) {
+  if (g.M > 128 && contract_supported(g)) return launch_contract(g, s);
+  return launch_gemm_nt(g, s);
+}
+
+int run_triangle_contraction(const bf16_t* a_buf, const bf16_t* b_buf, bf16_t* t_buf, int n, int valid_channels, int outgoing, hipStream_t s) {
+  // outgoing: t[c][i][j] = sum_k a'[c][i][k] b'[c][j][k]
+  // incoming: t[c][i][j] = sum_k b'[c][i][k] a'[c][j][k]  (a', b' stored transposed by the prologue)
+  GemmArgs g;
+  g.A = outgoing ? a_buf : b_buf;
+  g.B = outgoing ? b_buf : a_buf;
+  g.C = t_buf;
+  // (the hidden layer has as many channels as the pair tensor: the padded ones are zero and are left out)
+  g.M = g.N = n; g.K = (int)pad8(n); g.batch = valid_channels;
+  g.lda = g.ldb = g.ldc = pad8(n);
+  g.sA = g.sB = g.sC = tri_plane(n);
+  return contraction(g, s);
+}
+
 extern "C" {
 
 int af3_abi_version(void) { return AF3_ABI_VERSION; }
@@ -83,14 +105,6 @@ const char* af3_error_string(int code) {
 }
 
 // ------------------------------------------------------ triangle multiplication
-// The N x N x N contraction of the triangle multiplication: the 256x256-tile
-// kernel once a token count fills at least part of a second 128-row tile,
-// the general GEMM below that.
-static int contraction(const GemmArgs& g, hipStream_t s) {
-  if (g.M > 128 && contract_supported(g)) return launch_contract(g, s);
-  return launch_gemm_nt(g, s);
-}
-
 size_t af3_triangle_multiplication_workspace_bytes(int64_t n) {
   if (n <= 0) return 0;
   return 3 * align_up((size_t)C_PAIR * tri_plane(n) * sizeof(bf16_t), 256);
@@ -127,17 +141,7 @@ static int triangle_multiplication_impl(
   int rc = launch_trimul_prologue(a, s);
   if (rc) return rc;
 
-  // outgoing: t[c][i][j] = sum_k a'[c][i][k] b'[c][j][k]
-  // incoming: t[c][i][j] = sum_k b'[c][i][k] a'[c][j][k]  (a', b' stored transposed by the prologue)
-  GemmArgs g;
-  g.A = a.outgoing ? a_buf : b_buf;
-  g.B = a.outgoing ? b_buf : a_buf;
-  g.C = t_buf;
-  // (the hidden layer has as many channels as the pair tensor: the padded ones are zero and are left out)
-  g.M = g.N = (int)n; g.K = (int)np; g.batch = valid_channels;
-  g.lda = g.ldb = g.ldc = np;
-  g.sA = g.sB = g.sC = plane;
-  rc = contraction(g, s);
+  rc = run_triangle_contraction(a_buf, b_buf, t_buf, (int)n, valid_channels, a.outgoing, s);
   if (rc) return rc;
   return launch_trimul_epilogue(a, s);
 }

@@ -355,6 +355,43 @@ struct TriAttnArgs {
 };
 int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream);
 
+// --------------------------------------------------------------- pair_step.hip
+// One run of per-pixel operators between two long products (contraction, attention core), in place on `pair`.
+enum {
+  PAIR_STEP_INCOMING,       // outgoing epilogue, incoming prologue
+  PAIR_STEP_PROJECT_START,  // incoming epilogue, starting-node projections
+  PAIR_STEP_PROJECT_END,    // starting-node output, ending-node projections
+  PAIR_STEP_LAST,           // ending-node output, transition (and pair logits)
+  PAIR_STEP_NEXT,           // the same, and the outgoing prologue of the block that follows
+};
+constexpr int PAIR_STEP_MAX_HIDDEN = 512;  // hidden units of the transition
+struct PairStepArgs {
+  LnWidth lw;
+  int valid_c = 128, io_f32 = 0, N = 0, Np = 0, ldn = 0, hidden = 0, logit_heads = 0;
+  int64_t plane = 0;
+  void* pair = nullptr;
+  // f_*: weights in fragment order (pair_frags of af3_pairformer_block)
+  const float *ln1_w = nullptr, *ln1_b = nullptr;  // gate and output projection of the operator before
+  const bf16_t *f_gate = nullptr, *f_out = nullptr;
+  const float *ln_c_w = nullptr, *ln_c_b = nullptr;
+  const bf16_t *t_buf = nullptr, *og = nullptr;
+  const float *ln2_w = nullptr, *ln2_b = nullptr;  // transition
+  const bf16_t *f_w1 = nullptr, *f_w2 = nullptr;
+  const float *ln3_w = nullptr, *ln3_b = nullptr;  // prologue or projections of the operator behind
+  const bf16_t *f_next = nullptr, *f_bias = nullptr;
+  const float* mask = nullptr;                     // prologue
+  bf16_t *a_buf = nullptr, *b_buf = nullptr;
+  bf16_t *q = nullptr, *k = nullptr, *vt = nullptr;
+  uint16_t* bias = nullptr;
+  float q_scale = 1.f, bias_scale = 1.f;
+  const float *sl_ln_w = nullptr, *sl_ln_b = nullptr;  // pair logits of the single track, or none
+  const bf16_t* f_logits = nullptr;
+  float* logits = nullptr;
+};
+int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s);
+// the long product of a triangle multiplication, between the planes of its prologue and its epilogue (api.hip)
+int run_triangle_contraction(const bf16_t* a_buf, const bf16_t* b_buf, bf16_t* t_buf, int n, int valid_channels, int outgoing, hipStream_t s);
+
 // -------------------------------------------------------------------- embed.hip
 struct PairEmbedArgs {
   const float* lr = nullptr;    // [n][ld_lr]: left projection, then right

@@ -269,22 +269,28 @@ __global__ __launch_bounds__(256, 2) void trimul_epilogue_kernel(TriMulArgs a) {
     const int j = lane & 31, hh = lane >> 5;
     const int px = wave * 32 + j;
     const int xaddr = half_swap_addr();
-    float v[8][8];
-    float s1 = 0.f;
+    float v[8][8], part[8];
+    // (sums over the eight channels of a k-step, then over the k-steps, then over the halves of the wave, in the order of
+    // pair_step.hip, whose threads hold eight channels each)
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks)
+    for (int ks = 0; ks < 8; ++ks) {
+      part[ks] = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         v[ks][e] = bf2f(sT[(16 * ks + 8 * hh + e) * LDX + px]);
-        s1 += v[ks][e];
+        part[ks] += v[ks][e];
       }
+    }
+    float s1 = sum_k_steps(part);
     s1 += half_swap(xaddr, s1);
     const float mean = s1 * a.lw.inv_c;
-    float s2 = 0.f;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks)
+    for (int ks = 0; ks < 8; ++ks) {
+      part[ks] = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) { const float d = v[ks][e] - mean; s2 += d * d; }
+      for (int e = 0; e < 8; ++e) { const float d = v[ks][e] - mean; part[ks] = fmaf(d, d, part[ks]); }
+    }
+    float s2 = sum_k_steps(part);
     s2 += half_swap(xaddr, s2);
     const float rstd = rsqrtf((s2 - a.lw.pad * mean * mean) * a.lw.inv_c + LN_EPS);
     const bool ok = t.valid(px);

@@ -10,6 +10,7 @@
 namespace {
 
 inline size_t align_up(size_t v) { return (v + 255) / 256 * 256; }
+inline int64_t up8(int64_t v) { return (v + 7) / 8 * 8; }
 
 // bump allocator over the caller's workspace
 struct Carver {
@@ -26,14 +27,24 @@ struct Carver {
   }
 };
 
-// `waiter` waits for everything enqueued on `on` so far.  The event lives only for the two calls: the runtime keeps
-// what a pending wait needs.
-int order_streams(hipStream_t on, hipStream_t waiter) {
-  hipEvent_t e;
-  if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return AF3_ERR_LAUNCH;
-  const bool ok = hipEventRecord(e, on) == hipSuccess && hipStreamWaitEvent(waiter, e, 0) == hipSuccess;
-  return hipEventDestroy(e) == hipSuccess && ok ? AF3_OK : AF3_ERR_LAUNCH;
-}
+// `waiter` waits for everything enqueued on `on` so far.  An event may be recorded again while waits for its earlier
+// recordings are pending, and be destroyed after that: the runtime keeps what a pending wait needs.  (Creating and
+// destroying one costs the host as much as a launch: once a call, not once a block.)
+struct Event {
+  hipEvent_t e = nullptr;
+  ~Event() {
+    if (e) (void)hipEventDestroy(e);
+  }
+  int record(hipStream_t on) {
+    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return AF3_ERR_LAUNCH;
+    return hipEventRecord(e, on) == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+  }
+  int wait(hipStream_t waiter) { return !e || hipStreamWaitEvent(waiter, e, 0) == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH; }
+  int order(hipStream_t on, hipStream_t waiter) {
+    const int rc = record(on);
+    return rc != AF3_OK ? rc : wait(waiter);
+  }
+};
 
 #define STEP(call)               \
   do {                           \
@@ -53,6 +64,97 @@ int pair_operators(const af3_pairformer_block& b, void* pair, int dt, const floa
                                            wsb, s));
   return af3_transition_forward_padded(pair, dt, b.pt_ln_w, b.pt_ln_b, b.pt_w1, b.pt_w2, b.pair_hidden, pair, 1, n * n,
                                        b.valid_channels, s);
+}
+
+// ---- the pair operators at few tokens: a run of them between two long products in one kernel (pair_step.hip) ----
+// A step takes the chain of one tile of 32 positions where a kernel of its own per operator takes several of tiles of 128,
+// and eight launches a block take the place of fourteen; past some number of tiles what every tile fetches of the weights
+// costs more than that saves.  Runs of 4 blocks, us a block, one kernel per operator -> steps (bf16 / fp32 stream):
+//   64 tokens 136 -> 92 / 143 -> 91,  128: 166 -> 124 / 173 -> 123,  160: 205 -> 179 / 213 -> 182,
+//   208: 286 -> 268 / 306 -> 279,  224: 265 -> 264 / 283 -> 275,  256: 287 -> 288 / 323 -> 302
+constexpr int64_t PAIR_STEP_POSITIONS = 208 * 208;
+bool pair_steps_apply(const af3_pairformer_block& b, int64_t n) {
+  return b.pair_frags && n <= 8192 && n * tri_ldn(n) <= PAIR_STEP_POSITIONS && b.num_head_pair == 4 && b.valid_channels >= 8 &&
+         b.valid_channels <= 128 && b.valid_channels % 4 == 0 && b.pair_hidden > 0 && b.pair_hidden % 64 == 0 &&
+         b.pair_hidden <= PAIR_STEP_MAX_HIDDEN;
+}
+// Scratch.  q, k and the operands of the contraction are never alive together, nor are its result and the attention's.
+struct PairStepScratch {
+  bf16_t *qa = nullptr, *kb = nullptr, *vt = nullptr, *ogt = nullptr;
+  uint16_t* bias = nullptr;
+  static size_t plane_bytes(int64_t n) { return (size_t)128 * tri_plane(n) * 2; }  // (tri_plane(n) >= n n)
+  static size_t bytes(int64_t n) {
+    return 3 * align_up(plane_bytes(n)) + align_up((size_t)n * 128 * tri_ldn(n) * 2) + align_up((size_t)tri_bias_elems(n, 4) * 2);
+  }
+  bool carve(int64_t n, void* ws, size_t wsb) {
+    Carver w(ws, wsb);
+    qa = static_cast<bf16_t*>(w.take(plane_bytes(n)));
+    kb = static_cast<bf16_t*>(w.take(plane_bytes(n)));
+    ogt = static_cast<bf16_t*>(w.take(plane_bytes(n)));
+    vt = static_cast<bf16_t*>(w.take((size_t)n * 128 * tri_ldn(n) * 2));
+    bias = static_cast<uint16_t*>(w.take((size_t)tri_bias_elems(n, 4) * 2));
+    return w.ok;
+  }
+};
+
+// One block's pair operators.  `first`: no step before has made the outgoing prologue.  `next`: the block whose outgoing
+// prologue the last step makes, or null.  `logits`: where the pair logits of the single track go, or null; they are
+// written behind `logits_free`.
+int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_block* next, bool first, void* pair, int dt,
+                            const float* mask, const float* mask_in, int64_t n, void* ws, size_t wsb, float* logits,
+                            Event* logits_free, hipStream_t s) {
+  if (!pair || (dt != AF3_F32 && dt != AF3_BF16) || ((uintptr_t)pair & 15) || ((uintptr_t)mask & 15) || ((uintptr_t)mask_in & 15))
+    return AF3_ERR_BAD_ARG;
+  PairStepScratch w;
+  if (!w.carve(n, ws, wsb)) return AF3_ERR_WORKSPACE;
+  const int c = b.valid_channels, hidden = b.pair_hidden;
+  PairStepArgs a;
+  a.lw = ln_width(c);
+  a.valid_c = c; a.io_f32 = dt == AF3_F32; a.N = (int)n; a.Np = (int)up8(n); a.ldn = (int)tri_ldn(n); a.plane = tri_plane(n);
+  a.pair = pair; a.hidden = hidden;
+  a.t_buf = a.og = w.ogt; a.a_buf = a.q = w.qa; a.b_buf = a.k = w.kb; a.vt = w.vt; a.bias = w.bias;
+  a.bias_scale = 1.4426950408889634f;  // base-2 logits, as grid_self_attn_impl
+  a.q_scale = a.bias_scale / sqrtf((float)(c / 4));
+  // pair_frags, in rows of 128
+  auto tm = [&](const af3_pairformer_block& x, int d, int row) { return x.pair_frags + (d * 768 + row) * 128; };
+  auto ta = [&](int d, int row) { return b.pair_frags + (1536 + d * 672 + row) * 128; };
+  const uint16_t* w1 = b.pair_frags + 2880 * 128;
+  TriAttnArgs core;
+  core.q = w.qa; core.k = w.kb; core.vt = w.vt; core.bias = w.bias; core.mask = mask; core.og = w.ogt; core.N = (int)n; core.ldn = a.ldn;
+
+  if (first) {
+    TriMulArgs p;
+    p.lw = a.lw; p.valid_c = c; p.pair = pair; p.mask = mask; p.io_f32 = a.io_f32; p.N = a.N; p.Np = a.Np; p.plane = a.plane;
+    p.ln_in_w = b.tm_ln_in_w[0]; p.ln_in_b = b.tm_ln_in_b[0]; p.w_pg = b.tm_w_proj_gate[0];
+    p.a_buf = w.qa; p.b_buf = w.kb;
+    STEP(launch_trimul_prologue(p, s));
+  }
+  for (int d = 0; d < 2; ++d) {
+    STEP(run_triangle_contraction(w.qa, w.kb, w.ogt, (int)n, c, d == 0, s));
+    a.ln1_w = b.tm_ln_in_w[d]; a.ln1_b = b.tm_ln_in_b[d]; a.f_gate = tm(b, d, 0); a.f_out = tm(b, d, 128);
+    a.ln_c_w = b.tm_ln_c_w[d]; a.ln_c_b = b.tm_ln_c_b[d];
+    if (d == 0) {
+      a.ln3_w = b.tm_ln_in_w[1]; a.ln3_b = b.tm_ln_in_b[1]; a.f_next = tm(b, 1, 256); a.mask = mask_in ? mask_in : mask;
+      STEP(launch_pair_step(a, PAIR_STEP_INCOMING, s));
+    } else {
+      a.ln3_w = b.ta_ln_w[0]; a.ln3_b = b.ta_ln_b[0]; a.f_next = ta(0, 0); a.f_bias = ta(0, 384);
+      STEP(launch_pair_step(a, PAIR_STEP_PROJECT_START, s));
+    }
+  }
+  STEP(launch_triattn_flash(core, s));
+  a.ln1_w = b.ta_ln_w[0]; a.ln1_b = b.ta_ln_b[0]; a.f_gate = ta(0, 416); a.f_out = ta(0, 544);
+  a.ln3_w = b.ta_ln_w[1]; a.ln3_b = b.ta_ln_b[1]; a.f_next = ta(1, 0); a.f_bias = ta(1, 384);
+  STEP(launch_pair_step(a, PAIR_STEP_PROJECT_END, s));
+  STEP(launch_triattn_flash(core, s));
+  a.ln1_w = b.ta_ln_w[1]; a.ln1_b = b.ta_ln_b[1]; a.f_gate = ta(1, 416); a.f_out = ta(1, 544);
+  a.ln2_w = b.pt_ln_w; a.ln2_b = b.pt_ln_b; a.f_w1 = w1; a.f_w2 = w1 + 2 * hidden * 128;
+  if (logits) {
+    a.sl_ln_w = b.sl_ln_w; a.sl_ln_b = b.sl_ln_b; a.f_logits = w1 + 3 * hidden * 128; a.logit_heads = b.num_head; a.logits = logits;
+    if (logits_free) STEP(logits_free->wait(s));
+  }
+  if (!next) return launch_pair_step(a, PAIR_STEP_LAST, s);
+  a.ln3_w = next->tm_ln_in_w[0]; a.ln3_b = next->tm_ln_in_b[0]; a.f_next = tm(*next, 0, 256); a.mask = mask;
+  return launch_pair_step(a, PAIR_STEP_NEXT, s);
 }
 
 int single_update(const af3_pairformer_block& b, void* single, int dt, const float* mask, const float* logits, int64_t n,
@@ -78,7 +180,6 @@ int single_update(const af3_pairformer_block& b, void* single, int dt, const flo
   return product(y, b.st_w2, single, dt, c, h, AF3_LINEAR_GATE_RES, single);
 }
 
-inline int64_t up8(int64_t v) { return (v + 7) / 8 * 8; }
 inline bool msa_size_ok(int64_t rows, int64_t n) { return rows > 0 && n > 0 && n <= 8192 && rows <= (1ll << 30) / n; }
 
 size_t opm_bytes(int64_t rows, int64_t n) {
@@ -213,15 +314,20 @@ int af3_evoformer_stack_forward(const af3_msa_block* const* blocks, int num_bloc
     msa_attention_args(b, avg, u);
     msa_transition_args(b.mt_ln_w, b.mt_ln_b, b.mt_w1, b.mt_w2, b.mt_hidden, u);
     STEP(launch_msa_update(u, s));
-    STEP(pair_operators(b.pair, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace,
-                        pair_workspace_bytes, stream));
+    if (pair_steps_apply(b.pair, n))
+      STEP(pair_operators_in_steps(b.pair, nullptr, true, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace,
+                                   pair_workspace_bytes, nullptr, nullptr, s));
+    else
+      STEP(pair_operators(b.pair, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace,
+                          pair_workspace_bytes, stream));
   }
   return AF3_OK;
 }
 
 size_t af3_pairformer_stack_workspace_bytes(int64_t n, int num_head_pair) {
   const size_t a = af3_triangle_multiplication_workspace_bytes(n), b = af3_grid_self_attn_workspace_bytes(n, num_head_pair);
-  return a > b ? a : b;
+  const size_t c = n > 0 && n * tri_ldn(n) <= PAIR_STEP_POSITIONS ? PairStepScratch::bytes(n) : 0;
+  return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
 size_t af3_pairformer_single_workspace_bytes(int64_t n, int c_single, int single_hidden) {
@@ -248,31 +354,38 @@ int af3_pairformer_stack_forward(
   hipStream_t main_s = static_cast<hipStream_t>(stream);
   hipStream_t side_s = single_stream ? static_cast<hipStream_t>(single_stream) : main_s;
   const bool two = side_s != main_s;
-  if (two) STEP(order_streams(main_s, side_s));
-  hipEvent_t read_done[2] = {nullptr, nullptr};  // behind the attention that reads logits buffer 0 / 1
+  Event ready, read_done[2];  // behind the pair logits; behind the attention that reads logits buffer 0 / 1
+  if (two) STEP(ready.order(main_s, side_s));
   int rc = AF3_OK;
   for (int i = 0; i < num_blocks && rc == AF3_OK; ++i) {
     const af3_pairformer_block& b = *blocks[i];
-    rc = pair_operators(b, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes, stream);
-    if (rc != AF3_OK || !b.with_single) continue;
-    // the only reader of `pair` on the single path: it stays in front of whatever updates `pair` next
-    float* lg = logits + (size_t)(num_blocks > 1 ? i & 1 : 0) * b.num_head * ((n + 3) / 4 * 4) * n;
-    hipEvent_t& done = read_done[i & 1];
-    if (done && hipStreamWaitEvent(main_s, done, 0) != hipSuccess) rc = AF3_ERR_LAUNCH;
-    if (rc == AF3_OK)
-      rc = af3_pair_logits_quads_forward(pair, pair_dtype, b.sl_ln_w, b.sl_ln_b, b.sl_w, b.num_head, lg, n, stream);
-    if (rc == AF3_OK && two) rc = order_streams(main_s, side_s);
+    float* lg = nullptr;
+    Event* free = nullptr;
+    if (b.with_single) {
+      lg = logits + (size_t)(num_blocks > 1 ? i & 1 : 0) * b.num_head * ((n + 3) / 4 * 4) * n;
+      free = &read_done[i & 1];
+    }
+    // the pair logits are the only thing the single track reads of `pair`: they are made in front of whatever updates it next
+    if (pair_steps_apply(b, n)) {
+      const bool chained = i > 0 && pair_steps_apply(*blocks[i - 1], n);
+      const af3_pairformer_block* next = i + 1 < num_blocks && pair_steps_apply(*blocks[i + 1], n) ? blocks[i + 1] : nullptr;
+      rc = pair_operators_in_steps(b, next, !chained, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes,
+                                   lg, free, main_s);
+      if (rc != AF3_OK || !b.with_single) continue;
+    } else {
+      rc = pair_operators(b, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes, stream);
+      if (rc != AF3_OK || !b.with_single) continue;
+      rc = free->wait(main_s);
+      if (rc == AF3_OK)
+        rc = af3_pair_logits_quads_forward(pair, pair_dtype, b.sl_ln_w, b.sl_ln_b, b.sl_w, b.num_head, lg, n, stream);
+    }
+    if (rc == AF3_OK && two) rc = ready.order(main_s, side_s);
     if (rc == AF3_OK)
       rc = single_update(b, single, single_dtype, seq_mask, lg, n, single_workspace, single_workspace_bytes, side_s);
-    if (rc == AF3_OK && two && i + 2 < num_blocks) {
-      if (!done && hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess) rc = AF3_ERR_LAUNCH;
-      else if (hipEventRecord(done, side_s) != hipSuccess) rc = AF3_ERR_LAUNCH;
-    }
+    if (rc == AF3_OK && two && i + 2 < num_blocks) rc = read_done[i & 1].record(side_s);
   }
-  for (hipEvent_t e : read_done)
-    if (e && hipEventDestroy(e) != hipSuccess && rc == AF3_OK) rc = AF3_ERR_LAUNCH;
   if (two && join) {
-    const int jrc = order_streams(side_s, main_s);
+    const int jrc = ready.order(side_s, main_s);
     if (rc == AF3_OK) rc = jrc;
   }
   return rc;

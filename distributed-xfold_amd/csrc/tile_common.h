@@ -210,6 +210,19 @@ __device__ __forceinline__ void load_ln_tile(const TIO* x, const Tile& t, const 
   }
 }
 
+// Channel sums of the LayerNorm of a contraction's result: eight channels one after the other, then the eight k-steps of a
+// half (channels 16 ks + 8 half ..) in this order, then the two halves.  sum_k_steps: all k-steps in one lane;
+// sum_chunks: 16 lanes, lane 2 ks + half of a row of 16, the halves included.
+__device__ __forceinline__ float sum_k_steps(const float* s) {
+  return ((s[0] + s[1]) + (s[4] + s[5])) + ((s[2] + s[3]) + (s[6] + s[7]));
+}
+__device__ __forceinline__ float sum_chunks(float s) {
+  s += dpp_mov<0x4E>(s);   // quad_perm [2,3,0,1]: ks ^ 1
+  s += dpp_mov<0x128>(s);  // row_ror:8: ks ^ 4
+  s += dpp_mov<0x124>(s);  // row_ror:4: the other two of these sums, ks ^ 2 (either way round: the lanes 8 apart agree)
+  return s + dpp_mov<0xB1>(s);  // quad_perm [1,0,3,2]: the halves
+}
+
 // In-place LayerNorm of the rows of sX (bf16 in LDS), same thread mapping.
 __device__ __forceinline__ void ln_inplace_tile(bf16_t* sX, const float* lnw, const float* lnb, int tid) {
   const int chunk = tid & 15, prow = tid >> 4;

@@ -22,7 +22,7 @@ class PairformerBlockStruct(C.Structure):
         [(k, _vp * 2) for k in ("tm_ln_in_w", "tm_ln_in_b", "tm_ln_c_w", "tm_ln_c_b", "tm_w_proj_gate", "tm_w_out",
                                 "tm_w_gating", "ta_ln_w", "ta_ln_b", "ta_w_bias", "ta_w_qkvg", "ta_w_out")]
         + [(k, _vp) for k in ("pt_ln_w", "pt_ln_b", "pt_w1", "pt_w2", "sl_ln_w", "sl_ln_b", "sl_w", "sa_ln_w", "sa_ln_b",
-                              "sa_w_qkvg", "sa_q_b", "sa_w_out", "st_ln_w", "st_ln_b", "st_w1", "st_w2")]
+                              "sa_w_qkvg", "sa_q_b", "sa_w_out", "st_ln_w", "st_ln_b", "st_w1", "st_w2", "pair_frags")]
         + [(k, C.c_int32) for k in ("valid_channels", "num_head_pair", "pair_hidden", "with_single", "num_head",
                                     "c_single", "single_hidden")])
 

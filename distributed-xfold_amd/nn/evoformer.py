@@ -282,9 +282,9 @@ class EvoformerBlock(HipModule):
               ("mt_w2", t["w2_64"], (64, s.mt_hidden)))
         p = L.PairformerBlockStruct()
         p.device = s.device
-        fill_pair_weights(p, *track, self.c_pair)
+        frags = fill_pair_weights(p, *track, self.c_pair)
         s.pair = p
-        self._native = (s, packs)
+        self._native = (s, packs, frags)
         return s
 
     @torch.no_grad()

@@ -11,7 +11,8 @@ import torch.nn as nn
 from .. import check, ops
 from .. import lib as L
 from .attention import GridSelfAttention
-from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, packs_of, pad_channels, pad_rows, point
+from .base import (HipModule, as_written, bf16, drop_mesh, f32, fragments, in_check_mode, packs_of, pad_channels, pad_rows,
+                   point, swap23)
 from .diffusion_transformer import AdaLNZero, AdaptiveLayerNorm, SelfAttention
 from .primitives import Transition
 from .triangle_multiplication import TriangleMultiplication
@@ -33,8 +34,8 @@ def one_sequence(single, seq_mask) -> bool:
     return single.dim() == 2 and (seq_mask is None or seq_mask.dim() == 1)
 
 
-def fill_pair_weights(s, tm_out, tm_in, ta_start, ta_end, transition, c_pair) -> None:
-    """The pair operators' packed weights into an af3_pairformer_block."""
+def fill_pair_weights(s, tm_out, tm_in, ta_start, ta_end, transition, c_pair, w_logits=None) -> torch.Tensor:
+    """The pair operators' packed weights into an af3_pairformer_block; returns what only the structure points at."""
     vec, mat = (128,), (128, 128)
     for d, (tm, ta) in enumerate(((tm_out, ta_start), (tm_in, ta_end))):
         p, q = tm.packed(), ta.packed()
@@ -49,6 +50,20 @@ def fill_pair_weights(s, tm_out, tm_in, ta_start, ta_end, transition, c_pair) ->
     point(s, ("pt_ln_w", p["ln_w"], vec), ("pt_ln_b", p["ln_b"], vec), ("pt_w1", p["w1"], (hidden // 64, 128, 128)),
           ("pt_w2", p["w2"], (128, hidden)))
     s.valid_channels, s.num_head_pair, s.pair_hidden = c_pair, ta_start.num_head, hidden
+    mats = []
+    for tm in (tm_out, tm_in):
+        q = tm.packed()
+        mats += [q["w_gl"], q["w_out"], q["w_proj_gate"].view(-1, 128)]
+    for ta in (ta_start, ta_end):
+        q = ta.packed()
+        w = swap23(q["w_qkvg"])
+        mats += [w[0], w[1], q["w_qkvg"][2], q["w_bias"], w[3], q["w_out"]]
+    mats += [p["w1"].view(-1, 128), p["w2"]]
+    if w_logits is not None:
+        mats.append(w_logits)
+    frags = torch.cat([fragments(m) for m in mats])
+    s.pair_frags = frags.data_ptr()
+    return frags
 
 
 class PairformerBlock(HipModule):
@@ -127,7 +142,7 @@ class PairformerBlock(HipModule):
             return self._native[0]
         by = dict(zip(mods, packs))
         s = L.PairformerBlockStruct()
-        fill_pair_weights(s, *track, self.c_pair)
+        frags = fill_pair_weights(s, *track, self.c_pair, by[self]["w_logits"] if self.with_single else None)
         s.with_single = int(self.with_single)
         if self.with_single:
             c, p, a, o, t = self.c_single, by[self], by[sa], by[sa.adaptive_zero_init], by[st]
@@ -138,7 +153,7 @@ class PairformerBlock(HipModule):
                   ("sa_q_b", a["q_b"], (c,)), ("sa_w_out", o["w"], (c, c)), ("st_ln_w", t["ln_w"], (c,)),
                   ("st_ln_b", t["ln_b"], (c,)), ("st_w1", t["w1"], (2 * hidden, c)), ("st_w2", t["w2"], (c, hidden)))
             s.num_head, s.c_single, s.single_hidden = self.n_heads, c, hidden
-        self._native = (s, packs)
+        self._native = (s, packs, frags)
         return s
 
     def forward(self, pair: torch.Tensor, pair_mask: torch.Tensor, single: Optional[torch.Tensor] = None,

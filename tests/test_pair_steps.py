@@ -1,0 +1,121 @@
+"""The pair operators at few tokens, a run of them in one kernel (pair_step.hip), against one kernel per operator."""
+
+import pytest
+import torch
+
+
+def _block(pkg, c=128, factor=4, seed=0, device="cuda", std=0.05, heads=16):
+    """A block with random weights: LayerNorm weights around 1, everything else N(0, std)."""
+    gen = torch.Generator(device=device).manual_seed(seed)
+    with torch.device(device):
+        blk = pkg.nn.PairformerBlock(c_pair=c, num_intermediate_factor=factor, with_single=c == 128, n_heads=heads,
+                                     c_single=24 * heads)
+    with torch.no_grad():
+        for name, p in blk.named_parameters():
+            p.normal_(0.0, std, generator=gen)
+            if p.dim() == 1 and name.endswith("weight"):
+                p += 1.0
+    blk.invalidate()
+    return blk
+
+
+def _inputs(n, c, io, padding, seed=1, heads=16):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    seq = (torch.arange(n, device="cuda") < n - padding).float()
+    pair = torch.randn(n, n, c, generator=gen, device="cuda").to(io)
+    single = torch.randn(n, 24 * heads, generator=gen, device="cuda").to(io)
+    return pair, (seq[:, None] * seq[None, :]).contiguous(), single, seq
+
+
+def _run(blk, pair, mask, single, seq):
+    out = blk(pair.clone(), mask, single.clone(), seq) if blk.with_single else (blk(pair.clone(), mask),)
+    torch.cuda.synchronize()
+    return out
+
+
+def _run_general(blk, *inputs):
+    s = blk.native()
+    frags, s.pair_frags = s.pair_frags, None
+    try:
+        return _run(blk, *inputs)
+    finally:
+        s.pair_frags = frags
+
+
+# sizes: one pixel; rows shorter than a group of 16 positions, one longer; tiles that cross rows and that do not; a key tile
+# of 64 and one more; the contraction's two kernels; both sizes of patches; the largest.  Hidden layers of one chunk, a part
+# of one and two; more than one block of 32 heads.
+CASES = [(1, 128, 4, 16, 0), (7, 128, 4, 16, 2), (16, 128, 4, 16, 0), (17, 128, 4, 40, 3), (33, 128, 1, 16, 0), (63, 128, 4, 16, 5),
+         (64, 128, 2, 16, 0), (65, 128, 4, 16, 30), (127, 128, 4, 16, 0), (129, 128, 3, 16, 11), (208, 128, 4, 16, 9),
+         (24, 64, 1, 16, 3), (65, 64, 2, 16, 0), (90, 96, 4, 16, 1), (136, 64, 2, 16, 7)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("io", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,c,factor,heads,padding", CASES)
+def test_steps_give_the_bits_of_one_kernel_per_operator(gpu_pkg, n, c, factor, heads, padding, io):
+    """The same sums in the same order, rounded at the same places."""
+    blk, inputs = _block(gpu_pkg, c, factor, n, heads=heads), _inputs(n, c, io, padding, heads=heads)
+    got, want = _run(blk, *inputs), _run_general(blk, *inputs)
+    for x, y, before in zip(got, want, (inputs[0], inputs[2])):
+        assert torch.isfinite(x).all() and not torch.equal(x, before) and torch.equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [5, 48, 130])
+def test_a_run_of_blocks_is_its_blocks_one_by_one(gpu_pkg, n):
+    """The last step of a block makes the next block's first operands: the same bits as a call per block."""
+    blocks, inputs = [_block(gpu_pkg, seed=i) for i in range(3)], _inputs(n, 128, torch.bfloat16, 2)
+    pair, mask, single, seq = inputs
+    got = gpu_pkg.nn.pairformer_loop(blocks, pair.clone(), mask, single.clone(), seq)
+    want = (pair, single)
+    for blk in blocks:
+        want = _run(blk, want[0], mask, want[1], seq)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.gpu
+def test_incoming_mask_of_its_own(gpu_pkg):
+    """An Evoformer block gives the incoming product the transposed mask: one that is not symmetric."""
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    n, rows = 43, 9
+    with torch.device("cuda"):
+        blk = gpu_pkg.nn.EvoformerBlock()
+    with torch.no_grad():
+        for name, p in blk.named_parameters():
+            p.normal_(0.0, 0.05, generator=gen)
+            if p.dim() == 1 and name.endswith("weight"):
+                p += 1.0
+    blk.invalidate()
+    pair, msa = torch.randn(n, n, 128, generator=gen, device="cuda"), torch.randn(rows, n, 64, generator=gen, device="cuda")
+    mask, msa_mask = (torch.rand(n, n, generator=gen, device="cuda") > 0.3).float(), torch.ones(rows, n, device="cuda")
+    got = blk(msa.clone(), pair.clone(), msa_mask, mask)[1]
+    s = blk.native()
+    frags, s.pair.pair_frags = s.pair.pair_frags, None
+    want = blk(msa.clone(), pair.clone(), msa_mask, mask)[1]
+    s.pair.pair_frags = frags
+    assert torch.equal(got, want)
+
+
+def test_fragment_order(pkg):
+    """[row / 32][column / 16][(column / 8) % 2][row % 32][column % 8]; exchanged rows are their own inverse."""
+    base = pkg.nn.base
+    w = torch.arange(64 * 48).reshape(64, 48)
+    f = base.fragments(w).reshape(2, 3, 2, 32, 8)
+    for r in (0, 5, 31, 32, 63):
+        for c in (0, 7, 8, 15, 16, 47):
+            assert f[r // 32, c // 16, c // 8 % 2, r % 32, c % 8] == w[r, c]
+    s = base.swap23(w)
+    assert torch.equal(s[4], w[8]) and torch.equal(s[27], w[23]) and torch.equal(base.swap23(s), w)
+
+
+@pytest.mark.parametrize("factor,rows", [(4, 2880 + 1536 + 32), (2, 2880 + 768 + 32)])
+def test_all_matrices_of_a_block_are_in_its_fragments(pkg, factor, rows):
+    blk = _block(pkg, factor=factor, device="cpu")
+    s = blk.native()
+    frags = blk._native[2]
+    assert s.pair_frags == frags.data_ptr() and frags.dtype == torch.bfloat16 and frags.numel() == rows * 128
+    # the first matrix and the last
+    want = pkg.nn.base.fragments(blk.triangle_multiplication_outgoing.packed()["w_gl"])
+    assert torch.equal(frags[:want.numel()], want)
+    assert torch.equal(frags[-32 * 128:], pkg.nn.base.fragments(blk.packed()["w_logits"]))
