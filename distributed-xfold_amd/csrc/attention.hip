@@ -66,9 +66,11 @@ void flash_kernel(FlashArgs a) {
   const int hh = lane >> 5, j = lane & 31;
   const int xaddr = half_swap_addr();
   // Batch entries that share a slab of a non-batched pair bias must meet in one L2 for that slab to be
-  // fetched from memory once: workgroup ids are dealt round-robin to the 8 XCDs, each with an L2 of its
-  // own, so id -> (xcd, slot) -> logical id gives every XCD a contiguous range of logical ids, and
-  // logical = (q_tile * H + head) * B + batch has the sharing entries as its fastest index.
+  // fetched from memory once, and so must the query tiles that share a head's K and V: workgroup ids are dealt
+  // round-robin to the 8 XCDs, each with an L2 of its own, so id -> (xcd, slot) -> logical id gives every XCD a
+  // contiguous range of logical ids, and logical = (head * query tiles + query tile) * B + batch gives it a few
+  // heads, with the entries that share a slab side by side (16 heads x 48, 5 samples of 768: 36.2 -> 35.2 us
+  // against query tiles as the slowest index).
   int b, h, q0;
   if (a.bias_mod > 0) {
     // (windows of a few keys: the workgroups are short and the bias slabs small; plain order)
@@ -80,9 +82,10 @@ void flash_kernel(FlashArgs a) {
     const int per_xcd = (gridDim.x + 7) >> 3;
     const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (logical >= a.n_blocks) return;  // workgroup-uniform, before any barrier
+    const int tiles = (a.Sq + NW * 32 - 1) / (NW * 32), rest = logical / a.B;
     b = logical % a.B;
-    h = (logical / a.B) % a.H;
-    q0 = (logical / (a.B * a.H)) * (NW * 32) + wave * 32;
+    h = rest / tiles;
+    q0 = rest % tiles * (NW * 32) + wave * 32;
   }
   const int d = a.d;
   const int qi = min(q0 + j, a.Sq - 1);  // clamped for loads; stores are guarded
@@ -672,21 +675,11 @@ bool window_fits(const FlashArgs& a) {
          a.table_rows > 0 && a.table_rows * (a.k_ss > a.v_ss ? a.k_ss : a.v_ss) < (1ll << 30);
 }
 
-// Queries per workgroup: 128 (four waves share the K / V tiles), or 64 when
-// that would leave the 256 CUs with too few workgroups, or 32 for the short
-// query windows of the atom cross-attention.
+// Queries per workgroup: 128 (four waves share the K / V tiles), 64, or 32 for
+// the short query windows of the atom cross-attention.
 template <int KSTEPS, int DVT>
 int launch_nw(const FlashArgs& a, hipStream_t stream) {
   const int64_t heads = (int64_t)a.H * a.B;
-  // Four waves share each staged K / V tile once there are enough 128-query
-  // workgroups to cover the chip; below that, two waves per workgroup spread
-  // the work over twice as many CUs.
-  const int nw = a.Sq <= 32 ? 1 : (((a.Sq + 127) / 128) * heads < 256 ? 2 : 4);
-  const int64_t n_blocks = (int64_t)((a.Sq + nw * 32 - 1) / (nw * 32)) * heads;
-  if (n_blocks <= 0 || n_blocks > 0x7ffffff0) return AF3_ERR_BAD_ARG;
-  FlashArgs fa = a;
-  fa.n_blocks = (int)n_blocks;
-  const dim3 grid((unsigned)((n_blocks + 7) / 8 * 8));  // whole rounds over the 8 XCDs; the surplus ids return at once
   // The form with fixed per-lane offsets: no row table, a bias that can be fetched 16 bytes at a time, and
   // offsets inside a key tile / a bias plane that fit 32 bits.
   const int64_t quad_step = a.bias_squad ? a.bias_squad : 4;
@@ -694,6 +687,16 @@ int launch_nw(const FlashArgs& a, hipStream_t stream) {
                     (a.bias_sh & 3) == 0 && (a.bias_squad & 3) == 0 && ((uintptr_t)a.bias & 15) == 0 &&
                     a.k_ss > 0 && a.v_ss > 0 && a.k_ss < (1 << 22) && a.v_ss < (1 << 22) && a.bias_sq >= 0 &&
                     quad_step > 0 && (int64_t)a.Sq * a.bias_sq + quad_step < (1 << 28);
+  // Four waves share each staged K / V tile once there are enough 128-query workgroups to cover the chip; below that, two
+  // waves per workgroup spread the work over twice as many CUs.  Not with head dimension 48, where the form with fixed
+  // offsets needs four waves to share the staging registers: it is faster than twice the workgroups of the general form
+  // (16 heads x 48, 5 samples of 100, 200, 384 tokens, projections included: 18.4 us for 18.6, 25.2 for 28.7, 32.1 for 37.9).
+  const int nw = a.Sq <= 32 ? 1 : (((a.Sq + 127) / 128) * heads < 256 && !(KSTEPS == 3 && fast) ? 2 : 4);
+  const int64_t n_blocks = (int64_t)((a.Sq + nw * 32 - 1) / (nw * 32)) * heads;
+  if (n_blocks <= 0 || n_blocks > 0x7ffffff0) return AF3_ERR_BAD_ARG;
+  FlashArgs fa = a;
+  fa.n_blocks = (int)n_blocks;
+  const dim3 grid((unsigned)((n_blocks + 7) / 8 * 8));  // whole rounds over the 8 XCDs; the surplus ids return at once
   // (with a single wave, or with head dimension 48 and fewer than four waves, to share the K / V staging
   // registers between, the second register set of that form no longer fits: those take the general form)
 #define AF3_FLASH_LAUNCH(NW_)                                                                                   \
