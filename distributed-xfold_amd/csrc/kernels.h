@@ -378,7 +378,7 @@ struct PairStepArgs {
   const float *ln2_w = nullptr, *ln2_b = nullptr;  // transition
   const bf16_t *f_w1 = nullptr, *f_w2 = nullptr;
   const float *ln3_w = nullptr, *ln3_b = nullptr;  // prologue or projections of the operator behind
-  const bf16_t *f_next = nullptr, *f_bias = nullptr;
+  const bf16_t *f_next = nullptr, *f_v = nullptr;  // f_next: projection and gate rows, or q and k;  f_v: v, then the pair-bias heads
   const float* mask = nullptr;                     // prologue
   bf16_t *a_buf = nullptr, *b_buf = nullptr;
   bf16_t *q = nullptr, *k = nullptr, *vt = nullptr;

@@ -222,8 +222,8 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
         load_frags<8>(a.f_next, pg + (r & 1) * 2 + (r >> 1) * 8, 8, 0, lane, d);
       } else {
         constexpr int r = n - OCT_NEXT;
-        if constexpr (r < 3) load_frags<8>(a.f_next, 4 * r + wave, 8, 0, lane, d);
-        else if (wave == 0) load_frags<8>(a.f_bias, 0, 8, 0, lane, d);
+        if constexpr (r < 2) load_frags<8>(a.f_next, 4 * r + wave, 8, 0, lane, d);
+        else if (r == 2 || wave == 0) load_frags<8>(a.f_v, r == 2 ? wave : 4, 8, 0, lane, d);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -238,10 +238,11 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
   uint32_t warm = 0u;
   {
     const uint32_t line = (blockIdx.x >> 3) * 256u + (uint32_t)tid;
-    const uint32_t own_lines = TRANSITION ? (uint32_t)(3 * a.hidden + (a.logits ? (a.logit_heads + 31) / 32 * 32 : 0)) * 2u : 0u;
-    const uint32_t next_lines = NEXT == NEXT_PROLOGUE ? 1024u : NEXT == NEXT_PROJECT ? 832u : 0u;  // 512 rows; q, k, v, bias
-    if (line < own_lines) warm = *reinterpret_cast<const uint32_t*>(at32(a.f_w1, line * 64u));
-    else if (line < own_lines + next_lines) warm = *reinterpret_cast<const uint32_t*>(at32(a.f_next, (line - own_lines) * 64u));
+    const uint32_t n0 = TRANSITION ? (uint32_t)a.hidden * 4u : 0u, n1 = TRANSITION ? (uint32_t)a.hidden * 2u : 0u;  // 2 lines a row
+    constexpr uint32_t n2 = NEXT == NEXT_PROLOGUE ? 1024u : NEXT == NEXT_PROJECT ? 512u : 0u, n3 = NEXT == NEXT_PROJECT ? 320u : 0u;
+    const bf16_t* const from = line < n0 ? a.f_w1 : line < n0 + n1 ? a.f_w2 - n0 * 64 : line < n0 + n1 + n2 ? a.f_next - (n0 + n1) * 64
+                                                                                             : a.f_v - (n0 + n1 + n2) * 64;
+    if (line < n0 + n1 + n2 + n3) warm = *reinterpret_cast<const uint32_t*>(from + line * 64u);
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -593,7 +594,7 @@ int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s) {
   const bool project = step == PAIR_STEP_PROJECT_START || step == PAIR_STEP_PROJECT_END, transition = step >= PAIR_STEP_LAST;
   if (epilogue ? !a.t_buf || !a.ln_c_w || !a.ln_c_b || a.plane < tri_plane(a.N) || a.valid_c < 1 || a.valid_c > C : !a.og) return AF3_ERR_BAD_ARG;
   if (prologue && (!a.a_buf || !a.b_buf || !a.f_next || !a.ln3_w || !a.ln3_b || a.plane < tri_plane(a.N))) return AF3_ERR_BAD_ARG;
-  if (project && (!a.q || !a.k || !a.vt || !a.bias || !a.f_next || !a.f_bias || !a.ln3_w || !a.ln3_b)) return AF3_ERR_BAD_ARG;
+  if (project && (!a.q || !a.k || !a.vt || !a.bias || !a.f_next || !a.f_v || !a.ln3_w || !a.ln3_b)) return AF3_ERR_BAD_ARG;
   if (transition && (!a.f_w1 || !a.f_w2 || !a.ln2_w || !a.ln2_b || a.hidden <= 0 || (a.hidden & 63) || a.hidden > MAX_HIDDEN)) return AF3_ERR_BAD_ARG;
   if (a.logits && (!transition || !a.f_logits || !a.sl_ln_w || !a.sl_ln_b || a.logit_heads <= 0)) return AF3_ERR_BAD_ARG;
   switch (step) {

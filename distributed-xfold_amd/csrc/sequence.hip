@@ -116,9 +116,11 @@ int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_
   a.bias_scale = 1.4426950408889634f;  // base-2 logits, as grid_self_attn_impl
   a.q_scale = a.bias_scale / sqrtf((float)(c / 4));
   // pair_frags, in rows of 128
-  auto tm = [&](const af3_pairformer_block& x, int d, int row) { return x.pair_frags + (d * 768 + row) * 128; };
-  auto ta = [&](int d, int row) { return b.pair_frags + (1536 + d * 672 + row) * 128; };
-  const uint16_t* w1 = b.pair_frags + 2880 * 128;
+  auto qkg = [&](int d, int row) { return b.pair_frags + (d * 384 + row) * 128; };
+  auto tm = [&](const af3_pairformer_block& x, int d, int row) { return x.pair_frags + (768 + d * 768 + row) * 128; };
+  auto ta = [&](int d, int row) { return b.pair_frags + (2304 + d * 288 + row) * 128; };
+  const uint16_t* const w1 = b.pair_frags + 2880 * 128;
+  const int logit_rows = b.with_single ? (b.num_head + 31) / 32 * 32 : 0;
   TriAttnArgs core;
   core.q = w.qa; core.k = w.kb; core.vt = w.vt; core.bias = w.bias; core.mask = mask; core.og = w.ogt; core.N = (int)n; core.ldn = a.ldn;
 
@@ -137,19 +139,19 @@ int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_
       a.ln3_w = b.tm_ln_in_w[1]; a.ln3_b = b.tm_ln_in_b[1]; a.f_next = tm(b, 1, 256); a.mask = mask_in ? mask_in : mask;
       STEP(launch_pair_step(a, PAIR_STEP_INCOMING, s));
     } else {
-      a.ln3_w = b.ta_ln_w[0]; a.ln3_b = b.ta_ln_b[0]; a.f_next = ta(0, 0); a.f_bias = ta(0, 384);
+      a.ln3_w = b.ta_ln_w[0]; a.ln3_b = b.ta_ln_b[0]; a.f_next = qkg(0, 0); a.f_v = ta(0, 0);
       STEP(launch_pair_step(a, PAIR_STEP_PROJECT_START, s));
     }
   }
   STEP(launch_triattn_flash(core, s));
-  a.ln1_w = b.ta_ln_w[0]; a.ln1_b = b.ta_ln_b[0]; a.f_gate = ta(0, 416); a.f_out = ta(0, 544);
-  a.ln3_w = b.ta_ln_w[1]; a.ln3_b = b.ta_ln_b[1]; a.f_next = ta(1, 0); a.f_bias = ta(1, 384);
+  a.ln1_w = b.ta_ln_w[0]; a.ln1_b = b.ta_ln_b[0]; a.f_gate = qkg(0, 256); a.f_out = ta(0, 160);
+  a.ln3_w = b.ta_ln_w[1]; a.ln3_b = b.ta_ln_b[1]; a.f_next = qkg(1, 0); a.f_v = ta(1, 0);
   STEP(launch_pair_step(a, PAIR_STEP_PROJECT_END, s));
   STEP(launch_triattn_flash(core, s));
-  a.ln1_w = b.ta_ln_w[1]; a.ln1_b = b.ta_ln_b[1]; a.f_gate = ta(1, 416); a.f_out = ta(1, 544);
-  a.ln2_w = b.pt_ln_w; a.ln2_b = b.pt_ln_b; a.f_w1 = w1; a.f_w2 = w1 + 2 * hidden * 128;
+  a.ln1_w = b.ta_ln_w[1]; a.ln1_b = b.ta_ln_b[1]; a.f_gate = qkg(1, 256); a.f_out = ta(1, 160);
+  a.ln2_w = b.pt_ln_w; a.ln2_b = b.pt_ln_b; a.f_w1 = w1; a.f_w2 = w1 + (2 * hidden + logit_rows) * 128;
   if (logits) {
-    a.sl_ln_w = b.sl_ln_w; a.sl_ln_b = b.sl_ln_b; a.f_logits = w1 + 3 * hidden * 128; a.logit_heads = b.num_head; a.logits = logits;
+    a.sl_ln_w = b.sl_ln_w; a.sl_ln_b = b.sl_ln_b; a.f_logits = w1 + 2 * hidden * 128; a.logit_heads = b.num_head; a.logits = logits;
     if (logits_free) STEP(logits_free->wait(s));
   }
   if (!next) return launch_pair_step(a, PAIR_STEP_LAST, s);

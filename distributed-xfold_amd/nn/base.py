@@ -82,17 +82,13 @@ def pack_swiglu(w1: torch.Tensor, block: int) -> torch.Tensor:
     return torch.cat([a, b], dim=1).reshape(2 * hidden, -1).contiguous()
 
 
-def fragments(w: torch.Tensor) -> torch.Tensor:
+def fragments(w: torch.Tensor, swap23: bool = False) -> torch.Tensor:
     """A matrix [rows, k] (multiples of 32 and 16) in the order in which MFMA fragments are loaded: 16-byte pieces of 8
-    columns, lane by lane, 32 rows x 16 columns at a time."""
+    columns, lane by lane, 32 rows x 16 columns at a time.  swap23: with bits 2 and 3 of the row number exchanged (eight
+    consecutive rows are then eight consecutive accumulator registers of a lane)."""
     rows, k = w.shape
-    return w.reshape(rows // 32, 32, k // 16, 2, 8).permute(0, 2, 3, 1, 4).reshape(-1)
-
-
-def swap23(w: torch.Tensor) -> torch.Tensor:
-    """Rows [..., rows, k] with bits 2 and 3 of the row number exchanged: eight consecutive rows of the weight are then
-    eight consecutive accumulator registers of an MFMA lane."""
-    return w.unflatten(-2, (-1, 2, 2, 4)).transpose(-3, -4).flatten(-5, -2)
+    v = w.reshape(rows // 32, 2, 2, 2, 4, k // 16, 2, 8)
+    return v.permute(0, 5, 6, 1, *((3, 2) if swap23 else (2, 3)), 4, 7).reshape(-1)
 
 
 def point(s, *fields) -> None:

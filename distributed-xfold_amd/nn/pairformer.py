@@ -12,7 +12,7 @@ from .. import check, ops
 from .. import lib as L
 from .attention import GridSelfAttention
 from .base import (HipModule, as_written, bf16, drop_mesh, f32, fragments, in_check_mode, packs_of, pad_channels, pad_rows,
-                   point, swap23)
+                   point)
 from .diffusion_transformer import AdaLNZero, AdaptiveLayerNorm, SelfAttention
 from .primitives import Transition
 from .triangle_multiplication import TriangleMultiplication
@@ -50,18 +50,19 @@ def fill_pair_weights(s, tm_out, tm_in, ta_start, ta_end, transition, c_pair, w_
     point(s, ("pt_ln_w", p["ln_w"], vec), ("pt_ln_b", p["ln_b"], vec), ("pt_w1", p["w1"], (hidden // 64, 128, 128)),
           ("pt_w2", p["w2"], (128, hidden)))
     s.valid_channels, s.num_head_pair, s.pair_hidden = c_pair, ta_start.num_head, hidden
-    mats = []
+    # (gathered first and reordered together: packing is paid for at every new set of weights)
+    plain, turned = [], []
     for tm in (tm_out, tm_in):
         q = tm.packed()
-        mats += [q["w_gl"], q["w_out"], q["w_proj_gate"].view(-1, 128)]
+        plain += [q["w_gl"], q["w_out"], q["w_proj_gate"].view(-1, 128)]
     for ta in (ta_start, ta_end):
         q = ta.packed()
-        w = swap23(q["w_qkvg"])
-        mats += [w[0], w[1], q["w_qkvg"][2], q["w_bias"], w[3], q["w_out"]]
-    mats += [p["w1"].view(-1, 128), p["w2"]]
+        plain += [q["w_qkvg"][2], q["w_bias"], q["w_out"]]
+        turned += [q["w_qkvg"][0:2].view(-1, 128), q["w_qkvg"][3]]
+    plain.append(p["w1"].view(-1, 128))
     if w_logits is not None:
-        mats.append(w_logits)
-    frags = torch.cat([fragments(m) for m in mats])
+        plain.append(w_logits)
+    frags = torch.cat([fragments(torch.cat(turned), swap23=True), fragments(torch.cat(plain)), fragments(p["w2"])])
     s.pair_frags = frags.data_ptr()
     return frags
 

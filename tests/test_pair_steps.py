@@ -105,8 +105,8 @@ def test_fragment_order(pkg):
     for r in (0, 5, 31, 32, 63):
         for c in (0, 7, 8, 15, 16, 47):
             assert f[r // 32, c // 16, c // 8 % 2, r % 32, c % 8] == w[r, c]
-    s = base.swap23(w)
-    assert torch.equal(s[4], w[8]) and torch.equal(s[27], w[23]) and torch.equal(base.swap23(s), w)
+    g = base.fragments(w, swap23=True).reshape(2, 3, 2, 32, 8)
+    assert torch.equal(g[:, :, :, 4], f[:, :, :, 8]) and torch.equal(g[:, :, :, 27], f[:, :, :, 23]) and torch.equal(g[:, :, :, 3], f[:, :, :, 3])
 
 
 @pytest.mark.parametrize("factor,rows", [(4, 2880 + 1536 + 32), (2, 2880 + 768 + 32)])
@@ -115,7 +115,12 @@ def test_all_matrices_of_a_block_are_in_its_fragments(pkg, factor, rows):
     s = blk.native()
     frags = blk._native[2]
     assert s.pair_frags == frags.data_ptr() and frags.dtype == torch.bfloat16 and frags.numel() == rows * 128
-    # the first matrix and the last
-    want = pkg.nn.base.fragments(blk.triangle_multiplication_outgoing.packed()["w_gl"])
-    assert torch.equal(frags[:want.numel()], want)
-    assert torch.equal(frags[-32 * 128:], pkg.nn.base.fragments(blk.packed()["w_logits"]))
+    q = blk.pair_attention1.packed()["w_qkvg"]
+    assert torch.equal(frags[:128 * 128], pkg.nn.base.fragments(q[0], swap23=True))
+    at = 768 * 128      # the matrices in their own order of rows, up to the transition's second
+    for w in (blk.triangle_multiplication_outgoing.packed()["w_gl"], blk.triangle_multiplication_outgoing.packed()["w_out"]):
+        assert torch.equal(frags[at:at + 128 * 128], pkg.nn.base.fragments(w))
+        at += 128 * 128
+    w2 = blk.pair_transition.packed()["w2"]
+    assert torch.equal(frags[-w2.numel():], pkg.nn.base.fragments(w2))
+    assert torch.equal(frags[-w2.numel() - 32 * 128:-w2.numel()], pkg.nn.base.fragments(blk.packed()["w_logits"]))
