@@ -70,7 +70,7 @@ int pair_operators(const af3_pairformer_block& b, void* pair, int dt, const floa
 // A step takes the chain of one tile of 32 positions where a kernel of its own per operator takes several of tiles of 128,
 // and eight launches a block take the place of fourteen; past some number of tiles what every tile fetches of the weights
 // costs more than that saves.  Runs of 4 blocks, us a block, one kernel per operator -> steps (bf16 / fp32 stream):
-//   64 tokens 136 -> 92 / 143 -> 91,  128: 166 -> 124 / 173 -> 123,  160: 205 -> 179 / 213 -> 182,
+//   64 tokens 136 -> 85 / 143 -> 88,  128: 166 -> 121 / 173 -> 121,  160: 205 -> 179 / 213 -> 182,
 //   208: 286 -> 268 / 306 -> 279,  224: 265 -> 264 / 283 -> 275,  256: 287 -> 288 / 323 -> 302
 constexpr int64_t PAIR_STEP_POSITIONS = 208 * 208;
 bool pair_steps_apply(const af3_pairformer_block& b, int64_t n) {
@@ -84,8 +84,15 @@ struct PairStepScratch {
   uint16_t* bias = nullptr;
   static size_t plane_bytes(int64_t n) { return (size_t)128 * tri_plane(n) * 2; }  // (tri_plane(n) >= n n)
   static size_t bytes(int64_t n) {
-    return 3 * align_up(plane_bytes(n)) + align_up((size_t)n * 128 * tri_ldn(n) * 2) + align_up((size_t)tri_bias_elems(n, 4) * 2);
+    return 3 * align_up(plane_bytes(n)) + align_up((size_t)n * 128 * tri_ldn(n) * 2) + align_up((size_t)tri_bias_elems(n, 4) * 2) +
+           LOGIT_RING * logit_bytes(n, 16);
   }
+  // Pair logits of the last blocks, where the single track runs on a stream of its own.  With two buffers every block waits
+  // for the attention two blocks back, and an event recorded and waited for costs the host 13 us, where a launch costs 3.5:
+  // at 64 tokens the launches set the pace.  With eight it is one wait in four blocks (runs of 4 blocks, us a block: 93 -> 83).
+  static constexpr int LOGIT_RING = 8;
+  static size_t logit_bytes(int64_t n, int heads) { return align_up((size_t)heads * n * ((n + 3) / 4 * 4) * 4); }
+  float* ring(int64_t n) const { return reinterpret_cast<float*>(reinterpret_cast<char*>(bias) + align_up((size_t)tri_bias_elems(n, 4) * 2)); }
   bool carve(int64_t n, void* ws, size_t wsb) {
     Carver w(ws, wsb);
     qa = static_cast<bf16_t*>(w.take(plane_bytes(n)));
@@ -356,16 +363,32 @@ int af3_pairformer_stack_forward(
   hipStream_t main_s = static_cast<hipStream_t>(stream);
   hipStream_t side_s = single_stream ? static_cast<hipStream_t>(single_stream) : main_s;
   const bool two = side_s != main_s;
-  Event ready, read_done[2];  // behind the pair logits; behind the attention that reads logits buffer 0 / 1
+  // The pair logits of the run's k-th single track are in buffer k % buffers: two, the caller's, or at few tokens more of
+  // them in the workspace (which nothing else uses before the streams have been joined).
+  float* first = logits;
+  int buffers = num_blocks > 1 ? 2 : 1;
+  size_t logit_size = logits ? (size_t)blocks[0]->num_head * ((n + 3) / 4 * 4) * n : 0;
+  if (two && join) {
+    bool all = true;
+    for (int i = 0; i < num_blocks; ++i) all = all && pair_steps_apply(*blocks[i], n) && blocks[i]->num_head <= 16;
+    PairStepScratch w;
+    if (all && workspace_bytes >= PairStepScratch::bytes(n) && w.carve(n, workspace, workspace_bytes)) {
+      first = w.ring(n);
+      logit_size = PairStepScratch::logit_bytes(n, 16) / 4;
+      buffers = PairStepScratch::LOGIT_RING;
+    }
+  }
+  const int half = buffers > 1 ? buffers / 2 : 1;
+  Event ready, read_done[2];  // behind the pair logits; behind the last attention that reads a buffer of either half
   if (two) STEP(ready.order(main_s, side_s));
-  int rc = AF3_OK;
+  int rc = AF3_OK, k = 0;
   for (int i = 0; i < num_blocks && rc == AF3_OK; ++i) {
     const af3_pairformer_block& b = *blocks[i];
     float* lg = nullptr;
     Event* free = nullptr;
     if (b.with_single) {
-      lg = logits + (size_t)(num_blocks > 1 ? i & 1 : 0) * b.num_head * ((n + 3) / 4 * 4) * n;
-      free = &read_done[i & 1];
+      lg = first + (k % buffers) * logit_size;
+      if (k % half == 0) free = &read_done[k / half & 1];
     }
     // the pair logits are the only thing the single track reads of `pair`: they are made in front of whatever updates it next
     if (pair_steps_apply(b, n)) {
@@ -377,14 +400,15 @@ int af3_pairformer_stack_forward(
     } else {
       rc = pair_operators(b, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes, stream);
       if (rc != AF3_OK || !b.with_single) continue;
-      rc = free->wait(main_s);
+      if (free) rc = free->wait(main_s);
       if (rc == AF3_OK)
         rc = af3_pair_logits_quads_forward(pair, pair_dtype, b.sl_ln_w, b.sl_ln_b, b.sl_w, b.num_head, lg, n, stream);
     }
     if (rc == AF3_OK && two) rc = ready.order(main_s, side_s);
     if (rc == AF3_OK)
       rc = single_update(b, single, single_dtype, seq_mask, lg, n, single_workspace, single_workspace_bytes, side_s);
-    if (rc == AF3_OK && two && i + 2 < num_blocks) rc = read_done[i & 1].record(side_s);
+    if (rc == AF3_OK && two && k % half == half - 1 && i + half + 1 < num_blocks) rc = read_done[k / half & 1].record(side_s);
+    ++k;
   }
   if (two && join) {
     const int jrc = ready.order(side_s, main_s);

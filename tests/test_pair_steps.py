@@ -62,10 +62,11 @@ def test_steps_give_the_bits_of_one_kernel_per_operator(gpu_pkg, n, c, factor, h
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [5, 48, 130])
-def test_a_run_of_blocks_is_its_blocks_one_by_one(gpu_pkg, n):
-    """The last step of a block makes the next block's first operands: the same bits as a call per block."""
-    blocks, inputs = [_block(gpu_pkg, seed=i) for i in range(3)], _inputs(n, 128, torch.bfloat16, 2)
+@pytest.mark.parametrize("n,count", [(5, 3), (48, 19), (130, 10)])
+def test_a_run_of_blocks_is_its_blocks_one_by_one(gpu_pkg, n, count):
+    """The last step of a block makes the next block's first operands, and the buffers of the pair logits come round again
+    after eight blocks: the same bits as a call per block."""
+    blocks, inputs = [_block(gpu_pkg, seed=i) for i in range(count)], _inputs(n, 128, torch.bfloat16, 2)
     pair, mask, single, seq = inputs
     got = gpu_pkg.nn.pairformer_loop(blocks, pair.clone(), mask, single.clone(), seq)
     want = (pair, single)
