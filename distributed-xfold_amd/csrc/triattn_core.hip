@@ -9,10 +9,11 @@
 //   mask    : fp32 [N][N] 0/1 or null
 //
 // What sets the pace on this machine (measured): a wave64 exp2 occupies the SIMD's issue port
-// for 8 cycles, any other vector instruction for 4-5, a 32x32x16 MFMA for about 16 of the 32
-// cycles it takes in the matrix unit - and vector work of OTHER waves does not issue while a
-// wave has an MFMA waiting for the unit.  So vector and matrix work overlap only inside one
-// wave's own instruction stream.  The other cost is what a workgroup pulls in from L2 per key
+// for 8 cycles, any other vector instruction for 4-5, a 32x32x16 MFMA for 9 to 16 of the 32
+// cycles it takes in the matrix unit, whichever wave it comes from; what is left of them another
+// wave's vector instructions fill.  From some 700 tokens on the clock gives way as well (1.95 to
+// 2.07 GHz in this kernel, 2.35 in arithmetic alone), to the loads more than to the arithmetic.
+// The other cost is what a workgroup pulls in from L2 per key
 // tile: with every load taken out of the key-tile loop (operands reused, results wrong) the
 // kernel runs 30 % faster, 17 % of which remain when the same loads all hit the CU's own
 // cache, i.e. are the loads into LDS as such, the rest is the L2 traffic (8 KB of K / V^T per
@@ -121,7 +122,7 @@ __device__ __forceinline__ void scale_in_place(f32x16& o, float f) {
   }
 }
 
-template <int R, bool HAS_BIAS>
+template <int R, bool HAS_BIAS, bool SPARE>
 __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
   // [buffer][row] as separate arrays: a load in flight to one of them provably does not alias
   // a fragment read from another
@@ -159,8 +160,16 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
   if (pair_idx >= H * NG) return;
   const int rg = pair_idx / H;
   const int h = pair_idx % H;
-  const int q0 = qt * QW;
-  const int qw = q0 + wave * 32 + j;
+  // SPARE: the blocks of 32 queries leave some wave of a tile without one.  They are shared out evenly between the tiles
+  // of a (row group, head); a wave without a block takes part in the loads and the barriers only and leaves its SIMD to
+  // the other workgroup on the CU (which wave that is changes from workgroup to workgroup).  Computing on clamped queries
+  // instead, as the other form does where no wave is without: 387 tokens 106 us against 99, 450 131 against 129, 600
+  // 253 against 245; with a block for every wave the even form is the slower one, 768 tokens 434 against 430.
+  const int blocks = (N + 31) / 32, first = SPARE ? qt * blocks / QT : qt * 4;
+  const int turn = SPARE ? (wave + slot + (slot >> 5)) & 3 : wave;
+  const bool active = !SPARE || turn < (qt + 1) * blocks / QT - first;
+  const int qblk = active ? first + turn : first;
+  const int qw = active ? qblk * 32 + j : N;
   const int qi = min(qw, N - 1);
   const int nkt = (N + KT - 1) / KT;
   const int nk64 = nkt * KT;
@@ -293,9 +302,8 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
       dma16<0>(vglob[r], (uint32_t)(dv_row * ldn + (col < ldn ? col : 0)) * 2u, buf + wave * 1024);
     };
     // bias tiles of this wave's 32-query block: 4 KB per key tile
-    const int wave_blk = q0 + wave * 32 < N ? (q0 >> 5) + wave : 0;
     const char* bbase =
-        HAS_BIAS ? reinterpret_cast<const char*>(a.bias + tri_bias_offset(N, h, wave_blk * 32, 0)) : nullptr;
+        HAS_BIAS ? reinterpret_cast<const char*>(a.bias + tri_bias_offset(N, h, qblk * 32, 0)) : nullptr;
     // The bias tile of key tile t + 1 (four 1 KB fp16 fragments; fragment i = 2 u + st: keys
     // 32 u + 16 st + 8 hh .. + 8 of this lane's query, bytes 32 j + 16 hh of run i) is only ever
     // read by this wave, so it goes from memory straight into registers, requested when tile t
@@ -430,8 +438,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
       float linc = 0.f;
       // From here to the end: one basic block in a fixed order.  Each of the four P.V MFMAs of the
       // previous virtual tile is issued in front of eight exponentials of this one (the matrix
-      // unit works while the wave goes on issuing vector instructions; another wave's would not
-      // get in), with its V^T fragment read from LDS one group ahead.
+      // unit works while the wave goes on issuing vector instructions), with its V^T fragment read from LDS one group ahead.
       bf16x8 vf = lds16(vb + va[0]);
       u32x4 bfr[4];  // the next key tile's bias fragments (the last row of this one fetches them)
       if (HAS_BIAS && RR == R - 1) {
@@ -570,16 +577,35 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
       t_n2 = pop();
     };
     int last_ph = 0;
-    while (true) {
-      step(std::integral_constant<int, 0>{});
-      last_ph = 0;
-      if (t_cur >= nkt) break;
-      step(std::integral_constant<int, 1>{});
-      last_ph = 1;
-      if (t_cur >= nkt) break;
+    if (SPARE && !active) {
+      // the loads and barriers of the steps
+      for (int ph = 0; t_cur < nkt; ph ^= 1) {
+        dma_barrier();
+        if (R == 2) {
+          dma_k(t_n1, R - 1, ph == 0 ? KBUF(1, R - 1) : KBUF(0, R - 1));
+          dma_k(t_n2, 0, ph == 0 ? KBUF(0, 0) : KBUF(1, 0));
+          dma_v(t_n1, 0, ph == 0 ? VBUF(1, 0) : VBUF(0, 0));
+          dma_v(t_n1, R - 1, ph == 0 ? VBUF(1, R - 1) : VBUF(0, R - 1));
+        } else {
+          dma_k(t_n1, 0, ph == 0 ? KBUF(1, 0) : KBUF(0, 0));
+          dma_v(t_cur, 0, ph == 0 ? VBUF(0, 0) : VBUF(1, 0));
+        }
+        t_cur = t_n1;
+        t_n1 = t_n2;
+        t_n2 = pop();
+      }
+    } else {
+      while (true) {
+        step(std::integral_constant<int, 0>{});
+        last_ph = 0;
+        if (t_cur >= nkt) break;
+        step(std::integral_constant<int, 1>{});
+        last_ph = 1;
+        if (t_cur >= nkt) break;
+      }
     }
     dma_barrier();  // every load into LDS has landed (none is in flight when the workgroup ends)
-    drain(last_ph == 0 ? VBUF(0, R - 1) : VBUF(1, R - 1));
+    if (active) drain(last_ph == 0 ? VBUF(0, R - 1) : VBUF(1, R - 1));
     if (pass == 1) break;
     // (lanes of queries past the end work on clamped operands and, in a partly filled bias block, on
     // bias values nobody wrote: they have no say)
@@ -689,12 +715,9 @@ int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream) {
     }
     hipLaunchKernelGGL(kernel, grid, block, dyn, stream, a);
   };
-  if (R == 2) {
-    if (a.bias) launch(triattn_flash_kernel<2, true>);
-    else launch(triattn_flash_kernel<2, false>);
-  } else {
-    if (a.bias) launch(triattn_flash_kernel<1, true>);
-    else launch(triattn_flash_kernel<1, false>);
-  }
+  const bool spare = (a.N + 31) / 32 % 4 != 0;
+  if (!a.bias) launch(R == 2 ? triattn_flash_kernel<2, false, false> : triattn_flash_kernel<1, false, false>);
+  else if (R == 2) launch(spare ? triattn_flash_kernel<2, true, true> : triattn_flash_kernel<2, true, false>);
+  else launch(spare ? triattn_flash_kernel<1, true, true> : triattn_flash_kernel<1, true, false>);
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
