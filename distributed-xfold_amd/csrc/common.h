@@ -153,6 +153,17 @@ __device__ __forceinline__ float group16_sum(float v) {
   v += dpp_mov<0x124>(v); v += dpp_mov<0x128>(v);
   return v;
 }
+// the same over each aligned group of 8 lanes (row_half_mirror: the other quad of the eight)
+__device__ __forceinline__ float group8_sum(float v) {
+  v += dpp_mov<0xB1>(v); v += dpp_mov<0x4E>(v);
+  return v + dpp_mov<0x141>(v);
+}
+template <int LANES>
+__device__ __forceinline__ float group_sum(float v) {
+  static_assert(LANES == 16 || LANES == 8, "lanes");
+  if constexpr (LANES == 16) return group16_sum(v);
+  else return group8_sum(v);
+}
 // Exchange with the other half of the wave (lane l <-> lane l ^ 32) through
 // ds_bpermute with the byte address computed once per kernel:
 //   const int xaddr = half_swap_addr();  ...  other = half_swap(xaddr, mine);

@@ -180,12 +180,12 @@ int launch_atom_pair_cond(const float* row, const float* col, const float* tp, c
 // the same arithmetic bit for bit.
 struct LnWidth {
   float inv_c = 1.f / 128.f;  // 1 / valid channels
-  float pad = 0.f;            // 128 - valid channels
+  float pad = 0.f;            // channels (128) - valid channels
 };
-inline LnWidth ln_width(int valid) {
+inline LnWidth ln_width(int valid, int channels = 128) {
   LnWidth w;
   w.inv_c = 1.f / (float)valid;
-  w.pad = (float)(128 - valid);
+  w.pad = (float)(channels - valid);
   return w;
 }
 
@@ -350,7 +350,7 @@ struct TriAttnArgs {
   const uint16_t* bias = nullptr;  // fp16 bits, fragment order (tri_bias_offset), or null
   const float* mask = nullptr;   // [N][N] 0/1 or null
   bf16_t* og = nullptr;          // [(b*N + s)][128] normalised attention output (the gate is applied by attn_out)
-  int N = 0;
+  int N = 0, head_dim = 32;      // head_dim 32 or 16: q, k [b][h][s][head_dim], vt [b][h][head_dim][ldn], og rows of 4 head_dim
   int64_t ldn = 0;
 };
 int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream);
@@ -358,15 +358,17 @@ int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream);
 // --------------------------------------------------------------- pair_step.hip
 // One run of per-pixel operators between two long products (contraction, attention core), in place on `pair`.
 enum {
+  PAIR_STEP_FIRST,          // the outgoing prologue alone (64 channels)
   PAIR_STEP_INCOMING,       // outgoing epilogue, incoming prologue
   PAIR_STEP_PROJECT_START,  // incoming epilogue, starting-node projections
   PAIR_STEP_PROJECT_END,    // starting-node output, ending-node projections
   PAIR_STEP_LAST,           // ending-node output, transition (and pair logits)
   PAIR_STEP_NEXT,           // the same, and the outgoing prologue of the block that follows
 };
-constexpr int PAIR_STEP_MAX_HIDDEN = 512;  // hidden units of the transition
+inline int pair_step_max_hidden(int channels) { return channels == 128 ? 512 : 128; }  // hidden units of the transition
 struct PairStepArgs {
   LnWidth lw;
+  int channels = 128;  // of the pair tensor and the weights, 128 or 64
   int valid_c = 128, io_f32 = 0, N = 0, Np = 0, ldn = 0, hidden = 0, logit_heads = 0;
   int64_t plane = 0;
   void* pair = nullptr;

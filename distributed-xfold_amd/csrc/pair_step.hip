@@ -1,4 +1,4 @@
-// Steps of the 128-channel pair path at few tokens: the operators between two long products, one kernel.
+// Steps of the pair path, 128 channels at few tokens and 64 channels: the operators between two long products, one kernel.
 //
 // Up to some two hundred tokens the pair tensor is a few hundred tiles of 128 positions, and a kernel of pair_tile.hip is
 // one tile's chain of loads, LayerNorm, products and stores, run by a part of the CUs while the rest idles: at 64 tokens
@@ -22,6 +22,12 @@
 //   outgoing epilogue + incoming prologue 10.8 / 20.3 (11.6 + 6.7 / 12.3 + 13.2), in patches of 4 x 8 / 8 x 8 pixels
 //   incoming epilogue + projections 8.7 / 18.9 (11.6 + 7.7 / 12.3 + 13.5), output + projections 8.2 / 18.4 (10.0 + 7.7 / 10.7 + 13.5)
 //   output + transition + logits + prologue 14.3 / 35 (10.0 + 15.8 + 4.6 + 6.7 / 10.7 + 19.1 + 5.0 + 13.2)
+//
+// 64 channels (the template embedding): workgroups of two waves, otherwise the same code.  A quarter of the weights to a
+// position and half of the rest, so that here the steps are the faster form whatever the number of tokens, and the tensor
+// need not be padded to 128 channels and back (bf16, 301 tokens, us a block: 345 -> 221, 768: 1940 -> 1460; kernel alone
+// at 301, bound by what it moves, 25 to 40 MB, and vector issue: outgoing prologue 13, outgoing epilogue + incoming
+// prologue 31 (8 x 8 patches 36: twice the accumulators cost the third workgroup of a SIMD), the other steps 20 to 21).
 // Tiles of 64 positions (half the weights a position) run slower up to 128 tokens and no faster at 160 to 256, but for the
 // patches.
 #include <type_traits>
@@ -32,9 +38,11 @@
 
 namespace {
 
-constexpr int H = 4, D = 32;
-constexpr int MAX_HIDDEN = PAIR_STEP_MAX_HIDDEN, HIDDEN_CHUNK = 256;
-enum { IN_EPILOGUE, IN_ATTENTION };
+constexpr int H = 4;
+// hidden units of the transition: a chunk, and how many of them there are room for
+constexpr int hidden_chunk_of(int channels) { return 2 * channels; }
+constexpr int hidden_chunks(int channels) { return channels == 128 ? 2 : 1; }
+enum { IN_NONE, IN_EPILOGUE, IN_ATTENTION };
 enum { MAP_ROWS, MAP_COLUMNS, MAP_PATCH };
 enum { NEXT_NONE, NEXT_PROLOGUE, NEXT_PROJECT };
 
@@ -103,11 +111,14 @@ __device__ __forceinline__ void load_frags(const bf16_t* w, int blk, int nks, in
 #pragma unroll
   for (int i = 0; i < n; ++i) f[i] = as_frag(*reinterpret_cast<const u32x4*>(at32(p + i * 512, (uint32_t)lane * 8u)));
 }
-template <typename TIO, int PB, int IN, int MAP, bool TRANSITION, int NEXT>
-__global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
+template <typename TIO, int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT>
+__global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(PairStepArgs a) {
   using E = Elem<TIO>;
   constexpr int TS = 32 * PB;           // positions per tile, in blocks of an MFMA's 32
-  constexpr int NB = PB == 1 && !TRANSITION ? 4 : 3;  // weight octets in flight
+  constexpr int C = CH, D = C / H, LDX = C + 8, LDS_F = C + 4;
+  constexpr int WAVES = C / 32, NT = 2 * C, CHUNKS = C / 8, KS = C / 16;
+  constexpr int HIDDEN_CHUNK = hidden_chunk_of(C), MAX_HIDDEN = HIDDEN_CHUNK * hidden_chunks(C);
+  constexpr int NB = C == 64 || (PB == 1 && !TRANSITION) ? 4 : 3;  // pieces of the weights in flight
   constexpr int LDT = TS + 2;           // LDS row stride (bf16) of a channel's positions: the 16 lanes of a pixel, 8 channels apart, on 8 banks
   constexpr int LDH = HIDDEN_CHUNK + 8;
   constexpr int U_BYTES = TS * LDS_F * 4;
@@ -122,7 +133,7 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
   bf16_t* const sH = reinterpret_cast<bf16_t*>(sU);  // a chunk of the transition's hidden layer, [LDS row][unit]
   const int tid = threadIdx.x, lane = tid & 63, hh = lane >> 5, j = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int chunk = tid & 15, prow = tid >> 4;  // as in load_ln_tile: eight channels of rows prow, prow + 16, ..
+  const int chunk = tid % CHUNKS, prow = tid / CHUNKS;  // as in load_ln_tile: eight channels of rows prow, prow + 16, ..
 
   StepTile<PB, MAP> t;
   t.N = a.N;
@@ -157,23 +168,24 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
   f32x4 param = {0.f, 0.f, 0.f, 0.f};
   {
     // arrays 0, 1: input norm; 2, 3: contraction's or transition's; 4, 5: last stage's; 6, 7: logits'
-    const float* const lo = wave == 0 ? a.ln1_w : wave == 1 ? (IN == IN_EPILOGUE ? a.ln_c_w : a.ln2_w) : wave == 2 ? a.ln3_w : a.sl_ln_w;
-    const float* const hi = wave == 0 ? a.ln1_b : wave == 1 ? (IN == IN_EPILOGUE ? a.ln_c_b : a.ln2_b) : wave == 2 ? a.ln3_b : a.sl_ln_b;
-    const float* const src = lane < 32 ? lo : hi;
-    if (src) param = *reinterpret_cast<const f32x4*>(src + j * 4);
+    const int n = tid / (C / 4);
+    const float* const w = n < 2 ? a.ln1_w : n < 4 ? (IN == IN_EPILOGUE ? a.ln_c_w : a.ln2_w) : n < 6 ? a.ln3_w : a.sl_ln_w;
+    const float* const b = n < 2 ? a.ln1_b : n < 4 ? (IN == IN_EPILOGUE ? a.ln_c_b : a.ln2_b) : n < 6 ? a.ln3_b : a.sl_ln_b;
+    const float* const src = (n & 1) ? b : w;
+    if (src) param = *reinterpret_cast<const f32x4*>(src + tid % (C / 4) * 4);
   }
   u32x4 tt[2 * PB];
   u32x4 og[PB][2];
   if constexpr (IN == IN_EPILOGUE) {
 #pragma unroll
     for (int u = 0; u < 2 * PB; ++u) {
-      const int idx = tid + 256 * u, c = idx / (4 * PB);
+      const int idx = tid + NT * u, c = idx / (4 * PB);
       const Pixel x = t.at(idx % (4 * PB) * 8);
       const bool ok = x.o < a.N && x.r < a.Np && c < a.valid_c;  // (positions past N in the row: zeroed with their pixel)
       tt[u] = *reinterpret_cast<const u32x4*>(at32(a.t_buf, ok ? (uint32_t)(c * plane + x.o * a.Np + x.r) : 0u));
       if (!ok) tt[u] = u32x4{0u, 0u, 0u, 0u};
     }
-  } else {
+  } else if constexpr (IN == IN_ATTENTION) {
     // the attention output lies in the frame of the operator that made it: starting node (rows) before a step over
     // columns, ending node (columns) before a step over rows
 #pragma unroll
@@ -191,39 +203,39 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
     }
   }
 
-  // The wave's weights, eight fragments (32 rows, 8 k-steps) at a time, in the order of their use; octet n + NB is asked for
-  // as soon as octet n has been multiplied.
-  constexpr int OCT_LOGITS = TRANSITION ? 2 + 6 * (MAX_HIDDEN / HIDDEN_CHUNK) : 2, OCT_NEXT = OCT_LOGITS + (TRANSITION ? 1 : 0);
+  // The wave's weights, 32 rows of all k-steps (eight fragments or four) at a time, in the order of their use; piece n + NB
+  // is asked for as soon as piece n has been multiplied.
+  constexpr int OCT_HIDDEN = IN == IN_NONE ? 0 : 2, OCT_LOGITS = OCT_HIDDEN + (TRANSITION ? 6 * hidden_chunks(C) : 0);
+  constexpr int OCT_NEXT = OCT_LOGITS + (TRANSITION && C == 128 ? 1 : 0);
   constexpr int OCTETS = OCT_NEXT + (NEXT == NEXT_NONE ? 0 : 4);
   const int pg = (wave >> 1) * 4 + (wave & 1);  // 32 projection rows; the gate rows that go with them are two blocks on
   const int n_hidden = a.hidden >> 5, nks = a.hidden >> 4;
-  bf16x8 w[NB][8];
+  bf16x8 w[NB][KS];
   auto fetch = [&](auto n_c) {
     constexpr int n = decltype(n_c)::value;
     if constexpr (n < OCTETS) {
       bf16x8* const d = w[n % NB];
-      if constexpr (n == 0) load_frags<8>(a.f_gate, wave, 8, 0, lane, d);
-      else if constexpr (n == 1) load_frags<8>(a.f_out, wave, 8, 0, lane, d);
+      if constexpr (n < OCT_HIDDEN) load_frags<KS>(n == 0 ? a.f_gate : a.f_out, wave, KS, 0, lane, d);
       else if constexpr (n < OCT_LOGITS) {
-        constexpr int c = (n - 2) / 6, r = (n - 2) % 6;
+        constexpr int c = (n - OCT_HIDDEN) / 6, r = (n - OCT_HIDDEN) % 6;
         if constexpr (r < 4) {
           // hidden block hb of 32 units: rows 32 (hb & 1) of the 64 "a" rows of chunk hb / 2, then of its 64 "b" rows
-          const int hb = min(c * (HIDDEN_CHUNK / 32) + wave + 4 * (r >> 1), n_hidden - 1);
-          load_frags<8>(a.f_w1, (hb >> 1) * 4 + (hb & 1) + 2 * (r & 1), 8, 0, lane, d);
+          const int hb = min(c * (HIDDEN_CHUNK / 32) + wave + WAVES * (r >> 1), n_hidden - 1);
+          load_frags<KS>(a.f_w1, (hb >> 1) * 4 + (hb & 1) + 2 * (r & 1), KS, 0, lane, d);
         } else {
-          constexpr int k0 = c * (HIDDEN_CHUNK / 16) + (r - 4) * 8;  // (k-steps come in fours)
-          load_frags<4>(a.f_w2, wave, nks, min(k0, nks - 4), lane, d);
-          load_frags<4>(a.f_w2, wave, nks, min(k0 + 4, nks - 4), lane, d + 4);
+          constexpr int k0 = c * (HIDDEN_CHUNK / 16) + (r - 4) * KS;  // (k-steps come in fours)
+#pragma unroll
+          for (int q = 0; q < KS; q += 4) load_frags<4>(a.f_w2, wave, nks, min(k0 + q, nks - 4), lane, d + q);
         }
       } else if constexpr (n < OCT_NEXT) {
-        if (a.logits && wave * 32 < a.logit_heads) load_frags<8>(a.f_logits, wave, 8, 0, lane, d);
+        if (a.logits && wave * 32 < a.logit_heads) load_frags<KS>(a.f_logits, wave, KS, 0, lane, d);
       } else if constexpr (NEXT == NEXT_PROLOGUE) {
         constexpr int r = n - OCT_NEXT;
-        load_frags<8>(a.f_next, pg + (r & 1) * 2 + (r >> 1) * 8, 8, 0, lane, d);
+        load_frags<KS>(a.f_next, pg + (r & 1) * 2 + (r >> 1) * (C / 16), KS, 0, lane, d);
       } else {
         constexpr int r = n - OCT_NEXT;
-        if constexpr (r < 2) load_frags<8>(a.f_next, 4 * r + wave, 8, 0, lane, d);
-        else if (r == 2 || wave == 0) load_frags<8>(a.f_v, r == 2 ? wave : 4, 8, 0, lane, d);
+        if constexpr (r < 2) load_frags<KS>(a.f_next, WAVES * r + wave, KS, 0, lane, d);
+        else if (r == 2 || wave == 0) load_frags<KS>(a.f_v, r == 2 ? wave : WAVES, KS, 0, lane, d);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -237,21 +249,23 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
   // which reach each stage at about the same time, find it in L2.
   uint32_t warm = 0u;
   {
-    const uint32_t line = (blockIdx.x >> 3) * 256u + (uint32_t)tid;
-    const uint32_t n0 = TRANSITION ? (uint32_t)a.hidden * 4u : 0u, n1 = TRANSITION ? (uint32_t)a.hidden * 2u : 0u;  // 2 lines a row
-    constexpr uint32_t n2 = NEXT == NEXT_PROLOGUE ? 1024u : NEXT == NEXT_PROJECT ? 512u : 0u, n3 = NEXT == NEXT_PROJECT ? 320u : 0u;
+    constexpr uint32_t LINES = C / 64;  // a row of C
+    const uint32_t line = (blockIdx.x >> 3) * (uint32_t)NT + (uint32_t)tid;
+    const uint32_t n0 = TRANSITION ? (uint32_t)a.hidden * 2u * LINES : 0u, n1 = TRANSITION ? (uint32_t)a.hidden * LINES : 0u;
+    constexpr uint32_t n2 = NEXT == NEXT_PROLOGUE ? 4 * C * LINES : NEXT == NEXT_PROJECT ? 2 * C * LINES : 0u;
+    constexpr uint32_t n3 = NEXT == NEXT_PROJECT ? (C + 32) * LINES : 0u;
     const bf16_t* const from = line < n0 ? a.f_w1 : line < n0 + n1 ? a.f_w2 - n0 * 64 : line < n0 + n1 + n2 ? a.f_next - (n0 + n1) * 64
                                                                                              : a.f_v - (n0 + n1 + n2) * 64;
     if (line < n0 + n1 + n2 + n3) warm = *reinterpret_cast<const uint32_t*>(from + line * 64u);
   }
   __builtin_amdgcn_sched_barrier(0);
 
-  bf16x8 xf[PB][8];
+  bf16x8 xf[PB][KS];
   auto frags_of = [&](const bf16_t* s) {
 #pragma unroll
     for (int b = 0; b < PB; ++b)
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) xf[b][ks] = lds_frag(s, LDX, 32 * b, ks * 16, lane);
+      for (int ks = 0; ks < KS; ++ks) xf[b][ks] = lds_frag(s, LDX, 32 * b, ks * 16, lane);
   };
   // octet n (32 rows) x the tile: T form (a lane owns a position), D form (a lane owns a channel)
   // (`tile`: its fragments come out of LDS one by one, where there are no registers to hold them)
@@ -263,13 +277,17 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks)
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int b = 0; b < PB; ++b) {
         const bf16x8 x = tile ? lds_frag(tile, LDX, 32 * b, ks * 16, lane) : xf[b][ks];
         acc[b] = decltype(d_form)::value ? mfma32(x, wn[ks], acc[b]) : mfma32(wn[ks], x, acc[b]);
       }
     fetch(OCTET(n + NB));
+  };
+  auto sum_channels = [](float v) {
+    if constexpr (CHUNKS == 16) return sum_chunks(v);
+    else return group8_sum(v);
   };
   using T_form = std::false_type;
   using D_form = std::true_type;
@@ -279,7 +297,7 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
     load_param8(sP + (2 * which + 1) * C + chunk * 8, 0.f, lb);
 #pragma unroll
     for (int u = 0; u < 2 * PB; ++u) {
-      u32x4 pk = ln_pixel8<TIO>(raw[u], lw, lb, false, a.lw.inv_c, a.lw.pad);
+      u32x4 pk = ln_pixel8<TIO, CHUNKS>(raw[u], lw, lb, false, a.lw.inv_c, a.lw.pad);
       if (!mine[u].ok) pk = u32x4{0u, 0u, 0u, 0u};
       *reinterpret_cast<u32x4*>(dst + (prow + 16 * u) * LDX + chunk * 8) = pk;
     }
@@ -306,22 +324,24 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
     }
   };
 
-  // ---- gate and output projection of the operator before ----
-  *reinterpret_cast<f32x4*>(sP + (tid >> 5) * C + j * 4) = param;
+  *reinterpret_cast<f32x4*>(sP + tid * 4) = param;
+  if (NEXT == NEXT_PROLOGUE && tid < TS) sMask[tid] = mk;
   lds_barrier();
+  f32x16 acc[PB];
+  // ---- gate and output projection of the operator before ----
+  if constexpr (IN != IN_NONE) {
   norm(0, sA);
   if constexpr (IN == IN_EPILOGUE) {
 #pragma unroll
     for (int u = 0; u < 2 * PB; ++u) {
-      const int idx = tid + 256 * u;
+      const int idx = tid + NT * u;
       uint32_t* const d = reinterpret_cast<uint32_t*>(sT + idx / (4 * PB) * LDT + idx % (4 * PB) * 8);
       d[0] = tt[u].x; d[1] = tt[u].y; d[2] = tt[u].z; d[3] = tt[u].w;
     }
   }
-  if (NEXT == NEXT_PROLOGUE && tid < TS) sMask[tid] = mk;
   lds_barrier();
   frags_of(sA);
-  f32x16 gate[PB], acc[PB];
+  f32x16 gate[PB];
   product(OCTET(0), T_form{}, gate);
   if constexpr (IN == IN_EPILOGUE) {
     // LayerNorm of the contraction's result over its channels
@@ -337,10 +357,10 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
         v[e] = bf2f(sT[(chunk * 8 + e) * LDT + pos]);
         s1 += v[e];
       }
-      const float mean = sum_chunks(s1) * a.lw.inv_c;
+      const float mean = sum_channels(s1) * a.lw.inv_c;
 #pragma unroll
       for (int e = 0; e < 8; ++e) { const float d = v[e] - mean; s2 = fmaf(d, d, s2); }
-      const float rstd = rsqrtf((sum_chunks(s2) - a.lw.pad * mean * mean) * a.lw.inv_c + LN_EPS);
+      const float rstd = rsqrtf((sum_channels(s2) - a.lw.pad * mean * mean) * a.lw.inv_c + LN_EPS);
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = mine[u].ok ? (v[e] - mean) * rstd * lw[e] + lb[e] : 0.f;
       *reinterpret_cast<u32x4*>(sB + p * LDX + chunk * 8) = pack8(o);
@@ -372,6 +392,7 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
       for (int r = 0; r < 16; ++r) acc[b][r] *= gate[b][r];
   }
   add_to_stream(acc);  // (sT was last read in front of the barrier above)
+  }
 
   // ---- transition, a chunk of the hidden layer at a time ----
   if constexpr (TRANSITION) {
@@ -385,14 +406,14 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) sum[b][r] = 0.f;
     auto hidden_chunk = [&](auto c_c) {
-      constexpr int c = decltype(c_c)::value, n0 = 2 + 6 * c;
+      constexpr int c = decltype(c_c)::value, n0 = OCT_HIDDEN + 6 * c;
       if (c > 0) lds_barrier();  // the chunk before has been multiplied
       auto block = [&](auto i_c) {
         constexpr int i = decltype(i_c)::value;
         f32x16 y[PB];
         product(OCTET(n0 + 2 * i), T_form{}, acc, tile);
         product(OCTET(n0 + 2 * i + 1), T_form{}, y, tile);
-        if (c * (HIDDEN_CHUNK / 32) + wave + 4 * i < n_hidden) {
+        if (c * (HIDDEN_CHUNK / 32) + wave + WAVES * i < n_hidden) {
 #pragma unroll
           for (int b = 0; b < PB; ++b)
 #pragma unroll
@@ -403,7 +424,7 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
               u32x2 v;
               v.x = pack2bf(h[0], h[1]);
               v.y = pack2bf(h[2], h[3]);
-              *reinterpret_cast<u32x2*>(sH + (32 * b + j) * LDH + (wave + 4 * i) * 32 + 8 * g + 4 * hh) = v;
+              *reinterpret_cast<u32x2*>(sH + (32 * b + j) * LDH + (wave + WAVES * i) * 32 + 8 * g + 4 * hh) = v;
             }
         }
       };
@@ -414,44 +435,45 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
       auto second = [&](auto h_c) {
         constexpr int h = decltype(h_c)::value, n = n0 + 4 + h;
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (c * (HIDDEN_CHUNK / 16) + 8 * h + k < nks)
+        for (int k = 0; k < KS; ++k)
+          if (c * (HIDDEN_CHUNK / 16) + KS * h + k < nks)
 #pragma unroll
-            for (int b = 0; b < PB; ++b) sum[b] = mfma32(w[n % NB][k], lds_frag(sH, LDH, 32 * b, (8 * h + k) * 16, lane), sum[b]);
+            for (int b = 0; b < PB; ++b) sum[b] = mfma32(w[n % NB][k], lds_frag(sH, LDH, 32 * b, (KS * h + k) * 16, lane), sum[b]);
         fetch(OCTET(n + NB));
       };
       second(std::integral_constant<int, 0>{});
       second(std::integral_constant<int, 1>{});
     };
-    static_assert(MAX_HIDDEN == 2 * HIDDEN_CHUNK, "two chunks");
     hidden_chunk(std::integral_constant<int, 0>{});
-    hidden_chunk(std::integral_constant<int, 1>{});
+    if constexpr (hidden_chunks(C) > 1) hidden_chunk(std::integral_constant<int, 1>{});
     lds_barrier();  // every wave is done with the hidden layer
     add_to_stream(sum);
   }
+  if constexpr (IN != IN_NONE)
 #pragma unroll
   for (int u = 0; u < 2 * PB; ++u)
     if (mine[u].ok) store_raw<TIO>(at32(pair, t.pix(mine[u]) * C + chunk * 8), raw[u]);
   asm volatile("" ::"v"(warm));
   if constexpr (NEXT == NEXT_NONE)
-    if (!a.logits) return;
+    if (C != 128 || !a.logits) return;
 
   // ---- what the next long product takes ----
   if constexpr (NEXT != NEXT_NONE) norm(2, sA);
-  if (TRANSITION && a.logits) norm(3, sB);
+  if constexpr (TRANSITION && C == 128)
+    if (a.logits) norm(3, sB);
   lds_barrier();
-  if constexpr (TRANSITION) {
+  if constexpr (TRANSITION && C == 128) {
     // pair logits with quads of keys outermost, [head][key / 4][query][key % 4], keys past the end of the last quad zero
     const int quads = (a.N + 3) >> 2;
-    for (int blk = wave; a.logits && blk * 32 < a.logit_heads; blk += 4) {
-      if (blk > 3) load_frags<8>(a.f_logits, blk, 8, 0, lane, w[OCT_LOGITS % NB]);
+    for (int blk = wave; a.logits && blk * 32 < a.logit_heads; blk += WAVES) {
+      if (blk >= WAVES) load_frags<KS>(a.f_logits, blk, KS, 0, lane, w[OCT_LOGITS % NB]);
       frags_of(sB);
 #pragma unroll
       for (int b = 0; b < PB; ++b) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) acc[b] = mfma32(w[OCT_LOGITS % NB][ks], xf[b][ks], acc[b]);
+        for (int ks = 0; ks < KS; ++ks) acc[b] = mfma32(w[OCT_LOGITS % NB][ks], xf[b][ks], acc[b]);
         if (own[b].o < a.N && own[b].r < quads * 4) {
           float* const d = at32(a.logits, (uint32_t)((own[b].r >> 2) * a.N * 4 + own[b].o * 4 + (own[b].r & 3)));
 #pragma unroll
@@ -516,20 +538,20 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
   }
   if constexpr (NEXT == NEXT_PROJECT) {
     frags_of(sA);
-    // a wave is one head: q, k in T form, v in D form
+    // a wave is one head of 32 or two of 16: q, k in T form, v in D form
     auto qk = [&](auto c_c) {
       constexpr int c = decltype(c_c)::value;
       product(OCTET(OCT_NEXT + c), T_form{}, acc);
 #pragma unroll
       for (int b = 0; b < PB; ++b)
         if (own[b].ok) {
-          bf16_t* const dst = at32(c == 0 ? a.q : a.k, (uint32_t)((own[b].o * H + wave) * a.N + own[b].r) * D + 8 * hh);
+          bf16_t* const dst = at32(c == 0 ? a.q : a.k, (uint32_t)((own[b].o * H + wave * (32 / D)) * a.N + own[b].r) * D + 8 * hh);
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
             float f[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) f[e] = c == 0 ? acc[b][8 * u + e] * a.q_scale : acc[b][8 * u + e];
-            *reinterpret_cast<u32x4*>(dst + 16 * u) = pack8(f);
+            *reinterpret_cast<u32x4*>(dst + (D == 32 ? 16 * u : u * a.N * D)) = pack8(f);
           }
         }
     };
@@ -538,10 +560,10 @@ __global__ __launch_bounds__(256, 2) void pair_step_kernel(PairStepArgs a) {
     product(OCTET(OCT_NEXT + 2), D_form{}, acc);
 #pragma unroll
     for (int b = 0; b < PB; ++b) {
-      // channel j of head `wave`, positions 16 hh ..; the middle quads of a group of 16 keys change places (tri_vt_pos)
+      // channel j of the wave's 32, positions 16 hh ..; the middle quads of a group of 16 keys change places (tri_vt_pos)
       const Pixel x = t.at(32 * b + 16 * hh);
       if (x.o < a.N) {
-        bf16_t* const dst = at32(a.vt, (uint32_t)(((x.o * H + wave) * D + j) * a.ldn + x.r));
+        bf16_t* const dst = at32(a.vt, (uint32_t)((x.o * C + wave * 32 + j) * a.ldn + x.r));
         const float lo[8] = {acc[b][0], acc[b][1], acc[b][2], acc[b][3], acc[b][8], acc[b][9], acc[b][10], acc[b][11]};
         const float hi[8] = {acc[b][4], acc[b][5], acc[b][6], acc[b][7], acc[b][12], acc[b][13], acc[b][14], acc[b][15]};
         *reinterpret_cast<u32x4*>(dst) = pack8(lo);
@@ -575,36 +597,50 @@ bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // pieces.
 constexpr int64_t WIDE_PATCHES = 256 * 64;
 
-template <int PB, int IN, int MAP, bool TRANSITION, int NEXT>
+template <int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT>
 int launch_tiles(const PairStepArgs& a, hipStream_t s) {
   const int64_t blocks = MAP == MAP_PATCH ? ((int64_t)(a.Np / (4 * PB)) * (a.Np / 8) + 7) / 8 * 8 : ((int64_t)a.N * a.ldn + 32 * PB - 1) / (32 * PB);
   if (blocks <= 0 || blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
-  const dim3 grid((unsigned)blocks), block(256);
-  if (a.io_f32) hipLaunchKernelGGL((pair_step_kernel<float, PB, IN, MAP, TRANSITION, NEXT>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((pair_step_kernel<bf16_t, PB, IN, MAP, TRANSITION, NEXT>), grid, block, 0, s, a);
+  const dim3 grid((unsigned)blocks), block(2 * CH);
+  if (a.io_f32) hipLaunchKernelGGL((pair_step_kernel<float, CH, PB, IN, MAP, TRANSITION, NEXT>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((pair_step_kernel<bf16_t, CH, PB, IN, MAP, TRANSITION, NEXT>), grid, block, 0, s, a);
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
 }  // namespace
 
 int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s) {
-  if (a.N <= 0 || a.N > 8192 || a.Np < a.N || (a.Np & 7) || a.ldn != tri_ldn(a.N) || !a.pair || !a.f_gate || !a.f_out || !a.ln1_w ||
-      !a.ln1_b || !al16(a.pair) || !al16(a.f_gate) || !al16(a.f_out))
+  if (a.N <= 0 || a.N > 8192 || a.Np < a.N || (a.Np & 7) || a.ldn != tri_ldn(a.N) || !a.pair || !al16(a.pair) ||
+      (a.channels != 128 && a.channels != 64) || a.valid_c < 1 || a.valid_c > a.channels)
     return AF3_ERR_BAD_ARG;
-  const bool epilogue = step <= PAIR_STEP_PROJECT_START, prologue = step == PAIR_STEP_INCOMING || step == PAIR_STEP_NEXT;
+  // every array is addressed with 32 bits
+  if (a.plane * a.channels * 2 >= (1ll << 32) || (int64_t)a.N * a.ldn * a.channels * (a.io_f32 ? 4 : 2) >= (1ll << 32)) return AF3_ERR_BAD_ARG;
+  const bool first = step == PAIR_STEP_FIRST, epilogue = step == PAIR_STEP_INCOMING || step == PAIR_STEP_PROJECT_START;
+  const bool prologue = first || step == PAIR_STEP_INCOMING || step == PAIR_STEP_NEXT;
   const bool project = step == PAIR_STEP_PROJECT_START || step == PAIR_STEP_PROJECT_END, transition = step >= PAIR_STEP_LAST;
-  if (epilogue ? !a.t_buf || !a.ln_c_w || !a.ln_c_b || a.plane < tri_plane(a.N) || a.valid_c < 1 || a.valid_c > C : !a.og) return AF3_ERR_BAD_ARG;
+  if (!first && (!a.f_gate || !a.f_out || !a.ln1_w || !a.ln1_b || !al16(a.f_gate) || !al16(a.f_out))) return AF3_ERR_BAD_ARG;
+  if (epilogue && (!a.t_buf || !a.ln_c_w || !a.ln_c_b || a.plane < tri_plane(a.N))) return AF3_ERR_BAD_ARG;
+  if (!epilogue && !first && !a.og) return AF3_ERR_BAD_ARG;
   if (prologue && (!a.a_buf || !a.b_buf || !a.f_next || !a.ln3_w || !a.ln3_b || a.plane < tri_plane(a.N))) return AF3_ERR_BAD_ARG;
   if (project && (!a.q || !a.k || !a.vt || !a.bias || !a.f_next || !a.f_v || !a.ln3_w || !a.ln3_b)) return AF3_ERR_BAD_ARG;
-  if (transition && (!a.f_w1 || !a.f_w2 || !a.ln2_w || !a.ln2_b || a.hidden <= 0 || (a.hidden & 63) || a.hidden > MAX_HIDDEN)) return AF3_ERR_BAD_ARG;
-  if (a.logits && (!transition || !a.f_logits || !a.sl_ln_w || !a.sl_ln_b || a.logit_heads <= 0)) return AF3_ERR_BAD_ARG;
-  switch (step) {
+  if (transition && (!a.f_w1 || !a.f_w2 || !a.ln2_w || !a.ln2_b || a.hidden <= 0 || (a.hidden & 63) || a.hidden > pair_step_max_hidden(a.channels)))
+    return AF3_ERR_BAD_ARG;
+  if (a.logits && (a.channels != 128 || !transition || !a.f_logits || !a.sl_ln_w || !a.sl_ln_b || a.logit_heads <= 0)) return AF3_ERR_BAD_ARG;
+  if (a.channels == 64) switch (step) {
+    case PAIR_STEP_FIRST: return launch_tiles<64, 1, IN_NONE, MAP_ROWS, false, NEXT_PROLOGUE>(a, s);
+    case PAIR_STEP_INCOMING: return launch_tiles<64, 1, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
+    case PAIR_STEP_PROJECT_START: return launch_tiles<64, 1, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
+    case PAIR_STEP_PROJECT_END: return launch_tiles<64, 1, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
+    case PAIR_STEP_LAST: return launch_tiles<64, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_NONE>(a, s);
+    case PAIR_STEP_NEXT: return launch_tiles<64, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_PROLOGUE>(a, s);
+  }
+  else switch (step) {
     case PAIR_STEP_INCOMING:
-      if ((int64_t)a.N * a.ldn >= WIDE_PATCHES) return launch_tiles<2, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
-      return launch_tiles<1, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
-    case PAIR_STEP_PROJECT_START: return launch_tiles<1, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
-    case PAIR_STEP_PROJECT_END: return launch_tiles<1, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
-    case PAIR_STEP_LAST: return launch_tiles<1, IN_ATTENTION, MAP_ROWS, true, NEXT_NONE>(a, s);
-    case PAIR_STEP_NEXT: return launch_tiles<1, IN_ATTENTION, MAP_ROWS, true, NEXT_PROLOGUE>(a, s);
+      if ((int64_t)a.N * a.ldn >= WIDE_PATCHES) return launch_tiles<128, 2, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
+      return launch_tiles<128, 1, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
+    case PAIR_STEP_PROJECT_START: return launch_tiles<128, 1, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
+    case PAIR_STEP_PROJECT_END: return launch_tiles<128, 1, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
+    case PAIR_STEP_LAST: return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_NONE>(a, s);
+    case PAIR_STEP_NEXT: return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_PROLOGUE>(a, s);
   }
   return AF3_ERR_BAD_ARG;
 }

@@ -72,20 +72,25 @@ int pair_operators(const af3_pairformer_block& b, void* pair, int dt, const floa
 // costs more than that saves.  Runs of 4 blocks, us a block, one kernel per operator -> steps (bf16 / fp32 stream):
 //   64 tokens 136 -> 85 / 143 -> 88,  128: 166 -> 121 / 173 -> 121,  160: 205 -> 179 / 213 -> 182,
 //   208: 286 -> 268 / 306 -> 279,  224: 265 -> 264 / 283 -> 275,  256: 287 -> 288 / 323 -> 302
+// Pair tensors of 64 channels have no other kernels (64 / 301 / 768 / 2048 tokens, bf16, a block on its own: 100 -> 46,
+// 345 -> 221, 1940 -> 1460, 22400 -> 18800 against one zero-padded to 128; their 32-bit offsets end at 3072).
 constexpr int64_t PAIR_STEP_POSITIONS = 208 * 208;
 bool pair_steps_apply(const af3_pairformer_block& b, int64_t n) {
-  return b.pair_frags && n <= 8192 && n * tri_ldn(n) <= PAIR_STEP_POSITIONS && b.num_head_pair == 4 && b.valid_channels >= 8 &&
-         b.valid_channels <= 128 && b.valid_channels % 4 == 0 && b.pair_hidden > 0 && b.pair_hidden % 64 == 0 &&
-         b.pair_hidden <= PAIR_STEP_MAX_HIDDEN;
+  const int c = b.pair_channels == 64 ? 64 : 128;
+  return b.pair_frags && n <= 8192 && (c == 64 ? n <= AF3_PAIR64_MAX_TOKENS : n * tri_ldn(n) <= PAIR_STEP_POSITIONS) &&
+         b.num_head_pair == 4 && b.valid_channels >= 8 && b.valid_channels <= c && b.valid_channels % 4 == 0 &&
+         (c == 128 || b.valid_channels == 64) && b.pair_hidden > 0 && b.pair_hidden % 64 == 0 &&
+         b.pair_hidden <= pair_step_max_hidden(c);
 }
 // Scratch.  q, k and the operands of the contraction are never alive together, nor are its result and the attention's.
 struct PairStepScratch {
   bf16_t *qa = nullptr, *kb = nullptr, *vt = nullptr, *ogt = nullptr;
   uint16_t* bias = nullptr;
-  static size_t plane_bytes(int64_t n) { return (size_t)128 * tri_plane(n) * 2; }  // (tri_plane(n) >= n n)
-  static size_t bytes(int64_t n) {
-    return 3 * align_up(plane_bytes(n)) + align_up((size_t)n * 128 * tri_ldn(n) * 2) + align_up((size_t)tri_bias_elems(n, 4) * 2) +
-           LOGIT_RING * logit_bytes(n, 16);
+  static size_t plane_bytes(int64_t n, int c) { return (size_t)c * tri_plane(n) * 2; }  // (tri_plane(n) >= n n)
+  static size_t vt_bytes(int64_t n, int c) { return (size_t)n * c * tri_ldn(n) * 2; }
+  static size_t bytes(int64_t n, int c) {
+    return 3 * align_up(plane_bytes(n, c)) + align_up(vt_bytes(n, c)) + align_up((size_t)tri_bias_elems(n, 4) * 2) +
+           (c == 128 ? LOGIT_RING * logit_bytes(n, 16) : 0);
   }
   // Pair logits of the last blocks, where the single track runs on a stream of its own.  With two buffers every block waits
   // for the attention two blocks back, and an event recorded and waited for costs the host 13 us, where a launch costs 3.5:
@@ -93,12 +98,12 @@ struct PairStepScratch {
   static constexpr int LOGIT_RING = 8;
   static size_t logit_bytes(int64_t n, int heads) { return align_up((size_t)heads * n * ((n + 3) / 4 * 4) * 4); }
   float* ring(int64_t n) const { return reinterpret_cast<float*>(reinterpret_cast<char*>(bias) + align_up((size_t)tri_bias_elems(n, 4) * 2)); }
-  bool carve(int64_t n, void* ws, size_t wsb) {
+  bool carve(int64_t n, int c, void* ws, size_t wsb) {
     Carver w(ws, wsb);
-    qa = static_cast<bf16_t*>(w.take(plane_bytes(n)));
-    kb = static_cast<bf16_t*>(w.take(plane_bytes(n)));
-    ogt = static_cast<bf16_t*>(w.take(plane_bytes(n)));
-    vt = static_cast<bf16_t*>(w.take((size_t)n * 128 * tri_ldn(n) * 2));
+    qa = static_cast<bf16_t*>(w.take(plane_bytes(n, c)));
+    kb = static_cast<bf16_t*>(w.take(plane_bytes(n, c)));
+    ogt = static_cast<bf16_t*>(w.take(plane_bytes(n, c)));
+    vt = static_cast<bf16_t*>(w.take(vt_bytes(n, c)));
     bias = static_cast<uint16_t*>(w.take((size_t)tri_bias_elems(n, 4) * 2));
     return w.ok;
   }
@@ -113,25 +118,30 @@ int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_
   if (!pair || (dt != AF3_F32 && dt != AF3_BF16) || ((uintptr_t)pair & 15) || ((uintptr_t)mask & 15) || ((uintptr_t)mask_in & 15))
     return AF3_ERR_BAD_ARG;
   PairStepScratch w;
-  if (!w.carve(n, ws, wsb)) return AF3_ERR_WORKSPACE;
-  const int c = b.valid_channels, hidden = b.pair_hidden;
+  const int c = b.valid_channels, hidden = b.pair_hidden, wide = b.pair_channels == 64 ? 64 : 128;
+  if (!w.carve(n, wide, ws, wsb)) return AF3_ERR_WORKSPACE;
   PairStepArgs a;
-  a.lw = ln_width(c);
+  a.channels = wide;
+  a.lw = ln_width(c, wide);
   a.valid_c = c; a.io_f32 = dt == AF3_F32; a.N = (int)n; a.Np = (int)up8(n); a.ldn = (int)tri_ldn(n); a.plane = tri_plane(n);
   a.pair = pair; a.hidden = hidden;
   a.t_buf = a.og = w.ogt; a.a_buf = a.q = w.qa; a.b_buf = a.k = w.kb; a.vt = w.vt; a.bias = w.bias;
   a.bias_scale = 1.4426950408889634f;  // base-2 logits, as grid_self_attn_impl
   a.q_scale = a.bias_scale / sqrtf((float)(c / 4));
-  // pair_frags, in rows of 128
-  auto qkg = [&](int d, int row) { return b.pair_frags + (d * 384 + row) * 128; };
-  auto tm = [&](const af3_pairformer_block& x, int d, int row) { return x.pair_frags + (768 + d * 768 + row) * 128; };
-  auto ta = [&](int d, int row) { return b.pair_frags + (2304 + d * 288 + row) * 128; };
-  const uint16_t* const w1 = b.pair_frags + 2880 * 128;
+  // pair_frags, in rows of 128 (64)
+  auto qkg = [&](int d, int mat) { return b.pair_frags + (d * 3 + mat) * wide * wide; };
+  auto tm = [&](const af3_pairformer_block& x, int d, int mat) { return x.pair_frags + (6 + d * 6 + mat) * wide * wide; };
+  auto ta = [&](int d, int row) { return b.pair_frags + (18 * wide + d * (2 * wide + 32) + row) * wide; };
+  const uint16_t* const w1 = b.pair_frags + (22 * wide + 64) * wide;
   const int logit_rows = b.with_single ? (b.num_head + 31) / 32 * 32 : 0;
   TriAttnArgs core;
   core.q = w.qa; core.k = w.kb; core.vt = w.vt; core.bias = w.bias; core.mask = mask; core.og = w.ogt; core.N = (int)n; core.ldn = a.ldn;
+  core.head_dim = wide / 4;
 
-  if (first) {
+  if (first && wide == 64) {
+    a.ln3_w = b.tm_ln_in_w[0]; a.ln3_b = b.tm_ln_in_b[0]; a.f_next = tm(b, 0, 2); a.mask = mask;
+    STEP(launch_pair_step(a, PAIR_STEP_FIRST, s));
+  } else if (first) {
     TriMulArgs p;
     p.lw = a.lw; p.valid_c = c; p.pair = pair; p.mask = mask; p.io_f32 = a.io_f32; p.N = a.N; p.Np = a.Np; p.plane = a.plane;
     p.ln_in_w = b.tm_ln_in_w[0]; p.ln_in_b = b.tm_ln_in_b[0]; p.w_pg = b.tm_w_proj_gate[0];
@@ -140,10 +150,10 @@ int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_
   }
   for (int d = 0; d < 2; ++d) {
     STEP(run_triangle_contraction(w.qa, w.kb, w.ogt, (int)n, c, d == 0, s));
-    a.ln1_w = b.tm_ln_in_w[d]; a.ln1_b = b.tm_ln_in_b[d]; a.f_gate = tm(b, d, 0); a.f_out = tm(b, d, 128);
+    a.ln1_w = b.tm_ln_in_w[d]; a.ln1_b = b.tm_ln_in_b[d]; a.f_gate = tm(b, d, 0); a.f_out = tm(b, d, 1);
     a.ln_c_w = b.tm_ln_c_w[d]; a.ln_c_b = b.tm_ln_c_b[d];
     if (d == 0) {
-      a.ln3_w = b.tm_ln_in_w[1]; a.ln3_b = b.tm_ln_in_b[1]; a.f_next = tm(b, 1, 256); a.mask = mask_in ? mask_in : mask;
+      a.ln3_w = b.tm_ln_in_w[1]; a.ln3_b = b.tm_ln_in_b[1]; a.f_next = tm(b, 1, 2); a.mask = mask_in ? mask_in : mask;
       STEP(launch_pair_step(a, PAIR_STEP_INCOMING, s));
     } else {
       a.ln3_w = b.ta_ln_w[0]; a.ln3_b = b.ta_ln_b[0]; a.f_next = qkg(0, 0); a.f_v = ta(0, 0);
@@ -151,18 +161,18 @@ int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_
     }
   }
   STEP(launch_triattn_flash(core, s));
-  a.ln1_w = b.ta_ln_w[0]; a.ln1_b = b.ta_ln_b[0]; a.f_gate = qkg(0, 256); a.f_out = ta(0, 160);
+  a.ln1_w = b.ta_ln_w[0]; a.ln1_b = b.ta_ln_b[0]; a.f_gate = qkg(0, 2); a.f_out = ta(0, wide + 32);
   a.ln3_w = b.ta_ln_w[1]; a.ln3_b = b.ta_ln_b[1]; a.f_next = qkg(1, 0); a.f_v = ta(1, 0);
   STEP(launch_pair_step(a, PAIR_STEP_PROJECT_END, s));
   STEP(launch_triattn_flash(core, s));
-  a.ln1_w = b.ta_ln_w[1]; a.ln1_b = b.ta_ln_b[1]; a.f_gate = qkg(1, 256); a.f_out = ta(1, 160);
-  a.ln2_w = b.pt_ln_w; a.ln2_b = b.pt_ln_b; a.f_w1 = w1; a.f_w2 = w1 + (2 * hidden + logit_rows) * 128;
+  a.ln1_w = b.ta_ln_w[1]; a.ln1_b = b.ta_ln_b[1]; a.f_gate = qkg(1, 2); a.f_out = ta(1, wide + 32);
+  a.ln2_w = b.pt_ln_w; a.ln2_b = b.pt_ln_b; a.f_w1 = w1; a.f_w2 = w1 + (2 * hidden + logit_rows) * wide;
   if (logits) {
-    a.sl_ln_w = b.sl_ln_w; a.sl_ln_b = b.sl_ln_b; a.f_logits = w1 + 2 * hidden * 128; a.logit_heads = b.num_head; a.logits = logits;
+    a.sl_ln_w = b.sl_ln_w; a.sl_ln_b = b.sl_ln_b; a.f_logits = w1 + 2 * hidden * wide; a.logit_heads = b.num_head; a.logits = logits;
     if (logits_free) STEP(logits_free->wait(s));
   }
   if (!next) return launch_pair_step(a, PAIR_STEP_LAST, s);
-  a.ln3_w = next->tm_ln_in_w[0]; a.ln3_b = next->tm_ln_in_b[0]; a.f_next = tm(*next, 0, 256); a.mask = mask;
+  a.ln3_w = next->tm_ln_in_w[0]; a.ln3_b = next->tm_ln_in_b[0]; a.f_next = tm(*next, 0, 2); a.mask = mask;
   return launch_pair_step(a, PAIR_STEP_NEXT, s);
 }
 
@@ -297,7 +307,7 @@ int af3_evoformer_stack_forward(const af3_msa_block* const* blocks, int num_bloc
   if (!blocks || num_blocks <= 0 || !msa || !msa_mask || !pair || !msa_size_ok(rows, n)) return AF3_ERR_BAD_ARG;
   if ((msa_dtype != AF3_F32 && msa_dtype != AF3_BF16) || (pair_dtype != AF3_F32 && pair_dtype != AF3_BF16)) return AF3_ERR_BAD_ARG;
   for (int i = 0; i < num_blocks; ++i)
-    if (!blocks[i] || blocks[i]->epsilon != blocks[0]->epsilon) return AF3_ERR_BAD_ARG;
+    if (!blocks[i] || blocks[i]->epsilon != blocks[0]->epsilon || blocks[i]->pair.pair_channels == 64) return AF3_ERR_BAD_ARG;
   if (workspace_bytes < af3_msa_workspace_bytes(rows, n)) return AF3_ERR_WORKSPACE;  // (in place: before the first launch)
   for (int i = 0; i < num_blocks; ++i)
     if (pair_workspace_bytes < af3_pairformer_stack_workspace_bytes(n, blocks[i]->pair.num_head_pair)) return AF3_ERR_WORKSPACE;
@@ -335,8 +345,10 @@ int af3_evoformer_stack_forward(const af3_msa_block* const* blocks, int num_bloc
 
 size_t af3_pairformer_stack_workspace_bytes(int64_t n, int num_head_pair) {
   const size_t a = af3_triangle_multiplication_workspace_bytes(n), b = af3_grid_self_attn_workspace_bytes(n, num_head_pair);
-  const size_t c = n > 0 && n * tri_ldn(n) <= PAIR_STEP_POSITIONS ? PairStepScratch::bytes(n) : 0;
-  return a > b ? (a > c ? a : c) : (b > c ? b : c);
+  size_t most = a > b ? a : b;
+  if (n > 0 && n * tri_ldn(n) <= PAIR_STEP_POSITIONS && PairStepScratch::bytes(n, 128) > most) most = PairStepScratch::bytes(n, 128);
+  if (n > 0 && n <= AF3_PAIR64_MAX_TOKENS && PairStepScratch::bytes(n, 64) > most) most = PairStepScratch::bytes(n, 64);
+  return most;
 }
 
 size_t af3_pairformer_single_workspace_bytes(int64_t n, int c_single, int single_hidden) {
@@ -356,6 +368,10 @@ int af3_pairformer_stack_forward(
     if (!blocks[i]) return AF3_ERR_BAD_ARG;
     const af3_pairformer_block& b = *blocks[i];
     if (workspace_bytes < af3_pairformer_stack_workspace_bytes(n, b.num_head_pair)) return AF3_ERR_WORKSPACE;
+    // (a pair tensor of 64 channels is what the step kernels alone take)
+    if ((b.pair_channels != 0 && b.pair_channels != 128 && b.pair_channels != 64) ||
+        (b.pair_channels == 64) != (blocks[0]->pair_channels == 64) || (b.pair_channels == 64 && (!pair_steps_apply(b, n) || b.with_single)))
+      return AF3_ERR_BAD_ARG;
     if (!b.with_single) continue;
     if (!single || !logits || b.num_head != blocks[0]->num_head || b.c_single != blocks[0]->c_single) return AF3_ERR_BAD_ARG;
     if (single_workspace_bytes < af3_pairformer_single_workspace_bytes(n, b.c_single, b.single_hidden)) return AF3_ERR_WORKSPACE;
@@ -372,7 +388,7 @@ int af3_pairformer_stack_forward(
     bool all = true;
     for (int i = 0; i < num_blocks; ++i) all = all && pair_steps_apply(*blocks[i], n) && blocks[i]->num_head <= 16;
     PairStepScratch w;
-    if (all && workspace_bytes >= PairStepScratch::bytes(n) && w.carve(n, workspace, workspace_bytes)) {
+    if (all && workspace_bytes >= PairStepScratch::bytes(n, 128) && w.carve(n, 128, workspace, workspace_bytes)) {
       first = w.ring(n);
       logit_size = PairStepScratch::logit_bytes(n, 16) / 4;
       buffers = PairStepScratch::LOGIT_RING;

@@ -128,7 +128,7 @@ __device__ __forceinline__ void load_param8(const float* p, float fill, float* o
   }
 }
 
-// LayerNorm of one pixel's eight channels (the thread's share: 16 lanes cooperate on the
+// LayerNorm of one pixel's eight channels (the thread's share: LANES lanes cooperate on the
 // pixel's statistics) -> packed bf16.
 //
 // This phase is vector arithmetic per element and a large share of every tile
@@ -140,7 +140,7 @@ __device__ __forceinline__ void load_param8(const float* p, float fill, float* o
 // select when every pixel of the tile is in range.  The fp32 stream keeps the
 // two-pass form.  Zero-padded channels (fewer than 128 real ones) add nothing to
 // either sum; the two-pass form takes their pad * mean^2 out again.
-template <typename TIO>
+template <typename TIO, int LANES = 16>
 __device__ __forceinline__ u32x4 ln_pixel8(const typename Elem<TIO>::Raw& raw, const float* w, const float* b,
                                            bool skip_ln, float inv_c, float pad) {
   using E = Elem<TIO>;
@@ -151,8 +151,8 @@ __device__ __forceinline__ u32x4 ln_pixel8(const typename Elem<TIO>::Raw& raw, c
     float s = 0.f, q = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) { s += v[e]; q = fmaf(v[e], v[e], q); }
-    const float mean = group16_sum(s) * inv_c;
-    const float var = fmaxf(fmaf(group16_sum(q), inv_c, -mean * mean), 0.f);
+    const float mean = group_sum<LANES>(s) * inv_c;
+    const float var = fmaxf(fmaf(group_sum<LANES>(q), inv_c, -mean * mean), 0.f);
     // (an already normalised input comes with w = 1, b = 0: scale 1 and shift 0 pass it through unchanged)
     const float rstd = skip_ln ? 1.f : rsqrtf(var + LN_EPS);
     const float shift = skip_ln ? 0.f : -mean * rstd;
@@ -162,12 +162,12 @@ __device__ __forceinline__ u32x4 ln_pixel8(const typename Elem<TIO>::Raw& raw, c
     float s = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) s += v[e];
-    const float mean = group16_sum(s) * inv_c;
+    const float mean = group_sum<LANES>(s) * inv_c;
     float q = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) { const float d = v[e] - mean; q += d * d; }
     // (zero-padded channels, if any, each put mean^2 into the sum)
-    const float rstd = rsqrtf((group16_sum(q) - pad * mean * mean) * inv_c + LN_EPS);
+    const float rstd = rsqrtf((group_sum<LANES>(q) - pad * mean * mean) * inv_c + LN_EPS);
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = skip_ln ? v[e] : (v[e] - mean) * rstd * w[e] + b[e];
   }

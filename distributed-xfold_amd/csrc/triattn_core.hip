@@ -1,8 +1,8 @@
-// Triangle attention, the flash-attention core (4 heads of 32 channels).
+// Triangle attention, the flash-attention core (4 heads of 32 channels, or of 16).
 //
 // Operands (all produced by triattn_proj_kernel, see kernels.h):
-//   Q, K    : bf16 [b][h][s][32]  (Q pre-multiplied by log2(e)/sqrt(32))
-//   Vt      : bf16 [b][h][32][ldn], V transposed, ldn = N rounded up to 16, columns
+//   Q, K    : bf16 [b][h][s][D]  (Q pre-multiplied by log2(e)/sqrt(D))
+//   Vt      : bf16 [b][h][D][ldn], V transposed, ldn = N rounded up to 16, columns
 //             permuted inside every aligned group of 16 (tri_vt_pos) so that the 8 keys one
 //             lane feeds to a P.V MFMA are 16 contiguous bytes
 //   bias    : fp16, pair bias * log2(e) in MFMA-fragment order (tri_bias_offset)
@@ -38,7 +38,8 @@
 //     each of those four MFMAs is issued in front of eight exponentials of the same wave, its
 //     V^T fragment read from LDS one group ahead.  Row sums are taken from the bf16
 //     probabilities by v_dot2c_f32_bf16 against a pair of ones (per lane, i.e. per half of the
-//     keys; the halves are added once at the end).
+//     keys; the halves are added once at the end).  Heads of 16 leave half of the P.V product's
+//     rows to spare: a row of ones behind V^T makes the sum there (768 tokens 3 % of a block).
 //   * K and V^T tiles go from global memory straight into LDS (global_load_lds_dwordx4: no
 //     staging registers, no LDS store instructions), double-buffered per row with one barrier
 //     per key tile; unpadded rows with XOR-permuted 16-byte chunks keep the fragment reads
@@ -53,10 +54,10 @@
 
 namespace {
 
-constexpr int H = 4, D = 32;
+constexpr int H = 4;
 constexpr int KT = 64;    // keys per tile
 constexpr int QW = 128;   // queries per workgroup (32 per wave)
-constexpr int TILE_BYTES = KT * D * 2;  // a K tile [64 keys][32] or a V^T tile [32][64 keys], bf16
+constexpr int tile_bytes(int d) { return KT * d * 2; }  // a K tile [64 keys][d] or a V^T tile [d][64 keys], bf16
 constexpr uint32_t BF16_ONE = 0x3F80u, BF16_NEG_INF = 0xFF80u, BF16_NEG_1E9 = 0xCE6Eu;
 // A tile's scores, relative to the base, may rise to 2^T_HI before the base is moved (fp32 and
 // bf16 share their exponent range, so nothing is lost up there); the first tile with an unmasked
@@ -122,18 +123,23 @@ __device__ __forceinline__ void scale_in_place(f32x16& o, float f) {
   }
 }
 
-template <int R, bool HAS_BIAS, bool SPARE>
+template <int R, bool HAS_BIAS, int D, bool SPARE>
 __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
+  constexpr int TILE_BYTES = tile_bytes(D);
+  constexpr int KS = D / 16;  // k-steps of the score product
   // [buffer][row] as separate arrays: a load in flight to one of them provably does not alias
   // a fragment read from another
   __shared__ __attribute__((aligned(1024))) char sK00[TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) char sK01[R > 1 ? TILE_BYTES : 16];
   __shared__ __attribute__((aligned(1024))) char sK10[TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) char sK11[R > 1 ? TILE_BYTES : 16];
-  __shared__ __attribute__((aligned(1024))) char sV00[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) char sV01[R > 1 ? TILE_BYTES : 16];
-  __shared__ __attribute__((aligned(1024))) char sV10[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) char sV11[R > 1 ? TILE_BYTES : 16];
+  // Heads of 16: a V^T tile has one row more, of ones.  The sixteen rows of the P.V product that no channel needs read it,
+  // so that O's register 8 is the row's sum of probabilities.
+  constexpr int V_BYTES = TILE_BYTES + (D == 16 ? KT * 2 : 0);
+  __shared__ __attribute__((aligned(1024))) char sV00[V_BYTES];
+  __shared__ __attribute__((aligned(1024))) char sV01[R > 1 ? V_BYTES : 16];
+  __shared__ __attribute__((aligned(1024))) char sV10[V_BYTES];
+  __shared__ __attribute__((aligned(1024))) char sV11[R > 1 ? V_BYTES : 16];
   __shared__ uint32_t sLive[R];      // per row: some key is unmasked
   __shared__ uint8_t sFlag[R * 64];  // per row and key tile (the first 64): 1 = some key unmasked, 3 = all 64 of them
   __shared__ float sMean[D];
@@ -192,7 +198,17 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
   // and comes out of L2; Q comes from memory and is requested right behind the first batch of
   // mask values: loads return in order, so the mask pass does not wait for it, and it travels
   // while the mask pass, the barriers and the first tiles' loads are under way.
-  bf16x8 qf[R][2];
+  bf16x8 qf[R][KS];
+  if (D == 16 && tid < KT / 8) {
+    const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+    const int at = TILE_BYTES + tid % (KT / 8) * 16;
+    *reinterpret_cast<u32x4*>(sV00 + at) = ones;
+    *reinterpret_cast<u32x4*>(sV10 + at) = ones;
+    if constexpr (R > 1) {
+      *reinterpret_cast<u32x4*>(sV01 + at) = ones;
+      *reinterpret_cast<u32x4*>(sV11 + at) = ones;
+    }
+  }
   // What a wave finds out about a tile is one byte in LDS, written by all its lanes alike; the
   // workgroup's bit masks of live and of wholly unmasked tiles are ballots over those bytes.
   bool my_any[R];
@@ -212,7 +228,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
         const int64_t row = ((int64_t)brow[r] * H + h) * N + qi;
         const bf16_t* qp = a.q + row * D + 8 * hh;
         qf[r][0] = as_frag(*reinterpret_cast<const u32x4*>(qp));
-        qf[r][1] = as_frag(*reinterpret_cast<const u32x4*>(qp + 16));
+        if constexpr (KS == 2) qf[r][1] = as_frag(*reinterpret_cast<const u32x4*>(qp + 16));
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -282,24 +298,30 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
       vglob[r] = reinterpret_cast<const char*>(a.vt + bh * D * a.ldn);
     }
     // fragment reads: K row (32 u + j), chunk (2 ks + hh) ^ ((j >> 2) & 3); V^T row j, chunk (2 s + hh) ^ ((j >> 1) & 7)
+    // heads of 16: K in blocks of 32 rows, the rows' first chunks and then their second ones; V^T row min(j, 16)
     const int ksw = (j >> 2) & 3;
-    const int ka0 = j * 64 + ((hh ^ ksw) << 4), ka1 = j * 64 + (((2 + hh) ^ ksw) << 4);
-    const int vsw = (j >> 1) & 7;
+    const int ka0 = D == 16 ? j * 16 + hh * 512 : j * 64 + ((hh ^ ksw) << 4), ka1 = j * 64 + (((2 + hh) ^ ksw) << 4);
+    const int vrow = min(j, D), vsw = (vrow >> 1) & 7;
     int va[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) va[s] = j * 128 + (((2 * s + hh) ^ vsw) << 4);
+    for (int s = 0; s < 4; ++s) va[s] = vrow * 128 + (((2 * s + hh) ^ vsw) << 4);
     // loads into LDS: K keys 16 w + lane / 4, position lane % 4; V^T rows 8 w + lane / 8, position lane % 8
-    const int dk_key = 16 * wave + (lane >> 2);
-    const uint32_t dk_chunk = (uint32_t)(((lane & 3) ^ ((dk_key >> 2) & 3)) << 4);
-    const int dv_row = 8 * wave + (lane >> 3);
+    // heads of 16: K by the first two waves, V^T by the other two
+    const int part = D == 16 ? wave & 1 : wave;
+    const bool loads_k = D == 32 || wave < 2, loads_v = D == 32 || wave >= 2;
+    const int dk_key = D == 16 ? 32 * part + j : 16 * part + (lane >> 2);
+    const uint32_t dk_chunk = D == 16 ? (uint32_t)(hh << 4) : (uint32_t)(((lane & 3) ^ ((dk_key >> 2) & 3)) << 4);
+    const int dv_row = 8 * part + (lane >> 3);
     const int dv_col = ((lane & 7) ^ ((dv_row >> 1) & 7)) * 8;
     auto dma_k = [&](int tile, int r, char* buf) {  // a tile past the end re-reads the last one (never used)
+      if (!loads_k) return;
       const int key = min(min(tile, nkt - 1) * KT + dk_key, N - 1);
-      dma16<0>(kglob[r], (uint32_t)key * (D * 2u) + dk_chunk, buf + wave * 1024);
+      dma16<0>(kglob[r], (uint32_t)key * (D * 2u) + dk_chunk, buf + part * 1024);
     };
     auto dma_v = [&](int tile, int r, char* buf) {
+      if (!loads_v) return;
       const int col = min(tile, nkt - 1) * KT + dv_col;  // columns past ldn: any finite data will do (P is zero there)
-      dma16<0>(vglob[r], (uint32_t)(dv_row * ldn + (col < ldn ? col : 0)) * 2u, buf + wave * 1024);
+      dma16<0>(vglob[r], (uint32_t)(dv_row * ldn + (col < ldn ? col : 0)) * 2u, buf + part * 1024);
     };
     // bias tiles of this wave's 32-query block: 4 KB per key tile
     const char* bbase =
@@ -335,13 +357,21 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
     f32x16 zero16;
 #pragma unroll
     for (int e = 0; e < 16; ++e) zero16[e] = 0.f;
-    // scores of one row's virtual tile: the two halves of the head dimension on top of the bias
-    auto scores = [&](const bf16x8& k00, const bf16x8& k01, const bf16x8& k10, const bf16x8& k11, const bf16x8* q,
-                      f32x16& s0, f32x16& s1) {
-      s0 = mfma32(k00, q[0], bt[0]);
-      s1 = mfma32(k10, q[0], bt[1]);
-      s0 = mfma32(k01, q[1], s0);
-      s1 = mfma32(k11, q[1], s1);
+    // K fragments of 64 keys [k-step][half of the keys], and one row's scores on top of the bias
+    auto load_k_frags = [&](const char* kb, bf16x8 (&k)[KS][2]) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        k[0][u] = lds16(kb + u * (TILE_BYTES / 2) + ka0);
+        if constexpr (KS == 2) k[1][u] = lds16(kb + u * (TILE_BYTES / 2) + ka1);
+      }
+    };
+    auto scores = [&](const bf16x8 (&k)[KS][2], const bf16x8* q, f32x16& s0, f32x16& s1) {
+      s0 = mfma32(k[0][0], q[0], bt[0]);
+      s1 = mfma32(k[0][1], q[0], bt[1]);
+      if constexpr (KS == 2) {
+        s0 = mfma32(k[1][0], q[1], s0);
+        s1 = mfma32(k[1][1], q[1], s1);
+      }
     };
 #pragma unroll
     for (int e = 0; e < 16; ++e) bt[0][e] = bt[1][e] = 0.f;
@@ -357,9 +387,9 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
     // with every tile on the careful route.
     bool allow_fast = true;
     uint64_t bad = 0ull;
-    float lmax[R];      // largest sum of one fast tile
+    float lmax[R];      // largest sum of one fast tile (heads of 16: of all tiles, whenever O was rescaled)
     bool used_fast[R];  // this wave took some tile of the row the fast way
-    bf16x8 kpre[4];  // R == 2: row 0's K fragments of the next key tile
+    bf16x8 kpre[KS][2];  // R == 2: row 0's K fragments of the next key tile
     u32x4 pp[4];  // probabilities of the previous virtual tile (bf16 B fragments), zero before the first
 
     // One virtual tile = (key tile, row RR): scores, softmax, and meanwhile the previous
@@ -370,6 +400,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
       const char* kb = KBUF(PH, RR);
       const char* vb = VBUF(VPH, PR);
       if (R == 1 && pend) {
+        if constexpr (D == 16) lmax[0] = fmaxf(lmax[0], o[0][8]);
         scale_in_place(o[0], pend_alpha);
         pend = false;
       }
@@ -379,12 +410,16 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
       const bool step3 = based[RR] || !fast;
       // Two rows per wave: row 0's K tile has been in LDS since the barrier before the previous
       // virtual tile, whose last group of exponentials fetched these fragments (kpre).
-      const bool pre = R == 2 && RR == 0;
-      const bf16x8 k00 = pre ? kpre[0] : lds16(kb + ka0), k01 = pre ? kpre[1] : lds16(kb + ka1);
-      const bf16x8 k10 = pre ? kpre[2] : lds16(kb + 2048 + ka0), k11 = pre ? kpre[3] : lds16(kb + 2048 + ka1);
+      bf16x8 kf[KS][2];
+      if constexpr (R == 2 && RR == 0) {
+#pragma unroll
+        for (int i = 0; i < 2 * KS; ++i) kf[i >> 1][i & 1] = kpre[i >> 1][i & 1];
+      } else {
+        load_k_frags(kb, kf);
+      }
       bf16x8 af0, af1;
       f32x16 s0, s1;
-      scores(k00, k01, k10, k11, qf[RR], s0, s1);
+      scores(kf, qf[RR], s0, s1);
       if (step3) {
         const uint16_t* mc = sCode + RR * nk64 + tile * KT;
         const uint32_t c0 = mc[j], c1 = mc[32 + j];
@@ -426,9 +461,10 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
           pend_alpha = alpha;
           pend = true;
         } else {
+          if constexpr (D == 16) lmax[RR] = fmaxf(lmax[RR], o[RR][8]);  // (an infinity may become a NaN here)
           scale_in_place(o[RR], alpha);
         }
-        scores(k00, k01, k10, k11, qf[RR], s0, s1);
+        scores(kf, qf[RR], s0, s1);
         s0 = mfma32(af0, as_frag(qm[RR]), s0);
         s1 = mfma32(af1, as_frag(qm[RR]), s1);
       } else {
@@ -453,11 +489,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
           vf = lds16(vb + va[s + 1]);
           __builtin_amdgcn_sched_barrier(0);
         } else if (R == 2 && RR == 1) {
-          const char* kn = KBUF(PH ^ 1, 0);
-          kpre[0] = lds16(kn + ka0);
-          kpre[1] = lds16(kn + ka1);
-          kpre[2] = lds16(kn + 2048 + ka0);
-          kpre[3] = lds16(kn + 2048 + ka1);
+          load_k_frags(KBUF(PH ^ 1, 0), kpre);
           __builtin_amdgcn_sched_barrier(0);
         }
         o[PR] = mfma32(vcur, as_frag(pp[s]), o[PR]);
@@ -477,12 +509,12 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
         // pins the exponentials to this group (without it they sink to where their values are used,
         // the next iteration's MFMAs)
         asm volatile("" : "+v"(pp[s].x), "+v"(pp[s].y), "+v"(pp[s].z), "+v"(pp[s].w));
-        linc = dot2_ones(pp[s].w, dot2_ones(pp[s].z, dot2_ones(pp[s].y, dot2_ones(pp[s].x, linc))));
+        if constexpr (D == 32) linc = dot2_ones(pp[s].w, dot2_ones(pp[s].z, dot2_ones(pp[s].y, dot2_ones(pp[s].x, linc))));
         __builtin_amdgcn_sched_barrier(0);
       }
-      lrun[RR] += linc;
+      if constexpr (D == 32) lrun[RR] += linc;
       if (fast) {
-        lmax[RR] = fmaxf(lmax[RR], linc);
+        if constexpr (D == 32) lmax[RR] = fmaxf(lmax[RR], linc);
         // If the row passes its check at the end, its total is at least 2^-30 over at most 4096
         // keys: a lower bound of the running maximum, all the careful route's lower guard needs
         // (if it does not, the rows are repeated and what a careful tile decided meanwhile is void).
@@ -493,6 +525,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
     // the tail of the pipeline: the last virtual tile's probabilities
     auto drain = [&](const char* vb) {
       constexpr int PR = R - 1;
+      if (D == 16 && R == 1 && pend) lmax[0] = fmaxf(lmax[0], o[0][8]);
       if (R == 1 && pend) scale_in_place(o[0], pend_alpha);  // what was accumulated before the last tile moved the base
 #pragma unroll
       for (int s = 0; s < 4; ++s) o[PR] = mfma32(lds16(vb + va[s]), as_frag(pp[s]), o[PR]);
@@ -521,7 +554,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
     }
     int t_cur = pop(), t_n1 = pop(), t_n2 = pop();
     // the buffer the first virtual tile reads its "previous" V^T from must hold finite data
-    *reinterpret_cast<u32x4*>(VBUF(1, R - 1) + tid * 16) = u32x4{0u, 0u, 0u, 0u};
+    if (tid * 16 < TILE_BYTES) *reinterpret_cast<u32x4*>(VBUF(1, R - 1) + tid * 16) = u32x4{0u, 0u, 0u, 0u};
     // the first tiles' loads into LDS and the first bias tile's ordinary loads travel together
     dma_k(t_cur, 0, KBUF(0, 0));
     if (R == 2) {
@@ -540,10 +573,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
     }
     if (R == 2) {
       dma_barrier();
-      kpre[0] = lds16(KBUF(0, 0) + ka0);
-      kpre[1] = lds16(KBUF(0, 0) + ka1);
-      kpre[2] = lds16(KBUF(0, 0) + 2048 + ka0);
-      kpre[3] = lds16(KBUF(0, 0) + 2048 + ka1);
+      load_k_frags(KBUF(0, 0), kpre);
     }
     // Every ordinary load issued so far (Q, the first bias tile) is waited for HERE, with a wait
     // the compiler can see: otherwise it keeps a vmcnt(0) for them at the top of the loop, where
@@ -612,8 +642,8 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (!used_fast[r] || dead[r]) continue;
-      const float lt = lrun[r] + half_swap(xaddr, lrun[r]);
-      bad |= __ballot(qw < N && (!(lmax[r] < 0x1p60f) || lt < 0x1p-30f));
+      const float lt = D == 16 ? o[r][8] : lrun[r] + half_swap(xaddr, lrun[r]);
+      bad |= __ballot(qw < N && (!((D == 16 ? fmaxf(lt, lmax[r]) : lmax[r]) < 0x1p60f) || lt < 0x1p-30f));
     }
     if (bad != 0ull && lane == 0) sRedo = 1u;
     lds_barrier();  // also: every wave is done with the K / V^T tiles before a second pass loads over them
@@ -623,7 +653,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
 
   // a query's keys are split over the two half-waves
 #pragma unroll
-  for (int r = 0; r < R; ++r) lrun[r] += half_swap(xaddr, lrun[r]);
+  for (int r = 0; r < R; ++r) lrun[r] = D == 16 ? o[r][8] : lrun[r] + half_swap(xaddr, lrun[r]);
 
   // ---- rows whose keys are all masked: the reference replaces every logit by the same -1e9,
   // the softmax is exactly uniform and each query's output is the mean of V over the N keys ----
@@ -631,7 +661,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
   for (int r = 0; r < R; ++r) {
     if (!dead[r]) continue;
     lds_barrier();
-    const int v_d = tid >> 3, c8 = (tid & 7) * 8;
+    const int v_d = (tid >> 3) & (D - 1), c8 = (tid & 7) * 8;
     const bf16_t* vrow = a.vt + (((int64_t)brow[r] * H + h) * D + v_d) * a.ldn;
     float acc = 0.f;
     // columns N..ldn-1 are zero; eight loads in flight at a time (one at a time, each waits out a
@@ -659,7 +689,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
     if ((tid & 7) == 0) sMean[v_d] = acc;
     lds_barrier();
 #pragma unroll
-    for (int e = 0; e < 16; ++e) o[r][e] = sMean[8 * (e >> 2) + 4 * hh + (e & 3)];
+    for (int e = 0; e < 16; ++e) o[r][e] = sMean[(8 * (e >> 2) + 4 * hh + (e & 3)) & (D - 1)];
     lrun[r] = (float)N;
   }
 
@@ -668,9 +698,9 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
   for (int r = 0; r < R; ++r) {
     if (!bvalid[r]) continue;
     const float inv = 1.f / lrun[r];  // the sum over both half-waves' keys
-    bf16_t* op = a.og + ((int64_t)brow[r] * N + qw) * 128 + h * D + 4 * hh;
+    bf16_t* op = a.og + ((int64_t)brow[r] * N + qw) * (H * D) + h * D + 4 * hh;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
+    for (int g = 0; g < D / 8; ++g) {
       u32x2 w;
       w.x = pack2bf(o[r][4 * g] * inv, o[r][4 * g + 1] * inv);
       w.y = pack2bf(o[r][4 * g + 2] * inv, o[r][4 * g + 3] * inv);
@@ -687,7 +717,7 @@ bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream) {
   if (!a.q || !a.k || !a.vt || !a.og || a.N <= 0 || a.N > 8192) return AF3_ERR_BAD_ARG;
-  if (a.ldn < a.N || (a.ldn & 15)) return AF3_ERR_BAD_ARG;
+  if (a.ldn < a.N || (a.ldn & 15) || (a.head_dim != 32 && a.head_dim != 16)) return AF3_ERR_BAD_ARG;
   if (!al16(a.q) || !al16(a.k) || !al16(a.vt) || !al16(a.og) || !al16(a.bias)) return AF3_ERR_BAD_ARG;
   const int QT = (a.N + QW - 1) / QW;
   const int nkt = (a.N + KT - 1) / KT;
@@ -697,14 +727,15 @@ int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream) {
   int R = (int64_t)((a.N + 1) / 2) * H * QT >= 700 ? 2 : 1;
   // static LDS: K / V buffers, small arrays; dynamic: the mask codes.  Two workgroups must fit a
   // CU's 160 KB.
-  const size_t stat2 = 8 * TILE_BYTES + 512;
+  const int tile = tile_bytes(a.head_dim);
+  const size_t stat2 = 8 * (size_t)tile + 1024;
   if (R == 2 && stat2 + 2 * (size_t)nkt * KT * sizeof(uint16_t) > 80 * 1024) R = 1;
   const int NG = (a.N + R - 1) / R;
   const int64_t blocks = ((int64_t)H * NG + 7) / 8 * 8 * QT;
   if (blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
   const size_t dyn = (size_t)R * nkt * KT * sizeof(uint16_t);
   const dim3 grid((unsigned)blocks), block(256);
-  const size_t stat = (R == 2 ? 8 : 4) * TILE_BYTES + 512;
+  const size_t stat = (R == 2 ? 8 : 4) * (size_t)tile + 1024;
   auto launch = [&](void (*kernel)(TriAttnArgs)) {
     // more than 64 KB of LDS per workgroup in all (static + dynamic) has to be asked for
     // (a per-function, per-device setting of the runtime: no allocation, no synchronisation)
@@ -716,8 +747,16 @@ int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL(kernel, grid, block, dyn, stream, a);
   };
   const bool spare = (a.N + 31) / 32 % 4 != 0;
-  if (!a.bias) launch(R == 2 ? triattn_flash_kernel<2, false, false> : triattn_flash_kernel<1, false, false>);
-  else if (R == 2) launch(spare ? triattn_flash_kernel<2, true, true> : triattn_flash_kernel<2, true, false>);
-  else launch(spare ? triattn_flash_kernel<1, true, true> : triattn_flash_kernel<1, true, false>);
+  if (a.head_dim == 16) {
+    if (!a.bias) return AF3_ERR_BAD_ARG;  // (nobody asks for it)
+    if (R == 2) launch(spare ? triattn_flash_kernel<2, true, 16, true> : triattn_flash_kernel<2, true, 16, false>);
+    else launch(spare ? triattn_flash_kernel<1, true, 16, true> : triattn_flash_kernel<1, true, 16, false>);
+  } else if (!a.bias) {
+    launch(R == 2 ? triattn_flash_kernel<2, false, 32, false> : triattn_flash_kernel<1, false, 32, false>);
+  } else if (R == 2) {
+    launch(spare ? triattn_flash_kernel<2, true, 32, true> : triattn_flash_kernel<2, true, 32, false>);
+  } else {
+    launch(spare ? triattn_flash_kernel<1, true, 32, true> : triattn_flash_kernel<1, true, 32, false>);
+  }
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }

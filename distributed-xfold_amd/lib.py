@@ -11,6 +11,7 @@ LIB_PATH = os.path.join(_HERE, "libaf3hip.so")
 AF3_BF16, AF3_F32 = 0, 1
 STATIC_SCRATCH_BYTES = 32 << 20      # AF3_STATIC_SCRATCH_BYTES
 LINEAR_PLAIN, LINEAR_SWIGLU, LINEAR_GATE_RES, LINEAR_REGROUP32, LINEAR_ROWGATE_RES = 0, 2, 3, 4, 5
+PAIR64_MAX_TOKENS = 3072    # AF3_PAIR64_MAX_TOKENS
 
 _vp, _i, _i64, _sz, _f = C.c_void_p, C.c_int, C.c_int64, C.c_size_t, C.c_float
 
@@ -24,7 +25,7 @@ class PairformerBlockStruct(C.Structure):
         + [(k, _vp) for k in ("pt_ln_w", "pt_ln_b", "pt_w1", "pt_w2", "sl_ln_w", "sl_ln_b", "sl_w", "sa_ln_w", "sa_ln_b",
                               "sa_w_qkvg", "sa_q_b", "sa_w_out", "st_ln_w", "st_ln_b", "st_w1", "st_w2", "pair_frags")]
         + [(k, C.c_int32) for k in ("valid_channels", "num_head_pair", "pair_hidden", "with_single", "num_head",
-                                    "c_single", "single_hidden")])
+                                    "c_single", "single_hidden", "pair_channels")])
 
 
 class MsaBlockStruct(C.Structure):

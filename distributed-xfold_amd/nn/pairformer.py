@@ -51,20 +51,47 @@ def fill_pair_weights(s, tm_out, tm_in, ta_start, ta_end, transition, c_pair, w_
           ("pt_w2", p["w2"], (128, hidden)))
     s.valid_channels, s.num_head_pair, s.pair_hidden = c_pair, ta_start.num_head, hidden
     # (gathered first and reordered together: packing is paid for at every new set of weights)
-    plain, turned = [], []
+    plain, turned, w2 = [], [], p["w2"]
+    s.pair_channels = c = 64 if pair_of_64(ta_start, transition, c_pair) and w_logits is None else 128
+    heads, d = ta_start.num_head, c_pair // ta_start.num_head
     for tm in (tm_out, tm_in):
         q = tm.packed()
-        plain += [q["w_gl"], q["w_out"], q["w_proj_gate"].view(-1, 128)]
+        pg = q["w_proj_gate"]                        # 64 channels fill the first group of either operand
+        plain += [q["w_gl"][:c, :c], q["w_out"][:c, :c], (pg if c == 128 else pg[::2, :, :c]).reshape(-1, c)]
     for ta in (ta_start, ta_end):
         q = ta.packed()
-        plain += [q["w_qkvg"][2], q["w_bias"], q["w_out"]]
-        turned += [q["w_qkvg"][0:2].view(-1, 128), q["w_qkvg"][3]]
-    plain.append(p["w1"].view(-1, 128))
+        qkvg, w_out = q["w_qkvg"], q["w_out"]
+        if c == 64:                                  # without the padding of every head to 32 rows
+            qkvg = qkvg.view(4, heads, 32, 128)[:, :, :d, :c].reshape(4, c, c)
+            w_out = w_out.view(128, heads, 32)[:c, :, :d].reshape(c, c)
+        plain += [qkvg[2], q["w_bias"][:, :c], w_out]
+        turned += [qkvg[0:2].reshape(-1, c), qkvg[3]]
+    plain.append(p["w1"][:, :, :c].reshape(-1, c))
     if w_logits is not None:
         plain.append(w_logits)
-    frags = torch.cat([fragments(torch.cat(turned), swap23=True), fragments(torch.cat(plain)), fragments(p["w2"])])
+    frags = torch.cat([fragments(torch.cat(turned), swap23=True), fragments(torch.cat(plain)), fragments(w2[:c])])
     s.pair_frags = frags.data_ptr()
     return frags
+
+
+def pair_of_64(att, transition, c_pair) -> bool:
+    """Whether the library has kernels for the pair operators on 64 channels as they are (the template embedding of
+    nn/d_template.py:198-201), without zero-padding the tensor to 128."""
+    return c_pair == 64 and att.num_head == 4 and transition.packed()["w2"].shape[1] <= 128
+
+
+def takes_64(s, pair: torch.Tensor) -> bool:
+    """Whether a block whose structure is `s` may be given this [N, N, 64] tensor itself."""
+    return s.pair_channels == 64 and pair.shape[0] <= L.PAIR64_MAX_TOKENS and pair.data_ptr() % 16 == 0
+
+
+def padded_128(s) -> "L.PairformerBlockStruct":
+    """The structure for the same block on a tensor zero-padded to 128 channels."""
+    if s.pair_channels != 64:
+        return s
+    p = L.PairformerBlockStruct.from_buffer_copy(s)
+    p.device, p.pair_channels, p.pair_frags = s.device, 128, None
+    return p
 
 
 class PairformerBlock(HipModule):
@@ -178,10 +205,12 @@ class PairformerBlock(HipModule):
                                  join=single_stream is None)
             return pair, single
         if not self.with_single and self.one_call:
-            # (fewer than 128 channels, the template embedding of nn/d_template.py:198-201: the five operators run on
-            # the 128-channel kernels over one zero-padded copy of the tensor, which stays padded in between)
-            x = pad_channels(pair) if self.c_pair < 128 else pair
-            ops.pairformer_stack([self.native()], x, pair_mask, None, None)
+            # (fewer than 128 channels and not the 64 that have kernels of their own: the five operators run on the
+            # 128-channel kernels over one zero-padded copy of the tensor, which stays padded in between)
+            s, x = self.native(), pair
+            if self.c_pair < 128 and not takes_64(s, pair):
+                s, x = padded_128(s), pad_channels(pair)
+            ops.pairformer_stack([s], x, pair_mask, None, None)
             if x is not pair:
                 pair.copy_(x[..., :self.c_pair])
             return pair

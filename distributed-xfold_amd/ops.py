@@ -224,13 +224,14 @@ def transition128(act, layernorm_weight, layernorm_bias, w1_packed, w2, residual
 
 @_uses_scratch
 def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incoming=None, single_stream=None, join=True):
-    """A run of Pairformer blocks in one call (af3_pairformer_stack_forward), pair [N, N, 128] and single [N, c]
-    updated in place.  `blocks`: af3_pairformer_block structures (nn.PairformerBlock.native()); `single_stream`: a
+    """A run of Pairformer blocks in one call (af3_pairformer_stack_forward), pair [N, N, 128] (64 where the blocks'
+    pair_channels say so) and single [N, c] updated in place.  `blocks`: af3_pairformer_block structures (nn.PairformerBlock.native()); `single_stream`: a
     torch stream for the single updates, see the entry point."""
     lib = _L.load()
     _gpu(pair, "pair")
-    if pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair.shape[2] != 128:
-        raise ValueError(f"pair: expected [N, N, 128], got {tuple(pair.shape)}")
+    channels = blocks[0].pair_channels or 128
+    if pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair.shape[2] != channels:
+        raise ValueError(f"pair: expected [N, N, {channels}], got {tuple(pair.shape)}")
     n, dev = pair.shape[0], pair.device
     _weights_with(pair, *blocks)
     io = _dt(pair)

@@ -499,8 +499,8 @@ int af3_pair_cond_init_forward(const void* pair, int pair_dtype, float in_scale,
  *
  * af3_pairformer_block: the packed weights of one block, each array in the layout
  * of the entry point named beside it.
- * pair [n,n,128] (zero-padded when valid_channels < 128) and single [n,c_single]
- * are updated in place.  pair_mask [n,n] or NULL; pair_mask_incoming, when not
+ * pair [n,n,128] (zero-padded when valid_channels < 128; [n,n,64] when pair_channels is 64)
+ * and single [n,c_single] are updated in place.  pair_mask [n,n] or NULL; pair_mask_incoming, when not
  * NULL, replaces it for the incoming triangle multiplication (the Evoformer block
  * transposes it, nn/d_pairformer.py:217); seq_mask [n] or NULL.
  * with_single = 0 in a block leaves `single` alone.
@@ -537,11 +537,17 @@ typedef struct af3_pairformer_block {
   /* NULL, or the pair operators' matrices once more, for runs of operators in one kernel at few tokens: every matrix
    * W [rows][k] as [row / 32][column / 16][(column / 8) % 2][row % 32][column % 8], one after the other.  With bits 2
    * and 3 of the row number exchanged, for [0], [1]: q, k and the gate of ta_w_qkvg; then, for [0], [1]: tm_w_gating,
-   * tm_w_out, tm_w_proj_gate; for [0], [1]: v of ta_w_qkvg, ta_w_bias, ta_w_out; pt_w1; with_single sl_w; pt_w2 */
+   * tm_w_out, tm_w_proj_gate; for [0], [1]: v of ta_w_qkvg, ta_w_bias, ta_w_out; pt_w1; with_single sl_w; pt_w2.  pair_channels 64: without the padding, matrices of 64 columns and
+   * rows (ta_w_bias 32 rows, pt_w1 2 pair_hidden rows) and of tm_w_proj_gate the two groups that hold channels. */
   const uint16_t* pair_frags;
   int32_t valid_channels, num_head_pair, pair_hidden; /* pair_hidden: hidden units of the pair transition */
   int32_t with_single, num_head, c_single, single_hidden;
+  /* 0 or 128: the pair tensor has 128 channels.  64: it has 64, the same in all blocks of a call; then pair_frags, 64
+   * valid_channels, four heads, pair_hidden at most 128 (a multiple of 64), no single track and at most
+   * AF3_PAIR64_MAX_TOKENS tokens.  The other weights are those of the padded operators. */
+  int32_t pair_channels;
 } af3_pairformer_block;
+#define AF3_PAIR64_MAX_TOKENS 3072
 size_t af3_pairformer_stack_workspace_bytes(int64_t n_token, int num_head_pair);
 size_t af3_pairformer_single_workspace_bytes(int64_t n_token, int c_single, int single_hidden);
 int af3_pairformer_stack_forward(
