@@ -124,7 +124,7 @@ __device__ __forceinline__ void scale_in_place(f32x16& o, float f) {
 }
 
 template <int R, bool HAS_BIAS, int D, bool SPARE>
-__global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
+__global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriAttnArgs a) {
   constexpr int TILE_BYTES = tile_bytes(D);
   constexpr int KS = D / 16;  // k-steps of the score product
   // [buffer][row] as separate arrays: a load in flight to one of them provably does not alias
@@ -333,9 +333,12 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
     // the last row of tile t computes its exponentials the fragments are turned into fp32 on
     // the matrix unit, bt = I * bias^T with an fp16 identity: the initial value of the score
     // accumulators of every row of tile t + 1 (four MFMAs per key tile, each issued between
-    // two groups of exponentials).  (Staged through LDS like K and V^T, by loads into LDS two
+    // two groups of exponentials).  With one row per wave (LATE) there is nothing to share: the fragments start the tile's
+    // own score product, requested behind that of the tile before, and without bt's registers a third wave fits the SIMD
+    // (201 -> 168; 160 tokens 16.5 -> 13.8 us, 208 25.6 -> 22.2).  (Staged through LDS like K and V^T, by loads into LDS two
     // tiles ahead, the same kernel ran 3.5 % slower: a load into LDS costs the wave more than
     // a load into registers, and the fragments cost an LDS read each on top.)
+    constexpr bool LATE = R == 1 && HAS_BIAS;
     f32x16 bt[2];
     u32x4 bnext[4];
     auto load_bias = [&](int tile) {
@@ -366,8 +369,17 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
       }
     };
     auto scores = [&](const bf16x8 (&k)[KS][2], const bf16x8* q, f32x16& s0, f32x16& s1) {
-      s0 = mfma32(k[0][0], q[0], bt[0]);
-      s1 = mfma32(k[0][1], q[0], bt[1]);
+      if constexpr (LATE) {
+        s0 = mfma32_f16(idf[0], as_frag_f16(bnext[0]), zero16);
+        s1 = mfma32_f16(idf[0], as_frag_f16(bnext[2]), zero16);
+        s0 = mfma32_f16(idf[1], as_frag_f16(bnext[1]), s0);
+        s1 = mfma32_f16(idf[1], as_frag_f16(bnext[3]), s1);
+        s0 = mfma32(k[0][0], q[0], s0);
+        s1 = mfma32(k[0][1], q[0], s1);
+      } else {
+        s0 = mfma32(k[0][0], q[0], bt[0]);
+        s1 = mfma32(k[0][1], q[0], bt[1]);
+      }
       if constexpr (KS == 2) {
         s0 = mfma32(k[1][0], q[1], s0);
         s1 = mfma32(k[1][1], q[1], s1);
@@ -392,6 +404,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
     bf16x8 kpre[KS][2];  // R == 2: row 0's K fragments of the next key tile
     u32x4 pp[4];  // probabilities of the previous virtual tile (bf16 B fragments), zero before the first
 
+    int t_cur = 0, t_n1 = 0, t_n2 = 0;  // this key tile and the next two
     // One virtual tile = (key tile, row RR): scores, softmax, and meanwhile the previous
     // virtual tile's probabilities go into its row sums and its O.
     auto iter = [&](auto PHc, auto RRc, int tile) {
@@ -475,9 +488,10 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
       // From here to the end: one basic block in a fixed order.  Each of the four P.V MFMAs of the
       // previous virtual tile is issued in front of eight exponentials of this one (the matrix
       // unit works while the wave goes on issuing vector instructions), with its V^T fragment read from LDS one group ahead.
+      if constexpr (LATE) load_bias(t_n1);
       bf16x8 vf = lds16(vb + va[0]);
       u32x4 bfr[4];  // the next key tile's bias fragments (the last row of this one fetches them)
-      if (HAS_BIAS && RR == R - 1) {
+      if (HAS_BIAS && !LATE && RR == R - 1) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) bfr[i] = bnext[i];  // (the registers are free for the next request)
       }
@@ -496,7 +510,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
         float p8[8];
 #pragma unroll
         for (int e = 0; e < 4; ++e) p8[e] = __builtin_amdgcn_exp2f(s < 2 ? s0[8 * (s & 1) + e] : s1[8 * (s & 1) + e]);
-        if (HAS_BIAS && RR == R - 1) {
+        if (HAS_BIAS && !LATE && RR == R - 1) {
           // fragments 2 u + st: bt[u] = I(st = 0) * f(2 u) + I(st = 1) * f(2 u + 1); group s does (u, st) = (s / 2, s % 2)
           asm volatile("" : "+v"(p8[0]), "+v"(p8[1]), "+v"(p8[2]), "+v"(p8[3]));
           bt[s >> 1] = mfma32_f16(idf[s & 1], as_frag_f16(bfr[s]), (s & 1) ? bt[s >> 1] : zero16);
@@ -552,7 +566,7 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
       lmax[r] = 0.f;
       used_fast[r] = false;
     }
-    int t_cur = pop(), t_n1 = pop(), t_n2 = pop();
+    t_cur = pop(); t_n1 = pop(); t_n2 = pop();
     // the buffer the first virtual tile reads its "previous" V^T from must hold finite data
     if (tid * 16 < TILE_BYTES) *reinterpret_cast<u32x4*>(VBUF(1, R - 1) + tid * 16) = u32x4{0u, 0u, 0u, 0u};
     // the first tiles' loads into LDS and the first bias tile's ordinary loads travel together
@@ -563,7 +577,9 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
       dma_v(t_cur, 0, VBUF(0, 0));
       dma_v(t_cur, 1, VBUF(0, 1));
     }
-    if (HAS_BIAS) {
+    if constexpr (LATE) {
+      load_bias(t_cur);
+    } else if (HAS_BIAS) {
       const char* p = bbase + (size_t)t_cur * 4096u + (j * 32 + hh * 16);
       u32x4 f[4];
 #pragma unroll
@@ -597,7 +613,6 @@ __global__ __launch_bounds__(256, 2) void triattn_flash_kernel(TriAttnArgs a) {
         iter(P0{}, std::integral_constant<int, R - 1>{}, t_cur);
       } else {
         dma_barrier();
-        load_bias(t_n1);  // R == 1: requested behind the barrier, used at the end of this virtual tile
         dma_k(t_n1, 0, KBUF(PH ^ 1, 0));
         dma_v(t_cur, 0, VBUF(PH, 0));
         iter(P0{}, std::integral_constant<int, 0>{}, t_cur);
@@ -721,10 +736,13 @@ int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream) {
   if (!al16(a.q) || !al16(a.k) || !al16(a.vt) || !al16(a.og) || !al16(a.bias)) return AF3_ERR_BAD_ARG;
   const int QT = (a.N + QW - 1) / QW;
   const int nkt = (a.N + KT - 1) / KT;
-  // Two rows per wave once that still leaves the CUs one and a half rounds of workgroups (two to a CU): N = 187
-  // 19.5 us (20.3 with one row), 256 25.4 (28.5), 301 48.5 (53.8), 340 56.3 (65.4), but 160 18.6 (18.2); one row below that
-  // (and when the per-key mask codes of two rows would not fit the LDS share of a workgroup).
-  int R = (int64_t)((a.N + 1) / 2) * H * QT >= 700 ? 2 : 1;
+  // One row per wave leaves room for three waves to a SIMD, two rows share one load of the bias.  The line lies where the
+  // workgroups are enough rounds for the traffic to count more than the waves that hide each other's waits; us, one row
+  // against two: 64 tokens 4.3 (5.8), 160 13.8 (17.0), 208 22.2 (24.5), 256 25.5 (26.4), 310 52.9 (54.0), but 320 53.5
+  // (52.9), 384 74.6 (71.8), 512 150 (143), 768 452 (429).  Heads of 16, whose row is less to load, a pair block: 187 tokens
+  // 111 (113), 301 199 (205), 420 381 (384), but 512 491 (480), 768 1484 (1409).
+  // (One row, too, when the per-key mask codes of two would not fit the LDS share of a workgroup.)
+  int R = (int64_t)((a.N + 1) / 2) * H * QT >= (a.head_dim == 16 ? 3500 : 1920) ? 2 : 1;
   // static LDS: K / V buffers, small arrays; dynamic: the mask codes.  Two workgroups must fit a
   // CU's 160 KB.
   const int tile = tile_bytes(a.head_dim);
