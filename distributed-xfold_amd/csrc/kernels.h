@@ -140,6 +140,11 @@ struct RowNormArgs {
   const float *scale2 = nullptr, *shift2 = nullptr;
   bf16_t* y2 = nullptr;
   int64_t ld_cond2 = 0;
+  // C > 128: memory that the kernels behind this one will read (weights), brought nearer by workgroups of its own;
+  // pieces of 128 bytes
+  const void* warm[3] = {nullptr, nullptr, nullptr};
+  uint32_t warm_lines[3] = {0, 0, 0};
+  unsigned row_blocks = 0;  // set by launch_row_norm
   int samples = 1;  // set by launch_row_norm
   int param_vec = 0, cond_vec = 0;  // set by launch_row_norm: arrays aligned for 16-byte loads
 };

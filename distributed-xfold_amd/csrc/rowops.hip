@@ -55,9 +55,29 @@ __device__ __forceinline__ int64_t cond_row(const RowNormArgs& a, int64_t row) {
 // A row is a chain of two memory round trips, the activations and (the conditioning of an adaptive norm is as large as
 // the row, twice over in fp32) the parameters, with two reductions between them: with the parameters asked for at the
 // start it is one (500 rows of 768: 4.3 us, was 4.9).  NCH chunks of 512 channels.
+//
+// A model's weights are more than the last-level cache holds, so every product behind a norm starts with a trip to HBM
+// that a few hundred rows do not cover (500x768x768 6.7 us with its weights in HBM, 5.8 in the cache; x1536 9.5, 7.8;
+// 500x3072x768 10.1, 7.6), while this kernel leaves half of the CUs idle.  Workgroups behind those of the rows touch
+// every line of what the next kernels read, and nobody waits for them but the kernel's end.  (A token transformer of 24
+// blocks, 311 MB of weights: 500 rows 1.93 -> 1.80 ms, 3840 rows 3.8 -> 3.5 ms.)
+constexpr int WARM_LINES = 4;  // per thread (8: 500 rows of 768 behind 5.9 MB of weights 4 % slower, 1 or 2: no faster)
 template <typename TIn, int NCH>
 __global__ __launch_bounds__(256) void ln_rows_kernel(RowNormArgs a) {
   const int lane = threadIdx.x & 63;
+  if (blockIdx.x >= a.row_blocks) {
+    const uint32_t n0 = a.warm_lines[0], n1 = n0 + a.warm_lines[1], n2 = n1 + a.warm_lines[2];
+    uint32_t got[WARM_LINES];
+#pragma unroll
+    for (int u = 0; u < WARM_LINES; ++u) {
+      const uint32_t i = ((blockIdx.x - a.row_blocks) * WARM_LINES + u) * 256u + threadIdx.x;
+      const char* p = static_cast<const char*>(i < n0 ? a.warm[0] : i < n1 ? a.warm[1] : a.warm[2]);
+      got[u] = i < n2 ? *reinterpret_cast<const uint32_t*>(p + (size_t)(i - (i < n0 ? 0u : i < n1 ? n0 : n1)) * 128) : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < WARM_LINES; ++u) asm volatile("" ::"v"(got[u]));
+    return;
+  }
   const int64_t row = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= a.rows) return;
   const TIn* x = reinterpret_cast<const TIn*>(a.x) + row * a.ldx;
@@ -176,9 +196,11 @@ int launch_small(RowNormArgs a, hipStream_t stream) {
 }
 
 template <typename TIn>
-int launch_wide(const RowNormArgs& a, hipStream_t stream) {
-  const int64_t blocks = (a.rows + 3) / 4;
-  if (blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
+int launch_wide(RowNormArgs a, hipStream_t stream) {
+  const int64_t lines = (int64_t)a.warm_lines[0] + a.warm_lines[1] + a.warm_lines[2];
+  const int64_t row_blocks = (a.rows + 3) / 4, blocks = row_blocks + (lines + 256 * WARM_LINES - 1) / (256 * WARM_LINES);
+  a.row_blocks = (unsigned)row_blocks;
+  if (lines > 0x7fffffff || blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
   const dim3 grid((unsigned)blocks), block(256);
   switch ((a.C + 511) / 512) {
     case 1: hipLaunchKernelGGL((ln_rows_kernel<TIn, 1>), grid, block, 0, stream, a); break;

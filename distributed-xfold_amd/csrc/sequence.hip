@@ -440,6 +440,7 @@ size_t af3_diffusion_transformer_workspace_bytes(int64_t batch, int64_t seq, int
          align_up(af3_batch_diffusion_self_attention_workspace_bytes(batch, seq, channels));
 }
 
+static constexpr size_t WARM_LOGIT_BYTES = (size_t)4 << 20;
 int af3_diffusion_transformer_forward(
     const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t batch, int64_t seq, int channels,
     int hidden, int num_head, const float* key_mask, const float* const* pair_logits, int bias_quad_major,
@@ -456,15 +457,33 @@ int af3_diffusion_transformer_forward(
   const size_t ab = af3_batch_diffusion_self_attention_workspace_bytes(batch, seq, c);
   void* aw = w.take(ab);
   if (!w.ok) return AF3_ERR_WORKSPACE;
+  // Adaptive LayerNorm of act, with the weights of the products up to the next one on their way into the last-level cache
+  // (rowops.hip), and the pair logits where they are no more than the weights.  The conditioning of those products, rows of
+  // 6 KB some 300 KB apart, costs more that way than it saves.
+  struct Range {
+    const void* p;
+    size_t bytes;
+  };
+  auto norm = [&](const float* ss, Range r0, Range r1, Range r2) -> int {
+    RowNormArgs a;
+    if (act_dtype != AF3_F32 && act_dtype != AF3_BF16) return AF3_ERR_BAD_ARG;
+    a.x = act; a.x_f32 = act_dtype == AF3_F32; a.y = x; a.rows = rows; a.ldx = a.ldy = c; a.C = c;
+    a.scale = ss; a.shift = ss + c; a.cond_rows = cond_rows; a.ld_cond = ld_ss;
+    int k = 0;
+    for (const Range& r : {r0, r1, r2})
+      if (r.p) { a.warm[k] = r.p; a.warm_lines[k] = (uint32_t)(r.bytes / 128); ++k; }
+    return launch_row_norm(a, static_cast<hipStream_t>(stream));
+  };
+  const size_t all_logits = (size_t)num_head * seq * seq * 4, logit_bytes = all_logits <= WARM_LOGIT_BYTES ? all_logits : 0;
   for (int i = 0; i < num_blocks; ++i) {
     const af3_diffusion_block& b = blocks[i];
     const float *ss = scale_shift + (int64_t)2 * i * 2 * c, *g = gate + (int64_t)2 * i * c;
-    STEP(af3_layer_norm_forward(act, act_dtype, x, rows, c, nullptr, nullptr, ss, ss + c, cond_rows, ld_ss, stream));
+    STEP(norm(ss, {b.w_q, (size_t)4 * c * c * 2}, {b.w_out, (size_t)c * c * 2}, {pair_logits[i], logit_bytes}));
     STEP(af3_batch_diffusion_self_attention_forward(x, key_mask, 1, pair_logits[i], bias_quad_major, b.w_q, b.q_b, num_head, y,
                                                     AF3_BF16, batch, seq, c, aw, ab, stream));
     STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, cond_rows, ld_g, act,
                             act_dtype, stream));
-    STEP(af3_layer_norm_forward(act, act_dtype, x, rows, c, nullptr, nullptr, ss + 2 * c, ss + 3 * c, cond_rows, ld_ss, stream));
+    STEP(norm(ss + 2 * c, {b.w_tr1, (size_t)2 * hidden * c * 2}, {b.w_tr2, (size_t)hidden * c * 2}, {nullptr, 0}));
     STEP(af3_linear_forward(x, b.w_tr1, nullptr, y, AF3_BF16, rows, 2 * hidden, c, AF3_LINEAR_SWIGLU, 1.f, 0, nullptr, 0, 0, nullptr, 0,
                             stream));
     STEP(af3_linear_forward(y, b.w_tr2, nullptr, act, act_dtype, rows, c, hidden, AF3_LINEAR_GATE_RES, 1.f, 0, g + c, cond_rows, ld_g,
