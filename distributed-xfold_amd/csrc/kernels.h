@@ -399,6 +399,21 @@ int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s);
 // the long product of a triangle multiplication, between the planes of its prologue and its epilogue (api.hip)
 int run_triangle_contraction(const bf16_t* a_buf, const bf16_t* b_buf, bf16_t* t_buf, int n, int valid_channels, int outgoing, hipStream_t s);
 
+// --------------------------------------------------------------- atom_step.hip
+// act [samples][atoms][128] += gate1 (y W_out^T), then += gate2 transition(LN(act)); gates and scale / shift per atom
+constexpr int ATOM_STEP_MAX_HIDDEN = 256;
+struct AtomStepArgs {
+  void* act = nullptr;
+  int io_f32 = 0, atoms = 0, samples = 0, hidden = 0;
+  const bf16_t* y = nullptr;                             // [samples][atoms][128]
+  const bf16_t *f_out = nullptr, *f_w1 = nullptr, *f_w2 = nullptr;  // weights in fragment order
+  const float *gate1 = nullptr, *gate2 = nullptr;        // [atoms][128]
+  const float* scale = nullptr;                          // [atoms][ld_cond]: 128 scales (before their sigmoid), 128 shifts
+  int64_t ld_cond = 0;
+};
+bool atom_tail_applies(const AtomStepArgs& a);
+int launch_atom_tail(const AtomStepArgs& a, hipStream_t s);
+
 // -------------------------------------------------------------------- embed.hip
 struct PairEmbedArgs {
   const float* lr = nullptr;    // [n][ld_lr]: left projection, then right

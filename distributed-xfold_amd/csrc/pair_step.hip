@@ -82,35 +82,6 @@ struct StepTile {
   }
 };
 
-// element `off` (32 bits: every array here is below 2 GB) of an array
-template <typename T>
-__device__ __forceinline__ T* at32(T* base, uint32_t off) {
-  return reinterpret_cast<T*>(reinterpret_cast<char*>(base) + off * (uint32_t)sizeof(T));
-}
-template <typename T>
-__device__ __forceinline__ const T* at32(const T* base, uint32_t off) {
-  return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + off * (uint32_t)sizeof(T));
-}
-
-template <typename TIO> __device__ __forceinline__ typename Elem<TIO>::Raw pack_raw(const float* v);
-template <> __device__ __forceinline__ Elem<bf16_t>::Raw pack_raw<bf16_t>(const float* v) { return {pack8(v)}; }
-template <> __device__ __forceinline__ Elem<float>::Raw pack_raw<float>(const float* v) {
-  return {f32x4{v[0], v[1], v[2], v[3]}, f32x4{v[4], v[5], v[6], v[7]}};
-}
-template <typename TIO> __device__ __forceinline__ void store_raw(TIO* p, const typename Elem<TIO>::Raw& r);
-template <> __device__ __forceinline__ void store_raw<bf16_t>(bf16_t* p, const Elem<bf16_t>::Raw& r) { *reinterpret_cast<u32x4*>(p) = r.v; }
-template <> __device__ __forceinline__ void store_raw<float>(float* p, const Elem<float>::Raw& r) {
-  *reinterpret_cast<f32x4*>(p) = r.a;
-  *reinterpret_cast<f32x4*>(p + 4) = r.b;
-}
-
-// fragments of 32 weight rows (block `blk`) for `n` k-steps from k-step k0 on, of a matrix with `nks` k-steps
-template <int n>
-__device__ __forceinline__ void load_frags(const bf16_t* w, int blk, int nks, int k0, int lane, bf16x8* f) {
-  const bf16_t* p = w + (blk * nks + k0) * 512;  // (uniform)
-#pragma unroll
-  for (int i = 0; i < n; ++i) f[i] = as_frag(*reinterpret_cast<const u32x4*>(at32(p + i * 512, (uint32_t)lane * 8u)));
-}
 template <typename TIO, int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT>
 __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(PairStepArgs a) {
   using E = Elem<TIO>;

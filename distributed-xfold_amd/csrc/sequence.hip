@@ -535,6 +535,14 @@ int af3_atom_transformer_forward(
     STEP(run_gathered_attention(xq, xk, key_rows, pl, bias_quad_major, mask_q, mask_k, subsets, b.w_q, b.w_kv, b.q_b, num_head, y,
                                 AF3_BF16, samples * subsets, queries, keys, samples, atoms, c, aw, ab,
                                 static_cast<hipStream_t>(stream)));
+    AtomStepArgs tail;
+    tail.act = act; tail.io_f32 = act_dtype == AF3_F32; tail.atoms = (int)atoms; tail.samples = (int)samples; tail.hidden = hidden;
+    tail.y = y; tail.gate1 = g; tail.gate2 = g + atoms * c; tail.scale = ss + 2 * c; tail.ld_cond = ld_q;
+    tail.f_out = b.frags; tail.f_w1 = b.frags ? b.frags + c * c : nullptr; tail.f_w2 = b.frags ? tail.f_w1 + 2 * hidden * c : nullptr;
+    if (c == 128 && rows <= 0x7fffffff && atom_tail_applies(tail)) {
+      STEP(launch_atom_tail(tail, static_cast<hipStream_t>(stream)));
+      continue;
+    }
     STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, atoms, 0, act, act_dtype,
                             stream));
     STEP(af3_layer_norm_forward(act, act_dtype, xq, rows, c, nullptr, nullptr, ss + 2 * c, ss + 3 * c, atoms, ld_q, stream));

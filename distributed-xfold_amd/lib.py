@@ -40,7 +40,7 @@ class MsaBlockStruct(C.Structure):
 class DiffusionBlockStruct(C.Structure):
     """af3_diffusion_block."""
     device = None
-    _fields_ = [(k, _vp) for k in ("w_q", "w_kv", "q_b", "w_out", "w_tr1", "w_tr2")]
+    _fields_ = [(k, _vp) for k in ("w_q", "w_kv", "q_b", "w_out", "w_tr1", "w_tr2", "frags")]
 
 
 # name -> (restype, argtypes); must list every symbol include/af3_hip.h declares

@@ -13,7 +13,7 @@ import torch.nn as nn
 from .. import check
 from .. import lib as L
 from .. import ops
-from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode, pack_swiglu, packs_of, pad_rows, point
+from .base import HipModule, as_written, bf16, drop_mesh, f32, fragments, in_check_mode, pack_swiglu, packs_of, pad_rows, point
 
 
 def plain_blocks(blocks, norms, attention: type, num_head: int) -> bool:
@@ -41,7 +41,7 @@ def block_table(owner: HipModule, blocks, c: int):
     held = owner._native
     if held is not None and len(held[1]) == len(packs) and all(map(operator.is_, held[1], packs)):
         return held[0]
-    table = (L.DiffusionBlockStruct * len(blocks))()
+    table, frags = (L.DiffusionBlockStruct * len(blocks))(), []
     table.device, table.hidden = None, packs[3]["w"].shape[1]
     for i, s in enumerate(table):
         att, att_out, tr, tr_out = packs[4 * i:4 * i + 4]
@@ -53,7 +53,10 @@ def block_table(owner: HipModule, blocks, c: int):
         point(s, ("q_b", att["q_b"], (c,)), ("w_out", att_out["w"], (c, c)), ("w_tr1", tr["w1"], (2 * table.hidden, c)),
               ("w_tr2", tr_out["w"], (c, table.hidden)))
         table.device = s.device
-    owner._native = (table, packs)
+        if "w_kv" in att and c == 128 and table.hidden % 64 == 0:
+            frags.append(torch.cat([fragments(torch.cat([att_out["w"], tr["w1"]])), fragments(tr_out["w"])]))
+            s.frags = frags[-1].data_ptr()
+    owner._native = (table, packs, frags)
     return table
 
 
