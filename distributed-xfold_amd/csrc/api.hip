@@ -557,6 +557,7 @@ int af3_gathered_cross_attention_forward(
     const uint16_t* w_qg, const uint16_t* w_kv, const float* query_b, int num_head,
     void* out, int out_dtype, int64_t batch, int64_t sq, int64_t sk, int64_t samples, int64_t n_atoms, int channels,
     void* workspace, size_t workspace_bytes, af3_stream_t stream) {
+  if (!q_data || !atom_data) return AF3_ERR_BAD_ARG;
   return run_gathered_attention(q_data, atom_data, key_rows, pair_logits, 0, mask_q, mask_k, bias_batches, w_qg, w_kv, query_b,
                                 num_head, out, out_dtype, batch, sq, sk, samples, n_atoms, channels, workspace, workspace_bytes,
                                 static_cast<hipStream_t>(stream));
@@ -745,12 +746,20 @@ int run_linear(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int
   return launch_gemm_nt(g, stream);
 }
 
+bool gathered_projections(void* workspace, size_t workspace_bytes, int64_t query_rows, int64_t atom_rows, int channels, bf16_t** qg,
+                          bf16_t** kv) {
+  Carver ws(workspace, workspace_bytes);
+  *qg = ws.take<bf16_t>((size_t)query_rows * 2 * channels);
+  *kv = ws.take<bf16_t>((size_t)atom_rows * 2 * channels);
+  return ws.ok;
+}
+
 int run_gathered_attention(const bf16_t* q_data, const bf16_t* atom_data, const int32_t* key_rows, const float* pair_logits,
                            int bias_quad_major, const float* mask_q, const float* mask_k, int64_t bias_batches, const bf16_t* w_qg,
                            const bf16_t* w_kv, const float* query_b, int num_head, void* out, int out_dtype, int64_t batch,
                            int64_t sq, int64_t sk, int64_t samples, int64_t n_atoms, int channels, void* workspace,
                            size_t workspace_bytes, hipStream_t stream) {
-  if (!q_data || !atom_data || !key_rows || !w_qg || !w_kv || !out) return AF3_ERR_BAD_ARG;
+  if (!q_data != !atom_data || !key_rows || !w_qg || !w_kv || !out) return AF3_ERR_BAD_ARG;
   if (bad_dtype(out_dtype) || batch <= 0 || sq <= 0 || sk <= 0 || samples <= 0 || n_atoms <= 0 || channels <= 0 ||
       (channels & 7) || num_head <= 0 || channels % num_head)
     return AF3_ERR_BAD_ARG;
@@ -760,12 +769,11 @@ int run_gathered_attention(const bf16_t* q_data, const bf16_t* atom_data, const 
   if (batch * sq > 0x7fffffff || samples * n_atoms > 0x7fffffff) return AF3_ERR_BAD_ARG;
   const int d = channels / num_head;
   if (d != 24 && d != 32 && d != 48) return AF3_ERR_UNSUPPORTED;
-  Carver ws(workspace, workspace_bytes);
-  bf16_t* qg = ws.take<bf16_t>((size_t)batch * sq * 2 * channels);
-  bf16_t* kv = ws.take<bf16_t>((size_t)samples * n_atoms * 2 * channels);
-  if (!ws.ok) return AF3_ERR_WORKSPACE;
+  bf16_t *qg, *kv;
+  if (!gathered_projections(workspace, workspace_bytes, batch * sq, samples * n_atoms, channels, &qg, &kv)) return AF3_ERR_WORKSPACE;
   hipStream_t s = stream;
 
+  if (q_data) {
   GemmArgs g;
   g.A = q_data; g.B = w_qg; g.C = qg;
   g.M = (int)(batch * sq); g.N = 2 * channels; g.K = channels;
@@ -782,6 +790,7 @@ int run_gathered_attention(const bf16_t* q_data, const bf16_t* atom_data, const 
   g2.lda = channels; g2.ldb = channels; g2.ldc = 2 * channels;
   rc = launch_gemm_nt(g2, s);
   if (rc) return rc;
+  }
 
   FlashArgs f;
   f.q = qg; f.g = qg + channels; f.k = kv; f.v = kv + channels;

@@ -92,6 +92,9 @@ int run_gathered_attention(const bf16_t* q_data, const bf16_t* atom_data, const 
                            const bf16_t* w_kv, const float* query_b, int num_head, void* out, int out_dtype, int64_t batch,
                            int64_t sq, int64_t sk, int64_t samples, int64_t n_atoms, int channels, void* workspace,
                            size_t workspace_bytes, hipStream_t stream);
+// where in its workspace the projections are (false: too small); with q_data and atom_data null they are there already
+bool gathered_projections(void* workspace, size_t workspace_bytes, int64_t query_rows, int64_t atom_rows, int channels, bf16_t** qg,
+                          bf16_t** kv);
 // Which bias entries a launch reads.  Column c takes bias[c] when the epilogue is not segmented, or
 // when c lies in a segment whose op is SEG_BIAS_SCALE; the kernels read whole groups of entries
 // (gemm_nt_kernel up to 8 from a multiple of 8, the large tile 4 from a multiple of 4, the last
@@ -400,7 +403,8 @@ int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s);
 int run_triangle_contraction(const bf16_t* a_buf, const bf16_t* b_buf, bf16_t* t_buf, int n, int valid_channels, int outgoing, hipStream_t s);
 
 // --------------------------------------------------------------- atom_step.hip
-// act [samples][atoms][128] += gate1 (y W_out^T), then += gate2 transition(LN(act)); gates and scale / shift per atom
+// Tail: act [samples][atoms][128] += gate1 (y W_out^T), then += gate2 transition(LN(act)).  Head: the projections of the
+// attention behind it, of act's two LayerNorms.  Gates and scale / shift per atom.
 constexpr int ATOM_STEP_MAX_HIDDEN = 256;
 struct AtomStepArgs {
   void* act = nullptr;
@@ -408,11 +412,16 @@ struct AtomStepArgs {
   const bf16_t* y = nullptr;                             // [samples][atoms][128]
   const bf16_t *f_out = nullptr, *f_w1 = nullptr, *f_w2 = nullptr;  // weights in fragment order
   const float *gate1 = nullptr, *gate2 = nullptr;        // [atoms][128]
-  const float* scale = nullptr;                          // [atoms][ld_cond]: 128 scales (before their sigmoid), 128 shifts
-  int64_t ld_cond = 0;
+  const float *scale = nullptr, *scale_q = nullptr;      // [atoms][ld_cond]: 128 scales (before their sigmoid), 128 shifts
+  const float* scale_k = nullptr;                        // [atoms][ld_cond_k]
+  int64_t ld_cond = 0, ld_cond_k = 0;
+  const bf16_t* f_head = nullptr;                        // q, gate, k, v
+  const float* q_bias = nullptr;                         // [128] or null
+  float q_scale = 1.f;
+  bf16_t *qg = nullptr, *kv = nullptr;                   // [samples][atoms][256]: q, gate;  k, v
 };
-bool atom_tail_applies(const AtomStepArgs& a);
-int launch_atom_tail(const AtomStepArgs& a, hipStream_t s);
+bool atom_steps_apply(const AtomStepArgs& a);
+int launch_atom_step(const AtomStepArgs& a, bool tail, bool head, hipStream_t s);
 
 // -------------------------------------------------------------------- embed.hip
 struct PairEmbedArgs {

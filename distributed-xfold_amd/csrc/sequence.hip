@@ -517,11 +517,50 @@ int af3_atom_transformer_forward(
   const size_t ab = af3_gathered_cross_attention_workspace_bytes(samples * subsets, queries, samples, atoms, c);
   void* aw = w.take(ab);
   if (!w.ok) return AF3_ERR_WORKSPACE;
+  // everything between two attentions in one kernel, where all blocks' weights are there in its order
+  auto step_args = [&](int i) {
+    const af3_diffusion_block& b = blocks[i];
+    const float *ss = scale_shift_q + (int64_t)2 * i * 2 * c, *g = gate + (int64_t)2 * i * atoms * c;
+    AtomStepArgs a;
+    a.act = act; a.io_f32 = act_dtype == AF3_F32; a.atoms = (int)atoms; a.samples = (int)samples; a.hidden = hidden;
+    a.y = y; a.gate1 = g; a.gate2 = g + atoms * c; a.scale = ss + 2 * c; a.ld_cond = ld_q;
+    a.f_out = b.frags;
+    if (b.frags) { a.f_w1 = b.frags + c * c; a.f_w2 = a.f_w1 + 2 * hidden * c; }
+    return a;
+  };
+  auto attention_args = [&](AtomStepArgs& a, int i) {  // the attention behind the step is block i's
+    const af3_diffusion_block& b = blocks[i];
+    a.f_head = b.frags ? b.frags + (c + 3 * hidden) * c : nullptr;
+    a.scale_q = scale_shift_q + (int64_t)2 * i * 2 * c;
+    a.scale_k = scale_shift_k + (int64_t)i * 2 * c; a.ld_cond_k = ld_k;
+    a.q_bias = b.q_b; a.q_scale = 1.0f / sqrtf((float)(c / num_head));
+    (void)gathered_projections(aw, ab, rows, rows, c, &a.qg, &a.kv);
+  };
+  bool steps = c == 128 && rows <= 0x7fffffff && (act_dtype == AF3_F32 || act_dtype == AF3_BF16);
+  for (int i = 0; i < num_blocks && steps; ++i) {
+    AtomStepArgs a = step_args(i);
+    attention_args(a, i);
+    steps = atom_steps_apply(a);
+  }
   for (int i = 0; i < num_blocks; ++i) {
     const af3_diffusion_block& b = blocks[i];
+    const float* pl = pair_logits ? pair_logits + (int64_t)i * subsets * num_head * queries * keys : nullptr;
+    if (steps) {
+      AtomStepArgs a = step_args(i);
+      if (i == 0) {
+        attention_args(a, 0);
+        STEP(launch_atom_step(a, false, true, static_cast<hipStream_t>(stream)));
+      }
+      STEP(run_gathered_attention(nullptr, nullptr, key_rows, pl, bias_quad_major, mask_q, mask_k, subsets, b.w_q, b.w_kv, b.q_b, num_head, y,
+                                  AF3_BF16, samples * subsets, queries, keys, samples, atoms, c, aw, ab,
+                                  static_cast<hipStream_t>(stream)));
+      const bool more = i + 1 < num_blocks;
+      attention_args(a, more ? i + 1 : i);
+      STEP(launch_atom_step(a, true, more, static_cast<hipStream_t>(stream)));
+      continue;
+    }
     const float *ss = scale_shift_q + (int64_t)2 * i * 2 * c, *sk = scale_shift_k + (int64_t)i * 2 * c;
     const float* g = gate + (int64_t)2 * i * atoms * c;
-    const float* pl = pair_logits ? pair_logits + (int64_t)i * subsets * num_head * queries * keys : nullptr;
     if (c <= 128) {
       RowNormArgs ln;
       ln.x = act; ln.x_f32 = act_dtype == AF3_F32; ln.rows = rows; ln.ldx = ln.ldy = ln.C = c;
@@ -535,14 +574,6 @@ int af3_atom_transformer_forward(
     STEP(run_gathered_attention(xq, xk, key_rows, pl, bias_quad_major, mask_q, mask_k, subsets, b.w_q, b.w_kv, b.q_b, num_head, y,
                                 AF3_BF16, samples * subsets, queries, keys, samples, atoms, c, aw, ab,
                                 static_cast<hipStream_t>(stream)));
-    AtomStepArgs tail;
-    tail.act = act; tail.io_f32 = act_dtype == AF3_F32; tail.atoms = (int)atoms; tail.samples = (int)samples; tail.hidden = hidden;
-    tail.y = y; tail.gate1 = g; tail.gate2 = g + atoms * c; tail.scale = ss + 2 * c; tail.ld_cond = ld_q;
-    tail.f_out = b.frags; tail.f_w1 = b.frags ? b.frags + c * c : nullptr; tail.f_w2 = b.frags ? tail.f_w1 + 2 * hidden * c : nullptr;
-    if (c == 128 && rows <= 0x7fffffff && atom_tail_applies(tail)) {
-      STEP(launch_atom_tail(tail, static_cast<hipStream_t>(stream)));
-      continue;
-    }
     STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, atoms, 0, act, act_dtype,
                             stream));
     STEP(af3_layer_norm_forward(act, act_dtype, xq, rows, c, nullptr, nullptr, ss + 2 * c, ss + 3 * c, atoms, ld_q, stream));

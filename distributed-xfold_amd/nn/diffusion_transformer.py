@@ -54,7 +54,8 @@ def block_table(owner: HipModule, blocks, c: int):
               ("w_tr2", tr_out["w"], (c, table.hidden)))
         table.device = s.device
         if "w_kv" in att and c == 128 and table.hidden % 64 == 0:
-            frags.append(torch.cat([fragments(torch.cat([att_out["w"], tr["w1"]])), fragments(tr_out["w"])]))
+            frags.append(torch.cat([fragments(torch.cat([att_out["w"], tr["w1"]])), fragments(tr_out["w"]),
+                                    fragments(torch.cat([att["w_qg"], att["w_kv"]]), swap23=True)]))
             s.frags = frags[-1].data_ptr()
     owner._native = (table, packs, frags)
     return table

@@ -657,8 +657,9 @@ typedef struct af3_diffusion_block {
   const uint16_t* w_out; /* [c][c] */
   const uint16_t* w_tr1; /* [2 hidden][c], packed for AF3_LINEAR_SWIGLU */
   const uint16_t* w_tr2; /* [c][hidden] */
-  /* atom: NULL, or w_out, w_tr1 and w_tr2 once more, for the block's tail in one kernel (c = 128, hidden at most 256 and a
-   * multiple of 64), in the order of af3_pairformer_block's pair_frags; diffusion: not read */
+  /* atom: NULL, or w_out, w_tr1, w_tr2 and, with the exchanged rows, w_q, w_kv once more, in the order of
+   * af3_pairformer_block's pair_frags: what lies between two attentions is then one kernel (c = 128, hidden at most 256
+   * and a multiple of 64, in all blocks of a call); diffusion: not read */
   const uint16_t* frags;
 } af3_diffusion_block;
 size_t af3_diffusion_transformer_workspace_bytes(int64_t batch, int64_t seq, int channels, int hidden);
