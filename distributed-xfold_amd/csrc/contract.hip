@@ -480,26 +480,27 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
     }
   };
 
-  // Outer-product mean of the tile's 8 x 8 token pairs (b, d): pair = (res ? pair : 0) + (W vec(outer) + bias) * gate.
-  // The outer products go to the slab buffers (which hold nothing by now) as 64 rows of 1024 bf16, chunk c of row r at
+  // Outer-product mean of the tile's 2 IT x 8 token pairs (b, d): pair = (res ? pair : 0) + (W vec(outer) + bias) * gate.
+  // The outer products go to the slab buffers (which hold nothing by now) as 16 IT rows of 1024 bf16, chunk c of row r at
   // position c ^ (c >> 4 & 3) ^ (r & 15): both the 8-byte writes and the fragment reads spread over the banks.  Wave w
   // takes outputs 32 w .. 32 w + 31 of all pairs; its share of the weights, packed in the order of its loads, comes
   // from L2, 64 KB per tile (W's rows in the order swap23: eight consecutive outputs per lane).
   // 768 tokens, 1024 MSA rows: 1080 us, of which a tile's K loop is two thirds.  As two products with the outer products
-  // in memory between them (six times 205 + 66 us) the same bits took 1630; 187 tokens, 301 rows 47 (75), 160 tokens,
-  // 128 rows 25 (55).
-  f32x16 outer[2];    // 32 outputs x 32 pairs each
-  float outer_gate[2];
-  u32x4 outer_res[2][2][2];
+  // in memory between them (six times 205 + 66 us) the same bits took 1630; 187 tokens, 301 rows 47 (75; with
+  // tiles of 192 rows 41), 160 tokens, 128 rows 25 (55).
+  constexpr int PH = IT == 2 ? 1 : 2;  // a tile's 2 IT x 8 token pairs, 32 at a time
+  f32x16 outer[PH];                    // 32 outputs x 32 pairs each
+  float outer_gate[PH];
+  u32x4 outer_res[PH][2][2];
   auto outer_pixel = [&](const Tile& t, int p, bool* ok) {
     const int n = g.N >> 5, b = (t.m0 >> 5) + 4 * p + (l31 >> 3), d = (t.n0 >> 5) + (l31 & 7);
-    *ok = b < n && d < n;
+    *ok = b < n && d < n && 4 * p + (l31 >> 3) < 2 * IT;
     return (int64_t)min(b, n - 1) * n + min(d, n - 1);
   };
   auto outer_tile = [&](const Tile& t) {
     constexpr int KSTEPS = 64, RW = 8, RX = 6;  // fragments under way: weights from L2, outer products from LDS
     const bf16_t* wp = uniform_ptr(g.w2 + wave * KSTEPS * 512) + lane * 8;
-    u32x4 wf[RW], xf[RX][2];
+    u32x4 wf[RW], xf[RX][PH];
     auto load_w = [&](int ks) {
       if (ks < KSTEPS) wf[ks % RW] = *reinterpret_cast<const u32x4*>(wp + ks * 512);
     };
@@ -513,7 +514,7 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
     const uint32_t st = (uint32_t)((8 * (wm >> 5) + (wn >> 5)) * 2048 + 8 * hh);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const uint32_t chunk = (uint32_t)(4 * l31 + (q ^ (l31 >> 2 & 3))) ^ (uint32_t)(wn >> 5);
+      const uint32_t chunk = (uint32_t)(4 * l31 + (q ^ (l31 >> 2 & 3))) ^ (uint32_t)((wn >> 5) + 8 * (wm >> 5 & 1));
 #pragma unroll
       for (int it = 0; it < IT; ++it)
 #pragma unroll
@@ -530,11 +531,11 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
       if (ks < KSTEPS) {
         const uint32_t at = rd ^ (uint32_t)((2 * ks ^ (ks >> 3 & 3)) << 4);
 #pragma unroll
-        for (int p = 0; p < 2; ++p) xf[ks % RX][p] = *reinterpret_cast<const u32x4*>(smem + at + p * 65536);
+        for (int p = 0; p < PH; ++p) xf[ks % RX][p] = *reinterpret_cast<const u32x4*>(smem + at + p * 65536);
       }
     };
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
+    for (int p = 0; p < PH; ++p)
 #pragma unroll
       for (int r = 0; r < 16; ++r) outer[p][r] = 0.f;
 #pragma unroll
@@ -547,7 +548,7 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
       }
       if (ks == KSTEPS / 2) {  // what the results are joined with
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
+        for (int p = 0; p < PH; ++p) {
           bool ok;
           const int64_t pix = outer_pixel(t, p, &ok);
           outer_gate[p] = g.gate[pix];
@@ -566,13 +567,13 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
       load_w(ks + RW - 1);
       read_x(ks + RX - 1);
 #pragma unroll
-      for (int p = 0; p < 2; ++p) outer[p] = mfma32(as_frag(wf[ks % RW]), as_frag(xf[ks % RX][p]), outer[p]);
+      for (int p = 0; p < PH; ++p) outer[p] = mfma32(as_frag(wf[ks % RW]), as_frag(xf[ks % RX][p]), outer[p]);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
   auto outer_store = [&](const Tile& t) {
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
+    for (int p = 0; p < PH; ++p) {
       bool ok;
       const int64_t pix = outer_pixel(t, p, &ok);
 #pragma unroll
@@ -743,10 +744,22 @@ int launch_outer_mean(const GemmArgs& g, hipStream_t stream) {
     return AF3_ERR_BAD_ARG;
   if (!al16(g.A) || !al16(g.B) || !al16(g.C) || !al16(g.w2) || !al16(g.bias) || !al16(g.res_f32) || !al16(g.res_bf16))
     return AF3_ERR_BAD_ARG;
-  const int64_t tiles = (g.M + 255) / 256, slots = ((tiles + 3) / 4 * ((tiles + 7) / 8) + 7) / 8 * 256;
+  // Tiles of 256, 192 or 128 rows, by what their rounds cost (an XCD's CUs take 4 x 8 tiles at a time): a slab of 64 MSA
+  // rows 0.31 us for every 64 tile rows, the epilogue 10 us, of 32 token pairs 6.  The whole operator, tokens x MSA rows, us
+  // with 256 / 192 / 128 rows: 64 x 512 44.3 / 41.3 / 36.4, 96 x 512 46.6 / 42.5 / 49.1, 128 x 512 47.1 / 60.1 / 52.3,
+  // 160 x 128 47.2 / 53.8 / 52.0, 187 x 301 79.0 / 73.2 / 77.6, 187 x 1024 132 / 116 / 133, 260 x 1024 216 / 217 / 250.
+  const int64_t tn = (g.M + 255) / 256, nk = (g.K + CK - 1) / CK;
+  auto slots_of = [&](int it) { return ((g.M + 64 * it - 1) / (64 * it) + 3) / 4 * ((tn + 7) / 8); };
+  auto cost = [&](int it) { return (slots_of(it) + 7) / 8 * (it * nk + (it == 2 ? 20 : 32)); };
+  int it = 4;
+  if (cost(3) * 20 < cost(it) * 19) it = 3;
+  if (cost(2) * 20 < cost(it) * 19) it = 2;
+  const int64_t slots = (slots_of(it) + 7) / 8 * 256;
   if (slots > 0x3fffffff) return AF3_ERR_BAD_ARG;
-  hipLaunchKernelGGL(contract_kernel<BIG_OUTER_MEAN>, dim3((unsigned)std::min<int64_t>(slots, cu_count() / 8 * 8)), dim3(256), 0,
-                     stream, g);
+  const dim3 grid((unsigned)std::min<int64_t>(slots, cu_count() / 8 * 8)), block(256);
+  if (it == 2) hipLaunchKernelGGL((contract_kernel<BIG_OUTER_MEAN, 2>), grid, block, 0, stream, g);
+  else if (it == 3) hipLaunchKernelGGL((contract_kernel<BIG_OUTER_MEAN, 3>), grid, block, 0, stream, g);
+  else hipLaunchKernelGGL((contract_kernel<BIG_OUTER_MEAN, 4>), grid, block, 0, stream, g);
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
 
