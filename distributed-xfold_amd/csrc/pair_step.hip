@@ -567,6 +567,9 @@ bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // Patches of 8 x 8 pixels from one workgroup per CU on: what a patch writes of a transposed operand is then whole 16-byte
 // pieces.
 constexpr int64_t WIDE_PATCHES = 256 * 64;
+// Projections behind an epilogue or an output in tiles of 64 positions: half of the weights' traffic, where there are tiles
+// enough; us, 32 / 64 positions, 301 tokens 48 / 45 (epilogue), 46 / 43 (output); 160 tokens 18.9 / 19.5, 18.4 / 18.6.
+constexpr int64_t WIDE_ROWS = 208 * 208 + 1;
 
 template <int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT>
 int launch_tiles(const PairStepArgs& a, hipStream_t s) {
@@ -608,8 +611,12 @@ int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s) {
     case PAIR_STEP_INCOMING:
       if ((int64_t)a.N * a.ldn >= WIDE_PATCHES) return launch_tiles<128, 2, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
       return launch_tiles<128, 1, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
-    case PAIR_STEP_PROJECT_START: return launch_tiles<128, 1, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
-    case PAIR_STEP_PROJECT_END: return launch_tiles<128, 1, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
+    case PAIR_STEP_PROJECT_START:
+      if ((int64_t)a.N * a.ldn >= WIDE_ROWS) return launch_tiles<128, 2, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
+      return launch_tiles<128, 1, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
+    case PAIR_STEP_PROJECT_END:
+      if ((int64_t)a.N * a.ldn >= WIDE_ROWS) return launch_tiles<128, 2, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
+      return launch_tiles<128, 1, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
     case PAIR_STEP_LAST: return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_NONE>(a, s);
     case PAIR_STEP_NEXT: return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_PROLOGUE>(a, s);
   }

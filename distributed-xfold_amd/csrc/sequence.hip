@@ -52,20 +52,6 @@ struct Event {
     if (rc_ != AF3_OK) return rc_; \
   } while (0)
 
-int pair_operators(const af3_pairformer_block& b, void* pair, int dt, const float* mask, const float* mask_in, int64_t n,
-                   void* ws, size_t wsb, af3_stream_t s) {
-  for (int d = 0; d < 2; ++d)
-    STEP(af3_triangle_multiplication_forward_padded(pair, dt, d == 1 && mask_in ? mask_in : mask, d, b.tm_ln_in_w[d], b.tm_ln_in_b[d],
-                                                    b.tm_w_proj_gate[d], b.tm_ln_c_w[d], b.tm_ln_c_b[d], b.tm_w_out[d],
-                                                    b.tm_w_gating[d], pair, 1, n, b.valid_channels, ws, wsb, s));
-  for (int d = 0; d < 2; ++d)
-    STEP(af3_grid_self_attn_forward_padded(pair, dt, mask, d, b.ta_ln_w[d], b.ta_ln_b[d], b.ta_w_bias[d], nullptr,
-                                           b.ta_w_qkvg[d], b.ta_w_out[d], b.num_head_pair, pair, 1, n, b.valid_channels, ws,
-                                           wsb, s));
-  return af3_transition_forward_padded(pair, dt, b.pt_ln_w, b.pt_ln_b, b.pt_w1, b.pt_w2, b.pair_hidden, pair, 1, n * n,
-                                       b.valid_channels, s);
-}
-
 // ---- the pair operators at few tokens: a run of them between two long products in one kernel (pair_step.hip) ----
 // A step takes the chain of one tile of 32 positions where a kernel of its own per operator takes several of tiles of 128,
 // and eight launches a block take the place of fourteen; past some number of tiles what every tile fetches of the weights
@@ -75,9 +61,14 @@ int pair_operators(const af3_pairformer_block& b, void* pair, int dt, const floa
 // Pair tensors of 64 channels have no other kernels (64 / 301 / 768 / 2048 tokens, bf16, a block on its own: 100 -> 46,
 // 345 -> 221, 1940 -> 1460, 22400 -> 18800 against one zero-padded to 128; their 32-bit offsets end at 3072).
 constexpr int64_t PAIR_STEP_POSITIONS = 208 * 208;
-bool pair_steps_apply(const af3_pairformer_block& b, int64_t n) {
+// Beyond, the two steps that end in an attention's projections stay the faster form for a while (they only read the tensor's
+// rows as they lie, and half of a tile's weights): runs of 4 blocks, us a block, without -> with them (bf16 / fp32 stream),
+// 209 tokens 251 -> 239 / 267 -> 253, 301: 393 -> 385 / 448 -> 428, 387: 640 -> 630 / 732 -> 703, 420: 714 -> 708 /
+// 829 -> 810, 450: 830 -> 835 / 982 -> 966.
+constexpr int64_t PROJECT_STEP_POSITIONS = 400 * 400;
+bool pair_steps_apply(const af3_pairformer_block& b, int64_t n, int64_t positions = PAIR_STEP_POSITIONS) {
   const int c = b.pair_channels == 64 ? 64 : 128;
-  return b.pair_frags && n <= 8192 && (c == 64 ? n <= AF3_PAIR64_MAX_TOKENS : n * tri_ldn(n) <= PAIR_STEP_POSITIONS) &&
+  return b.pair_frags && n <= 8192 && (c == 64 ? n <= AF3_PAIR64_MAX_TOKENS : n * tri_ldn(n) <= positions) &&
          b.num_head_pair == 4 && b.valid_channels >= 8 && b.valid_channels <= c && b.valid_channels % 4 == 0 &&
          (c == 128 || b.valid_channels == 64) && b.pair_hidden > 0 && b.pair_hidden % 64 == 0 &&
          b.pair_hidden <= pair_step_max_hidden(c);
@@ -90,7 +81,7 @@ struct PairStepScratch {
   static size_t vt_bytes(int64_t n, int c) { return (size_t)n * c * tri_ldn(n) * 2; }
   static size_t bytes(int64_t n, int c) {
     return 3 * align_up(plane_bytes(n, c)) + align_up(vt_bytes(n, c)) + align_up((size_t)tri_bias_elems(n, 4) * 2) +
-           (c == 128 ? LOGIT_RING * logit_bytes(n, 16) : 0);
+           (c == 128 && n * tri_ldn(n) <= PAIR_STEP_POSITIONS ? LOGIT_RING * logit_bytes(n, 16) : 0);
   }
   // Pair logits of the last blocks, where the single track runs on a stream of its own.  With two buffers every block waits
   // for the attention two blocks back, and an event recorded and waited for costs the host 13 us, where a launch costs 3.5:
@@ -109,10 +100,10 @@ struct PairStepScratch {
   }
 };
 
-// One block's pair operators.  `first`: no step before has made the outgoing prologue.  `next`: the block whose outgoing
+// One block's pair operators.  `partly`: in steps only where an attention's projections are the second half.  `first`: no step before has made the outgoing prologue.  `next`: the block whose outgoing
 // prologue the last step makes, or null.  `logits`: where the pair logits of the single track go, or null; they are
 // written behind `logits_free`.
-int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_block* next, bool first, void* pair, int dt,
+int pair_operators_in_steps(const af3_pairformer_block& b, bool partly, const af3_pairformer_block* next, bool first, void* pair, int dt,
                             const float* mask, const float* mask_in, int64_t n, void* ws, size_t wsb, float* logits,
                             Event* logits_free, hipStream_t s) {
   if (!pair || (dt != AF3_F32 && dt != AF3_BF16) || ((uintptr_t)pair & 15) || ((uintptr_t)mask & 15) || ((uintptr_t)mask_in & 15))
@@ -138,21 +129,29 @@ int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_
   core.q = w.qa; core.k = w.kb; core.vt = w.vt; core.bias = w.bias; core.mask = mask; core.og = w.ogt; core.N = (int)n; core.ldn = a.ldn;
   core.head_dim = wide / 4;
 
+  auto product = [&](int d) {  // a triangle multiplication's prologue or epilogue as a kernel of its own
+    TriMulArgs p;
+    p.lw = a.lw; p.valid_c = c; p.pair = p.out = pair; p.mask = d == 1 && mask_in ? mask_in : mask; p.io_f32 = a.io_f32;
+    p.N = a.N; p.Np = a.Np; p.plane = a.plane; p.outgoing = d == 0; p.residual = 1;
+    p.ln_in_w = b.tm_ln_in_w[d]; p.ln_in_b = b.tm_ln_in_b[d]; p.ln_c_w = b.tm_ln_c_w[d]; p.ln_c_b = b.tm_ln_c_b[d];
+    p.w_pg = b.tm_w_proj_gate[d]; p.w_gl = b.tm_w_gating[d]; p.w_out = b.tm_w_out[d];
+    p.a_buf = w.qa; p.b_buf = w.kb; p.t_buf = w.ogt;
+    return p;
+  };
   if (first && wide == 64) {
     a.ln3_w = b.tm_ln_in_w[0]; a.ln3_b = b.tm_ln_in_b[0]; a.f_next = tm(b, 0, 2); a.mask = mask;
     STEP(launch_pair_step(a, PAIR_STEP_FIRST, s));
   } else if (first) {
-    TriMulArgs p;
-    p.lw = a.lw; p.valid_c = c; p.pair = pair; p.mask = mask; p.io_f32 = a.io_f32; p.N = a.N; p.Np = a.Np; p.plane = a.plane;
-    p.ln_in_w = b.tm_ln_in_w[0]; p.ln_in_b = b.tm_ln_in_b[0]; p.w_pg = b.tm_w_proj_gate[0];
-    p.a_buf = w.qa; p.b_buf = w.kb;
-    STEP(launch_trimul_prologue(p, s));
+    STEP(launch_trimul_prologue(product(0), s));
   }
   for (int d = 0; d < 2; ++d) {
     STEP(run_triangle_contraction(w.qa, w.kb, w.ogt, (int)n, c, d == 0, s));
     a.ln1_w = b.tm_ln_in_w[d]; a.ln1_b = b.tm_ln_in_b[d]; a.f_gate = tm(b, d, 0); a.f_out = tm(b, d, 1);
     a.ln_c_w = b.tm_ln_c_w[d]; a.ln_c_b = b.tm_ln_c_b[d];
-    if (d == 0) {
+    if (d == 0 && partly) {
+      STEP(launch_trimul_epilogue(product(0), s));
+      STEP(launch_trimul_prologue(product(1), s));
+    } else if (d == 0) {
       a.ln3_w = b.tm_ln_in_w[1]; a.ln3_b = b.tm_ln_in_b[1]; a.f_next = tm(b, 1, 2); a.mask = mask_in ? mask_in : mask;
       STEP(launch_pair_step(a, PAIR_STEP_INCOMING, s));
     } else {
@@ -165,6 +164,14 @@ int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_
   a.ln3_w = b.ta_ln_w[1]; a.ln3_b = b.ta_ln_b[1]; a.f_next = qkg(1, 0); a.f_v = ta(1, 0);
   STEP(launch_pair_step(a, PAIR_STEP_PROJECT_END, s));
   STEP(launch_triattn_flash(core, s));
+  if (partly) {
+    AttnOutArgs o;
+    o.lw = a.lw; o.og = w.ogt; o.ld_og = 128; o.w_gate = b.ta_w_qkvg[1] + 3 * 128 * 128; o.w_out = b.ta_w_out[1];
+    o.pair = o.out = pair; o.ln_w = b.ta_ln_w[1]; o.ln_b = b.ta_ln_b[1];
+    o.io_f32 = a.io_f32; o.N = a.N; o.transpose = o.residual = 1;
+    STEP(launch_attn_out(o, s));
+    return af3_transition_forward_padded(pair, dt, b.pt_ln_w, b.pt_ln_b, b.pt_w1, b.pt_w2, hidden, pair, 1, n * n, c, s);
+  }
   a.ln1_w = b.ta_ln_w[1]; a.ln1_b = b.ta_ln_b[1]; a.f_gate = qkg(1, 2); a.f_out = ta(1, wide + 32);
   a.ln2_w = b.pt_ln_w; a.ln2_b = b.pt_ln_b; a.f_w1 = w1; a.f_w2 = w1 + (2 * hidden + logit_rows) * wide;
   if (logits) {
@@ -174,6 +181,23 @@ int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_
   if (!next) return launch_pair_step(a, PAIR_STEP_LAST, s);
   a.ln3_w = next->tm_ln_in_w[0]; a.ln3_b = next->tm_ln_in_b[0]; a.f_next = tm(*next, 0, 2); a.mask = mask;
   return launch_pair_step(a, PAIR_STEP_NEXT, s);
+}
+
+// every operator in a kernel of its own, or nearly
+int pair_operators(const af3_pairformer_block& b, void* pair, int dt, const float* mask, const float* mask_in, int64_t n,
+                   void* ws, size_t wsb, hipStream_t s) {
+  if (pair_steps_apply(b, n, PROJECT_STEP_POSITIONS))
+    return pair_operators_in_steps(b, true, nullptr, true, pair, dt, mask, mask_in, n, ws, wsb, nullptr, nullptr, s);
+  for (int d = 0; d < 2; ++d)
+    STEP(af3_triangle_multiplication_forward_padded(pair, dt, d == 1 && mask_in ? mask_in : mask, d, b.tm_ln_in_w[d], b.tm_ln_in_b[d],
+                                                    b.tm_w_proj_gate[d], b.tm_ln_c_w[d], b.tm_ln_c_b[d], b.tm_w_out[d],
+                                                    b.tm_w_gating[d], pair, 1, n, b.valid_channels, ws, wsb, s));
+  for (int d = 0; d < 2; ++d)
+    STEP(af3_grid_self_attn_forward_padded(pair, dt, mask, d, b.ta_ln_w[d], b.ta_ln_b[d], b.ta_w_bias[d], nullptr,
+                                           b.ta_w_qkvg[d], b.ta_w_out[d], b.num_head_pair, pair, 1, n, b.valid_channels, ws,
+                                           wsb, s));
+  return af3_transition_forward_padded(pair, dt, b.pt_ln_w, b.pt_ln_b, b.pt_w1, b.pt_w2, b.pair_hidden, pair, 1, n * n,
+                                       b.valid_channels, s);
 }
 
 int single_update(const af3_pairformer_block& b, void* single, int dt, const float* mask, const float* logits, int64_t n,
@@ -334,11 +358,11 @@ int af3_evoformer_stack_forward(const af3_msa_block* const* blocks, int num_bloc
     msa_transition_args(b.mt_ln_w, b.mt_ln_b, b.mt_w1, b.mt_w2, b.mt_hidden, u);
     STEP(launch_msa_update(u, s));
     if (pair_steps_apply(b.pair, n))
-      STEP(pair_operators_in_steps(b.pair, nullptr, true, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace,
+      STEP(pair_operators_in_steps(b.pair, false, nullptr, true, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace,
                                    pair_workspace_bytes, nullptr, nullptr, s));
     else
       STEP(pair_operators(b.pair, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace,
-                          pair_workspace_bytes, stream));
+                          pair_workspace_bytes, s));
   }
   return AF3_OK;
 }
@@ -346,7 +370,7 @@ int af3_evoformer_stack_forward(const af3_msa_block* const* blocks, int num_bloc
 size_t af3_pairformer_stack_workspace_bytes(int64_t n, int num_head_pair) {
   const size_t a = af3_triangle_multiplication_workspace_bytes(n), b = af3_grid_self_attn_workspace_bytes(n, num_head_pair);
   size_t most = a > b ? a : b;
-  if (n > 0 && n * tri_ldn(n) <= PAIR_STEP_POSITIONS && PairStepScratch::bytes(n, 128) > most) most = PairStepScratch::bytes(n, 128);
+  if (n > 0 && n * tri_ldn(n) <= PROJECT_STEP_POSITIONS && PairStepScratch::bytes(n, 128) > most) most = PairStepScratch::bytes(n, 128);
   if (n > 0 && n <= AF3_PAIR64_MAX_TOKENS && PairStepScratch::bytes(n, 64) > most) most = PairStepScratch::bytes(n, 64);
   return most;
 }
@@ -410,11 +434,11 @@ int af3_pairformer_stack_forward(
     if (pair_steps_apply(b, n)) {
       const bool chained = i > 0 && pair_steps_apply(*blocks[i - 1], n);
       const af3_pairformer_block* next = i + 1 < num_blocks && pair_steps_apply(*blocks[i + 1], n) ? blocks[i + 1] : nullptr;
-      rc = pair_operators_in_steps(b, next, !chained, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes,
+      rc = pair_operators_in_steps(b, false, next, !chained, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes,
                                    lg, free, main_s);
       if (rc != AF3_OK || !b.with_single) continue;
     } else {
-      rc = pair_operators(b, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes, stream);
+      rc = pair_operators(b, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes, main_s);
       if (rc != AF3_OK || !b.with_single) continue;
       if (free) rc = free->wait(main_s);
       if (rc == AF3_OK)

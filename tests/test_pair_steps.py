@@ -47,7 +47,8 @@ def _run_general(blk, *inputs):
 # of one and two; more than one block of 32 heads.
 CASES = [(1, 128, 4, 16, 0), (7, 128, 4, 16, 2), (16, 128, 4, 16, 0), (17, 128, 4, 40, 3), (33, 128, 1, 16, 0), (63, 128, 4, 16, 5),
          (64, 128, 2, 16, 0), (65, 128, 4, 16, 30), (127, 128, 4, 16, 0), (129, 128, 3, 16, 11), (208, 128, 4, 16, 9),
-         (24, 96, 1, 16, 3), (90, 96, 4, 16, 1)]
+         (24, 96, 1, 16, 3), (90, 96, 4, 16, 1),
+         (209, 128, 4, 16, 9), (217, 96, 2, 16, 0), (398, 128, 2, 16, 29)]      # steps in part: just past the line, the last
 
 
 @pytest.mark.gpu
