@@ -39,8 +39,8 @@ __global__ __launch_bounds__(256, 3) void trimul_prologue_kernel(TriMulArgs a) {
   // Steps of 64 weight rows (32 projection rows and the 32 matching gate rows) per tile.  A wave
   // runs them as a software pipeline: the 16 MFMAs of step s are issued one by one with, behind each, the
   // gating arithmetic (mask * proj * sigmoid(gate), packing, staging) of one register pair of step s - 1.
-  // Inside one wave the matrix unit works while the wave goes on issuing vector instructions; between
-  // waves of a SIMD it does not, so phases run back to back cost the sum of the two.  One barrier per step:
+  // The matrix unit works while the wave goes on issuing vector instructions; the three waves of a SIMD run in
+  // step with each other, so phases run back to back would cost nearly the sum of the two.  One barrier per step:
   // the weights and the staged results are double-buffered.
   __shared__ __attribute__((aligned(16))) bf16_t sX[TM * LDX];  // LN tile; then [S0 | S1 | W odd steps]
   __shared__ __attribute__((aligned(16))) bf16_t sW0[64 * LDX];  // weights of the even steps
@@ -513,8 +513,8 @@ __global__ __launch_bounds__(256, 2) void transition_kernel(TransitionArgs a) {
   //
   // The slabs run as a software pipeline inside each wave: the MFMAs of GEMM1 of slab h are issued one by
   // one with the gating of slab h - 1 between them, and the MFMAs of GEMM2 of slab h - 1 follow as their
-  // fragments become complete.  Phases run back to back would cost the sum of the matrix unit's and the
-  // vector unit's time (the two do not overlap between the waves of a SIMD).  W1 slabs are double-
+  // fragments become complete.  Phases run back to back would cost nearly the sum of the matrix unit's and
+  // the vector unit's time (the two waves of a SIMD run in step with each other).  W1 slabs are double-
   // buffered, W2 slabs triple-buffered (a W2 slab is used one iteration after its W1 slab); one barrier
   // per slab.
   __shared__ __attribute__((aligned(1024))) char smem[2 * TM * LDX * 2];  // 69.6 KB

@@ -704,7 +704,7 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
     if ((tid & 7) == 0) sMean[v_d] = acc;
     lds_barrier();
 #pragma unroll
-    for (int e = 0; e < 16; ++e) o[r][e] = sMean[(8 * (e >> 2) + 4 * hh + (e & 3)) & (D - 1)];
+    for (int e = 0; e < 16; ++e) o[r][e] = sMean[8 * ((e >> 2) & (D / 8 - 1)) + 4 * hh + (e & 3)];
     lrun[r] = (float)N;
   }
 
