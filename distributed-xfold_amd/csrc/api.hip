@@ -66,13 +66,17 @@ void* static_scratch_ptr() {
 
 }  // namespace
 
-// The N x N x N contraction of the triangle multiplication: the 256x256-tile
-// kernel once a token count fills at least part of a second 128-row tile,
-// the general GEMM below that.
-static int contraction(const GemmArgs& g, hipStream_t s) {
-  if (g.M > 128 && contract_supported(g)) return launch_contract(g, s);
+// A batch of products on the 256x256-tile kernel, or on the general GEMM (the same sums in the same order).
+static int batched_product(GemmArgs g, bool large, hipStream_t s) {
+  if (large && contract_supported(g)) return launch_contract(g, s);
+  g.small_tiles = 1;
   return launch_gemm_nt(g, s);
 }
+// The N x N x N contraction of the triangle multiplication: the large tile once a channel fills enough of one, and, with few
+// channels, there are enough of them.  us, general / large, 128 channels: 132 tokens 8.0 / 8.4, 160 8.4 / 8.9, 192 8.8 / 9.4,
+// but 200 12.9 / 12.0, 256 13.3 / 12.4.  64 channels, a pair block with two of them: 160 tokens 95.5 / 100, 256 141 / 146,
+// 301 201 / 207, 340 252 / 256, 387 355 / 357.
+static int contraction(const GemmArgs& g, hipStream_t s) { return batched_product(g, g.M > (g.batch > 64 ? 192 : 340), s); }
 
 int run_triangle_contraction(const bf16_t* a_buf, const bf16_t* b_buf, bf16_t* t_buf, int n, int valid_channels, int outgoing, hipStream_t s) {
   // outgoing: t[c][i][j] = sum_k a'[c][i][k] b'[c][j][k]
@@ -483,7 +487,11 @@ int af3_batched_nt_product_forward(
   g.M = (int)m; g.N = (int)n; g.K = (int)k; g.batch = (int)batch;
   g.lda = g.ldb = k; g.ldc = n;
   g.sA = m * k; g.sB = n * k; g.sC = m * n;
-  return contraction(g, static_cast<hipStream_t>(stream));
+  // The large tile where there are some hundred of them.  Eight products m x n x m, us, general / large: 160 x 1024 (32 tiles)
+  // 4.6 / 7.6, 187 x 2408 (80) 6.6 / 8.3, 640 x 1024 (96) 13.6 / 14.4, but 160 x 4096 (128) 9.6 / 8.8, 300 x 2408 (160)
+  // 12.3 / 11.2, 768 x 8192 (768) 91 / 68.
+  const int64_t tiles = ((m + 255) / 256) * ((n + 255) / 256) * batch;
+  return batched_product(g, m > 128 && tiles > 100, static_cast<hipStream_t>(stream));
 }
 
 // --------------------------------------------------- windowed (atom) cross-attention

@@ -408,7 +408,7 @@ static int mid_tile_choice(const GemmArgs& g) {
 int gemm_big_tile_choice(const GemmArgs& g) {
   constexpr int64_t BIG_TILE_MIN_TILES = 120;
   const int64_t tiles = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256) * g.batch;
-  if (mid_tile_choice(g) != MID_NONE) return -1;
+  if (g.small_tiles || mid_tile_choice(g) != MID_NONE) return -1;
   return g.M > 128 && g.N > 128 && tiles >= BIG_TILE_MIN_TILES ? big_tile_mode(g) : -1;
 }
 

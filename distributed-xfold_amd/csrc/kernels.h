@@ -33,6 +33,7 @@ struct GemmArgs {
   int regroup32 = 0;
   const bf16_t* w2 = nullptr;  // launch_outer_mean only
   int xcd_m = 0;               // set by the launchers: XcdWalk::rows
+  int small_tiles = 0;  // never the 256x256 tile (same sums, same order)
   int split_k = 0;  // the K range may be summed in parts by several waves (another order of summation)
 };
 int launch_gemm_nt(const GemmArgs& g, hipStream_t stream);
