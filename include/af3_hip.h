@@ -48,8 +48,11 @@ typedef void* af3_stream_t; /* a hipStream_t */
  * an existing entry point changes, so a caller that packed operands for another
  * version can tell.  2: af3_grid_attention_core_forward takes no gate and
  * leaves the normalised, ungated output; its pair bias is fp16 in fragment
- * order and vt has its quads swapped (version 1 took a bf16 bias and a gate). */
-#define AF3_ABI_VERSION 2
+ * order and vt has its quads swapped (version 1 took a bf16 bias and a gate).
+ * 3: af3_pairformer_block (so af3_msa_block, which holds one, too) has pair_frags
+ * and pair_channels, af3_diffusion_block has frags.  A caller of version 2 passes
+ * shorter structures, from which this library would take other fields. */
+#define AF3_ABI_VERSION 3
 int af3_abi_version(void);
 const char* af3_error_string(int code);
 
@@ -503,7 +506,8 @@ int af3_pair_cond_init_forward(const void* pair, int pair_dtype, float in_scale,
  * and single [n,c_single] are updated in place.  pair_mask [n,n] or NULL; pair_mask_incoming, when not
  * NULL, replaces it for the incoming triangle multiplication (the Evoformer block
  * transposes it, nn/d_pairformer.py:217); seq_mask [n] or NULL.
- * with_single = 0 in a block leaves `single` alone.
+ * with_single = 0 in a block leaves `single` alone.  Every field is read but the single
+ * track's of such a block: pair_frags and pair_channels that are not used are NULL and 0.
  * single_stream: NULL, or a second stream on which the updates of `single` run
  * beside the pair operators of the next block (they meet only in the pair
  * logits).  The call makes single_stream wait for what `stream` holds on entry,

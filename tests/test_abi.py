@@ -5,6 +5,7 @@ host-side weight packing / module plumbing behaves (no GPU compute)."""
 import ctypes
 import os
 import re
+import zlib
 
 import pytest
 import torch
@@ -57,11 +58,60 @@ def test_ctypes_table_matches_header(pkg):
 def test_error_strings_and_version(pkg):
     lib = pkg.lib.load()
     # the library reports the version its header declares
-    assert lib.af3_abi_version() == header_abi_version() == 2
+    assert lib.af3_abi_version() == header_abi_version() == pkg.lib.ABI_VERSION == 3
     assert lib.af3_error_string(0) == b"ok"
     assert b"workspace" in lib.af3_error_string(-2)
     with pytest.raises(pkg.lib.Af3Error):
         pkg.lib.check(-1, "x")
+
+
+def header_structures():
+    """The structures of the header as ctypes classes, by name."""
+    text = re.sub(r"/\*.*?\*/", "", open(HEADER).read(), flags=re.S)
+    made = {}
+    for name, body in re.findall(r"typedef struct (\w+) \{(.*?)\} \1;", text, flags=re.S):
+        fields = []
+        for declaration in filter(None, map(str.strip, body.split(";"))):
+            base, names = re.match(r"(?:const\s+)?(\w+)\s*(.*)", declaration, re.S).groups()
+            for one in names.split(","):
+                star, field, count = re.match(r"\s*(\*?)\s*(\w+)(?:\[(\d+)\])?\s*$", one).groups()
+                kind = ctypes.c_void_p if star else {"int32_t": ctypes.c_int32, "float": ctypes.c_float, **made}[base]
+                fields.append((field, kind * int(count) if count else kind))
+        made[name] = type(name, (ctypes.Structure,), {"_fields_": fields})
+    return made
+
+
+def layout(structure):
+    return [(name, getattr(structure, name).offset, getattr(structure, name).size) for name, *_ in structure._fields_]
+
+
+# size of each structure and a checksum of its fields' names and places, for every version of the interface that has had
+# structures: a changed layout is a new version
+STRUCTURES = {
+    2: {"af3_pairformer_block": (352, 1444406801), "af3_msa_block": (496, 3613447587), "af3_diffusion_block": (48, 2401195420)},
+    3: {"af3_pairformer_block": (360, 1619487416), "af3_msa_block": (504, 2391246903), "af3_diffusion_block": (56, 874399464)},
+}
+
+
+def test_layout_of_the_structures_belongs_to_the_interface_version():
+    def fingerprint(structure):
+        places = " ".join(f"{name}@{offset}" for name, offset, _ in layout(structure))
+        return ctypes.sizeof(structure), zlib.crc32(places.encode())
+    assert {name: fingerprint(s) for name, s in header_structures().items()} == STRUCTURES[header_abi_version()]
+
+
+def test_ctypes_structures_match_the_header(pkg):
+    L, made = pkg.lib, header_structures()
+    for ours, name in ((L.PairformerBlockStruct, "af3_pairformer_block"), (L.MsaBlockStruct, "af3_msa_block"),
+                       (L.DiffusionBlockStruct, "af3_diffusion_block")):
+        assert layout(ours) == layout(made[name]) and ctypes.sizeof(ours) == ctypes.sizeof(made[name])
+
+
+def test_a_library_of_another_interface_version_is_refused(pkg, monkeypatch):
+    monkeypatch.setattr(pkg.lib, "_lib", None)
+    monkeypatch.setattr(pkg.lib, "ABI_VERSION", header_abi_version() - 1)
+    with pytest.raises(pkg.lib.Af3Error, match="interface version"):
+        pkg.lib.load()
 
 
 def test_workspace_queries(pkg):
