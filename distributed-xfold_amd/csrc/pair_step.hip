@@ -89,6 +89,7 @@ __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(Pai
   constexpr int C = CH, D = C / H, LDX = C + 8, LDS_F = C + 4;
   constexpr int WAVES = C / 32, NT = 2 * C, CHUNKS = C / 8, KS = C / 16;
   constexpr int HIDDEN_CHUNK = hidden_chunk_of(C), MAX_HIDDEN = HIDDEN_CHUNK * hidden_chunks(C);
+  static_assert(PB == 1 || !TRANSITION, "a transition's fragments and sums fit the registers at 32 positions only");
   constexpr int NB = C == 64 || (PB == 1 && !TRANSITION) ? 4 : 3;  // pieces of the weights in flight
   constexpr int LDT = TS + 2;           // LDS row stride (bf16) of a channel's positions: the 16 lanes of a pixel, 8 channels apart, on 8 banks
   constexpr int LDH = HIDDEN_CHUNK + 8;
@@ -239,8 +240,7 @@ __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(Pai
       for (int ks = 0; ks < KS; ++ks) xf[b][ks] = lds_frag(s, LDX, 32 * b, ks * 16, lane);
   };
   // octet n (32 rows) x the tile: T form (a lane owns a position), D form (a lane owns a channel)
-  // (`tile`: its fragments come out of LDS one by one, where there are no registers to hold them)
-  auto product = [&](auto n_c, auto d_form, f32x16* acc, const bf16_t* tile = nullptr) {
+  auto product = [&](auto n_c, auto d_form, f32x16* acc) {
     constexpr int n = decltype(n_c)::value;
     const bf16x8* const wn = w[n % NB];
 #pragma unroll
@@ -250,10 +250,8 @@ __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(Pai
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int b = 0; b < PB; ++b) {
-        const bf16x8 x = tile ? lds_frag(tile, LDX, 32 * b, ks * 16, lane) : xf[b][ks];
-        acc[b] = decltype(d_form)::value ? mfma32(x, wn[ks], acc[b]) : mfma32(wn[ks], x, acc[b]);
-      }
+      for (int b = 0; b < PB; ++b)
+        acc[b] = decltype(d_form)::value ? mfma32(xf[b][ks], wn[ks], acc[b]) : mfma32(wn[ks], xf[b][ks], acc[b]);
     fetch(OCTET(n + NB));
   };
   auto sum_channels = [](float v) {
@@ -369,8 +367,7 @@ __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(Pai
   if constexpr (TRANSITION) {
     norm(1, sA);
     lds_barrier();  // (also: the staged results have been read, the hidden layer may take their place)
-    const bf16_t* const tile = PB == 2 ? sA : nullptr;
-    if constexpr (PB == 1) frags_of(sA);
+    frags_of(sA);
     f32x16 sum[PB];
 #pragma unroll
     for (int b = 0; b < PB; ++b)
@@ -382,8 +379,8 @@ __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(Pai
       auto block = [&](auto i_c) {
         constexpr int i = decltype(i_c)::value;
         f32x16 y[PB];
-        product(OCTET(n0 + 2 * i), T_form{}, acc, tile);
-        product(OCTET(n0 + 2 * i + 1), T_form{}, y, tile);
+        product(OCTET(n0 + 2 * i), T_form{}, acc);
+        product(OCTET(n0 + 2 * i + 1), T_form{}, y);
         if (c * (HIDDEN_CHUNK / 32) + wave + WAVES * i < n_hidden) {
 #pragma unroll
           for (int b = 0; b < PB; ++b)
@@ -562,7 +559,6 @@ __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(Pai
 }
 
 bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
-
 
 // Patches of 8 x 8 pixels from one workgroup per CU on: what a patch writes of a transposed operand is then whole 16-byte
 // pieces.
