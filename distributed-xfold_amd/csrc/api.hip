@@ -782,22 +782,22 @@ int run_gathered_attention(const bf16_t* q_data, const bf16_t* atom_data, const 
   hipStream_t s = stream;
 
   if (q_data) {
-  GemmArgs g;
-  g.A = q_data; g.B = w_qg; g.C = qg;
-  g.M = (int)(batch * sq); g.N = 2 * channels; g.K = channels;
-  g.lda = channels; g.ldb = channels; g.ldc = 2 * channels;
-  g.epi = EPI_SEGMENTED; g.seg_len = channels;
-  g.seg_ops = SEG_BIAS_SCALE | (SEG_SIGMOID << 4);
-  g.alpha = 1.0f / sqrtf((float)d);
-  g.bias = query_b; g.bias_len = channels;  // the query segment's columns only
-  int rc = launch_gemm_nt(g, s);
-  if (rc) return rc;
-  GemmArgs g2;
-  g2.A = atom_data; g2.B = w_kv; g2.C = kv;
-  g2.M = (int)(samples * n_atoms); g2.N = 2 * channels; g2.K = channels;
-  g2.lda = channels; g2.ldb = channels; g2.ldc = 2 * channels;
-  rc = launch_gemm_nt(g2, s);
-  if (rc) return rc;
+    GemmArgs g;
+    g.A = q_data; g.B = w_qg; g.C = qg;
+    g.M = (int)(batch * sq); g.N = 2 * channels; g.K = channels;
+    g.lda = channels; g.ldb = channels; g.ldc = 2 * channels;
+    g.epi = EPI_SEGMENTED; g.seg_len = channels;
+    g.seg_ops = SEG_BIAS_SCALE | (SEG_SIGMOID << 4);
+    g.alpha = 1.0f / sqrtf((float)d);
+    g.bias = query_b; g.bias_len = channels;  // the query segment's columns only
+    int rc = launch_gemm_nt(g, s);
+    if (rc) return rc;
+    GemmArgs g2;
+    g2.A = atom_data; g2.B = w_kv; g2.C = kv;
+    g2.M = (int)(samples * n_atoms); g2.N = 2 * channels; g2.K = channels;
+    g2.lda = channels; g2.ldb = channels; g2.ldc = 2 * channels;
+    rc = launch_gemm_nt(g2, s);
+    if (rc) return rc;
   }
 
   FlashArgs f;

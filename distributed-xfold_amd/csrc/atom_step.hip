@@ -177,62 +177,62 @@ __global__ __launch_bounds__(256, 2) void atom_step_kernel(AtomStepArgs a) {
   f32x4 cond_k[2][4];
 
   if constexpr (TAIL) {
-  // ---- output projection ----
+    // ---- output projection ----
 #pragma unroll
-  for (int u = 0; u < 2; ++u) *reinterpret_cast<u32x4*>(sA + (prow + 16 * u) * LDX + chunk * 8) = yv[u];
-  lds_barrier();
-  frags_of(sA);
-  f32x16 second;
-  product(PIECE(0), acc);
-  load_cond(a.scale, a.ld_cond, cond);
-  add_to_stream(acc);  // (its barrier: every wave has read the attention's tile)
+    for (int u = 0; u < 2; ++u) *reinterpret_cast<u32x4*>(sA + (prow + 16 * u) * LDX + chunk * 8) = yv[u];
+    lds_barrier();
+    frags_of(sA);
+    f32x16 second;
+    product(PIECE(0), acc);
+    load_cond(a.scale, a.ld_cond, cond);
+    add_to_stream(acc);  // (its barrier: every wave has read the attention's tile)
 
-  // ---- transition ----
-  norm(cond, sA, nullptr, nullptr);
-  load_gate(a.gate2);
-  lds_barrier();  // (also: the staged results have been read, the hidden layer may take their place)
+    // ---- transition ----
+    norm(cond, sA, nullptr, nullptr);
+    load_gate(a.gate2);
+    lds_barrier();  // (also: the staged results have been read, the hidden layer may take their place)
 
-  frags_of(sA);
-  auto block = [&](auto i_c) {
-    constexpr int i = decltype(i_c)::value;
-    product(PIECE(1 + 2 * i), acc);
-    product(PIECE(2 + 2 * i), second);
-    if (wave + 4 * i < n_hidden) {
+    frags_of(sA);
+    auto block = [&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      product(PIECE(1 + 2 * i), acc);
+      product(PIECE(2 + 2 * i), second);
+      if (wave + 4 * i < n_hidden) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        float h[4];
+        for (int g = 0; g < 4; ++g) {
+          float h[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = acc[4 * g + e] * sigmoidf_(acc[4 * g + e]) * second[4 * g + e];
-        u32x2 v;
-        v.x = pack2bf(h[0], h[1]);
-        v.y = pack2bf(h[2], h[3]);
-        *reinterpret_cast<u32x2*>(sH + j * LDH + (wave + 4 * i) * 32 + 8 * g + 4 * hh) = v;
+          for (int e = 0; e < 4; ++e) h[e] = acc[4 * g + e] * sigmoidf_(acc[4 * g + e]) * second[4 * g + e];
+          u32x2 v;
+          v.x = pack2bf(h[0], h[1]);
+          v.y = pack2bf(h[2], h[3]);
+          *reinterpret_cast<u32x2*>(sH + j * LDH + (wave + 4 * i) * 32 + 8 * g + 4 * hh) = v;
+        }
       }
+    };
+    block(std::integral_constant<int, 0>{});
+    block(std::integral_constant<int, 1>{});
+    lds_barrier();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    auto half = [&](auto h_c) {
+      constexpr int h = decltype(h_c)::value;
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (8 * h + k < nks) acc = mfma32(w[(5 + h) % NB][k], lds_frag(sH, LDH, 0, (8 * h + k) * 16, lane), acc);
+      fetch(PIECE(5 + h + NB));
+    };
+    half(std::integral_constant<int, 0>{});
+    half(std::integral_constant<int, 1>{});
+    if constexpr (HEAD) {
+      load_cond(a.scale_q, a.ld_cond, cond);
+      load_cond(a.scale_k, a.ld_cond_k, cond_k);
     }
-  };
-  block(std::integral_constant<int, 0>{});
-  block(std::integral_constant<int, 1>{});
-  lds_barrier();
+    lds_barrier();  // every wave is done with the hidden layer
+    add_to_stream(acc);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  auto half = [&](auto h_c) {
-    constexpr int h = decltype(h_c)::value;
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (8 * h + k < nks) acc = mfma32(w[(5 + h) % NB][k], lds_frag(sH, LDH, 0, (8 * h + k) * 16, lane), acc);
-    fetch(PIECE(5 + h + NB));
-  };
-  half(std::integral_constant<int, 0>{});
-  half(std::integral_constant<int, 1>{});
-  if constexpr (HEAD) {
-    load_cond(a.scale_q, a.ld_cond, cond);
-    load_cond(a.scale_k, a.ld_cond_k, cond_k);
-  }
-  lds_barrier();  // every wave is done with the hidden layer
-  add_to_stream(acc);
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
-    if (ok[u]) store_raw<TIO>(act + (int64_t)atom[u] * C + chunk * 8, raw[u]);
+    for (int u = 0; u < 2; ++u)
+      if (ok[u]) store_raw<TIO>(act + (int64_t)atom[u] * C + chunk * 8, raw[u]);
   }
 
   // ---- the next attention's operands ----

@@ -144,7 +144,8 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
   // two slab buffers and the waves' output staging areas
   __shared__ __attribute__((aligned(1024))) char smem[2 * SLAB];
   __shared__ __attribute__((aligned(16))) char sOut[MODE == BIG_OUTER_MEAN ? 16 : 4 * EPI_BYTES];
-  __shared__ __attribute__((aligned(16))) float sColBias[MODE == BIG_COLUMN_OPS ? 4 * 128 : MODE == BIG_OUTER_MEAN ? 128 : 4];  // (a wave's) 128 bias values
+  // (a wave's) 128 bias values
+  __shared__ __attribute__((aligned(16))) float sColBias[MODE == BIG_COLUMN_OPS ? 4 * 128 : MODE == BIG_OUTER_MEAN ? 128 : 4];
 
   const int tid = threadIdx.x, lane = tid & 63;
   if (MODE == BIG_OUTER_MEAN && tid < 128) sColBias[tid] = g.bias[tid];  // (read behind many barriers)

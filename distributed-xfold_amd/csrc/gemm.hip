@@ -65,8 +65,8 @@ __device__ __forceinline__ void wait_loads_but() {
 }
 
 // A workgroup of WM x WN x WK waves computes BM = 32 MT WM rows x BN = 32 NT WN columns; ST slab buffers per group.
-// CLEAN: K is a multiple of the slab depth.  KIND: the epilogue.  VEC: all of its loads and stores are 16-byte ones (without: element by element, for odd column
-// counts and unaligned operands).  WPS: waves per SIMD the tile's LDS leaves room for; the
+// CLEAN: K is a multiple of the slab depth.  KIND: the epilogue.  VEC: all of its loads and stores are 16-byte ones (without:
+// element by element, for odd column counts and unaligned operands).  WPS: waves per SIMD the tile's LDS leaves room for; the
 // registers have to as well (a wave more or less per SIMD is up to a factor of two in the short products).
 enum { KIND_COLUMNS = 0, KIND_GATE_RES = 1, KIND_SWIGLU = 2 };
 template <int MT, int NT, int WM, int WN, int WK, int ST, int WPS, bool CLEAN, int KIND, bool VEC, bool OUT_F32>

@@ -91,7 +91,8 @@ __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(Pai
   constexpr int HIDDEN_CHUNK = hidden_chunk_of(C), MAX_HIDDEN = HIDDEN_CHUNK * hidden_chunks(C);
   static_assert(PB == 1 || !TRANSITION, "a transition's fragments and sums fit the registers at 32 positions only");
   constexpr int NB = C == 64 || (PB == 1 && !TRANSITION) ? 4 : 3;  // pieces of the weights in flight
-  constexpr int LDT = TS + 2;           // LDS row stride (bf16) of a channel's positions: the 16 lanes of a pixel, 8 channels apart, on 8 banks
+  // LDS row stride (bf16) of a channel's positions: the 16 lanes of a pixel, 8 channels apart, on 8 banks
+  constexpr int LDT = TS + 2;
   constexpr int LDH = HIDDEN_CHUNK + 8;
   constexpr int U_BYTES = TS * LDS_F * 4;
   static_assert(U_BYTES >= C * LDT * 2 && U_BYTES >= TS * LDH * 2, "what takes turns in the staging tile fits");
@@ -299,68 +300,68 @@ __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(Pai
   f32x16 acc[PB];
   // ---- gate and output projection of the operator before ----
   if constexpr (IN != IN_NONE) {
-  norm(0, sA);
-  if constexpr (IN == IN_EPILOGUE) {
+    norm(0, sA);
+    if constexpr (IN == IN_EPILOGUE) {
 #pragma unroll
-    for (int u = 0; u < 2 * PB; ++u) {
-      const int idx = tid + NT * u;
-      uint32_t* const d = reinterpret_cast<uint32_t*>(sT + idx / (4 * PB) * LDT + idx % (4 * PB) * 8);
-      d[0] = tt[u].x; d[1] = tt[u].y; d[2] = tt[u].z; d[3] = tt[u].w;
-    }
-  }
-  lds_barrier();
-  frags_of(sA);
-  f32x16 gate[PB];
-  product(OCTET(0), T_form{}, gate);
-  if constexpr (IN == IN_EPILOGUE) {
-    // LayerNorm of the contraction's result over its channels
-    float lw[8], lb[8];
-    load_param8(sP + 2 * C + chunk * 8, 1.f, lw);
-    load_param8(sP + 3 * C + chunk * 8, 0.f, lb);
-#pragma unroll
-    for (int u = 0; u < 2 * PB; ++u) {
-      const int p = prow + 16 * u, pos = t.position(p);
-      float v[8], o[8], s1 = 0.f, s2 = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        v[e] = bf2f(sT[(chunk * 8 + e) * LDT + pos]);
-        s1 += v[e];
+      for (int u = 0; u < 2 * PB; ++u) {
+        const int idx = tid + NT * u;
+        uint32_t* const d = reinterpret_cast<uint32_t*>(sT + idx / (4 * PB) * LDT + idx % (4 * PB) * 8);
+        d[0] = tt[u].x; d[1] = tt[u].y; d[2] = tt[u].z; d[3] = tt[u].w;
       }
-      const float mean = sum_channels(s1) * a.lw.inv_c;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) { const float d = v[e] - mean; s2 = fmaf(d, d, s2); }
-      const float rstd = rsqrtf((sum_channels(s2) - a.lw.pad * mean * mean) * a.lw.inv_c + LN_EPS);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = mine[u].ok ? (v[e] - mean) * rstd * lw[e] + lb[e] : 0.f;
-      *reinterpret_cast<u32x4*>(sB + p * LDX + chunk * 8) = pack8(o);
     }
+    lds_barrier();
+    frags_of(sA);
+    f32x16 gate[PB];
+    product(OCTET(0), T_form{}, gate);
+    if constexpr (IN == IN_EPILOGUE) {
+      // LayerNorm of the contraction's result over its channels
+      float lw[8], lb[8];
+      load_param8(sP + 2 * C + chunk * 8, 1.f, lw);
+      load_param8(sP + 3 * C + chunk * 8, 0.f, lb);
 #pragma unroll
-    for (int b = 0; b < PB; ++b)
+      for (int u = 0; u < 2 * PB; ++u) {
+        const int p = prow + 16 * u, pos = t.position(p);
+        float v[8], o[8], s1 = 0.f, s2 = 0.f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) gate[b][r] = sigmoidf_(gate[b][r]);
-  } else {
-    // gated attention output: the lane's registers 8 u .. are channels 32 wave + 16 u + 8 hh .. of its position
+        for (int e = 0; e < 8; ++e) {
+          v[e] = bf2f(sT[(chunk * 8 + e) * LDT + pos]);
+          s1 += v[e];
+        }
+        const float mean = sum_channels(s1) * a.lw.inv_c;
 #pragma unroll
-    for (int b = 0; b < PB; ++b)
+        for (int e = 0; e < 8; ++e) { const float d = v[e] - mean; s2 = fmaf(d, d, s2); }
+        const float rstd = rsqrtf((sum_channels(s2) - a.lw.pad * mean * mean) * a.lw.inv_c + LN_EPS);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        float f[8];
-        unpack8(og[b][u], f);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] *= sigmoidf_(gate[b][8 * u + e]);
-        *reinterpret_cast<u32x4*>(sB + (32 * b + j) * LDX + wave * 32 + 16 * u + 8 * hh) = own[b].ok ? pack8(f) : u32x4{0u, 0u, 0u, 0u};
+        for (int e = 0; e < 8; ++e) o[e] = mine[u].ok ? (v[e] - mean) * rstd * lw[e] + lb[e] : 0.f;
+        *reinterpret_cast<u32x4*>(sB + p * LDX + chunk * 8) = pack8(o);
       }
-  }
-  lds_barrier();
-  frags_of(sB);
-  product(OCTET(1), T_form{}, acc);
-  if constexpr (IN == IN_EPILOGUE) {
 #pragma unroll
-    for (int b = 0; b < PB; ++b)
+      for (int b = 0; b < PB; ++b)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[b][r] *= gate[b][r];
-  }
-  add_to_stream(acc);  // (sT was last read in front of the barrier above)
+        for (int r = 0; r < 16; ++r) gate[b][r] = sigmoidf_(gate[b][r]);
+    } else {
+      // gated attention output: the lane's registers 8 u .. are channels 32 wave + 16 u + 8 hh .. of its position
+#pragma unroll
+      for (int b = 0; b < PB; ++b)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          float f[8];
+          unpack8(og[b][u], f);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[e] *= sigmoidf_(gate[b][8 * u + e]);
+          *reinterpret_cast<u32x4*>(sB + (32 * b + j) * LDX + wave * 32 + 16 * u + 8 * hh) = own[b].ok ? pack8(f) : u32x4{0u, 0u, 0u, 0u};
+        }
+    }
+    lds_barrier();
+    frags_of(sB);
+    product(OCTET(1), T_form{}, acc);
+    if constexpr (IN == IN_EPILOGUE) {
+#pragma unroll
+      for (int b = 0; b < PB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[b][r] *= gate[b][r];
+    }
+    add_to_stream(acc);  // (sT was last read in front of the barrier above)
   }
 
   // ---- transition, a chunk of the hidden layer at a time ----
@@ -419,8 +420,8 @@ __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(Pai
   }
   if constexpr (IN != IN_NONE)
 #pragma unroll
-  for (int u = 0; u < 2 * PB; ++u)
-    if (mine[u].ok) store_raw<TIO>(at32(pair, t.pix(mine[u]) * C + chunk * 8), raw[u]);
+    for (int u = 0; u < 2 * PB; ++u)
+      if (mine[u].ok) store_raw<TIO>(at32(pair, t.pix(mine[u]) * C + chunk * 8), raw[u]);
   asm volatile("" ::"v"(warm));
   if constexpr (NEXT == NEXT_NONE)
     if (C != 128 || !a.logits) return;
@@ -569,7 +570,8 @@ constexpr int64_t WIDE_ROWS = 208 * 208 + 1;
 
 template <int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT>
 int launch_tiles(const PairStepArgs& a, hipStream_t s) {
-  const int64_t blocks = MAP == MAP_PATCH ? ((int64_t)(a.Np / (4 * PB)) * (a.Np / 8) + 7) / 8 * 8 : ((int64_t)a.N * a.ldn + 32 * PB - 1) / (32 * PB);
+  const int64_t blocks = MAP == MAP_PATCH ? ((int64_t)(a.Np / (4 * PB)) * (a.Np / 8) + 7) / 8 * 8
+                                          : ((int64_t)a.N * a.ldn + 32 * PB - 1) / (32 * PB);
   if (blocks <= 0 || blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
   const dim3 grid((unsigned)blocks), block(2 * CH);
   if (a.io_f32) hipLaunchKernelGGL((pair_step_kernel<float, CH, PB, IN, MAP, TRANSITION, NEXT>), grid, block, 0, s, a);
@@ -583,7 +585,8 @@ int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s) {
       (a.channels != 128 && a.channels != 64) || a.valid_c < 1 || a.valid_c > a.channels)
     return AF3_ERR_BAD_ARG;
   // every array is addressed with 32 bits
-  if (a.plane * a.channels * 2 >= (1ll << 32) || (int64_t)a.N * a.ldn * a.channels * (a.io_f32 ? 4 : 2) >= (1ll << 32)) return AF3_ERR_BAD_ARG;
+  if (a.plane * a.channels * 2 >= (1ll << 32) || (int64_t)a.N * a.ldn * a.channels * (a.io_f32 ? 4 : 2) >= (1ll << 32))
+    return AF3_ERR_BAD_ARG;
   const bool first = step == PAIR_STEP_FIRST, epilogue = step == PAIR_STEP_INCOMING || step == PAIR_STEP_PROJECT_START;
   const bool prologue = first || step == PAIR_STEP_INCOMING || step == PAIR_STEP_NEXT;
   const bool project = step == PAIR_STEP_PROJECT_START || step == PAIR_STEP_PROJECT_END, transition = step >= PAIR_STEP_LAST;
@@ -592,9 +595,11 @@ int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s) {
   if (!epilogue && !first && !a.og) return AF3_ERR_BAD_ARG;
   if (prologue && (!a.a_buf || !a.b_buf || !a.f_next || !a.ln3_w || !a.ln3_b || a.plane < tri_plane(a.N))) return AF3_ERR_BAD_ARG;
   if (project && (!a.q || !a.k || !a.vt || !a.bias || !a.f_next || !a.f_v || !a.ln3_w || !a.ln3_b)) return AF3_ERR_BAD_ARG;
-  if (transition && (!a.f_w1 || !a.f_w2 || !a.ln2_w || !a.ln2_b || a.hidden <= 0 || (a.hidden & 63) || a.hidden > pair_step_max_hidden(a.channels)))
+  if (transition && (!a.f_w1 || !a.f_w2 || !a.ln2_w || !a.ln2_b || a.hidden <= 0 || (a.hidden & 63) ||
+                     a.hidden > pair_step_max_hidden(a.channels)))
     return AF3_ERR_BAD_ARG;
-  if (a.logits && (a.channels != 128 || !transition || !a.f_logits || !a.sl_ln_w || !a.sl_ln_b || a.logit_heads <= 0)) return AF3_ERR_BAD_ARG;
+  if (a.logits && (a.channels != 128 || !transition || !a.f_logits || !a.sl_ln_w || !a.sl_ln_b || a.logit_heads <= 0))
+    return AF3_ERR_BAD_ARG;
   if (a.channels == 64) switch (step) {
     case PAIR_STEP_FIRST: return launch_tiles<64, 1, IN_NONE, MAP_ROWS, false, NEXT_PROLOGUE>(a, s);
     case PAIR_STEP_INCOMING: return launch_tiles<64, 1, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);

@@ -541,8 +541,9 @@ typedef struct af3_pairformer_block {
   /* NULL, or the pair operators' matrices once more, for runs of operators in one kernel at few tokens: every matrix
    * W [rows][k] as [row / 32][column / 16][(column / 8) % 2][row % 32][column % 8], one after the other.  With bits 2
    * and 3 of the row number exchanged, for [0], [1]: q, k and the gate of ta_w_qkvg; then, for [0], [1]: tm_w_gating,
-   * tm_w_out, tm_w_proj_gate; for [0], [1]: v of ta_w_qkvg, ta_w_bias, ta_w_out; pt_w1; with_single sl_w; pt_w2.  pair_channels 64: without the padding, matrices of 64 columns and
-   * rows (ta_w_bias 32 rows, pt_w1 2 pair_hidden rows) and of tm_w_proj_gate the two groups that hold channels. */
+   * tm_w_out, tm_w_proj_gate; for [0], [1]: v of ta_w_qkvg, ta_w_bias, ta_w_out; pt_w1; with_single sl_w; pt_w2.
+   * pair_channels 64: without the padding, matrices of 64 columns and rows (ta_w_bias 32 rows, pt_w1 2 pair_hidden rows)
+   * and of tm_w_proj_gate the two groups that hold channels. */
   const uint16_t* pair_frags;
   int32_t valid_channels, num_head_pair, pair_hidden; /* pair_hidden: hidden units of the pair transition */
   int32_t with_single, num_head, c_single, single_hidden;
