@@ -81,8 +81,9 @@ def pair_of_64(att, transition, c_pair) -> bool:
 
 
 def takes_64(s, pair: torch.Tensor) -> bool:
-    """Whether a block whose structure is `s` may be given this [N, N, 64] tensor itself."""
-    return s.pair_channels == 64 and pair.shape[0] <= L.PAIR64_MAX_TOKENS and pair.data_ptr() % 16 == 0
+    """Whether a block whose structure is `s` takes this [N, N, 64] tensor as it is.  Its size decides and not its address:
+    the statistics of a LayerNorm over zero-padded channels are rounded otherwise, and move outputs by bf16 places."""
+    return s.pair_channels == 64 and pair.shape[0] <= L.PAIR64_MAX_TOKENS
 
 
 def padded_128(s) -> "L.PairformerBlockStruct":
@@ -210,6 +211,8 @@ class PairformerBlock(HipModule):
             s, x = self.native(), pair
             if self.c_pair < 128 and not takes_64(s, pair):
                 s, x = padded_128(s), pad_channels(pair)
+            elif self.c_pair < 128 and pair.data_ptr() % 16:     # the kernels' loads are of 16 bytes
+                x = pair.clone()
             ops.pairformer_stack([s], x, pair_mask, None, None)
             if x is not pair:
                 pair.copy_(x[..., :self.c_pair])

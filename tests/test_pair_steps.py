@@ -110,6 +110,20 @@ def test_64_channels_that_are_padded_after_all(gpu_pkg):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("io", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [9, 150])
+def test_64_channels_at_any_address(gpu_pkg, n, io):
+    """The bits do not depend on where the tensor begins."""
+    blk, (pair, mask, _, _) = _block(gpu_pkg, 64, 2, n), _inputs(n, 64, io, 2)
+    want = blk(pair.clone(), mask)
+    store = torch.full((pair.numel() + 5,), 7.0, dtype=io, device="cuda")
+    odd = store[3:-2].view(pair.shape).copy_(pair)
+    got = blk(odd, mask)
+    assert want.data_ptr() % 16 == 0 and odd.data_ptr() % 16 and got.data_ptr() == odd.data_ptr() and torch.equal(got, want)
+    assert (store[:3] == 7.0).all() and (store[-2:] == 7.0).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,count", [(5, 3), (48, 19), (130, 10)])
 def test_a_run_of_blocks_is_its_blocks_one_by_one(gpu_pkg, n, count):
     """The last step of a block makes the next block's first operands, and the buffers of the pair logits come round again
