@@ -276,7 +276,7 @@ def evoformer_block_ms(pkg, n, dev, rows=1024, iters=10):
 
 def template_block_ms(pkg, n, dev, iters=10):
     """The Pairformer block of the template embedding (nn/d_template.py:198-201): 64 pair channels, transition
-    factor 2, no single track.  It runs on the 128-channel kernels over zero-padded operands."""
+    factor 2, no single track.  It runs on kernels for 64 channels, on the tensor itself."""
     import torch
     g = torch.Generator().manual_seed(5)
     blk = random_init_(pkg.nn.PairformerBlock(c_pair=64, num_intermediate_factor=2, with_single=False), g).to(dev)
@@ -286,7 +286,7 @@ def template_block_ms(pkg, n, dev, iters=10):
     pm = (seq[:, None] * seq[None, :]).contiguous()
     ms = gpu_time_ms(lambda: blk(pair, pm), iters, warm_ms=40.0)
     return {"workload": f"one Pairformer block on 64 pair channels (template embedding), N_token={n}, bf16, "
-                        "10% trailing tokens masked, padded to the 128-channel kernels",
+                        "10% trailing tokens masked, kernels for 64 channels on the tensor itself",
             "ms_per_block": round(ms, 3)}
 
 

@@ -1,7 +1,8 @@
-// Whole-module entry points: the launches of a run of blocks, enqueued in one call.  Host code only; every step is
-// one of the library's own entry points with the same arguments a caller would give it.
+// Whole-module entry points: the launches of a run of blocks, enqueued in one call.  Host code only; a step is one of the
+// library's own entry points with the arguments a caller would give it, or one kernel for several of them (pair_step.hip,
+// atom_step.hip, the Evoformer's msa.hip).
 //
-// Why it exists: a launch costs about 3.7 us of host time from C (measured, back to back), and about 11 us through
+// Why it exists: a launch costs 2.7 to 3.7 us of host time from C (by machine, back to back), and about 11 us through
 // the Python operator layer (argument checks, tensor allocation, ctypes).  Up to a few hundred tokens the kernels
 // themselves take 4 to 10 us, so that the operator layer, not the GPU, set the pace of a block.
 #include "../../include/af3_hip.h"
@@ -54,17 +55,27 @@ struct Event {
 
 // ---- the pair operators at few tokens: a run of them between two long products in one kernel (pair_step.hip) ----
 // A step takes the chain of one tile of 32 positions where a kernel of its own per operator takes several of tiles of 128,
-// and eight launches a block take the place of fourteen; past some number of tiles what every tile fetches of the weights
-// costs more than that saves.  Runs of 4 blocks, us a block, one kernel per operator -> steps (bf16 / fp32 stream):
-//   64 tokens 136 -> 85 / 143 -> 88,  128: 166 -> 121 / 173 -> 121,  160: 205 -> 179 / 213 -> 182,
-//   208: 286 -> 268 / 306 -> 279,  224: 265 -> 264 / 283 -> 275,  256: 287 -> 288 / 323 -> 302
+// and eight launches a block take the place of thirteen; past some number of tiles what every tile fetches of the weights
+// costs more than that saves.  All three forms in turn, us a block: one kernel per operator / steps in part (below) / steps
+// throughout, in runs of 4 blocks on a bf16 and on an fp32 stream, and a single Evoformer block of 64 rows (bf16; its last
+// step makes no prologue for a next block):
+//    64 tokens  135 / 116 /  92    143 / 121 /  92    154 / 137 / 119
+//   128         164 / 148 / 121    169 / 151 / 120    199 / 184 / 168
+//   160         194 / 180 / 166    202 / 188 / 169    237 / 226 / 216
+//   192         236 / 219 / 202    250 / 233 / 211    287 / 271 / 264
+//   208         256 / 244 / 235    272 / 258 / 246    315 / 305 / 302
+//   224         265 / 256 / 252    286 / 274 / 264    324 / 315 / 319
+//   240         273 / 262 / 267    297 / 285 / 282    330 / 323 / 330
+// The line lies below the first size at which steps throughout are not the fastest form in every one of these (216 tokens, the
+// same number of tiles to a row as 224: still by 1 to 5 %).
 // Pair tensors of 64 channels have no other kernels (64 / 301 / 768 / 2048 tokens, bf16, a block on its own: 100 -> 46,
 // 345 -> 221, 1940 -> 1460, 22400 -> 18800 against one zero-padded to 128; their 32-bit offsets end at 3072).
 constexpr int64_t PAIR_STEP_POSITIONS = 208 * 208;
 // Beyond, the two steps that end in an attention's projections stay the faster form for a while (they only read the tensor's
 // rows as they lie, and half of a tile's weights): runs of 4 blocks, us a block, without -> with them (bf16 / fp32 stream),
-// 209 tokens 251 -> 239 / 267 -> 253, 301: 393 -> 385 / 448 -> 428, 387: 640 -> 630 / 732 -> 703, 420: 714 -> 708 /
-// 829 -> 810, 450: 830 -> 835 / 982 -> 966.
+// 209 tokens 250 -> 239 / 267 -> 253, 301: 391 -> 384 / 442 -> 423, 340: 492 -> 481 / 561 -> 538, 400: 659 -> 644 /
+// 763 -> 734.  Past the line the gain gets smaller and depends on the machine: 420: 712 -> 699 or 714 -> 708, 450: 814 -> 805 or
+// 830 -> 835 on a bf16 stream.
 constexpr int64_t PROJECT_STEP_POSITIONS = 400 * 400;
 bool pair_steps_apply(const af3_pairformer_block& b, int64_t n, int64_t positions = PAIR_STEP_POSITIONS) {
   const int c = b.pair_channels == 64 ? 64 : 128;
@@ -84,11 +95,14 @@ struct PairStepScratch {
            (c == 128 && n * tri_ldn(n) <= PAIR_STEP_POSITIONS ? LOGIT_RING * logit_bytes(n, 16) : 0);
   }
   // Pair logits of the last blocks, where the single track runs on a stream of its own.  With two buffers every block waits
-  // for the attention two blocks back, and an event recorded and waited for costs the host 13 us, where a launch costs 3.5:
-  // at 64 tokens the launches set the pace.  With eight it is one wait in four blocks (runs of 4 blocks, us a block: 93 -> 83).
+  // for the attention two blocks back, and an event costs the host some 20 us (recorded 3, waited for 15 to 17), where a launch
+  // costs 2.7 to 3.7: at 64 tokens the launches set the pace.  With eight it is one wait in four blocks (runs of 4 blocks, us a
+  // block: 93 -> 83).
   static constexpr int LOGIT_RING = 8;
   static size_t logit_bytes(int64_t n, int heads) { return align_up((size_t)heads * n * ((n + 3) / 4 * 4) * 4); }
-  float* ring(int64_t n) const { return reinterpret_cast<float*>(reinterpret_cast<char*>(bias) + align_up((size_t)tri_bias_elems(n, 4) * 2)); }
+  float* ring(int64_t n) const {
+    return reinterpret_cast<float*>(reinterpret_cast<char*>(bias) + align_up((size_t)tri_bias_elems(n, 4) * 2));
+  }
   bool carve(int64_t n, int c, void* ws, size_t wsb) {
     Carver w(ws, wsb);
     qa = static_cast<bf16_t*>(w.take(plane_bytes(n, c)));
@@ -100,9 +114,9 @@ struct PairStepScratch {
   }
 };
 
-// One block's pair operators.  `partly`: in steps only where an attention's projections are the second half.  `first`: no step before has made the outgoing prologue.  `next`: the block whose outgoing
-// prologue the last step makes, or null.  `logits`: where the pair logits of the single track go, or null; they are
-// written behind `logits_free`.
+// One block's pair operators.  `partly`: in steps only where an attention's projections are the second half.  `first`: no
+// step before has made the outgoing prologue.  `next`: the block whose outgoing prologue the last step makes, or null.
+// `logits`: where the pair logits of the single track go, or null; they are written behind `logits_free`.
 int pair_operators_in_steps(const af3_pairformer_block& b, bool partly, const af3_pairformer_block* next, bool first, void* pair, int dt,
                             const float* mask, const float* mask_in, int64_t n, void* ws, size_t wsb, float* logits,
                             Event* logits_free, hipStream_t s) {
@@ -358,8 +372,8 @@ int af3_evoformer_stack_forward(const af3_msa_block* const* blocks, int num_bloc
     msa_transition_args(b.mt_ln_w, b.mt_ln_b, b.mt_w1, b.mt_w2, b.mt_hidden, u);
     STEP(launch_msa_update(u, s));
     if (pair_steps_apply(b.pair, n))
-      STEP(pair_operators_in_steps(b.pair, false, nullptr, true, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace,
-                                   pair_workspace_bytes, nullptr, nullptr, s));
+      STEP(pair_operators_in_steps(b.pair, false, nullptr, true, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n,
+                                   pair_workspace, pair_workspace_bytes, nullptr, nullptr, s));
     else
       STEP(pair_operators(b.pair, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace,
                           pair_workspace_bytes, s));
@@ -394,7 +408,8 @@ int af3_pairformer_stack_forward(
     if (workspace_bytes < af3_pairformer_stack_workspace_bytes(n, b.num_head_pair)) return AF3_ERR_WORKSPACE;
     // (a pair tensor of 64 channels is what the step kernels alone take)
     if ((b.pair_channels != 0 && b.pair_channels != 128 && b.pair_channels != 64) ||
-        (b.pair_channels == 64) != (blocks[0]->pair_channels == 64) || (b.pair_channels == 64 && (!pair_steps_apply(b, n) || b.with_single)))
+        (b.pair_channels == 64) != (blocks[0]->pair_channels == 64) ||
+        (b.pair_channels == 64 && (!pair_steps_apply(b, n) || b.with_single)))
       return AF3_ERR_BAD_ARG;
     if (!b.with_single) continue;
     if (!single || !logits || b.num_head != blocks[0]->num_head || b.c_single != blocks[0]->c_single) return AF3_ERR_BAD_ARG;
@@ -526,8 +541,8 @@ size_t af3_atom_transformer_workspace_bytes(int64_t samples, int64_t subsets, in
 int af3_atom_transformer_forward(
     const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t samples, int64_t subsets,
     int64_t queries, int64_t keys, int channels, int hidden, int num_head, const int32_t* key_rows, const float* mask_q,
-    const float* mask_k, const float* pair_logits, int bias_quad_major, const float* scale_shift_q, const float* scale_shift_k, const float* gate,
-    void* workspace, size_t workspace_bytes, af3_stream_t stream) {
+    const float* mask_k, const float* pair_logits, int bias_quad_major, const float* scale_shift_q, const float* scale_shift_k,
+    const float* gate, void* workspace, size_t workspace_bytes, af3_stream_t stream) {
   if (!blocks || num_blocks <= 0 || !act || !key_rows || !scale_shift_q || !scale_shift_k || !gate || samples <= 0 ||
       subsets <= 0 || queries <= 0 || keys <= 0 || channels <= 0 || hidden <= 0 || num_head <= 0)
     return AF3_ERR_BAD_ARG;

@@ -556,8 +556,9 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
     for (int s = 0; s < 4; ++s) pp[s] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      // A zero that the compiler cannot see: of a known one it makes sixteen scalar registers, spills others to lanes for them
-      // (two rows: 79 lane moves a wave) and copies them from there.  Four blocks at 768 tokens 9337 -> 9319 us, 387 2465 -> 2459.
+      // A zero that the compiler cannot see: of a known one it makes sixteen scalar registers, since this is a template over the
+      // head dimension, spills others to lanes for them (two rows: 84 lane moves) and copies them from there.  Four blocks at
+      // 768 tokens 9337 -> 9319 us, 387 2465 -> 2459: what the template had cost, no more.
       float zero = 0.f;
       asm("" : "+v"(zero));
 #pragma unroll

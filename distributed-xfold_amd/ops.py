@@ -225,8 +225,8 @@ def transition128(act, layernorm_weight, layernorm_bias, w1_packed, w2, residual
 @_uses_scratch
 def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incoming=None, single_stream=None, join=True):
     """A run of Pairformer blocks in one call (af3_pairformer_stack_forward), pair [N, N, 128] (64 where the blocks'
-    pair_channels say so) and single [N, c] updated in place.  `blocks`: af3_pairformer_block structures (nn.PairformerBlock.native()); `single_stream`: a
-    torch stream for the single updates, see the entry point."""
+    pair_channels say so) and single [N, c] updated in place.  `blocks`: af3_pairformer_block structures
+    (nn.PairformerBlock.native()); `single_stream`: a torch stream for the single updates, see the entry point."""
     lib = _L.load()
     _gpu(pair, "pair")
     channels = blocks[0].pair_channels or 128
