@@ -97,7 +97,7 @@ def test_64_channels_far_from_zero(gpu_pkg, n):
 
 @pytest.mark.gpu
 def test_64_channels_that_are_padded_after_all(gpu_pkg):
-    """A tensor that does not begin on 16 bytes, and blocks the 64-channel kernels do not take."""
+    """Blocks the 64-channel kernels do not take; and a tensor that does not begin on 16 bytes, which is copied."""
     blk, (pair, mask, _, _) = _block(gpu_pkg, 64, 2, 5), _inputs(40, 64, torch.bfloat16, 3)
     want = blk(pair.clone(), mask)
     store = torch.empty(pair.numel() + 1, dtype=pair.dtype, device="cuda")
@@ -107,6 +107,16 @@ def test_64_channels_that_are_padded_after_all(gpu_pkg):
     wide = _block(gpu_pkg, 64, 4, 5)
     assert wide.native().pair_channels == 128
     assert torch.isfinite(wide(pair.clone(), mask)).all()
+
+
+@pytest.mark.gpu
+def test_64_channels_past_the_last_size_of_their_kernels(gpu_pkg, monkeypatch):
+    """Padded, by a structure of its own: the bits of the 128-channel kernels (the last size made small)."""
+    blk, inputs = _block(gpu_pkg, 64, 2, 5), _inputs(40, 64, torch.bfloat16, 3)
+    want = _run_general(blk, *inputs)[0]
+    assert not torch.equal(_run(blk, *inputs)[0], want)
+    monkeypatch.setattr(gpu_pkg.lib, "PAIR64_MAX_TOKENS", 39)
+    assert torch.equal(_run(blk, *inputs)[0], want) and blk.native().pair_channels == 64
 
 
 @pytest.mark.gpu
