@@ -361,6 +361,7 @@ struct TriAttnArgs {
   bf16_t* og = nullptr;          // [(b*N + s)][128] normalised attention output (the gate is applied by attn_out)
   int N = 0, head_dim = 32;      // head_dim 32 or 16: q, k [b][h][s][head_dim], vt [b][h][head_dim][ldn], og rows of 4 head_dim
   int64_t ldn = 0;
+  int tile_blocks = 0, tile_extra = 0;  // (launch_triattn_flash) blocks of 32 queries per query tile, and how many tiles have one more
 };
 int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream);
 

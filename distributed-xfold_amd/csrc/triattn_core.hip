@@ -58,6 +58,7 @@ constexpr int H = 4;
 constexpr int KT = 64;    // keys per tile
 constexpr int QW = 128;   // queries per workgroup (32 per wave)
 constexpr int tile_bytes(int d) { return KT * d * 2; }  // a K tile [64 keys][d] or a V^T tile [d][64 keys], bf16
+constexpr int RSRC_RAW = 0x00020000;  // last word of a raw (unstructured, range-checked) buffer descriptor
 constexpr uint32_t BF16_ONE = 0x3F80u, BF16_NEG_INF = 0xFF80u, BF16_NEG_1E9 = 0xCE6Eu;
 // A tile's scores, relative to the base, may rise to 2^T_HI before the base is moved (fp32 and
 // bf16 share their exponent range, so nothing is lost up there); the first tile with an unmasked
@@ -140,11 +141,10 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
   __shared__ __attribute__((aligned(1024))) char sV01[R > 1 ? V_BYTES : 16];
   __shared__ __attribute__((aligned(1024))) char sV10[V_BYTES];
   __shared__ __attribute__((aligned(1024))) char sV11[R > 1 ? V_BYTES : 16];
-  __shared__ uint32_t sLive[R];      // per row: some key is unmasked
-  __shared__ uint8_t sFlag[R * 64];  // per row and key tile (the first 64): 1 = some key unmasked, 3 = all 64 of them
+  __shared__ __attribute__((aligned(16))) uint64_t sBits[4][R][2];  // per wave and row, a bit per key tile: see the mask pass
   __shared__ float sMean[D];
   __shared__ uint32_t sRedo;  // a wave's unmasked-tile shortcut went wrong: the workgroup repeats its rows without it
-  extern __shared__ __attribute__((aligned(16))) uint16_t sCode[];  // [R][nkt * 64] mask code per key
+  extern __shared__ __attribute__((aligned(16))) uint16_t sCode[];  // [R][nkt * 64] mask code per key of the tiles that need one
 #define KBUF(ph, r) ((ph) == 0 ? ((r) == 0 ? sK00 : sK01) : ((r) == 0 ? sK10 : sK11))
 #define VBUF(ph, r) ((ph) == 0 ? ((r) == 0 ? sV00 : sV01) : ((r) == 0 ? sV10 : sV11))
 
@@ -154,15 +154,13 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
   const int xaddr = half_swap_addr();
   const int N = a.N;
   const int ldn = (int)a.ldn;
-  const int QT = (N + QW - 1) / QW;
   const int NG = (N + R - 1) / R;  // groups of R rows
-  // Workgroup ids are dealt round-robin to the 8 XCDs.  The query tiles of one (row group,
-  // head) share its K / V and run back to back on one XCD; the (row group, head) pairs are
-  // dealt to the XCDs in turn, so every XCD works on one head at a time (pair % 4 follows
+  // Workgroup ids are dealt round-robin to the 8 XCDs (the x dimension of the grid).  The query tiles of one (row group,
+  // head) share its K / V and run back to back on one XCD (y); the (row group, head) pairs are
+  // dealt to the XCDs in turn (z), so every XCD works on one head at a time (pair % 4 follows
   // from xcd % 4) and finds that head's bias in its L2.
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int qt = slot % QT;
-  const int pair_idx = (slot / QT) * 8 + xcd;
+  const int qt = blockIdx.y, slot = blockIdx.z * gridDim.y + qt;
+  const int pair_idx = blockIdx.z * 8 + blockIdx.x;
   if (pair_idx >= H * NG) return;
   const int rg = pair_idx / H;
   const int h = pair_idx % H;
@@ -171,12 +169,13 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
   // the other workgroup on the CU (which wave that is changes from workgroup to workgroup).  Computing on clamped queries
   // instead, as the other form does where no wave is without: 387 tokens 106 us against 99, 450 131 against 129, 600
   // 253 against 245; with a block for every wave the even form is the slower one, 768 tokens 434 against 430.
-  const int blocks = (N + 31) / 32, first = SPARE ? qt * blocks / QT : qt * 4;
+  const int first = SPARE ? qt * a.tile_blocks + min(qt, a.tile_extra) : qt * 4;
   const int turn = SPARE ? (wave + slot + (slot >> 5)) & 3 : wave;
-  const bool active = !SPARE || turn < (qt + 1) * blocks / QT - first;
+  const bool active = !SPARE || turn < a.tile_blocks + (qt < a.tile_extra ? 1 : 0);
   const int qblk = active ? first + turn : first;
-  const int qw = active ? qblk * 32 + j : N;
-  const int qi = min(qw, N - 1);
+  const int nq = active ? min(32, N - qblk * 32) : 0;  // queries of this wave (past the end it works on clamped ones)
+  const uint64_t query_lanes = nq == 32 ? ~0ull : ((1ull << max(nq, 0)) - 1ull) * 0x100000001ull;
+  const int qi = min(qblk * 32 + j, N - 1);
   const int nkt = (N + KT - 1) / KT;
   const int nk64 = nkt * KT;
 
@@ -188,40 +187,112 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
     brow[r] = min(rg * R + r, N - 1);
   }
 
-  // ---- mask pass: per-key codes for the mask k-step, live key tiles, dead rows ----
-  if (tid < R) sLive[tid] = 0u;
-  if (tid < R * 16) reinterpret_cast<uint32_t*>(sFlag)[tid] = 0u;
-  if (tid == 0) sRedo = 0u;
-  lds_barrier();
-  // A wave takes every fourth key tile; the mask values of eight of its tiles and all rows are
-  // requested together (one trip per 32 key tiles, not one per tile and row).  The mask is small
-  // and comes out of L2; Q comes from memory and is requested right behind the first batch of
-  // mask values: loads return in order, so the mask pass does not wait for it, and it travels
-  // while the mask pass, the barriers and the first tiles' loads are under way.
-  bf16x8 qf[R][KS];
-  if (D == 16 && tid < KT / 8) {
-    const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
-    const int at = TILE_BYTES + tid % (KT / 8) * 16;
-    *reinterpret_cast<u32x4*>(sV00 + at) = ones;
-    *reinterpret_cast<u32x4*>(sV10 + at) = ones;
-    if constexpr (R > 1) {
-      *reinterpret_cast<u32x4*>(sV01 + at) = ones;
-      *reinterpret_cast<u32x4*>(sV11 + at) = ones;
-    }
+  // ---- per-lane constants ----
+  u32x4 qm[R];  // Q side of the mask k-step: slot 0 = 1.0 (times the key's code), slot 1 = -base
+  const char* kglob[R];
+  const char* vglob[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int64_t bh = (int64_t)brow[r] * H + h;
+    qm[r] = u32x4{hh == 0 ? (BF16_ONE | 0x80000000u) : 0u, 0u, 0u, 0u};  // -0.0 in slot 1
+    kglob[r] = reinterpret_cast<const char*>(a.k + bh * N * D);
+    vglob[r] = reinterpret_cast<const char*>(a.vt + bh * D * a.ldn);
   }
-  // What a wave finds out about a tile is one byte in LDS, written by all its lanes alike; the
-  // workgroup's bit masks of live and of wholly unmasked tiles are ballots over those bytes.
-  bool my_any[R];
+  // fragment reads: K row (32 u + j), chunk (2 ks + hh) ^ ((j >> 2) & 3); V^T row j, chunk (2 s + hh) ^ ((j >> 1) & 7)
+  // heads of 16: K in blocks of 32 rows, the rows' first chunks and then their second ones; V^T row min(j, 16)
+  const int ksw = (j >> 2) & 3;
+  const int ka0 = D == 16 ? j * 16 + hh * 512 : j * 64 + ((hh ^ ksw) << 4), ka1 = j * 64 + (((2 + hh) ^ ksw) << 4);
+  const int vrow = min(j, D), vsw = (vrow >> 1) & 7;
+  int va[4];
 #pragma unroll
-  for (int r = 0; r < R; ++r) my_any[r] = false;
-  for (int t0 = 0; t0 < nkt; t0 += 32) {
-    float mv[R][8];
+  for (int s = 0; s < 4; ++s) va[s] = vrow * 128 + (((2 * s + hh) ^ vsw) << 4);
+  // loads into LDS: K keys 16 w + lane / 4, position lane % 4; V^T rows 8 w + lane / 8, position lane % 8
+  // heads of 16: K by the first two waves, V^T by the other two
+  const int part = D == 16 ? wave & 1 : wave;
+  const bool loads_k = D == 32 || wave < 2, loads_v = D == 32 || wave >= 2;
+  const int dk_key = D == 16 ? 32 * part + j : 16 * part + (lane >> 2);
+  const uint32_t dk_chunk = D == 16 ? (uint32_t)(hh << 4) : (uint32_t)(((lane & 3) ^ ((dk_key >> 2) & 3)) << 4);
+  const int dv_row = 8 * part + (lane >> 3);
+  const int dv_col = ((lane & 7) ^ ((dv_row >> 1) & 7)) * 8;
+  auto dma_k = [&](int tile, int r, char* buf) {  // a tile past the end re-reads the last one (never used)
+    if (!loads_k) return;
+    const int key = min(min(tile, nkt - 1) * KT + dk_key, N - 1);
+    dma16<0>(kglob[r], (uint32_t)key * (D * 2u) + dk_chunk, buf + part * 1024);
+  };
+  auto dma_v = [&](int tile, int r, char* buf) {
+    if (!loads_v) return;
+    const int col = min(tile, nkt - 1) * KT + dv_col;  // columns past ldn: any finite data will do (P is zero there)
+    dma16<0>(vglob[r], (uint32_t)(dv_row * ldn + (col < ldn ? col : 0)) * 2u, buf + part * 1024);
+  };
+  // bias tiles of this wave's 32-query block: 4 KB per key tile
+  const char* bbase =
+      HAS_BIAS ? reinterpret_cast<const char*>(a.bias + tri_bias_offset(N, h, qblk * 32, 0)) : nullptr;
+  // The bias tile of key tile t + 1 (four 1 KB fp16 fragments; fragment i = 2 u + st: keys
+  // 32 u + 16 st + 8 hh .. + 8 of this lane's query, bytes 32 j + 16 hh of run i) is only ever
+  // read by this wave, so it goes from memory straight into registers, requested when tile t
+  // begins.  The wait that the barrier in the middle of tile t needs anyway covers it.  While
+  // the last row of tile t computes its exponentials the fragments are turned into fp32 on
+  // the matrix unit, bt = I * bias^T with an fp16 identity: the initial value of the score
+  // accumulators of every row of tile t + 1 (four MFMAs per key tile, each issued between
+  // two groups of exponentials).  With one row per wave (LATE) there is nothing to share: the fragments start the tile's
+  // own score product, requested behind that of the tile before, and without bt's registers a third wave fits the SIMD
+  // (201 -> 168; 160 tokens 16.5 -> 13.8 us, 208 25.6 -> 22.2).  (Staged through LDS like K and V^T, by loads into LDS two
+  // tiles ahead, the same kernel ran 3.5 % slower: a load into LDS costs the wave more than
+  // a load into registers, and the fragments cost an LDS read each on top.)
+  constexpr bool LATE = R == 1 && HAS_BIAS;
+  f32x16 bt[2];
+  u32x4 bnext[4];
+  auto load_bias = [&](int tile) {
+    if (!HAS_BIAS) return;
+    const char* p = bbase + (size_t)min(tile, nkt - 1) * 4096u + (j * 32 + hh * 16);
 #pragma unroll
-    for (int r = 0; r < R; ++r)
+    for (int i = 0; i < 4; ++i) bnext[i] = *reinterpret_cast<const u32x4*>(p + 1024 * i);
+  };
+  auto first_loads = [&](int cur, int next) {
+    dma_k(cur, 0, KBUF(0, 0));
+    if (R == 2) {
+      dma_k(cur, R - 1, KBUF(0, R - 1));
+      dma_k(next, 0, KBUF(1, 0));
+      dma_v(cur, 0, VBUF(0, 0));
+      dma_v(cur, R - 1, VBUF(0, R - 1));
+    }
+  };
+
+  // ---- mask pass: per-key codes for the mask k-step, live key tiles, dead rows ----
+  // A wave takes every fourth key tile; the mask values of four of its tiles and all rows are requested together.  Behind the
+  // first batch go Q, the first bias tile and the loads into LDS for the first key tile, as if that were tile 0 (and the one
+  // after it tile 1; they are unless a sequence begins with 64 masked keys, and then these are loaded again below): a
+  // workgroup begins with one trip to memory.  What costs here are not the trips but the instructions: up to some 400 tokens
+  // a workgroup has few key tiles to spread them over, so the mask comes through range-checked loads off one address (what
+  // lies past the row reads as masked), a wholly unmasked tile costs a comparison and two scalar instructions (no codes: its
+  // few readers on the careful route know it), and what the waves found out meets in LDS as bit masks.  Of a workgroup's 17000
+  // cycles at 301 tokens 3600 went by before the end of this pass and 2100 more before the loop (us, two trips and a byte per
+  // tile before / now: 100 tokens 6.58 / 6.30, 187 15.55 / 14.77, 256 24.9 / 23.8, 320 50.9 / 49.5, from 400 on +-1 %).
+  bf16x8 qf[R][KS];
+  // (a key tile's bit: the first 63 tiles one each, the others share the last one; `all_bits` knows the first 64 only)
+  uint64_t any_bits[R], all_bits[R];
+  __amdgpu_buffer_rsrc_t mrow[R];
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        mv[r][u] = a.mask ? a.mask[(int64_t)brow[r] * N + min((t0 + 4 * u + wave) * KT + lane, N - 1)] : 1.f;
-    if (t0 == 0) {
+  for (int r = 0; r < R; ++r) {
+    any_bits[r] = all_bits[r] = 0ull;
+    mrow[r] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.mask ? a.mask + (int64_t)brow[r] * N : nullptr), 0, a.mask ? N * 4 : 0,
+                                                RSRC_RAW);
+  }
+  for (int t0 = wave; t0 < nkt || t0 == wave; t0 += 16) {
+    float mv[R][4];
+    if (a.mask) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          mv[r][u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mrow[r], (t0 * KT + lane) * 4 + u * 4 * KT * 4, 0, 0));
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) mv[r][u] = (t0 + 4 * u) * KT + lane < N ? 1.f : 0.f;
+    }
+    if (t0 == wave) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -230,50 +301,76 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
         qf[r][0] = as_frag(*reinterpret_cast<const u32x4*>(qp));
         if constexpr (KS == 2) qf[r][1] = as_frag(*reinterpret_cast<const u32x4*>(qp + 16));
       }
+      load_bias(0);
       __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int tile = t0 + 4 * u + wave;
-        if (tile < nkt) {
-          const int key = tile * KT + lane;
-          const bool on = key < N && mv[r][u] != 0.f;
-          sCode[r * nk64 + key] = (uint16_t)(key >= N ? BF16_NEG_INF : (mv[r][u] == 0.f ? BF16_NEG_1E9 : 0u));
-          const uint64_t on_lanes = __ballot(on);
-          my_any[r] = my_any[r] || on_lanes != 0ull;
-          if (tile < 64) sFlag[r * 64 + tile] = (uint8_t)((on_lanes != 0ull ? 1 : 0) | (on_lanes == ~0ull ? 2 : 0));
+      first_loads(0, 1);
+      if (tid == 0) sRedo = 0u;
+      if (D == 16 && tid < KT / 8) {
+        const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+        const int at = TILE_BYTES + tid % (KT / 8) * 16;
+        *reinterpret_cast<u32x4*>(sV00 + at) = ones;
+        *reinterpret_cast<u32x4*>(sV10 + at) = ones;
+        if constexpr (R > 1) {
+          *reinterpret_cast<u32x4*>(sV01 + at) = ones;
+          *reinterpret_cast<u32x4*>(sV11 + at) = ones;
         }
       }
-  }
+      // the buffer the first virtual tile reads its "previous" V^T from must hold finite data
+      if (tid * 16 < TILE_BYTES) *reinterpret_cast<u32x4*>(VBUF(1, R - 1) + tid * 16) = u32x4{0u, 0u, 0u, 0u};
+    }
 #pragma unroll
-  for (int r = 0; r < R; ++r)
-    if (my_any[r]) sLive[r] = 1u;
-  lds_barrier();
+    for (int u = 0; u < 4; ++u) {
+      const int tile = t0 + 4 * u;
+      if (tile >= nkt) break;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const uint64_t on_lanes = __ballot(mv[r][u] != 0.f);
+        const uint64_t bit = 1ull << min(tile, 63);
+        if (on_lanes != 0ull) any_bits[r] |= bit;
+        if (on_lanes == ~0ull && tile < 64) {
+          all_bits[r] |= bit;
+        } else {
+          const int key = tile * KT + lane;
+          sCode[r * nk64 + key] = (uint16_t)(key >= N ? BF16_NEG_INF : (mv[r][u] == 0.f ? BF16_NEG_1E9 : 0u));
+        }
+      }
+    }
+  }
+  if (lane < R) {
+    sBits[wave][lane][0] = R == 2 && lane == 1 ? any_bits[R - 1] : any_bits[0];
+    sBits[wave][lane][1] = R == 2 && lane == 1 ? all_bits[R - 1] : all_bits[0];
+  }
+  dma_barrier();  // (a workgroup without a live key has its loads into LDS behind it, too)
   bool dead[R];
   uint64_t live = 0ull;
   uint64_t plain[R];  // tiles of 64 unmasked keys below N (none beyond the 64th tile): they need no mask k-step
   bool all_dead = true;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    dead[r] = __builtin_amdgcn_readfirstlane(sLive[r]) == 0u;
-    const uint32_t flag = lane < nkt ? sFlag[r * 64 + lane] : 0u;
+    u32x4 w = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w |= *reinterpret_cast<const u32x4*>(&sBits[i][r][0]);
+    const uint64_t any = (uint64_t)__builtin_amdgcn_readfirstlane(w.y) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane(w.x);
+    plain[r] = (uint64_t)__builtin_amdgcn_readfirstlane(w.w) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane(w.z);
+    dead[r] = any == 0ull;
     all_dead = all_dead && dead[r];
-    live |= __ballot((flag & 1u) != 0u);
-    plain[r] = __ballot((flag & 2u) != 0u);
+    live |= any;
   }
   // next live tile, or nkt when none is left; more than 64 tiles are simply taken in order
-  uint64_t rest = live;
+  uint64_t rest = 0ull;
   int seq = 0;
   auto pop = [&]() {
-    if (nkt > 64) return seq < nkt ? seq++ : nkt;
-    if (rest == 0ull) return nkt;
-    const int tile = __builtin_ctzll(rest);
+    const bool found = rest != 0ull;
+    const int tile = found ? __builtin_ctzll(rest) : seq;
     rest &= rest - 1;
+    seq = min(seq + (found ? 0 : 1), nkt);
     return tile;
   };
 
+  // mask code of a key (a tile of unmasked keys has none in LDS)
+  auto code = [&](int r, int tile, int key) -> uint32_t {
+    return tile < 64 && ((plain[r] >> tile) & 1ull) != 0ull ? 0u : sCode[r * nk64 + tile * KT + key];
+  };
   f32x16 o[R];
   float lrun[R], base[R], mrel[R];  // lrun: sum of the probabilities of THIS lane's keys (half of each tile)
 #pragma unroll
@@ -286,76 +383,15 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
   }
 
   if (!all_dead) {
-    // ---- per-lane constants ----
-    u32x4 qm[R];  // Q side of the mask k-step: slot 0 = 1.0 (times the key's code), slot 1 = -base
-    const char* kglob[R];
-    const char* vglob[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int64_t bh = (int64_t)brow[r] * H + h;
-      qm[r] = u32x4{hh == 0 ? (BF16_ONE | 0x80000000u) : 0u, 0u, 0u, 0u};  // -0.0 in slot 1
-      kglob[r] = reinterpret_cast<const char*>(a.k + bh * N * D);
-      vglob[r] = reinterpret_cast<const char*>(a.vt + bh * D * a.ldn);
-    }
-    // fragment reads: K row (32 u + j), chunk (2 ks + hh) ^ ((j >> 2) & 3); V^T row j, chunk (2 s + hh) ^ ((j >> 1) & 7)
-    // heads of 16: K in blocks of 32 rows, the rows' first chunks and then their second ones; V^T row min(j, 16)
-    const int ksw = (j >> 2) & 3;
-    const int ka0 = D == 16 ? j * 16 + hh * 512 : j * 64 + ((hh ^ ksw) << 4), ka1 = j * 64 + (((2 + hh) ^ ksw) << 4);
-    const int vrow = min(j, D), vsw = (vrow >> 1) & 7;
-    int va[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) va[s] = vrow * 128 + (((2 * s + hh) ^ vsw) << 4);
-    // loads into LDS: K keys 16 w + lane / 4, position lane % 4; V^T rows 8 w + lane / 8, position lane % 8
-    // heads of 16: K by the first two waves, V^T by the other two
-    const int part = D == 16 ? wave & 1 : wave;
-    const bool loads_k = D == 32 || wave < 2, loads_v = D == 32 || wave >= 2;
-    const int dk_key = D == 16 ? 32 * part + j : 16 * part + (lane >> 2);
-    const uint32_t dk_chunk = D == 16 ? (uint32_t)(hh << 4) : (uint32_t)(((lane & 3) ^ ((dk_key >> 2) & 3)) << 4);
-    const int dv_row = 8 * part + (lane >> 3);
-    const int dv_col = ((lane & 7) ^ ((dv_row >> 1) & 7)) * 8;
-    auto dma_k = [&](int tile, int r, char* buf) {  // a tile past the end re-reads the last one (never used)
-      if (!loads_k) return;
-      const int key = min(min(tile, nkt - 1) * KT + dk_key, N - 1);
-      dma16<0>(kglob[r], (uint32_t)key * (D * 2u) + dk_chunk, buf + part * 1024);
-    };
-    auto dma_v = [&](int tile, int r, char* buf) {
-      if (!loads_v) return;
-      const int col = min(tile, nkt - 1) * KT + dv_col;  // columns past ldn: any finite data will do (P is zero there)
-      dma16<0>(vglob[r], (uint32_t)(dv_row * ldn + (col < ldn ? col : 0)) * 2u, buf + part * 1024);
-    };
-    // bias tiles of this wave's 32-query block: 4 KB per key tile
-    const char* bbase =
-        HAS_BIAS ? reinterpret_cast<const char*>(a.bias + tri_bias_offset(N, h, qblk * 32, 0)) : nullptr;
-    // The bias tile of key tile t + 1 (four 1 KB fp16 fragments; fragment i = 2 u + st: keys
-    // 32 u + 16 st + 8 hh .. + 8 of this lane's query, bytes 32 j + 16 hh of run i) is only ever
-    // read by this wave, so it goes from memory straight into registers, requested when tile t
-    // begins.  The wait that the barrier in the middle of tile t needs anyway covers it.  While
-    // the last row of tile t computes its exponentials the fragments are turned into fp32 on
-    // the matrix unit, bt = I * bias^T with an fp16 identity: the initial value of the score
-    // accumulators of every row of tile t + 1 (four MFMAs per key tile, each issued between
-    // two groups of exponentials).  With one row per wave (LATE) there is nothing to share: the fragments start the tile's
-    // own score product, requested behind that of the tile before, and without bt's registers a third wave fits the SIMD
-    // (201 -> 168; 160 tokens 16.5 -> 13.8 us, 208 25.6 -> 22.2).  (Staged through LDS like K and V^T, by loads into LDS two
-    // tiles ahead, the same kernel ran 3.5 % slower: a load into LDS costs the wave more than
-    // a load into registers, and the fragments cost an LDS read each on top.)
-    constexpr bool LATE = R == 1 && HAS_BIAS;
-    f32x16 bt[2];
-    u32x4 bnext[4];
-    auto load_bias = [&](int tile) {
-      if (!HAS_BIAS) return;
-      const char* p = bbase + (size_t)min(tile, nkt - 1) * 4096u + (j * 32 + hh * 16);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) bnext[i] = *reinterpret_cast<const u32x4*>(p + 1024 * i);
-    };
     // Identity fragments (fp16): A-fragment of k-step st: lane (row i = j, half hh) holds
     // I[i][16 st + 8 hh + e], e = 0..7: a single 1.0 where 16 st + 8 hh + e == i.
     f16x8 idf[2];
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       const int e1 = j - 16 * st - 8 * hh;
-      uint32_t w[4] = {0u, 0u, 0u, 0u};
-      if (e1 >= 0 && e1 < 8) w[e1 >> 1] = (e1 & 1) ? (0x3C00u << 16) : 0x3C00u;
-      idf[st] = as_frag_f16(u32x4{w[0], w[1], w[2], w[3]});
+      const uint32_t one = (j & 1) ? (0x3C00u << 16) : 0x3C00u;
+      const int at = e1 >> 1;  // negative, or 4 and more, where this lane has none
+      idf[st] = as_frag_f16(u32x4{at == 0 ? one : 0u, at == 1 ? one : 0u, at == 2 ? one : 0u, at == 3 ? one : 0u});
     }
     f32x16 zero16;
 #pragma unroll
@@ -434,8 +470,7 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
       f32x16 s0, s1;
       scores(kf, qf[RR], s0, s1);
       if (step3) {
-        const uint16_t* mc = sCode + RR * nk64 + tile * KT;
-        const uint32_t c0 = mc[j], c1 = mc[32 + j];
+        const uint32_t c0 = code(RR, tile, j), c1 = code(RR, tile, 32 + j);
         af0 = as_frag(u32x4{hh == 0 ? (c0 | (BF16_ONE << 16)) : 0u, 0u, 0u, 0u});
         af1 = as_frag(u32x4{hh == 0 ? (c1 | (BF16_ONE << 16)) : 0u, 0u, 0u, 0u});
         s0 = mfma32(af0, as_frag(qm[RR]), s0);
@@ -447,8 +482,8 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
       mx = fmaxf(mx, half_swap(xaddr, mx));
       const float mnew = fmaxf(mrel[RR], mx);
       // (lanes of queries past the end have no say: in a partly filled block they see bias values nobody wrote)
-      const bool want = qw < N && (mx > T_HI || (mnew < T_LO && mnew > LIVE_MIN));
-      if (__any(want)) {
+      const bool want = mx > T_HI || (mnew < T_LO && mnew > LIVE_MIN);
+      if ((__ballot(want) & query_lanes) != 0ull) {
         // Move the base of every query of the wave to its running maximum (rounded to bf16, the
         // form the matrix unit takes it in), rescale what the row has accumulated, and repeat the
         // score product.  Lanes that have seen no unmasked key yet keep their base: their O and l
@@ -462,8 +497,7 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
         qm[RR].x = hh == 0 ? (BF16_ONE | ((uint32_t)f2bf(-nb) << 16)) : 0u;
         based[RR] = true;
         if (!step3) {
-          const uint16_t* mc = sCode + RR * nk64 + tile * KT;
-          const uint32_t c0 = mc[j], c1 = mc[32 + j];
+          const uint32_t c0 = code(RR, tile, j), c1 = code(RR, tile, 32 + j);
           af0 = as_frag(u32x4{hh == 0 ? (c0 | (BF16_ONE << 16)) : 0u, 0u, 0u, 0u});
           af1 = as_frag(u32x4{hh == 0 ? (c1 | (BF16_ONE << 16)) : 0u, 0u, 0u, 0u});
         }
@@ -549,8 +583,8 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
     for (int pass = 0; pass < 2; ++pass) {
     allow_fast = pass == 0;
     bad = 0ull;
-    rest = live;
-    seq = 0;
+    rest = nkt > 64 ? 0ull : live;
+    seq = nkt > 64 ? 0 : nkt;
     pend = false;
 #pragma unroll
     for (int s = 0; s < 4; ++s) pp[s] = u32x4{0u, 0u, 0u, 0u};
@@ -572,30 +606,17 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
       used_fast[r] = false;
     }
     t_cur = pop(); t_n1 = pop(); t_n2 = pop();
-    // the buffer the first virtual tile reads its "previous" V^T from must hold finite data
-    if (tid * 16 < TILE_BYTES) *reinterpret_cast<u32x4*>(VBUF(1, R - 1) + tid * 16) = u32x4{0u, 0u, 0u, 0u};
-    // the first tiles' loads into LDS and the first bias tile's ordinary loads travel together
-    dma_k(t_cur, 0, KBUF(0, 0));
-    if (R == 2) {
-      dma_k(t_cur, 1, KBUF(0, 1));
-      dma_k(t_n1, 0, KBUF(1, 0));
-      dma_v(t_cur, 0, VBUF(0, 0));
-      dma_v(t_cur, 1, VBUF(0, 1));
-    }
-    if constexpr (LATE) {
+    if (pass == 1 || t_cur != 0 || (R == 2 && t_n1 != 1 && t_n1 < nkt)) {
       load_bias(t_cur);
-    } else if (HAS_BIAS) {
-      const char* p = bbase + (size_t)t_cur * 4096u + (j * 32 + hh * 16);
-      u32x4 f[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) f[i] = *reinterpret_cast<const u32x4*>(p + 1024 * i);
-      bt[0] = mfma32_f16(idf[1], as_frag_f16(f[1]), mfma32_f16(idf[0], as_frag_f16(f[0]), zero16));
-      bt[1] = mfma32_f16(idf[1], as_frag_f16(f[3]), mfma32_f16(idf[0], as_frag_f16(f[2]), zero16));
-    }
-    if (R == 2) {
+      first_loads(t_cur, t_n1);
+      if (tid * 16 < TILE_BYTES) *reinterpret_cast<u32x4*>(VBUF(1, R - 1) + tid * 16) = u32x4{0u, 0u, 0u, 0u};
       dma_barrier();
-      load_k_frags(KBUF(0, 0), kpre);
     }
+    if (HAS_BIAS && !LATE) {
+      bt[0] = mfma32_f16(idf[1], as_frag_f16(bnext[1]), mfma32_f16(idf[0], as_frag_f16(bnext[0]), zero16));
+      bt[1] = mfma32_f16(idf[1], as_frag_f16(bnext[3]), mfma32_f16(idf[0], as_frag_f16(bnext[2]), zero16));
+    }
+    if (R == 2) load_k_frags(KBUF(0, 0), kpre);
     // Every ordinary load issued so far (Q, the first bias tile) is waited for HERE, with a wait
     // the compiler can see: otherwise it keeps a vmcnt(0) for them at the top of the loop, where
     // it would also wait, every iteration, for the loads into LDS issued just before.
@@ -663,7 +684,7 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
     for (int r = 0; r < R; ++r) {
       if (!used_fast[r] || dead[r]) continue;
       const float lt = D == 16 ? o[r][8] : lrun[r] + half_swap(xaddr, lrun[r]);
-      bad |= __ballot(qw < N && (!((D == 16 ? fmaxf(lt, lmax[r]) : lmax[r]) < 0x1p60f) || lt < 0x1p-30f));
+      bad |= query_lanes & __ballot((!((D == 16 ? fmaxf(lt, lmax[r]) : lmax[r]) < 0x1p60f) || lt < 0x1p-30f));
     }
     if (bad != 0ull && lane == 0) sRedo = 1u;
     lds_barrier();  // also: every wave is done with the K / V^T tiles before a second pass loads over them
@@ -671,6 +692,10 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
     }
   }
 
+  // (what follows takes the lane's numbers anew: kept over the loops they would cost registers there)
+  int tid_end = threadIdx.x;
+  asm volatile("" : "+v"(tid_end));
+  const int hh_end = (tid_end >> 5) & 1, j_end = tid_end & 31;
   // a query's keys are split over the two half-waves
 #pragma unroll
   for (int r = 0; r < R; ++r) lrun[r] = D == 16 ? o[r][8] : lrun[r] + half_swap(xaddr, lrun[r]);
@@ -709,16 +734,16 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriA
     if ((tid & 7) == 0) sMean[v_d] = acc;
     lds_barrier();
 #pragma unroll
-    for (int e = 0; e < 16; ++e) o[r][e] = sMean[8 * ((e >> 2) & (D / 8 - 1)) + 4 * hh + (e & 3)];
+    for (int e = 0; e < 16; ++e) o[r][e] = sMean[8 * ((e >> 2) & (D / 8 - 1)) + 4 * hh_end + (e & 3)];
     lrun[r] = (float)N;
   }
 
-  if (qw >= N) return;
+  if (j_end >= nq) return;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     if (!bvalid[r]) continue;
     const float inv = 1.f / lrun[r];  // the sum over both half-waves' keys
-    bf16_t* op = a.og + ((int64_t)brow[r] * N + qw) * (H * D) + h * D + 4 * hh;
+    bf16_t* op = a.og + ((int64_t)brow[r] * N + qblk * 32 + j_end) * (H * D) + h * D + 4 * hh_end;
 #pragma unroll
     for (int g = 0; g < D / 8; ++g) {
       u32x2 w;
@@ -754,10 +779,11 @@ int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream) {
   const size_t stat2 = 8 * (size_t)tile + 1024;
   if (R == 2 && stat2 + 2 * (size_t)nkt * KT * sizeof(uint16_t) > 80 * 1024) R = 1;
   const int NG = (a.N + R - 1) / R;
-  const int64_t blocks = ((int64_t)H * NG + 7) / 8 * 8 * QT;
-  if (blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
   const size_t dyn = (size_t)R * nkt * KT * sizeof(uint16_t);
-  const dim3 grid((unsigned)blocks), block(256);
+  const dim3 grid(8, QT, (H * NG + 7) / 8), block(256);
+  TriAttnArgs args = a;
+  args.tile_blocks = (a.N + 31) / 32 / QT;
+  args.tile_extra = (a.N + 31) / 32 % QT;
   const size_t stat = (R == 2 ? 8 : 4) * (size_t)tile + 1024;
   auto launch = [&](void (*kernel)(TriAttnArgs)) {
     // more than 64 KB of LDS per workgroup in all (static + dynamic) has to be asked for
@@ -767,7 +793,7 @@ int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream) {
                                 (int)dyn);
       (void)hipGetLastError();
     }
-    hipLaunchKernelGGL(kernel, grid, block, dyn, stream, a);
+    hipLaunchKernelGGL(kernel, grid, block, dyn, stream, args);
   };
   const bool spare = (a.N + 31) / 32 % 4 != 0;
   if (a.head_dim == 16) {
