@@ -346,19 +346,9 @@ static int self_attention_run(
   g.seg_ops = SEG_BIAS_SCALE | (SEG_PLAIN << 4) | (SEG_PLAIN << 8) | (SEG_SIGMOID << 12);
   g.alpha = 1.0f / sqrtf((float)d);
   g.bias = query_b; g.bias_len = channels;  // the query segment's columns only
-  int rc = launch_gemm_nt(g, s);
-  if (rc) return rc;
-
-  FlashArgs f;
-  f.q = qkvg; f.k = qkvg + channels; f.v = qkvg + 2 * channels; f.g = qkvg + 3 * channels;
-  f.q_ss = f.k_ss = f.v_ss = f.g_ss = 4 * channels;
-  f.q_sb = f.k_sb = f.v_sb = f.g_sb = seq * 4 * channels;
-  f.out = out; f.out_f32 = out_dtype == AF3_F32; f.o_ss = channels; f.o_sb = seq * channels;
-  f.B = (int)batch; f.H = num_head; f.Sq = f.Sk = (int)seq; f.d = d;
-  f.bias = nonbatched_bias; f.bias_sb = 0; f.bias_sh = seq * seq; f.bias_sq = seq;
-  if (bias_quad_major) { f.bias_sq = 4; f.bias_squad = seq * 4; f.bias_sh = (seq + 3) / 4 * 4 * seq; }
-  f.key_mask = key_mask; f.km_sb = mask_batches == batch && batch > 1 ? seq : 0;
-  return launch_flash_attention(f, s);
+  const int rc = launch_gemm_nt(g, s);
+  return rc ? rc : run_self_attend(qkvg, key_mask, mask_batches, nonbatched_bias, bias_quad_major, num_head, out, out_dtype, batch, seq,
+                                   channels, s);
 }
 
 int af3_batch_diffusion_self_attention_forward(
@@ -704,6 +694,21 @@ int af3_check_attention_f32(
 
 }  // extern "C"
 
+int run_self_attend(const bf16_t* qkvg, const float* key_mask, int64_t mask_batches, const float* nonbatched_bias, int bias_quad_major,
+                    int num_head, void* out, int out_dtype, int64_t batch, int64_t seq, int channels, hipStream_t s) {
+  const int d = channels / num_head;
+  FlashArgs f;
+  f.q = qkvg; f.k = qkvg + channels; f.v = qkvg + 2 * channels; f.g = qkvg + 3 * channels;
+  f.q_ss = f.k_ss = f.v_ss = f.g_ss = 4 * channels;
+  f.q_sb = f.k_sb = f.v_sb = f.g_sb = seq * 4 * channels;
+  f.out = out; f.out_f32 = out_dtype == AF3_F32; f.o_ss = channels; f.o_sb = seq * channels;
+  f.B = (int)batch; f.H = num_head; f.Sq = f.Sk = (int)seq; f.d = d;
+  f.bias = nonbatched_bias; f.bias_sb = 0; f.bias_sh = seq * seq; f.bias_sq = seq;
+  if (bias_quad_major) { f.bias_sq = 4; f.bias_squad = seq * 4; f.bias_sh = (seq + 3) / 4 * 4 * seq; }
+  f.key_mask = key_mask; f.km_sb = mask_batches == batch && batch > 1 ? seq : 0;
+  return launch_flash_attention(f, s);
+}
+
 int run_self_attention(const bf16_t* q_data, const float* key_mask, int64_t mask_batches, const float* nonbatched_bias,
                        int bias_quad_major, const bf16_t* w_qkvg, const float* query_b, int num_head, void* out, int out_dtype,
                        int64_t batch, int64_t seq, int channels, void* workspace, size_t workspace_bytes, int split_k,
@@ -752,6 +757,12 @@ int run_linear(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int
     g.ld_res = n;
   }
   return launch_gemm_nt(g, stream);
+}
+
+bf16_t* self_projections(void* workspace, size_t workspace_bytes, int64_t rows, int channels) {
+  Carver ws(workspace, workspace_bytes);
+  bf16_t* qkvg = ws.take<bf16_t>((size_t)rows * 4 * channels);
+  return ws.ok ? qkvg : nullptr;
 }
 
 bool gathered_projections(void* workspace, size_t workspace_bytes, int64_t query_rows, int64_t atom_rows, int channels, bf16_t** qg,

@@ -173,8 +173,11 @@ __device__ __forceinline__ float half_swap(int xaddr, float v) {
 }
 __device__ __forceinline__ float wave_sum(float v) {
   v = group16_sum(v);
-  v += __shfl_xor(v, 16); v += __shfl_xor(v, 32);
-  return v;
+  // the other group of 16, then the other half of the wave, exchanged between registers and not through LDS
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(h[0]) + __uint_as_float(h[1]);
 }
 __device__ __forceinline__ float wave_max(float v) {
   for (int m = 1; m < 64; m <<= 1) v = fmaxf(v, __shfl_xor(v, m));
@@ -188,6 +191,16 @@ __device__ __forceinline__ float wave_max(float v) {
 // between threads through global memory, so waiting for LDS alone is enough.
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// q + d[0]^2 + .. + d[7]^2 for q >= 0, one after the other; begin: q is 0 and the first two meet as fma(d0, d0, d1 * d1).  (A sum
+// of two products can be contracted either way; kernels that have to agree to the last bit say which.)
+__device__ __forceinline__ float add_squares8(const float* d, float q, bool begin) {
+  if (begin) q = __builtin_fmaf(d[0], d[0], d[1] * d[1]);
+  else q = __builtin_fmaf(d[1], d[1], __builtin_fmaf(d[0], d[0], q));
+#pragma unroll
+  for (int e = 2; e < 8; ++e) q = __builtin_fmaf(d[e], d[e], q);
+  return q;
 }
 
 #define LN_EPS 1e-5f

@@ -83,6 +83,10 @@ __device__ __forceinline__ bool xcd_rect_tile(int rows, int xcd, int slot, int t
 int run_linear(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int y_dtype, int64_t m, int n, int k, int mode,
                float alpha, int sigmoid, const float* gate, int64_t gate_rows, int64_t gate_ld, const void* residual,
                int res_dtype, int split_k, hipStream_t stream);
+// run_self_attention's second half, on projections that are there (its workspace holds them, self_projections)
+int run_self_attend(const bf16_t* qkvg, const float* key_mask, int64_t mask_batches, const float* nonbatched_bias, int bias_quad_major,
+                    int num_head, void* out, int out_dtype, int64_t batch, int64_t seq, int channels, hipStream_t s);
+bf16_t* self_projections(void* workspace, size_t workspace_bytes, int64_t rows, int channels);
 int run_self_attention(const bf16_t* q_data, const float* key_mask, int64_t mask_batches, const float* nonbatched_bias,
                        int bias_quad_major, const bf16_t* w_qkvg, const float* query_b, int num_head, void* out, int out_dtype,
                        int64_t batch, int64_t seq, int channels, void* workspace, size_t workspace_bytes, int split_k,
@@ -424,6 +428,29 @@ struct AtomStepArgs {
 };
 bool atom_steps_apply(const AtomStepArgs& a);
 int launch_atom_step(const AtomStepArgs& a, bool tail, bool head, hipStream_t s);
+
+// --------------------------------------------------------------- token_step.hip
+// Adaptive LayerNorm of rows of 768 channels and a product of them: with w in fragment order, [N][768], out[row][n0 ..] =
+// queries (bias, scale), keys, values, gate (sigmoid), N = 4 x 768, or with swiglu N / 2 hidden units (w in blocks of 64 rows).
+// Row s tokens + t is token t of sample s; its conditioning is row t.
+constexpr int TOKEN_STEP_CHANNELS = 768;
+struct NormProductArgs {
+  unsigned work_blocks = 0, magic_tiles = 0;  // (these by launch_norm_product)
+  int per_xcd = 0, total = 0, tiles = 0, tile_tokens = 0, magic_samples = 0;
+  int samples = 0, tokens = 0, N = 0, swiglu = 0;
+  int ld_cond = 0;
+  const bf16_t* x = nullptr;     // [samples][tokens][768]
+  const float* scale = nullptr;  // [tokens][ld_cond]: 768 scales (before their sigmoid), 768 shifts
+  const bf16_t* w = nullptr;
+  int64_t ldc = 0;
+  const float* q_bias = nullptr;  // [768] or null
+  float q_scale = 1.f;
+  bf16_t* out = nullptr;  // [samples][tokens][ldc]
+  const void* warm[3] = {nullptr, nullptr, nullptr};  // as RowNormArgs
+  uint32_t warm_lines[3] = {0, 0, 0};
+};
+bool norm_product_applies(const NormProductArgs& a);
+int launch_norm_product(const NormProductArgs& a, hipStream_t s);
 
 // -------------------------------------------------------------------- embed.hip
 struct PairEmbedArgs {

@@ -107,8 +107,10 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(RowNormArgs a) {
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     if ((i * 64 + lane) * 8 < a.C) {
+      float d[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) { const float d = v[i][e] - mean; q += d * d; }
+      for (int e = 0; e < 8; ++e) d[e] = v[i][e] - mean;
+      q = add_squares8(d, q, i == 0);
     }
   }
   const float rstd = rsqrtf(wave_sum(q) / (float)a.C + LN_EPS);

@@ -513,10 +513,48 @@ int af3_diffusion_transformer_forward(
       if (r.p) { a.warm[k] = r.p; a.warm_lines[k] = (uint32_t)(r.bytes / 128); ++k; }
     return launch_row_norm(a, static_cast<hipStream_t>(stream));
   };
+  // The norm and the product behind it in one kernel, where all blocks' weights are there in its order; it warms what the kernels
+  // up to the next one read, the next one's weights among it.
+  const int nh = num_head > 0 ? num_head : 1;
+  bf16_t* const qkvg = self_projections(aw, ab, rows, c);
+  const bool act_ok = act_dtype == AF3_BF16 && c == TOKEN_STEP_CHANNELS && cond_rows == seq && rows <= 0x7fffffff;
+  auto step = [&](int i, bool transition) {
+    const af3_diffusion_block& b = blocks[i];
+    NormProductArgs a;
+    a.x = static_cast<const bf16_t*>(act); a.samples = (int)batch; a.tokens = (int)seq;
+    a.scale = scale_shift + ((int64_t)2 * i + transition) * 2 * c; a.ld_cond = (int)ld_ss;
+    a.w = b.frags ? b.frags + (transition ? (int64_t)4 * c * c : 0) : nullptr;
+    a.swiglu = transition; a.N = transition ? 2 * hidden : 4 * c; a.ldc = transition ? hidden : 4 * c;
+    a.out = transition ? y : qkvg;
+    if (!transition) { a.q_bias = b.q_b; a.q_scale = 1.0f / sqrtf((float)(c / nh)); }
+    return a;
+  };
+  bool steps = act_ok && qkvg && c % nh == 0;
+  for (int i = 0; i < num_blocks && steps; ++i) steps = norm_product_applies(step(i, false)) && norm_product_applies(step(i, true));
+  if (bias_quad_major != 0 && (bias_quad_major != 1 || (seq & 3))) return AF3_ERR_BAD_ARG;
   const size_t all_logits = (size_t)num_head * seq * seq * 4, logit_bytes = all_logits <= WARM_LOGIT_BYTES ? all_logits : 0;
   for (int i = 0; i < num_blocks; ++i) {
     const af3_diffusion_block& b = blocks[i];
     const float *ss = scale_shift + (int64_t)2 * i * 2 * c, *g = gate + (int64_t)2 * i * c;
+    if (steps) {
+      auto warm = [](NormProductArgs& a, int k, const void* p, size_t bytes) { a.warm[k] = p; a.warm_lines[k] = (uint32_t)(bytes / 128); };
+      NormProductArgs a = step(i, false);
+      warm(a, 0, b.w_out, (size_t)c * c * 2);
+      warm(a, 1, b.frags + (int64_t)4 * c * c, (size_t)2 * hidden * c * 2);
+      warm(a, 2, pair_logits[i], logit_bytes);
+      STEP(launch_norm_product(a, static_cast<hipStream_t>(stream)));
+      STEP(run_self_attend(qkvg, key_mask, 1, pair_logits[i], bias_quad_major, num_head, y, AF3_BF16, batch, seq, c,
+                           static_cast<hipStream_t>(stream)));
+      STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, cond_rows, ld_g, act,
+                              act_dtype, stream));
+      a = step(i, true);
+      warm(a, 0, b.w_tr2, (size_t)hidden * c * 2);
+      if (i + 1 < num_blocks) warm(a, 1, blocks[i + 1].frags, (size_t)4 * c * c * 2);
+      STEP(launch_norm_product(a, static_cast<hipStream_t>(stream)));
+      STEP(af3_linear_forward(y, b.w_tr2, nullptr, act, act_dtype, rows, c, hidden, AF3_LINEAR_GATE_RES, 1.f, 0, g + c, cond_rows, ld_g,
+                              act, act_dtype, stream));
+      continue;
+    }
     STEP(norm(ss, {b.w_q, (size_t)4 * c * c * 2}, {b.w_out, (size_t)c * c * 2}, {pair_logits[i], logit_bytes}));
     STEP(af3_batch_diffusion_self_attention_forward(x, key_mask, 1, pair_logits[i], bias_quad_major, b.w_q, b.q_b, num_head, y,
                                                     AF3_BF16, batch, seq, c, aw, ab, stream));

@@ -1,0 +1,282 @@
+// The token transformer's adaptive LayerNorm and the product behind it (queries, keys, values and gate; or the SwiGLU
+// transition's first layer) in one kernel, for rows of 768 channels on a bf16 stream.
+//
+// At a few hundred rows the two are launches of 5 and 8 to 10 us, of which the norm is a trip to memory and two reductions, and
+// the product waits for the norm's last row before its first.  Here a workgroup keeps up to 32 normalised rows in LDS (48 KB)
+// and multiplies them with 256 rows of the weights; its eight waves own 32 of those each and stream their fragments (frags of
+// af3_diffusion_block) from L2 into registers, the first ones on their way while the rows are normalised.  Every row is
+// normalised by each of the twelve workgroups that need it: what that costs is the conditioning, 6 KB of fp32 a token, so a
+// tile holds all samples of its tokens, which share it.  With the weights' rows in the order of the accumulators a lane ends
+// with runs of eight result columns (or with both factors of eight hidden units) and stores them as they are.
+// Values are rounded where the separate kernels store them and every sum has their order: the same bits.
+//
+// What bounds it: 0.45 MB of weights, rows and conditioning through the CU's vector memory path (64 bytes a cycle: 3.3 us at
+// 2.1 GHz) and the norms' vector instructions, 700 a row, which overlap but for their ends.  100 tokens of 5 samples, cycles of a
+// wave: rows there 3700, norms 6000, barrier 1500, product 3000, result 1000.  9.3 and 9.0 us against 5.1 + 9.9 and 5.1 + 8.2; a
+// token transformer of 24 blocks, us, separate kernels / this: 1 x 100 tokens 1174 / 1024, 1 x 304 1380 / 1304, 3 x 100 1228 /
+// 1080, 5 x 40 1136 / 981, 5 x 100 1330 / 1132, 5 x 126 1424 / 1335.  Past one workgroup to a CU the twelvefold norms cost
+// more than they save: 5 x 160 1539 / 1529, 5 x 250 1928 / 2091, 5 x 384 2062 / 2483.
+#include <type_traits>
+
+#include "common.h"
+#include "kernels.h"
+#include "tile_common.h"
+
+namespace {
+
+constexpr int K = TOKEN_STEP_CHANNELS, ROWS = 32, NW = 8, BN = 32 * NW;
+constexpr int NKS = K / 16, PIECES = NKS / 8, NB = 5;  // k-steps; pieces of eight; pieces in flight
+constexpr int PANEL = K / 64 * ROWS * 128;             // slabs of 64 channels, [slab][row][128 bytes]
+constexpr int WARM_LINES = 4;  // per thread
+constexpr int CUS = 256, WARM_CUS = 24;  // of which some for the workgroups that warm
+
+// TPW: tokens of a wave, SMAX: samples at most
+template <int TPW, int SMAX, bool SWIGLU>
+__global__ __launch_bounds__(64 * NW, 2) void norm_product_kernel(NormProductArgs a) {
+  __shared__ __attribute__((aligned(1024))) char sP[PANEL];
+  const int tid = threadIdx.x, lane = tid & 63, hh = lane >> 5, j = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (blockIdx.x >= a.work_blocks) {
+    // workgroups on the idle CUs bring what the next kernels read into the last-level cache (see ln_rows_kernel)
+    const uint32_t n0 = a.warm_lines[0], n1 = n0 + a.warm_lines[1], n2 = n1 + a.warm_lines[2];
+    uint32_t got[WARM_LINES];
+#pragma unroll
+    for (int u = 0; u < WARM_LINES; ++u) {
+      const uint32_t i = ((blockIdx.x - a.work_blocks) * WARM_LINES + u) * (64u * NW) + tid;
+      const char* p = static_cast<const char*>(i < n0 ? a.warm[0] : i < n1 ? a.warm[1] : a.warm[2]);
+      got[u] = i < n2 ? *reinterpret_cast<const uint32_t*>(p + (size_t)(i - (i < n0 ? 0u : i < n1 ? n0 : n1)) * 128) : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < WARM_LINES; ++u) asm volatile("" ::"v"(got[u]));
+    return;
+  }
+  // A range of the weights' rows for every XCD, each with the tiles of all rows one after the other
+  const int idx = (int)(blockIdx.x & 7) * a.per_xcd + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= a.per_xcd || idx >= a.total) return;
+  const int tn = a.tiles == 1 ? idx : (int)__umulhi((uint32_t)idx, a.magic_tiles), tt_n = a.tile_tokens;  // idx / tiles
+  const int t0 = (idx - tn * a.tiles) * tt_n, n0 = tn * BN;
+
+  // ---- the rows this wave normalises: all samples of tokens wave, wave + 8, .. of the tile; six tokens of five samples: the
+  // last two tokens by two waves each, so that every SIMD has seven or eight rows ----
+  // (What is too many is a copy of the last and is not kept: the rows' chains run beside each other in one block, or two.)
+  const bool split = SMAX == 5 && tt_n == 6 && wave >= 4;
+  const int tt_0 = split ? 4 + ((wave - 4) >> 1) : wave, s_0 = split && (wave & 1) ? 3 : 0;
+  const int count = split ? 3 - (wave & 1) : a.samples;
+  auto each_row = [&](auto f) {
+#pragma unroll
+    for (int k = 0; k < TPW; ++k)
+#pragma unroll
+      for (int s = 0; s < min(SMAX, 3); ++s) f(k, s);
+    if constexpr (SMAX > 3) {
+      if (count > 3) {
+        f(0, 3);
+        f(0, 4);
+      }
+    }
+  };
+  u32x4 raw[TPW][SMAX][2];
+  f32x4 sc[TPW][2][2], sh[TPW][2][2];
+  const int c0 = lane * 8, c1 = min(512 + lane * 8, K - 8);
+#pragma unroll
+  for (int k = 0; k < TPW; ++k) {
+    const int token = min(t0 + min(tt_0 + NW * k, tt_n - 1), a.tokens - 1);
+    const bf16_t* x = a.x + (s_0 * a.tokens + token) * K;
+#pragma unroll
+    for (int s = 0; s < SMAX; ++s) {
+      raw[k][s][0] = *reinterpret_cast<const u32x4*>(x + c0);
+      raw[k][s][1] = *reinterpret_cast<const u32x4*>(x + c1);
+      x += s + 1 < count ? a.tokens * K : 0;
+    }
+    const float* p = a.scale + (int64_t)token * a.ld_cond;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        sc[k][i][q] = *reinterpret_cast<const f32x4*>(p + (i ? c1 : c0) + 4 * q);
+        sh[k][i][q] = *reinterpret_cast<const f32x4*>(p + K + (i ? c1 : c0) + 4 * q);
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  bf16x8 w[NB][8];
+  auto fetch = [&](auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (n < PIECES) load_frags<8>(a.w, n0 / 32 + wave, NKS, 8 * n, lane, w[n % NB]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#define PIECE(n) std::integral_constant<int, (n)>{}
+  // A wave cannot go on before the CU's vector memory path has taken its loads, 16 cycles each: the rows first, and when they
+  // are there one piece in front of each part of the normalisation, as far as there are registers.
+  constexpr int AHEAD = TPW == 1 ? 3 : 2;
+  const bool busy = tt_0 < tt_n;  // (waves without a token)
+  if (busy)
+#pragma unroll
+    for (int k = 0; k < TPW; ++k)
+#pragma unroll
+      for (int s = 0; s < SMAX; ++s) asm volatile("" ::"v"(raw[k][s][0].x), "v"(raw[k][s][1].x));
+  fetch(PIECE(0));
+
+  // adaptive LayerNorm, ln_rows_kernel's sums
+  const bool upper = 512 + lane * 8 < K;
+  float v[TPW][SMAX][16], rstd[TPW][SMAX];
+  if (busy)
+    each_row([&](int k, int s) {
+      float* x = v[k][s];
+      float sum = 0.f, more;
+      unpack8(raw[k][s][0], x);
+      unpack8(raw[k][s][1], x + 8);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sum += x[e];
+      more = sum;
+#pragma unroll
+      for (int e = 8; e < 16; ++e) more += x[e];
+      const float mean = wave_sum(upper ? more : sum) / (float)K;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) x[e] -= mean;
+    });
+  fetch(PIECE(1));
+  if (busy)
+    each_row([&](int k, int s) {
+      const float* d = v[k][s];
+      const float q = add_squares8(d, 0.f, true), more = add_squares8(d + 8, q, false);
+      rstd[k][s] = rsqrtf(wave_sum(upper ? more : q) / (float)K + LN_EPS);
+    });
+  if constexpr (AHEAD > 2) fetch(PIECE(2));
+  if (busy) {
+    float gain[TPW][16];
+#pragma unroll
+    for (int k = 0; k < TPW; ++k)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) gain[k][e] = sigmoidf_(sc[k][e >> 3][(e >> 2) & 1][e & 3]);
+    each_row([&](int k, int s) {
+      const int tt = tt_0 + NW * k, row = tt * a.samples + s_0 + s;
+      const bool keep = tt < tt_n && s < count;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float o[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float t = v[k][s][8 * i + e] * rstd[k][s];
+          o[e] = gain[k][8 * i + e] * t + sh[k][i][e >> 2][e & 3];
+        }
+        const int chunk = 64 * i + lane;  // chunk c of a slab's row lies at position c ^ (row / 2 % 8)
+        if (keep && (i == 0 || upper))
+          *reinterpret_cast<u32x4*>(sP + (chunk >> 3) * (ROWS * 128) + row * 128 + (((chunk & 7) ^ ((row >> 1) & 7)) << 4)) = pack8(o);
+      }
+    });
+  }
+  if constexpr (AHEAD < 3) fetch(PIECE(2));
+  fetch(PIECE(3));
+  fetch(PIECE(4));
+  // a lane's registers 8 u .. are result columns 32 wave + 16 u + 8 hh .. of row j (with swiglu 8 u: first and second factor of
+  // hidden units 16 wave + 8 hh ..)
+  const int col = n0 + 32 * wave + 8 * hh;
+  const bool queries = !SWIGLU && tn < K / BN;
+  float bias[16];
+  if constexpr (!SWIGLU) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) load_param8(queries && a.q_bias ? a.q_bias + col + 16 * u : nullptr, 0.f, bias + 8 * u);
+  }
+  lds_barrier();
+
+  // ---- the product, a lane owns a row ----
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  bf16x8 xf[2][8];
+  auto rows = [&](auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    if constexpr (n < PIECES)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int ks = 8 * n + i, c = 2 * (ks & 3) + hh;
+        xf[n & 1][i] = as_frag(*reinterpret_cast<const u32x4*>(sP + (ks >> 2) * (ROWS * 128) + j * 128 + ((c ^ ((j >> 1) & 7)) << 4)));
+      }
+  };
+  auto piece = [&](auto n_c) {  // (the next one's rows are read meanwhile)
+    constexpr int n = decltype(n_c)::value;
+    rows(PIECE(n + 1));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc = mfma32(w[n % NB][i], xf[n & 1][i], acc);
+    fetch(PIECE(n + NB));
+  };
+  rows(PIECE(0));
+  piece(PIECE(0));
+  piece(PIECE(1));
+  piece(PIECE(2));
+  piece(PIECE(3));
+  piece(PIECE(4));
+  piece(PIECE(5));
+  static_assert(PIECES == 6, "all of them");
+#undef PIECE
+
+  // ---- column operations, 64 bytes of a row to a wave (SwiGLU 32) ----
+  const int tt = (j * a.magic_samples) >> 16, token = t0 + tt;  // j / samples
+  if (tt >= tt_n || token >= a.tokens) return;
+  bf16_t* const out = a.out + ((int64_t)(j - tt * a.samples) * a.tokens + token) * a.ldc;
+  float o[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) o[r] = acc[r];
+  if constexpr (SWIGLU) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = o[e] * sigmoidf_(o[e]) * o[8 + e];
+    *reinterpret_cast<u32x4*>(out + n0 / 2 + 16 * wave + 8 * hh) = pack8(o);
+  } else {
+    if (queries) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[r] = (o[r] + bias[r]) * a.q_scale;
+    } else if (tn >= 3 * (K / BN)) {  // the gate
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[r] = sigmoidf_(o[r]);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) *reinterpret_cast<u32x4*>(out + col + 16 * u) = pack8(o + 8 * u);
+  }
+}
+
+bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+}  // namespace
+
+// Tokens of a tile, by the number of samples.  One of fewer leaves rows of the matrix instruction empty, but its norms are done
+// sooner: taken while every tile has a CU of its own (24 blocks, us: 1 x 100 tokens by 32 1174, by 8 1024; 3 x 152 by 8 1203, 3 x 160
+// by 10 1284; 5 x 76 by 4 1110, 5 x 80 by 6 1097).
+static int tile_tokens(const NormProductArgs& a) {
+  static constexpr int sizes[5][2] = {{8, 16}, {8, 16}, {8, 10}, {4, 8}, {4, 6}};
+  const int* const of = sizes[a.samples - 1];
+  return (int64_t)((a.tokens - 1) / of[0] + 1) * (a.N / BN) <= CUS - WARM_CUS ? of[0] : of[1];
+}
+
+bool norm_product_applies(const NormProductArgs& a) {
+  return a.x && a.w && a.out && a.scale && a.samples > 0 && a.samples <= 5 && a.tokens > 0 && a.N > 0 && a.N % BN == 0 &&
+         (a.swiglu || a.N == 4 * K) && (int64_t)((a.tokens - 1) / tile_tokens(a) + 1) * (a.N / BN) <= CUS && a.ld_cond >= 2 * K &&
+         a.ld_cond % 4 == 0 && a.ldc % 8 == 0 && al16(a.x) && al16(a.w) && al16(a.out) && al16(a.scale) && al16(a.q_bias);
+}
+
+int launch_norm_product(const NormProductArgs& args, hipStream_t s) {
+  if (!norm_product_applies(args)) return AF3_ERR_BAD_ARG;
+  NormProductArgs a = args;
+  a.tile_tokens = tile_tokens(a);
+  a.tiles = (a.tokens + a.tile_tokens - 1) / a.tile_tokens;
+  a.total = a.tiles * (a.N / BN);
+  a.per_xcd = (a.total + 7) / 8;
+  a.work_blocks = 8u * a.per_xcd;
+  a.magic_tiles = a.tiles == 1 ? 0u : 0xffffffffu / (uint32_t)a.tiles + 1u;  // idx / tiles = umulhi(idx, magic): idx tiles < 2^32
+  a.magic_samples = 65536 / a.samples + 1;                                   // row / samples, row < 32
+  // (no more workgroups that warm than there are CUs left: one that waits for a CU makes the kernel longer)
+  const int64_t lines = (int64_t)a.warm_lines[0] + a.warm_lines[1] + a.warm_lines[2];
+  const int64_t warm = (lines + 64 * NW * WARM_LINES - 1) / (64 * NW * WARM_LINES), idle = CUS - (int64_t)a.work_blocks;
+  const dim3 grid(a.work_blocks + (unsigned)(warm < idle ? warm : idle > 0 ? idle : 0)), block(64 * NW);
+#define LAUNCH(TPW, SMAX)                                                                           \
+  do {                                                                                              \
+    if (a.swiglu) hipLaunchKernelGGL((norm_product_kernel<TPW, SMAX, true>), grid, block, 0, s, a); \
+    else hipLaunchKernelGGL((norm_product_kernel<TPW, SMAX, false>), grid, block, 0, s, a);         \
+  } while (0)
+  if (a.samples > 3) LAUNCH(1, 5);
+  else if (a.samples > 1 && a.tile_tokens > 8) LAUNCH(2, 3);
+  else if (a.samples > 1) LAUNCH(1, 3);
+  else if (a.tile_tokens > 8) LAUNCH(2, 1);
+  else LAUNCH(1, 1);
+#undef LAUNCH
+  return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+}

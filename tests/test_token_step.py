@@ -1,0 +1,32 @@
+"""The token transformer's norms and the products behind them in one kernel (token_step.hip) against the operators one by one."""
+
+import pytest
+import torch
+
+
+# tiles hold all samples of 4 to 16 tokens, by the number of samples and of tiles: one token, tiles that are filled and that are
+# not, both sizes of every number of samples, one number that has no such kernel, more tokens than it takes, weights of 6 to 18 tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("samples,n,factor", [(1, 1, 2), (1, 33, 2), (1, 64, 1), (1, 200, 2), (1, 337, 2), (2, 17, 2), (2, 161, 1), (3, 31, 2),
+                                              (3, 155, 2), (4, 40, 3), (4, 81, 2), (5, 6, 2), (5, 77, 2), (5, 100, 2), (5, 130, 2), (6, 11, 2)])
+def test_the_steps_give_the_bits_of_the_operators(gpu_pkg, samples, n, factor):
+    g = torch.Generator(device="cuda").manual_seed(100 * samples + n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    with torch.device("cuda"):
+        mod = gpu_pkg.nn.DiffusionTransformer(num_blocks=2, super_block_size=1)
+        for tr in mod.transition_block:
+            tr.__init__(c_x=768, c_single_cond=384, num_intermediate_factor=factor, use_single_cond=True)
+    with torch.no_grad():
+        for p in mod.parameters():
+            p.normal_(0.0, 0.05, generator=g)
+    mod.invalidate()
+    act, cond, pair = rnd(samples, n, 768).bfloat16(), rnd(n, 384), rnd(n, n, 128)
+    act[0, 0] *= 1000                                            # rows of other sizes
+    act[-1, -1] = 0
+    mask = (torch.arange(n, device="cuda") < max(1, n - 1)).float()
+    run = lambda: mod(act.clone(), mask, cond, pair)
+    want, seen = run(), []
+    hook = mod.self_attention[1].adaptive_layernorm.register_forward_hook(lambda *a: seen.append(1))
+    got = run()
+    hook.remove()
+    assert seen and torch.isfinite(want).all() and not torch.equal(want, act) and torch.equal(got, want)
