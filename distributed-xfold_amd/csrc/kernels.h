@@ -449,6 +449,18 @@ struct NormProductArgs {
   const void* warm[3] = {nullptr, nullptr, nullptr};  // as RowNormArgs
   uint32_t warm_lines[3] = {0, 0, 0};
 };
+// act = (y w^T) gate + act in place: 768 columns, K = 768 or 1536, w in fragment order; gate row: row % cond_rows
+struct GatedProductArgs {
+  int per_xcd = 0, total = 0, tiles = 0;  // (these and the magic numbers by launch_gated_product)
+  unsigned magic_tiles = 0, magic_cond = 0;
+  int rows = 0, K = 0, cond_rows = 0;
+  const bf16_t *y = nullptr, *w = nullptr;  // [rows][K], [768][K]
+  bf16_t* act = nullptr;                    // [rows][768]
+  const float* gate = nullptr;              // [cond_rows][ld_gate]
+  int64_t ld_gate = 0;
+};
+bool gated_product_applies(const GatedProductArgs& a);
+int launch_gated_product(const GatedProductArgs& a, hipStream_t s);
 bool norm_product_applies(const NormProductArgs& a);
 int launch_norm_product(const NormProductArgs& a, hipStream_t s);
 

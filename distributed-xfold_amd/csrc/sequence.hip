@@ -529,6 +529,14 @@ int af3_diffusion_transformer_forward(
     if (!transition) { a.q_bias = b.q_b; a.q_scale = 1.0f / sqrtf((float)(c / nh)); }
     return a;
   };
+  auto back = [&](int i, bool transition) {  // the product behind either, with its gate, into the stream
+    const af3_diffusion_block& b = blocks[i];
+    GatedProductArgs a;
+    a.rows = (int)rows; a.K = transition ? hidden : c; a.cond_rows = (int)cond_rows; a.y = y; a.act = static_cast<bf16_t*>(act);
+    a.w = b.frags ? b.frags + (int64_t)(transition ? 5 * c + 2 * hidden : 4 * c + 2 * hidden) * c : nullptr;
+    a.gate = gate + ((int64_t)2 * i + transition) * c; a.ld_gate = ld_g;
+    return a;
+  };
   bool steps = act_ok && qkvg && c % nh == 0;
   for (int i = 0; i < num_blocks && steps; ++i) steps = norm_product_applies(step(i, false)) && norm_product_applies(step(i, true));
   if (bias_quad_major != 0 && (bias_quad_major != 1 || (seq & 3))) return AF3_ERR_BAD_ARG;
@@ -539,20 +547,26 @@ int af3_diffusion_transformer_forward(
     if (steps) {
       auto warm = [](NormProductArgs& a, int k, const void* p, size_t bytes) { a.warm[k] = p; a.warm_lines[k] = (uint32_t)(bytes / 128); };
       NormProductArgs a = step(i, false);
-      warm(a, 0, b.w_out, (size_t)c * c * 2);
+      const GatedProductArgs out = back(i, false), down = back(i, true);
+      const bool out_step = gated_product_applies(out), down_step = gated_product_applies(down);
+      warm(a, 0, out_step ? out.w : b.w_out, (size_t)c * c * 2);
       warm(a, 1, b.frags + (int64_t)4 * c * c, (size_t)2 * hidden * c * 2);
       warm(a, 2, pair_logits[i], logit_bytes);
       STEP(launch_norm_product(a, static_cast<hipStream_t>(stream)));
       STEP(run_self_attend(qkvg, key_mask, 1, pair_logits[i], bias_quad_major, num_head, y, AF3_BF16, batch, seq, c,
                            static_cast<hipStream_t>(stream)));
-      STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, cond_rows, ld_g, act,
-                              act_dtype, stream));
+      if (out_step) STEP(launch_gated_product(out, static_cast<hipStream_t>(stream)));
+      else
+        STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, cond_rows, ld_g, act,
+                                act_dtype, stream));
       a = step(i, true);
-      warm(a, 0, b.w_tr2, (size_t)hidden * c * 2);
+      warm(a, 0, down_step ? down.w : b.w_tr2, (size_t)hidden * c * 2);
       if (i + 1 < num_blocks) warm(a, 1, blocks[i + 1].frags, (size_t)4 * c * c * 2);
       STEP(launch_norm_product(a, static_cast<hipStream_t>(stream)));
-      STEP(af3_linear_forward(y, b.w_tr2, nullptr, act, act_dtype, rows, c, hidden, AF3_LINEAR_GATE_RES, 1.f, 0, g + c, cond_rows, ld_g,
-                              act, act_dtype, stream));
+      if (down_step) STEP(launch_gated_product(down, static_cast<hipStream_t>(stream)));
+      else
+        STEP(af3_linear_forward(y, b.w_tr2, nullptr, act, act_dtype, rows, c, hidden, AF3_LINEAR_GATE_RES, 1.f, 0, g + c, cond_rows,
+                                ld_g, act, act_dtype, stream));
       continue;
     }
     STEP(norm(ss, {b.w_q, (size_t)4 * c * c * 2}, {b.w_out, (size_t)c * c * 2}, {pair_logits[i], logit_bytes}));

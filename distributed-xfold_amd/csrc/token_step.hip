@@ -234,6 +234,112 @@ __global__ __launch_bounds__(64 * NW, 2) void norm_product_kernel(NormProductArg
   }
 }
 
+// 64 lanes x 16 bytes from memory (uniform base, a byte offset per lane) to 1 KB of LDS at `lds`.  Inline assembly, because the
+// compiler's own form makes later LDS reads wait for every such load in flight; the panel is read behind a wait of its own.
+__device__ __forceinline__ void load_to_lds(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:0" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
+
+// The products that lead back into the stream: act = (y w^T) gate + act, 768 result columns, K = 128 KP.  A workgroup takes 32
+// rows and 32 columns per wave; the rows go to LDS as a panel, all of them at once, the weights' fragments straight to registers,
+// gate and stream asked for behind them: one trip to memory, a chain of 48 or 96 matrix instructions (some 36 cycles each), and
+// the result back from the registers.  The general kernel's 32x32 tile, a slab at a time, takes 7.5 us on average of the two at
+// 500 rows.  Two waves share a panel where that keeps to one workgroup a CU, one has it alone at up to 320 rows.
+// A token transformer of 24 blocks with the norms in its other products, us, without this / with it: 5 x 40 tokens 981 / 867,
+// 5 x 100 1132 / 1044, 5 x 126 1335 / 1185, 1 x 100 1024 / 905, 3 x 100 1080 / 961, 2 x 300 1423 / 1330.
+template <int KP, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 1) void gated_product_kernel(GatedProductArgs a) {
+  constexpr int KK = 128 * KP, SLABS = KK / 64, RING = 5;
+  __shared__ __attribute__((aligned(1024))) char sP[SLABS * ROWS * 128];
+  const int lane = threadIdx.x & 63, hh = lane >> 5, j = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int idx = (int)(blockIdx.x & 7) * a.per_xcd + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= a.per_xcd || idx >= a.total) return;
+  const int tn = a.tiles == 1 ? idx : (int)__umulhi((uint32_t)idx, a.magic_tiles);
+  const int m0 = (idx - tn * a.tiles) * ROWS, n0 = (tn * WAVES + wave) * 32;
+
+  // the panel, slab by slab; a wave brings every WAVES-th group of eight rows
+  const bf16_t* const y = a.y + (int64_t)m0 * KK;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)sP;
+  uint32_t off[4 / WAVES];
+#pragma unroll
+  for (int i = 0; i < 4 / WAVES; ++i) {
+    const int row = 8 * (WAVES * i + wave) + (lane >> 3);
+    off[i] = (uint32_t)(min(row, a.rows - 1 - m0) * KK + ((lane & 7) ^ ((row >> 1) & 7)) * 8) * 2u;
+  }
+#pragma unroll
+  for (int s = 0; s < SLABS; ++s)
+#pragma unroll
+    for (int i = 0; i < 4 / WAVES; ++i)
+      load_to_lds(y + 64 * s, off[i], __builtin_amdgcn_readfirstlane(lds0 + s * (ROWS * 128) + (WAVES * i + wave) * 1024));
+  bf16x8 w[RING][8];
+  auto fetch = [&](auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (n < KP) load_frags<8>(a.w, tn * WAVES + wave, KK / 16, 8 * n, lane, w[n % RING]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#define PIECE(n) std::integral_constant<int, (n)>{}
+  fetch(PIECE(0));
+  fetch(PIECE(1));
+  fetch(PIECE(2));
+  // a lane's registers 8 u .. are columns 16 u + 8 hh .. of row j
+  const int row = min(m0 + j, a.rows - 1), col = n0 + 8 * hh;
+  const int cond = row - (a.cond_rows == 1 ? row : (int)__umulhi((uint32_t)row, a.magic_cond)) * a.cond_rows;
+  bf16_t* const act = a.act + (int64_t)row * K + col;
+  const float* const gp = a.gate + (int64_t)cond * a.ld_gate + col;
+  f32x4 gate[2][2];
+  u32x4 res[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    gate[u][0] = *reinterpret_cast<const f32x4*>(gp + 16 * u);
+    gate[u][1] = *reinterpret_cast<const f32x4*>(gp + 16 * u + 4);
+    res[u] = *reinterpret_cast<const u32x4*>(act + 16 * u);
+  }
+  fetch(PIECE(3));
+  fetch(PIECE(4));
+  // (what was asked for behind the panel may be on its way still)
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * RING + 6) : "memory");
+  lds_barrier();
+
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  bf16x8 xf[2][8];
+  auto rows = [&](auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    if constexpr (n < KP)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int ks = 8 * n + i, c = 2 * (ks & 3) + hh;
+        xf[n & 1][i] = as_frag(*reinterpret_cast<const u32x4*>(sP + (ks >> 2) * (ROWS * 128) + j * 128 + ((c ^ ((j >> 1) & 7)) << 4)));
+      }
+  };
+  auto piece = [&](auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    if constexpr (n < KP) {
+      rows(PIECE(n + 1));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc = mfma32(w[n % RING][i], xf[n & 1][i], acc);
+      fetch(PIECE(n + RING));
+    }
+  };
+  rows(PIECE(0));
+  piece(PIECE(0)); piece(PIECE(1)); piece(PIECE(2)); piece(PIECE(3)); piece(PIECE(4)); piece(PIECE(5));
+  piece(PIECE(6)); piece(PIECE(7)); piece(PIECE(8)); piece(PIECE(9)); piece(PIECE(10)); piece(PIECE(11));
+  static_assert(KP <= 12, "all of them");
+#undef PIECE
+  if (m0 + j >= a.rows) return;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    float o[8], x[8];
+    unpack8(res[u], x);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = (acc[8 * u + e] + 0.f) * gate[u][e >> 2][e & 3] + x[e];
+    *reinterpret_cast<u32x4*>(act + 16 * u) = pack8(o);
+  }
+}
+
 bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
@@ -277,6 +383,32 @@ int launch_norm_product(const NormProductArgs& args, hipStream_t s) {
   else if (a.samples > 1) LAUNCH(1, 3);
   else if (a.tile_tokens > 8) LAUNCH(2, 1);
   else LAUNCH(1, 1);
+#undef LAUNCH
+  return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+}
+
+bool gated_product_applies(const GatedProductArgs& a) {
+  return a.y && a.w && a.act && a.gate && a.rows > 0 && (a.K == 768 || a.K == 1536) && a.cond_rows > 0 && a.ld_gate >= K &&
+         a.ld_gate % 4 == 0 && al16(a.y) && al16(a.w) && al16(a.act) && al16(a.gate) && (int64_t)((a.rows - 1) / ROWS + 1) * (K / 64) <= CUS;
+}
+
+int launch_gated_product(const GatedProductArgs& args, hipStream_t s) {
+  if (!gated_product_applies(args)) return AF3_ERR_BAD_ARG;
+  GatedProductArgs a = args;
+  a.tiles = (a.rows + ROWS - 1) / ROWS;
+  const int waves = a.tiles * (K / 32) <= CUS ? 1 : 2;
+  a.total = a.tiles * (K / 32 / waves);
+  a.per_xcd = (a.total + 7) / 8;
+  a.magic_tiles = a.tiles == 1 ? 0u : 0xffffffffu / (uint32_t)a.tiles + 1u;
+  a.magic_cond = a.cond_rows == 1 ? 0u : 0xffffffffu / (uint32_t)a.cond_rows + 1u;
+  const dim3 grid(8u * a.per_xcd), block(64 * waves);
+#define LAUNCH(KP)                                                                                  \
+  do {                                                                                              \
+    if (waves == 1) hipLaunchKernelGGL((gated_product_kernel<KP, 1>), grid, block, 0, s, a);        \
+    else hipLaunchKernelGGL((gated_product_kernel<KP, 2>), grid, block, 0, s, a);                   \
+  } while (0)
+  if (a.K == 768) LAUNCH(6);
+  else LAUNCH(12);
 #undef LAUNCH
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }

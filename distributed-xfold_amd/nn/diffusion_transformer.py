@@ -59,7 +59,8 @@ def block_table(owner: HipModule, blocks, c: int):
             s.frags = frags[-1].data_ptr()
         elif "w_qkvg" in att and c == 768 and table.hidden % 128 == 0:
             w1 = tr["w1"].view(-1, 2, 2, 16, c).transpose(1, 2)      # 16 rows of either factor to a block of 32
-            frags.append(torch.cat([fragments(att["w_qkvg"], swap23=True), fragments(w1.reshape(-1, c), swap23=True)]))
+            frags.append(torch.cat([fragments(att["w_qkvg"], swap23=True), fragments(w1.reshape(-1, c), swap23=True),
+                                    fragments(att_out["w"], swap23=True), fragments(tr_out["w"], swap23=True)]))
             s.frags = frags[-1].data_ptr()
     owner._native = (table, packs, frags)
     return table
