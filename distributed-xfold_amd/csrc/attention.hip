@@ -26,6 +26,7 @@ namespace {
 
 constexpr int KT = 64;        // keys per LDS tile
 constexpr float NEG_INF = -__builtin_huge_valf();
+constexpr int RSRC_RAW = 0x00020000;  // last word of a raw (unstructured, range-checked) buffer descriptor
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef short v8s __attribute__((ext_vector_type(8)));
 // ds_read_b64_tr_b16: four 16-bit elements per lane, transposed within each group of 16 lanes
@@ -35,6 +36,20 @@ __device__ __forceinline__ v4s lds_read_tr16(const bf16_t* p) {
 constexpr float LOG2E = 1.4426950408889634f;
 // per-key code staged in LDS next to the K tile
 constexpr int KEY_MASKED = 1, KEY_PAD = 2, KEY_BEYOND = 4;
+
+// maximum of the lane's 32 logits as a tree of three-input maxima
+__device__ __forceinline__ float max3_of_32(const f32x16 (&s)[2]) {
+  float t3[11];
+#pragma unroll
+  for (int i = 0; i < 10; ++i) {
+    const int e = 3 * i;
+    t3[i] = fmaxf(fmaxf(s[e >> 4][e & 15], s[(e + 1) >> 4][(e + 1) & 15]), s[(e + 2) >> 4][(e + 2) & 15]);
+  }
+  t3[10] = fmaxf(s[1][14], s[1][15]);
+  const float t9a = fmaxf(fmaxf(t3[0], t3[1]), t3[2]), t9b = fmaxf(fmaxf(t3[3], t3[4]), t3[5]);
+  const float t9c = fmaxf(fmaxf(t3[6], t3[7]), t3[8]), t9d = fmaxf(t3[9], t3[10]);
+  return fmaxf(fmaxf(fmaxf(t9a, t9b), t9c), t9d);
+}
 
 // FAST: keys are rows of K / V as they stand (no row table) and the pair bias is present and 16-byte
 // addressable.  Then every address of the key-tile loop is a wave-uniform base that advances by a
@@ -344,17 +359,7 @@ void flash_kernel(FlashArgs a) {
           }
         }
     }
-    // maximum of the lane's 32 logits as a tree of three-input maxima
-    float t3[11];
-#pragma unroll
-    for (int i = 0; i < 10; ++i) {
-      const int e = 3 * i;
-      t3[i] = fmaxf(fmaxf(s[e >> 4][e & 15], s[(e + 1) >> 4][(e + 1) & 15]), s[(e + 2) >> 4][(e + 2) & 15]);
-    }
-    t3[10] = fmaxf(s[1][14], s[1][15]);
-    const float t9a = fmaxf(fmaxf(t3[0], t3[1]), t3[2]), t9b = fmaxf(fmaxf(t3[3], t3[4]), t3[5]);
-    const float t9c = fmaxf(fmaxf(t3[6], t3[7]), t3[8]), t9d = fmaxf(t3[9], t3[10]);
-    float mx = fmaxf(fmaxf(fmaxf(t9a, t9b), t9c), t9d);
+    float mx = max3_of_32(s);
     mx = fmaxf(mx, half_swap(xaddr, mx));
     bias_piece(1);
     // The base of the exponentials follows the maximum lazily: it moves only when a tile's maximum
@@ -452,6 +457,218 @@ void flash_kernel(FlashArgs a) {
         *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(a.out) + off) = w;
       }
     }
+}
+
+// ------------------------------------------------------------------ heads of 48 over plain keys
+// The token transformer's attention: 16 heads of 48, an fp32 pair bias, keys as they stand.  At 100 to 768 tokens a SIMD has one
+// or two of its waves, each a chain of key tiles, so what counts is the length of the chain: the arithmetic is flash_kernel's,
+// in its order (the same bits), with less around it.  K, V and the bias come through range-checked loads (what lies past the
+// last key reads as zeros or as whatever the plane holds; its logits become -inf), so a tile that is not full costs nothing
+// more; a masked key's logit is replaced by what stands beside it in LDS (two instructions a logit instead of nine); a tile's
+// bias is asked for two tiles ahead, into the accumulators as the exponentials empty them, its K and V one tile ahead.
+// Of 8.8 us at 100 tokens flash_kernel spent 2.2 before its first tile, 4.4 in two tiles and 1.4 behind them.  us, flash_kernel /
+// this, 16 heads: 5 x 40 tokens 7.7 / 5.3, 5 x 100 9.2 / 6.7, 5 x 256 12.0 / 9.4, 5 x 384 15.4 / 12.1, 1 x 768 25.1 / 20.9,
+// 5 x 768 32.1 / 28.7, 5 x 1536 106 / 94.  (The keys of a query shared out between two waves, 128 registers, four waves to a
+// SIMD: no faster from 128 tokens on, 6.9 and 28.0 at 100 and 768, and other bits.)
+constexpr int TOK_D = 48, TOK_LDK = 56, TOK_LDV = 96;
+constexpr int TOK_K_BYTES = KT * TOK_LDK * 2, TOK_TILE = TOK_K_BYTES + KT * TOK_LDV * 2;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void token_attention_kernel(FlashArgs a) {
+  constexpr int CHUNKS = KT * (TOK_D / 8), NL = 2 * CHUNKS / 256;  // 16-byte pieces of a K (V) tile; of both, per thread
+  __shared__ __attribute__((aligned(16))) char sTile[2][TOK_TILE];  // [buffer]: K rows, V rows
+  __shared__ __attribute__((aligned(16))) float sRep[2][KT];        // what takes the place of a masked key's logit, or 0
+  __shared__ int sAny[2];                                           // whether it does for any key of the tile
+
+  const int tid = threadIdx.x, lane = tid & 63, hh = lane >> 5, j = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // flash_kernel's order of workgroups: logical = (head * query tiles + query tile) * B + batch
+  const int logical = (int)(blockIdx.x & 7) * a.per_xcd + (int)(blockIdx.x >> 3);
+  if (logical >= a.n_blocks) return;
+  const int rest = a.B == 1 ? logical : (int)__umulhi((uint32_t)logical, a.magic_b), b = logical - rest * a.B;
+  const int h = a.q_tiles == 1 ? rest : (int)__umulhi((uint32_t)rest, a.magic_t);
+  const int q0 = (rest - h * a.q_tiles) * 128 + wave * 32, qi = min(q0 + j, a.Sq - 1);  // clamped for loads; stores are guarded
+  const int nkt = (a.Sk + KT - 1) / KT;
+
+  auto rows_of = [&](const bf16_t* p, int64_t sb, int64_t ss) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p + b * sb + h * TOK_D), 0, (int)((a.Sk - 1) * ss + TOK_D) * 2, RSRC_RAW);
+  };
+  const __amdgpu_buffer_rsrc_t kres = rows_of(a.k, a.k_sb, a.k_ss), vres = rows_of(a.v, a.v_sb, a.v_ss);
+  const int quad_step = (int)(a.bias_squad ? a.bias_squad : 4), quads = (a.Sk + 3) >> 2;
+  const __amdgpu_buffer_rsrc_t bres = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(a.bias + (int64_t)b * a.bias_sb + (int64_t)h * a.bias_sh), 0,
+      ((a.Sq - 1) * (int)a.bias_sq + (quads - 1) * quad_step + 4) * 4, RSRC_RAW);
+  const float* kmask = a.key_mask ? a.key_mask + (int64_t)b * a.km_sb : nullptr;
+
+  // bias of a tile in four parts of two quads: part p = registers 8 p .. of the 32,
+  // s[u][4 g + e] = bias(query, key 64 kt + 32 u + 8 g + 4 hh + e)
+  const uint32_t bias_lane = (uint32_t)(qi * (int)a.bias_sq + hh * quad_step) * 4u;
+  auto load_bias = [&](f32x16 (&s)[2], int kt, int part) {
+    const int u = part >> 1;
+#pragma unroll
+    for (int g = 2 * (part & 1); g < 2 * (part & 1) + 2; ++g) {
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(bres, bias_lane, (kt * (KT / 4) + 8 * u + 2 * g) * quad_step * 4, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[u][4 * g + e] = __uint_as_float(v[e]);
+    }
+  };
+  // piece i of this thread: K pieces first, then V (which of the two is uniform over a wave: CHUNKS is a multiple of 64)
+  u32x4 rc[NL];
+  uint32_t choff[NL], lds_at[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int e = tid + i * 256;
+    const bool is_v = e >= CHUNKS;
+    const int ch = is_v ? e - CHUNKS : e, c = ch % (TOK_D / 8), key = ch / (TOK_D / 8);
+    choff[i] = (uint32_t)(key * (int)(is_v ? a.v_ss : a.k_ss) + c * 8) * 2u;
+    lds_at[i] = (is_v ? TOK_K_BYTES + key * (TOK_LDV * 2) : key * (TOK_LDK * 2)) + c * 16;
+  }
+  float mask_value = 1.f;  // of key tid of the tile asked for last (threads 0..63)
+  auto load_tile = [&](int kt) {
+    const int ks = kt * KT * (int)a.k_ss * 2, vs = kt * KT * (int)a.v_ss * 2;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      if (wave * 64 + i * 256 < CHUNKS) rc[i] = __builtin_amdgcn_raw_buffer_load_b128(kres, choff[i], ks, 0);
+      else rc[i] = __builtin_amdgcn_raw_buffer_load_b128(vres, choff[i], vs, 0);
+    }
+    if (kmask && tid < KT) mask_value = kmask[min(kt * KT + tid, a.Sk - 1)];
+  };
+  auto store_tile = [&](int kt) {
+    const int buf = kt & 1;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<u32x4*>(sTile[buf] + lds_at[i]) = rc[i];
+    if (tid < KT) {
+      const float rep = kt * KT + tid >= a.Sk ? NEG_INF : (mask_value == 0.f ? -1e9f : 0.f);
+      sRep[buf][tid] = rep;
+      const bool any = __any(rep != 0.f);
+      if (tid == 0) sAny[buf] = any ? 1 : 0;
+    }
+  };
+
+  f32x16 setA[2], setB[2];
+  bf16x8 qf[3];
+#pragma unroll
+  for (int ks = 0; ks < 3; ++ks)
+    qf[ks] = as_frag(*reinterpret_cast<const u32x4*>(a.q + (int64_t)b * a.q_sb + (int64_t)qi * a.q_ss + h * TOK_D + 16 * ks + 8 * hh));
+  load_tile(0);
+#pragma unroll
+  for (int p = 0; p < 4; ++p) load_bias(setA, 0, p);
+  // V's columns 48..63 of either buffer, which the products read
+  for (int idx = tid; idx < 2 * KT * 2; idx += 256) {
+    const int row = idx >> 1;
+    *reinterpret_cast<u32x4*>(sTile[row / KT] + TOK_K_BYTES + (row % KT) * (TOK_LDV * 2) + TOK_D * 2 + (idx & 1) * 16) = u32x4{0u, 0u, 0u, 0u};
+  }
+  f32x16 o[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+  float m_run = NEG_INF, l_run = 0.f;
+  const bf16x8 onesf = as_frag(u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+  store_tile(0);
+  load_tile(1);
+#pragma unroll
+  for (int p = 0; p < 4; ++p) load_bias(setB, 1, p);
+  lds_barrier();
+
+  auto tile = [&](int kt, f32x16 (&s)[2]) {
+    const int buf = kt & 1;
+    const char* kv = sTile[buf];
+#pragma unroll
+    for (int ks = 0; ks < 3; ++ks)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        s[u] = mfma32(lds_frag(reinterpret_cast<const bf16_t*>(kv), TOK_LDK, u * 32, ks * 16, lane), qf[ks], s[u]);
+    if (__builtin_amdgcn_readfirstlane(sAny[buf])) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const f32x4 rep = *reinterpret_cast<const f32x4*>(&sRep[buf][8 * q + 4 * hh]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[q >> 2][4 * (q & 3) + e] = rep[e] != 0.f ? rep[e] : s[q >> 2][4 * (q & 3) + e];
+      }
+    }
+    float mx = max3_of_32(s);
+    const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+    mx = fmaxf(__uint_as_float(r2[0]), __uint_as_float(r2[1]));
+    constexpr float BASE_SLACK = 8.f;  // see flash_kernel
+    const float m_new = mx - m_run > BASE_SLACK ? mx : m_run;
+    const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * LOG2E);
+    m_run = m_new;
+    const float m2 = m_new * LOG2E;
+    bf16x8 pf[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      float pv[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[p >> 1][8 * (p & 1) + e], LOG2E, -m2));
+      pf[p] = as_frag(pack8(pv));
+      __builtin_amdgcn_sched_barrier(0);
+      load_bias(s, kt + 2, p);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // row sums of the rounded probabilities (ones * P)
+    f32x16 lsum;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) lsum[r] = 0.f;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) lsum = mfma32(onesf, pf[p], lsum);
+    l_run = l_run * alpha + lsum[0];
+    if (__any(alpha != 1.f)) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+    }
+    // the transposing reads of V: see flash_kernel
+    const int i16 = lane & 15;
+    const bf16_t* vbase = reinterpret_cast<const bf16_t*>(kv + TOK_K_BYTES) + (4 * hh + (i16 >> 2)) * TOK_LDV + 16 * ((lane >> 4) & 1) + 4 * (i16 & 3);
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const bf16_t* vp = vbase + 16 * p * TOK_LDV + t * 32;
+        const v4s lo = lds_read_tr16(vp), hi = lds_read_tr16(vp + 8 * TOK_LDV);
+        o[t] = mfma32(as_frag(__builtin_bit_cast(u32x4, v8s{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w})), pf[p], o[t]);
+      }
+    if (kt + 1 < nkt) {
+      store_tile(kt + 1);
+      load_tile(kt + 2);
+    }
+    lds_barrier();
+  };
+  // the output gate: asked for in front of the last tile
+  u32x2 gate[6];
+  const int64_t row = qi;
+  auto load_gate = [&]() {
+#pragma unroll
+    for (int g = 0; g < 6; ++g) gate[g] = u32x2{0x3F803F80u, 0x3F803F80u};
+    if (!a.g) return;
+    const bf16_t* gp = a.g + (int64_t)b * a.g_sb + row * a.g_ss + h * TOK_D + 4 * hh;
+#pragma unroll
+    for (int g = 0; g < 6; ++g) gate[g] = *reinterpret_cast<const u32x2*>(gp + 8 * g);
+  };
+  load_gate();
+  for (int kt = 0; kt < nkt; kt += 2) {
+    tile(kt, setA);
+    if (kt + 1 < nkt) tile(kt + 1, setB);
+  }
+
+  const float inv = 1.f / l_run;
+  if (q0 + j >= a.Sq) return;
+  const int64_t at = (int64_t)b * a.o_sb + row * a.o_ss + h * TOK_D + 4 * hh;
+#pragma unroll
+  for (int g = 0; g < 6; ++g) {  // head dimensions 8 g + 4 hh ..
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = o[g >> 2][4 * (g & 3) + e] * inv;
+    v[0] *= bflo(gate[g].x); v[1] *= bfhi(gate[g].x); v[2] *= bflo(gate[g].y); v[3] *= bfhi(gate[g].y);
+    if (a.out_f32) {
+      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + at + 8 * g) = f32x4{v[0], v[1], v[2], v[3]};
+    } else {
+      u32x2 w;
+      w.x = pack2bf(v[0], v[1]);
+      w.y = pack2bf(v[2], v[3]);
+      *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(a.out) + at + 8 * g) = w;
+    }
+  }
 }
 
 // ------------------------------------------------------------------ windows of gathered keys
@@ -688,13 +905,27 @@ int launch_nw(const FlashArgs& a, hipStream_t stream) {
                     a.k_ss > 0 && a.v_ss > 0 && a.k_ss < (1 << 22) && a.v_ss < (1 << 22) && a.bias_sq >= 0 &&
                     quad_step > 0 && (int64_t)a.Sq * a.bias_sq + quad_step < (1 << 28);
   // Four waves share each staged K / V tile once there are enough 128-query workgroups to cover the chip; below that, two
-  // waves per workgroup spread the work over twice as many CUs.  Not with head dimension 48, where the form with fixed
-  // offsets needs four waves to share the staging registers: it is faster than twice the workgroups of the general form
-  // (16 heads x 48, 5 samples of 100, 200, 384 tokens, projections included: 18.4 us for 18.6, 25.2 for 28.7, 32.1 for 37.9).
+  // waves per workgroup spread the work over twice as many CUs.  Not with head dimension 48 (and padding flags: without them
+  // token_attention_kernel has it), where the form with fixed offsets needs four waves to share the staging registers.
   const int nw = a.Sq <= 32 ? 1 : (((a.Sq + 127) / 128) * heads < 256 && !(KSTEPS == 3 && fast) ? 2 : 4);
   const int64_t n_blocks = (int64_t)((a.Sq + nw * 32 - 1) / (nw * 32)) * heads;
   if (n_blocks <= 0 || n_blocks > 0x7ffffff0) return AF3_ERR_BAD_ARG;
   FlashArgs fa = a;
+  if constexpr (KSTEPS == 3) {
+    // (byte offsets of 31 bits inside a sample's rows and a head's bias plane, two tiles past the end included; products of the
+    // workgroups' numbers and their divisors of 32)
+    const int64_t keys = (a.Sk + 191) / 64 * 64, limit = (int64_t)1 << 29, tiles = (a.Sq + 127) / 128, blocks = tiles * heads;
+    if (fast && !a.qpad && keys * (a.k_ss > a.v_ss ? a.k_ss : a.v_ss) < limit && (int64_t)a.Sq * a.bias_sq + (keys / 4) * quad_step < limit &&
+        blocks * a.B < (1ll << 32) && blocks * tiles < (1ll << 32)) {
+      fa.n_blocks = (int)blocks;
+      fa.per_xcd = (int)((blocks + 7) / 8);
+      fa.q_tiles = (int)tiles;
+      fa.magic_b = a.B == 1 ? 0u : 0xffffffffu / (uint32_t)a.B + 1u;
+      fa.magic_t = tiles == 1 ? 0u : 0xffffffffu / (uint32_t)tiles + 1u;
+      hipLaunchKernelGGL(token_attention_kernel, dim3(8u * fa.per_xcd), dim3(256), 0, stream, fa);
+      return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+    }
+  }
   fa.n_blocks = (int)n_blocks;
   const dim3 grid((unsigned)((n_blocks + 7) / 8 * 8));  // whole rounds over the 8 XCDs; the surplus ids return at once
   // (with a single wave, or with head dimension 48 and fewer than four waves, to share the K / V staging

@@ -311,6 +311,8 @@ struct FlashArgs {
   // negative row is a key with zero K and V.  Null: key s is row s of batch b.
   const int* key_rows = nullptr;
   int64_t table_rows = 0;  // rows of a sample's table: every entry of key_rows is below this
+  int per_xcd = 0, q_tiles = 0;  // (these and the magic numbers of their divisions by the launcher)
+  unsigned magic_b = 0, magic_t = 0;
   int n_blocks = 0;  // workgroups that have work (set by the launcher; the grid is rounded up to a multiple of 8)
 };
 int launch_flash_attention(const FlashArgs& a, hipStream_t stream);
