@@ -461,6 +461,23 @@ struct GatedProductArgs {
   const float* gate = nullptr;              // [cond_rows][ld_gate]
   int64_t ld_gate = 0;
 };
+// The products of the token transformer's blocks over any number of rows, [rows][K], w in fragment order: with `gate` into `out`
+// as above; N = 4 x 768 columns of queries (bias, scale), keys, values, gate (sigmoid), K = 768; or with swiglu N / 2 hidden units.
+struct RowsProductArgs {
+  int m_chunk = 0, n_chunk = 0, xcd_m = 0, xcd_shift = 0;  // (these and the magic numbers by launch_rows_product)
+  unsigned magic_chunk = 0, magic_cond = 0;
+  int rows = 0, N = 0, K = 0, swiglu = 0, cond_rows = 0;
+  const bf16_t *x = nullptr, *w = nullptr;
+  bf16_t* out = nullptr;
+  int64_t ldc = 0;
+  const float* q_bias = nullptr;
+  float q_scale = 1.f;
+  const float* gate = nullptr;
+  int64_t ld_gate = 0;
+};
+bool rows_product_applies(const RowsProductArgs& a);
+bool rows_product_better(const RowsProductArgs& a);  // ... and faster than af3_linear_forward's kernels
+int launch_rows_product(const RowsProductArgs& a, hipStream_t s);
 bool gated_product_applies(const GatedProductArgs& a);
 int launch_gated_product(const GatedProductArgs& a, hipStream_t s);
 bool norm_product_applies(const NormProductArgs& a);

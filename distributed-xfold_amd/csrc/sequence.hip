@@ -486,7 +486,7 @@ int af3_diffusion_transformer_forward(
     const float* scale_shift, const float* gate, int64_t cond_rows, void* workspace, size_t workspace_bytes,
     af3_stream_t stream) {
   if (!blocks || num_blocks <= 0 || !act || !pair_logits || !scale_shift || !gate || cond_rows <= 0 || batch <= 0 || seq <= 0 ||
-      channels <= 0 || hidden <= 0)
+      channels <= 0 || hidden <= 0 || num_head <= 0 || channels % num_head)
     return AF3_ERR_BAD_ARG;
   const int c = channels;
   const int64_t rows = batch * seq, ld_ss = (int64_t)2 * num_blocks * 2 * c, ld_g = (int64_t)2 * num_blocks * c;
@@ -515,7 +515,6 @@ int af3_diffusion_transformer_forward(
   };
   // The norm and the product behind it in one kernel, where all blocks' weights are there in its order; it warms what the kernels
   // up to the next one read, the next one's weights among it.
-  const int nh = num_head > 0 ? num_head : 1;
   bf16_t* const qkvg = self_projections(aw, ab, rows, c);
   const bool act_ok = act_dtype == AF3_BF16 && c == TOKEN_STEP_CHANNELS && cond_rows == seq && rows <= 0x7fffffff;
   auto step = [&](int i, bool transition) {
@@ -526,59 +525,91 @@ int af3_diffusion_transformer_forward(
     a.w = b.frags ? b.frags + (transition ? (int64_t)4 * c * c : 0) : nullptr;
     a.swiglu = transition; a.N = transition ? 2 * hidden : 4 * c; a.ldc = transition ? hidden : 4 * c;
     a.out = transition ? y : qkvg;
-    if (!transition) { a.q_bias = b.q_b; a.q_scale = 1.0f / sqrtf((float)(c / nh)); }
+    if (!transition) { a.q_bias = b.q_b; a.q_scale = 1.0f / sqrtf((float)(c / num_head)); }
     return a;
   };
-  auto back = [&](int i, bool transition) {  // the product behind either, with its gate, into the stream
+  // Where the norm stands by itself, the products that token_step.hip takes over any number of rows.
+  auto product = [&](int i, bool transition) {
     const af3_diffusion_block& b = blocks[i];
-    GatedProductArgs a;
-    a.rows = (int)rows; a.K = transition ? hidden : c; a.cond_rows = (int)cond_rows; a.y = y; a.act = static_cast<bf16_t*>(act);
-    a.w = b.frags ? b.frags + (int64_t)(transition ? 5 * c + 2 * hidden : 4 * c + 2 * hidden) * c : nullptr;
-    a.gate = gate + ((int64_t)2 * i + transition) * c; a.ld_gate = ld_g;
+    RowsProductArgs a;
+    a.rows = (int)rows; a.x = reinterpret_cast<const bf16_t*>(x); a.K = c; a.swiglu = transition; a.N = transition ? 2 * hidden : 4 * c;
+    a.ldc = transition ? hidden : 4 * c; a.out = transition ? reinterpret_cast<bf16_t*>(y) : qkvg;
+    a.w = act_ok && b.frags ? b.frags + (transition ? (int64_t)4 * c * c : 0) : nullptr;
+    if (!transition) { a.q_bias = b.q_b; a.q_scale = 1.0f / sqrtf((float)(c / num_head)); }
     return a;
   };
-  bool steps = act_ok && qkvg && c % nh == 0;
+  // The product behind either, with its gate, into the stream.
+  auto back = [&](int i, bool transition) {
+    const af3_diffusion_block& b = blocks[i];
+    RowsProductArgs a;
+    a.rows = (int)rows; a.x = reinterpret_cast<const bf16_t*>(y); a.N = c; a.K = transition ? hidden : c; a.ldc = c;
+    a.out = static_cast<bf16_t*>(act); a.gate = gate + ((int64_t)2 * i + transition) * c; a.ld_gate = ld_g; a.cond_rows = (int)cond_rows;
+    a.w = act_ok && b.frags ? b.frags + (int64_t)(transition ? 5 * c + 2 * hidden : 4 * c + 2 * hidden) * c : nullptr;
+    return a;
+  };
+  auto few_rows = [](const RowsProductArgs& r) {
+    GatedProductArgs a;
+    a.rows = r.rows; a.K = r.K; a.cond_rows = r.cond_rows; a.y = r.x; a.act = r.out; a.w = r.w; a.gate = r.gate; a.ld_gate = r.ld_gate;
+    return a;
+  };
+  // (the fragments that product_back reads, or the weights as they were given)
+  auto weights_back = [&](int i, bool transition) -> const void* {
+    const RowsProductArgs a = back(i, transition);
+    return gated_product_applies(few_rows(a)) || rows_product_better(a) ? (const void*)a.w : transition ? blocks[i].w_tr2 : blocks[i].w_out;
+  };
+  auto product_back = [&](int i, bool transition) -> int {
+    const RowsProductArgs a = back(i, transition);
+    const GatedProductArgs few = few_rows(a);
+    if (gated_product_applies(few)) return launch_gated_product(few, static_cast<hipStream_t>(stream));
+    if (rows_product_better(a)) return launch_rows_product(a, static_cast<hipStream_t>(stream));
+    const af3_diffusion_block& b = blocks[i];
+    return af3_linear_forward(y, transition ? b.w_tr2 : b.w_out, nullptr, act, act_dtype, rows, c, transition ? hidden : c,
+                              AF3_LINEAR_GATE_RES, 1.f, 0, gate + ((int64_t)2 * i + transition) * c, cond_rows, ld_g, act, act_dtype, stream);
+  };
+  bool steps = act_ok && qkvg;
   for (int i = 0; i < num_blocks && steps; ++i) steps = norm_product_applies(step(i, false)) && norm_product_applies(step(i, true));
   if (bias_quad_major != 0 && (bias_quad_major != 1 || (seq & 3))) return AF3_ERR_BAD_ARG;
   const size_t all_logits = (size_t)num_head * seq * seq * 4, logit_bytes = all_logits <= WARM_LOGIT_BYTES ? all_logits : 0;
   for (int i = 0; i < num_blocks; ++i) {
     const af3_diffusion_block& b = blocks[i];
-    const float *ss = scale_shift + (int64_t)2 * i * 2 * c, *g = gate + (int64_t)2 * i * c;
+    const float* ss = scale_shift + (int64_t)2 * i * 2 * c;
     if (steps) {
       auto warm = [](NormProductArgs& a, int k, const void* p, size_t bytes) { a.warm[k] = p; a.warm_lines[k] = (uint32_t)(bytes / 128); };
       NormProductArgs a = step(i, false);
-      const GatedProductArgs out = back(i, false), down = back(i, true);
-      const bool out_step = gated_product_applies(out), down_step = gated_product_applies(down);
-      warm(a, 0, out_step ? out.w : b.w_out, (size_t)c * c * 2);
+      warm(a, 0, weights_back(i, false), (size_t)c * c * 2);
       warm(a, 1, b.frags + (int64_t)4 * c * c, (size_t)2 * hidden * c * 2);
       warm(a, 2, pair_logits[i], logit_bytes);
       STEP(launch_norm_product(a, static_cast<hipStream_t>(stream)));
       STEP(run_self_attend(qkvg, key_mask, 1, pair_logits[i], bias_quad_major, num_head, y, AF3_BF16, batch, seq, c,
                            static_cast<hipStream_t>(stream)));
-      if (out_step) STEP(launch_gated_product(out, static_cast<hipStream_t>(stream)));
-      else
-        STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, cond_rows, ld_g, act,
-                                act_dtype, stream));
+      STEP(product_back(i, false));
       a = step(i, true);
-      warm(a, 0, down_step ? down.w : b.w_tr2, (size_t)hidden * c * 2);
+      warm(a, 0, weights_back(i, true), (size_t)hidden * c * 2);
       if (i + 1 < num_blocks) warm(a, 1, blocks[i + 1].frags, (size_t)4 * c * c * 2);
       STEP(launch_norm_product(a, static_cast<hipStream_t>(stream)));
-      if (down_step) STEP(launch_gated_product(down, static_cast<hipStream_t>(stream)));
-      else
-        STEP(af3_linear_forward(y, b.w_tr2, nullptr, act, act_dtype, rows, c, hidden, AF3_LINEAR_GATE_RES, 1.f, 0, g + c, cond_rows,
-                                ld_g, act, act_dtype, stream));
+      STEP(product_back(i, true));
       continue;
     }
-    STEP(norm(ss, {b.w_q, (size_t)4 * c * c * 2}, {b.w_out, (size_t)c * c * 2}, {pair_logits[i], logit_bytes}));
-    STEP(af3_batch_diffusion_self_attention_forward(x, key_mask, 1, pair_logits[i], bias_quad_major, b.w_q, b.q_b, num_head, y,
-                                                    AF3_BF16, batch, seq, c, aw, ab, stream));
-    STEP(af3_linear_forward(y, b.w_out, nullptr, act, act_dtype, rows, c, c, AF3_LINEAR_GATE_RES, 1.f, 0, g, cond_rows, ld_g, act,
-                            act_dtype, stream));
-    STEP(norm(ss + 2 * c, {b.w_tr1, (size_t)2 * hidden * c * 2}, {b.w_tr2, (size_t)hidden * c * 2}, {nullptr, 0}));
-    STEP(af3_linear_forward(x, b.w_tr1, nullptr, y, AF3_BF16, rows, 2 * hidden, c, AF3_LINEAR_SWIGLU, 1.f, 0, nullptr, 0, 0, nullptr, 0,
-                            stream));
-    STEP(af3_linear_forward(y, b.w_tr2, nullptr, act, act_dtype, rows, c, hidden, AF3_LINEAR_GATE_RES, 1.f, 0, g + c, cond_rows, ld_g,
-                            act, act_dtype, stream));
+    const RowsProductArgs in = product(i, false), hidden_in = product(i, true);
+    const bool in_rows = qkvg && rows_product_better(in), hidden_rows = rows_product_better(hidden_in);
+    STEP(norm(ss, {in_rows ? (const void*)in.w : b.w_q, (size_t)4 * c * c * 2}, {weights_back(i, false), (size_t)c * c * 2},
+              {pair_logits[i], logit_bytes}));
+    if (in_rows) {
+      STEP(launch_rows_product(in, static_cast<hipStream_t>(stream)));
+      STEP(run_self_attend(qkvg, key_mask, 1, pair_logits[i], bias_quad_major, num_head, y, AF3_BF16, batch, seq, c,
+                           static_cast<hipStream_t>(stream)));
+    } else {
+      STEP(af3_batch_diffusion_self_attention_forward(x, key_mask, 1, pair_logits[i], bias_quad_major, b.w_q, b.q_b, num_head, y,
+                                                      AF3_BF16, batch, seq, c, aw, ab, stream));
+    }
+    STEP(product_back(i, false));
+    STEP(norm(ss + 2 * c, {hidden_rows ? (const void*)hidden_in.w : b.w_tr1, (size_t)2 * hidden * c * 2},
+              {weights_back(i, true), (size_t)hidden * c * 2}, {nullptr, 0}));
+    if (hidden_rows) STEP(launch_rows_product(hidden_in, static_cast<hipStream_t>(stream)));
+    else
+      STEP(af3_linear_forward(x, b.w_tr1, nullptr, y, AF3_BF16, rows, 2 * hidden, c, AF3_LINEAR_SWIGLU, 1.f, 0, nullptr, 0, 0, nullptr, 0,
+                              stream));
+    STEP(product_back(i, true));
   }
   return AF3_OK;
 }

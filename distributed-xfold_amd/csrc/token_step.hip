@@ -17,6 +17,7 @@
 // 1080, 5 x 40 1136 / 981, 5 x 100 1330 / 1132, 5 x 126 1424 / 1335.  Past one workgroup to a CU the twelvefold norms cost
 // more than they save: 5 x 160 1539 / 1529, 5 x 250 1928 / 2091, 5 x 384 2062 / 2483.
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "kernels.h"
@@ -340,6 +341,157 @@ __global__ __launch_bounds__(64 * WAVES, 1) void gated_product_kernel(GatedProdu
   }
 }
 
+// The same products over more rows: x w^T with the weights' fragments straight from memory to registers and the rows through LDS.
+// A workgroup takes 64 rows x 128 columns, a wave all rows of 32 columns; slabs of 64 channels of the rows go straight into a ring
+// of LDS buffers that the four waves share, with one barrier a slab; a wave's fragments are RING slabs ahead.
+enum { ROWS_QKVG, ROWS_SWIGLU, ROWS_GATED };
+constexpr int RP_BM = 64, RP_BN = 128, RP_BUFFERS = 4, RP_RING = 4, RP_PER_CU = 3;
+static_assert(RP_RING >= RP_BUFFERS);  // (rows_product_younger counts on it)
+// loads of a wave issued behind its two for slab s of the rows, when it waits for these (step s - 1 of the loop)
+constexpr int rows_product_younger(int s, int slabs) {
+  int n = 0;
+  auto steps = [&](int from) {
+    for (int i = from; i < s - 1; ++i) n += (i + RP_BUFFERS < slabs ? 2 : 0) + (i + RP_RING < slabs ? 4 : 0);
+  };
+  if (s < RP_BUFFERS) {
+    n += 2 * (RP_BUFFERS - 1 - s) + 4 * (RP_RING - s);
+    steps(0);
+  } else {
+    n += s - RP_BUFFERS + RP_RING < slabs ? 4 : 0;
+    steps(s - RP_BUFFERS + 1);
+  }
+  return n < 63 ? n : 63;
+}
+template <typename F, int... I>
+__device__ __forceinline__ void each(F f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+template <int SLABS, int KIND>
+__global__ __launch_bounds__(256, RP_PER_CU) void rows_product_kernel(RowsProductArgs a) {
+  constexpr int KK = 64 * SLABS, BUF = RP_BM * 128;
+  __shared__ __attribute__((aligned(1024))) char sA[RP_BUFFERS * BUF];
+  const int lane = threadIdx.x & 63, hh = lane >> 5, j = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // XCD (i, k) of a grid of xcd_m x 8 / xcd_m takes a rectangle of m_chunk x n_chunk tiles, row tiles fastest
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int sn = a.m_chunk == 1 ? slot : (int)__umulhi((uint32_t)slot, a.magic_chunk);
+  const int tm = (xcd & (a.xcd_m - 1)) * a.m_chunk + slot - sn * a.m_chunk, tn = (xcd >> a.xcd_shift) * a.n_chunk + sn;
+  if (tm * RP_BM >= a.rows || tn * RP_BN >= a.N) return;
+  const int m0 = tm * RP_BM, blk = tn * (RP_BN / 32) + wave;
+
+  const bf16_t* const x = a.x + (int64_t)m0 * KK;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)sA + 2048 * wave;
+  uint32_t off[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 8 * (2 * wave + i) + (lane >> 3);
+    off[i] = (uint32_t)(min(row, a.rows - 1 - m0) * KK + ((lane & 7) ^ ((row >> 1) & 7)) * 8) * 2u;
+  }
+  auto bring = [&](auto s_c) {
+    constexpr int s = decltype(s_c)::value;
+    if constexpr (s < SLABS) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        load_to_lds(x + 64 * s, off[i], __builtin_amdgcn_readfirstlane(lds0 + (s % RP_BUFFERS) * BUF + 1024 * i));
+    }
+  };
+  bf16x8 w[RP_RING][4];
+  auto fetch = [&](auto s_c) {
+    constexpr int s = decltype(s_c)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (s < SLABS) load_frags<4>(a.w, blk, KK / 16, 4 * s, lane, w[s % RP_RING]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#define SLAB(n) std::integral_constant<int, (n)>{}
+  each([&](auto s_c) {
+    constexpr int s = decltype(s_c)::value;
+    if constexpr (s < RP_BUFFERS) bring(s_c);
+    fetch(s_c);
+  }, std::make_integer_sequence<int, RP_RING>{});
+
+  f32x16 acc[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+  bf16x8 xf[2][2][4];
+  auto rows = [&](auto s_c) {
+    constexpr int s = decltype(s_c)::value;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        xf[s & 1][t][ks] = as_frag(*reinterpret_cast<const u32x4*>(sA + (s % RP_BUFFERS) * BUF + (32 * t + j) * 128 +
+                                                                   (((2 * ks + hh) ^ ((j >> 1) & 7)) << 4)));
+  };
+  auto landed = [&](auto s_c) {  // slab s is in LDS, for every wave
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(rows_product_younger(decltype(s_c)::value, SLABS)) : "memory");
+    lds_barrier();
+  };
+  landed(SLAB(0));
+  rows(SLAB(0));
+  each([&](auto i_c) {
+    constexpr int i = decltype(i_c)::value;
+    if constexpr (i + 1 < SLABS) {
+      landed(SLAB(i + 1));  // (and every wave has slab i's fragments: its buffer is free)
+      bring(SLAB(i + RP_BUFFERS));
+      rows(SLAB(i + 1));
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[t] = mfma32(w[i % RP_RING][ks], xf[i & 1][t][ks], acc[t]);
+    fetch(SLAB(i + RP_RING));
+  }, std::make_integer_sequence<int, SLABS>{});
+#undef SLAB
+
+  // a lane's registers 8 u .. are columns 32 blk + 16 u + 8 hh .. of rows j and 32 + j (SwiGLU: both factors of hidden units
+  // 16 blk + 8 hh ..)
+  const int col = 32 * blk + 8 * hh, seg = tn / (K / RP_BN);
+  float bias[16];
+  if constexpr (KIND == ROWS_QKVG)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) load_param8(seg == 0 && a.q_bias ? a.q_bias + col + 16 * u : nullptr, 0.f, bias + 8 * u);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int row = m0 + 32 * t + j;
+    if (row >= a.rows) break;
+    bf16_t* const out = a.out + (int64_t)row * a.ldc;
+    float o[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[r] = acc[t][r];
+    if constexpr (KIND == ROWS_SWIGLU) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = o[e] * sigmoidf_(o[e]) * o[8 + e];
+      *reinterpret_cast<u32x4*>(out + 16 * blk + 8 * hh) = pack8(o);
+    } else if constexpr (KIND == ROWS_QKVG) {
+      if (seg == 0) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[r] = (o[r] + bias[r]) * a.q_scale;
+      } else if (seg == 3) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[r] = sigmoidf_(o[r]);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) *reinterpret_cast<u32x4*>(out + col + 16 * u) = pack8(o + 8 * u);
+    } else {
+      const int cond = row - (a.cond_rows == 1 ? row : (int)__umulhi((uint32_t)row, a.magic_cond)) * a.cond_rows;
+      const float* const gp = a.gate + (int64_t)cond * a.ld_gate + col;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        float g[8], r[8];
+        Elem<float>::load8(gp + 16 * u, g);
+        Elem<bf16_t>::load8(out + col + 16 * u, r);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[8 * u + e] = (o[8 * u + e] + 0.f) * g[e] + r[e];
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) *reinterpret_cast<u32x4*>(out + col + 16 * u) = pack8(o + 8 * u);
+    }
+  }
+}
+
 bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
@@ -410,5 +562,51 @@ int launch_gated_product(const GatedProductArgs& args, hipStream_t s) {
   if (a.K == 768) LAUNCH(6);
   else LAUNCH(12);
 #undef LAUNCH
+  return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+}
+
+bool rows_product_applies(const RowsProductArgs& a) {
+  return a.x && a.w && a.out && a.rows > 0 && a.rows < (1 << 20) && a.N > 0 && a.N % RP_BN == 0 && (a.K == 768 || a.K == 1536) &&
+         a.ldc % 8 == 0 && al16(a.x) && al16(a.w) && al16(a.out) && al16(a.q_bias) &&
+         (a.gate ? a.N == K && a.ldc == K && a.cond_rows > 0 && (int64_t)a.rows * a.cond_rows <= 0xffffffffll && a.ld_gate >= K && a.ld_gate % 4 == 0 && al16(a.gate)
+                 : a.K == K && (a.swiglu || a.N == 4 * K));
+}
+
+// Faster than the products of gemm.hip (us at these rows, those / this):
+//   queries, keys, values, gate  340: 8.5 / 5.9   700: 10.7 / 9.4  1280: 13.6 / 10.2  1920: 17.3 / 13.3  2560: 19.9 / 16.7
+//                                3000: 24.8 / 22.2  3840: 25.0 / 24.0  5000: 31.0 / 30.3  7680: 51.3 / 48.8
+//   SwiGLU                       340: 6.7 / 5.2  1280: 10.0 / 8.9  2560: 15.6 / 15.0  3000: 18.7 / 19.0  3840: 19.2 / 21.5  5000: 24.1 / 27.5
+//   768 gated                    700: 6.7 / 6.6  1280: 7.0 / 6.6  1920: 8.4 / 6.8  2560: 9.4 / 7.0  2730: 10.6 / 11.5  3840: 11.4 / 11.9
+//   1536 gated                   700: 9.0 / 9.1  1280: 9.2 / 9.1  1920: 11.9 / 9.7  2560: 13.5 / 10.3  2730: 16.7 / 17.3  3840: 17.8 / 17.2
+// A tile of half the rows fills the chip sooner and pays for it with twice the reads of the weights: up to the rows whose 768
+// columns are one tile to a CU.  The widest of them has so much work to hand out that finer tiles lose nothing further on.
+bool rows_product_better(const RowsProductArgs& a) {
+  return rows_product_applies(a) && ((!a.gate && !a.swiglu) || (a.rows + RP_BM - 1) / RP_BM * (K / RP_BN) <= CUS);
+}
+
+int launch_rows_product(const RowsProductArgs& args, hipStream_t s) {
+  if (!rows_product_applies(args)) return AF3_ERR_BAD_ARG;
+  RowsProductArgs a = args;
+  const int tiles_m = (a.rows + RP_BM - 1) / RP_BM, tiles_n = a.N / RP_BN, per_round = CUS / 8 * RP_PER_CU;
+  // the grid of XCDs with the fewest rounds of RP_PER_CU workgroups to a CU, and of those the one that fetches least
+  int64_t best = -1;
+  for (int m = 1, shift = 0; m <= 8; m *= 2, ++shift) {
+    const int mc = (tiles_m + m - 1) / m, nc = (tiles_n + 8 / m - 1) / (8 / m);
+    const int64_t cost = ((int64_t)(mc * nc + per_round - 1) / per_round << 32) + mc * RP_BM + nc * RP_BN;
+    if (best >= 0 && cost >= best) continue;
+    best = cost;
+    a.xcd_m = m; a.xcd_shift = shift; a.m_chunk = mc; a.n_chunk = nc;
+  }
+  a.magic_chunk = a.m_chunk == 1 ? 0u : 0xffffffffu / (uint32_t)a.m_chunk + 1u;
+  a.magic_cond = a.cond_rows <= 1 ? 0u : 0xffffffffu / (uint32_t)a.cond_rows + 1u;
+  const dim3 grid(8u * a.m_chunk * a.n_chunk), block(256);
+  if (a.gate) {
+    if (a.K == 768) hipLaunchKernelGGL((rows_product_kernel<12, ROWS_GATED>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((rows_product_kernel<24, ROWS_GATED>), grid, block, 0, s, a);
+  } else if (a.swiglu) {
+    hipLaunchKernelGGL((rows_product_kernel<12, ROWS_SWIGLU>), grid, block, 0, s, a);
+  } else {
+    hipLaunchKernelGGL((rows_product_kernel<12, ROWS_QKVG>), grid, block, 0, s, a);
+  }
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }

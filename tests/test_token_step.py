@@ -1,14 +1,17 @@
-"""The token transformer's norms and the products behind them in one kernel (token_step.hip) against the operators one by one."""
+"""The token transformer's kernels (token_step.hip) against the operators one by one."""
 
 import pytest
 import torch
 
 
 # tiles hold all samples of 4 to 16 tokens, by the number of samples and of tiles: one token, tiles that are filled and that are
-# not, both sizes of every number of samples, one number that has no such kernel, more tokens than it takes, weights of 6 to 18 tiles
+# not, both sizes of every number of samples, one number that has no such kernel, more tokens than it takes, weights of 6 to 18 tiles;
+# products over rows: a row and two past a tile of 64, the most that the gated product of few rows takes and one more, the most for
+# all three and one tile more
 @pytest.mark.gpu
 @pytest.mark.parametrize("samples,n,factor", [(1, 1, 2), (1, 33, 2), (1, 64, 1), (1, 200, 2), (1, 337, 2), (2, 17, 2), (2, 161, 1), (3, 31, 2),
-                                              (3, 155, 2), (4, 40, 3), (4, 81, 2), (5, 6, 2), (5, 77, 2), (5, 100, 2), (5, 130, 2), (6, 11, 2)])
+                                              (3, 155, 2), (4, 40, 3), (4, 81, 2), (5, 6, 2), (5, 77, 2), (5, 100, 2), (5, 130, 2), (6, 11, 2),
+                                              (6, 21, 2), (6, 112, 1), (6, 113, 2), (7, 384, 2), (7, 385, 2)])
 def test_the_steps_give_the_bits_of_the_operators(gpu_pkg, samples, n, factor):
     g = torch.Generator(device="cuda").manual_seed(100 * samples + n)
     rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
