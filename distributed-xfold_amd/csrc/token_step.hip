@@ -13,9 +13,9 @@
 // What bounds it: 0.45 MB of weights, rows and conditioning through the CU's vector memory path (64 bytes a cycle: 3.3 us at
 // 2.1 GHz) and the norms' vector instructions, 700 a row, which overlap but for their ends.  100 tokens of 5 samples, cycles of a
 // wave: rows there 3700, norms 6000, barrier 1500, product 3000, result 1000.  9.3 and 9.0 us against 5.1 + 9.9 and 5.1 + 8.2; a
-// token transformer of 24 blocks, us, separate kernels / this: 1 x 100 tokens 1174 / 1024, 1 x 304 1380 / 1304, 3 x 100 1228 /
-// 1080, 5 x 40 1136 / 981, 5 x 100 1330 / 1132, 5 x 126 1424 / 1335.  Past one workgroup to a CU the twelvefold norms cost
-// more than they save: 5 x 160 1539 / 1529, 5 x 250 1928 / 2091, 5 x 384 2062 / 2483.
+// token transformer of 24 blocks, us, norm and rows_product_kernel / this: 1 x 100 tokens 975 / 844, 1 x 256 1112 / 1038, 3 x 100
+// 1015 / 907, 4 x 128 1095 / 1031, 5 x 60 966 / 849, 5 x 100 1081 / 989, 5 x 126 1222 / 1194.  At one workgroup to a CU the
+// twelvefold norms cost what they save (3 x 200 1185 / 1197); past it, more.
 #include <type_traits>
 #include <utility>
 
@@ -343,7 +343,9 @@ __global__ __launch_bounds__(64 * WAVES, 1) void gated_product_kernel(GatedProdu
 
 // The same products over more rows: x w^T with the weights' fragments straight from memory to registers and the rows through LDS.
 // A workgroup takes 64 rows x 128 columns, a wave all rows of 32 columns; slabs of 64 channels of the rows go straight into a ring
-// of LDS buffers that the four waves share, with one barrier a slab; a wave's fragments are RING slabs ahead.
+// of LDS buffers that the four waves share, with one barrier a slab; a wave's fragments are RP_RING slabs ahead.  Bound by the CU's vector memory path: 3 KB of weights and rows
+// for 16 matrix instructions of a wave.  Three workgroups a CU with four slabs ahead, two with six to eight (us, queries to gate
+// at 640, 1920 and 3840 rows): 6.6 13.2 24.0, 6.8 13.4 24.3.
 enum { ROWS_QKVG, ROWS_SWIGLU, ROWS_GATED };
 constexpr int RP_BM = 64, RP_BN = 128, RP_BUFFERS = 4, RP_RING = 4, RP_PER_CU = 3;
 static_assert(RP_RING >= RP_BUFFERS);  // (rows_product_younger counts on it)
