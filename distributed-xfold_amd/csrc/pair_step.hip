@@ -1,9 +1,11 @@
-// Steps of the pair path, 128 channels at few tokens and 64 channels: the operators between two long products, one kernel.
+// Steps of the pair path: the operators between two long products, one kernel (128 channels up to the sizes that sequence.hip
+// sets, 64 channels throughout).
 //
 // Up to some two hundred tokens the pair tensor is a few hundred tiles of 128 positions, and a kernel of pair_tile.hip is
 // one tile's chain of loads, LayerNorm, products and stores, run by a part of the CUs while the rest idles: at 64 tokens
-// thirteen dependent launches of 4 to 16 us a block.  All but the contraction and the attention core work on a pixel at
-// a time, so here each run of them between two of those is one kernel, on tiles of 32 positions, four times as many:
+// thirteen dependent launches of 4 to 16 us a block.  Beyond, each of them is a pass over the tensor.  All but the contraction
+// and the attention core work on a pixel at a time, so here each run of them between two of those is one kernel, on tiles of 32
+// or 64 positions:
 //
 //   outgoing epilogue  + incoming prologue           (patches of 4 x 8 pixels: the one reads rows, the other writes columns)
 //   incoming epilogue  + starting-node projections   (rows)
@@ -17,19 +19,22 @@
 // is rounded where the operators of pair_tile.hip store it, so the values are the same.
 //
 // What bounds it: at 64 tokens (128 tiles, one to a CU) the tile's chain, in which a weight that is not in L2 yet costs a
-// trip to memory; with more tiles what each fetches of the weights (0.6 MB in the last step, from L2 at 140 B/ns and CU) and
-// vector issue.  Kernel alone, us (in brackets the kernels whose place it takes), at 64 / 160 tokens, bf16 stream:
-//   outgoing epilogue + incoming prologue 10.8 / 20.3 (11.6 + 6.7 / 12.3 + 13.2), in patches of 4 x 8 / 8 x 8 pixels
-//   incoming epilogue + projections 8.7 / 18.9 (11.6 + 7.7 / 12.3 + 13.5), output + projections 8.2 / 18.4 (10.0 + 7.7 / 10.7 + 13.5)
-//   output + transition + logits + prologue 14.3 / 35 (10.0 + 15.8 + 4.6 + 6.7 / 10.7 + 19.1 + 5.0 + 13.2)
+// trip to memory; with more tiles, and with a transition about equally, what a tile fetches of the weights (0.6 MB from L2 at
+// 140 B/ns and CU, 4.3 us), vector issue (3.2 us a tile of 32 positions) and the matrix unit (2.3), which overlap as far as
+// the waves of a SIMD do: 9.5 us a tile with two of them.  So the registers go to a third wave or to twice the positions for a
+// weight, and not to weights in flight: one or two pieces of 32 rows, where four (three with a transition) were no faster at 64
+// tokens and kept the third wave out.  Kernel alone, us, at 64 / 128 / 160 / 200 / 301 tokens, bf16 stream (128: fp32):
+//   outgoing epilogue + incoming prologue 10.4 / 17.8 / 21.1 / 33 / -, in patches of 4 x 8 / 8 x 8 pixels
+//   incoming epilogue + projections 7.9 / 15.5 / 19.1 / 24.5 / 42, output + projections 8.0 / 14.5 / 18.8 / 23.8 / 41
+//     (three and four pieces: 8.4 / 16.1 / 19.9 / 27.1 / 43, 8.2 / 14.9 / 19.2 / 25.9 / 41)
+//   output + transition + logits + prologue 13.9 / 22.7 / 31.6 / 47 / - (three pieces, tiles of 32: 14.1 / 22.9 / 36.4 / 53.4 / -)
 //
 // 64 channels (the template embedding): workgroups of two waves, otherwise the same code.  A quarter of the weights to a
 // position and half of the rest, so that here the steps are the faster form whatever the number of tokens, and the tensor
 // need not be padded to 128 channels and back (bf16, 301 tokens, us a block: 345 -> 221, 768: 1940 -> 1460; kernel alone
-// at 301, bound by what it moves, 25 to 40 MB, and vector issue: outgoing prologue 13, outgoing epilogue + incoming
-// prologue 31 (8 x 8 patches 36: twice the accumulators cost the third workgroup of a SIMD), the other steps 20 to 21).
-// Tiles of 64 positions (half the weights a position) run slower up to 128 tokens and no faster at 160 to 256, but for the
-// patches.
+// at 301, bound by what it moves, 25 to 40 MB, and vector issue, four waves to a SIMD / three with twice the weights in flight:
+// outgoing prologue 13.1 / 13.9, outgoing epilogue + incoming prologue 32.5 / 32.9 (8 x 8 patches 36), incoming epilogue +
+// projections 20.5 / 21.9, output + projections 20.1 / 20.6, output + transition 20.2 / 22.0).
 #include <type_traits>
 
 #include "common.h"
@@ -82,15 +87,19 @@ struct StepTile {
   }
 };
 
-template <typename TIO, int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT>
-__global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(PairStepArgs a) {
+// Pieces of the weights (32 rows) in flight: what the registers leave beside the waves of a SIMD.
+constexpr int pieces_in_flight(int ch, int pb, int waves, bool transition) {
+  return ch == 128 && transition && (pb == 2 || waves == 3) ? 1 : 2;
+}
+
+template <typename TIO, int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT, int PER_SIMD>
+__global__ __launch_bounds__(2 * CH, PER_SIMD) void pair_step_kernel(PairStepArgs a) {
   using E = Elem<TIO>;
   constexpr int TS = 32 * PB;           // positions per tile, in blocks of an MFMA's 32
   constexpr int C = CH, D = C / H, LDX = C + 8, LDS_F = C + 4;
   constexpr int WAVES = C / 32, NT = 2 * C, CHUNKS = C / 8, KS = C / 16;
   constexpr int HIDDEN_CHUNK = hidden_chunk_of(C), MAX_HIDDEN = HIDDEN_CHUNK * hidden_chunks(C);
-  static_assert(PB == 1 || !TRANSITION, "a transition's fragments and sums fit the registers at 32 positions only");
-  constexpr int NB = C == 64 || (PB == 1 && !TRANSITION) ? 4 : 3;  // pieces of the weights in flight
+  constexpr int NB = pieces_in_flight(C, PB, PER_SIMD, TRANSITION);
   // LDS row stride (bf16) of a channel's positions: the 16 lanes of a pixel, 8 channels apart, on 8 banks
   constexpr int LDT = TS + 2;
   constexpr int LDH = HIDDEN_CHUNK + 8;
@@ -215,9 +224,7 @@ __global__ __launch_bounds__(2 * CH, CH == 64 ? 3 : 2) void pair_step_kernel(Pai
   };
 #define OCTET(n) std::integral_constant<int, (n)>{}
   fetch(OCTET(0));
-  fetch(OCTET(1));
-  fetch(OCTET(2));
-  if constexpr (NB > 3) fetch(OCTET(3));
+  if constexpr (NB > 1) fetch(OCTET(1));
   // Weights further down the chain: the workgroups of an XCD between them touch every cache line once, so that the tiles,
   // which reach each stage at about the same time, find it in L2.
   uint32_t warm = 0u;
@@ -564,18 +571,29 @@ bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // Patches of 8 x 8 pixels from one workgroup per CU on: what a patch writes of a transposed operand is then whole 16-byte
 // pieces.
 constexpr int64_t WIDE_PATCHES = 256 * 64;
-// Projections behind an epilogue or an output in tiles of 64 positions: half of the weights' traffic, where there are tiles
-// enough; us, 32 / 64 positions, 301 tokens 48 / 45 (epilogue), 46 / 43 (output); 160 tokens 18.9 / 19.5, 18.4 / 18.6.
+// Projections behind an epilogue or an output in tiles of 64 positions: half of the weights' traffic, where there are rounds of
+// workgroups enough (two a CU against three); us, 32 / 64 positions, 160 tokens 19.1 / 19.5 (epilogue), 18.8 / 18.3 (output), 208
+// 24.6 / 27.0, 23.9 / 25.3, 240 30.5 / 29.3, 29.2 / 28.8, 301 44.0 / 41.8, 42.4 / 40.7, 400 68.6 / 64.3, 66.9 / 63.6.
 constexpr int64_t WIDE_ROWS = 208 * 208 + 1;
+// The steps with a transition: tiles of 32 positions, two or three workgroups to a CU, or tiles of 64 (half of the weights'
+// traffic), two to a CU, by the rounds that they make on 256 CUs; us, with the next prologue, two / three / wide: 128 tokens (512
+// tiles of 32) 22.8 / 23.2 / 25.0, 152 (760) 31.2 / 29.1 / 31.2, 160 (800) 36.4 / 36.0 / 31.6, 181 (1086, wide ones 543) 45.1 / 43.1 /
+// 46.7, 192 (1152) 45.8 / 42.8 / 46.6, 208 (1352) 52.7 / 49.3 / 48.2.
+enum TransitionForm { TWO_A_SIMD, THREE_A_SIMD, WIDE };
+TransitionForm transition_form(int64_t positions) {
+  const int64_t tiles = (positions + 31) / 32;
+  if (tiles <= 2 * 256) return TWO_A_SIMD;
+  return tiles <= 3 * 256 || (tiles > 4 * 256 && tiles <= 5 * 256) ? THREE_A_SIMD : WIDE;
+}
 
-template <int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT>
+template <int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT, int PER_SIMD = CH == 64 ? 4 : PB == 2 ? 2 : 3>
 int launch_tiles(const PairStepArgs& a, hipStream_t s) {
   const int64_t blocks = MAP == MAP_PATCH ? ((int64_t)(a.Np / (4 * PB)) * (a.Np / 8) + 7) / 8 * 8
                                           : ((int64_t)a.N * a.ldn + 32 * PB - 1) / (32 * PB);
   if (blocks <= 0 || blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
   const dim3 grid((unsigned)blocks), block(2 * CH);
-  if (a.io_f32) hipLaunchKernelGGL((pair_step_kernel<float, CH, PB, IN, MAP, TRANSITION, NEXT>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((pair_step_kernel<bf16_t, CH, PB, IN, MAP, TRANSITION, NEXT>), grid, block, 0, s, a);
+  if (a.io_f32) hipLaunchKernelGGL((pair_step_kernel<float, CH, PB, IN, MAP, TRANSITION, NEXT, PER_SIMD>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((pair_step_kernel<bf16_t, CH, PB, IN, MAP, TRANSITION, NEXT, PER_SIMD>), grid, block, 0, s, a);
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
 }  // namespace
@@ -600,6 +618,8 @@ int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s) {
     return AF3_ERR_BAD_ARG;
   if (a.logits && (a.channels != 128 || !transition || !a.f_logits || !a.sl_ln_w || !a.sl_ln_b || a.logit_heads <= 0))
     return AF3_ERR_BAD_ARG;
+  const int64_t positions = (int64_t)a.N * a.ldn;
+  const TransitionForm form = transition_form(positions);
   if (a.channels == 64) switch (step) {
     case PAIR_STEP_FIRST: return launch_tiles<64, 1, IN_NONE, MAP_ROWS, false, NEXT_PROLOGUE>(a, s);
     case PAIR_STEP_INCOMING: return launch_tiles<64, 1, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
@@ -613,13 +633,19 @@ int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s) {
       if ((int64_t)a.N * a.ldn >= WIDE_PATCHES) return launch_tiles<128, 2, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
       return launch_tiles<128, 1, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
     case PAIR_STEP_PROJECT_START:
-      if ((int64_t)a.N * a.ldn >= WIDE_ROWS) return launch_tiles<128, 2, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
+      if (positions >= WIDE_ROWS) return launch_tiles<128, 2, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
       return launch_tiles<128, 1, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
     case PAIR_STEP_PROJECT_END:
-      if ((int64_t)a.N * a.ldn >= WIDE_ROWS) return launch_tiles<128, 2, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
+      if (positions >= WIDE_ROWS) return launch_tiles<128, 2, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
       return launch_tiles<128, 1, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
-    case PAIR_STEP_LAST: return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_NONE>(a, s);
-    case PAIR_STEP_NEXT: return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_PROLOGUE>(a, s);
+    case PAIR_STEP_LAST:
+      if (form == TWO_A_SIMD) return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_NONE, 2>(a, s);
+      if (form == THREE_A_SIMD) return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_NONE>(a, s);
+      return launch_tiles<128, 2, IN_ATTENTION, MAP_ROWS, true, NEXT_NONE>(a, s);
+    case PAIR_STEP_NEXT:
+      if (form == TWO_A_SIMD) return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_PROLOGUE, 2>(a, s);
+      if (form == THREE_A_SIMD) return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_PROLOGUE>(a, s);
+      return launch_tiles<128, 2, IN_ATTENTION, MAP_ROWS, true, NEXT_PROLOGUE>(a, s);
   }
   return AF3_ERR_BAD_ARG;
 }

@@ -53,33 +53,30 @@ struct Event {
     if (rc_ != AF3_OK) return rc_; \
   } while (0)
 
-// ---- the pair operators at few tokens: a run of them between two long products in one kernel (pair_step.hip) ----
-// A step takes the chain of one tile of 32 positions where a kernel of its own per operator takes several of tiles of 128,
-// and eight launches a block take the place of thirteen; past some number of tiles what every tile fetches of the weights
-// costs more than that saves.  All three forms in turn, us a block: one kernel per operator / steps in part (below) / steps
-// throughout, in runs of 4 blocks on a bf16 and on an fp32 stream, and a single Evoformer block of 64 rows (bf16; its last
-// step makes no prologue for a next block):
-//    64 tokens  135 / 116 /  92    143 / 121 /  92    154 / 137 / 119
-//   128         164 / 148 / 121    169 / 151 / 120    199 / 184 / 168
-//   160         194 / 180 / 166    202 / 188 / 169    237 / 226 / 216
-//   192         236 / 219 / 202    250 / 233 / 211    287 / 271 / 264
-//   208         256 / 244 / 235    272 / 258 / 246    315 / 305 / 302
-//   224         265 / 256 / 252    286 / 274 / 264    324 / 315 / 319
-//   240         273 / 262 / 267    297 / 285 / 282    330 / 323 / 330
-// The line lies below the first size at which steps throughout are not the fastest form in every one of these (216 tokens, the
-// same number of tiles to a row as 224: still by 1 to 5 %).
+// ---- the pair operators in steps: a run of them between two long products in one kernel (pair_step.hip) ----
+// Few tokens: a step takes the chain of one tile of 32 or 64 positions where a kernel of its own per operator takes several of
+// tiles of 128, and eight launches a block take the place of thirteen.  Many tokens: a step saves the passes over the tensor that
+// its operators would make one by one, at the price of the weights, which every tile fetches anew; on an fp32 stream, whose passes
+// are twice the bytes, that pays for much longer.  us, kernels per operator (up to 400 tokens with the two steps that end in
+// projections) / steps: a stack of 4 blocks on a bf16 stream, one block on it, a stack of 4 on an fp32 stream
+//   209 tokens   948 / 897     288 / 277    1003 / 945
+//   301         1513 / 1452    431 / 419    1683 / 1560
+//   387         2518 / 2456    691 / 675    2817 / 2654
+//   512         3971 / 3914   1020 / 1033   4777 / 4333
+//   550         5298 / 5204   1361 / 1352   5990 / 5689
+//   600         6160 / 6233   1599 / 1609   7035 / 6789
+//   768         9686 / 9771   2469 / 2505  11183 / 10607;  3 blocks: 1024 19673 / 18762, 1280 33765 / 32302, 1536 52463 / 52510
 // Pair tensors of 64 channels have no other kernels (64 / 301 / 768 / 2048 tokens, bf16, a block on its own: 100 -> 46,
 // 345 -> 221, 1940 -> 1460, 22400 -> 18800 against one zero-padded to 128; their 32-bit offsets end at 3072).
-constexpr int64_t PAIR_STEP_POSITIONS = 208 * 208;
-// Beyond, the two steps that end in an attention's projections stay the faster form for a while (they only read the tensor's
-// rows as they lie, and half of a tile's weights): runs of 4 blocks, us a block, without -> with them (bf16 / fp32 stream),
-// 209 tokens 250 -> 239 / 267 -> 253, 301: 391 -> 384 / 442 -> 423, 340: 492 -> 481 / 561 -> 538, 400: 659 -> 644 /
-// 763 -> 734.  Past the line the gain gets smaller and depends on the machine: 420: 712 -> 699 or 714 -> 708, 450: 814 -> 805 or
-// 830 -> 835 on a bf16 stream.
-constexpr int64_t PROJECT_STEP_POSITIONS = 400 * 400;
-bool pair_steps_apply(const af3_pairformer_block& b, int64_t n, int64_t positions = PAIR_STEP_POSITIONS) {
+constexpr int64_t BF16_STEP_POSITIONS = 500 * 500, F32_STEP_POSITIONS = 1280 * 1280;
+// The outgoing epilogue and the incoming prologue are one step while its patches are one round of workgroups: it stores transposed
+// operands 8 or 16 bytes at a time, which costs more than the pass and the launch it saves beyond (a stack of 4 blocks, us, two
+// kernels / one: 128 tokens 495 / 474, 176 673 / 653, 192 735 / 742, 256 1036 / 1064, 387 2456 / 2535; fp32 stream 176 712 / 687).
+constexpr int64_t INCOMING_STEP_POSITIONS = 184 * 184;
+bool pair_steps_apply(const af3_pairformer_block& b, int64_t n, int dt) {
   const int c = b.pair_channels == 64 ? 64 : 128;
-  return b.pair_frags && n <= 8192 && (c == 64 ? n <= AF3_PAIR64_MAX_TOKENS : n * tri_ldn(n) <= positions) &&
+  return b.pair_frags && n <= 8192 &&
+         (c == 64 ? n <= AF3_PAIR64_MAX_TOKENS : n * tri_ldn(n) <= (dt == AF3_F32 ? F32_STEP_POSITIONS : BF16_STEP_POSITIONS)) &&
          b.num_head_pair == 4 && b.valid_channels >= 8 && b.valid_channels <= c && b.valid_channels % 4 == 0 &&
          (c == 128 || b.valid_channels == 64) && b.pair_hidden > 0 && b.pair_hidden % 64 == 0 &&
          b.pair_hidden <= pair_step_max_hidden(c);
@@ -92,13 +89,14 @@ struct PairStepScratch {
   static size_t vt_bytes(int64_t n, int c) { return (size_t)n * c * tri_ldn(n) * 2; }
   static size_t bytes(int64_t n, int c) {
     return 3 * align_up(plane_bytes(n, c)) + align_up(vt_bytes(n, c)) + align_up((size_t)tri_bias_elems(n, 4) * 2) +
-           (c == 128 && n * tri_ldn(n) <= PAIR_STEP_POSITIONS ? LOGIT_RING * logit_bytes(n, 16) : 0);
+           (c == 128 && n * tri_ldn(n) <= LOGIT_RING_POSITIONS ? LOGIT_RING * logit_bytes(n, 16) : 0);
   }
   // Pair logits of the last blocks, where the single track runs on a stream of its own.  With two buffers every block waits
   // for the attention two blocks back, and an event costs the host some 20 us (recorded 3, waited for 15 to 17), where a launch
   // costs 2.7 to 3.7: at 64 tokens the launches set the pace.  With eight it is one wait in four blocks (runs of 4 blocks, us a
   // block: 93 -> 83).
   static constexpr int LOGIT_RING = 8;
+  static constexpr int64_t LOGIT_RING_POSITIONS = 208 * 208;  // (beyond, the kernels set the pace)
   static size_t logit_bytes(int64_t n, int heads) { return align_up((size_t)heads * n * ((n + 3) / 4 * 4) * 4); }
   float* ring(int64_t n) const {
     return reinterpret_cast<float*>(reinterpret_cast<char*>(bias) + align_up((size_t)tri_bias_elems(n, 4) * 2));
@@ -114,10 +112,10 @@ struct PairStepScratch {
   }
 };
 
-// One block's pair operators.  `partly`: in steps only where an attention's projections are the second half.  `first`: no
-// step before has made the outgoing prologue.  `next`: the block whose outgoing prologue the last step makes, or null.
+// One block's pair operators.  `first`: no step before has made the outgoing prologue.  `next`: the block whose outgoing prologue
+// the last step makes, or null.
 // `logits`: where the pair logits of the single track go, or null; they are written behind `logits_free`.
-int pair_operators_in_steps(const af3_pairformer_block& b, bool partly, const af3_pairformer_block* next, bool first, void* pair, int dt,
+int pair_operators_in_steps(const af3_pairformer_block& b, const af3_pairformer_block* next, bool first, void* pair, int dt,
                             const float* mask, const float* mask_in, int64_t n, void* ws, size_t wsb, float* logits,
                             Event* logits_free, hipStream_t s) {
   if (!pair || (dt != AF3_F32 && dt != AF3_BF16) || ((uintptr_t)pair & 15) || ((uintptr_t)mask & 15) || ((uintptr_t)mask_in & 15))
@@ -162,7 +160,7 @@ int pair_operators_in_steps(const af3_pairformer_block& b, bool partly, const af
     STEP(run_triangle_contraction(w.qa, w.kb, w.ogt, (int)n, c, d == 0, s));
     a.ln1_w = b.tm_ln_in_w[d]; a.ln1_b = b.tm_ln_in_b[d]; a.f_gate = tm(b, d, 0); a.f_out = tm(b, d, 1);
     a.ln_c_w = b.tm_ln_c_w[d]; a.ln_c_b = b.tm_ln_c_b[d];
-    if (d == 0 && partly) {
+    if (d == 0 && wide == 128 && n * tri_ldn(n) > INCOMING_STEP_POSITIONS) {
       STEP(launch_trimul_epilogue(product(0), s));
       STEP(launch_trimul_prologue(product(1), s));
     } else if (d == 0) {
@@ -178,14 +176,6 @@ int pair_operators_in_steps(const af3_pairformer_block& b, bool partly, const af
   a.ln3_w = b.ta_ln_w[1]; a.ln3_b = b.ta_ln_b[1]; a.f_next = qkg(1, 0); a.f_v = ta(1, 0);
   STEP(launch_pair_step(a, PAIR_STEP_PROJECT_END, s));
   STEP(launch_triattn_flash(core, s));
-  if (partly) {
-    AttnOutArgs o;
-    o.lw = a.lw; o.og = w.ogt; o.ld_og = 128; o.w_gate = b.ta_w_qkvg[1] + 3 * 128 * 128; o.w_out = b.ta_w_out[1];
-    o.pair = o.out = pair; o.ln_w = b.ta_ln_w[1]; o.ln_b = b.ta_ln_b[1];
-    o.io_f32 = a.io_f32; o.N = a.N; o.transpose = o.residual = 1;
-    STEP(launch_attn_out(o, s));
-    return af3_transition_forward_padded(pair, dt, b.pt_ln_w, b.pt_ln_b, b.pt_w1, b.pt_w2, hidden, pair, 1, n * n, c, s);
-  }
   a.ln1_w = b.ta_ln_w[1]; a.ln1_b = b.ta_ln_b[1]; a.f_gate = qkg(1, 2); a.f_out = ta(1, wide + 32);
   a.ln2_w = b.pt_ln_w; a.ln2_b = b.pt_ln_b; a.f_w1 = w1; a.f_w2 = w1 + (2 * hidden + logit_rows) * wide;
   if (logits) {
@@ -197,11 +187,11 @@ int pair_operators_in_steps(const af3_pairformer_block& b, bool partly, const af
   return launch_pair_step(a, PAIR_STEP_NEXT, s);
 }
 
-// every operator in a kernel of its own, or nearly
+// one block by itself
 int pair_operators(const af3_pairformer_block& b, void* pair, int dt, const float* mask, const float* mask_in, int64_t n,
                    void* ws, size_t wsb, hipStream_t s) {
-  if (pair_steps_apply(b, n, PROJECT_STEP_POSITIONS))
-    return pair_operators_in_steps(b, true, nullptr, true, pair, dt, mask, mask_in, n, ws, wsb, nullptr, nullptr, s);
+  if (pair_steps_apply(b, n, dt))
+    return pair_operators_in_steps(b, nullptr, true, pair, dt, mask, mask_in, n, ws, wsb, nullptr, nullptr, s);
   for (int d = 0; d < 2; ++d)
     STEP(af3_triangle_multiplication_forward_padded(pair, dt, d == 1 && mask_in ? mask_in : mask, d, b.tm_ln_in_w[d], b.tm_ln_in_b[d],
                                                     b.tm_w_proj_gate[d], b.tm_ln_c_w[d], b.tm_ln_c_b[d], b.tm_w_out[d],
@@ -371,12 +361,7 @@ int af3_evoformer_stack_forward(const af3_msa_block* const* blocks, int num_bloc
     msa_attention_args(b, avg, u);
     msa_transition_args(b.mt_ln_w, b.mt_ln_b, b.mt_w1, b.mt_w2, b.mt_hidden, u);
     STEP(launch_msa_update(u, s));
-    if (pair_steps_apply(b.pair, n))
-      STEP(pair_operators_in_steps(b.pair, false, nullptr, true, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n,
-                                   pair_workspace, pair_workspace_bytes, nullptr, nullptr, s));
-    else
-      STEP(pair_operators(b.pair, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace,
-                          pair_workspace_bytes, s));
+    STEP(pair_operators(b.pair, pair, pair_dtype, pair_mask, pair_mask ? mask_in : nullptr, n, pair_workspace, pair_workspace_bytes, s));
   }
   return AF3_OK;
 }
@@ -384,7 +369,7 @@ int af3_evoformer_stack_forward(const af3_msa_block* const* blocks, int num_bloc
 size_t af3_pairformer_stack_workspace_bytes(int64_t n, int num_head_pair) {
   const size_t a = af3_triangle_multiplication_workspace_bytes(n), b = af3_grid_self_attn_workspace_bytes(n, num_head_pair);
   size_t most = a > b ? a : b;
-  if (n > 0 && n * tri_ldn(n) <= PROJECT_STEP_POSITIONS && PairStepScratch::bytes(n, 128) > most) most = PairStepScratch::bytes(n, 128);
+  if (n > 0 && n * tri_ldn(n) <= F32_STEP_POSITIONS && PairStepScratch::bytes(n, 128) > most) most = PairStepScratch::bytes(n, 128);
   if (n > 0 && n <= AF3_PAIR64_MAX_TOKENS && PairStepScratch::bytes(n, 64) > most) most = PairStepScratch::bytes(n, 64);
   return most;
 }
@@ -409,7 +394,7 @@ int af3_pairformer_stack_forward(
     // (a pair tensor of 64 channels is what the step kernels alone take)
     if ((b.pair_channels != 0 && b.pair_channels != 128 && b.pair_channels != 64) ||
         (b.pair_channels == 64) != (blocks[0]->pair_channels == 64) ||
-        (b.pair_channels == 64 && (!pair_steps_apply(b, n) || b.with_single)))
+        (b.pair_channels == 64 && (!pair_steps_apply(b, n, pair_dtype) || b.with_single)))
       return AF3_ERR_BAD_ARG;
     if (!b.with_single) continue;
     if (!single || !logits || b.num_head != blocks[0]->num_head || b.c_single != blocks[0]->c_single) return AF3_ERR_BAD_ARG;
@@ -424,8 +409,8 @@ int af3_pairformer_stack_forward(
   int buffers = num_blocks > 1 ? 2 : 1;
   size_t logit_size = logits ? (size_t)blocks[0]->num_head * ((n + 3) / 4 * 4) * n : 0;
   if (two && join) {
-    bool all = true;
-    for (int i = 0; i < num_blocks; ++i) all = all && pair_steps_apply(*blocks[i], n) && blocks[i]->num_head <= 16;
+    bool all = n * tri_ldn(n) <= PairStepScratch::LOGIT_RING_POSITIONS;
+    for (int i = 0; i < num_blocks; ++i) all = all && pair_steps_apply(*blocks[i], n, pair_dtype) && blocks[i]->num_head <= 16;
     PairStepScratch w;
     if (all && workspace_bytes >= PairStepScratch::bytes(n, 128) && w.carve(n, 128, workspace, workspace_bytes)) {
       first = w.ring(n);
@@ -446,10 +431,10 @@ int af3_pairformer_stack_forward(
       if (k % half == 0) free = &read_done[k / half & 1];
     }
     // the pair logits are the only thing the single track reads of `pair`: they are made in front of whatever updates it next
-    if (pair_steps_apply(b, n)) {
-      const bool chained = i > 0 && pair_steps_apply(*blocks[i - 1], n);
-      const af3_pairformer_block* next = i + 1 < num_blocks && pair_steps_apply(*blocks[i + 1], n) ? blocks[i + 1] : nullptr;
-      rc = pair_operators_in_steps(b, false, next, !chained, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes,
+    if (pair_steps_apply(b, n, pair_dtype)) {
+      const bool chained = i > 0 && pair_steps_apply(*blocks[i - 1], n, pair_dtype);
+      const af3_pairformer_block* next = i + 1 < num_blocks && pair_steps_apply(*blocks[i + 1], n, pair_dtype) ? blocks[i + 1] : nullptr;
+      rc = pair_operators_in_steps(b, next, !chained, pair, pair_dtype, pair_mask, pair_mask_incoming, n, workspace, workspace_bytes,
                                    lg, free, main_s);
       if (rc != AF3_OK || !b.with_single) continue;
     } else {

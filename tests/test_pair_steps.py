@@ -48,7 +48,11 @@ def _run_general(blk, *inputs):
 CASES = [(1, 128, 4, 16, 0), (7, 128, 4, 16, 2), (16, 128, 4, 16, 0), (17, 128, 4, 40, 3), (33, 128, 1, 16, 0), (63, 128, 4, 16, 5),
          (64, 128, 2, 16, 0), (65, 128, 4, 16, 30), (127, 128, 4, 16, 0), (129, 128, 3, 16, 11), (208, 128, 4, 16, 9),
          (24, 96, 1, 16, 3), (90, 96, 4, 16, 1),
-         (209, 128, 4, 16, 9), (217, 96, 2, 16, 0), (398, 128, 2, 16, 29)]      # steps in part: just past the line, the last
+         (209, 128, 4, 16, 9), (217, 96, 2, 16, 0), (398, 128, 2, 16, 29),
+         # a transition in tiles of 32 and 64 positions, by the rounds they make; the incoming product's step and its two kernels;
+         # the last sizes of a bf16 stream, and one that only an fp32 stream takes in steps
+         (152, 128, 4, 16, 7), (153, 128, 4, 16, 0), (176, 128, 1, 40, 5), (177, 128, 4, 16, 11), (193, 128, 2, 16, 0),
+         (493, 128, 4, 16, 17), (545, 96, 4, 16, 0)]
 
 
 @pytest.mark.gpu
