@@ -420,8 +420,15 @@ int af3_pairformer_stack_forward(
   }
   const int half = buffers > 1 ? buffers / 2 : 1;
   Event ready, read_done[2];  // behind the pair logits; behind the last attention that reads a buffer of either half
-  if (two) STEP(ready.order(main_s, side_s));
-  int rc = AF3_OK, k = 0;
+  int singles = 0;
+  for (int i = 0; i < num_blocks; ++i) singles += blocks[i]->with_single ? 1 : 0;
+  // (the wait in front of the first update of `single` is for what `stream` holds on entry, too)
+  if (two && singles == 0) STEP(ready.order(main_s, side_s));
+  // Where launches set the pace the updates of two blocks wait for the streams' meeting together, but for the last one, which has no
+  // pair operators to run beside.  With the wait on entry, that is four meetings for four blocks instead of six: 64 tokens 408 -> 362
+  // us, 45 400 -> 352, 128 480 -> 470; past 144 tokens the pair operators are longer than what an update waits for (176: 683 -> 689).
+  const bool by_two = buffers == PairStepScratch::LOGIT_RING && n * tri_ldn(n) <= 144 * 144;
+  int rc = AF3_OK, k = 0, done = 0, from = 0;  // single tracks whose logits are on their way, those enqueued; the block of the next one
   for (int i = 0; i < num_blocks && rc == AF3_OK; ++i) {
     const af3_pairformer_block& b = *blocks[i];
     float* lg = nullptr;
@@ -444,11 +451,17 @@ int af3_pairformer_stack_forward(
       if (rc == AF3_OK)
         rc = af3_pair_logits_quads_forward(pair, pair_dtype, b.sl_ln_w, b.sl_ln_b, b.sl_w, b.num_head, lg, n, stream);
     }
-    if (rc == AF3_OK && two) rc = ready.order(main_s, side_s);
-    if (rc == AF3_OK)
-      rc = single_update(b, single, single_dtype, seq_mask, lg, n, single_workspace, single_workspace_bytes, side_s);
-    if (rc == AF3_OK && two && k % half == half - 1 && i + half + 1 < num_blocks) rc = read_done[k / half & 1].record(side_s);
     ++k;
+    if (rc != AF3_OK || (by_two && k % 2 == 1 && k + 1 < singles)) continue;
+    if (two) rc = ready.order(main_s, side_s);
+    for (; from <= i && rc == AF3_OK; ++from) {
+      const af3_pairformer_block& t = *blocks[from];
+      if (!t.with_single) continue;
+      rc = single_update(t, single, single_dtype, seq_mask, first + (done % buffers) * logit_size, n, single_workspace,
+                         single_workspace_bytes, side_s);
+      if (rc == AF3_OK && two && done % half == half - 1 && from + half + 1 < num_blocks) rc = read_done[done / half & 1].record(side_s);
+      ++done;
+    }
   }
   if (two && join) {
     const int jrc = ready.order(side_s, main_s);

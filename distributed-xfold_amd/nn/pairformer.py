@@ -270,7 +270,9 @@ def pairformer_loop(blocks, pair, pair_mask, single, seq_mask, overlap_single: b
             and b.c_single == blocks[0].c_single for b in blocks):
         if not (pair.is_contiguous() and single.is_contiguous()):
             raise ValueError("pair and single must be contiguous (they are updated in place)")
-        ops.pairformer_stack([b.native() for b in blocks], pair, pair_mask, single, seq_mask, single_stream=side)
+        # (one block's update has nothing to run beside)
+        ops.pairformer_stack([b.native() for b in blocks], pair, pair_mask, single, seq_mask,
+                             single_stream=side if len(blocks) > 1 else None)
         return pair, single
     main = torch.cuda.current_stream(pair.device)
     side.wait_stream(main)          # whatever produced `single` and `seq_mask`

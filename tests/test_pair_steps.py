@@ -201,3 +201,17 @@ def test_all_matrices_of_a_block_are_in_its_fragments(pkg, factor, rows):
     w2 = blk.pair_transition.packed()["w2"]
     assert torch.equal(frags[-w2.numel():], pkg.nn.base.fragments(w2))
     assert torch.equal(frags[-w2.numel() - 32 * 128:-w2.numel()], pkg.nn.base.fragments(blk.packed()["w_logits"]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,blocks", [(40, 1), (40, 2), (40, 3), (33, 11), (133, 5), (145, 4)])
+def test_stacks_give_the_bits_of_their_blocks(gpu_pkg, n, blocks):
+    """The streams of a stack meet for one or two blocks at a time, and more blocks than the eight buffers of pair logits go round."""
+    run = [_block(gpu_pkg, seed=i) for i in range(blocks)]
+    pair, mask, single, seq = _inputs(n, 128, torch.bfloat16, 3)
+    want = (pair.clone(), single.clone())
+    for blk in run:
+        want = blk(*want[:1], mask, want[1], seq)
+    for _ in range(3):
+        got = gpu_pkg.nn.pairformer_loop(run, pair.clone(), mask, single.clone(), seq)
+        assert all(torch.isfinite(x).all() and torch.equal(x, y) for x, y in zip(got, want))
