@@ -248,14 +248,14 @@ static int grid_self_attn_impl(
 static int transition_impl(
     const void* act, int io_dtype, const float* ln_w, const float* ln_b,
     const uint16_t* w1_packed, const uint16_t* w2, int hidden,
-    void* out, int residual, int64_t rows, int valid_channels, af3_stream_t stream) {
+    void* out, int residual, int64_t rows, int valid_channels, int rounded, af3_stream_t stream) {
   if (!act || !out || !ln_w || !ln_b || !w1_packed || !w2) return AF3_ERR_BAD_ARG;
   if (bad_dtype(io_dtype) || rows <= 0 || rows > 0x7fffffff || hidden <= 0 || (hidden & 63)) return AF3_ERR_BAD_ARG;
   if (valid_channels < 8 || valid_channels > C_PAIR) return AF3_ERR_BAD_ARG;
   TransitionArgs t;
   t.lw = ln_width(valid_channels);
   t.x = act; t.out = out; t.io_f32 = io_dtype == AF3_F32; t.N = (int)rows; t.hidden = hidden;
-  t.residual = residual != 0; t.ln_w = ln_w; t.ln_b = ln_b; t.w1 = w1_packed; t.w2 = w2;
+  t.residual = residual != 0; t.rounded = rounded; t.ln_w = ln_w; t.ln_b = ln_b; t.w1 = w1_packed; t.w2 = w2;
   return launch_transition(t, static_cast<hipStream_t>(stream));
 }
 
@@ -299,13 +299,18 @@ int af3_transition_forward(
     const void* act, int io_dtype, const float* ln_w, const float* ln_b,
     const uint16_t* w1_packed, const uint16_t* w2, int hidden,
     void* out, int residual, int64_t rows, af3_stream_t stream) {
-  return transition_impl(act, io_dtype, ln_w, ln_b, w1_packed, w2, hidden, out, residual, rows, C_PAIR, stream);
+  return transition_impl(act, io_dtype, ln_w, ln_b, w1_packed, w2, hidden, out, residual, rows, C_PAIR, 0, stream);
 }
 int af3_transition_forward_padded(
     const void* act, int io_dtype, const float* ln_w, const float* ln_b,
     const uint16_t* w1_packed, const uint16_t* w2, int hidden,
     void* out, int residual, int64_t rows, int valid_channels, af3_stream_t stream) {
-  return transition_impl(act, io_dtype, ln_w, ln_b, w1_packed, w2, hidden, out, residual, rows, valid_channels, stream);
+  return transition_impl(act, io_dtype, ln_w, ln_b, w1_packed, w2, hidden, out, residual, rows, valid_channels, 0, stream);
+}
+int af3_pair_cond_transition_forward(
+    const float* act, const float* ln_w, const float* ln_b, const uint16_t* w1_packed, const uint16_t* w2, int hidden,
+    float* out, int residual, int64_t rows, af3_stream_t stream) {
+  return transition_impl(act, AF3_F32, ln_w, ln_b, w1_packed, w2, hidden, out, residual, rows, C_PAIR, 1, stream);
 }
 
 // ------------------------------------------- pair-biased self-attention (single / diffusion)

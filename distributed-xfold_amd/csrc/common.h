@@ -158,6 +158,11 @@ __device__ __forceinline__ float group8_sum(float v) {
   v += dpp_mov<0xB1>(v); v += dpp_mov<0x4E>(v);
   return v + dpp_mov<0x141>(v);
 }
+// group16_sum by halving: lanes 1, 2, 4 and 8 apart meet (row_mirror: the other eight), the same order in every lane
+__device__ __forceinline__ float group16_sum_halving(float v) {
+  v = group8_sum(v);
+  return v + dpp_mov<0x140>(v);
+}
 template <int LANES>
 __device__ __forceinline__ float group_sum(float v) {
   static_assert(LANES == 16 || LANES == 8, "lanes");

@@ -279,6 +279,7 @@ struct TransitionArgs {
   const void* x = nullptr;  // [N][128]
   void* out = nullptr;
   int io_f32 = 0, N = 0, hidden = 0, residual = 0;
+  int rounded = 0;  // fp32 rows only: see ln_pixel8
   const float *ln_w = nullptr, *ln_b = nullptr;
   const bf16_t* w1 = nullptr;  // [hidden/64][128][128]: 64 a rows then 64 b rows per slab
   const bf16_t* w2 = nullptr;  // [128][hidden]

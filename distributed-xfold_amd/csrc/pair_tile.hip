@@ -502,7 +502,7 @@ __device__ __forceinline__ void dma_lds_barrier() {
 constexpr int W1_SLAB = 64 * 256;  // 32 "a" rows + 32 "b" rows of 128 bf16: 16 KB
 constexpr int W2_SLAB = 128 * 64;  // 128 output rows x 32 hidden units: 8 KB
 
-template <typename TIO>
+template <typename TIO, bool ROUNDED = false>
 __global__ __launch_bounds__(256, 2) void transition_kernel(TransitionArgs a) {
   // The hidden layer is walked in slabs of 32 units.  Per slab a wave issues 16 MFMAs of GEMM1 (T form:
   // a^T and b^T, 32 hidden x 32 pixels each), 32 SiLU-gate evaluations per lane pair of registers and 8
@@ -572,7 +572,7 @@ __global__ __launch_bounds__(256, 2) void transition_kernel(TransitionArgs a) {
   };
   load_slab(0, w1buf0, w2buf0);
 
-  load_ln_tile<TIO>(x, t, a.ln_w, a.ln_b, sX, tid, false, a.lw.inv_c, a.lw.pad);
+  load_ln_tile<TIO, ROUNDED>(x, t, a.ln_w, a.ln_b, sX, tid, false, a.lw.inv_c, a.lw.pad);
   lds_barrier();
   bf16x8 xf[8];
   load_x_frags(sX, wave, lane, xf);
@@ -874,6 +874,7 @@ int launch_transition(const TransitionArgs& a, hipStream_t s) {
   // x is [rows][128]; handled as `rows` positions in one long row
   if (a.N <= 0 || !a.x || !a.out || !a.w1 || !a.w2 || a.hidden <= 0 || (a.hidden & 63)) return AF3_ERR_BAD_ARG;
   if (!aligned16(a.x) || !aligned16(a.out) || !aligned16(a.w1) || !aligned16(a.w2)) return AF3_ERR_BAD_ARG;
+  if (a.rounded) return a.io_f32 ? launch_tiles(transition_kernel<float, true>, a, a.N, s) : AF3_ERR_BAD_ARG;
   return a.io_f32 ? launch_tiles(transition_kernel<float>, a, a.N, s)
                   : launch_tiles(transition_kernel<bf16_t>, a, a.N, s);
 }

@@ -140,7 +140,9 @@ __device__ __forceinline__ void load_param8(const float* p, float fill, float* o
 // select when every pixel of the tile is in range.  The fp32 stream keeps the
 // two-pass form.  Zero-padded channels (fewer than 128 real ones) add nothing to
 // either sum; the two-pass form takes their pad * mean^2 out again.
-template <typename TIO, int LANES = 16>
+// ROUNDED (fp32 rows): rowops.hip's row LayerNorm to the last bit, with its order of the sums and the product with the weight
+// rounded before the bias is added.
+template <typename TIO, int LANES = 16, bool ROUNDED = false>
 __device__ __forceinline__ u32x4 ln_pixel8(const typename Elem<TIO>::Raw& raw, const float* w, const float* b,
                                            bool skip_ln, float inv_c, float pad) {
   using E = Elem<TIO>;
@@ -162,14 +164,30 @@ __device__ __forceinline__ u32x4 ln_pixel8(const typename Elem<TIO>::Raw& raw, c
     float s = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) s += v[e];
-    const float mean = group_sum<LANES>(s) * inv_c;
+    auto sum = [](float x) { return ROUNDED ? group16_sum_halving(x) : group_sum<LANES>(x); };
+    const float mean = sum(s) * inv_c;
     float q = 0.f;
+    if constexpr (ROUNDED) {
+      float d[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { const float d = v[e] - mean; q += d * d; }
+      for (int e = 0; e < 8; ++e) d[e] = v[e] - mean;
+      q = add_squares8(d, 0.f, true);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) { const float d = v[e] - mean; q += d * d; }
+    }
     // (zero-padded channels, if any, each put mean^2 into the sum)
-    const float rstd = rsqrtf((group_sum<LANES>(q) - pad * mean * mean) * inv_c + LN_EPS);
+    const float rstd = rsqrtf((sum(q) - pad * mean * mean) * inv_c + LN_EPS);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = skip_ln ? v[e] : (v[e] - mean) * rstd * w[e] + b[e];
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (ROUNDED) {
+#pragma clang fp contract(off)
+        const float t = (v[e] - mean) * rstd * w[e];
+        o[e] = t + b[e];
+      } else {
+        o[e] = skip_ln ? v[e] : (v[e] - mean) * rstd * w[e] + b[e];
+      }
+    }
   }
   return pack8(o);
 }
@@ -181,7 +199,7 @@ __device__ __forceinline__ u32x4 ln_pixel8(const typename Elem<TIO>::Raw& raw, c
 // unconditional (an out-of-range position re-reads some valid pixel) and all
 // issued before any value is converted: a load under a lane mask, or one whose
 // value is touched at once, costs a full memory round trip per pixel.
-template <typename TIO, typename Tile>
+template <typename TIO, bool ROUNDED = false, typename Tile>
 __device__ __forceinline__ void load_ln_tile(const TIO* x, const Tile& t, const float* lnw,
                                              const float* lnb, bf16_t* sX, int tid, bool skip_ln = false,
                                              float inv_c = 1.f / C, float pad = 0.f) {
@@ -203,7 +221,7 @@ __device__ __forceinline__ void load_ln_tile(const TIO* x, const Tile& t, const 
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       const int p = (base + i) * 16 + prow;
-      u32x4 pk = ln_pixel8<TIO>(raw[i], w, b, skip_ln, inv_c, pad);
+      u32x4 pk = ln_pixel8<TIO, 16, ROUNDED>(raw[i], w, b, skip_ln, inv_c, pad);
       if (!full && !t.valid(p)) pk = u32x4{0u, 0u, 0u, 0u};
       *reinterpret_cast<u32x4*>(sX + p * LDX + chunk * 8) = pk;
     }

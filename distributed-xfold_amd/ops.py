@@ -191,11 +191,13 @@ def grid_self_attn(pair, mask, transpose, act_norm_weight, act_norm_bias, w_pair
     return out
 
 
-def transition128(act, layernorm_weight, layernorm_bias, w1_packed, w2, residual=False, out=None, valid_channels=128):
+def transition128(act, layernorm_weight, layernorm_bias, w1_packed, w2, residual=False, out=None, valid_channels=128,
+                  pair_cond=False):
     """transition_forward (csrc/Alpha_Attention.cpp:116-125) for 128-channel rows.
-    `valid_channels` < 128: rows and weights are zero-padded to 128 channels."""
+    `valid_channels` < 128: rows and weights are zero-padded to 128 channels.  `pair_cond`: fp32 rows with the roundings of
+    a row LayerNorm and two linear layers (af3_pair_cond_transition_forward)."""
     lib = _L.load()
-    _gpu(act, "act")
+    _gpu(act, "act", torch.float32 if pair_cond else None)
     if act.shape[-1] != 128:
         raise ValueError("act: last dimension must be 128")
     io = _dt(act)
@@ -209,6 +211,11 @@ def transition128(act, layernorm_weight, layernorm_bias, w1_packed, w2, residual
         out = act if residual else torch.empty_like(act)
     else:
         _gpu(out, "out", act.dtype, act.shape)
+    if pair_cond:
+        rc = lib.af3_pair_cond_transition_forward(_p(act), _p(layernorm_weight), _p(layernorm_bias), _p(w1_packed), _p(w2),
+                                                  int(hidden), _p(out), int(bool(residual)), rows, _stream(act.device))
+        _L.check(rc, "af3_pair_cond_transition_forward")
+        return out
     if valid_channels != 128:
         rc = lib.af3_transition_forward_padded(_p(act), io, _p(layernorm_weight), _p(layernorm_bias), _p(w1_packed),
                                                _p(w2), int(hidden), _p(out), int(bool(residual)), rows,

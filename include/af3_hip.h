@@ -127,6 +127,14 @@ int af3_transition_forward(
     const float* layernorm_weight, const float* layernorm_bias,
     const uint16_t* w1_packed, const uint16_t* w2, int hidden,
     void* out, int residual, int64_t rows, af3_stream_t stream);
+/* The same for the unconditioned transitions of the diffusion head's pair conditioning
+ * (nn/d_diffusion_transformer.py:120-145), rows of fp32: the values of a row LayerNorm
+ * (af3_layer_norm_forward) and two af3_linear_forward, bit for bit, in one pass.
+ */
+int af3_pair_cond_transition_forward(
+    const float* act, const float* layernorm_weight, const float* layernorm_bias,
+    const uint16_t* w1_packed, const uint16_t* w2, int hidden,
+    float* out, int residual, int64_t rows, af3_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * The three pair operators above on FEWER than 128 pair channels: the Pairformer

@@ -271,3 +271,25 @@ def test_two_threads_on_one_stream(gpu_pkg):
     torch.cuda.synchronize()
     for i in range(2):
         assert len(got[i]) == 20 and all(torch.equal(a, b) for out in got[i] for a, b in zip(out, want[i]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,factor", [(1, 2), (127, 1), (128, 2), (129, 2), (1700, 4), (120001, 2)])
+@pytest.mark.parametrize("residual", [True, False])
+def test_unconditioned_transition_in_one_kernel(gpu_pkg, rows, factor, residual):
+    """128 channels without conditioning: the bits of the LayerNorm and the two products, which a tensor off 16 bytes takes."""
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    with torch.device("cuda"):
+        mod = gpu_pkg.nn.DiffusionTransition(c_x=128, c_single_cond=None, num_intermediate_factor=factor)
+    with torch.no_grad():
+        for name, p in mod.named_parameters():
+            p.normal_(0.0, 0.1, generator=g)
+            if p.dim() == 1 and name.endswith("weight"):
+                p += 1.0
+    mod.invalidate()
+    x = torch.randn(rows, 128, generator=g, device="cuda") * 3 + 1
+    got = mod.run(x.clone(), None, residual=residual)
+    norm = mod.adaptive_layernorm.packed()
+    h = gpu_pkg.ops.linear(gpu_pkg.ops.layer_norm(x, norm["ln_w"], norm["ln_b"]), mod.packed()["w1"], mode=gpu_pkg.lib.LINEAR_SWIGLU)
+    want = mod.adaptive_zero_init.run(h, None, x.dtype, residual=x.clone() if residual else None)
+    assert got.dtype == torch.float32 and torch.isfinite(got).all() and torch.equal(got, want) and not torch.equal(got, x)
