@@ -2,7 +2,8 @@
 // Each stands for a run of single operations (ten to forty launches of 2 to 5 us, most of them on a few kilobytes, and
 // as many passes over the pair tensor), and rounds as they do: every operation of its own, nothing fused into an FMA.
 //
-// Trunk pass at 160 tokens, 128 MSA rows: embedding 380 us in 78 launches before.
+// Trunk pass at 160 tokens, 128 MSA rows: embedding 380 us in 78 launches before.  The head's atom conditioning at 384 tokens: 75
+// launches less, whose host time (1060 us, 590 now) the GPU had nothing else to do in; a new batch 4460 -> 4080 us.
 #pragma clang fp contract(off)
 #include "common.h"
 #include "kernels.h"
@@ -113,6 +114,76 @@ struct MaskRows {
   }
 };
 
+// eight channels of an atom: ((((p0 w0 + p1 w1) + p2 w2) + mask w) + element) + asinh(charge) w, + four characters, * mask.  The weights
+// as a linear layer holds them, [channel][input]: 200 KB that stay in L2.  9216 atoms: 11 us in place of 23 launches of 3 to 8.
+struct AtomEmbed {
+  AtomEmbedArgs a;
+  __device__ __forceinline__ void operator()(int64_t item) const {
+    const int chunks = a.channels / 8;
+    const int64_t atom = item / chunks;
+    const int c0 = (int)(item - atom * chunks) * 8;
+    auto index = [](int64_t v, int size) { return v + (v < 0 ? size : 0); };
+    const float m = a.mask[atom], charge = asinhf(a.charge[atom]), *const p = a.positions + atom * 3;
+    const int64_t element = index(a.element[atom], 128);
+    int64_t chars[4];
+    bool ok = element >= 0 && element < 128;  // (else the atom is not a number)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      chars[j] = index(a.chars[atom * 4 + j], 64);
+      ok = ok && chars[j] >= 0 && chars[j] < 64;
+    }
+    float o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int c = c0 + e;
+      float x = p[0] * a.w_pos[c * 3];
+      x = x + p[1] * a.w_pos[c * 3 + 1];
+      x = x + p[2] * a.w_pos[c * 3 + 2];
+      x = x + m * a.w_mask[c];
+      x = x + (ok ? a.w_element[c * 128 + element] : __builtin_nanf(""));
+      x = x + charge * a.w_charge[c];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x = x + (ok ? a.w_chars[c * 256 + 64 * j + chars[j]] : 0.f);
+      o[e] = x * m;
+    }
+    Elem<float>::store8(a.out + item * 8, o);
+  }
+};
+
+// Atoms gathered into another layout, eight channels of a row: out = src * mask [+ add * add_mask], and what else an atom has.
+// (One pass each for queries and keys in place of nine gathers of three or four launches.)
+struct GatherAtoms {
+  GatherAtomsArgs a;
+  __device__ __forceinline__ void operator()(int64_t item) const {
+    const int chunks = a.channels / 8;
+    const int64_t row = item / chunks;
+    const int c = (int)(item - row * chunks) * 8;
+    const int64_t at = a.idx[row], add_at = a.add ? a.add_idx[row] : 0;
+    const bool ok = at >= 0 && at < a.slots && add_at >= 0 && add_at < a.add_rows;  // (else the row is not a number)
+    const float m = a.exists[row] ? 1.f : 0.f;
+    float o[8], x[8];
+    Elem<float>::load8(a.cond + (ok ? at : 0) * a.channels + c, o);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = ok ? o[e] * m : __builtin_nanf("");
+    if (a.add) {
+      const float am = a.add_exists[row] ? 1.f : 0.f;
+      Elem<float>::load8(a.add + (ok ? add_at : 0) * a.channels + c, x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float t = x[e] * am;
+        o[e] = o[e] + t;
+      }
+    }
+    Elem<float>::store8(a.out_cond + item * 8, o);
+    if (c != 0) return;
+    const int64_t from = ok ? at : 0;
+    a.out_mask[row] = a.mask[from] * m;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) a.out_pos[row * 3 + e] = a.pos[from * 3 + e] * m;
+    a.out_uid[row] = ok && a.exists[row] && at < a.uids ? (int)a.uid[at] : 0;
+  }
+};
+
 constexpr float SIGMA2 = 256.f, SIGMA = 16.f;  // of the data
 
 // positions [samples][atoms][3] against mask [atoms]
@@ -191,6 +262,23 @@ int launch_add_rows(const float* a, const float* b, int64_t ld_b, int64_t mod, v
 int launch_mask_rows(bf16_t* x, const float* mask, int64_t mod, int64_t rows, int channels, hipStream_t s) {
   if (!x || !mask || rows <= 0 || mod <= 0 || channels <= 0 || (channels & 7) || !al16(x)) return AF3_ERR_BAD_ARG;
   return launch_each(rows * (channels / 8), s, MaskRows{x, mask, mod, channels / 8});
+}
+
+int launch_atom_embed(const AtomEmbedArgs& a, hipStream_t s) {
+  if (!a.positions || !a.mask || !a.element || !a.charge || !a.chars || !a.w_pos || !a.w_mask || !a.w_element || !a.w_charge ||
+      !a.w_chars || !a.out || a.atoms <= 0 || a.channels <= 0 || (a.channels & 7) || !al16(a.out))
+    return AF3_ERR_BAD_ARG;
+  return launch_each(a.atoms * (a.channels / 8), s, AtomEmbed{a});
+}
+
+int launch_gather_atoms(const GatherAtomsArgs& a, hipStream_t s) {
+  if (!a.idx || !a.exists || !a.cond || !a.mask || !a.pos || !a.uid || !a.out_cond || !a.out_mask || !a.out_pos || !a.out_uid ||
+      a.rows <= 0 || a.slots <= 0 || a.uids <= 0 || a.channels <= 0 || (a.channels & 7) || !al16(a.cond) || !al16(a.out_cond))
+    return AF3_ERR_BAD_ARG;
+  if (a.add && (!a.add_idx || !a.add_exists || a.add_rows <= 0 || !al16(a.add))) return AF3_ERR_BAD_ARG;
+  GatherAtomsArgs args = a;
+  if (!a.add) args.add_rows = 1;
+  return launch_each(a.rows * (a.channels / 8), s, GatherAtoms{args});
 }
 
 int launch_positions(int op, const float* x, const float* y, const float* mask, const float* level, const float* other, float f,

@@ -502,6 +502,27 @@ int launch_contacts(const int64_t* idx0, const uint8_t* ok0, int n0, const int64
 int launch_add_rows(const float* a, const float* b, int64_t ld_b, int64_t mod, void* out, int out_f32, int64_t rows, int channels,
                     hipStream_t s);
 int launch_mask_rows(bf16_t* x, const float* mask, int64_t mod, int64_t rows, int channels, hipStream_t s);
+struct AtomEmbedArgs {
+  const float *positions = nullptr, *mask = nullptr, *charge = nullptr;  // [atoms][3], [atoms], [atoms]
+  const int64_t *element = nullptr, *chars = nullptr;                    // [atoms] below 128, [atoms][4] below 64
+  // [channels][3], [channels], [channels][128], [channels], [channels][4 * 64]
+  const float *w_pos = nullptr, *w_mask = nullptr, *w_element = nullptr, *w_charge = nullptr, *w_chars = nullptr;
+  float* out = nullptr;  // [atoms][channels]
+  int64_t atoms = 0;
+  int channels = 0;
+};
+int launch_atom_embed(const AtomEmbedArgs& a, hipStream_t s);
+struct GatherAtomsArgs {
+  const int64_t *idx = nullptr, *add_idx = nullptr, *uid = nullptr;  // [rows], [rows], [uids]
+  const uint8_t *exists = nullptr, *add_exists = nullptr;            // [rows]
+  const float *cond = nullptr, *add = nullptr;                       // [slots][channels]; [add_rows][channels] or null
+  const float *mask = nullptr, *pos = nullptr;                       // [slots], [slots][3]
+  float *out_cond = nullptr, *out_mask = nullptr, *out_pos = nullptr;
+  int* out_uid = nullptr;
+  int64_t rows = 0, slots = 0, add_rows = 0, uids = 0;
+  int channels = 0;
+};
+int launch_gather_atoms(const GatherAtomsArgs& a, hipStream_t s);
 enum { POS_SCALE = 0, POS_BLEND = 1, POS_PLACE = 2, POS_STEP = 3 };
 int launch_positions(int op, const float* x, const float* y, const float* mask, const float* level, const float* other, float f,
                      float* out, int64_t samples, int64_t atoms, hipStream_t s);

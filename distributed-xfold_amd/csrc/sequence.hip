@@ -733,6 +733,27 @@ int af3_mask_rows_forward(uint16_t* x, const float* mask, int64_t mod, int64_t r
   return launch_mask_rows(x, mask, mod, rows, channels, static_cast<hipStream_t>(stream));
 }
 
+int af3_atom_embed_forward(const float* positions, const float* mask, const int64_t* element, const float* charge,
+                           const int64_t* atom_name_chars, const float* w_pos, const float* w_mask, const float* w_element,
+                           const float* w_charge, const float* w_chars, float* out, int64_t atoms, int channels, af3_stream_t stream) {
+  AtomEmbedArgs a;
+  a.positions = positions; a.mask = mask; a.element = element; a.charge = charge; a.chars = atom_name_chars;
+  a.w_pos = w_pos; a.w_mask = w_mask; a.w_element = w_element; a.w_charge = w_charge; a.w_chars = w_chars;
+  a.out = out; a.atoms = atoms; a.channels = channels;
+  return launch_atom_embed(a, static_cast<hipStream_t>(stream));
+}
+
+int af3_gather_atoms_forward(const int64_t* idx, const uint8_t* exists, int64_t rows, const float* cond, const float* mask,
+                             const float* positions, int64_t slots, const int64_t* uid, int64_t uids, const int64_t* add_idx,
+                             const uint8_t* add_exists, const float* add, int64_t add_rows, float* out_cond, float* out_mask,
+                             float* out_positions, int32_t* out_uid, int channels, af3_stream_t stream) {
+  GatherAtomsArgs a;
+  a.idx = idx; a.exists = exists; a.rows = rows; a.cond = cond; a.mask = mask; a.pos = positions; a.slots = slots;
+  a.uid = uid; a.uids = uids; a.add_idx = add_idx; a.add_exists = add_exists; a.add = add; a.add_rows = add_rows;
+  a.out_cond = out_cond; a.out_mask = out_mask; a.out_pos = out_positions; a.out_uid = out_uid; a.channels = channels;
+  return launch_gather_atoms(a, static_cast<hipStream_t>(stream));
+}
+
 int af3_positions_forward(int op, const float* x, const float* y, const float* mask, const float* level, const float* next,
                           float factor, float* out, int64_t samples, int64_t atoms, af3_stream_t stream) {
   return launch_positions(op, x, y, mask, level, next, factor, out, samples, atoms, static_cast<hipStream_t>(stream));

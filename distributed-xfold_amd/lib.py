@@ -64,6 +64,9 @@ SIGNATURES = {
     "af3_contact_matrix_forward": (_i, [_vp, _vp, _i, _vp, _vp, _i, _vp, _i64, _vp]),
     "af3_pair_embed_forward": (
         _i, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i64, _vp]),
+    "af3_atom_embed_forward": (_i, [_vp] * 11 + [_i64, _i, _vp]),
+    "af3_gather_atoms_forward": (
+        _i, [_vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _i, _vp]),
     "af3_add_rows_forward": (_i, [_vp, _vp, _i64, _i64, _vp, _i, _i64, _i, _vp]),
     "af3_mask_rows_forward": (_i, [_vp, _vp, _i64, _i64, _i, _vp]),
     "af3_positions_forward": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _f, _vp, _i64, _i64, _vp]),

@@ -14,6 +14,7 @@ is what the reference does on every call.
 
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
 from typing import Any, Optional
 
@@ -125,11 +126,17 @@ class AtomCrossAttEncoder(HipModule):
             d["w_pos"] = f32(self.atom_positions_to_features.weight)
         return d
 
-    def _per_atom_conditioning(self, batch):
-        """:87-156 -> (act [N, A, 128], pair_act [N, A, A, 16]), fp32.  The
-        one-hot inputs of :98-110 are table look-ups into the weight columns."""
+    def _per_atom_single(self, batch):
+        """:87-111 -> act [N, A, 128], fp32.  The one-hot inputs of :98-110 are
+        table look-ups into the weight columns."""
         rs = batch.ref_structure
         m = rs.mask.float()
+        if not in_check_mode() and m.is_cuda and m.numel() and self.c_query % 8 == 0:
+            plain = lambda t: t.contiguous()
+            w = lambda layer: layer.weight.detach().float().contiguous()
+            return ops.atom_embed(plain(rs.positions.float()), plain(m), plain(rs.element.long()), plain(rs.charge.float()),
+                                  plain(rs.atom_name_chars.long()), w(self.embed_ref_pos), w(self.embed_ref_mask),
+                                  w(self.embed_ref_element), w(self.embed_ref_charge), w(self.embed_ref_atom_name))
         act = _lin(rs.positions, self.embed_ref_pos) + _lin(m[:, :, None], self.embed_ref_mask)
         act = act + self.embed_ref_element.weight.float().t()[rs.element.long()]
         act = act + _lin(torch.arcsinh(rs.charge.float())[:, :, None], self.embed_ref_charge)
@@ -137,7 +144,12 @@ class AtomCrossAttEncoder(HipModule):
         chars = rs.atom_name_chars.long()
         for j in range(4):
             act = act + wn[j][chars[..., j]]
-        act = act * m[:, :, None]
+        return act * m[:, :, None]
+
+    def _per_atom_conditioning(self, batch):
+        """:87-156 -> (act [N, A, 128], pair_act [N, A, A, 16]), fp32."""
+        rs = batch.ref_structure
+        act = self._per_atom_single(batch)
         pair_act = (_lin(act, self.single_to_pair_cond_row, relu_input=True)[:, :, None, :]
                     + _lin(act, self.single_to_pair_cond_col, relu_input=True)[:, None, :, :])
         pos = rs.positions.float()
@@ -146,26 +158,51 @@ class AtomCrossAttEncoder(HipModule):
         pair_act = pair_act + _lin(1.0 / (1 + (d * d).sum(-1, keepdim=True)), self.embed_pair_distances)
         return act, pair_act
 
+    @staticmethod
+    def _layouts(batch, tok_single, ts):
+        """:168-179, 205-215, 268-283: conditioning, mask, position and uid of the atoms in the layout of the queries, with the
+        tokens' `ts` on top of the conditioning, and in that of the keys."""
+        aca, rs, mask = batch.atom_cross_att, batch.ref_structure, batch.predicted_structure_info.atom_mask
+        t2q, tok, q2k = aca.token_atoms_to_queries, aca.tokens_to_queries, aca.queries_to_keys
+        pos, uid = rs.positions.float(), rs.ref_space_uid
+        infos = (t2q, q2k) if ts is None else (t2q, q2k, tok)
+        slots, rows = mask.numel(), t2q.gather_idxs.numel()
+        used = [tok_single, mask, pos, uid] + [t for i in infos for t in (i.gather_idxs, i.gather_mask)]
+        if (not in_check_mode() and all(t.is_cuda and t.is_contiguous() and t.numel() for t in used)
+                and mask.dtype == torch.float32 and uid.dtype == torch.int64 and tok_single.shape[-1] % 8 == 0
+                and tok_single.dtype == torch.float32 and pos.shape == mask.shape + (3,) and uid.shape == mask.shape
+                and tok_single.shape[:-1] == mask.shape
+                and all(i.gather_idxs.dtype == torch.int64 and i.gather_mask.dtype == torch.bool
+                        and i.gather_mask.shape == i.gather_idxs.shape for i in infos)
+                and math.prod(t2q.input_shape) == slots and math.prod(q2k.input_shape) == rows == slots
+                and (ts is None or (ts.is_contiguous() and ts.dim() == 2 and math.prod(tok.input_shape) == ts.shape[0]
+                                    and tok.gather_idxs.shape == t2q.gather_idxs.shape))):
+            q = ops.gather_atoms(t2q, tok_single, mask, pos, uid, tok, ts)
+            return q + ops.gather_atoms(q2k, *q[:3], uid)
+        q_cond = convert(t2q, tok_single, (-3, -2))
+        q_mask = convert(t2q, mask, (-2, -1))
+        if ts is not None:
+            q_cond = q_cond + convert(tok, ts, (-2,))
+        k_cond = convert(q2k, q_cond, (-3, -2))
+        k_mask = convert(q2k, q_mask, (-2, -1))
+        q_pos = convert(t2q, pos, (-3, -2))
+        q_uid = convert(t2q, uid, (-2, -1))
+        k_pos = convert(q2k, q_pos, (-3, -2))
+        # :279-283: the keys' uid is gathered from the token-atom layout with the query-layout gather
+        k_uid = convert(q2k, uid, (-2, -1))
+        return q_cond, q_mask, q_pos, q_uid, k_cond, k_mask, k_pos, k_uid
+
     @torch.no_grad()
     def conditioning(self, batch, trunk_single_cond, trunk_pair_cond) -> EncoderConditioning:
         """The position-independent part of `forward` (:168-179, 205-311)."""
         p = self.packed()
         aca = batch.atom_cross_att
-        tok_single, _ = self._per_atom_conditioning(batch)
-        q_cond = convert(aca.token_atoms_to_queries, tok_single, (-3, -2))
-        q_mask = convert(aca.token_atoms_to_queries, batch.predicted_structure_info.atom_mask, (-2, -1))
+        tok_single = self._per_atom_single(batch)
+        ts = None
         if trunk_single_cond is not None:
             ts = _ln_lin(trunk_single_cond, self.lnorm_trunk_single_cond, self.embed_trunk_single_cond,
                          p.get("ts_ln"), p.get("ts_w"))
-            q_cond = q_cond + convert(aca.tokens_to_queries, ts, (-2,))
-        k_cond = convert(aca.queries_to_keys, q_cond, (-3, -2))
-        k_mask = convert(aca.queries_to_keys, q_mask, (-2, -1))
-        rs = batch.ref_structure
-        q_pos = convert(aca.token_atoms_to_queries, rs.positions.float(), (-3, -2))
-        q_uid = convert(aca.token_atoms_to_queries, rs.ref_space_uid, (-2, -1))
-        k_pos = convert(aca.queries_to_keys, q_pos, (-3, -2))
-        # :279-283: the keys' uid is gathered from the token-atom layout with the query-layout gather
-        k_uid = convert(aca.queries_to_keys, rs.ref_space_uid, (-2, -1))
+        q_cond, q_mask, q_pos, q_uid, k_cond, k_mask, k_pos, k_uid = self._layouts(batch, tok_single, ts)
         row = _lin(q_cond, self.single_to_pair_cond_row_1, relu_input=True)
         col = _lin(k_cond, self.single_to_pair_cond_col_1, relu_input=True)
         tp = None

@@ -315,6 +315,55 @@ def add_rows(a, b, out_dtype):
     return out
 
 
+def atom_embed(positions, mask, element, charge, chars, w_pos, w_mask, w_element, w_charge, w_chars):
+    """The reference conformer's per-atom embedding [.., channels] (af3_atom_embed_forward): positions [.., 3], mask, charge
+    [..] fp32, element [..], chars [.., 4] int64; weights fp32 as the linear layers hold them."""
+    lib = _L.load()
+    shape, c = tuple(mask.shape), w_pos.shape[0]
+    _gpu(positions, "positions", torch.float32, shape + (3,))
+    _gpu(mask, "mask", torch.float32)
+    _gpu(element, "element", torch.int64, shape)
+    _gpu(charge, "charge", torch.float32, shape)
+    _gpu(chars, "chars", torch.int64, shape + (4,))
+    for nm, w, k in (("w_pos", w_pos, 3), ("w_mask", w_mask, 1), ("w_element", w_element, 128), ("w_charge", w_charge, 1),
+                     ("w_chars", w_chars, 256)):
+        _gpu(w, nm, torch.float32, (c, k))
+    out = torch.empty(shape + (c,), dtype=torch.float32, device=mask.device)
+    rc = lib.af3_atom_embed_forward(_p(positions), _p(mask), _p(element), _p(charge), _p(chars), _p(w_pos), _p(w_mask),
+                                    _p(w_element), _p(w_charge), _p(w_chars), _p(out), mask.numel(), c, _stream(mask.device))
+    _L.check(rc, "af3_atom_embed_forward")
+    return out
+
+
+def gather_atoms(info, cond, mask, positions, uid, add_info=None, add=None):
+    """Atoms in the layout of `info` (gather_idxs int64, gather_mask bool): cond [.., c], mask [..], positions [.., 3] fp32 and
+    uid int64 in the layout given, `add` [rows, c] fp32 gathered by `add_info` on top of cond -> (cond, mask, positions, uid
+    int32) (af3_gather_atoms_forward)."""
+    lib = _L.load()
+    idx, exists, c, slots = info.gather_idxs, info.gather_mask, cond.shape[-1], mask.numel()
+    shape, dev = tuple(idx.shape), cond.device
+    infos = ((info, ""),) if add is None else ((info, ""), (add_info, "add_"))
+    for i, nm in infos:
+        _gpu(i.gather_idxs, nm + "gather_idxs", torch.int64, shape)
+        _gpu(i.gather_mask, nm + "gather_mask", torch.bool, shape)
+    _gpu(cond, "cond", torch.float32)
+    _gpu(mask, "mask", torch.float32)
+    _gpu(positions, "positions", torch.float32)
+    _gpu(uid, "uid", torch.int64)
+    if cond.numel() != slots * c or positions.numel() != slots * 3 or positions.shape[-1] != 3:
+        raise ValueError("cond, mask and positions: expected the same slots")
+    if add is not None:
+        _gpu(add, "add", torch.float32, (add.shape[0], c))
+    out = (torch.empty(shape + (c,), dtype=torch.float32, device=dev), torch.empty(shape, dtype=torch.float32, device=dev),
+           torch.empty(shape + (3,), dtype=torch.float32, device=dev), torch.empty(shape, dtype=torch.int32, device=dev))
+    rc = lib.af3_gather_atoms_forward(
+        _p(idx), _p(exists), idx.numel(), _p(cond), _p(mask), _p(positions), slots, _p(uid), uid.numel(),
+        None if add is None else _p(add_info.gather_idxs), None if add is None else _p(add_info.gather_mask), _p(add),
+        0 if add is None else add.shape[0], *[_p(t) for t in out], c, _stream(dev))
+    _L.check(rc, "af3_gather_atoms_forward")
+    return out
+
+
 def mask_rows(x, mask):
     """x [.., r, c] bf16 times mask [r] fp32 in bf16, in place."""
     lib = _L.load()

@@ -581,6 +581,13 @@ int af3_pairformer_stack_forward(
  *   channel (residue offset 66, token offset 66, same entity, chain offset 6).
  * af3_add_rows_forward: out[r] = a[r] + b[r % mod], a [rows,channels], b [mod][ld_b].
  * af3_mask_rows_forward: x[r] *= mask[r % mod] in bf16, x [rows,channels] in place.
+ * af3_atom_embed_forward: out [atoms,channels], the reference conformer's embedding
+ *   (nn/d_atom_cross_attention.py:93-111) with the weights as the linear layers hold them:
+ *   positions, mask, element (one of 128), asinh(charge), four characters (of 64), times mask.
+ * af3_gather_atoms_forward: atoms in another layout (rows of it; idx into the slots of the
+ *   one given, exists 0 or 1 as a byte): out_cond = cond[idx] exists + add[add_idx]
+ *   add_exists, out_mask, out_positions = .. [idx] exists, out_uid = uid[idx] exists.
+ *   add NULL: none.  A row whose index lies outside comes out as NaN.
  * af3_positions_forward on x [samples,atoms,3], mask [atoms]; level, next: device scalars
  *   op 0: x mask / sqrt(level^2 + 256)
  *   op 1: (c_skip x + c_out y) mask, the head's blend of input and update at noise `level`
@@ -596,6 +603,14 @@ int af3_pair_embed_forward(const float* lr, int64_t ld_lr, const float* prev, co
 int af3_add_rows_forward(const float* a, const float* b, int64_t ld_b, int64_t mod, void* out, int out_dtype, int64_t rows,
                          int channels, af3_stream_t stream);
 int af3_mask_rows_forward(uint16_t* x, const float* mask, int64_t mod, int64_t rows, int channels, af3_stream_t stream);
+int af3_atom_embed_forward(const float* positions, const float* mask, const int64_t* element, const float* charge,
+                           const int64_t* atom_name_chars, const float* w_pos, const float* w_mask, const float* w_element,
+                           const float* w_charge, const float* w_chars, float* out, int64_t atoms, int channels,
+                           af3_stream_t stream);
+int af3_gather_atoms_forward(const int64_t* idx, const uint8_t* exists, int64_t rows, const float* cond, const float* mask,
+                             const float* positions, int64_t slots, const int64_t* uid, int64_t uids, const int64_t* add_idx,
+                             const uint8_t* add_exists, const float* add, int64_t add_rows, float* out_cond, float* out_mask,
+                             float* out_positions, int32_t* out_uid, int channels, af3_stream_t stream);
 int af3_positions_forward(int op, const float* x, const float* y, const float* mask, const float* level, const float* next,
                           float factor, float* out, int64_t samples, int64_t atoms, af3_stream_t stream);
 

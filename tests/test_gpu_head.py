@@ -402,3 +402,30 @@ def test_a_translation_per_sample(gpu_pkg):
     for i in range(2):
         compare(f"sample {i}", got[i], run(trans[:, i, 0, 0])[i], 1e-4, 1e-3)
     assert not torch.allclose(got[0], run(trans[:, 1, 0, 0])[0], rtol=1e-3, atol=1e-3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,padding", [(8, 0), (40, 5), (132, 0)])
+def test_atom_conditioning_in_three_kernels(gpu_pkg, monkeypatch, n, padding):
+    """The atoms' embedding and their layouts against the single operations they stand for, bit for bit."""
+    from distributed_xfold_amd.nn import atom_cross_attention as module
+    with torch.device("cuda"):
+        enc = gpu_pkg.nn.AtomCrossAttEncoder(with_trunk_single_cond=True)
+    batch = gpu_pkg.nn.atom_layout.synthetic_batch(n, torch.Generator().manual_seed(n), n_padding_tokens=padding).to("cuda")
+    rs = batch.ref_structure
+    rs.charge = torch.randn(rs.charge.shape, device="cuda") * 3
+    rs.element[0, :2] = torch.tensor([-1, 127], device="cuda")         # the last one, named twice
+    rs.atom_name_chars[0, 0] = torch.tensor([0, 63, -64, -1], device="cuda")
+    ts = torch.randn(n, 128, device="cuda")
+    outs = []
+    for single_operations in (False, True):
+        monkeypatch.setattr(module, "in_check_mode", lambda: single_operations)
+        act = enc._per_atom_single(batch)
+        outs.append([act, *enc._layouts(batch, act, ts), *enc._layouts(batch, act, None)])
+    for x, y in zip(*outs):
+        assert x.shape == y.shape and torch.isfinite(x.float()).all() and torch.equal(x, y.to(x.dtype))
+    assert all((x != 0).any() for x in outs[0])
+    # an index out of its table is not taken for another atom
+    monkeypatch.setattr(module, "in_check_mode", lambda: False)
+    rs.element[0, 0] = 128
+    assert enc._per_atom_single(batch)[0, 0].isnan().all()
