@@ -72,11 +72,14 @@ static int batched_product(GemmArgs g, bool large, hipStream_t s) {
   g.small_tiles = 1;
   return launch_gemm_nt(g, s);
 }
-// The N x N x N contraction of the triangle multiplication: the large tile once a channel fills enough of one, and, with few
-// channels, there are enough of them.  us, general / large, 128 channels: 132 tokens 8.0 / 8.4, 160 8.4 / 8.9, 192 8.8 / 9.4,
-// but 200 12.9 / 12.0, 256 13.3 / 12.4.  64 channels, a pair block with two of them: 160 tokens 95.5 / 100, 256 141 / 146,
-// 301 201 / 207, 340 252 / 256, 387 355 / 357.
-static int contraction(const GemmArgs& g, hipStream_t s) { return batched_product(g, g.M > (g.batch > 64 ? 192 : 340), s); }
+// The N x N x N contraction of the triangle multiplication: at few tokens a channel's panels in one trip (panel.hip has the line and
+// both sides of it), past those the large tile once a channel fills enough of one, and, with few channels, there are enough of them.
+// us, general / large, 128 channels: 256 tokens 13.3 / 12.4.  64 channels, a pair block with two of them: 340 tokens 252 / 256,
+// 387 355 / 357.
+static int contraction(const GemmArgs& g, hipStream_t s) {
+  if (panel_product_applies(g)) return launch_panel_product(g, s);
+  return batched_product(g, g.batch > 64 || g.M > 340, s);
+}
 
 int run_triangle_contraction(const bf16_t* a_buf, const bf16_t* b_buf, bf16_t* t_buf, int n, int valid_channels, int outgoing, hipStream_t s) {
   // outgoing: t[c][i][j] = sum_k a'[c][i][k] b'[c][j][k]

@@ -37,6 +37,9 @@ struct GemmArgs {
   int split_k = 0;  // the K range may be summed in parts by several waves (another order of summation)
 };
 int launch_gemm_nt(const GemmArgs& g, hipStream_t stream);
+// panel.hip: square products of up to a few hundred rows a batch entry
+bool panel_product_applies(const GemmArgs& g);
+int launch_panel_product(const GemmArgs& g, hipStream_t stream);
 
 // Which tiles of a product run on which XCD.  Each XCD has an L2 of its own, 4 MB, and fetches for itself every row of A
 // and B that its tiles touch.  rows = 0: the XCDs share the tiles (batch, n, m), m fastest, in eight runs: every XCD
