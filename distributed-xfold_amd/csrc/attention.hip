@@ -905,18 +905,20 @@ int launch_nw(const FlashArgs& a, hipStream_t stream) {
                     a.k_ss > 0 && a.v_ss > 0 && a.k_ss < (1 << 22) && a.v_ss < (1 << 22) && a.bias_sq >= 0 &&
                     quad_step > 0 && (int64_t)a.Sq * a.bias_sq + quad_step < (1 << 28);
   // Four waves share each staged K / V tile once there are enough 128-query workgroups to cover the chip; below that, two
-  // waves per workgroup spread the work over twice as many CUs.  Not with head dimension 48 (and padding flags: without them
-  // token_attention_kernel has it), where the form with fixed offsets needs four waves to share the staging registers.
+  // waves per workgroup spread the work over twice as many CUs.  Not with head dimension 48 (and padding flags or a bias
+  // shared by batch % bias_mod: without them token_attention_kernel has it), where the form with fixed offsets needs four waves to
+  // share the staging registers.
   const int nw = a.Sq <= 32 ? 1 : (((a.Sq + 127) / 128) * heads < 256 && !(KSTEPS == 3 && fast) ? 2 : 4);
   const int64_t n_blocks = (int64_t)((a.Sq + nw * 32 - 1) / (nw * 32)) * heads;
   if (n_blocks <= 0 || n_blocks > 0x7ffffff0) return AF3_ERR_BAD_ARG;
   FlashArgs fa = a;
   if constexpr (KSTEPS == 3) {
-    // (byte offsets of 31 bits inside a sample's rows and a head's bias plane, two tiles past the end included; products of the
-    // workgroups' numbers and their divisors of 32)
+    // (padding flags, and a bias that entries share by batch % bias_mod, are flash_kernel's; byte offsets of 31 bits inside a
+    // sample's rows and a head's bias plane, two tiles past the end included; products of the workgroups' numbers and their divisors
+    // of 32)
     const int64_t keys = (a.Sk + 191) / 64 * 64, limit = (int64_t)1 << 29, tiles = (a.Sq + 127) / 128, blocks = tiles * heads;
-    if (fast && !a.qpad && keys * (a.k_ss > a.v_ss ? a.k_ss : a.v_ss) < limit && (int64_t)a.Sq * a.bias_sq + (keys / 4) * quad_step < limit &&
-        blocks * a.B < (1ll << 32) && blocks * tiles < (1ll << 32)) {
+    if (fast && !a.qpad && a.bias_mod == 0 && keys * (a.k_ss > a.v_ss ? a.k_ss : a.v_ss) < limit &&
+        (int64_t)a.Sq * a.bias_sq + (keys / 4) * quad_step < limit && blocks * a.B < (1ll << 32) && blocks * tiles < (1ll << 32)) {
       fa.n_blocks = (int)blocks;
       fa.per_xcd = (int)((blocks + 7) / 8);
       fa.q_tiles = (int)tiles;

@@ -35,3 +35,30 @@ def test_token_attention_gives_the_bits_of_the_general_form(gpu_pkg, batch, n, m
     assert torch.equal(run(logits), want) and torch.equal(run(gpu_pkg.ops.quad_major_bias(logits)), want)
     one = gpu_pkg.ops.batch_diffusion_self_attention(x[:1].contiguous(), keep, logits, w, qb, h, out_dtype=torch.float32)
     assert torch.equal(one, run(logits).view(batch, n, c)[:1].reshape(one.shape))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,shared,sq,sk", [(2, 1, 4, 4), (4, 2, 36, 68), (6, 3, 33, 36), (6, 1, 128, 200), (5, 5, 130, 64), (3, 1, 1, 132)])
+def test_a_bias_that_batch_entries_share(gpu_pkg, batch, shared, sq, sk):
+    """Cross-attention of heads of 48 without padding masks: entry b reads the logits b % shared, against float64 arithmetic on the
+    projections as they are stored.  What is left are roundings to 8 bits (probabilities, a projection that falls on the other side of
+    one): 1e-2 of the result's rms."""
+    g = torch.Generator(device="cuda").manual_seed(100 * batch + sk)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    c, h = 192, 4
+    q, m, qb = rnd(batch, sq, c).bfloat16(), rnd(batch, sk, c).bfloat16(), rnd(c)
+    w_qg, w_kv = ((rnd(2 * c, c) * 0.07).bfloat16() for _ in range(2))
+    logits = rnd(shared, h, sq, sk) * 3
+    got = gpu_pkg.ops.batch_diffusion_cross_attention(q, m, logits, None, None, w_qg, w_kv, qb, h, out_dtype=torch.float32)
+    heads = lambda x: x.bfloat16().double().view(batch, -1, h, c // h).transpose(1, 2).contiguous()
+    (pq, pg), (pk, pv) = (x.double().matmul(w.double().t()).split(c, -1) for x, w in ((q, w_qg), (m, w_kv)))
+    s = heads((pq + qb.double()) / (c // h) ** 0.5).matmul(heads(pk).transpose(2, 3).contiguous())
+    s = s + logits.double()[torch.arange(batch, device="cuda") % shared]
+    want = (s.softmax(-1).matmul(heads(pv)) * heads(torch.sigmoid(pg))).transpose(1, 2)
+    scale = want.pow(2).mean().sqrt()
+    assert (got - want).pow(2).mean().sqrt() <= 1e-2 * scale and (got - want).abs().max() <= 0.1 * scale
+    # ... as if the entries that share it had been called by themselves
+    for b in range(batch):
+        one = gpu_pkg.ops.batch_diffusion_cross_attention(q[b:b + 1].contiguous(), m[b:b + 1].contiguous(), logits[b % shared][None].contiguous(),
+                                                          None, None, w_qg, w_kv, qb, h, out_dtype=torch.float32)
+        assert torch.equal(one[0], got[b])
