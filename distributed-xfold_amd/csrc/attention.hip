@@ -488,24 +488,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void t
   const int q0 = (rest - h * a.q_tiles) * 128 + wave * 32, qi = min(q0 + j, a.Sq - 1);  // clamped for loads; stores are guarded
   const int nkt = (a.Sk + KT - 1) / KT;
 
-  auto rows_of = [&](const bf16_t* p, int64_t sb, int64_t ss) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p + b * sb + h * TOK_D), 0, (int)((a.Sk - 1) * ss + TOK_D) * 2, RSRC_RAW);
+  // The descriptor of a tile begins at its first key (or quad) and ends where the plane does: a lane's offset never changes, and all
+  // of what lies past the last key is past the descriptor's end by that offset alone (the scalar one stays 0: what it may add
+  // to a checked offset is not laid down).
+  auto from = [](const void* p, int bytes, int at) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(static_cast<const char*>(p) + at), 0, max(bytes - at, 0), RSRC_RAW);
   };
-  const __amdgpu_buffer_rsrc_t kres = rows_of(a.k, a.k_sb, a.k_ss), vres = rows_of(a.v, a.v_sb, a.v_ss);
+  const bf16_t *const kg = a.k + b * a.k_sb + h * TOK_D, *const vg = a.v + b * a.v_sb + h * TOK_D;
+  const int k_bytes = ((a.Sk - 1) * (int)a.k_ss + TOK_D) * 2, v_bytes = ((a.Sk - 1) * (int)a.v_ss + TOK_D) * 2;
+  const int k_step = KT * (int)a.k_ss * 2, v_step = KT * (int)a.v_ss * 2;
   const int quad_step = (int)(a.bias_squad ? a.bias_squad : 4), quads = (a.Sk + 3) >> 2;
-  const __amdgpu_buffer_rsrc_t bres = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(a.bias + (int64_t)b * a.bias_sb + (int64_t)h * a.bias_sh), 0,
-      ((a.Sq - 1) * (int)a.bias_sq + (quads - 1) * quad_step + 4) * 4, RSRC_RAW);
+  const float* const bg = a.bias + (int64_t)b * a.bias_sb + (int64_t)h * a.bias_sh;
+  const int b_bytes = ((a.Sq - 1) * (int)a.bias_sq + (quads - 1) * quad_step + 4) * 4, b_step = KT / 4 * quad_step * 4;
   const float* kmask = a.key_mask ? a.key_mask + (int64_t)b * a.km_sb : nullptr;
 
   // bias of a tile in four parts of two quads: part p = registers 8 p .. of the 32,
   // s[u][4 g + e] = bias(query, key 64 kt + 32 u + 8 g + 4 hh + e)
-  const uint32_t bias_lane = (uint32_t)(qi * (int)a.bias_sq + hh * quad_step) * 4u;
+  uint32_t quad_at[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) quad_at[i] = (uint32_t)(qi * (int)a.bias_sq + (hh + 2 * i) * quad_step) * 4u;
   auto load_bias = [&](f32x16 (&s)[2], int kt, int part) {
     const int u = part >> 1;
+    const __amdgpu_buffer_rsrc_t rest = from(bg, b_bytes, kt * b_step);
 #pragma unroll
     for (int g = 2 * (part & 1); g < 2 * (part & 1) + 2; ++g) {
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(bres, bias_lane, (kt * (KT / 4) + 8 * u + 2 * g) * quad_step * 4, 0);
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rest, quad_at[4 * u + g], 0, 0);
 #pragma unroll
       for (int e = 0; e < 4; ++e) s[u][4 * g + e] = __uint_as_float(v[e]);
     }
@@ -523,11 +530,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void t
   }
   float mask_value = 1.f;  // of key tid of the tile asked for last (threads 0..63)
   auto load_tile = [&](int kt) {
-    const int ks = kt * KT * (int)a.k_ss * 2, vs = kt * KT * (int)a.v_ss * 2;
+    const __amdgpu_buffer_rsrc_t krest = from(kg, k_bytes, kt * k_step), vrest = from(vg, v_bytes, kt * v_step);
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      if (wave * 64 + i * 256 < CHUNKS) rc[i] = __builtin_amdgcn_raw_buffer_load_b128(kres, choff[i], ks, 0);
-      else rc[i] = __builtin_amdgcn_raw_buffer_load_b128(vres, choff[i], vs, 0);
+      if (wave * 64 + i * 256 < CHUNKS) rc[i] = __builtin_amdgcn_raw_buffer_load_b128(krest, choff[i], 0, 0);
+      else rc[i] = __builtin_amdgcn_raw_buffer_load_b128(vrest, choff[i], 0, 0);
     }
     if (kmask && tid < KT) mask_value = kmask[min(kt * KT + tid, a.Sk - 1)];
   };

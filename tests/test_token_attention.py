@@ -62,3 +62,30 @@ def test_a_bias_that_batch_entries_share(gpu_pkg, batch, shared, sq, sk):
         one = gpu_pkg.ops.batch_diffusion_cross_attention(q[b:b + 1].contiguous(), m[b:b + 1].contiguous(), logits[b % shared][None].contiguous(),
                                                           None, None, w_qg, w_kv, qb, h, out_dtype=torch.float32)
         assert torch.equal(one[0], got[b])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quads", [False, True])
+@pytest.mark.parametrize("batch,n", [(1, 4), (2, 36), (1, 64), (2, 68), (5, 100), (1, 132), (1, 260)])
+def test_what_lies_behind_the_last_key_is_not_read(gpu_pkg, batch, n, quads):
+    """A last tile that is not full, and the tiles asked for past it, with NaN behind the projections and behind the logits: the bits
+    of zeros in their place."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    c, h, lib = 768, 16, gpu_pkg.lib.load()
+    x, w, qb = rnd(batch, n, c).bfloat16(), (rnd(4 * c, c) * 0.05).bfloat16(), rnd(c)
+    plane = rnd(h, n, n) * 3
+    if quads:
+        plane = gpu_pkg.ops.quad_major_bias(plane)
+    need, outs = lib.af3_batch_diffusion_self_attention_workspace_bytes(batch, n, c), []
+    for behind in (0.0, float("nan")):
+        ws = torch.full((need // 2 + 512 * 4 * c,), behind, dtype=torch.bfloat16, device="cuda")
+        logits = torch.full((plane.numel() + 256 * (n + 4),), behind, device="cuda")
+        logits[:plane.numel()] = plane.flatten()
+        out = torch.empty(batch, n, h, c // h, device="cuda")
+        gpu_pkg.lib.check(lib.af3_batch_diffusion_self_attention_forward(
+            x.data_ptr(), None, 1, logits.data_ptr(), int(quads), w.data_ptr(), qb.data_ptr(), h, out.data_ptr(), gpu_pkg.lib.AF3_F32,
+            batch, n, c, ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream), "self-attention")
+        outs.append(out)
+    assert torch.isfinite(outs[1]).all() and torch.equal(*outs)
+    assert torch.equal(outs[0], gpu_pkg.ops.batch_diffusion_self_attention(x, None, plane, w, qb, h, out_dtype=torch.float32))
