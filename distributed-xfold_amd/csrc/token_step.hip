@@ -299,8 +299,10 @@ __global__ __launch_bounds__(64 * WAVES, 1) void gated_product_kernel(GatedProdu
   }
   fetch(PIECE(3));
   fetch(PIECE(4));
-  // (what was asked for behind the panel may be on its way still)
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * RING + 6) : "memory");
+  // The fragments asked for behind the panel may be on their way still.  Loads issued behind it that are not counted only make the
+  // wait longer, ones counted and not issued would end it too soon: so the fragments alone, which sched_barrier keeps where they
+  // are, and not gate and stream (the first matrix instruction waits for more than the six loads that this costs).
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * RING) : "memory");
   lds_barrier();
 
   f32x16 acc;
@@ -343,13 +345,14 @@ __global__ __launch_bounds__(64 * WAVES, 1) void gated_product_kernel(GatedProdu
 
 // The same products over more rows: x w^T with the weights' fragments straight from memory to registers and the rows through LDS.
 // A workgroup takes 64 rows x 128 columns, a wave all rows of 32 columns; slabs of 64 channels of the rows go straight into a ring
-// of LDS buffers that the four waves share, with one barrier a slab; a wave's fragments are RP_RING slabs ahead.  Bound by the CU's vector memory path: 3 KB of weights and rows
-// for 16 matrix instructions of a wave.  Three workgroups a CU with four slabs ahead, two with six to eight (us, queries to gate
-// at 640, 1920 and 3840 rows): 6.6 13.2 24.0, 6.8 13.4 24.3.
+// of LDS buffers that the four waves share, with one barrier a slab; a wave's fragments are RP_RING slabs ahead.  Bound by the CU's
+// vector memory path: 3 KB of weights and rows for 16 matrix instructions of a wave.  Three workgroups a CU with four slabs ahead,
+// two with six to eight (us, queries to gate at 640, 1920 and 3840 rows): 6.6 13.2 24.0, 6.8 13.4 24.3.
 enum { ROWS_QKVG, ROWS_SWIGLU, ROWS_GATED };
 constexpr int RP_BM = 64, RP_BN = 128, RP_BUFFERS = 4, RP_RING = 4, RP_PER_CU = 3;
 static_assert(RP_RING >= RP_BUFFERS);  // (rows_product_younger counts on it)
-// loads of a wave issued behind its two for slab s of the rows, when it waits for these (step s - 1 of the loop)
+// loads of a wave issued behind its two for slab s of the rows, when it waits for these (step s - 1 of the loop): statements and loads
+// that sched_barrier keeps in this order; any others issued between them only make the wait longer
 constexpr int rows_product_younger(int s, int slabs) {
   int n = 0;
   auto steps = [&](int from) {
