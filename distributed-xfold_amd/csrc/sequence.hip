@@ -572,7 +572,9 @@ int af3_diffusion_transformer_forward(
     const af3_diffusion_block& b = blocks[i];
     const float* ss = scale_shift + (int64_t)2 * i * 2 * c;
     if (steps) {
-      auto warm = [](NormProductArgs& a, int k, const void* p, size_t bytes) { a.warm[k] = p; a.warm_lines[k] = (uint32_t)(bytes / 128); };
+      auto warm = [](NormProductArgs& a, int k, const void* p, size_t bytes) {  // (a null entry of pair_logits is no bias)
+        if (p) { a.warm[k] = p; a.warm_lines[k] = (uint32_t)(bytes / 128); }
+      };
       NormProductArgs a = step(i, false);
       warm(a, 0, weights_back(i, false), (size_t)c * c * 2);
       warm(a, 1, b.frags + (int64_t)4 * c * c, (size_t)2 * hidden * c * 2);

@@ -671,7 +671,7 @@ int af3_evoformer_stack_forward(
  *
  * af3_diffusion_transformer_forward: act [batch,seq,c] in act_dtype, key_mask [seq]
  *   or NULL, pair_logits: num_blocks HOST pointers to device planes [num_head,seq,seq]
- *   fp32, or [num_head,seq/4,seq,4] with bias_quad_major.
+ *   fp32, or [num_head,seq/4,seq,4] with bias_quad_major; NULL: none for that block.
  * af3_atom_transformer_forward: act [samples,subsets,queries,c]; key k of subset s is
  *   atom key_rows[s,k] of the sample's subsets * queries (negative: empty slot, K = V
  *   = 0), see af3_gathered_cross_attention_forward; scale_shift_k [subsets * queries]

@@ -1,5 +1,7 @@
 """The token transformer's kernels (token_step.hip) against the operators one by one."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -33,3 +35,29 @@ def test_the_steps_give_the_bits_of_the_operators(gpu_pkg, samples, n, factor):
     got = run()
     hook.remove()
     assert seen and torch.isfinite(want).all() and not torch.equal(want, act) and torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("samples,n", [(1, 40), (5, 100), (6, 20)])
+def test_a_null_plane_of_logits_is_no_bias(gpu_pkg, samples, n):
+    """The library call takes one pointer to pair logits for each block; the bits of logits that are zero."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    with torch.device("cuda"):
+        mod = gpu_pkg.nn.DiffusionTransformer(num_blocks=2, super_block_size=1)
+    with torch.no_grad():
+        for p in mod.parameters():
+            p.normal_(0.0, 0.05, generator=g)
+    lib, L, c = gpu_pkg.lib.load(), gpu_pkg.lib, 768
+    table = gpu_pkg.nn.diffusion_transformer.block_table(mod, mod._blocks(), c)
+    act, ss, gate = rnd(samples, n, c).bfloat16(), rnd(n, 4, 2 * c), torch.sigmoid(rnd(n, 4, c))
+    logits, zeros, outs = rnd(16, n, n), torch.zeros(16, n, n, device="cuda"), []
+    need = lib.af3_diffusion_transformer_workspace_bytes(samples, n, c, table.hidden)
+    for second in (zeros.data_ptr(), None):
+        x, ws = act.clone(), torch.empty(need, dtype=torch.uint8, device="cuda")
+        planes = (ctypes.c_void_p * 2)(logits.data_ptr(), second)
+        L.check(lib.af3_diffusion_transformer_forward(
+            table, 2, x.data_ptr(), L.AF3_BF16, samples, n, c, table.hidden, 16, None, planes, 0, ss.data_ptr(), gate.data_ptr(), n,
+            ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream), "transformer")
+        outs.append(x)
+    assert torch.isfinite(outs[0]).all() and not torch.equal(outs[0], act) and torch.equal(*outs)
