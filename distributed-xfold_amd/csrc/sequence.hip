@@ -494,6 +494,8 @@ int af3_diffusion_transformer_forward(
   const size_t ab = af3_batch_diffusion_self_attention_workspace_bytes(batch, seq, c);
   void* aw = w.take(ab);
   if (!w.ok) return AF3_ERR_WORKSPACE;
+  for (int i = 0; i < num_blocks; ++i)  // (`frags` stand beside the weights, not in their place)
+    if (!blocks[i].w_q || !blocks[i].w_out || !blocks[i].w_tr1 || !blocks[i].w_tr2) return AF3_ERR_BAD_ARG;
   // Adaptive LayerNorm of act, with the weights of the products up to the next one on their way into the last-level cache
   // (rowops.hip), and the pair logits where they are no more than the weights.  The conditioning of those products, rows of
   // 6 KB some 300 KB apart, costs more that way than it saves.

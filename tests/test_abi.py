@@ -191,6 +191,24 @@ def test_gathered_cross_attention_and_regrouped_store_reject_bad_arguments(pkg):
     assert lib.af3_linear_forward(one, one, None, one, 0, 64, 64, 8, 3, 1.0, 0, one, 1, 32, None, 0, None) == -1  # gate rows overlap
 
 
+@pytest.mark.parametrize("samples", [5, 6])            # few rows, and the route of many
+@pytest.mark.parametrize("missing", ["w_q", "w_out", "w_tr1", "w_tr2"])
+def test_diffusion_transformer_wants_its_weights_beside_the_fragments(pkg, missing, samples):
+    """A block without one of its matrices is refused, in the first block or in a later one, with fragments or without."""
+    lib, one = pkg.lib.load(), 1 << 20
+    for at in (0, 1):
+        for frags in (one, None):
+            blocks = (pkg.lib.DiffusionBlockStruct * 2)()
+            for b in blocks:
+                for name in ("w_q", "q_b", "w_out", "w_tr1", "w_tr2", "frags"):
+                    setattr(b, name, one)
+                b.frags = frags
+            setattr(blocks[at], missing, None)
+            planes = (ctypes.c_void_p * 2)(one, one)
+            assert lib.af3_diffusion_transformer_forward(blocks, 2, one, pkg.lib.AF3_BF16, samples, 100, 768, 1536, 16, None, planes, 0, one,
+                                                         one, 100, one, 1 << 40, None) == -1
+
+
 def test_quad_major_bias_layout_and_its_argument_check(pkg):
     """[H, Sq, Sk] -> [H, Sk/4, Sq, 4]: element (h, q, k) at ((h * Sk/4 + k/4) * Sq + q) * 4 + k%4."""
     bias = torch.arange(2 * 6 * 8, dtype=torch.float32).reshape(2, 6, 8)
