@@ -159,7 +159,7 @@ struct GatherAtoms {
     const int64_t row = item / chunks;
     const int c = (int)(item - row * chunks) * 8;
     const int64_t at = a.idx[row], add_at = a.add ? a.add_idx[row] : 0;
-    const bool ok = at >= 0 && at < a.slots && add_at >= 0 && add_at < a.add_rows;  // (else the row is not a number)
+    const bool ok = at >= 0 && at < a.slots && add_at >= 0 && add_at < a.add_rows;  // (else the row is not a number, its uid 0)
     const float m = a.exists[row] ? 1.f : 0.f;
     float o[8], x[8];
     Elem<float>::load8(a.cond + (ok ? at : 0) * a.channels + c, o);
@@ -177,9 +177,9 @@ struct GatherAtoms {
     Elem<float>::store8(a.out_cond + item * 8, o);
     if (c != 0) return;
     const int64_t from = ok ? at : 0;
-    a.out_mask[row] = a.mask[from] * m;
+    a.out_mask[row] = ok ? a.mask[from] * m : __builtin_nanf("");
 #pragma unroll
-    for (int e = 0; e < 3; ++e) a.out_pos[row * 3 + e] = a.pos[from * 3 + e] * m;
+    for (int e = 0; e < 3; ++e) a.out_pos[row * 3 + e] = ok ? a.pos[from * 3 + e] * m : __builtin_nanf("");
     a.out_uid[row] = ok && a.exists[row] && at < a.uids ? (int)a.uid[at] : 0;
   }
 };

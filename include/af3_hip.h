@@ -587,7 +587,8 @@ int af3_pairformer_stack_forward(
  * af3_gather_atoms_forward: atoms in another layout (rows of it; idx into the slots of the
  *   one given, exists 0 or 1 as a byte): out_cond = cond[idx] exists + add[add_idx]
  *   add_exists, out_mask, out_positions = .. [idx] exists, out_uid = uid[idx] exists.
- *   add NULL: none.  A row whose index lies outside comes out as NaN.
+ *   add NULL: none.  A row with an index (either of the two) that lies outside comes out as
+ *   NaN in all three, its uid as 0.
  * af3_positions_forward on x [samples,atoms,3], mask [atoms]; level, next: device scalars
  *   op 0: x mask / sqrt(level^2 + 256)
  *   op 1: (c_skip x + c_out y) mask, the head's blend of input and update at noise `level`

@@ -5,6 +5,8 @@ seconds, and size-independent properties at 768 tokens x 5 samples.
 Tolerances: bf16 path rms error of the position UPDATE (denoised minus the
 skip term) <= 1e-2 of its rms, max <= 8e-2; fp32 check mode 2e-4 / 2e-3."""
 
+import types
+
 import pytest
 import torch
 
@@ -429,3 +431,24 @@ def test_atom_conditioning_in_three_kernels(gpu_pkg, monkeypatch, n, padding):
     monkeypatch.setattr(module, "in_check_mode", lambda: False)
     rs.element[0, 0] = 128
     assert enc._per_atom_single(batch)[0, 0].isnan().all()
+
+
+@pytest.mark.gpu
+def test_an_atom_index_outside_its_table_gives_nan_everywhere(gpu_pkg):
+    """Either index of a row out of range: conditioning, mask and position are NaN, the uid is 0, and the other rows are as they were."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    info = lambda n: types.SimpleNamespace(gather_idxs=torch.randint(0, n, (6, 32), generator=g, device="cuda"),
+                                           gather_mask=torch.ones(6, 32, dtype=torch.bool, device="cuda"))
+    atoms, tokens = info(192), info(8)
+    args = rnd(6, 32, 128), (rnd(6, 32) > 0).float(), rnd(6, 32, 3), torch.randint(1, 9, (6, 32), generator=g, device="cuda")
+    ones = torch.ones(8, 128, device="cuda")
+    want = gpu_pkg.ops.gather_atoms(atoms, *args, tokens, ones)
+    bad = torch.zeros(6, 32, dtype=torch.bool, device="cuda")
+    for which, at, value in ((atoms, (0, 0), 192), (atoms, (1, 5), -1), (atoms, (5, 31), 2 ** 40), (tokens, (2, 3), 8), (tokens, (4, 0), -1)):
+        which.gather_idxs[at] = value
+        bad[at] = True
+    got = gpu_pkg.ops.gather_atoms(atoms, *args, tokens, ones)
+    for x, y in zip(got[:3], want[:3]):
+        assert x[bad].isnan().all() and torch.equal(x[~bad], y[~bad])
+    assert (got[3][bad] == 0).all() and torch.equal(got[3][~bad], want[3][~bad])
