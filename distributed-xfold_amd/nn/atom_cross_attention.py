@@ -97,6 +97,7 @@ class AtomCrossAttEncoder(HipModule):
         self.embed_ref_pos, self.embed_ref_mask = lin(3, ca), lin(1, ca)
         self.embed_ref_element, self.embed_ref_charge = lin(128, ca), lin(1, ca)
         self.embed_ref_atom_name = lin(64 * 4, ca)
+        # (of the conformer's pair embedding, :112-156, which `conditioning` does not read: here for the state dict alone)
         self.single_to_pair_cond_row, self.single_to_pair_cond_col = lin(ca, cp), lin(ca, cp)
         self.embed_pair_offsets, self.embed_pair_distances = lin(3, cp), lin(1, cp)
         self.single_to_pair_cond_row_1, self.single_to_pair_cond_col_1 = lin(ca, cp), lin(ca, cp)
@@ -145,18 +146,6 @@ class AtomCrossAttEncoder(HipModule):
         for j in range(4):
             act = act + wn[j][chars[..., j]]
         return act * m[:, :, None]
-
-    def _per_atom_conditioning(self, batch):
-        """:87-156 -> (act [N, A, 128], pair_act [N, A, A, 16]), fp32."""
-        rs = batch.ref_structure
-        act = self._per_atom_single(batch)
-        pair_act = (_lin(act, self.single_to_pair_cond_row, relu_input=True)[:, :, None, :]
-                    + _lin(act, self.single_to_pair_cond_col, relu_input=True)[:, None, :, :])
-        pos = rs.positions.float()
-        d = pos[:, :, None, :] - pos[:, None, :, :]
-        pair_act = pair_act + _lin(d, self.embed_pair_offsets)
-        pair_act = pair_act + _lin(1.0 / (1 + (d * d).sum(-1, keepdim=True)), self.embed_pair_distances)
-        return act, pair_act
 
     @staticmethod
     def _layouts(batch, tok_single, ts):
