@@ -77,8 +77,8 @@ static int batched_product(GemmArgs g, bool large, hipStream_t s) {
 // us, general / large, 128 channels: 256 tokens 13.3 / 12.4.  64 channels, a pair block with two of them: 340 tokens 252 / 256,
 // 387 355 / 357.
 static int contraction(const GemmArgs& g, hipStream_t s) {
-  if (panel_product_applies(g)) return launch_panel_product(g, s);
-  return batched_product(g, g.batch > 64 || g.M > 340, s);
+  const int rc = launch_panel_product(g, s);
+  return rc != AF3_ERR_UNSUPPORTED ? rc : batched_product(g, g.batch > 64 || g.M > 340, s);
 }
 
 int run_triangle_contraction(const bf16_t* a_buf, const bf16_t* b_buf, bf16_t* t_buf, int n, int valid_channels, int outgoing, hipStream_t s) {

@@ -37,8 +37,7 @@ struct GemmArgs {
   int split_k = 0;  // the K range may be summed in parts by several waves (another order of summation)
 };
 int launch_gemm_nt(const GemmArgs& g, hipStream_t stream);
-// panel.hip: square products of up to a few hundred rows a batch entry
-bool panel_product_applies(const GemmArgs& g);
+// panel.hip: square products of up to a few hundred rows a batch entry; AF3_ERR_UNSUPPORTED for others
 int launch_panel_product(const GemmArgs& g, hipStream_t stream);
 
 // Which tiles of a product run on which XCD.  Each XCD has an L2 of its own, 4 MB, and fetches for itself every row of A

@@ -156,19 +156,15 @@ static bool panel_args(const GemmArgs& g, PanelArgs* a, int* lds) {
   return true;
 }
 
-bool panel_product_applies(const GemmArgs& g) {
-  PanelArgs a;
-  int lds;
-  return panel_args(g, &a, &lds);
-}
-
 int launch_panel_product(const GemmArgs& g, hipStream_t s) {
   PanelArgs a;
   int lds;
-  if (!panel_args(g, &a, &lds)) return AF3_ERR_BAD_ARG;
-  if (lds > 65536) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(panel_product_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (!panel_args(g, &a, &lds)) return AF3_ERR_UNSUPPORTED;
+  // (more than 64 KB have to be asked for; always for as much as there is, since another thread may be launching with another size)
+  if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(panel_product_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         PANEL_LDS) != hipSuccess) {
     (void)hipGetLastError();
+    return AF3_ERR_LAUNCH;
   }
   hipLaunchKernelGGL(panel_product_kernel, dim3((unsigned)((g.batch + 7) / 8 * 8 * a.parts * a.column_parts)), dim3(64 * WAVES), lds, s, a);
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;

@@ -787,10 +787,11 @@ int launch_triattn_flash(const TriAttnArgs& a, hipStream_t stream) {
   const size_t stat = (R == 2 ? 8 : 4) * (size_t)tile + 1024;
   auto launch = [&](void (*kernel)(TriAttnArgs)) {
     // more than 64 KB of LDS per workgroup in all (static + dynamic) has to be asked for
-    // (a per-function, per-device setting of the runtime: no allocation, no synchronisation)
+    // (a per-function, per-device setting of the runtime: no allocation, no synchronisation; always for the most tokens, since
+    // another thread may be launching with another size)
     if (stat + dyn > 65536) {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)dyn);
+                                (int)(2 * 8192 * sizeof(uint16_t)));
       (void)hipGetLastError();
     }
     hipLaunchKernelGGL(kernel, grid, block, dyn, stream, args);

@@ -1,5 +1,7 @@
 """The triangle contraction at few tokens, on the kernel that takes a channel's panels in one trip and on either side of its line."""
 
+import threading
+
 import pytest
 import torch
 
@@ -41,3 +43,34 @@ def test_panels_of_half_the_channels(gpu_pkg, n):
     want = O.triangle_multiplication(pair.double(), mask.double(), {k: v.double().cuda() for k, v in p.items()}, True)
     scale = want.pow(2).mean().sqrt()
     assert (got - want).pow(2).mean().sqrt() <= 1e-2 * scale and (got - want).abs().max() <= 8e-2 * scale
+
+
+@pytest.mark.gpu
+def test_panels_of_several_sizes_from_several_threads(gpu_pkg):
+    """Sizes that ask for different amounts of LDS, launched by threads with a stream each."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    sizes, got, failed = (97, 160, 193, 224), {}, []
+    start = threading.Barrier(len(sizes))
+    ops = {n: [torch.randn(128, n, (n + 7) // 8 * 8, generator=g, device="cuda").bfloat16() for _ in range(2)] for n in sizes}
+    for n in sizes:
+        for x in ops[n]:
+            x[..., n:] = 0
+    want = {n: gpu_pkg.ops.triangle_contraction(*ops[n]) for n in sizes}
+    torch.cuda.synchronize()
+
+    def work(n):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                start.wait()
+                got[n] = [gpu_pkg.ops.triangle_contraction(*ops[n]) for _ in range(100)]
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:
+            failed.append((n, e))
+    threads = [threading.Thread(target=work, args=(n,)) for n in sizes]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed
+    for n in sizes:
+        assert all(torch.equal(x[..., :n], want[n][..., :n]) for x in got[n])
