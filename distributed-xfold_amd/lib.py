@@ -8,7 +8,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libaf3hip.so")
 
-ABI_VERSION = 3                      # AF3_ABI_VERSION: of the structures and argument lists below
+ABI_VERSION = 4                      # AF3_ABI_VERSION: of the structures and argument lists below
 AF3_BF16, AF3_F32 = 0, 1
 STATIC_SCRATCH_BYTES = 32 << 20      # AF3_STATIC_SCRATCH_BYTES
 LINEAR_PLAIN, LINEAR_SWIGLU, LINEAR_GATE_RES, LINEAR_REGROUP32, LINEAR_ROWGATE_RES = 0, 2, 3, 4, 5

@@ -51,8 +51,10 @@ typedef void* af3_stream_t; /* a hipStream_t */
  * order and vt has its quads swapped (version 1 took a bf16 bias and a gate).
  * 3: af3_pairformer_block (so af3_msa_block, which holds one, too) has pair_frags
  * and pair_channels, af3_diffusion_block has frags.  A caller of version 2 passes
- * shorter structures, from which this library would take other fields. */
-#define AF3_ABI_VERSION 3
+ * shorter structures, from which this library would take other fields.
+ * 4: af3_diffusion_transformer_forward reads frags of af3_diffusion_block, in an
+ * order of its own.  A caller of version 3 may have left anything there. */
+#define AF3_ABI_VERSION 4
 int af3_abi_version(void);
 const char* af3_error_string(int code);
 
