@@ -5,6 +5,9 @@ import ctypes
 import pytest
 import torch
 
+from bf16_tolerances import RMS_TOL, cap
+from oracle import af3_oracle as O
+
 
 # tiles hold all samples of 4 to 16 tokens, by the number of samples and of tiles: one token, tiles that are filled and that are
 # not, both sizes of every number of samples, one number that has no such kernel, more tokens than it takes, weights of 6 to 18 tiles;
@@ -61,3 +64,26 @@ def test_a_null_plane_of_logits_is_no_bias(gpu_pkg, samples, n):
             ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream), "transformer")
         outs.append(x)
     assert torch.isfinite(outs[0]).all() and not torch.equal(outs[0], act) and torch.equal(*outs)
+
+
+# norm and product in one kernel with the gated one (one to five samples, the most rows of either, one more), in kernels of their own
+# (2688 rows are the most for all three products, 2695 take one of them)
+@pytest.mark.gpu
+@pytest.mark.parametrize("samples,n", [(1, 33), (3, 100), (5, 126), (5, 134), (5, 135), (7, 384), (7, 385)])
+def test_a_bf16_stream_against_the_oracle(gpu_pkg, samples, n):
+    """The update of two blocks to the tolerances of an fp32 stream, and four roundings of the stream to 8 bits on top: each at most
+    2^-9 of a value, of their rms no more than that (independent: twice for four) and at most four times at any place."""
+    g = torch.Generator().manual_seed(n)
+    rb = O.round_bf16
+    p = {k: rb(v) for k, v in O.make_diffusion_transformer_params(g, num_blocks=2, super_block_size=2, std=0.05).items()}
+    mod = gpu_pkg.nn.DiffusionTransformer(num_blocks=2, super_block_size=2)
+    mod.load_state_dict(p)
+    mod = mod.cuda()
+    act, cond, pair = (rb(torch.randn(*s, generator=g)).cuda() for s in ((samples, n, 768), (n, 384), (n, n, 128)))
+    mask = (torch.arange(n, device="cuda") < n - n // 8).float()
+    got = mod(act.bfloat16(), mask, cond, pair).double()
+    want = O.diffusion_transformer(act.double(), mask.double(), cond.double(), pair.double(), {k: v.double().cuda() for k, v in p.items()}, 16, 2, 2)
+    rms = lambda x: x.pow(2).mean().sqrt()
+    scale = rms(want - act)
+    assert rms(got - want) <= RMS_TOL * scale + 2 * 2.0 ** -9 * rms(want)
+    assert (got - want).abs().max() <= cap("diffusion_transformer") * scale + 4 * 2.0 ** -9 * want.abs().max()
