@@ -53,7 +53,6 @@ __device__ __forceinline__ void multiply(const PanelArgs& a, const char* sA, con
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[r][c][e] = 0.f;
   const int steps = a.stride >> 1;  // (the stride is one more than the chunks of a row, two to a step)
-#pragma unroll 4
   for (int k = 0; k < steps; ++k) {
     bf16x8 fa[NR], fb[NC];
 #pragma unroll

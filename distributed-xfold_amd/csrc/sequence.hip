@@ -68,6 +68,8 @@ struct Event {
 //   768         9686 / 9771   2469 / 2505  11183 / 10607;  3 blocks: 1024 19673 / 18762, 1280 33765 / 32302, 1536 52463 / 52510
 // Pair tensors of 64 channels have no other kernels (64 / 301 / 768 / 2048 tokens, bf16, a block on its own: 100 -> 46,
 // 345 -> 221, 1940 -> 1460, 22400 -> 18800 against one zero-padded to 128; their 32-bit offsets end at 3072).
+// The bf16 line lies below 512 tokens, the first size at which one of the two is behind (a block on its own, by 1 %); 550 is ahead
+// once more, by 1 to 2 %, 600 behind.
 constexpr int64_t BF16_STEP_POSITIONS = 500 * 500, F32_STEP_POSITIONS = 1280 * 1280;
 // The outgoing epilogue and the incoming prologue are one step while its patches are one round of workgroups: it stores transposed
 // operands 8 or 16 bytes at a time, which costs more than the pass and the launch it saves beyond (a stack of 4 blocks, us, two
@@ -425,8 +427,9 @@ int af3_pairformer_stack_forward(
   // (the wait in front of the first update of `single` is for what `stream` holds on entry, too)
   if (two && singles == 0) STEP(ready.order(main_s, side_s));
   // Where launches set the pace the updates of two blocks wait for the streams' meeting together, but for the last one, which has no
-  // pair operators to run beside.  With the wait on entry, that is four meetings for four blocks instead of six: 64 tokens 408 -> 362
-  // us, 45 400 -> 352, 128 480 -> 470; past 144 tokens the pair operators are longer than what an update waits for (176: 683 -> 689).
+  // pair operators to run beside.  With the wait on entry, that is four meetings for four blocks instead of six: 64 tokens 381 -> 343
+  // us (321 -> 308 in a process that launches faster), 45 382 -> 339, 128 464 -> 454; past 144 tokens the pair operators are longer
+  // than what an update waits for (176, two together: 683 -> 689).
   const bool by_two = buffers == PairStepScratch::LOGIT_RING && n * tri_ldn(n) <= 144 * 144;
   int rc = AF3_OK, k = 0, done = 0, from = 0;  // single tracks whose logits are on their way, those enqueued; the block of the next one
   for (int i = 0; i < num_blocks && rc == AF3_OK; ++i) {

@@ -503,7 +503,8 @@ bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 // Tokens of a tile, by the number of samples.  One of fewer leaves rows of the matrix instruction empty, but its norms are done
 // sooner: taken while every tile has a CU of its own (24 blocks, us: 1 x 100 tokens by 32 1174, by 8 1024; 3 x 152 by 8 1203, 3 x 160
-// by 10 1284; 5 x 76 by 4 1110, 5 x 80 by 6 1097).
+// by 10 1284; 5 x 76 by 4 1110, 5 x 80 by 6 1097).  Five samples are the most: a wave keeps all rows of its token in registers
+// while it normalises them (222 and 233 of 256 with five); six take norm and product in kernels of their own.
 static int tile_tokens(const NormProductArgs& a) {
   static constexpr int sizes[5][2] = {{8, 16}, {8, 16}, {8, 10}, {4, 8}, {4, 6}};
   const int* const of = sizes[a.samples - 1];

@@ -692,7 +692,8 @@ typedef struct af3_diffusion_block {
    * af3_pairformer_block's pair_frags: what lies between two attentions is then one kernel (c = 128, hidden at most 256
    * and a multiple of 64, in all blocks of a call); diffusion: NULL, or for c = 768 and hidden a multiple of 128 w_q, w_tr1,
    * w_out and w_tr2 once more in that order, the rows exchanged, w_tr1's in blocks of 16 of the first factor and 16 of the
-   * second: at few rows the block is then five kernels (bf16 activations, a conditioning row per token, at most 5 samples) */
+   * second: read in their place by most products (bf16 activations, a conditioning row per token), and at few rows of at
+   * most 5 samples the block is then five kernels.  The others are needed all the same. */
   const uint16_t* frags;
 } af3_diffusion_block;
 size_t af3_diffusion_transformer_workspace_bytes(int64_t batch, int64_t seq, int channels, int hidden);
