@@ -89,7 +89,7 @@ struct StepTile {
 
 // Pieces of the weights (32 rows) in flight: what the registers leave beside the waves of a SIMD.
 constexpr int pieces_in_flight(int ch, int pb, int waves, bool transition) {
-  return ch == 128 && transition && (pb == 2 || waves == 3) ? 1 : 2;
+  return ch == 128 && (waves == 4 || (transition && (pb == 2 || waves == 3))) ? 1 : 2;
 }
 
 template <typename TIO, int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT, int PER_SIMD>
@@ -575,6 +575,11 @@ constexpr int64_t WIDE_PATCHES = 256 * 64;
 // workgroups enough (two a CU against three); us, 32 / 64 positions, 160 tokens 19.1 / 19.5 (epilogue), 18.8 / 18.3 (output), 208
 // 24.6 / 27.0, 23.9 / 25.3, 240 30.5 / 29.3, 29.2 / 28.8, 301 44.0 / 41.8, 42.4 / 40.7, 400 68.6 / 64.3, 66.9 / 63.6.
 constexpr int64_t WIDE_ROWS = 208 * 208 + 1;
+// ... and between three tiles of 32 to a CU and three and a half a fourth workgroup instead of a second round of a few: three / four,
+// 157 tokens (785 tiles) 19.3 / 17.7 (epilogue), 18.0 / 17.4 (output), 160 (800) 18.7 / 17.0, 17.3 / 16.7, 176 (968) 20.2 / 20.5, 17.8 /
+// 18.5.  Its 128 registers leave one piece of the weights in flight, which costs where it saves no round: 64 tokens 7.6 / 7.9, 7.8 /
+// 8.0, 130 15.8 / 15.5, 15.4 / 16.6, 200 (1300) 23.2 / 23.7, 23.0 / 23.4.
+bool four_a_simd(int64_t positions) { return positions > 32 * 3 * 256 && positions <= 32 * 7 * 128; }
 // The steps with a transition: tiles of 32 positions, two or three workgroups to a CU, or tiles of 64 (half of the weights'
 // traffic), two to a CU, by the rounds that they make on 256 CUs; us, with the next prologue, two / three / wide: 128 tokens (512
 // tiles of 32) 22.8 / 23.2 / 25.0, 152 (760) 31.2 / 29.1 / 31.2, 160 (800) 36.4 / 36.0 / 31.6, 181 (1086, wide ones 543) 45.1 / 43.1 /
@@ -634,9 +639,11 @@ int launch_pair_step(const PairStepArgs& a, int step, hipStream_t s) {
       return launch_tiles<128, 1, IN_EPILOGUE, MAP_PATCH, false, NEXT_PROLOGUE>(a, s);
     case PAIR_STEP_PROJECT_START:
       if (positions >= WIDE_ROWS) return launch_tiles<128, 2, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
+      if (four_a_simd(positions)) return launch_tiles<128, 1, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT, 4>(a, s);
       return launch_tiles<128, 1, IN_EPILOGUE, MAP_ROWS, false, NEXT_PROJECT>(a, s);
     case PAIR_STEP_PROJECT_END:
       if (positions >= WIDE_ROWS) return launch_tiles<128, 2, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
+      if (four_a_simd(positions)) return launch_tiles<128, 1, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT, 4>(a, s);
       return launch_tiles<128, 1, IN_ATTENTION, MAP_COLUMNS, false, NEXT_PROJECT>(a, s);
     case PAIR_STEP_LAST:
       if (form == TWO_A_SIMD) return launch_tiles<128, 1, IN_ATTENTION, MAP_ROWS, true, NEXT_NONE, 2>(a, s);

@@ -68,6 +68,17 @@ def test_steps_give_the_bits_of_one_kernel_per_operator(gpu_pkg, n, c, factor, h
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("io", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,c,factor,padding", [(154, 128, 4, 0), (160, 128, 4, 9), (162, 96, 4, 3), (163, 128, 4, 0)])
+def test_projections_four_workgroups_to_a_cu(gpu_pkg, n, c, factor, padding, io):
+    """The first and the last sizes of that form, a short last tile, and one size past them."""
+    blk, inputs = _block(gpu_pkg, c, factor, n), _inputs(n, c, io, padding)
+    got, want = _run(blk, *inputs), _run_general(blk, *inputs)
+    for x, y, before in zip(got, want, (inputs[0], inputs[2])):
+        assert torch.isfinite(x).all() and not torch.equal(x, before) and torch.equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("io", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,factor,padding", [(1, 2, 0), (7, 2, 2), (16, 1, 0), (17, 2, 3), (33, 2, 0), (64, 1, 5), (65, 2, 30),
                                               (127, 2, 0), (129, 1, 9), (187, 2, 11), (208, 2, 0), (301, 2, 11), (515, 2, 40)])
 def test_64_channels_as_they_are(gpu_pkg, n, factor, padding, io):
