@@ -434,6 +434,23 @@ struct AtomStepArgs {
 bool atom_steps_apply(const AtomStepArgs& a);
 int launch_atom_step(const AtomStepArgs& a, bool tail, bool head, hipStream_t s);
 
+// -------------------------------------------------------------- single_step.hip
+// LayerNorm of rows of 384 channels and a product of them, w row-major [N][384]: out[row][..] = queries (bias, scale), keys, values,
+// gate (sigmoid), N = 4 x 384, or with swiglu N / 2 hidden units (w in blocks of 32 + 32 rows).
+constexpr int SINGLE_STEP_CHANNELS = 384, SINGLE_STEP_ROWS = 400;
+struct SingleStepArgs {
+  const void* x = nullptr;  // [rows][384]
+  int io_f32 = 0, rows = 0, N = 0, swiglu = 0;
+  const float *ln_w = nullptr, *ln_b = nullptr;
+  const bf16_t* w = nullptr;
+  const float* q_bias = nullptr;  // [384] or null
+  float q_scale = 1.f;
+  bf16_t* out = nullptr;  // [rows][ldc]
+  int64_t ldc = 0;
+};
+bool single_step_applies(const SingleStepArgs& a);
+int launch_single_step(const SingleStepArgs& a, hipStream_t s);
+
 // --------------------------------------------------------------- token_step.hip
 // Adaptive LayerNorm of rows of 768 channels and a product of them: with w in fragment order, [N][768], out[row][n0 ..] =
 // queries (bias, scale), keys, values, gate (sigmoid), N = 4 x 768, or with swiglu N / 2 hidden units (w in blocks of 64 rows).

@@ -221,11 +221,30 @@ int single_update(const af3_pairformer_block& b, void* single, int dt, const flo
   auto product = [&](const uint16_t* in, const uint16_t* wt, void* out, int out_dt, int n_out, int k, int mode, const void* res) {
     return run_linear(in, wt, nullptr, out, out_dt, n, n_out, k, mode, 1.f, 0, nullptr, 0, 0, res, dt, 1, st);
   };
-  STEP(af3_layer_norm_forward(single, dt, x, n, c, b.sa_ln_w, b.sa_ln_b, nullptr, nullptr, 0, 0, s));
-  STEP(run_self_attention(x, mask, 1, logits, 1, b.sa_w_qkvg, b.sa_q_b, b.num_head, y, AF3_BF16, 1, n, c, aw, ab, 1, st));
+  // Up to SINGLE_STEP_ROWS rows either norm and the product behind it are one kernel.
+  const int d = b.num_head > 0 && c % b.num_head == 0 ? c / b.num_head : 0;
+  bf16_t* const qkvg = self_projections(aw, ab, n, c);
+  SingleStepArgs in, hidden;
+  in.x = hidden.x = single; in.io_f32 = hidden.io_f32 = dt == AF3_F32; in.rows = hidden.rows = n <= SINGLE_STEP_ROWS ? (int)n : 0;
+  in.ln_w = b.sa_ln_w; in.ln_b = b.sa_ln_b; in.w = b.sa_w_qkvg; in.N = 4 * c; in.ldc = 4 * c; in.out = qkvg;
+  in.q_bias = b.sa_q_b; in.q_scale = 1.0f / sqrtf((float)d);
+  hidden.ln_w = b.st_ln_w; hidden.ln_b = b.st_ln_b; hidden.w = b.st_w1; hidden.N = 2 * h; hidden.swiglu = 1; hidden.ldc = h; hidden.out = y;
+  const bool steps = c == SINGLE_STEP_CHANNELS && (dt == AF3_F32 || dt == AF3_BF16) && (d == 16 || d == 24 || d == 32 || d == 48) &&
+                     single_step_applies(in) && single_step_applies(hidden);
+  if (steps) {
+    STEP(launch_single_step(in, st));
+    STEP(run_self_attend(qkvg, mask, 1, logits, 1, b.num_head, y, AF3_BF16, 1, n, c, st));
+  } else {
+    STEP(af3_layer_norm_forward(single, dt, x, n, c, b.sa_ln_w, b.sa_ln_b, nullptr, nullptr, 0, 0, s));
+    STEP(run_self_attention(x, mask, 1, logits, 1, b.sa_w_qkvg, b.sa_q_b, b.num_head, y, AF3_BF16, 1, n, c, aw, ab, 1, st));
+  }
   STEP(product(y, b.sa_w_out, single, dt, c, c, AF3_LINEAR_GATE_RES, single));
-  STEP(af3_layer_norm_forward(single, dt, x, n, c, b.st_ln_w, b.st_ln_b, nullptr, nullptr, 0, 0, s));
-  STEP(product(x, b.st_w1, y, AF3_BF16, 2 * h, c, AF3_LINEAR_SWIGLU, nullptr));
+  if (steps) {
+    STEP(launch_single_step(hidden, st));
+  } else {
+    STEP(af3_layer_norm_forward(single, dt, x, n, c, b.st_ln_w, b.st_ln_b, nullptr, nullptr, 0, 0, s));
+    STEP(product(x, b.st_w1, y, AF3_BF16, 2 * h, c, AF3_LINEAR_SWIGLU, nullptr));
+  }
   return product(y, b.st_w2, single, dt, c, h, AF3_LINEAR_GATE_RES, single);
 }
 
