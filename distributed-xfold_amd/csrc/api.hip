@@ -785,7 +785,7 @@ int run_gathered_attention(const bf16_t* q_data, const bf16_t* atom_data, const 
                            int bias_quad_major, const float* mask_q, const float* mask_k, int64_t bias_batches, const bf16_t* w_qg,
                            const bf16_t* w_kv, const float* query_b, int num_head, void* out, int out_dtype, int64_t batch,
                            int64_t sq, int64_t sk, int64_t samples, int64_t n_atoms, int channels, void* workspace,
-                           size_t workspace_bytes, hipStream_t stream) {
+                           size_t workspace_bytes, hipStream_t stream, const int* windows) {
   if (!q_data != !atom_data || !key_rows || !w_qg || !w_kv || !out) return AF3_ERR_BAD_ARG;
   if (bad_dtype(out_dtype) || batch <= 0 || sq <= 0 || sk <= 0 || samples <= 0 || n_atoms <= 0 || channels <= 0 ||
       (channels & 7) || num_head <= 0 || channels % num_head)
@@ -824,7 +824,7 @@ int run_gathered_attention(const bf16_t* q_data, const bf16_t* atom_data, const 
   f.q_ss = f.g_ss = f.k_ss = f.v_ss = 2 * channels;
   f.q_sb = f.g_sb = sq * 2 * channels;
   f.k_sb = f.v_sb = n_atoms * 2 * channels;   // one K / V table per sample
-  f.key_rows = key_rows; f.table_rows = n_atoms;
+  f.key_rows = key_rows; f.table_rows = n_atoms; f.windows = windows;
   f.out = out; f.out_f32 = out_dtype == AF3_F32; f.o_ss = channels; f.o_sb = sq * channels;
   f.B = (int)batch; f.H = num_head; f.Sq = (int)sq; f.Sk = (int)sk; f.d = d;
   f.bias = pair_logits; f.bias_sb = (int64_t)num_head * sq * sk; f.bias_sh = sq * sk;

@@ -47,10 +47,13 @@ __global__ __launch_bounds__(256, 2) void atom_step_kernel(AtomStepArgs a) {
   const int chunk = tid & 15, prow = tid >> 4;
 
   // The samples' rows of the same atoms, which share their conditioning, run back to back on one XCD.
-  const int tiles = (a.atoms + TS - 1) / TS, total = tiles * a.samples, per = (total + 7) >> 3;
+  const int all = (a.atoms + TS - 1) / TS, tiles = a.tiles ? min(a.tiles[0], all) : all, total = tiles * a.samples, per = (total + 7) >> 3;
   const int idx = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per || idx >= total) return;
-  const int a0 = __builtin_amdgcn_readfirstlane(idx / a.samples) * TS, sample = __builtin_amdgcn_readfirstlane(idx % a.samples);
+  const int place = __builtin_amdgcn_readfirstlane(idx / a.samples), sample = __builtin_amdgcn_readfirstlane(idx % a.samples);
+  const int tile = a.tiles ? a.tiles[1 + place] : place;
+  if ((unsigned)tile >= (unsigned)all) return;
+  const int a0 = tile * TS;
   TIO* const act = reinterpret_cast<TIO*>(a.act) + (int64_t)sample * a.atoms * C;
   const bf16_t* const y = a.y + (int64_t)sample * a.atoms * C;
   int atom[2];

@@ -716,10 +716,12 @@ __global__ __launch_bounds__(256, TILES == 2 ? 2 : 4) void window_kernel(FlashAr
   const int h = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hh = lane >> 5, j = lane & 31;
   const int xaddr = half_swap_addr();
-  const int per_xcd = (int)(gridDim.x >> 3), logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (logical >= a.B) return;
-  const int samples = a.B / a.bias_mod;
-  const int bb = logical / samples, sample = logical % samples, b = sample * a.bias_mod + bb;
+  const int samples = a.B / a.bias_mod, work = a.windows ? min(a.windows[0], a.bias_mod) * samples : a.B;
+  const int per_xcd = (work + 7) >> 3, logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || logical >= work) return;
+  const int place = logical / samples, sample = logical - place * samples, bb = a.windows ? a.windows[1 + place] : place;
+  if ((unsigned)bb >= (unsigned)a.bias_mod) return;
+  const int b = sample * a.bias_mod + bb;
   const int qi = min(j, a.Sq - 1);
   const bool q_ok = j < a.Sq;
 

@@ -229,6 +229,52 @@ struct StepPositions {
   }
 };
 
+// The windows of an atom layout that somebody reads, in their order.  A layout has room for every token's 24 atoms and as many empty
+// slots behind the last atom as there are fewer, half of the windows and more.  Asked for are a window with an atom in it (mask) and
+// one that the way back reads; and all of them should any key be a row that neither of these names, whose value would then count.
+// One workgroup, the rows as bits in LDS: 18432 rows and 73728 keys 11 us, once a batch.
+constexpr int WINDOW_THREADS = 1024, WINDOW_ROWS = 1 << 19;
+__global__ __launch_bounds__(WINDOW_THREADS) void atom_windows_kernel(AtomWindowsArgs a) {
+  __shared__ uint32_t want[WINDOW_ROWS / 32];
+  __shared__ int stray, live_of[WINDOW_THREADS / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rows = a.windows * a.queries;
+  if (tid == 0) stray = 0;
+  for (int r0 = 0; r0 < rows; r0 += WINDOW_THREADS) {
+    const int r = r0 + tid;
+    const uint64_t b = __ballot(r < rows && a.mask[min(r, rows - 1)] != 0.f);
+    if ((lane & 31) == 0 && r < rows) want[r >> 5] = (uint32_t)(lane ? b >> 32 : b);
+  }
+  __syncthreads();
+  for (int64_t i = tid; i < a.slots; i += WINDOW_THREADS) {
+    const int64_t r = a.back_idx[i];
+    if (a.back_exists[i] && r >= 0 && r < rows) atomicOr(&want[r >> 5], 1u << (r & 31));
+  }
+  __syncthreads();
+  for (int64_t i = tid; i < (int64_t)a.windows * a.keys; i += WINDOW_THREADS) {
+    const int r = a.key_rows[i];
+    if (r >= 0 && r < rows && !(want[r >> 5] >> (r & 31) & 1)) stray = 1;
+  }
+  __syncthreads();
+  int before = 0;
+  for (int w0 = 0; w0 < a.windows; w0 += WINDOW_THREADS) {
+    const int w = w0 + tid;
+    bool live = w < a.windows && stray;
+    if (w < a.windows)
+      for (int r = w * a.queries; r < (w + 1) * a.queries && !live; ++r) live = want[r >> 5] >> (r & 31) & 1;
+    const uint64_t b = __ballot(live);
+    if (lane == 0) live_of[wave] = __popcll(b);
+    __syncthreads();
+    int at = before;
+    for (int v = 0; v < WINDOW_THREADS / 64; ++v) {
+      if (v < wave) at += live_of[v];
+      before += live_of[v];
+    }
+    if (live) a.out[1 + at + __popcll(b & ((1ull << lane) - 1))] = w;
+    __syncthreads();
+  }
+  if (tid == 0) a.out[0] = before;
+}
+
 bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
@@ -279,6 +325,17 @@ int launch_gather_atoms(const GatherAtomsArgs& a, hipStream_t s) {
   GatherAtomsArgs args = a;
   if (!a.add) args.add_rows = 1;
   return launch_each(a.rows * (a.channels / 8), s, GatherAtoms{args});
+}
+
+bool atom_windows_apply(const AtomWindowsArgs& a) {
+  return a.mask && a.back_idx && a.back_exists && a.slots > 0 && a.key_rows && a.out && a.windows > 0 && a.queries > 0 && a.keys > 0 &&
+         (int64_t)a.windows * a.queries <= WINDOW_ROWS;
+}
+
+int launch_atom_windows(const AtomWindowsArgs& a, hipStream_t s) {
+  if (!atom_windows_apply(a)) return AF3_ERR_BAD_ARG;
+  hipLaunchKernelGGL(atom_windows_kernel, dim3(1), dim3(WINDOW_THREADS), 0, s, a);
+  return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
 }
 
 int launch_positions(int op, const float* x, const float* y, const float* mask, const float* level, const float* other, float f,

@@ -98,7 +98,7 @@ int run_gathered_attention(const bf16_t* q_data, const bf16_t* atom_data, const 
                            int bias_quad_major, const float* mask_q, const float* mask_k, int64_t bias_batches, const bf16_t* w_qg,
                            const bf16_t* w_kv, const float* query_b, int num_head, void* out, int out_dtype, int64_t batch,
                            int64_t sq, int64_t sk, int64_t samples, int64_t n_atoms, int channels, void* workspace,
-                           size_t workspace_bytes, hipStream_t stream);
+                           size_t workspace_bytes, hipStream_t stream, const int* windows = nullptr);
 // where in its workspace the projections are (false: too small); with q_data and atom_data null they are there already
 bool gathered_projections(void* workspace, size_t workspace_bytes, int64_t query_rows, int64_t atom_rows, int channels, bf16_t** qg,
                           bf16_t** kv);
@@ -314,6 +314,8 @@ struct FlashArgs {
   // negative row is a key with zero K and V.  Null: key s is row s of batch b.
   const int* key_rows = nullptr;
   int64_t table_rows = 0;  // rows of a sample's table: every entry of key_rows is below this
+  // window_kernel: the entries b % bias_mod that are asked for, their number first; the others' results are not written.  Null: all.
+  const int* windows = nullptr;
   int per_xcd = 0, q_tiles = 0;  // (these and the magic numbers of their divisions by the launcher)
   unsigned magic_b = 0, magic_t = 0;
   int n_blocks = 0;  // workgroups that have work (set by the launcher; the grid is rounded up to a multiple of 8)
@@ -430,6 +432,7 @@ struct AtomStepArgs {
   const float* q_bias = nullptr;                         // [128] or null
   float q_scale = 1.f;
   bf16_t *qg = nullptr, *kv = nullptr;                   // [samples][atoms][256]: q, gate;  k, v
+  const int* tiles = nullptr;                            // the runs of 32 atoms that are asked for, their number first; null: all
 };
 bool atom_steps_apply(const AtomStepArgs& a);
 int launch_atom_step(const AtomStepArgs& a, bool tail, bool head, hipStream_t s);
@@ -531,6 +534,18 @@ struct AtomEmbedArgs {
   int channels = 0;
 };
 int launch_atom_embed(const AtomEmbedArgs& a, hipStream_t s);
+// windows of an atom layout that somebody reads (af3_atom_windows_forward)
+struct AtomWindowsArgs {
+  const float* mask = nullptr;             // [windows][queries]
+  const int64_t* back_idx = nullptr;       // [slots] into the windows' rows
+  const uint8_t* back_exists = nullptr;    // [slots]
+  int64_t slots = 0;
+  const int32_t* key_rows = nullptr;       // [windows][keys], negative: none
+  int windows = 0, queries = 0, keys = 0;
+  int32_t* out = nullptr;                  // [1 + windows]
+};
+bool atom_windows_apply(const AtomWindowsArgs& a);
+int launch_atom_windows(const AtomWindowsArgs& a, hipStream_t s);
 struct GatherAtomsArgs {
   const int64_t *idx = nullptr, *add_idx = nullptr, *uid = nullptr;  // [rows], [rows], [uids]
   const uint8_t *exists = nullptr, *add_exists = nullptr;            // [rows]

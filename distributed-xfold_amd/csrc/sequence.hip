@@ -645,11 +645,11 @@ size_t af3_atom_transformer_workspace_bytes(int64_t samples, int64_t subsets, in
          align_up(af3_gathered_cross_attention_workspace_bytes(samples * subsets, queries, samples, subsets * queries, channels));
 }
 
-int af3_atom_transformer_forward(
+static int atom_transformer(
     const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t samples, int64_t subsets,
     int64_t queries, int64_t keys, int channels, int hidden, int num_head, const int32_t* key_rows, const float* mask_q,
     const float* mask_k, const float* pair_logits, int bias_quad_major, const float* scale_shift_q, const float* scale_shift_k,
-    const float* gate, void* workspace, size_t workspace_bytes, af3_stream_t stream) {
+    const float* gate, const int32_t* windows, void* workspace, size_t workspace_bytes, af3_stream_t stream) {
   if (!blocks || num_blocks <= 0 || !act || !key_rows || !scale_shift_q || !scale_shift_k || !gate || samples <= 0 ||
       subsets <= 0 || queries <= 0 || keys <= 0 || channels <= 0 || hidden <= 0 || num_head <= 0)
     return AF3_ERR_BAD_ARG;
@@ -670,7 +670,7 @@ int af3_atom_transformer_forward(
     AtomStepArgs a;
     a.act = act; a.io_f32 = act_dtype == AF3_F32; a.atoms = (int)atoms; a.samples = (int)samples; a.hidden = hidden;
     a.y = y; a.gate1 = g; a.gate2 = g + atoms * c; a.scale = ss + 2 * c; a.ld_cond = ld_q;
-    a.f_out = b.frags;
+    a.f_out = b.frags; a.tiles = windows;
     if (b.frags) { a.f_w1 = b.frags + c * c; a.f_w2 = a.f_w1 + 2 * hidden * c; }
     return a;
   };
@@ -688,6 +688,10 @@ int af3_atom_transformer_forward(
     attention_args(a, i);
     steps = atom_steps_apply(a);
   }
+  // (a window's queries are a tile of the steps, and its attention is window_kernel's: what makes neither takes all of them)
+  if (!steps || queries != 32 || num_head != 4 || keys > 128 || (keys & 3) || !pair_logits || ((uintptr_t)pair_logits & 15) ||
+      atoms >= 1 << 22)
+    windows = nullptr;
   for (int i = 0; i < num_blocks; ++i) {
     const af3_diffusion_block& b = blocks[i];
     const float* pl = pair_logits ? pair_logits + (int64_t)i * subsets * num_head * queries * keys : nullptr;
@@ -699,7 +703,7 @@ int af3_atom_transformer_forward(
       }
       STEP(run_gathered_attention(nullptr, nullptr, key_rows, pl, bias_quad_major, mask_q, mask_k, subsets, b.w_q, b.w_kv, b.q_b, num_head, y,
                                   AF3_BF16, samples * subsets, queries, keys, samples, atoms, c, aw, ab,
-                                  static_cast<hipStream_t>(stream)));
+                                  static_cast<hipStream_t>(stream), windows));
       const bool more = i + 1 < num_blocks;
       attention_args(a, more ? i + 1 : i);
       STEP(launch_atom_step(a, true, more, static_cast<hipStream_t>(stream)));
@@ -730,6 +734,25 @@ int af3_atom_transformer_forward(
   }
   return AF3_OK;
 }
+int af3_atom_transformer_forward(
+    const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t samples, int64_t subsets,
+    int64_t queries, int64_t keys, int channels, int hidden, int num_head, const int32_t* key_rows, const float* mask_q,
+    const float* mask_k, const float* pair_logits, int bias_quad_major, const float* scale_shift_q, const float* scale_shift_k,
+    const float* gate, void* workspace, size_t workspace_bytes, af3_stream_t stream) {
+  return atom_transformer(blocks, num_blocks, act, act_dtype, samples, subsets, queries, keys, channels, hidden, num_head, key_rows, mask_q,
+                          mask_k, pair_logits, bias_quad_major, scale_shift_q, scale_shift_k, gate, nullptr, workspace, workspace_bytes,
+                          stream);
+}
+int af3_atom_transformer_windows_forward(
+    const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t samples, int64_t subsets,
+    int64_t queries, int64_t keys, int channels, int hidden, int num_head, const int32_t* key_rows, const float* mask_q,
+    const float* mask_k, const float* pair_logits, int bias_quad_major, const float* scale_shift_q, const float* scale_shift_k,
+    const float* gate, const int32_t* windows, void* workspace, size_t workspace_bytes, af3_stream_t stream) {
+  if (!windows) return AF3_ERR_BAD_ARG;
+  return atom_transformer(blocks, num_blocks, act, act_dtype, samples, subsets, queries, keys, channels, hidden, num_head, key_rows, mask_q,
+                          mask_k, pair_logits, bias_quad_major, scale_shift_q, scale_shift_k, gate, windows, workspace, workspace_bytes,
+                          stream);
+}
 
 // ------------------------------------------------------------- element-wise passes
 int af3_contact_matrix_forward(const int64_t* idx0, const uint8_t* exists0, int count0, const int64_t* idx1, const uint8_t* exists1,
@@ -755,6 +778,14 @@ int af3_add_rows_forward(const float* a, const float* b, int64_t ld_b, int64_t m
   return launch_add_rows(a, b, ld_b, mod, out, out_dtype == AF3_F32, rows, channels, static_cast<hipStream_t>(stream));
 }
 
+int af3_atom_windows_forward(const float* mask, const int64_t* back_idx, const uint8_t* back_exists, int64_t slots, const int32_t* key_rows,
+                             int64_t subsets, int64_t queries, int64_t keys, int32_t* windows, af3_stream_t stream) {
+  if (subsets <= 0 || subsets > 0x7fffffff || queries <= 0 || queries > 0x7fffffff || keys <= 0 || keys > 0x7fffffff) return AF3_ERR_BAD_ARG;
+  AtomWindowsArgs a;
+  a.mask = mask; a.back_idx = back_idx; a.back_exists = back_exists; a.slots = slots; a.key_rows = key_rows;
+  a.windows = (int)subsets; a.queries = (int)queries; a.keys = (int)keys; a.out = windows;
+  return launch_atom_windows(a, static_cast<hipStream_t>(stream));
+}
 int af3_mask_rows_forward(uint16_t* x, const float* mask, int64_t mod, int64_t rows, int channels, af3_stream_t stream) {
   return launch_mask_rows(x, mask, mod, rows, channels, static_cast<hipStream_t>(stream));
 }

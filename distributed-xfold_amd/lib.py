@@ -117,6 +117,9 @@ SIGNATURES = {
     "af3_atom_transformer_workspace_bytes": (_sz, [_i64, _i64, _i64, _i, _i]),
     "af3_atom_transformer_forward": (
         _i, [_vp, _i, _vp, _i, _i64, _i64, _i64, _i64, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "af3_atom_transformer_windows_forward": (
+        _i, [_vp, _i, _vp, _i, _i64, _i64, _i64, _i64, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "af3_atom_windows_forward": (_i, [_vp, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp]),
     "af3_linear_bias_span": (_i, [_i64, _i, _i, _i, _i, _vp, _vp]),
     "af3_grid_attention_core_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "af3_check_gemm_f32": (

@@ -23,7 +23,7 @@ import torch.nn as nn
 
 from .. import check, ops
 from .atom_layout import GatherInfo, convert
-from .base import HipModule, bf16, drop_mesh, f32, in_check_mode
+from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode
 from .diffusion_transformer import DiffusionCrossAttTransformer
 
 
@@ -49,6 +49,11 @@ def _ln_lin(x: torch.Tensor, norm: nn.LayerNorm, layer: nn.Linear, ln_w, w_bf16)
     return ops.linear(ops.layer_norm(x.contiguous(), ln_w), w_bf16, out_dtype=torch.float32)
 
 
+def _windows_of(transformer, windows) -> dict:
+    """The argument for a transformer that knows it, and whose result nobody else sees."""
+    return {"windows": windows} if windows is not None and as_written((transformer, DiffusionCrossAttTransformer)) else {}
+
+
 @dataclass
 class AtomCrossAttEncoderOutput:
     token_act: torch.Tensor             # [(samples), N, per_token_channels]
@@ -59,6 +64,7 @@ class AtomCrossAttEncoderOutput:
     keys_single_cond: torch.Tensor      # [S, 128, 128]
     pair_cond: torch.Tensor             # [S, 32, 128, 16]
     transformer_cond: Any = None        # conditioning of the atom transformers (shared by encoder and decoder)
+    windows: Optional[torch.Tensor] = None    # the subsets with atoms in them (ops.atom_windows)
 
 
 @dataclass
@@ -70,6 +76,7 @@ class EncoderConditioning:
     pair_cond: torch.Tensor
     transformer_cond: Any
     atom_count: Optional[torch.Tensor] = None      # [N], atoms per token, at least 1e-10
+    windows: Optional[torch.Tensor] = None         # the subsets with atoms in them (ops.atom_windows)
 
 
 class AtomCrossAttEncoder(HipModule):
@@ -229,11 +236,14 @@ class AtomCrossAttEncoder(HipModule):
                                           w(self.embed_pair_distances_1), w(self.embed_pair_offsets_valid),
                                           w(self.pair_mlp_1), w(self.pair_mlp_2), w(self.pair_mlp_3))
         q_cond, k_cond = q_cond.contiguous(), k_cond.contiguous()
-        tcond = None
+        tcond = windows = None
         if not in_check_mode():
             tcond = self.atom_transformer_encoder.conditioning(q_cond, k_cond, pair_act,
                                                                keys_are_query_atoms=aca.queries_to_keys)
-        return EncoderConditioning(q_mask, q_cond, k_mask, k_cond, pair_act, tcond, self._atom_count(batch))
+            back = aca.queries_to_token_atoms
+            if as_written((self.atom_transformer_encoder, DiffusionCrossAttTransformer)) and q_mask.is_cuda and q_mask.dim() == 2:
+                windows = ops.atom_windows(q_mask.float().contiguous(), back.gather_idxs, back.gather_mask, tcond[4])
+        return EncoderConditioning(q_mask, q_cond, k_mask, k_cond, pair_act, tcond, self._atom_count(batch), windows)
 
     @staticmethod
     def _atom_count(batch):
@@ -280,7 +290,8 @@ class AtomCrossAttEncoder(HipModule):
         q_act = self.atom_transformer_encoder(
             queries_act=q_act, queries_mask=c.queries_mask, queries_to_keys=aca.queries_to_keys,
             keys_mask=c.keys_mask, queries_single_cond=c.queries_single_cond,
-            keys_single_cond=c.keys_single_cond, pair_cond=c.pair_cond, cond=c.transformer_cond)
+            keys_single_cond=c.keys_single_cond, pair_cond=c.pair_cond, cond=c.transformer_cond,
+            **_windows_of(self.atom_transformer_encoder, c.windows))
         if q_act.dtype == torch.bfloat16:
             q_act = ops.mask_rows(q_act, c.queries_mask.float().contiguous())
         else:
@@ -310,7 +321,7 @@ class AtomCrossAttEncoder(HipModule):
             if not batched:
                 tok_act = tok_act[0]
         return AtomCrossAttEncoderOutput(tok_act, skip, c.queries_mask, c.queries_single_cond, c.keys_mask,
-                                         c.keys_single_cond, c.pair_cond, c.transformer_cond)
+                                         c.keys_single_cond, c.pair_cond, c.transformer_cond, c.windows)
 
 
 class AtomCrossAttDecoder(HipModule):
@@ -383,7 +394,8 @@ class AtomCrossAttDecoder(HipModule):
         q_act = self.atom_transformer_decoder(
             queries_act=q_act, queries_mask=enc.queries_mask, queries_to_keys=aca.queries_to_keys,
             keys_mask=enc.keys_mask, queries_single_cond=enc.queries_single_cond,
-            keys_single_cond=enc.keys_single_cond, pair_cond=enc.pair_cond, cond=transformer_cond)
+            keys_single_cond=enc.keys_single_cond, pair_cond=enc.pair_cond, cond=transformer_cond,
+            **_windows_of(self.atom_transformer_decoder, enc.windows))
         if fused:
             # LayerNorm, projection to the position update and conversion to the token-atom layout in one
             # pass over the atoms that exist (their query mask is one)

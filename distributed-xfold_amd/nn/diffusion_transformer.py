@@ -568,7 +568,9 @@ class DiffusionCrossAttTransformer(HipModule):
         return logits, ss_q, ss_k, gate, key_rows
 
     def forward(self, queries_act, queries_mask, queries_to_keys, keys_mask, queries_single_cond,
-                keys_single_cond, pair_cond, cond=None):
+                keys_single_cond, pair_cond, cond=None, windows=None):
+        """`windows` (ops.atom_windows): the subsets whose rows the caller reads; those of the others may come back
+        as they were, or updated."""
         if in_check_mode():
             return check.cross_att_transformer(self, queries_act, queries_mask, queries_to_keys, keys_mask,
                                                queries_single_cond, keys_single_cond, pair_cond)
@@ -581,7 +583,8 @@ class DiffusionCrossAttTransformer(HipModule):
         if key_rows is not None and self._one_call(blocks):
             table = block_table(self, blocks, self.c_query)
             return ops.atom_transformer(table, queries_act, key_rows, queries_mask, keys_mask,
-                                        logits.to(torch.float32).contiguous(), ss_q, ss_k, gate, self.num_head, table.hidden)
+                                        logits.to(torch.float32).contiguous(), ss_q, ss_k, gate, self.num_head, table.hidden,
+                                        windows=windows)
         for i, (att, tr) in enumerate(blocks):
             cond = ss_q[:, 2 * i], ss_k[:, i], gate[2 * i]
             if key_rows is not None:

@@ -514,10 +514,11 @@ def diffusion_transformer(blocks, act, mask, pair_logits, scale_shift, gate, num
 
 @_uses_scratch
 def atom_transformer(blocks, act, key_rows, mask_q, mask_k, pair_logits, scale_shift_q, scale_shift_k, gate, num_head,
-                     hidden):
+                     hidden, windows=None):
     """The blocks of the windowed atom transformer in one call (af3_atom_transformer_forward), act
     [(B,) S, Q, C] updated in place.  key_rows [S, K] int32; pair_logits [blocks, S, H, Q, K] or [blocks, S, H, K / 4, Q, 4]; scale_shift_q
-    [S Q, 2 blocks, 2 C], scale_shift_k [S Q, blocks, 2 C], gate [2 blocks, S Q, C] fp32."""
+    [S Q, 2 blocks, 2 C], scale_shift_k [S Q, blocks, 2 C], gate [2 blocks, S Q, C] fp32.  `windows` (atom_windows): the
+    subsets that the caller reads; act of the others is then not to be read."""
     lib = _L.load()
     _gpu(act, "act")
     _weights_with(act, blocks)
@@ -533,11 +534,32 @@ def atom_transformer(blocks, act, key_rows, mask_q, mask_k, pair_logits, scale_s
     _gpu(gate, "gate", torch.float32, (2 * nb, s * q, c))
     mq, mk = _mask_f32(mask_q.reshape(s, q), (s, q), "mask_q"), _mask_f32(mask_k.reshape(s, k), (s, k), "mask_k")
     ws = _ws(lib.af3_atom_transformer_workspace_bytes(b, s, q, c, hidden), act.device)
-    rc = lib.af3_atom_transformer_forward(
+    call, some = lib.af3_atom_transformer_forward, ()
+    if windows is not None:
+        call, some = lib.af3_atom_transformer_windows_forward, (_p(_gpu(windows, "windows", torch.int32, (s + 1,))),)
+    rc = call(
         blocks, nb, _p(act), _dt(act), b, s, q, k, c, hidden, num_head, _p(key_rows), _p(mq), _p(mk), _p(pair_logits), int(quads),
-        _p(scale_shift_q), _p(scale_shift_k), _p(gate), _p(ws), ws.numel(), _stream(act.device))
+        _p(scale_shift_q), _p(scale_shift_k), _p(gate), *some, _p(ws), ws.numel(), _stream(act.device))
     _L.check(rc, "af3_atom_transformer_forward")
     return act
+
+
+def atom_windows(mask, back_idx, back_exists, key_rows):
+    """The subsets of an atom layout that somebody reads, their number first (af3_atom_windows_forward): int32 [S + 1], or None
+    for what the kernel does not take.  mask [S, Q] fp32; back_idx, back_exists: the gather from the subsets back to the
+    tokens' slots; key_rows [S, K] int32."""
+    lib = _L.load()
+    s, q = mask.shape
+    for t, dtype in ((mask, torch.float32), (back_idx, torch.int64), (back_exists, torch.bool), (key_rows, torch.int32)):
+        if not t.is_cuda or t.dtype != dtype or not t.is_contiguous() or not t.numel():
+            return None
+    if back_idx.shape != back_exists.shape or key_rows.dim() != 2 or key_rows.shape[0] != s or s * q > 1 << 19:
+        return None
+    out = torch.empty(s + 1, dtype=torch.int32, device=mask.device)
+    rc = lib.af3_atom_windows_forward(_p(mask), _p(back_idx), _p(back_exists), back_idx.numel(), _p(key_rows), s, q,
+                                      key_rows.shape[1], _p(out), _stream(mask.device))
+    _L.check(rc, "af3_atom_windows_forward")
+    return out
 
 
 @_uses_scratch

@@ -680,6 +680,12 @@ int af3_evoformer_stack_forward(
  *   = 0), see af3_gathered_cross_attention_forward; scale_shift_k [subsets * queries]
  *   [num_blocks][2 c] per atom, pair_logits [num_blocks,subsets,num_head,queries,keys] or,
  *   with bias_quad_major, [num_blocks,subsets,num_head,keys/4,queries,4], gate here [2 num_blocks][subsets * queries][c].
+ * af3_atom_transformer_windows_forward: the same for a caller that reads only some of the subsets: windows (device)
+ *   holds their number and then their indices, each below `subsets`.  act of the others is left as it is or updated.
+ *   No key of a listed subset (a row of key_rows that is not negative) may lie in one that is not.
+ * af3_atom_windows_forward: such a list, windows [1 + subsets], in ascending order: the subsets with a query whose
+ *   mask [subsets,queries] is not 0, and those that the way back reads (back_idx [slots] where back_exists is not 0);
+ *   all of them if some key is a row that neither names.  subsets * queries at most 2^19.
  */
 typedef struct af3_diffusion_block {
   const uint16_t* w_q;  /* diffusion: [4 c][c] q, k, v, gate;  atom: [2 c][c] q, gate */
@@ -708,6 +714,14 @@ int af3_atom_transformer_forward(
     int64_t queries, int64_t keys, int channels, int hidden, int num_head, const int32_t* key_rows, const float* mask_q,
     const float* mask_k, const float* pair_logits, int bias_quad_major, const float* scale_shift_q, const float* scale_shift_k,
     const float* gate, void* workspace, size_t workspace_bytes, af3_stream_t stream);
+int af3_atom_transformer_windows_forward(
+    const af3_diffusion_block* blocks, int num_blocks, void* act, int act_dtype, int64_t samples, int64_t subsets,
+    int64_t queries, int64_t keys, int channels, int hidden, int num_head, const int32_t* key_rows, const float* mask_q,
+    const float* mask_k, const float* pair_logits, int bias_quad_major, const float* scale_shift_q, const float* scale_shift_k,
+    const float* gate, const int32_t* windows, void* workspace, size_t workspace_bytes, af3_stream_t stream);
+int af3_atom_windows_forward(const float* mask, const int64_t* back_idx, const uint8_t* back_exists, int64_t slots,
+                             const int32_t* key_rows, int64_t subsets, int64_t queries, int64_t keys, int32_t* windows,
+                             af3_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * Diagnostic, no counterpart in the reference.  The dense kernels fetch a
