@@ -499,7 +499,6 @@ struct RowsProductArgs {
   int64_t ld_gate = 0;
 };
 bool rows_product_applies(const RowsProductArgs& a);
-bool rows_product_better(const RowsProductArgs& a);  // ... and faster than af3_linear_forward's kernels
 int launch_rows_product(const RowsProductArgs& a, hipStream_t s);
 bool gated_product_applies(const GatedProductArgs& a);
 int launch_gated_product(const GatedProductArgs& a, hipStream_t s);

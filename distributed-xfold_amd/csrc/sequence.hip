@@ -577,13 +577,13 @@ int af3_diffusion_transformer_forward(
   // (the fragments that product_back reads, or the weights as they were given)
   auto weights_back = [&](int i, bool transition) -> const void* {
     const RowsProductArgs a = back(i, transition);
-    return gated_product_applies(few_rows(a)) || rows_product_better(a) ? (const void*)a.w : transition ? blocks[i].w_tr2 : blocks[i].w_out;
+    return gated_product_applies(few_rows(a)) || rows_product_applies(a) ? (const void*)a.w : transition ? blocks[i].w_tr2 : blocks[i].w_out;
   };
   auto product_back = [&](int i, bool transition) -> int {
     const RowsProductArgs a = back(i, transition);
     const GatedProductArgs few = few_rows(a);
     if (gated_product_applies(few)) return launch_gated_product(few, static_cast<hipStream_t>(stream));
-    if (rows_product_better(a)) return launch_rows_product(a, static_cast<hipStream_t>(stream));
+    if (rows_product_applies(a)) return launch_rows_product(a, static_cast<hipStream_t>(stream));
     const af3_diffusion_block& b = blocks[i];
     return af3_linear_forward(y, transition ? b.w_tr2 : b.w_out, nullptr, act, act_dtype, rows, c, transition ? hidden : c,
                               AF3_LINEAR_GATE_RES, 1.f, 0, gate + ((int64_t)2 * i + transition) * c, cond_rows, ld_g, act, act_dtype, stream);
@@ -615,7 +615,7 @@ int af3_diffusion_transformer_forward(
       continue;
     }
     const RowsProductArgs in = product(i, false), hidden_in = product(i, true);
-    const bool in_rows = qkvg && rows_product_better(in), hidden_rows = rows_product_better(hidden_in);
+    const bool in_rows = qkvg && rows_product_applies(in), hidden_rows = rows_product_applies(hidden_in);
     STEP(norm(ss, {in_rows ? (const void*)in.w : b.w_q, (size_t)4 * c * c * 2}, {weights_back(i, false), (size_t)c * c * 2},
               {pair_logits[i], logit_bytes}));
     if (in_rows) {

@@ -344,27 +344,29 @@ __global__ __launch_bounds__(64 * WAVES, 1) void gated_product_kernel(GatedProdu
 }
 
 // The same products over more rows: x w^T with the weights' fragments straight from memory to registers and the rows through LDS.
-// A workgroup takes 64 rows x 128 columns, a wave all rows of 32 columns; slabs of 64 channels of the rows go straight into a ring
-// of LDS buffers that the four waves share, with one barrier a slab; a wave's fragments are RP_RING slabs ahead.  Bound by the CU's
-// vector memory path: 3 KB of weights and rows for 16 matrix instructions of a wave.  Three workgroups a CU with four slabs ahead,
-// two with six to eight (us, queries to gate at 640, 1920 and 3840 rows): 6.6 13.2 24.0, 6.8 13.4 24.3.
+// A workgroup takes 32 RB rows (two to four blocks: rows_product_blocks) x 128 columns, a wave all rows of 32 columns; slabs of 64
+// channels of the rows go straight into a ring of LDS buffers that the four waves share, with one barrier a slab; a wave's
+// fragments are RP_RING slabs ahead; the result goes out through LDS, in whole lines.  Cycles of a workgroup of 96 x 128, all of 3840
+// rows: first slab there 3700, loop 8400 (4600 of it the matrix unit's), result 2700.  What bounds it is the CU's vector memory path,
+// 16 KB of weights and 4 RB KB of rows a slab, and in large tiles that the chip's results leave all at once.  Results stored from the
+// accumulators, 32 bytes of a row at a time, were slower where there is a gate and a stream to read the same way: 768 columns at
+// 3840 rows 11.7 / 15.7 us (K = 768 / 1536) against 8.6 / 14.1, at 1920 (two blocks) 6.6 / 9.8 against 6.0 / 8.9.  Two column blocks a
+// wave (192 x 256 at 3840 rows, queries to gate 23.1 us): the chip's only round ends in 8500 cycles of results.
 enum { ROWS_QKVG, ROWS_SWIGLU, ROWS_GATED };
-constexpr int RP_BM = 64, RP_BN = 128, RP_BUFFERS = 4, RP_RING = 4, RP_PER_CU = 3;
-static_assert(RP_RING >= RP_BUFFERS);  // (rows_product_younger counts on it)
-// loads of a wave issued behind its two for slab s of the rows, when it waits for these (step s - 1 of the loop): statements and loads
-// that sched_barrier keeps in this order; any others issued between them only make the wait longer
-constexpr int rows_product_younger(int s, int slabs) {
+constexpr int RP_BN = 128, RP_BUFFERS = 4, RP_RING = 4;
+static_assert(RP_RING == RP_BUFFERS);  // (rows_product_younger counts on it)
+// loads of a wave issued behind its own for slab s of the rows, when it waits for these (in step s - 1 of the loop): statements and
+// loads that sched_barrier keeps in this order; any others issued between them only make the wait longer
+constexpr int rows_product_younger(int s, int slabs, int rows) {
   int n = 0;
-  auto steps = [&](int from) {
-    for (int i = from; i < s - 1; ++i) n += (i + RP_BUFFERS < slabs ? 2 : 0) + (i + RP_RING < slabs ? 4 : 0);
+  bool behind = false;
+  auto issue = [&](int slab) {  // rows, then fragments: in front of the loop, and in each of its steps before the wait
+    if (behind && slab < slabs) n += rows;
+    if (slab == s) behind = true;
+    if (behind && slab < slabs) n += 4;
   };
-  if (s < RP_BUFFERS) {
-    n += 2 * (RP_BUFFERS - 1 - s) + 4 * (RP_RING - s);
-    steps(0);
-  } else {
-    n += s - RP_BUFFERS + RP_RING < slabs ? 4 : 0;
-    steps(s - RP_BUFFERS + 1);
-  }
+  for (int i = 0; i < RP_BUFFERS; ++i) issue(i);
+  for (int i = 0; i + 1 < s; ++i) issue(i + RP_BUFFERS);
   return n < 63 ? n : 63;
 }
 template <typename F, int... I>
@@ -372,9 +374,9 @@ __device__ __forceinline__ void each(F f, std::integer_sequence<int, I...>) {
   (f(std::integral_constant<int, I>{}), ...);
 }
 
-template <int SLABS, int KIND>
-__global__ __launch_bounds__(256, RP_PER_CU) void rows_product_kernel(RowsProductArgs a) {
-  constexpr int KK = 64 * SLABS, BUF = RP_BM * 128;
+template <int SLABS, int KIND, int RB>
+__global__ __launch_bounds__(256, RB == 2 ? 3 : 2) void rows_product_kernel(RowsProductArgs a) {
+  constexpr int KK = 64 * SLABS, BM = 32 * RB, BN = RP_BN, BUF = BM * 128;
   __shared__ __attribute__((aligned(1024))) char sA[RP_BUFFERS * BUF];
   const int lane = threadIdx.x & 63, hh = lane >> 5, j = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -382,22 +384,23 @@ __global__ __launch_bounds__(256, RP_PER_CU) void rows_product_kernel(RowsProduc
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   const int sn = a.m_chunk == 1 ? slot : (int)__umulhi((uint32_t)slot, a.magic_chunk);
   const int tm = (xcd & (a.xcd_m - 1)) * a.m_chunk + slot - sn * a.m_chunk, tn = (xcd >> a.xcd_shift) * a.n_chunk + sn;
-  if (tm * RP_BM >= a.rows || tn * RP_BN >= a.N) return;
-  const int m0 = tm * RP_BM, blk = tn * (RP_BN / 32) + wave;
+  if (tm * BM >= a.rows || tn * BN >= a.N) return;
+  const int m0 = tm * BM, blk = tn * 4 + wave;
 
+  // a wave brings RB of a slab's 4 RB groups of eight rows
   const bf16_t* const x = a.x + (int64_t)m0 * KK;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)sA + 2048 * wave;
-  uint32_t off[2];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)sA + 1024 * RB * wave;
+  uint32_t off[RB];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int row = 8 * (2 * wave + i) + (lane >> 3);
+  for (int i = 0; i < RB; ++i) {
+    const int row = 8 * (RB * wave + i) + (lane >> 3);
     off[i] = (uint32_t)(min(row, a.rows - 1 - m0) * KK + ((lane & 7) ^ ((row >> 1) & 7)) * 8) * 2u;
   }
   auto bring = [&](auto s_c) {
     constexpr int s = decltype(s_c)::value;
     if constexpr (s < SLABS) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < RB; ++i)
         load_to_lds(x + 64 * s, off[i], __builtin_amdgcn_readfirstlane(lds0 + (s % RP_BUFFERS) * BUF + 1024 * i));
     }
   };
@@ -415,84 +418,122 @@ __global__ __launch_bounds__(256, RP_PER_CU) void rows_product_kernel(RowsProduc
     fetch(s_c);
   }, std::make_integer_sequence<int, RP_RING>{});
 
-  f32x16 acc[2];
+  f32x16 acc[RB];
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < RB; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
-  bf16x8 xf[2][2][4];
-  auto rows = [&](auto s_c) {
+  bf16x8 xf[2][RB];
+  auto rows = [&](auto s_c, int ks) {  // k-step ks of slab s
     constexpr int s = decltype(s_c)::value;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-        xf[s & 1][t][ks] = as_frag(*reinterpret_cast<const u32x4*>(sA + (s % RP_BUFFERS) * BUF + (32 * t + j) * 128 +
-                                                                   (((2 * ks + hh) ^ ((j >> 1) & 7)) << 4)));
+    for (int t = 0; t < RB; ++t)
+      xf[ks & 1][t] = as_frag(*reinterpret_cast<const u32x4*>(sA + (s % RP_BUFFERS) * BUF + (32 * t + j) * 128 +
+                                                              (((2 * ks + hh) ^ ((j >> 1) & 7)) << 4)));
   };
   auto landed = [&](auto s_c) {  // slab s is in LDS, for every wave
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(rows_product_younger(decltype(s_c)::value, SLABS)) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(rows_product_younger(decltype(s_c)::value, SLABS, RB)) : "memory");
     lds_barrier();
   };
+  // gated: gate and stream for eight columns of rows tid / 16, ..
+  const int tid = threadIdx.x;
+  constexpr int EACH = KIND == ROWS_GATED ? BM / 16 : 1;
+  float g[EACH][8];
+  u32x4 res[EACH];
+  auto load_gates = [&]() {
+    if constexpr (KIND == ROWS_GATED) {
+#pragma unroll
+      for (int e = 0; e < EACH; ++e) {
+        const int row = min(m0 + (tid >> 4) + 16 * e, a.rows - 1), col = tn * BN + (tid & 15) * 8;
+        const int cond = row - (a.cond_rows == 1 ? row : (int)__umulhi((uint32_t)row, a.magic_cond)) * a.cond_rows;
+        Elem<float>::load8(a.gate + (int64_t)cond * a.ld_gate + col, g[e]);
+        res[e] = *reinterpret_cast<const u32x4*>(a.out + (int64_t)row * a.ldc + col);
+      }
+    }
+  };
   landed(SLAB(0));
-  rows(SLAB(0));
+  rows(SLAB(0), 0);
   each([&](auto i_c) {
     constexpr int i = decltype(i_c)::value;
-    if constexpr (i + 1 < SLABS) {
-      landed(SLAB(i + 1));  // (and every wave has slab i's fragments: its buffer is free)
-      bring(SLAB(i + RP_BUFFERS));
-      rows(SLAB(i + 1));
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (ks < 3) {
+        rows(i_c, ks + 1);
+      } else if constexpr (i + 1 < SLABS) {
+        landed(SLAB(i + 1));  // (and every wave has slab i's fragments: its buffer is free)
+        bring(SLAB(i + RP_BUFFERS));
+        rows(SLAB(i + 1), 0);
+        if constexpr (i + 2 == SLABS) load_gates();  // (no counted wait behind it)
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < RB; ++t) acc[t] = mfma32(w[i % RP_RING][ks], xf[ks & 1][t], acc[t]);
     }
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int t = 0; t < 2; ++t) acc[t] = mfma32(w[i % RP_RING][ks], xf[i & 1][t][ks], acc[t]);
     fetch(SLAB(i + RP_RING));
   }, std::make_integer_sequence<int, SLABS>{});
 #undef SLAB
 
-  // a lane's registers 8 u .. are columns 32 blk + 16 u + 8 hh .. of rows j and 32 + j (SwiGLU: both factors of hidden units
-  // 16 blk + 8 hh ..)
-  const int col = 32 * blk + 8 * hh, seg = tn / (K / RP_BN);
-  float bias[16];
-  if constexpr (KIND == ROWS_QKVG)
+  // A lane's registers 8 u .. are columns 32 c + 16 u + 8 hh .. of row 32 t + j for column block c of the wave (SwiGLU: both factors of
+  // hidden units 16 c + 8 hh ..): 32 bytes of a row to a store.  So the tile goes through LDS, where the slabs were, and out in
+  // whole lines; pieces of 16 bytes at piece ^ (row % 16).
+  lds_barrier();
+  if constexpr (KIND == ROWS_GATED) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) load_param8(seg == 0 && a.q_bias ? a.q_bias + col + 16 * u : nullptr, 0.f, bias + 8 * u);
+    for (int t = 0; t < RB; ++t)
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int row = m0 + 32 * t + j;
-    if (row >= a.rows) break;
-    bf16_t* const out = a.out + (int64_t)row * a.ldc;
-    float o[16];
+      for (int p = 0; p < 4; ++p)
+        *reinterpret_cast<f32x4*>(sA + (32 * t + j) * 512 + (((8 * wave + 4 * (p >> 1) + 2 * hh + (p & 1)) ^ (j & 15)) << 4)) =
+            f32x4{acc[t][4 * p], acc[t][4 * p + 1], acc[t][4 * p + 2], acc[t][4 * p + 3]};
+    lds_barrier();
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[r] = acc[t][r];
-    if constexpr (KIND == ROWS_SWIGLU) {
+    for (int e = 0; e < EACH; ++e) {
+      const int r = (tid >> 4) + 16 * e, row = m0 + r;
+      float o[8], x[8];
+      unpack8(res[e], x);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = o[e] * sigmoidf_(o[e]) * o[8 + e];
-      *reinterpret_cast<u32x4*>(out + 16 * blk + 8 * hh) = pack8(o);
-    } else if constexpr (KIND == ROWS_QKVG) {
-      if (seg == 0) {
+      for (int q = 0; q < 2; ++q) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(sA + r * 512 + (((2 * (tid & 15) + q) ^ (r & 15)) << 4));
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[r] = (o[r] + bias[r]) * a.q_scale;
-      } else if (seg == 3) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[r] = sigmoidf_(o[r]);
+        for (int k = 0; k < 4; ++k) o[4 * q + k] = (v[k] + 0.f) * g[e][4 * q + k] + x[4 * q + k];
       }
+      if (row < a.rows) *reinterpret_cast<u32x4*>(a.out + (int64_t)row * a.ldc + tn * BN + (tid & 15) * 8) = pack8(o);
+    }
+  } else {
+    constexpr int COLS = KIND == ROWS_SWIGLU ? BN / 2 : BN, PIECES = COLS / 8;
+    const int seg = tn / (K / BN);
+    float bias[16];
+    if constexpr (KIND == ROWS_QKVG)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) *reinterpret_cast<u32x4*>(out + col + 16 * u) = pack8(o + 8 * u);
-    } else {
-      const int cond = row - (a.cond_rows == 1 ? row : (int)__umulhi((uint32_t)row, a.magic_cond)) * a.cond_rows;
-      const float* const gp = a.gate + (int64_t)cond * a.ld_gate + col;
+      for (int u = 0; u < 2; ++u)
+        load_param8(seg == 0 && a.q_bias ? a.q_bias + 32 * blk + 16 * u + 8 * hh : nullptr, 0.f, bias + 8 * u);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        float g[8], r[8];
-        Elem<float>::load8(gp + 16 * u, g);
-        Elem<bf16_t>::load8(out + col + 16 * u, r);
+    for (int t = 0; t < RB; ++t) {
+      char* const at = sA + (32 * t + j) * (2 * COLS);
+      float o[16];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[8 * u + e] = (o[8 * u + e] + 0.f) * g[e] + r[e];
+      for (int r = 0; r < 16; ++r) o[r] = acc[t][r];
+      if constexpr (KIND == ROWS_SWIGLU) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = o[e] * sigmoidf_(o[e]) * o[8 + e];
+        *reinterpret_cast<u32x4*>(at + (((2 * wave + hh) ^ (j & (PIECES - 1))) << 4)) = pack8(o);
+      } else {
+        if (seg == 0) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[r] = (o[r] + bias[r]) * a.q_scale;
+        } else if (seg == 3) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[r] = sigmoidf_(o[r]);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) *reinterpret_cast<u32x4*>(at + (((4 * wave + 2 * u + hh) ^ (j & (PIECES - 1))) << 4)) = pack8(o + 8 * u);
       }
+    }
+    lds_barrier();
 #pragma unroll
-      for (int u = 0; u < 2; ++u) *reinterpret_cast<u32x4*>(out + col + 16 * u) = pack8(o + 8 * u);
+    for (int e = 0; e < BM * PIECES / 256; ++e) {
+      const int i = tid + 256 * e, r = i / PIECES, p = i % PIECES;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(sA + r * (2 * COLS) + ((p ^ (r & (PIECES - 1))) << 4));
+      if (m0 + r < a.rows) *reinterpret_cast<u32x4*>(a.out + (int64_t)(m0 + r) * a.ldc + tn * COLS + p * 8) = v;
     }
   }
 }
@@ -578,27 +619,37 @@ bool rows_product_applies(const RowsProductArgs& a) {
                  : a.K == K && (a.swiglu || a.N == 4 * K));
 }
 
-// Faster than the products of gemm.hip (us at these rows, those / this):
-//   queries, keys, values, gate  340: 8.5 / 5.9   700: 10.7 / 9.4  1280: 13.6 / 10.2  1920: 17.3 / 13.3  2560: 19.9 / 16.7
-//                                3000: 24.8 / 22.2  3840: 25.0 / 24.0  5000: 31.0 / 30.3  7680: 51.3 / 48.8
-//   SwiGLU                       340: 6.7 / 5.2  1280: 10.0 / 8.9  2560: 15.6 / 15.0  3000: 18.7 / 19.0  3840: 19.2 / 21.5  5000: 24.1 / 27.5
-//   768 gated                    700: 6.7 / 6.6  1280: 7.0 / 6.6  1920: 8.4 / 6.8  2560: 9.4 / 7.0  2730: 10.6 / 11.5  3840: 11.4 / 11.9
-//   1536 gated                   700: 9.0 / 9.1  1280: 9.2 / 9.1  1920: 11.9 / 9.7  2560: 13.5 / 10.3  2730: 16.7 / 17.3  3840: 17.8 / 17.2
-// A tile of half the rows fills the chip sooner and pays for it with twice the reads of the weights: up to the rows whose 768
-// columns are one tile to a CU.  The widest of them has so much work to hand out that finer tiles lose nothing further on.
-bool rows_product_better(const RowsProductArgs& a) {
-  return rows_product_applies(a) && ((!a.gate && !a.swiglu) || (a.rows + RP_BM - 1) / RP_BM * (K / RP_BN) <= CUS);
+// Row blocks of a workgroup's tile.  A CU's time goes by the tiles that it gets, one after the other or at once, and a tile's by its
+// rows, less for a row the more there are, as they share the weights (us a tile, queries to gate: 3.25, 4.6 and 6.0): the blocks
+// with which the CU that gets most is done first.  us at these rows, two / three / four blocks / af3_linear_forward's kernels:
+//   queries to gate  700: 8.7 7.1 8.4 9.6   1280: 9.9 12.1 9.6 11.8   1920: 13.5 12.6 14.5 15.7  2560: 16.1 16.9 15.8 18.7
+//                    3200: 20.0 20.5 20.3 -   3840: 22.8 21.8 22.5 -   5600: 33.3 30.1 31.1 -     7680: 44.7 40.3 39.7 -
+//   SwiGLU           700: 7.7 6.4 7.6 8.9   1280: 9.2 10.8 8.7 9.9    1920: 12.3 11.6 13.3 13.2  2560: 15.3 14.8 14.5 16.9
+//                    3840: 21.4 19.7 21.2 20.6  5000: 27.2 26.8 25.1 25.5  5600: 30.7 28.3 30.0 35.6  7680: 40.7 36.8 36.6 36.8
+//   768 gated        700: 5.8 7.0 8.2 6.7   1920: 6.2 7.4 8.6 8.1     2560: 6.6 7.7 8.9 8.9      2730: 9.3 7.9 9.2 10.2
+//                    3840: 10.2 8.5 9.8 12.1  4600: 10.6 15.6 11.7 15.5  5600: 15.5 13.9 17.1 18.1  7680: 16.5 16.2 17.7 20.0
+//   1536 gated       700: 8.4 9.9 11.8 9.0  1920: 8.9 10.4 12.3 12.2  2560: 9.7 11.4 13.0 14.1   2730: 14.7 12.0 13.6 16.4
+//                    3840: 16.2 14.6 15.6 19.1  4600: 17.0 21.0 17.1 20.1  5600: 24.3 20.7 25.5 25.1  7680: 26.3 24.1 26.2 28.0
+static int rows_product_blocks(const RowsProductArgs& a) {
+  static constexpr int weight[3] = {65, 90, 120};
+  int best = 0, rb = 2;
+  for (int i = 0; i < 3; ++i) {
+    const int64_t tiles = (int64_t)((a.rows + 32 * (i + 2) - 1) / (32 * (i + 2))) * (a.N / RP_BN);
+    const int64_t cost = (tiles + CUS - 1) / CUS * weight[i];
+    if (i == 0 || cost < best) { best = (int)cost; rb = i + 2; }
+  }
+  return rb;
 }
 
-int launch_rows_product(const RowsProductArgs& args, hipStream_t s) {
-  if (!rows_product_applies(args)) return AF3_ERR_BAD_ARG;
+template <int RB>
+static int launch_rows(const RowsProductArgs& args, hipStream_t s) {
   RowsProductArgs a = args;
-  const int tiles_m = (a.rows + RP_BM - 1) / RP_BM, tiles_n = a.N / RP_BN, per_round = CUS / 8 * RP_PER_CU;
-  // the grid of XCDs with the fewest rounds of RP_PER_CU workgroups to a CU, and of those the one that fetches least
+  const int tiles_m = (a.rows + 32 * RB - 1) / (32 * RB), tiles_n = a.N / RP_BN, per_round = CUS / 8 * (RB == 2 ? 3 : 2);
+  // the grid of XCDs with the fewest rounds of workgroups, and of those the one that fetches least
   int64_t best = -1;
   for (int m = 1, shift = 0; m <= 8; m *= 2, ++shift) {
     const int mc = (tiles_m + m - 1) / m, nc = (tiles_n + 8 / m - 1) / (8 / m);
-    const int64_t cost = ((int64_t)(mc * nc + per_round - 1) / per_round << 32) + mc * RP_BM + nc * RP_BN;
+    const int64_t cost = ((int64_t)(mc * nc + per_round - 1) / per_round << 32) + mc * 32 * RB + nc * RP_BN;
     if (best >= 0 && cost >= best) continue;
     best = cost;
     a.xcd_m = m; a.xcd_shift = shift; a.m_chunk = mc; a.n_chunk = nc;
@@ -607,12 +658,21 @@ int launch_rows_product(const RowsProductArgs& args, hipStream_t s) {
   a.magic_cond = a.cond_rows <= 1 ? 0u : 0xffffffffu / (uint32_t)a.cond_rows + 1u;
   const dim3 grid(8u * a.m_chunk * a.n_chunk), block(256);
   if (a.gate) {
-    if (a.K == 768) hipLaunchKernelGGL((rows_product_kernel<12, ROWS_GATED>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((rows_product_kernel<24, ROWS_GATED>), grid, block, 0, s, a);
+    if (a.K == 768) hipLaunchKernelGGL((rows_product_kernel<12, ROWS_GATED, RB>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((rows_product_kernel<24, ROWS_GATED, RB>), grid, block, 0, s, a);
   } else if (a.swiglu) {
-    hipLaunchKernelGGL((rows_product_kernel<12, ROWS_SWIGLU>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((rows_product_kernel<12, ROWS_SWIGLU, RB>), grid, block, 0, s, a);
   } else {
-    hipLaunchKernelGGL((rows_product_kernel<12, ROWS_QKVG>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((rows_product_kernel<12, ROWS_QKVG, RB>), grid, block, 0, s, a);
   }
   return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+}
+
+int launch_rows_product(const RowsProductArgs& a, hipStream_t s) {
+  if (!rows_product_applies(a)) return AF3_ERR_BAD_ARG;
+  switch (rows_product_blocks(a)) {
+    case 2: return launch_rows<2>(a, s);
+    case 3: return launch_rows<3>(a, s);
+    default: return launch_rows<4>(a, s);
+  }
 }

@@ -40,6 +40,14 @@ def test_the_steps_give_the_bits_of_the_operators(gpu_pkg, samples, n, factor):
     assert seen and torch.isfinite(want).all() and not torch.equal(want, act) and torch.equal(got, want)
 
 
+# tiles of 96 and of 128 rows in every product, the last one short, full and by a row too long; hidden layers of 768 and 1536
+@pytest.mark.gpu
+@pytest.mark.parametrize("samples,n,factor", [(7, 95, 2), (6, 112, 1), (7, 137, 2), (7, 141, 1), (6, 160, 2), (7, 391, 2), (7, 384, 1), (6, 641, 2),
+                                              (7, 577, 1)])
+def test_rows_in_larger_tiles(gpu_pkg, samples, n, factor):
+    test_the_steps_give_the_bits_of_the_operators(gpu_pkg, samples, n, factor)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("samples,n", [(1, 40), (5, 100), (6, 20)])
 def test_a_null_plane_of_logits_is_no_bias(gpu_pkg, samples, n):
