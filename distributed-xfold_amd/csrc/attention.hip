@@ -65,6 +65,7 @@ template <int KSTEPS, int DVT, int NW, bool FAST>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(KSTEPS == 3 && NW == 1 ? 1 : 2)))
 void flash_kernel(FlashArgs a) {
   constexpr int KD = KSTEPS * 16;  // padded q/k head dim
+  constexpr bool SUM_COLUMN = KSTEPS == 3;  // (heads of 48: KD is the head's, so that the columns behind it are free)
   constexpr int LDK = KD + 8;      // sK row stride (bf16)
   constexpr int NT = NW * 64;
   __shared__ __attribute__((aligned(16))) bf16_t sK[2][KT * LDK];
@@ -216,12 +217,12 @@ void flash_kernel(FlashArgs a) {
     }
   };
   // V columns that no chunk covers (head dimension padding: columns KD .. 32 DVT - 1 of either buffer) must
-  // read as zero
+  // read as zero; with heads of 48 the first of them as ones, and the row sum comes out of the products with V
   if constexpr (KD < DVT * 32) {
     constexpr int PAD = DVT * 32 - KD;  // a multiple of 16
     for (int idx = tid; idx < 2 * KT * (PAD / 2); idx += NT) {
       const int row = idx / (PAD / 2), w = idx % (PAD / 2);
-      reinterpret_cast<uint32_t*>(&sV[row / KT][(row % KT) * LDV + KD])[w] = 0u;
+      reinterpret_cast<uint32_t*>(&sV[row / KT][(row % KT) * LDV + KD])[w] = SUM_COLUMN && w == 0 ? 0x3F80u : 0u;
     }
   }  // (no tile store touches these columns; the barrier after the first tile's stores orders them too)
 
@@ -383,15 +384,18 @@ void flash_kernel(FlashArgs a) {
         if (half == 1) bias_piece(2 + u);
       }
     // row sums of the ROUNDED probabilities on the matrix unit (ones * P), so
-    // that the weights that multiply V sum to exactly one after normalisation
-    f32x16 lsum;
+    // that the weights that multiply V sum to exactly one after normalisation;
+    // SUM_COLUMN: a column of ones beside V's, in the products below
+    if constexpr (!SUM_COLUMN) {
+      f32x16 lsum;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) lsum[r] = 0.f;
+      for (int r = 0; r < 16; ++r) lsum[r] = 0.f;
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int half = 0; half < 2; ++half) lsum = mfma32(onesf, pf[u][half], lsum);
-    l_run = l_run * alpha + lsum[0];
+        for (int half = 0; half < 2; ++half) lsum = mfma32(onesf, pf[u][half], lsum);
+      l_run = l_run * alpha + lsum[0];
+    }
     if (__any(alpha != 1.f)) {
 #pragma unroll
       for (int t = 0; t < DVT; ++t)
@@ -430,6 +434,10 @@ void flash_kernel(FlashArgs a) {
     for (int kt = 0; kt < nkt; ++kt) tile(kt, setA, setB);
   }
 
+  if constexpr (SUM_COLUMN) {  // row 48 of o, register 8 of the second block's lower half
+    const auto sum = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[DVT - 1][8]), __float_as_uint(o[DVT - 1][8]), false, false);
+    l_run = __uint_as_float(sum[0]);
+  }
   const float inv = 1.f / l_run;  // the ones * P sums cover both half-waves' keys
   if (!q_ok) return;
   // o[t][4g + e] = out(query j, head-dim 32t + 8g + 4hh + e)
@@ -466,10 +474,16 @@ void flash_kernel(FlashArgs a) {
 // last key reads as zeros or as whatever the plane holds; its logits become -inf), so a tile that is not full costs nothing
 // more; a masked key's logit is replaced by what stands beside it in LDS (two instructions a logit instead of nine); a tile's
 // bias is asked for two tiles ahead, into the accumulators as the exponentials empty them, its K and V one tile ahead.
-// Of 8.8 us at 100 tokens flash_kernel spent 2.2 before its first tile, 4.4 in two tiles and 1.4 behind them.  us, flash_kernel /
-// this, 16 heads: 5 x 40 tokens 7.7 / 5.3, 5 x 100 9.2 / 6.7, 5 x 256 12.0 / 9.4, 5 x 384 15.4 / 12.1, 1 x 768 25.1 / 20.9,
-// 5 x 768 32.1 / 28.7, 5 x 1536 106 / 94.  (The keys of a query shared out between two waves, 128 registers, four waves to a
-// SIMD: no faster from 128 tokens on, 6.9 and 28.0 at 100 and 768, and other bits.)
+// Of 8.8 us at 100 tokens flash_kernel spent 2.2 before its first tile, 4.4 in two tiles and 1.4 behind them; us, flash_kernel /
+// this, 16 heads: 5 x 40 tokens 7.7 / 5.3, 5 x 256 12.0 / 9.4, 1 x 768 25.1 / 20.9, 5 x 1536 106 / 94.
+// The row sum is a 49th column of V, of ones, in the product with V (four products a tile and their wait less), and a quarter's
+// products stand beside the next quarter's exponentials.  us, the sum by products of its own and all of V's behind the last
+// exponential / this: 5 x 40 5.1 / 4.9, 5 x 200 9.9 / 9.4, 1 x 384 11.8 / 11.1, 5 x 384 13.0 / 12.1, 3 x 512 14.8 / 13.8,
+// 1 x 768 21.4 / 21.9, 5 x 768 32.6 / 32.3, 5 x 1536 103.7 / 101.2.  What is left of a tile's 2800 cycles at 768 tokens: 330 K
+// products, 470 maximum, 980 exponentials and V, 310 (5 samples) to 640 (one) waiting for the bias, which comes from HBM, 510 the next tile's way
+// into LDS, 410 barrier.  No faster: a third set of bias registers (over 256, spills), the bias touched three to six tiles
+// ahead, the LDS stores in the middle of the tile (5 x 768 and up slower), the keys of a query shared out between two waves
+// of 128 registers (from 128 tokens on the same).
 constexpr int TOK_D = 48, TOK_LDK = 56, TOK_LDV = 96;
 constexpr int TOK_K_BYTES = KT * TOK_LDK * 2, TOK_TILE = TOK_K_BYTES + KT * TOK_LDV * 2;
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void token_attention_kernel(FlashArgs a) {
@@ -496,7 +510,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void t
   };
   const bf16_t *const kg = a.k + b * a.k_sb + h * TOK_D, *const vg = a.v + b * a.v_sb + h * TOK_D;
   const int k_bytes = ((a.Sk - 1) * (int)a.k_ss + TOK_D) * 2, v_bytes = ((a.Sk - 1) * (int)a.v_ss + TOK_D) * 2;
-  const int k_step = KT * (int)a.k_ss * 2, v_step = KT * (int)a.v_ss * 2;
   const int quad_step = (int)(a.bias_squad ? a.bias_squad : 4), quads = (a.Sk + 3) >> 2;
   const float* const bg = a.bias + (int64_t)b * a.bias_sb + (int64_t)h * a.bias_sh;
   const int b_bytes = ((a.Sq - 1) * (int)a.bias_sq + (quads - 1) * quad_step + 4) * 4, b_step = KT / 4 * quad_step * 4;
@@ -520,28 +533,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void t
   // piece i of this thread: K pieces first, then V (which of the two is uniform over a wave: CHUNKS is a multiple of 64)
   u32x4 rc[NL];
   uint32_t choff[NL], lds_at[NL];
+  const char* from_key[NL];  // (uniform) of the tile asked for next, and the bytes that are left from there
+  int left[NL], step[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int e = tid + i * 256;
-    const bool is_v = e >= CHUNKS;
+    const bool is_v = e >= CHUNKS, wave_v = wave * 64 + i * 256 >= CHUNKS;
+    from_key[i] = reinterpret_cast<const char*>(wave_v ? vg : kg);
+    left[i] = wave_v ? v_bytes : k_bytes;
+    step[i] = KT * 2 * (int)(wave_v ? a.v_ss : a.k_ss);
     const int ch = is_v ? e - CHUNKS : e, c = ch % (TOK_D / 8), key = ch / (TOK_D / 8);
     choff[i] = (uint32_t)(key * (int)(is_v ? a.v_ss : a.k_ss) + c * 8) * 2u;
     lds_at[i] = (is_v ? TOK_K_BYTES + key * (TOK_LDV * 2) : key * (TOK_LDK * 2)) + c * 16;
   }
   float mask_value = 1.f;  // of key tid of the tile asked for last (threads 0..63)
   auto load_tile = [&](int kt) {
-    const __amdgpu_buffer_rsrc_t krest = from(kg, k_bytes, kt * k_step), vrest = from(vg, v_bytes, kt * v_step);
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      if (wave * 64 + i * 256 < CHUNKS) rc[i] = __builtin_amdgcn_raw_buffer_load_b128(krest, choff[i], 0, 0);
-      else rc[i] = __builtin_amdgcn_raw_buffer_load_b128(vrest, choff[i], 0, 0);
+      rc[i] = __builtin_amdgcn_raw_buffer_load_b128(from(from_key[i], left[i], 0), choff[i], 0, 0);
+      from_key[i] += step[i];
+      left[i] -= step[i];
     }
     if (kmask && tid < KT) mask_value = kmask[min(kt * KT + tid, a.Sk - 1)];
   };
   auto store_tile = [&](int kt) {
-    const int buf = kt & 1;
 #pragma unroll
-    for (int i = 0; i < NL; ++i) *reinterpret_cast<u32x4*>(sTile[buf] + lds_at[i]) = rc[i];
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<u32x4*>(sTile[kt & 1] + lds_at[i]) = rc[i];
+  };
+  auto store_mask = [&](int kt) {
+    const int buf = kt & 1;
     if (tid < KT) {
       const float rep = kt * KT + tid >= a.Sk ? NEG_INF : (mask_value == 0.f ? -1e9f : 0.f);
       sRep[buf][tid] = rep;
@@ -558,19 +578,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void t
   load_tile(0);
 #pragma unroll
   for (int p = 0; p < 4; ++p) load_bias(setA, 0, p);
-  // V's columns 48..63 of either buffer, which the products read
+  // V's columns 48..63 of either buffer, which the products read: ones in the first, whose product is the row sum, and zeros
   for (int idx = tid; idx < 2 * KT * 2; idx += 256) {
     const int row = idx >> 1;
-    *reinterpret_cast<u32x4*>(sTile[row / KT] + TOK_K_BYTES + (row % KT) * (TOK_LDV * 2) + TOK_D * 2 + (idx & 1) * 16) = u32x4{0u, 0u, 0u, 0u};
+    *reinterpret_cast<u32x4*>(sTile[row / KT] + TOK_K_BYTES + (row % KT) * (TOK_LDV * 2) + TOK_D * 2 + (idx & 1) * 16) =
+        u32x4{idx & 1 ? 0u : 0x3F80u, 0u, 0u, 0u};
   }
   f32x16 o[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
-  float m_run = NEG_INF, l_run = 0.f;
-  const bf16x8 onesf = as_frag(u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+  float m_run = NEG_INF;
   store_tile(0);
+  store_mask(0);
   load_tile(1);
 #pragma unroll
   for (int p = 0; p < 4; ++p) load_bias(setB, 1, p);
@@ -579,11 +600,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void t
   auto tile = [&](int kt, f32x16 (&s)[2]) {
     const int buf = kt & 1;
     const char* kv = sTile[buf];
+    bf16x8 kf[3][2];
 #pragma unroll
     for (int ks = 0; ks < 3; ++ks)
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
-        s[u] = mfma32(lds_frag(reinterpret_cast<const bf16_t*>(kv), TOK_LDK, u * 32, ks * 16, lane), qf[ks], s[u]);
+      for (int u = 0; u < 2; ++u) kf[ks][u] = lds_frag(reinterpret_cast<const bf16_t*>(kv), TOK_LDK, u * 32, ks * 16, lane);
+    if (kt + 1 < nkt) store_mask(kt + 1);  // (the other buffer was last read in front of the barrier)
+#pragma unroll
+    for (int ks = 0; ks < 3; ++ks)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) s[u] = mfma32(kf[ks][u], qf[ks], s[u]);
+    // V's fragments, read while the exponentials' base is found (the transposing reads: see flash_kernel)
+    const int i16 = lane & 15;
+    const bf16_t* vbase = reinterpret_cast<const bf16_t*>(kv + TOK_K_BYTES) + (4 * hh + (i16 >> 2)) * TOK_LDV + 16 * ((lane >> 4) & 1) + 4 * (i16 & 3);
+    v4s vf[2][2][2];
+    auto read_v = [&](int p) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const bf16_t* vp = vbase + 16 * p * TOK_LDV + t * 32;
+        vf[p & 1][t][0] = lds_read_tr16(vp);
+        vf[p & 1][t][1] = lds_read_tr16(vp + 8 * TOK_LDV);
+      }
+    };
+    read_v(0);
+    __builtin_amdgcn_sched_barrier(0);
     if (__builtin_amdgcn_readfirstlane(sAny[buf])) {
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
@@ -600,41 +640,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void t
     const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * LOG2E);
     m_run = m_new;
     const float m2 = m_new * LOG2E;
-    bf16x8 pf[4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      float pv[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[p >> 1][8 * (p & 1) + e], LOG2E, -m2));
-      pf[p] = as_frag(pack8(pv));
-      __builtin_amdgcn_sched_barrier(0);
-      load_bias(s, kt + 2, p);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // row sums of the rounded probabilities (ones * P)
-    f32x16 lsum;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) lsum[r] = 0.f;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) lsum = mfma32(onesf, pf[p], lsum);
-    l_run = l_run * alpha + lsum[0];
     if (__any(alpha != 1.f)) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
     }
-    // the transposing reads of V: see flash_kernel
-    const int i16 = lane & 15;
-    const bf16_t* vbase = reinterpret_cast<const bf16_t*>(kv + TOK_K_BYTES) + (4 * hh + (i16 >> 2)) * TOK_LDV + 16 * ((lane >> 4) & 1) + 4 * (i16 & 3);
+    // a quarter's products run beside the next one's exponentials
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
+    for (int p = 0; p < 4; ++p) {
+      float pv[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[p >> 1][8 * (p & 1) + e], LOG2E, -m2));
+      const bf16x8 pf = as_frag(pack8(pv));
+      __builtin_amdgcn_sched_barrier(0);
+      if (p < 3) read_v(p + 1);
+      load_bias(s, kt + 2, p);
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        const bf16_t* vp = vbase + 16 * p * TOK_LDV + t * 32;
-        const v4s lo = lds_read_tr16(vp), hi = lds_read_tr16(vp + 8 * TOK_LDV);
-        o[t] = mfma32(as_frag(__builtin_bit_cast(u32x4, v8s{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w})), pf[p], o[t]);
+        const v4s lo = vf[p & 1][t][0], hi = vf[p & 1][t][1];
+        o[t] = mfma32(as_frag(__builtin_bit_cast(u32x4, v8s{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w})), pf, o[t]);
       }
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if (kt + 1 < nkt) {
       store_tile(kt + 1);
       load_tile(kt + 2);
@@ -658,7 +686,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void t
     if (kt + 1 < nkt) tile(kt + 1, setB);
   }
 
-  const float inv = 1.f / l_run;
+  // the sum of the rounded probabilities: row 48 of o, register 8 of the second block's lower half
+  const auto sum = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[1][8]), __float_as_uint(o[1][8]), false, false);
+  const float inv = 1.f / __uint_as_float(sum[0]);
   if (q0 + j >= a.Sq) return;
   const int64_t at = (int64_t)b * a.o_sb + row * a.o_ss + h * TOK_D + 4 * hh;
 #pragma unroll
