@@ -64,6 +64,7 @@ template <int KSTEPS, int DVT, int NW, bool FAST>
 // head dimension 48 stages twelve chunks per thread and is given the whole register file)
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(KSTEPS == 3 && NW == 1 ? 1 : 2)))
 void flash_kernel(FlashArgs a) {
+  args_at_once<FlashArgs>();
   constexpr int KD = KSTEPS * 16;  // padded q/k head dim
   constexpr bool SUM_COLUMN = KSTEPS == 3;  // (heads of 48: KD is the head's, so that the columns behind it are free)
   constexpr int LDK = KD + 8;      // sK row stride (bf16)
@@ -487,6 +488,7 @@ void flash_kernel(FlashArgs a) {
 constexpr int TOK_D = 48, TOK_LDK = 56, TOK_LDV = 96;
 constexpr int TOK_K_BYTES = KT * TOK_LDK * 2, TOK_TILE = TOK_K_BYTES + KT * TOK_LDV * 2;
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void token_attention_kernel(FlashArgs a) {
+  args_at_once<FlashArgs>();
   constexpr int CHUNKS = KT * (TOK_D / 8), NL = 2 * CHUNKS / 256;  // 16-byte pieces of a K (V) tile; of both, per thread
   __shared__ __attribute__((aligned(16))) char sTile[2][TOK_TILE];  // [buffer]: K rows, V rows
   __shared__ __attribute__((aligned(16))) float sRep[2][KT];        // what takes the place of a masked key's logit, or 0
@@ -739,6 +741,7 @@ __device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
 constexpr int WKEYS = 128;
 template <int TILES>
 __global__ __launch_bounds__(256, TILES == 2 ? 2 : 4) void window_kernel(FlashArgs a) {
+  args_at_once<FlashArgs>();
   __shared__ __attribute__((aligned(1024))) bf16_t sK[64 * TILES * 128];
   __shared__ __attribute__((aligned(1024))) bf16_t sV[64 * TILES * 128];
   __shared__ __attribute__((aligned(16))) int sCode[WKEYS];

@@ -133,6 +133,7 @@ enum { BIG_PLAIN = 0, BIG_COLUMN_OPS = 1, BIG_SWIGLU = 2, BIG_OUTER_MEAN = 3 };
 
 template <int MODE, int IT = 4>
 __global__ __launch_bounds__(256, 1) void contract_kernel(GemmArgs g) {
+  args_at_once<GemmArgs>();
   constexpr int CM = 64 * IT, WM = 32 * IT;  // block and wave extent along i
   constexpr int SLAB_A = CM * ROWB;
   constexpr int LA = 2 * IT, NLOAD = LA + 8;  // loads per wave and slab, of which A

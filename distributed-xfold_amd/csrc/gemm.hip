@@ -71,6 +71,7 @@ __device__ __forceinline__ void wait_loads_but() {
 enum { KIND_COLUMNS = 0, KIND_GATE_RES = 1, KIND_SWIGLU = 2 };
 template <int MT, int NT, int WM, int WN, int WK, int ST, int WPS, bool CLEAN, int KIND, bool VEC, bool OUT_F32>
 __global__ __launch_bounds__(64 * WM * WN * WK, WPS) void gemm_nt_kernel(GemmArgs g) {
+  args_at_once<GemmArgs>();
   constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN, NTHR = 64 * WM * WN * WK, GW = WM * WN;
   constexpr int SLAB = (BM + BN) * ROWB;     // A rows first, then B rows
   constexpr int NLOAD = (BM + BN) / 8 / GW;  // 1 KB loads per wave and slab

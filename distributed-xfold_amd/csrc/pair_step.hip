@@ -94,6 +94,7 @@ constexpr int pieces_in_flight(int ch, int pb, int waves, bool transition) {
 
 template <typename TIO, int CH, int PB, int IN, int MAP, bool TRANSITION, int NEXT, int PER_SIMD>
 __global__ __launch_bounds__(2 * CH, PER_SIMD) void pair_step_kernel(PairStepArgs a) {
+  args_at_once<PairStepArgs>();
   using E = Elem<TIO>;
   constexpr int TS = 32 * PB;           // positions per tile, in blocks of an MFMA's 32
   constexpr int C = CH, D = C / H, LDX = C + 8, LDS_F = C + 4;

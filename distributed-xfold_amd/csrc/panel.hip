@@ -82,6 +82,7 @@ __device__ __forceinline__ void multiply(const PanelArgs& a, const char* sA, con
 }
 
 __global__ __launch_bounds__(64 * WAVES) void panel_product_kernel(PanelArgs a) {
+  args_at_once<PanelArgs>();
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -22,6 +22,7 @@ constexpr int KSTEPS = K / 16 / 2, GROUP = 6;  // of a wave; of these, whose fra
 
 template <typename TIO, bool SWIGLU>
 __global__ __launch_bounds__(256, 2) void single_step_kernel(SingleStepArgs a) {
+  args_at_once<SingleStepArgs>();
   using E = Elem<TIO>;
   constexpr int EACH = ROWS / 16;  // rows of a group of sixteen lanes
   // slabs of 64 channels, [slab][row][128 bytes], chunk c (16 bytes) of a row at position c ^ (row / 2 % 8)

@@ -34,6 +34,7 @@ constexpr int CUS = 256, WARM_CUS = 24;  // of which some for the workgroups tha
 // TPW: tokens of a wave, SMAX: samples at most
 template <int TPW, int SMAX, bool SWIGLU>
 __global__ __launch_bounds__(64 * NW, 2) void norm_product_kernel(NormProductArgs a) {
+  args_at_once<NormProductArgs>();
   __shared__ __attribute__((aligned(1024))) char sP[PANEL];
   const int tid = threadIdx.x, lane = tid & 63, hh = lane >> 5, j = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -250,6 +251,7 @@ __device__ __forceinline__ void load_to_lds(const void* base, uint32_t off, uint
 // 5 x 100 1132 / 1044, 5 x 126 1335 / 1185, 1 x 100 1024 / 905, 3 x 100 1080 / 961, 2 x 300 1423 / 1330.
 template <int KP, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, 1) void gated_product_kernel(GatedProductArgs a) {
+  args_at_once<GatedProductArgs>();
   constexpr int KK = 128 * KP, SLABS = KK / 64, RING = 5;
   __shared__ __attribute__((aligned(1024))) char sP[SLABS * ROWS * 128];
   const int lane = threadIdx.x & 63, hh = lane >> 5, j = lane & 31;
@@ -376,6 +378,7 @@ __device__ __forceinline__ void each(F f, std::integer_sequence<int, I...>) {
 
 template <int SLABS, int KIND, int RB>
 __global__ __launch_bounds__(256, RB == 2 ? 3 : 2) void rows_product_kernel(RowsProductArgs a) {
+  args_at_once<RowsProductArgs>();
   constexpr int KK = 64 * SLABS, BM = 32 * RB, BN = RP_BN, BUF = BM * 128;
   __shared__ __attribute__((aligned(1024))) char sA[RP_BUFFERS * BUF];
   const int lane = threadIdx.x & 63, hh = lane >> 5, j = lane & 31;

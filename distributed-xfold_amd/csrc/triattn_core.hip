@@ -126,6 +126,7 @@ __device__ __forceinline__ void scale_in_place(f32x16& o, float f) {
 
 template <int R, bool HAS_BIAS, int D, bool SPARE>
 __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void triattn_flash_kernel(TriAttnArgs a) {
+  args_at_once<TriAttnArgs>();
   constexpr int TILE_BYTES = tile_bytes(D);
   constexpr int KS = D / 16;  // k-steps of the score product
   // [buffer][row] as separate arrays: a load in flight to one of them provably does not alias
