@@ -77,6 +77,11 @@ template <> struct Elem<bf16_t> {
   static constexpr int kBatch = 8;  // 8-element groups to keep in flight at a time (4 VGPRs each)
   static __device__ __forceinline__ Raw load_raw(const bf16_t* p) { return Raw{*reinterpret_cast<const u32x4*>(p)}; }
   static __device__ __forceinline__ void unpack_raw(const Raw& r, float* f) { unpack8(r.v, f); }
+  struct Raw4 { u32x2 v; };
+  static __device__ __forceinline__ Raw4 load_raw4(const bf16_t* p) { return Raw4{*reinterpret_cast<const u32x2*>(p)}; }
+  static __device__ __forceinline__ void unpack_raw4(const Raw4& r, float* f) {
+    f[0] = bflo(r.v.x); f[1] = bfhi(r.v.x); f[2] = bflo(r.v.y); f[3] = bfhi(r.v.y);
+  }
 };
 template <> struct Elem<float> {
   static __device__ __forceinline__ void load8(const float* p, float* f) {
@@ -101,6 +106,9 @@ template <> struct Elem<float> {
     f[0] = r.a.x; f[1] = r.a.y; f[2] = r.a.z; f[3] = r.a.w;
     f[4] = r.b.x; f[5] = r.b.y; f[6] = r.b.z; f[7] = r.b.w;
   }
+  struct Raw4 { f32x4 v; };
+  static __device__ __forceinline__ Raw4 load_raw4(const float* p) { return Raw4{*reinterpret_cast<const f32x4*>(p)}; }
+  static __device__ __forceinline__ void unpack_raw4(const Raw4& r, float* f) { f[0] = r.v.x; f[1] = r.v.y; f[2] = r.v.z; f[3] = r.v.w; }
 };
 
 // sigmoid through the hardware exp2 / reciprocal (about 1 ulp each): four
@@ -206,6 +214,43 @@ __device__ __forceinline__ float add_squares8(const float* d, float q, bool begi
 #pragma unroll
   for (int e = 2; e < 8; ++e) q = __builtin_fmaf(d[e], d[e], q);
   return q;
+}
+
+__device__ __forceinline__ float add_squares4(const float* d, float q) {
+  q = __builtin_fmaf(d[1], d[1], __builtin_fmaf(d[0], d[0], q));
+  return __builtin_fmaf(d[3], d[3], __builtin_fmaf(d[2], d[2], q));
+}
+
+// Rows of 513 to 768 channels: a lane takes eight channels from 8 lane on and four from 512 + 4 lane on, so that at 768 none is
+// idle.  The bf16 values of both parts.
+__device__ __forceinline__ void unpack12(const u32x4 a, const u32x2 b, float* f) {
+  unpack8(a, f);
+  f[8] = bflo(b.x); f[9] = bfhi(b.x); f[10] = bflo(b.y); f[11] = bfhi(b.y);
+}
+// x / 768.f, the same bits (a correctly rounded quotient from the rounded reciprocal and the exact remainder) in four instructions
+// instead of some twelve; an infinity, whose remainder is none, stays one.
+__device__ __forceinline__ float over_768(float x) {
+  const float r = 1.f / 768.f, q = x * r;
+  return fminf(__builtin_fmaf(__builtin_fmaf(-q, 768.f, x), r, q), __builtin_huge_valf());
+}
+
+// A word of N lines of 128 bytes, first, first + step, .. of three ranges one behind the other, into the last-level cache.  (The
+// ranges by value: chosen between in memory, each line's address was a load of its own with a wait behind it and the line before.)
+template <int N>
+__device__ __forceinline__ void bring_lines(const void* const (&range)[3], const uint32_t (&lines)[3], uint32_t first, uint32_t step) {
+  uintptr_t p0 = (uintptr_t)range[0], p1 = (uintptr_t)range[1], p2 = (uintptr_t)range[2];
+  uint32_t n0 = lines[0], n1 = n0 + lines[1], n2 = n1 + lines[2];
+  asm volatile("" : "+s"(p0), "+s"(p1), "+s"(p2), "+s"(n0), "+s"(n1), "+s"(n2));
+  uint32_t got[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const uint32_t i = first + u * step;
+    const uintptr_t p = i < n0 ? p0 : i < n1 ? p1 : p2;
+    got[u] = 0u;
+    if (i < n2) got[u] = *reinterpret_cast<const __attribute__((address_space(1))) uint32_t*>(p + (size_t)(i - (i < n0 ? 0u : i < n1 ? n0 : n1)) * 128);
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) asm volatile("" ::"v"(got[u]));
 }
 
 // A kernel's arguments lie in memory, and what it reads of them it reads where it needs them: a first trip for what the workgroup

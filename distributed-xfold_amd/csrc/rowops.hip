@@ -60,24 +60,16 @@ __device__ __forceinline__ int64_t cond_row(const RowNormArgs& a, int64_t row) {
 // that a few hundred rows do not cover (500x768x768 6.7 us with its weights in HBM, 5.8 in the cache; x1536 9.5, 7.8;
 // 500x3072x768 10.1, 7.6), while this kernel leaves half of the CUs idle.  Workgroups behind those of the rows touch
 // every line of what the next kernels read, and nobody waits for them but the kernel's end.  (A token transformer of 24
-// blocks, 311 MB of weights: 500 rows 1.93 -> 1.80 ms, 3840 rows 3.8 -> 3.5 ms.)
+// blocks, 311 MB of weights: 500 rows 1.93 -> 1.80 ms, 3840 rows 3.8 -> 3.5 ms.)  All lines of a thread at once: one after the
+// other, they are what the kernel's end waits for (5 x 384 rows 6.5 us against 5.1).
 constexpr int WARM_LINES = 4;  // per thread (8: 500 rows of 768 behind 5.9 MB of weights 4 % slower, 1 or 2: no faster)
+__device__ __forceinline__ void warm_lines(const RowNormArgs& a) {
+  bring_lines<WARM_LINES>(a.warm, a.warm_lines, (blockIdx.x - a.row_blocks) * (WARM_LINES * 256u) + threadIdx.x, 256u);
+}
 template <typename TIn, int NCH>
 __global__ __launch_bounds__(256) void ln_rows_kernel(RowNormArgs a) {
   const int lane = threadIdx.x & 63;
-  if (blockIdx.x >= a.row_blocks) {
-    const uint32_t n0 = a.warm_lines[0], n1 = n0 + a.warm_lines[1], n2 = n1 + a.warm_lines[2];
-    uint32_t got[WARM_LINES];
-#pragma unroll
-    for (int u = 0; u < WARM_LINES; ++u) {
-      const uint32_t i = ((blockIdx.x - a.row_blocks) * WARM_LINES + u) * 256u + threadIdx.x;
-      const char* p = static_cast<const char*>(i < n0 ? a.warm[0] : i < n1 ? a.warm[1] : a.warm[2]);
-      got[u] = i < n2 ? *reinterpret_cast<const uint32_t*>(p + (size_t)(i - (i < n0 ? 0u : i < n1 ? n0 : n1)) * 128) : 0u;
-    }
-#pragma unroll
-    for (int u = 0; u < WARM_LINES; ++u) asm volatile("" ::"v"(got[u]));
-    return;
-  }
+  if (blockIdx.x >= a.row_blocks) return warm_lines(a);
   const int64_t row = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= a.rows) return;
   const TIn* x = reinterpret_cast<const TIn*>(a.x) + row * a.ldx;
@@ -123,6 +115,71 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(RowNormArgs a) {
       p[i].finish(a, v[i], mean, rstd, o);
       *reinterpret_cast<u32x4*>(y + c) = pack8(o);
     }
+  }
+}
+
+// The adaptive norm of 768 channels, twelve to a lane (unpack12) where two chunks of 512 leave a quarter of the lanes without a
+// channel.  With several samples on one conditioning a wave takes S of a token's rows: its scale and shift, four times a row's
+// bytes, are fetched once and their sigmoid is taken once, and the rows' chains run beside each other.  us, a row to a wave of
+// ln_rows_kernel / this: 1 x 768 rows 6.0 / 5.6, 5 x 256 6.2 / 5.1, 3 x 512 6.2 / 5.1, 5 x 384 6.6 / 5.1, 8 x 384 7.5 / 5.4, 5 x 768
+// 8.0 / 5.9, 5 x 1536 12.9 / 8.4.  What bounds it: the conditioning's trip from memory, and the lines brought nearer beside it.
+template <typename TIn, int S>
+__global__ __launch_bounds__(256) void ln_rows_768_kernel(RowNormArgs a) {
+  args_at_once<RowNormArgs>();
+  if (blockIdx.x >= a.row_blocks) return warm_lines(a);
+  const int lane = threadIdx.x & 63, c0 = lane * 8, c1 = 512 + lane * 4;
+  const uint32_t item = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), cond_rows = (uint32_t)a.cond_rows;
+  const uint32_t group = item / cond_rows, token = item - group * cond_rows;
+  const int s0 = (int)group * S, count = min(S, a.samples - s0);
+  if (count <= 0) return;
+  const TIn* x = reinterpret_cast<const TIn*>(a.x) + ((int64_t)s0 * cond_rows + token) * a.ldx;
+  typename Elem<TIn>::Raw raw[S];
+  typename Elem<TIn>::Raw4 raw4[S];
+#pragma unroll
+  for (int k = 0; k < S; ++k) {
+    raw[k] = Elem<TIn>::load_raw(x + c0);
+    raw4[k] = Elem<TIn>::load_raw4(x + c1);
+    x += k + 1 < count ? cond_rows * a.ldx : 0;
+  }
+  f32x4 sc[3], sh[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int64_t at = token * a.ld_cond + (i < 2 ? c0 + 4 * i : c1);
+    sc[i] = *reinterpret_cast<const f32x4*>(a.scale + at);
+    sh[i] = *reinterpret_cast<const f32x4*>(a.shift + at);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  float v[S][12], rstd[S];
+#pragma unroll
+  for (int k = 0; k < S; ++k) {
+    float s = 0.f;
+    Elem<TIn>::unpack_raw(raw[k], v[k]);
+    Elem<TIn>::unpack_raw4(raw4[k], v[k] + 8);
+#pragma unroll
+    for (int e = 0; e < 12; ++e) s += v[k][e];
+    const float mean = over_768(wave_sum(s));
+#pragma unroll
+    for (int e = 0; e < 12; ++e) v[k][e] -= mean;
+    rstd[k] = rsqrtf(over_768(wave_sum(add_squares4(v[k] + 8, add_squares8(v[k], 0.f, true)))) + LN_EPS);
+  }
+  __builtin_amdgcn_sched_barrier(0);  // (the conditioning comes from further away than the rows: nothing of it in front of their sums)
+  float gain[12];
+#pragma unroll
+  for (int e = 0; e < 12; ++e) gain[e] = sigmoidf_(sc[e >> 2][e & 3]);
+  bf16_t* y = a.y + ((int64_t)s0 * cond_rows + token) * a.ldy;
+#pragma unroll
+  for (int k = 0; k < S; ++k) {
+    float o[12];
+#pragma unroll
+    for (int e = 0; e < 12; ++e) {
+      const float t = v[k][e] * rstd[k];
+      o[e] = gain[e] * t + sh[e >> 2][e & 3];
+    }
+    if (k < count) {
+      *reinterpret_cast<u32x4*>(y + c0) = pack8(o);
+      *reinterpret_cast<u32x2*>(y + c1) = u32x2{pack2bf(o[8], o[9]), pack2bf(o[10], o[11])};
+    }
+    y += cond_rows * a.ldy;
   }
 }
 
@@ -200,10 +257,29 @@ int launch_small(RowNormArgs a, hipStream_t stream) {
 template <typename TIn>
 int launch_wide(RowNormArgs a, hipStream_t stream) {
   const int64_t lines = (int64_t)a.warm_lines[0] + a.warm_lines[1] + a.warm_lines[2];
-  const int64_t row_blocks = (a.rows + 3) / 4, blocks = row_blocks + (lines + 256 * WARM_LINES - 1) / (256 * WARM_LINES);
+  const bool twelve = a.C == 768 && a.scale && !a.weight && !a.bias && a.cond_vec && a.rows % a.cond_rows == 0;
+  int s = 1;
+  if (twelve) {  // as many of a token's rows to a wave as registers let run at once, shared out evenly (one to a wave: 5 x 768 rows 8.3 us
+                 // against 7.4, 5 x 1536 10.8 against 8.9; three: 8.2 and 9.4)
+    a.samples = (int)(a.rows / a.cond_rows);
+    const int groups = (a.samples + 4) / 5;
+    s = (a.samples + groups - 1) / groups;
+  }
+  const int64_t waves = twelve ? a.cond_rows * ((a.samples + s - 1) / s) : a.rows;
+  const int64_t row_blocks = (waves + 3) / 4, blocks = row_blocks + (lines + 256 * WARM_LINES - 1) / (256 * WARM_LINES);
   a.row_blocks = (unsigned)row_blocks;
   if (lines > 0x7fffffff || blocks > 0x7fffffff) return AF3_ERR_BAD_ARG;
   const dim3 grid((unsigned)blocks), block(256);
+  if (twelve) {
+    switch (s) {
+      case 1: hipLaunchKernelGGL((ln_rows_768_kernel<TIn, 1>), grid, block, 0, stream, a); break;
+      case 2: hipLaunchKernelGGL((ln_rows_768_kernel<TIn, 2>), grid, block, 0, stream, a); break;
+      case 3: hipLaunchKernelGGL((ln_rows_768_kernel<TIn, 3>), grid, block, 0, stream, a); break;
+      case 4: hipLaunchKernelGGL((ln_rows_768_kernel<TIn, 4>), grid, block, 0, stream, a); break;
+      default: hipLaunchKernelGGL((ln_rows_768_kernel<TIn, 5>), grid, block, 0, stream, a); break;
+    }
+    return hipGetLastError() == hipSuccess ? AF3_OK : AF3_ERR_LAUNCH;
+  }
   switch ((a.C + 511) / 512) {
     case 1: hipLaunchKernelGGL((ln_rows_kernel<TIn, 1>), grid, block, 0, stream, a); break;
     case 2: hipLaunchKernelGGL((ln_rows_kernel<TIn, 2>), grid, block, 0, stream, a); break;

@@ -11,11 +11,12 @@
 // Values are rounded where the separate kernels store them and every sum has their order: the same bits.
 //
 // What bounds it: 0.45 MB of weights, rows and conditioning through the CU's vector memory path (64 bytes a cycle: 3.3 us at
-// 2.1 GHz) and the norms' vector instructions, 700 a row, which overlap but for their ends.  100 tokens of 5 samples, cycles of a
-// wave: rows there 3700, norms 6000, barrier 1500, product 3000, result 1000.  9.3 and 9.0 us against 5.1 + 9.9 and 5.1 + 8.2; a
-// token transformer of 24 blocks, us, norm and rows_product_kernel / this: 1 x 100 tokens 975 / 844, 1 x 256 1112 / 1038, 3 x 100
-// 1015 / 907, 4 x 128 1095 / 1031, 5 x 60 966 / 849, 5 x 100 1081 / 989, 5 x 126 1222 / 1194.  At one workgroup to a CU the
-// twelvefold norms cost what they save (3 x 200 1185 / 1197); past it, more.
+// 2.1 GHz) and the norms' vector instructions, which overlap but for their ends.  100 tokens of 5 samples: 9.2 us either, and
+// of a wave's 15000 cycles 3700 until the rows are there, 5000 norms, 3000 product, 1000 result, the rest at the barrier between.
+// (The norms with eight channels to a lane in two chunks, a quarter of the second without any, and the division by 768 as it
+// stands: 9.5 and 9.7 us.)  An evaluation of the diffusion head, us, norm and rows_product_kernel / this: 1 x 100 tokens 1143 / 1024,
+// 1 x 256 1286 / 1209, 3 x 120 1220 / 1141, 4 x 128 1265 / 1194, 5 x 60 1158 / 1033, 5 x 100 1267 / 1167, 5 x 120 1302 / 1251.  At one
+// workgroup to a CU the twelvefold norms cost what they save (3 x 200 1350 / 1363); past it, more.
 #include <type_traits>
 #include <utility>
 
@@ -40,16 +41,7 @@ __global__ __launch_bounds__(64 * NW, 2) void norm_product_kernel(NormProductArg
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (blockIdx.x >= a.work_blocks) {
     // workgroups on the idle CUs bring what the next kernels read into the last-level cache (see ln_rows_kernel)
-    const uint32_t n0 = a.warm_lines[0], n1 = n0 + a.warm_lines[1], n2 = n1 + a.warm_lines[2];
-    uint32_t got[WARM_LINES];
-#pragma unroll
-    for (int u = 0; u < WARM_LINES; ++u) {
-      const uint32_t i = ((blockIdx.x - a.work_blocks) * WARM_LINES + u) * (64u * NW) + tid;
-      const char* p = static_cast<const char*>(i < n0 ? a.warm[0] : i < n1 ? a.warm[1] : a.warm[2]);
-      got[u] = i < n2 ? *reinterpret_cast<const uint32_t*>(p + (size_t)(i - (i < n0 ? 0u : i < n1 ? n0 : n1)) * 128) : 0u;
-    }
-#pragma unroll
-    for (int u = 0; u < WARM_LINES; ++u) asm volatile("" ::"v"(got[u]));
+    bring_lines<WARM_LINES>(a.warm, a.warm_lines, (blockIdx.x - a.work_blocks) * (WARM_LINES * 64u * NW) + tid, 64u * NW);
     return;
   }
   // A range of the weights' rows for every XCD, each with the tiles of all rows one after the other
@@ -76,27 +68,27 @@ __global__ __launch_bounds__(64 * NW, 2) void norm_product_kernel(NormProductArg
       }
     }
   };
-  u32x4 raw[TPW][SMAX][2];
-  f32x4 sc[TPW][2][2], sh[TPW][2][2];
-  const int c0 = lane * 8, c1 = min(512 + lane * 8, K - 8);
+  u32x4 raw[TPW][SMAX];
+  u32x2 raw4[TPW][SMAX];
+  f32x4 sc[TPW][3], sh[TPW][3];
+  const int c0 = lane * 8, c1 = 512 + lane * 4;
 #pragma unroll
   for (int k = 0; k < TPW; ++k) {
     const int token = min(t0 + min(tt_0 + NW * k, tt_n - 1), a.tokens - 1);
     const bf16_t* x = a.x + (s_0 * a.tokens + token) * K;
 #pragma unroll
     for (int s = 0; s < SMAX; ++s) {
-      raw[k][s][0] = *reinterpret_cast<const u32x4*>(x + c0);
-      raw[k][s][1] = *reinterpret_cast<const u32x4*>(x + c1);
+      raw[k][s] = *reinterpret_cast<const u32x4*>(x + c0);
+      raw4[k][s] = *reinterpret_cast<const u32x2*>(x + c1);
       x += s + 1 < count ? a.tokens * K : 0;
     }
     const float* p = a.scale + (int64_t)token * a.ld_cond;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        sc[k][i][q] = *reinterpret_cast<const f32x4*>(p + (i ? c1 : c0) + 4 * q);
-        sh[k][i][q] = *reinterpret_cast<const f32x4*>(p + K + (i ? c1 : c0) + 4 * q);
-      }
+    for (int i = 0; i < 3; ++i) {
+      const int c = i < 2 ? c0 + 4 * i : c1;
+      sc[k][i] = *reinterpret_cast<const f32x4*>(p + c);
+      sh[k][i] = *reinterpret_cast<const f32x4*>(p + K + c);
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
   bf16x8 w[NB][8];
@@ -115,55 +107,49 @@ __global__ __launch_bounds__(64 * NW, 2) void norm_product_kernel(NormProductArg
 #pragma unroll
     for (int k = 0; k < TPW; ++k)
 #pragma unroll
-      for (int s = 0; s < SMAX; ++s) asm volatile("" ::"v"(raw[k][s][0].x), "v"(raw[k][s][1].x));
+      for (int s = 0; s < SMAX; ++s) asm volatile("" ::"v"(raw[k][s].x), "v"(raw4[k][s].x));
   fetch(PIECE(0));
 
-  // adaptive LayerNorm, ln_rows_kernel's sums
-  const bool upper = 512 + lane * 8 < K;
-  float v[TPW][SMAX][16], rstd[TPW][SMAX];
+  // adaptive LayerNorm, ln_rows_768_kernel's sums
+  float v[TPW][SMAX][12], rstd[TPW][SMAX];
   if (busy)
     each_row([&](int k, int s) {
       float* x = v[k][s];
-      float sum = 0.f, more;
-      unpack8(raw[k][s][0], x);
-      unpack8(raw[k][s][1], x + 8);
+      float sum = 0.f;
+      unpack12(raw[k][s], raw4[k][s], x);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sum += x[e];
-      more = sum;
+      for (int e = 0; e < 12; ++e) sum += x[e];
+      const float mean = over_768(wave_sum(sum));
 #pragma unroll
-      for (int e = 8; e < 16; ++e) more += x[e];
-      const float mean = wave_sum(upper ? more : sum) / (float)K;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) x[e] -= mean;
+      for (int e = 0; e < 12; ++e) x[e] -= mean;
     });
   fetch(PIECE(1));
   if (busy)
     each_row([&](int k, int s) {
       const float* d = v[k][s];
-      const float q = add_squares8(d, 0.f, true), more = add_squares8(d + 8, q, false);
-      rstd[k][s] = rsqrtf(wave_sum(upper ? more : q) / (float)K + LN_EPS);
+      rstd[k][s] = rsqrtf(over_768(wave_sum(add_squares4(d + 8, add_squares8(d, 0.f, true)))) + LN_EPS);
     });
   if constexpr (AHEAD > 2) fetch(PIECE(2));
   if (busy) {
-    float gain[TPW][16];
+    float gain[TPW][12];
 #pragma unroll
     for (int k = 0; k < TPW; ++k)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) gain[k][e] = sigmoidf_(sc[k][e >> 3][(e >> 2) & 1][e & 3]);
+      for (int e = 0; e < 12; ++e) gain[k][e] = sigmoidf_(sc[k][e >> 2][e & 3]);
+    // 16 bytes of slab lane / 8 and 8 of slab 8 + lane / 16; chunk c of a slab's row lies at position c ^ (row / 2 % 8)
+    char *const at0 = sP + (lane >> 3) * (ROWS * 128), *const at1 = sP + (8 + (lane >> 4)) * (ROWS * 128) + (lane & 1) * 8;
     each_row([&](int k, int s) {
-      const int tt = tt_0 + NW * k, row = tt * a.samples + s_0 + s;
+      const int tt = tt_0 + NW * k, row = tt * a.samples + s_0 + s, x = (row >> 1) & 7;
       const bool keep = tt < tt_n && s < count;
+      float o[12];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        float o[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float t = v[k][s][8 * i + e] * rstd[k][s];
-          o[e] = gain[k][8 * i + e] * t + sh[k][i][e >> 2][e & 3];
-        }
-        const int chunk = 64 * i + lane;  // chunk c of a slab's row lies at position c ^ (row / 2 % 8)
-        if (keep && (i == 0 || upper))
-          *reinterpret_cast<u32x4*>(sP + (chunk >> 3) * (ROWS * 128) + row * 128 + (((chunk & 7) ^ ((row >> 1) & 7)) << 4)) = pack8(o);
+      for (int e = 0; e < 12; ++e) {
+        const float t = v[k][s][e] * rstd[k][s];
+        o[e] = gain[k][e] * t + sh[k][e >> 2][e & 3];
+      }
+      if (keep) {
+        *reinterpret_cast<u32x4*>(at0 + row * 128 + (((lane & 7) ^ x) << 4)) = pack8(o);
+        *reinterpret_cast<u32x2*>(at1 + row * 128 + ((((lane >> 1) & 7) ^ x) << 4)) = u32x2{pack2bf(o[8], o[9]), pack2bf(o[10], o[11])};
       }
     });
   }
