@@ -316,6 +316,15 @@ int af3_pair_cond_transition_forward(
   return transition_impl(act, AF3_F32, ln_w, ln_b, w1_packed, w2, hidden, out, residual, rows, C_PAIR, 1, stream);
 }
 
+int af3_row_transition_forward(
+    float* act, const float* ln_w, const float* ln_b, const uint16_t* w1_frags, const uint16_t* w2_frags, int hidden,
+    int64_t rows, af3_stream_t stream) {
+  if (rows <= 0 || rows > 0x7fffffff) return AF3_ERR_BAD_ARG;
+  RowTransitionArgs a;
+  a.act = act; a.ln_w = ln_w; a.ln_b = ln_b; a.w1 = w1_frags; a.w2 = w2_frags; a.rows = (int)rows; a.hidden = hidden;
+  return launch_row_transition(a, static_cast<hipStream_t>(stream));
+}
+
 // ------------------------------------------- pair-biased self-attention (single / diffusion)
 size_t af3_batch_diffusion_self_attention_workspace_bytes(int64_t batch, int64_t seq, int channels) {
   if (batch <= 0 || seq <= 0 || channels <= 0) return 0;

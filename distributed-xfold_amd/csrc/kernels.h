@@ -454,6 +454,18 @@ struct SingleStepArgs {
 bool single_step_applies(const SingleStepArgs& a);
 int launch_single_step(const SingleStepArgs& a, hipStream_t s);
 
+// ----------------------------------------------------------- row_transition.hip
+// act += (silu(a) b) w2^T, (a, b) = LayerNorm(act) w1^T, rows of 384 fp32; w1 (rows in blocks of 32 of a and 32 of b) and w2
+// [384][hidden] in fragment order, bits 2 and 3 of a row number exchanged; hidden a multiple of 128
+constexpr int ROW_TRANSITION_CHANNELS = 384;
+struct RowTransitionArgs {
+  float* act = nullptr;  // [rows][384]
+  const float *ln_w = nullptr, *ln_b = nullptr;
+  const bf16_t *w1 = nullptr, *w2 = nullptr;
+  int rows = 0, hidden = 0;
+};
+int launch_row_transition(const RowTransitionArgs& a, hipStream_t s);
+
 // --------------------------------------------------------------- token_step.hip
 // Adaptive LayerNorm of rows of 768 channels and a product of them: with w in fragment order, [N][768], out[row][n0 ..] =
 // queries (bias, scale), keys, values, gate (sigmoid), N = 4 x 768, or with swiglu N / 2 hidden units (w in blocks of 64 rows).

@@ -56,6 +56,7 @@ SIGNATURES = {
         _i, [_vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _i64, _vp, _sz, _vp]),
     "af3_transition_forward": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _i, _i64, _vp]),
     "af3_pair_cond_transition_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _i64, _vp]),
+    "af3_row_transition_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i64, _vp]),
     "af3_triangle_multiplication_forward_padded": (
         _i, [_vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i64, _i, _vp, _sz, _vp]),
     "af3_grid_self_attn_forward_padded": (

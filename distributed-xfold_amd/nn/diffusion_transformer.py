@@ -112,6 +112,8 @@ class AdaLNZero(HipModule):
     """nn/d_diffusion_transformer.py:80-118: transition2(x), gated by
     sigmoid(adaptive_zero_cond(single_cond)) when conditioned."""
 
+    of_row_transition = False   # (set by the transition that takes the weights in fragment order as well)
+
     def __init__(self, *args, c_in: int = None, c_out: int = None, c_single_cond: int = None,
                  use_single_cond: bool = False, shard_out: bool = False) -> None:
         super().__init__()
@@ -126,6 +128,8 @@ class AdaLNZero(HipModule):
 
     def _pack(self):
         d = dict(w=bf16(self.transition2.weight))
+        if self.of_row_transition and d["w"].shape == (self.c_out, self.c_in):
+            d["w_frags"] = fragments(d["w"], swap23=True).reshape(d["w"].shape)
         if self.use_single_cond:
             d["w_cond"] = bf16(self.adaptive_zero_cond.weight)
             d["b_cond"] = f32(self.adaptive_zero_cond.bias)
@@ -150,6 +154,12 @@ class AdaLNZero(HipModule):
         return self.run(x.to(torch.bfloat16).contiguous(), single_cond, x.dtype)
 
 
+# Rows of 384 channels from which their transition is one kernel (af3_row_transition_forward), a tile of 64 for every second CU; us
+# on the device, norm and two products / one kernel: 2000 rows 20.1 / 28.9, 5000 29.6 / 30.5, 8192 36.1 / 32.6, 16384 58.2 / 38.5,
+# 20000 63.9 / 58.2, 76800 258 / 163, 307200 1078 / 640.
+ROW_TRANSITION_ROWS = 8192
+
+
 class DiffusionTransition(HipModule):
     """nn/d_diffusion_transformer.py:120-145."""
 
@@ -165,11 +175,14 @@ class DiffusionTransition(HipModule):
         self.transition1 = nn.Linear(c_x, 2 * c_x * num_intermediate_factor, bias=False)
         self.adaptive_zero_init = AdaLNZero(c_in=num_intermediate_factor * c_x, c_out=c_x,
                                             c_single_cond=c_single_cond, use_single_cond=use_single_cond)
+        self.adaptive_zero_init.of_row_transition = c_x == 384 and not use_single_cond
 
     def _pack(self):
         d = dict(w1=bf16(pack_swiglu(self.transition1.weight, 32)))
         if self.c_x == 128 and not self.use_single_cond:
             d["w1_64"] = bf16(pack_swiglu(self.transition1.weight, 64)).reshape(-1, 128, 128)
+        if self.c_x == 384 and not self.use_single_cond and d["w1"].shape == (768 * self.num_intermediate_factor, 384):
+            d["w1_frags"] = fragments(d["w1"], swap23=True).reshape(d["w1"].shape)
         return d
 
     def run(self, x, single_cond, residual: bool, cond=None):
@@ -182,6 +195,15 @@ class DiffusionTransition(HipModule):
             norm = self.adaptive_layernorm.packed()
             return ops.transition128(x, norm["ln_w"], norm["ln_b"], self.packed()["w1_64"], self.adaptive_zero_init.packed()["w"],
                                      residual=residual, pair_cond=True)
+        # 384 channels likewise, where there are rows enough
+        if (self.c_x == 384 and self.num_intermediate_factor <= 21 and residual and not self.use_single_cond and single_cond is None
+                and cond is None and x.is_cuda and x.is_contiguous() and x.dtype == torch.float32 and x.data_ptr() % 16 == 0
+                and ROW_TRANSITION_ROWS <= x.numel() // 384 < 2 ** 31
+                and as_written((self.adaptive_layernorm, AdaptiveLayerNorm), (self.adaptive_zero_init, AdaLNZero))):
+            norm, w1, w2 = (self.adaptive_layernorm.packed(), self.packed().get("w1_frags"),
+                            self.adaptive_zero_init.packed().get("w_frags"))
+            if w1 is not None and w2 is not None:       # (weights of the shapes that they were made with)
+                return ops.row_transition(x, norm["ln_w"], norm["ln_b"], w1, w2)
         ss, gate = cond if cond is not None else (None, None)
         xa = self.adaptive_layernorm(x, single_cond, scale_shift=ss)
         h = ops.linear(xa, self.packed()["w1"], mode=L.LINEAR_SWIGLU)

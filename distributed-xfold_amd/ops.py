@@ -229,6 +229,24 @@ def transition128(act, layernorm_weight, layernorm_bias, w1_packed, w2, residual
     return out
 
 
+def row_transition(act, layernorm_weight, layernorm_bias, w1_frags, w2_frags):
+    """act += its SwiGLU transition, rows of 384 fp32, in place (af3_row_transition_forward).  w1_frags, w2_frags: the weights
+    as `fragments(.., swap23=True)` lays them out, [2 hidden, 384] (packed in blocks of 32 before) and [384, hidden]."""
+    lib = _L.load()
+    hidden = w2_frags.shape[-1]
+    _gpu(act, "act", torch.float32)
+    if act.shape[-1] != 384:
+        raise ValueError("act: last dimension must be 384")
+    _gpu(layernorm_weight, "layernorm_weight", torch.float32, (384,))
+    _gpu(layernorm_bias, "layernorm_bias", torch.float32, (384,))
+    _gpu(w1_frags, "w1_frags", torch.bfloat16, (2 * hidden, 384))
+    _gpu(w2_frags, "w2_frags", torch.bfloat16, (384, hidden))
+    rc = lib.af3_row_transition_forward(_p(act), _p(layernorm_weight), _p(layernorm_bias), _p(w1_frags), _p(w2_frags),
+                                        int(hidden), act.numel() // 384, _stream(act.device))
+    _L.check(rc, "af3_row_transition_forward")
+    return act
+
+
 @_uses_scratch
 def pairformer_stack(blocks, pair, pair_mask, single, seq_mask, pair_mask_incoming=None, single_stream=None, join=True):
     """A run of Pairformer blocks in one call (af3_pairformer_stack_forward), pair [N, N, 128] (64 where the blocks'

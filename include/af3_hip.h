@@ -137,6 +137,14 @@ int af3_pair_cond_transition_forward(
     const float* act, const float* layernorm_weight, const float* layernorm_bias,
     const uint16_t* w1_packed, const uint16_t* w2, int hidden,
     float* out, int residual, int64_t rows, af3_stream_t stream);
+/* The same of rows of 384 channels (the head's single conditionings, nn/d_diffusion_transformer.py:120-145), in place:
+ * act [rows][384] fp32 += the transition of its rows, one pass.  hidden: a multiple of 128, at most 8192.  Weights in the
+ * order of the matrix instructions' fragments, bits 2 and 3 of the row numbers exchanged: w1_frags of the first layer's rows
+ * in blocks of 32 (silu half) and 32 (linear half), w2_frags of the second layer's [384][hidden].
+ */
+int af3_row_transition_forward(
+    float* act, const float* layernorm_weight, const float* layernorm_bias,
+    const uint16_t* w1_frags, const uint16_t* w2_frags, int hidden, int64_t rows, af3_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * The three pair operators above on FEWER than 128 pair channels: the Pairformer
