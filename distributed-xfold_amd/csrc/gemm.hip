@@ -459,6 +459,7 @@ int launch_gemm_nt(const GemmArgs& g_in, hipStream_t stream) {
   const int64_t T = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch;
   const bool wide = g.epi == EPI_SWIGLU;
   if (!vec) return launch_tile<1, 1, 2, 2, 1, 2, 4, false, false>(g, stream);
+  if (wide_product_applies(g)) return launch_wide_product(g, stream);  // (K = 384, many fp32 results)
   if (g.K % KS) return launch_tile<1, 1, 2, 2, 1, 2, 4, false>(g, stream);
   if (g.split_k && g.K > 256) {
     if (T <= 128 && !wide) return g.K >= 1024 ? launch_tile<1, 1, 1, 1, 8, 2, 2>(g, stream) : launch_tile<1, 1, 1, 1, 4, 2, 2>(g, stream);

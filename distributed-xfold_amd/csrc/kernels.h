@@ -37,6 +37,13 @@ struct GemmArgs {
   int split_k = 0;  // the K range may be summed in parts by several waves (another order of summation)
 };
 int launch_gemm_nt(const GemmArgs& g, hipStream_t stream);
+// wide_product.hip: K = 384, fp32 results of very many columns
+struct WideWalk {
+  int per_xcd = 0, total = 0, parts = 0, panels = 0;  // parts of a strip's rows, and their panels of 32
+  unsigned magic_parts = 0;
+};
+bool wide_product_applies(const GemmArgs& g);
+int launch_wide_product(const GemmArgs& g, hipStream_t stream);
 // panel.hip: square products of up to a few hundred rows a batch entry; AF3_ERR_UNSUPPORTED for others
 int launch_panel_product(const GemmArgs& g, hipStream_t stream);
 

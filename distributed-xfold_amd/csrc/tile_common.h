@@ -421,6 +421,12 @@ template <> __device__ __forceinline__ void store_raw<float>(float* p, const Ele
   *reinterpret_cast<f32x4*>(p + 4) = r.b;
 }
 
+// 64 lanes x 16 bytes from memory (uniform base, a byte offset per lane) to 1 KB of LDS at `lds`.  Inline assembly, because the
+// compiler's own form makes later LDS reads wait for every such load in flight; the panel is read behind a wait of its own.
+__device__ __forceinline__ void load_to_lds(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:0" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
+
 // fragments of 32 weight rows (block `blk`) for `n` k-steps from k-step k0 on, of a matrix with `nks` k-steps
 template <int n>
 __device__ __forceinline__ void load_frags(const bf16_t* w, int blk, int nks, int k0, int lane, bf16x8* f) {

@@ -222,12 +222,6 @@ __global__ __launch_bounds__(64 * NW, 2) void norm_product_kernel(NormProductArg
   }
 }
 
-// 64 lanes x 16 bytes from memory (uniform base, a byte offset per lane) to 1 KB of LDS at `lds`.  Inline assembly, because the
-// compiler's own form makes later LDS reads wait for every such load in flight; the panel is read behind a wait of its own.
-__device__ __forceinline__ void load_to_lds(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:0" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
-}
-
 // The products that lead back into the stream: act = (y w^T) gate + act, 768 result columns, K = 128 KP.  A workgroup takes 32
 // rows and 32 columns per wave; the rows go to LDS as a panel, all of them at once, the weights' fragments straight to registers,
 // gate and stream asked for behind them: one trip to memory, a chain of 48 or 96 matrix instructions (some 36 cycles each), and
