@@ -462,6 +462,15 @@ int af3_gathered_relu_mean_forward(const uint16_t* src, const int32_t* idx, cons
                                    static_cast<hipStream_t>(stream));
 }
 
+int af3_atom_aggregate_forward(const uint16_t* x, const int32_t* idx, const float* count, const uint16_t* w_frags, float* out,
+                               int64_t batch, int64_t n_src, int64_t n_out, int slots, af3_stream_t stream) {
+  if (batch <= 0 || batch > 0x7fffffff || n_out <= 0 || n_out > 0x7fffffff) return AF3_ERR_BAD_ARG;
+  AtomAggregateArgs a;
+  a.x = x; a.idx = idx; a.count = count; a.w = w_frags; a.out = out; a.n_src = n_src;
+  a.batch = (int)batch; a.tokens = (int)n_out; a.slots = slots;
+  return launch_atom_aggregate(a, static_cast<hipStream_t>(stream));
+}
+
 int af3_atom_position_features_forward(const float* positions, const int32_t* rows, const float* weight,
                                        const float* cond, void* out, int out_dtype, int64_t batch, int64_t n_slots,
                                        int64_t n_queries, int channels, af3_stream_t stream) {

@@ -197,6 +197,12 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// acc + the two bf16 values packed in `pair` (v_dot2c_f32_bf16 with a pair of ones)
+__device__ __forceinline__ float dot2_ones(uint32_t pair, float acc) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf2;
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, pair), __builtin_bit_cast(bf2, 0x3F803F80u), acc, false);
+}
+
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits
 // for every outstanding global load and STORE of the wave (vmcnt(0)), which
 // exposes the full HBM write latency at each barrier of a kernel that streams

@@ -461,6 +461,19 @@ struct SingleStepArgs {
 bool single_step_applies(const SingleStepArgs& a);
 int launch_single_step(const SingleStepArgs& a, hipStream_t s);
 
+// ----------------------------------------------------------- atom_aggregate.hip
+// out[b][t] = sum over slots s, idx[t][s] >= 0, of relu(bf16(x[b][idx[t][s]] w^T)) / count[t]; 128 channels to 768, w in fragment order
+struct AtomAggregateArgs {
+  const bf16_t* x = nullptr;   // [batch][n_src][128]
+  const int* idx = nullptr;    // [tokens][slots], below n_src; at most 32 slots
+  const float* count = nullptr;
+  const bf16_t* w = nullptr;
+  float* out = nullptr;        // [batch][tokens][768]
+  int64_t n_src = 0;
+  int batch = 0, tokens = 0, slots = 0;
+};
+int launch_atom_aggregate(const AtomAggregateArgs& a, hipStream_t s);
+
 // ----------------------------------------------------------- row_transition.hip
 // act += (silu(a) b) w2^T, (a, b) = LayerNorm(act) w1^T, rows of 384 fp32; w1 (rows in blocks of 32 of a and 32 of b) and w2
 // [384][hidden] in fragment order, bits 2 and 3 of a row number exchanged; hidden a multiple of 128

@@ -106,12 +106,6 @@ __device__ __forceinline__ float max32(const f32x16& a, const f32x16& b) {
   return fmaxf(fmaxf(fmaxf(t9a, t9b), t9c), t9d);
 }
 
-// acc + the two bf16 values packed in `pair` (v_dot2c_f32_bf16 with a pair of ones)
-__device__ __forceinline__ float dot2_ones(uint32_t pair, float acc) {
-  typedef __attribute__((ext_vector_type(2))) __bf16 bf2;
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, pair), __builtin_bit_cast(bf2, 0x3F803F80u), acc, false);
-}
-
 // o *= f with every register multiplied in place.  Written as plain C++ inside a rarely taken
 // branch, the compiler keeps the accumulator in two register tuples and copies all sixteen
 // registers on the path that does NOT multiply, every iteration.

@@ -88,6 +88,7 @@ SIGNATURES = {
     "af3_gather_rows_add_forward": (_i, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _vp]),
     "af3_position_update_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _vp]),
     "af3_gathered_relu_mean_forward": (_i, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _i, _vp]),
+    "af3_atom_aggregate_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _vp]),
     "af3_batch_diffusion_cross_attention_workspace_bytes": (_sz, [_i64, _i64, _i64, _i]),
     "af3_batch_diffusion_cross_attention_forward": (
         _i, [_vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i, _vp, _i, _i64, _i64, _i64, _i, _vp, _sz, _vp]),

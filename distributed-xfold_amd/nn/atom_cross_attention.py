@@ -23,7 +23,7 @@ import torch.nn as nn
 
 from .. import check, ops
 from .atom_layout import GatherInfo, convert
-from .base import HipModule, as_written, bf16, drop_mesh, f32, in_check_mode
+from .base import HipModule, as_written, bf16, drop_mesh, f32, fragments, in_check_mode
 from .diffusion_transformer import DiffusionCrossAttTransformer
 
 
@@ -124,6 +124,8 @@ class AtomCrossAttEncoder(HipModule):
 
     def _pack(self):
         d = dict(w_aggr=bf16(self.project_atom_features_for_aggr.weight))
+        if d["w_aggr"].shape == (768, 128):
+            d["w_aggr_frags"] = fragments(d["w_aggr"]).reshape(768, 128)
         if self.with_trunk_single_cond:
             d["ts_ln"] = f32(self.lnorm_trunk_single_cond.weight)
             d["ts_w"] = bf16(self.embed_trunk_single_cond.weight)
@@ -297,27 +299,29 @@ class AtomCrossAttEncoder(HipModule):
         else:
             q_act = q_act * qm.to(q_act.dtype)
         skip = q_act
-        if in_check_mode():
-            agg = check._lin(q_act.contiguous(), self.project_atom_features_for_aggr)
-        else:
-            agg = ops.linear(q_act.to(torch.bfloat16).contiguous(), self.packed()["w_aggr"])
         # mask_mean over the atoms of a token (:328-331); the gather zeroes the absent atoms
         count = c.atom_count if c.atom_count is not None else self._atom_count(batch)
         if in_check_mode():
+            agg = check._lin(q_act.contiguous(), self.project_atom_features_for_aggr)
             tok_atoms = convert(aca.queries_to_token_atoms, agg, (-3, -2))
             tok_act = torch.relu(tok_atoms).float().sum(-2) / count[..., None]
         else:
-            # conversion to the token-atom layout, ReLU and the mean in one pass over the atoms that exist
+            # projection, conversion to the token-atom layout, ReLU and the mean in one pass over the atoms that exist
             gi = aca.queries_to_token_atoms
             rows = getattr(gi, "_af3_rows32", None)
-            if rows is None or rows.device != agg.device:
+            if rows is None or rows.device != q_act.device:
                 rows = torch.where(gi.gather_mask, gi.gather_idxs, -1).to(torch.int32).contiguous()
                 try:
                     gi._af3_rows32 = rows          # the layout of a batch does not change between evaluations
                 except AttributeError:
                     pass
-            n_src = agg.shape[-3] * agg.shape[-2]
-            tok_act = ops.gathered_relu_mean(agg.reshape(-1, n_src, agg.shape[-1]), rows, count.contiguous())
+            p, x = self.packed(), q_act.to(torch.bfloat16).contiguous()
+            n_src = x.shape[-3] * x.shape[-2]
+            if "w_aggr_frags" in p and rows.dim() == 2 and rows.shape[1] <= 32:
+                tok_act = ops.atom_aggregate(x.reshape(-1, n_src, x.shape[-1]), rows, count.contiguous(), p["w_aggr_frags"])
+            else:
+                agg = ops.linear(x, p["w_aggr"])
+                tok_act = ops.gathered_relu_mean(agg.reshape(-1, n_src, agg.shape[-1]), rows, count.contiguous())
             if not batched:
                 tok_act = tok_act[0]
         return AtomCrossAttEncoderOutput(tok_act, skip, c.queries_mask, c.queries_single_cond, c.keys_mask,

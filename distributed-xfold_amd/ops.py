@@ -732,6 +732,29 @@ def gathered_relu_mean(src, idx, count):
     return out
 
 
+def atom_aggregate(x, idx, count, w_frags):
+    """out[b, t] = sum_a relu(x[b, idx[t, a]] @ w.T) / count[t] over the slots with idx >= 0, the product rounded to bf16
+    (af3_atom_aggregate_forward).  x [B, n_src, 128] bf16, idx [T, A] int32 with A <= 32, count [T] fp32, w_frags [768, 128]
+    bf16 as `fragments` lays it out -> [B, T, 768] fp32."""
+    lib = _L.load()
+    _gpu(x, "x", torch.bfloat16)
+    if x.dim() != 3 or x.shape[-1] != 128:
+        raise ValueError("x: expected [B, n_src, 128]")
+    b, n_src, _ = x.shape
+    if idx.dtype != torch.int32 or idx.dim() != 2 or not idx.is_contiguous() or idx.device != x.device:
+        raise ValueError("idx: expected a contiguous int32 [T, A] tensor on the device of x")
+    t, a = idx.shape
+    if a > 32:
+        raise ValueError("at most 32 slots")
+    rows_in_range(idx, n_src, "idx")
+    _gpu(count, "count", torch.float32, (t,))
+    _gpu(w_frags, "w_frags", torch.bfloat16, (768, 128))
+    out = torch.empty((b, t, 768), dtype=torch.float32, device=x.device)
+    rc = lib.af3_atom_aggregate_forward(_p(x), _p(idx), _p(count), _p(w_frags), _p(out), b, n_src, t, a, _stream(x.device))
+    _L.check(rc, "af3_atom_aggregate_forward")
+    return out
+
+
 def quad_major_bias(bias):
     """[..., Sq, Sk] -> [..., Sk/4, Sq, 4]: the pair-bias order in which the
     attention kernel's loads are contiguous (Sk a multiple of 4).  One strided

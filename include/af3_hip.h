@@ -318,6 +318,11 @@ int af3_transpose_bf16_forward(const uint16_t* in, uint16_t* out, int64_t rows, 
 int af3_gathered_relu_mean_forward(const uint16_t* src, const int32_t* idx, const float* count, float* out,
                                    int64_t batch, int64_t n_src, int64_t n_out, int slots, int channels,
                                    af3_stream_t stream);
+/* The projection in front of it as well: relu and mean of bf16(x w^T), x [batch][n_src][128] bf16, 768 result channels,
+ * w_frags: w [768][128] in the order of the matrix instructions' fragments; at most 32 slots.
+ */
+int af3_atom_aggregate_forward(const uint16_t* x, const int32_t* idx, const float* count, const uint16_t* w_frags, float* out,
+                               int64_t batch, int64_t n_src, int64_t n_out, int slots, af3_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * Embedding of the noisy atom positions, the head of the atom cross-attention
