@@ -589,6 +589,8 @@ struct GatherAtomsArgs {
 };
 int launch_gather_atoms(const GatherAtomsArgs& a, hipStream_t s);
 enum { POS_SCALE = 0, POS_BLEND = 1, POS_PLACE = 2, POS_STEP = 3 };
+int launch_augment_positions(const float* x, const float* rot, const float* shift, const float* mask, const float* noise, float* out,
+                             int64_t samples, int64_t atoms, hipStream_t s);
 int launch_positions(int op, const float* x, const float* y, const float* mask, const float* level, const float* other, float f,
                      float* out, int64_t samples, int64_t atoms, hipStream_t s);
 

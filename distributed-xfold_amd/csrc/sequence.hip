@@ -811,6 +811,10 @@ int af3_gather_atoms_forward(const int64_t* idx, const uint8_t* exists, int64_t 
   return launch_gather_atoms(a, static_cast<hipStream_t>(stream));
 }
 
+int af3_augment_positions_forward(const float* x, const float* rot, const float* shift, const float* mask, const float* noise, float* out,
+                                  int64_t samples, int64_t atoms, af3_stream_t stream) {
+  return launch_augment_positions(x, rot, shift, mask, noise, out, samples, atoms, static_cast<hipStream_t>(stream));
+}
 int af3_positions_forward(int op, const float* x, const float* y, const float* mask, const float* level, const float* next,
                           float factor, float* out, int64_t samples, int64_t atoms, af3_stream_t stream) {
   return launch_positions(op, x, y, mask, level, next, factor, out, samples, atoms, static_cast<hipStream_t>(stream));

@@ -70,6 +70,7 @@ SIGNATURES = {
         _i, [_vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _i, _vp]),
     "af3_add_rows_forward": (_i, [_vp, _vp, _i64, _i64, _vp, _i, _i64, _i, _vp]),
     "af3_mask_rows_forward": (_i, [_vp, _vp, _i64, _i64, _i, _vp]),
+    "af3_augment_positions_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "af3_positions_forward": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _f, _vp, _i64, _i64, _vp]),
     "af3_msa_workspace_bytes": (_sz, [_i64, _i64]),
     "af3_outer_product_mean_forward": (_i, [_vp, _vp, _i, _vp, _vp, _i, _i, _i64, _i64, _vp, _sz, _vp]),

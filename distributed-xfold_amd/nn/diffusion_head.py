@@ -319,9 +319,6 @@ class DiffusionSampler:
         if positions is None:
             positions = torch.randn((self.num_samples,) + tuple(mask.shape) + (3,), generator=generator, device=dev)
         positions = positions.float() * levels[0]
-        # the mean of random_augmentation divides by a count that no step changes
-        m = mask.to(positions.dtype)[None, ..., None]
-        count = torch.clamp(m.expand_as(positions[..., :1]).sum(dim=(-2, -3), keepdim=True), min=1e-6)
         mask_f = mask.float().contiguous()
         for i in range(self.diffusion_steps):
             rot = rotations[i] if rotations is not None else random_rotation(generator, dev)
@@ -333,9 +330,9 @@ class DiffusionSampler:
                     noise = noises[i] if noises is not None else torch.randn(positions.shape, generator=generator, device=dev)
                 noisy = positions + nscale[i] * noise
             else:   # random_augmentation, and the step's scalar of noise added
-                center = (m * positions).sum(dim=(-2, -3), keepdim=True) / count
-                turned = torch.einsum("...i,ij->...j", positions - center, rot.float())
-                noisy = ops.positions(ops.POS_PLACE, turned.contiguous(), trans.float().contiguous(), mask_f, nscale[i])
+                shape = (1,) * (4 - positions.dim()) + positions.shape
+                noisy = ops.augment_positions(positions.reshape((-1,) + mask_f.shape + (3,)).contiguous(), rot.float().contiguous(),
+                                              trans.float().reshape(3).contiguous(), mask_f, nscale[i]).view(shape)
             denoised = head(noisy, t_hat[i], batch, embeddings, single_cond[i], pair_cond, state=state)
             positions = ops.positions(ops.POS_STEP, noisy, denoised, None, t_hat[i], levels[i + 1], self.step_scale)
         return {"atom_positions": positions, "mask": mask}

@@ -422,6 +422,26 @@ def positions(op, x, y, mask, level, next_level=None, factor=0.0):
     return out
 
 
+def augment_positions(x, rot, shift, mask, noise):
+    """(x - masked mean) @ rot + shift, times mask, plus noise, a sample at a time (af3_augment_positions_forward): x
+    [samples, N, A, 3], mask [N, A], rot [3, 3], shift [3], `noise` a one-element device tensor, all fp32."""
+    lib = _L.load()
+    _gpu(x, "x", torch.float32)
+    _gpu(rot, "rot", torch.float32, (3, 3))
+    _gpu(shift, "shift", torch.float32, (3,))
+    _gpu(mask, "mask", torch.float32)
+    _gpu(noise, "noise", torch.float32)
+    if noise.numel() != 1:
+        raise ValueError(f"noise: expected one element, got {tuple(noise.shape)}")
+    if x.shape[-1] != 3 or x.shape[1:-1] != mask.shape:
+        raise ValueError("x: expected [samples, N, A, 3] over a mask [N, A]")
+    out = torch.empty_like(x)
+    rc = lib.af3_augment_positions_forward(_p(x), _p(rot), _p(shift), _p(mask), _p(noise), _p(out), x.shape[0], mask.numel(),
+                                           _stream(x.device))
+    _L.check(rc, "af3_augment_positions_forward")
+    return out
+
+
 def msa_in_range(rows, n) -> bool:
     """Whether the MSA track's own kernels take `rows` MSA rows of `n` tokens (their indices are 32 bits wide)."""
     return _L.load().af3_msa_workspace_bytes(rows, n) > 0

@@ -629,6 +629,11 @@ int af3_gather_atoms_forward(const int64_t* idx, const uint8_t* exists, int64_t 
                              float* out_positions, int32_t* out_uid, int channels, af3_stream_t stream);
 int af3_positions_forward(int op, const float* x, const float* y, const float* mask, const float* level, const float* next,
                           float factor, float* out, int64_t samples, int64_t atoms, af3_stream_t stream);
+/* The start of a sampling step (d_alphafold3.py:337-346): each sample less its masked mean, times rot [3][3] from the right, plus
+ * shift [3], times mask, plus *noise.  out is not x.
+ */
+int af3_augment_positions_forward(const float* x, const float* rot, const float* shift, const float* mask, const float* noise, float* out,
+                                  int64_t samples, int64_t atoms, af3_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * The Evoformer's MSA track on 64 channels (nn/d_primitives.py:42-70,
