@@ -313,8 +313,11 @@ class DiffusionTransformer(HipModule):
                 b_ss.append(torch.cat([aln.single_cond_scale.bias, torch.zeros_like(aln.single_cond_scale.bias)]))
                 w_gate.append(az.adaptive_zero_cond.weight)
                 b_gate.append(az.adaptive_zero_cond.bias)
-        return dict(ln_w=f32(self.pair_input_layer_norm.weight),
-                    w_logits=[pad_rows(bf16(m.weight), 32) for m in self.pair_logits_projection],
+        w_logits = [pad_rows(bf16(m.weight), 32) for m in self.pair_logits_projection]
+        n_out = self.super_block_size * self.num_head
+        if n_out % 32 == 0 and all(w.shape == (n_out, w_logits[0].shape[1]) for w in w_logits):     # one product for all super-blocks
+            w_logits = [torch.cat(w_logits)] if w_logits else w_logits
+        return dict(ln_w=f32(self.pair_input_layer_norm.weight), w_logits=w_logits,
                     w_ss=bf16(torch.cat(w_ss, dim=0)), b_ss=f32(torch.cat(b_ss)),
                     w_gate=bf16(torch.cat(w_gate, dim=0)), b_gate=f32(torch.cat(b_gate)))
 
@@ -339,12 +342,13 @@ class DiffusionTransformer(HipModule):
         and hands them to `forward(..., pair_logits=...)`."""
         p = self.packed()
         pair_cond = pair_cond.contiguous()
-        n_out = self.super_block_size * self.num_head
+        n_out, quads = self.super_block_size * self.num_head, pair_cond.shape[0] % 4 == 0
         out = []
-        for sb in range(self.num_super_blocks):
-            logits = ops.pair_logits(pair_cond, p["ln_w"], None, p["w_logits"][sb], n_out, quads=pair_cond.shape[0] % 4 == 0)
-            out.append(logits.view(self.super_block_size, self.num_head, *logits.shape[1:]))     # (b h) .. -> b h ..
-        return out
+        of = len(self.pair_logits_projection) if len(p["w_logits"]) == 1 else 1
+        for w in p["w_logits"]:     # of all super-blocks together, or of one after the other
+            logits = ops.pair_logits(pair_cond, p["ln_w"], None, w, of * n_out, quads=quads)
+            out += logits.view(of, self.super_block_size, self.num_head, *logits.shape[1:]).unbind()     # (b h) .. -> b h ..
+        return out[:self.num_super_blocks]
 
     def forward(self, act: torch.Tensor, mask: torch.Tensor, single_cond: torch.Tensor,
                 pair_cond: torch.Tensor, pair_logits=None) -> torch.Tensor:
