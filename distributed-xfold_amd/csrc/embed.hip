@@ -298,27 +298,48 @@ __global__ __launch_bounds__(AUGMENT_THREADS) void augment_positions_kernel(cons
 // The windows of an atom layout that somebody reads, in their order.  A layout has room for every token's 24 atoms and as many empty
 // slots behind the last atom as there are fewer, half of the windows and more.  Asked for are a window with an atom in it (mask) and
 // one that the way back reads; and all of them should any key be a row that neither of these names, whose value would then count.
-// One workgroup, the rows as bits in LDS: 18432 rows and 73728 keys 11 us, once a batch.
-constexpr int WINDOW_THREADS = 1024, WINDOW_ROWS = 1 << 19;
+// One workgroup, the rows as bits in LDS, eight loads of a thread on their way at a time: 9216 rows and 36864 keys 17 us (one load
+// at a time 32), twice as many 27 (60), once a batch.
+constexpr int BATCH = 8, WINDOW_THREADS = 1024, WINDOW_ROWS = 1 << 19;
 __global__ __launch_bounds__(WINDOW_THREADS) void atom_windows_kernel(AtomWindowsArgs a) {
   __shared__ uint32_t want[WINDOW_ROWS / 32];
   __shared__ int stray, live_of[WINDOW_THREADS / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rows = a.windows * a.queries;
   if (tid == 0) stray = 0;
-  for (int r0 = 0; r0 < rows; r0 += WINDOW_THREADS) {
-    const int r = r0 + tid;
-    const uint64_t b = __ballot(r < rows && a.mask[min(r, rows - 1)] != 0.f);
-    if ((lane & 31) == 0 && r < rows) want[r >> 5] = (uint32_t)(lane ? b >> 32 : b);
+  for (int r0 = 0; r0 < rows; r0 += BATCH * WINDOW_THREADS) {
+    float m[BATCH];
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) m[k] = a.mask[min(r0 + k * WINDOW_THREADS + tid, rows - 1)];
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) {
+      const int r = r0 + k * WINDOW_THREADS + tid;
+      const uint64_t b = __ballot(r < rows && m[k] != 0.f);
+      if ((lane & 31) == 0 && r < rows) want[r >> 5] = (uint32_t)(lane ? b >> 32 : b);
+    }
   }
   __syncthreads();
-  for (int64_t i = tid; i < a.slots; i += WINDOW_THREADS) {
-    const int64_t r = a.back_idx[i];
-    if (a.back_exists[i] && r >= 0 && r < rows) atomicOr(&want[r >> 5], 1u << (r & 31));
+  for (int64_t i0 = 0; i0 < a.slots; i0 += BATCH * WINDOW_THREADS) {
+    int64_t r[BATCH];
+    bool there[BATCH];
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) {
+      const int64_t i = min(i0 + k * WINDOW_THREADS + tid, a.slots - 1);
+      r[k] = a.back_idx[i];
+      there[k] = a.back_exists[i];
+    }
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k)  // (the last one again does no harm)
+      if (there[k] && r[k] >= 0 && r[k] < rows) atomicOr(&want[r[k] >> 5], 1u << (r[k] & 31));
   }
   __syncthreads();
-  for (int64_t i = tid; i < (int64_t)a.windows * a.keys; i += WINDOW_THREADS) {
-    const int r = a.key_rows[i];
-    if (r >= 0 && r < rows && !(want[r >> 5] >> (r & 31) & 1)) stray = 1;
+  const int64_t keys = (int64_t)a.windows * a.keys;
+  for (int64_t i0 = 0; i0 < keys; i0 += BATCH * WINDOW_THREADS) {
+    int r[BATCH];
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) r[k] = a.key_rows[min(i0 + k * WINDOW_THREADS + tid, keys - 1)];
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k)
+      if (r[k] >= 0 && r[k] < rows && !(want[r[k] >> 5] >> (r[k] & 31) & 1)) stray = 1;
   }
   __syncthreads();
   int before = 0;
