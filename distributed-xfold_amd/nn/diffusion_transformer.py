@@ -350,21 +350,27 @@ class DiffusionTransformer(HipModule):
             out += logits.view(of, self.super_block_size, self.num_head, *logits.shape[1:]).unbind()     # (b h) .. -> b h ..
         return out[:self.num_super_blocks]
 
+    def conditioning(self, single_cond: torch.Tensor):
+        """What all blocks take from single_cond [rows, c_single_cond]: scale and shift of their adaptive norms and their gates,
+        fp32 rows.  A row's depend on that row alone, so a caller with several single_conds may ask for them together and
+        hand `forward(..., cond=...)` the rows of each."""
+        p = self.packed()
+        ss_all = ops.linear(ops.layer_norm(single_cond), p["w_ss"], bias=p["b_ss"], out_dtype=torch.float32)
+        gate_all = ops.linear(single_cond.to(torch.bfloat16), p["w_gate"], bias=p["b_gate"], out_dtype=torch.float32,
+                              sigmoid=True)
+        return ss_all, gate_all
+
     def forward(self, act: torch.Tensor, mask: torch.Tensor, single_cond: torch.Tensor,
-                pair_cond: torch.Tensor, pair_logits=None) -> torch.Tensor:
+                pair_cond: torch.Tensor, pair_logits=None, cond=None) -> torch.Tensor:
         """act [B, N, c_act] (updated in place, as the reference's `act +=`),
-        mask [N] or [B, N], single_cond [N, c_single_cond], pair_cond [N, N, c_pair_cond]."""
+        mask [N] or [B, N], single_cond [N, c_single_cond], pair_cond [N, N, c_pair_cond]; `cond`: see `conditioning`."""
         if in_check_mode():
             return check.diffusion_transformer(self, act, mask, single_cond, pair_cond)
-        p = self.packed()
         if not act.is_contiguous():
             raise ValueError("act must be contiguous (it is updated in place)")
         c, n_mod = self.c_act, 2 * self.num_blocks
-        sc = single_cond.contiguous()
-        rows = sc.numel() // sc.shape[-1]
-        ss_all = ops.linear(ops.layer_norm(sc), p["w_ss"], bias=p["b_ss"], out_dtype=torch.float32)
-        gate_all = ops.linear(sc.to(torch.bfloat16), p["w_gate"], bias=p["b_gate"], out_dtype=torch.float32,
-                              sigmoid=True)
+        rows = single_cond.numel() // single_cond.shape[-1]
+        ss_all, gate_all = cond if cond is not None else self.conditioning(single_cond.contiguous())
         if pair_logits is None:
             pair_logits = self.pair_logits(pair_cond)
         ss_all, gate_all = ss_all.view(rows, n_mod, 2 * c), gate_all.view(rows, n_mod, c)
